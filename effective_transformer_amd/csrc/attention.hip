@@ -223,7 +223,8 @@ template <typename T, int NKT, int WAVES, int CPT, bool PF>
 __global__ __launch_bounds__(WAVES * kWave) void attention_kernel(
     const T* __restrict__ q_src, const T* __restrict__ k_src, const T* __restrict__ v_src, int layout, int packed_ld,
     const T* __restrict__ attr_mask, T* __restrict__ dst, const int32_t* __restrict__ seq_start,
-    const int32_t* __restrict__ word_idx, int batch, int seq_len, int heads, int heads_per_wg, float scaler) {
+    const int32_t* __restrict__ word_idx, int batch, int seq_len, int heads, int heads_per_wg, float scaler,
+    int split_out) {
   using Cfg = AttnCfg<T>;
   using Sm = AttnSmem<T, NKT>;
   using C = Chunk16<T>;
@@ -354,6 +355,8 @@ __global__ __launch_bounds__(WAVES * kWave) void attention_kernel(
     const int qt = wave + qi * WAVES;
     const int tq = qt < n_tiles ? tok_of_pos[qt * 16 + l16] : -1;
     out_row[qi] = tq >= 0 ? dst + (size_t)tq * H + g * (sizeof(T) == 2 ? 16 : 4) : nullptr;
+    if (sizeof(T) == 4 && split_out && tq >= 0)
+      out_row[qi] = reinterpret_cast<T*>(reinterpret_cast<uint16_t*>(dst) + (size_t)tq * 3 * H);
   }
 
   for (int head = h_begin; head < h_end; ++head) {
@@ -524,7 +527,8 @@ __global__ __launch_bounds__(WAVES * kWave) void attention_kernel(
             out4 v;
 #pragma unroll
             for (int r = 0; r < 4; ++r) v[r] = (T)o[dt][r];
-            *reinterpret_cast<out4*>(orow + dt * 16) = v;
+            if (split_out) store_split<4>(reinterpret_cast<uint16_t*>(out_row[qi]), head * kD + dt * 16 + g * 4, v);
+            else *reinterpret_cast<out4*>(orow + dt * 16) = v;
           }
         }
       }
@@ -537,7 +541,7 @@ __global__ __launch_bounds__(WAVES * kWave) void attention_kernel(
 template <typename T, int NKT>
 void attention_launch(const void* q, const void* k, const void* v, int layout, int packed_ld, const void* attr_mask,
                       void* dst, const int32_t* seq_start, const int32_t* word_idx, int batch, int seq_len, int heads,
-                      float scaler, hipStream_t stream) {
+                      float scaler, bool split_out, hipStream_t stream) {
   using Sm = AttnSmem<T, NKT>;
   constexpr int kCpr = kD * (int)sizeof(T) / 16;
   // Four wavefronts.  Eight at 128 keys in fp16 (one query tile per wavefront, 128 registers, two workgroups per CU)
@@ -561,7 +565,7 @@ void attention_launch(const void* q, const void* k, const void* v, int layout, i
   dim3 grid((heads + hpw - 1) / hpw, batch);
   kern<<<grid, kThreads, Sm::kBytes, stream>>>((const T*)q, (const T*)k, (const T*)v, layout, packed_ld,
                                                    (const T*)attr_mask, (T*)dst, seq_start, word_idx, batch, seq_len,
-                                                   heads, hpw, scaler);
+                                                   heads, hpw, scaler, split_out ? 1 : 0);
 }
 
 
@@ -590,7 +594,7 @@ template <typename T, int NKT>
 __global__ __launch_bounds__(kAttnThreads) void attention_long_kernel(
     const T* __restrict__ q_src, const T* __restrict__ k_src, const T* __restrict__ v_src, int layout, int packed_ld,
     const T* __restrict__ attr_mask, T* __restrict__ dst, const int32_t* __restrict__ seq_start,
-    const int32_t* __restrict__ word_idx, int batch, int seq_len, int heads, float scaler) {
+    const int32_t* __restrict__ word_idx, int batch, int seq_len, int heads, float scaler, int split_out) {
   using Sm = LongSmem<T>;
   using C = Chunk16<T>;
   using V16 = typename C::vec;
@@ -846,7 +850,8 @@ __global__ __launch_bounds__(kAttnThreads) void attention_long_kernel(
         float4v v;
 #pragma unroll
         for (int r = 0; r < 4; ++r) v[r] = o[dt][r];
-        *reinterpret_cast<float4v*>(orow + dt * 16) = v;
+        if (split_out) store_split<4>(reinterpret_cast<uint16_t*>(dst) + (size_t)tq * 3 * H, head * kD + dt * 16 + g * 4, v);
+        else *reinterpret_cast<float4v*>(orow + dt * 16) = v;
       }
     }
   }
@@ -855,12 +860,13 @@ __global__ __launch_bounds__(kAttnThreads) void attention_long_kernel(
 template <typename T, int NKT>
 void attention_long_launch(const void* q, const void* k, const void* v, int layout, int packed_ld, const void* attr_mask,
                            void* dst, const int32_t* seq_start, const int32_t* word_idx, int batch, int seq_len, int heads,
-                           float scaler, hipStream_t stream) {
+                           float scaler, bool split_out, hipStream_t stream) {
   const size_t smem = LongSmem<T>::kTileBytes + (size_t)NKT * 16 * sizeof(int);
   auto kern = attention_long_kernel<T, NKT>;
   dim3 grid((seq_len + 63) / 64, heads, batch);               // blocks of 64 queries that can hold a token
   kern<<<grid, kAttnThreads, smem, stream>>>((const T*)q, (const T*)k, (const T*)v, layout, packed_ld, (const T*)attr_mask,
-                                             (T*)dst, seq_start, word_idx, batch, seq_len, heads, scaler);
+                                             (T*)dst, seq_start, word_idx, batch, seq_len, heads, scaler,
+                                             split_out ? 1 : 0);
 }
 
 // ------------------------------------------------------------------------------------------
@@ -1177,7 +1183,7 @@ template <typename T>
 __global__ __launch_bounds__(kSplitThreads) void attention_split_kernel(
     const T* __restrict__ q_src, const T* __restrict__ k_src, const T* __restrict__ v_src, int layout, int packed_ld,
     const T* __restrict__ attr_mask, T* __restrict__ dst, const int32_t* __restrict__ seq_start,
-    const int32_t* __restrict__ word_idx, int batch, int seq_len, int heads, float scaler) {
+    const int32_t* __restrict__ word_idx, int batch, int seq_len, int heads, float scaler, int split_out) {
   static_assert(sizeof(T) == 4, "fp32 only: fp16 beyond 512 positions runs attention_wide_kernel");
   using Sm = LongSmem<T>;
   using C = Chunk16<T>;
@@ -1408,7 +1414,8 @@ __global__ __launch_bounds__(kSplitThreads) void attention_split_kernel(
       float4v v;
 #pragma unroll
       for (int r = 0; r < 4; ++r) v[r] = o[dt][r];
-      *reinterpret_cast<float4v*>(orow + dt * 16) = v;
+      if (split_out) store_split<4>(reinterpret_cast<uint16_t*>(dst) + (size_t)tq * 3 * H, head * kD + dt * 16 + g * 4, v);
+      else *reinterpret_cast<float4v*>(orow + dt * 16) = v;
     }
   }
 }
@@ -1695,7 +1702,7 @@ __global__ __launch_bounds__(kSplitThreads) void attention_wide_kernel(
 template <typename T>
 void attention_split_launch(const void* q, const void* k, const void* v, int layout, int packed_ld, const void* attr_mask,
                             void* dst, const int32_t* seq_start, const int32_t* word_idx, int batch, int seq_len, int heads,
-                            float scaler, hipStream_t stream) {
+                            float scaler, bool split_out, hipStream_t stream) {
   dim3 grid((seq_len + 63) / 64, heads, batch);              // blocks of 64 queries that can hold a token
   if constexpr (sizeof(T) == 2) {
     allow_dynamic_lds(reinterpret_cast<const void*>(attention_wide_kernel), kWideSmem);
@@ -1708,7 +1715,7 @@ void attention_split_launch(const void* q, const void* k, const void* v, int lay
     allow_dynamic_lds(reinterpret_cast<const void*>(kern), (int)smem);
     kern<<<grid, kSplitThreads, smem, stream>>>((const T*)q, (const T*)k, (const T*)v, layout, packed_ld,
                                                 (const T*)attr_mask, (T*)dst, seq_start, word_idx, batch, seq_len, heads,
-                                                scaler);
+                                                scaler, split_out ? 1 : 0);
   }
 }
 
@@ -1854,13 +1861,13 @@ void attention_generic_launch(const void* q, const void* k, const void* v, int l
 template <typename T>
 void attention_dispatch(const void* q, const void* k, const void* v, int layout, int packed_ld, const void* attr_mask,
                         void* dst, const int32_t* seq_start, const int32_t* word_idx, int batch, int seq_len, int heads,
-                        int d, float scaler, hipStream_t stream) {
+                        int d, float scaler, bool split_out, hipStream_t stream) {
   if (d != kD || !head_rows_16b<T>(q, k, v, layout, packed_ld, d))
     attention_generic_launch<T>(q, k, v, layout, packed_ld, attr_mask, dst, seq_start, word_idx, batch, seq_len, heads, d,
                                 scaler, stream);
   else if (seq_len > 512)
     attention_split_launch<T>(q, k, v, layout, packed_ld, attr_mask, dst, seq_start, word_idx, batch, seq_len, heads,
-                              scaler, stream);
+                              scaler, split_out, stream);
   else if (sizeof(T) == 2 && seq_len > 384)
     attention_resident_launch<32>(q, k, v, layout, packed_ld, attr_mask, dst, seq_start, word_idx, batch, seq_len, heads,
                                   scaler, stream);
@@ -1872,19 +1879,19 @@ void attention_dispatch(const void* q, const void* k, const void* v, int layout,
                                   scaler, stream);
   else if (seq_len > 256)
     attention_long_launch<T, 32>(q, k, v, layout, packed_ld, attr_mask, dst, seq_start, word_idx, batch, seq_len, heads,
-                                 scaler, stream);
+                                 scaler, split_out, stream);
   else if (seq_len > 128)
     attention_long_launch<T, 16>(q, k, v, layout, packed_ld, attr_mask, dst, seq_start, word_idx, batch, seq_len, heads,
-                                 scaler, stream);
+                                 scaler, split_out, stream);
   else if (seq_len <= 32)
     attention_launch<T, 2>(q, k, v, layout, packed_ld, attr_mask, dst, seq_start, word_idx, batch, seq_len, heads,
-                           scaler, stream);
+                           scaler, split_out, stream);
   else if (seq_len <= 64)
     attention_launch<T, 4>(q, k, v, layout, packed_ld, attr_mask, dst, seq_start, word_idx, batch, seq_len, heads,
-                           scaler, stream);
+                           scaler, split_out, stream);
   else
     attention_launch<T, 8>(q, k, v, layout, packed_ld, attr_mask, dst, seq_start, word_idx, batch, seq_len, heads,
-                           scaler, stream);
+                           scaler, split_out, stream);
 }
 
 }  // namespace
@@ -1947,15 +1954,20 @@ bool attention_supported(DType t, int seq_len, int d) {
   return d >= 1 && d <= kGenMaxD && seq_len >= 1 && seq_len <= kGenMaxSeq;
 }
 
+bool attention_writes_split(const void* q, const void* k, const void* v, int layout, int packed_ld, int d) {
+  return d == kD && head_rows_16b<float>(q, k, v, layout, packed_ld, d);
+}
+
 void launch_attention(DType t, const void* q, const void* k, const void* v, int layout, int packed_ld,
                       const void* attr_mask, void* dst, const int32_t* seq_start, const int32_t* word_idx, int batch,
-                      int seq_len, int heads, int d, float scaler, hipStream_t stream) {
+                      int seq_len, int heads, int d, float scaler, hipStream_t stream,
+                      bool split_out) {
   if (t == DType::F32)
     attention_dispatch<float>(q, k, v, layout, packed_ld, attr_mask, dst, seq_start, word_idx, batch, seq_len, heads, d,
-                              scaler, stream);
+                              scaler, split_out, stream);
   else
     attention_dispatch<_Float16>(q, k, v, layout, packed_ld, attr_mask, dst, seq_start, word_idx, batch, seq_len,
-                                 heads, d, scaler, stream);
+                                 heads, d, scaler, false, stream);
 }
 
 }  // namespace et

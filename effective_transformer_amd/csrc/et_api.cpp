@@ -168,23 +168,31 @@ et_status check_launch(et_handle h, const char* what) {
 bool dtype_ok(et_dtype d) { return d == ET_FP32 || d == ET_FP16; }
 et::DType to_dt(et_dtype d) { return d == ET_FP32 ? et::DType::F32 : et::DType::F16; }
 
+// fp32 layers of these hidden sizes run their products on split rows (gemm_split.hip); the rest on the fp32 kernels
+bool layer_splits(et_dtype dtype, int H) { return dtype == ET_FP32 && H % 32 == 0 && et::gemm_split_supported(H, 4 * H); }
+
 struct LayerWs {
-  size_t qkv, ctx, attn, inter, seq, wt, total;
+  size_t qkv, ctx, attn, attn_split, inter, seq, wt, total;
 };
 
 LayerWs layer_ws(et_dtype dtype, int B, int S, int heads, int d) {
   const size_t e = dtype == ET_FP32 ? 4 : 2;
   const size_t rows = (size_t)B * S, H = (size_t)heads * d;
+  const bool split = layer_splits(dtype, heads * d);
+  const size_t ea = split ? 6 : e;               // bytes of a value that only a product reads
   LayerWs w;
   size_t off = 0;
   w.qkv = off;   off += align_up(rows * 3 * H * e, 256);
-  w.ctx = off;   off += align_up(rows * H * e, 256);
+  w.ctx = off;   off += align_up(rows * H * ea, 256);
   w.attn = off;  off += align_up(rows * H * e, 256);
-  // whole tiles of 256 rows: the FFN's intermediate may be handed over in blocks of [256 rows][64 columns]
-  w.inter = off; off += align_up(align_up(rows, 256) * 4 * H * e, 256);
+  w.attn_split = off; off += split ? align_up(rows * H * ea, 256) : 0;
+  // whole tiles of 256 rows: the FFN's intermediate may be handed over in blocks of [256 rows][64 columns].  The split
+  // rows of from_tensor and to_tensor lie here while the Q/K/V projections read them, those of the layer's output once
+  // the intermediate has been consumed.
+  w.inter = off; off += align_up(align_up(rows, 256) * 4 * H * ea, 256);
   w.seq = off;   off += align_up(et::seq_table_words(B) * sizeof(int32_t), 256);
-  // fp16: k-contiguous copies of the six dense kernels (3 H^2 + H^2 + 4 H^2 + 4 H^2 elements) for the large-M GEMM
-  w.wt = off;    off += dtype == ET_FP16 ? align_up(12 * H * H * e, 256) : 0;
+  // k-contiguous copies (fp32: split rows) of the six dense kernels (3 H^2 + H^2 + 4 H^2 + 4 H^2 elements)
+  w.wt = off;    off += dtype == ET_FP16 || split ? align_up(12 * H * H * ea, 256) : 0;
   w.total = off;
   return w;
 }
@@ -223,6 +231,205 @@ float softmax_scaler(et_dtype dtype, int d) {
   float s = 1.0f / sqrtf((float)d);
   if (dtype == ET_FP16) s = (float)(_Float16)s;   // the reference holds the scaler in the element type
   return s;
+}
+
+// What a layer asks of its arguments whoever calls it; the tensors and the entry are the caller's to check.
+et_status layer_args_ok(et_handle h, et_dtype dtype, const et_layer_weights* w, const et_layer_prepared* prep, int B, int S,
+                        int heads, int d) {
+  ET_REQUIRE(h, w != nullptr, "null weights");
+  ET_REQUIRE(h, w->attr_kernel_Q && w->attr_kernel_K && w->attr_kernel_V && w->attr_bias_Q && w->attr_bias_K &&
+                    w->attr_bias_V && w->attr_output_kernel && w->attr_output_bias && w->attr_output_layernorm_gamma &&
+                    w->attr_output_layernorm_beta && w->inter_kernel && w->inter_bias && w->output_kernel &&
+                    w->output_bias && w->output_layernorm_gamma && w->output_layernorm_beta,
+             "null weight pointer");
+  const int H = heads * d, F = 4 * H;
+  const et::DType dt = to_dt(dtype);
+  et_status s;
+  if ((s = batch_fits_grid(h, B)) != ET_OK) return s;
+  if (!et::attention_supported(dt, S, d))
+    return fail(h, ET_UNSUPPORTED, "attention needs size_per_head <= 256 and seq_len <= 1024");
+  if (!et::gemm_supported(dt, H, H, 3) || !et::gemm_supported(dt, F, H, 1) || !et::gemm_supported(dt, H, F, 1))
+    return fail(h, ET_UNSUPPORTED, "hidden size not supported by the GEMM kernels");
+  if ((uint64_t)B * S * F * et::elem_size(dt) > 0xffffffffull)
+    return fail(h, ET_UNSUPPORTED, "activation matrix larger than 4 GB");
+  if (!et::bias_gelu_supported(dt, F) || !et::bias_residual_layernorm_supported(dt, H))
+    return fail(h, ET_UNSUPPORTED, "hidden size not supported by the row kernels");
+  if (prep) {
+    if (prep->seq_start && prep->seq_start_bytes < et_seq_workspace_bytes(B))
+      return fail(h, ET_WORKSPACE_TOO_SMALL, "et_layer_prepared.seq_start needs et_seq_workspace_bytes(batch_size) bytes");
+    ET_REQUIRE(h, (prep->attr_kernel_Q_t != nullptr) == (prep->attr_kernel_K_t != nullptr) &&
+                      (prep->attr_kernel_Q_t != nullptr) == (prep->attr_kernel_V_t != nullptr),
+               "prepared Q, K and V kernels go together");
+  }
+  return ET_OK;
+}
+
+// One layer of a batch whose arguments have been checked: launches only.
+struct LayerCall {
+  et_dtype dtype;
+  const et_layer_weights* w;
+  const et_layer_prepared* prep;      // may be null
+  const void *from, *to, *attr_mask;
+  const int32_t *count, *batch_idx, *word_idx;
+  const int32_t* seq_start;           // the batch's sequence table, or null: built here
+  void* out;
+  int B, S, heads, d;
+  int rows;                           // launches are sized for this many rows
+  char* workspace;
+  bool from_split_ready = false;      // split layers: the split rows of `from` are in the workspace's intermediate already
+  bool write_out_split = false;       //   ... and those of `out` are to be left there
+  hipStream_t stream;
+};
+et_status run_layer(et_handle h, const LayerCall& c);
+
+et_status run_layer(et_handle h, const LayerCall& c) {
+  const et_layer_weights* w = c.w;
+  const int B = c.B, S = c.S, H = c.heads * c.d, F = 4 * H, rows = c.rows;
+  const LayerWs ws = layer_ws(c.dtype, B, S, c.heads, c.d);
+  const et::DType dt = to_dt(c.dtype);
+  const int32_t* T = c.count;
+  hipStream_t st = c.stream;
+  et_status s;
+  const size_t e = et::elem_size(dt);
+  const bool split = layer_splits(c.dtype, H);
+  char* base = c.workspace;
+  void* qkv = base + ws.qkv;
+  void* ctx = base + ws.ctx;
+  void* attn = base + ws.attn;
+  void* inter = base + ws.inter;
+  const int32_t* seq_start = c.seq_start ? c.seq_start : (int32_t*)(base + ws.seq);
+
+  // The large-M fp16 GEMM reads k-contiguous weights with fewer LDS instructions.  Where the caller prepared such
+  // copies they are used wherever that kernel runs; otherwise the wide projections get a transposed copy in the
+  // workspace on every call (the caller's weights stay as they are).
+  static const et_layer_prepared kNoPrep = {nullptr, nullptr, nullptr, nullptr, nullptr, nullptr, nullptr, nullptr, 0, 0};
+  const et_layer_prepared& pp = c.prep ? *c.prep : kNoPrep;
+  const bool can_qkv = et::gemm_takes_transposed_b(dt, rows, 3 * H, H, H, 3);
+  const bool can_o = et::gemm_takes_transposed_b(dt, rows, H, H, H, 1);
+  const bool can_up = et::gemm_takes_transposed_b(dt, rows, F, F, H, 1);
+  const bool can_down = et::gemm_takes_transposed_b(dt, rows, H, H, F, 1);
+  // (the split products take their weights as split copies only)
+  const bool t_qkv = split || (can_qkv && (pp.attr_kernel_Q_t || et::gemm_prefers_transposed_b(dt, rows, 3 * H, H, H, 3)));
+  const bool t_o = split || (can_o && (pp.attr_output_kernel_t || et::gemm_prefers_transposed_b(dt, rows, H, H, H, 1)));
+  const bool t_up = split || (can_up && (pp.inter_kernel_t || et::gemm_prefers_transposed_b(dt, rows, F, F, H, 1)));
+  const bool t_down = split || (can_down && (pp.output_kernel_t || et::gemm_prefers_transposed_b(dt, rows, H, H, F, 1)));
+  char* wt = base + ws.wt;
+  const size_t HH = (size_t)H * H * (split ? 6 : e);
+  const void* wt_q = wt; const void* wt_k = wt + HH; const void* wt_v = wt + 2 * HH; const void* wt_o = wt + 3 * HH;
+  const void* wt_up = wt + 4 * HH; const void* wt_down = wt + 8 * HH;
+  {
+    et::TransposeJobs jobs;
+    if (t_qkv && pp.attr_kernel_Q_t) {
+      wt_q = pp.attr_kernel_Q_t; wt_k = pp.attr_kernel_K_t; wt_v = pp.attr_kernel_V_t;
+    } else if (t_qkv) {
+      jobs.add(w->attr_kernel_Q, wt, H, H);
+      jobs.add(w->attr_kernel_K, wt + HH, H, H);
+      jobs.add(w->attr_kernel_V, wt + 2 * HH, H, H);
+    }
+    if (t_o && pp.attr_output_kernel_t) wt_o = pp.attr_output_kernel_t;
+    else if (t_o) jobs.add(w->attr_output_kernel, wt + 3 * HH, H, H);
+    if (t_up && pp.inter_kernel_t) wt_up = pp.inter_kernel_t;
+    else if (t_up) jobs.add(w->inter_kernel, wt + 4 * HH, H, F);
+    if (t_down && pp.output_kernel_t) wt_down = pp.output_kernel_t;
+    else if (t_down) jobs.add(w->output_kernel, wt + 8 * HH, F, H);
+    // one launch builds the sequence start table and the transposed copies; none when the caller prepared both
+    const et::SeqStartJob seq{c.batch_idx, T, rows, B, (int32_t*)(base + ws.seq)};
+    if (split) {
+      et::launch_split_weights(jobs, st);
+      jobs.count = 0;
+    }
+    et::launch_transpose_weights(jobs, st, c.seq_start ? nullptr : &seq);
+  }
+  // split rows of the two inputs, in the room of the intermediate, which nothing needs before they have been read
+  const void *from_a = c.from, *to_a = c.to;
+  if (split) {
+    uint16_t* fs = (uint16_t*)inter;
+    if (!c.from_split_ready) et::launch_split_rows((const float*)c.from, fs, rows, H, T, st);
+    from_a = to_a = fs;
+    if (c.to != c.from) {
+      uint16_t* ts = fs + (size_t)rows * 3 * H;
+      et::launch_split_rows((const float*)c.to, ts, rows, H, T, st);
+      to_a = ts;
+    }
+  }
+  auto gemm = [&](const et::GemmGroups& g, void* C, int ldc, int n, int k) {
+    if (split) et::launch_gemm_split(g, C, ldc, rows, n, k, T, st);
+    else et::launch_gemm(dt, g, C, ldc, rows, n, k, T, st);
+  };
+  // Every matrix of the layer is read again by the kernel after the one that wrote it.  While the layer's matrices
+  // (from, Q/K/V, context, attention output, [T,4H], out) about fit the last-level cache, the GEMMs leave their
+  // outputs there (plain stores); beyond that the outputs would only displace the weights and the A rows.
+  const bool cached = (double)rows * (7.0 * H + F) * (double)e <= kCachedLayerBytes;
+  // Q = from.Wq + bq, K = to.Wk + bk, V = to.Wv + bv into one [T,3H] buffer (bert_transformer_op.cu.cc:105-156)
+  et::GemmGroups g3;
+  g3.groups = 3;
+  g3.c_cached = cached;
+  g3.A[0] = from_a; g3.A[1] = to_a; g3.A[2] = to_a;
+  g3.B[0] = t_qkv ? wt_q : w->attr_kernel_Q; g3.B[1] = t_qkv ? wt_k : w->attr_kernel_K; g3.B[2] = t_qkv ? wt_v : w->attr_kernel_V;
+  g3.bias[0] = w->attr_bias_Q; g3.bias[1] = w->attr_bias_K; g3.bias[2] = w->attr_bias_V;
+  g3.b_transposed = t_qkv;
+  gemm(g3, qkv, 3 * H, H, H);
+  if ((s = check_launch(h, "QKV projection")) != ET_OK) return s;
+  // QK^T, softmax, PV, un-pad (:159-192)
+  const char *q = (const char*)qkv, *k = q + (size_t)H * e, *v = k + (size_t)H * e;
+  const bool ctx_split = split && et::attention_writes_split(q, k, v, 1, 3 * H, c.d);
+  // (where the attention kernel writes floats only, they take the attention output's place until they are split)
+  et::launch_attention(dt, q, k, v, 1, 3 * H, c.attr_mask, split && !ctx_split ? attn : ctx, seq_start, c.word_idx, B, S,
+                       c.heads, c.d, softmax_scaler(c.dtype, c.d), st, ctx_split);
+  if (split && !ctx_split) et::launch_split_rows((const float*)attn, (uint16_t*)ctx, rows, H, T, st);
+  if ((s = check_launch(h, "attention")) != ET_OK) return s;
+  // attention output projection + bias + residual(from_tensor) + LayerNorm (:195-213)
+  et::GemmGroups g1;
+  g1.groups = 1;
+  g1.c_cached = cached;
+  g1.A[0] = ctx; g1.B[0] = t_o ? wt_o : w->attr_output_kernel; g1.bias[0] = nullptr;
+  g1.b_transposed = t_o;
+  gemm(g1, attn, H, H, H);
+  // Every weight matrix was last read a whole batch ago, and a GEMM's first round of tiles waits for each cold slice of
+  // it (13000 rows: FFN-down 63 us with cold weights, 53 with the weights in the last-level cache; 2 .. 3 us for the
+  // other projections).  The two LayerNorm kernels request the matrices that come next on their way, for batches in
+  // which those are small beside what the kernel moves anyway: this one the FFN-up weights and, while the layer's
+  // matrices are small enough for them to survive FFN-up, the FFN-down weights (12-layer BERT-base: -3 % at 4000
+  // tokens, -4.4 % at 8000 and 12000, -1 % at 16000); the last one the region the caller names, the next layer's
+  // attention weights (another -0.7 .. -1.6 % from 4000 to 40000 tokens, FFN-up included).
+  const bool warm_fits = (double)rows * (7.0 * H + F) * (double)e <= kWarmLayerBytes;
+  et::WarmList warm1, warm2;
+  // (whichever copy the GEMM reads, unless this call has just written it)
+  const void* b_up = t_up ? wt_up : w->inter_kernel;
+  const void* b_down = t_down ? wt_down : w->output_kernel;
+  if (rows >= F && !(t_up && !pp.inter_kernel_t)) warm1.add(b_up, (size_t)H * F * (split ? 6 : e));
+  if (rows >= F && warm_fits && !(t_down && !pp.output_kernel_t)) warm1.add(b_down, (size_t)H * F * (split ? 6 : e));
+  if (rows >= F) warm2.add(pp.warm, pp.warm_bytes);
+  // (split layers: the row kernel leaves its output as split rows too; rows it cannot hold in registers take a pass)
+  const bool ln_split = split && et::layernorm_row_in_registers(dt, H);
+  uint16_t* attn_split = (uint16_t*)(base + ws.attn_split);
+  et::launch_bias_residual_layernorm(dt, attn, c.from, w->attr_output_bias, w->attr_output_layernorm_gamma,
+                                     w->attr_output_layernorm_beta, rows, H, T, st, warm1, ln_split ? attn_split : nullptr);
+  if (split && !ln_split) et::launch_split_rows((const float*)attn, attn_split, rows, H, T, st);
+  if ((s = check_launch(h, "attention output")) != ET_OK) return s;
+  // FFN up + bias + GELU (:215-227, cuda/cuda_kernels.cu:88-150)
+  g1.A[0] = split ? (const void*)attn_split : attn; g1.B[0] = t_up ? wt_up : w->inter_kernel;
+  g1.b_transposed = t_up;
+  // bias + GELU are applied to each tile on its way out of the GEMM: no pass of its own over [T,4H]
+  g1.bias[0] = w->inter_bias; g1.gelu = true;
+  // where both FFN projections run the persistent k-contiguous kernel, [T,4H] goes from one to the other in blocks
+  const bool blocked = t_up && t_down && et::gemm_blocked_handover(dt, rows, F, H);
+  g1.c_blocked = blocked;
+  gemm(g1, inter, F, F, H);
+  g1.bias[0] = nullptr; g1.gelu = false; g1.c_blocked = false;
+  if ((s = check_launch(h, "FFN up")) != ET_OK) return s;
+  // FFN down + bias + residual(LN1 output) + LayerNorm (:229-247)
+  g1.A[0] = inter; g1.B[0] = t_down ? wt_down : w->output_kernel;
+  g1.b_transposed = t_down;
+  g1.a_blocked = blocked;
+  gemm(g1, c.out, H, H, F);
+  g1.a_blocked = false;
+  uint16_t* out_split = split && c.write_out_split ? (uint16_t*)inter : nullptr;
+  et::launch_bias_residual_layernorm(dt, c.out, attn, w->output_bias, w->output_layernorm_gamma,
+                                     w->output_layernorm_beta, rows, H, T, st, warm2, ln_split ? out_split : nullptr);
+  if (out_split && !ln_split) et::launch_split_rows((const float*)c.out, out_split, rows, H, T, st);
+  if ((s = check_launch(h, "FFN down")) != ET_OK) return s;
+  return ET_OK;
 }
 
 }  // namespace
@@ -459,148 +666,27 @@ et_status et_layer_with_prepared(et_handle h, et_dtype dtype, const et_layer_wei
   ET_REQUIRE(h, dtype_ok(dtype), "dtype must be ET_FP32 or ET_FP16");
   if ((s = dims_ok(h, batch_size, from_seq_len, head_num, size_per_head)) != ET_OK) return s;
   ET_REQUIRE(h, from_seq_len == to_seq_len, "only support from_seq_len == to_seq_len");
-  ET_REQUIRE(h, w != nullptr, "null weights");
-  ET_REQUIRE(h, w->attr_kernel_Q && w->attr_kernel_K && w->attr_kernel_V && w->attr_bias_Q && w->attr_bias_K &&
-                    w->attr_bias_V && w->attr_output_kernel && w->attr_output_bias && w->attr_output_layernorm_gamma &&
-                    w->attr_output_layernorm_beta && w->inter_kernel && w->inter_bias && w->output_kernel &&
-                    w->output_bias && w->output_layernorm_gamma && w->output_layernorm_beta,
-             "null weight pointer");
   ET_REQUIRE(h, from_tensor && to_tensor && attr_mask && valid_word_num_dev && batch_idx && word_idx && out,
              "null tensor pointer");
   ET_REQUIRE(h, out != from_tensor && out != to_tensor, "out must not alias from_tensor / to_tensor");
   ET_REQUIRE(h, workspace != nullptr, "null workspace");
-  const int B = batch_size, S = from_seq_len, H = head_num * size_per_head, F = 4 * H;
+  const int B = batch_size, S = from_seq_len;
   ET_REQUIRE(h, valid_word_num_hint >= -1 && valid_word_num_hint <= B * S, "valid_word_num_hint out of range");
-  const LayerWs ws = layer_ws(dtype, B, S, head_num, size_per_head);
-  if (workspace_bytes < ws.total) return fail(h, ET_WORKSPACE_TOO_SMALL, "et_layer needs et_layer_workspace_bytes(...)");
-  const et::DType dt = to_dt(dtype);
-  if ((s = batch_fits_grid(h, B)) != ET_OK) return s;
-  if (!et::attention_supported(dt, S, size_per_head))
-    return fail(h, ET_UNSUPPORTED, "attention needs size_per_head <= 256 and seq_len <= 1024");
-  if (!et::gemm_supported(dt, H, H, 3) || !et::gemm_supported(dt, F, H, 1) || !et::gemm_supported(dt, H, F, 1))
-    return fail(h, ET_UNSUPPORTED, "hidden size not supported by the GEMM kernels");
-  if ((uint64_t)B * S * F * et::elem_size(dt) > 0xffffffffull)
-    return fail(h, ET_UNSUPPORTED, "activation matrix larger than 4 GB");
-  if (!et::bias_gelu_supported(dt, F) || !et::bias_residual_layernorm_supported(dt, H))
-    return fail(h, ET_UNSUPPORTED, "hidden size not supported by the row kernels");
+  if (workspace_bytes < layer_ws(dtype, B, S, head_num, size_per_head).total)
+    return fail(h, ET_WORKSPACE_TOO_SMALL, "et_layer needs et_layer_workspace_bytes(...)");
+  if ((s = layer_args_ok(h, dtype, w, prep, B, S, head_num, size_per_head)) != ET_OK) return s;
   if (valid_word_num_hint == 0) return ET_OK;
-  const int rows = valid_word_num_hint > 0 ? valid_word_num_hint : B * S;
-  const int32_t* T = valid_word_num_dev;
-  hipStream_t st = (hipStream_t)stream;
-  const size_t e = et::elem_size(dt);
-  char* base = (char*)workspace;
-  void* qkv = base + ws.qkv;
-  void* ctx = base + ws.ctx;
-  void* attn = base + ws.attn;
-  void* inter = base + ws.inter;
-  int32_t* seq_start = (int32_t*)(base + ws.seq);
-
-  // The large-M fp16 GEMM reads k-contiguous weights with fewer LDS instructions.  Where the caller prepared such
-  // copies they are used wherever that kernel runs; otherwise the wide projections get a transposed copy in the
-  // workspace on every call (the caller's weights stay as they are).
-  static const et_layer_prepared kNoPrep = {nullptr, nullptr, nullptr, nullptr, nullptr, nullptr, nullptr, nullptr, 0, 0};
-  const et_layer_prepared& pp = prep ? *prep : kNoPrep;
-  if (pp.seq_start && pp.seq_start_bytes < et_seq_workspace_bytes(B))
-    return fail(h, ET_WORKSPACE_TOO_SMALL, "et_layer_prepared.seq_start needs et_seq_workspace_bytes(batch_size) bytes");
-  ET_REQUIRE(h, (pp.attr_kernel_Q_t != nullptr) == (pp.attr_kernel_K_t != nullptr) &&
-                    (pp.attr_kernel_Q_t != nullptr) == (pp.attr_kernel_V_t != nullptr),
-             "prepared Q, K and V kernels go together");
-  const bool can_qkv = et::gemm_takes_transposed_b(dt, rows, 3 * H, H, H, 3);
-  const bool can_o = et::gemm_takes_transposed_b(dt, rows, H, H, H, 1);
-  const bool can_up = et::gemm_takes_transposed_b(dt, rows, F, F, H, 1);
-  const bool can_down = et::gemm_takes_transposed_b(dt, rows, H, H, F, 1);
-  const bool t_qkv = can_qkv && (pp.attr_kernel_Q_t || et::gemm_prefers_transposed_b(dt, rows, 3 * H, H, H, 3));
-  const bool t_o = can_o && (pp.attr_output_kernel_t || et::gemm_prefers_transposed_b(dt, rows, H, H, H, 1));
-  const bool t_up = can_up && (pp.inter_kernel_t || et::gemm_prefers_transposed_b(dt, rows, F, F, H, 1));
-  const bool t_down = can_down && (pp.output_kernel_t || et::gemm_prefers_transposed_b(dt, rows, H, H, F, 1));
-  char* wt = base + ws.wt;
-  const size_t HH = (size_t)H * H * e;
-  const void* wt_q = wt; const void* wt_k = wt + HH; const void* wt_v = wt + 2 * HH; const void* wt_o = wt + 3 * HH;
-  const void* wt_up = wt + 4 * HH; const void* wt_down = wt + 8 * HH;
-  {
-    et::TransposeJobs jobs;
-    if (t_qkv && pp.attr_kernel_Q_t) {
-      wt_q = pp.attr_kernel_Q_t; wt_k = pp.attr_kernel_K_t; wt_v = pp.attr_kernel_V_t;
-    } else if (t_qkv) {
-      jobs.add(w->attr_kernel_Q, wt, H, H);
-      jobs.add(w->attr_kernel_K, wt + HH, H, H);
-      jobs.add(w->attr_kernel_V, wt + 2 * HH, H, H);
-    }
-    if (t_o && pp.attr_output_kernel_t) wt_o = pp.attr_output_kernel_t;
-    else if (t_o) jobs.add(w->attr_output_kernel, wt + 3 * HH, H, H);
-    if (t_up && pp.inter_kernel_t) wt_up = pp.inter_kernel_t;
-    else if (t_up) jobs.add(w->inter_kernel, wt + 4 * HH, H, F);
-    if (t_down && pp.output_kernel_t) wt_down = pp.output_kernel_t;
-    else if (t_down) jobs.add(w->output_kernel, wt + 8 * HH, F, H);
-    // one launch builds the sequence start table and the transposed copies; none when the caller prepared both
-    const et::SeqStartJob seq{batch_idx, T, rows, B, seq_start};
-    if (pp.seq_start) seq_start = const_cast<int32_t*>(pp.seq_start);
-    et::launch_transpose_weights(jobs, st, pp.seq_start ? nullptr : &seq);
-  }
-  // Every matrix of the layer is read again by the kernel after the one that wrote it.  While the layer's matrices
-  // (from, Q/K/V, context, attention output, [T,4H], out) about fit the last-level cache, the GEMMs leave their
-  // outputs there (plain stores); beyond that the outputs would only displace the weights and the A rows.
-  const bool cached = (double)rows * (7.0 * H + F) * (double)e <= kCachedLayerBytes;
-  // Q = from.Wq + bq, K = to.Wk + bk, V = to.Wv + bv into one [T,3H] buffer (bert_transformer_op.cu.cc:105-156)
-  et::GemmGroups g3;
-  g3.groups = 3;
-  g3.c_cached = cached;
-  g3.A[0] = from_tensor; g3.A[1] = to_tensor; g3.A[2] = to_tensor;
-  g3.B[0] = t_qkv ? wt_q : w->attr_kernel_Q; g3.B[1] = t_qkv ? wt_k : w->attr_kernel_K; g3.B[2] = t_qkv ? wt_v : w->attr_kernel_V;
-  g3.bias[0] = w->attr_bias_Q; g3.bias[1] = w->attr_bias_K; g3.bias[2] = w->attr_bias_V;
-  g3.b_transposed = t_qkv;
-  et::launch_gemm(dt, g3, qkv, 3 * H, rows, H, H, T, st);
-  if ((s = check_launch(h, "QKV projection")) != ET_OK) return s;
-  // QK^T, softmax, PV, un-pad (:159-192)
-  et::launch_attention(dt, qkv, (char*)qkv + (size_t)H * e, (char*)qkv + (size_t)2 * H * e, 1, 3 * H, attr_mask, ctx,
-                       seq_start, word_idx, B, S, head_num, size_per_head, softmax_scaler(dtype, size_per_head), st);
-  if ((s = check_launch(h, "attention")) != ET_OK) return s;
-  // attention output projection + bias + residual(from_tensor) + LayerNorm (:195-213)
-  et::GemmGroups g1;
-  g1.groups = 1;
-  g1.c_cached = cached;
-  g1.A[0] = ctx; g1.B[0] = t_o ? wt_o : w->attr_output_kernel; g1.bias[0] = nullptr;
-  g1.b_transposed = t_o;
-  et::launch_gemm(dt, g1, attn, H, rows, H, H, T, st);
-  // Every weight matrix was last read a whole batch ago, and a GEMM's first round of tiles waits for each cold slice of
-  // it (13000 rows: FFN-down 63 us with cold weights, 53 with the weights in the last-level cache; 2 .. 3 us for the
-  // other projections).  The two LayerNorm kernels request the matrices that come next on their way, for batches in
-  // which those are small beside what the kernel moves anyway: this one the FFN-up weights and, while the layer's
-  // matrices are small enough for them to survive FFN-up, the FFN-down weights (12-layer BERT-base: -3 % at 4000
-  // tokens, -4.4 % at 8000 and 12000, -1 % at 16000); the last one the region the caller names, the next layer's
-  // attention weights (another -0.7 .. -1.6 % from 4000 to 40000 tokens, FFN-up included).
-  const bool warm_fits = (double)rows * (7.0 * H + F) * (double)e <= kWarmLayerBytes;
-  et::WarmList warm1, warm2;
-  // (whichever copy the GEMM reads, unless this call has just written it)
-  const void* b_up = t_up ? wt_up : w->inter_kernel;
-  const void* b_down = t_down ? wt_down : w->output_kernel;
-  if (rows >= F && !(t_up && !pp.inter_kernel_t)) warm1.add(b_up, (size_t)H * F * e);
-  if (rows >= F && warm_fits && !(t_down && !pp.output_kernel_t)) warm1.add(b_down, (size_t)H * F * e);
-  if (rows >= F) warm2.add(pp.warm, pp.warm_bytes);
-  et::launch_bias_residual_layernorm(dt, attn, from_tensor, w->attr_output_bias, w->attr_output_layernorm_gamma,
-                                     w->attr_output_layernorm_beta, rows, H, T, st, warm1);
-  if ((s = check_launch(h, "attention output")) != ET_OK) return s;
-  // FFN up + bias + GELU (:215-227, cuda/cuda_kernels.cu:88-150)
-  g1.A[0] = attn; g1.B[0] = t_up ? wt_up : w->inter_kernel;
-  g1.b_transposed = t_up;
-  // bias + GELU are applied to each tile on its way out of the GEMM: no pass of its own over [T,4H]
-  g1.bias[0] = w->inter_bias; g1.gelu = true;
-  // where both FFN projections run the persistent k-contiguous kernel, [T,4H] goes from one to the other in blocks
-  const bool blocked = t_up && t_down && et::gemm_blocked_handover(dt, rows, F, H);
-  g1.c_blocked = blocked;
-  et::launch_gemm(dt, g1, inter, F, rows, F, H, T, st);
-  g1.bias[0] = nullptr; g1.gelu = false; g1.c_blocked = false;
-  if ((s = check_launch(h, "FFN up")) != ET_OK) return s;
-  // FFN down + bias + residual(LN1 output) + LayerNorm (:229-247)
-  g1.A[0] = inter; g1.B[0] = t_down ? wt_down : w->output_kernel;
-  g1.b_transposed = t_down;
-  g1.a_blocked = blocked;
-  et::launch_gemm(dt, g1, out, H, rows, H, F, T, st);
-  g1.a_blocked = false;
-  et::launch_bias_residual_layernorm(dt, out, attn, w->output_bias, w->output_layernorm_gamma,
-                                     w->output_layernorm_beta, rows, H, T, st, warm2);
-  if ((s = check_launch(h, "FFN down")) != ET_OK) return s;
-  return ET_OK;
+  LayerCall c;
+  c.dtype = dtype; c.w = w; c.prep = prep;
+  c.from = from_tensor; c.to = to_tensor; c.attr_mask = attr_mask;
+  c.count = valid_word_num_dev; c.batch_idx = batch_idx; c.word_idx = word_idx;
+  c.seq_start = prep ? prep->seq_start : nullptr;
+  c.out = out;
+  c.B = B; c.S = S; c.heads = head_num; c.d = size_per_head;
+  c.rows = valid_word_num_hint > 0 ? valid_word_num_hint : B * S;
+  c.workspace = (char*)workspace;
+  c.stream = (hipStream_t)stream;
+  return run_layer(h, c);
 }
 
 et_status et_output(et_handle h, et_dtype dtype, const void* from_tensor, const int32_t* valid_word_num_dev,
@@ -842,13 +928,48 @@ et_status et_transpose_weight(et_handle h, et_dtype dtype, const void* src, void
   Entry entry(h);
   et_status s = entry.status;
   if (s != ET_OK) return s;
-  ET_REQUIRE(h, dtype == ET_FP16, "dtype must be ET_FP16");
+  ET_REQUIRE(h, dtype_ok(dtype), "dtype must be ET_FP32 or ET_FP16");
   ET_REQUIRE(h, src && dst && src != dst, "null or aliased tensor pointer");
-  ET_REQUIRE(h, k >= 1 && n >= 1 && k % 8 == 0 && n % 8 == 0, "k and n must be positive multiples of 8");
   et::TransposeJobs jobs;
+  if (dtype == ET_FP32) {
+    ET_REQUIRE(h, k >= 1 && n >= 1 && et::gemm_split_supported(n, k), "k must be a multiple of 32 and n of 4");
+    jobs.add(src, dst, k, n);
+    et::launch_split_weights(jobs, (hipStream_t)stream);
+    return check_launch(h, "weight split");
+  }
+  ET_REQUIRE(h, k >= 1 && n >= 1 && k % 8 == 0 && n % 8 == 0, "k and n must be positive multiples of 8");
   jobs.add(src, dst, k, n);
   et::launch_transpose_weights(jobs, (hipStream_t)stream);
   return check_launch(h, "weight transpose");
+}
+
+et_status et_split_rows(et_handle h, const void* src, void* dst, int m, int k, const int32_t* m_dev, void* stream) {
+  Entry entry(h);
+  et_status s = entry.status;
+  if (s != ET_OK) return s;
+  ET_REQUIRE(h, src && dst && src != dst, "null or aliased tensor pointer");
+  ET_REQUIRE(h, m >= 0 && k >= 1 && k % 32 == 0, "k must be a positive multiple of 32");
+  if ((uint64_t)m * k / 8 >= 0x80000000ull) return fail(h, ET_UNSUPPORTED, "tensor too large for one launch");
+  et::launch_split_rows((const float*)src, (uint16_t*)dst, m, k, m_dev, (hipStream_t)stream);
+  return check_launch(h, "split rows");
+}
+
+et_status et_gemm_split(et_handle h, const void* A, const void* Bt, void* C, const void* bias, int gelu, int m, int n,
+                        int k, const int32_t* m_dev, void* stream) {
+  Entry entry(h);
+  et_status s = entry.status;
+  if (s != ET_OK) return s;
+  ET_REQUIRE(h, A && Bt && C, "null tensor pointer");
+  ET_REQUIRE(h, !gelu || bias, "null bias");
+  ET_REQUIRE(h, m >= 0 && n >= 1 && k >= 1, "bad dimensions");
+  if (!et::gemm_split_supported(n, k) || (gelu && n % 32 != 0))
+    return fail(h, ET_UNSUPPORTED, "et_gemm_split needs k % 32 == 0 and n % 4 == 0 (with gelu n % 32 == 0)");
+  et::GemmGroups g;
+  g.groups = 1;
+  g.A[0] = A; g.B[0] = Bt; g.bias[0] = bias;
+  g.gelu = gelu != 0;
+  et::launch_gemm_split(g, C, n, m, n, k, m_dev, (hipStream_t)stream);
+  return check_launch(h, "et_gemm_split");
 }
 
 namespace {

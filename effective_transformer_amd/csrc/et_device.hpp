@@ -135,6 +135,39 @@ __device__ __forceinline__ HV bias_gelu_half(HV v, HV bias) {
   return x * cdf;
 }
 
+// ---- split floats ------------------------------------------------------------------------
+// x = h + m + l exactly, three bfloat16 pieces, each the rest of the ones before it rounded to nearest (8 significand
+// bits and a sign apiece cover the 24 bits of a float).  Two values at a time, packed.  Infinities, NaNs and magnitudes
+// that round to a bfloat16 infinity (above 3.38e38) give NaN pieces.
+typedef __bf16 bf16x2 __attribute__((ext_vector_type(2)));
+__device__ __forceinline__ uint32_t round_pair_bf16(float& x0, float& x1) {      // returns the pieces, leaves the rests
+  const float2v v = {x0, x1};
+  const uint32_t p = __builtin_bit_cast(uint32_t, __builtin_convertvector(v, bf16x2));
+  x0 -= __builtin_bit_cast(float, p << 16);
+  x1 -= __builtin_bit_cast(float, p & 0xffff0000u);
+  return p;
+}
+// N consecutive values (N = 1, 2, 4 or 8; col a multiple of N) of a split row: [k / 32][h, m, l][32] bfloat16
+template <int N, typename V>
+__device__ __forceinline__ void store_split(uint16_t* row, int col, const V& v) {
+  constexpr int W = (N + 1) / 2;
+  uint16_t* p = row + (col >> 5) * 96 + (col & 31);
+  float x[2 * W];
+#pragma unroll
+  for (int j = 0; j < 2 * W; ++j) x[j] = j < N ? v[j < N ? j : 0] : 0.f;
+#pragma unroll
+  for (int piece = 0; piece < 3; ++piece) {
+    uint32_t w[W];
+#pragma unroll
+    for (int j = 0; j < W; ++j) w[j] = round_pair_bf16(x[2 * j], x[2 * j + 1]);
+    uint16_t* d = p + piece * 32;
+    if constexpr (N == 1) *d = (uint16_t)w[0];
+    else if constexpr (N == 2) *reinterpret_cast<uint32_t*>(d) = w[0];
+    else if constexpr (N == 4) *reinterpret_cast<u32x2*>(d) = u32x2{w[0], w[1]};
+    else *reinterpret_cast<u32x4*>(d) = u32x4{w[0], w[1], w[2], w[3]};
+  }
+}
+
 // seq_start[b] = first packed row of sequence b (b in [0, batch]; seq_start[batch] = T), written by the thread that
 // owns packed row t in [0, T]: it covers the sequences that begin at t (token-less sequences included).
 __device__ __forceinline__ void seq_start_for_row(const int32_t* __restrict__ batch_idx, int T, int t, int batch,

@@ -69,7 +69,9 @@ struct WarmList {
 };
 void launch_bias_residual_layernorm(DType t, void* out, const void* input, const void* bias,
                                     const void* gamma, const void* beta, int m, int n,
-                                    const int32_t* rows_dev, hipStream_t stream, const WarmList& warm = WarmList());
+                                    const int32_t* rows_dev, hipStream_t stream, const WarmList& warm = WarmList(),
+                                    uint16_t* split = nullptr);
+// split (fp32, rows in registers, n % 32 == 0): the output rows once more as split rows (see gemm_split.hip)
 
 // out[t,:] = LayerNorm(word[ids[p]] + type[type_ids[p]] + pos[word_idx[t]]) * gamma + beta for packed row t at padded
 // position p = batch_idx[t]*seq_len + word_idx[t]; eps 1e-12.  type_ids/type_table and pos_table may be null.
@@ -93,7 +95,10 @@ bool attention_supported(DType t, int seq_len, int d);
 // layout 0: padded [B,heads,S,d]; layout 1: packed rows with leading dimension packed_ld.
 void launch_attention(DType t, const void* q, const void* k, const void* v, int layout, int packed_ld,
                       const void* attr_mask, void* dst, const int32_t* seq_start, const int32_t* word_idx,
-                      int batch, int seq_len, int heads, int d, float scaler, hipStream_t stream);
+                      int batch, int seq_len, int heads, int d, float scaler, hipStream_t stream,
+                      bool split_out = false);
+// split_out (fp32): dst gets split rows (see gemm_split.hip) instead of float rows; only where this says so
+bool attention_writes_split(const void* q, const void* k, const void* v, int layout, int packed_ld, int d);
 
 // ---- gemm.hip ----------------------------------------------------------------------------
 // Up to three independent column groups share one launch (the Q/K/V projections): group g
@@ -152,6 +157,16 @@ struct SeqStartJob {
 void launch_transpose_weights(const TransposeJobs& jobs, hipStream_t stream, const SeqStartJob* seq = nullptr);
 void launch_gemm(DType t, const GemmGroups& g, void* C, int ldc, int m_bound, int n, int k,
                  const int32_t* rows_dev, hipStream_t stream);
+
+// ---- gemm_split.hip: fp32 products on the 16-bit matrix cores -----------------------------------------------------
+// Operands as split rows (6 k bytes per row, see gemm_split.hip): A [m], B [n] (k-contiguous weights).
+// C is float [m][ldc] (+ bias), or with g.gelu the split rows of gelu(A.B + bias) (3 ldc bfloat16 per row).
+bool gemm_split_supported(int n, int k);
+// float [m][k] -> split rows; float weights [k][n] -> n split rows (k a multiple of 32, n of 4), one launch for all jobs
+void launch_split_rows(const float* src, uint16_t* dst, int m, int k, const int32_t* rows_dev, hipStream_t stream);
+void launch_split_weights(const TransposeJobs& jobs, hipStream_t stream);
+void launch_gemm_split(const GemmGroups& g, void* C, int ldc, int m_bound, int n, int k, const int32_t* rows_dev,
+                       hipStream_t stream);
 
 // ---- generic.hip: element-wise kernels for the shapes the tuned kernels do not take ------------------------------
 // (rows or head rows that are no whole number of 16-byte pieces, GEMM k / n the MFMA tiles cannot take); the launchers

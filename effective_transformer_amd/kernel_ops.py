@@ -117,10 +117,11 @@ def gemm(a, b, bias=None, m: Optional[int] = None, m_dev: Optional[torch.Tensor]
 
 
 def transpose_weight(w, out: Optional[torch.Tensor] = None):
-    """[k, n] -> [n, k] (fp16), the layout gemm_bt takes."""
+    """[k, n] -> [n, k] (fp16), the layout gemm_bt takes; fp32: -> n split rows [n, 3 k] bfloat16, what gemm_split takes."""
     k, n = w.shape
     if out is None:
-        out = torch.empty(n, k, dtype=w.dtype, device=w.device)
+        out = torch.empty(n, k, dtype=w.dtype, device=w.device) if w.dtype == torch.float16 else \
+            torch.empty(n, 3 * k, dtype=torch.bfloat16, device=w.device)
     _call("et_transpose_weight", w.device, _dtype_code(w.dtype), _p(w), _p(out), k, n, _stream())
     return out
 
@@ -135,4 +136,24 @@ def gemm_bt(a, bt, bias=None, m: Optional[int] = None, m_dev: Optional[torch.Ten
         out = torch.zeros(rows, n, dtype=a.dtype, device=a.device)
     _call("et_gemm_bt_bias_gelu" if gelu else "et_gemm_bt", a.device, _dtype_code(a.dtype), _p(a), _p(bt), _p(out),
           _p(bias), rows if m is None else m, n, k, _p(m_dev), _stream())
+    return out
+
+
+def split_rows(a, m_dev: Optional[torch.Tensor] = None, out: Optional[torch.Tensor] = None):
+    """fp32 [m, k] -> split rows [m, 3 k] bfloat16 (layout: et_gemm_split in et.h)."""
+    rows, k = a.shape
+    if out is None:
+        out = torch.zeros(rows, 3 * k, dtype=torch.bfloat16, device=a.device)
+    _call("et_split_rows", a.device, _p(a), _p(out), rows, k, _p(m_dev), _stream())
+    return out
+
+
+def gemm_split(a, bt, bias=None, m_dev: Optional[torch.Tensor] = None, out: Optional[torch.Tensor] = None,
+               gelu: bool = False):
+    """Split rows a [m, 3 k], bt [n, 3 k] -> fp32 [m, n] (+ bias), or with gelu the split rows of gelu(product + bias)."""
+    rows, n, k = a.shape[0], bt.shape[0], a.shape[1] // 3
+    if out is None:
+        out = torch.zeros(rows, 3 * n, dtype=torch.bfloat16, device=a.device) if gelu else \
+            torch.zeros(rows, n, dtype=torch.float32, device=a.device)
+    _call("et_gemm_split", a.device, _p(a), _p(bt), _p(out), _p(bias), 1 if gelu else 0, rows, n, k, _p(m_dev), _stream())
     return out

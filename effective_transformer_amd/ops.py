@@ -203,15 +203,13 @@ class LayerWeights:
         self._prepared_tensors: List[torch.Tensor] = []
 
     def prepare(self, every_kernel: bool = True) -> "LayerWeights":
-        """For weights that stay as they are: k-contiguous ([out,in]) copies of the dense kernels, made once, which the
-        layer op then uses for its large-M GEMMs instead of transposing on every call (fp16 only; a no-op for fp32).
-        every_kernel=False: only the kernels of the wide projections (Q, K, V, FFN up), the ones the layer op would
-        transpose by itself."""
-        if self.t["attr_kernel_q"].dtype != torch.float16:
-            return self
-        # the k-contiguous kernels take k in multiples of 64 and n in multiples of 8; other hidden sizes run the [k][n] kernels
+        """For weights that stay as they are: the copies of the dense kernels that the layer op's GEMMs read, made once
+        instead of on every call.  fp16: k-contiguous ([out,in]); fp32: k-contiguous split rows (et_gemm_split in et.h).
+        every_kernel=False: only the kernels of the wide projections (Q, K, V, FFN up)."""
+        # hidden sizes the tuned GEMMs do not take have no copies: k in multiples of 64 in fp16, of 32 in fp32
         hq = self.t["attr_kernel_q"].shape[0]
-        if hq % 64 != 0:
+        half = self.t["attr_kernel_q"].dtype == torch.float16
+        if hq % (64 if half else 32) != 0:
             return self
         lib = _lib.load()
         dev = self.t["attr_kernel_q"].device
@@ -225,16 +223,16 @@ class LayerWeights:
         with torch.cuda.device(dev):
             # the copies of Q, K, V and the attention output kernel lie one behind the other: one region for the layer in
             # front of this one to request (et_layer_prepared.warm)
-            hq = self.t["attr_kernel_q"].shape[0]
             together = [nm for nm, _ in names if nm.startswith("attr_") and tuple(self.t[nm].shape) == (hq, hq)]
-            block = torch.empty(len(together), hq, hq, dtype=torch.float16, device=dev)
+            width, dt = (1, torch.float16) if half else (3, torch.bfloat16)
+            block = torch.empty(len(together), hq, width * hq, dtype=dt, device=dev)
             self.warm_block = block if len(together) >= 3 else None
             for src_name, field in names:
                 src = self.t[src_name]
                 k, n = src.shape
                 dst = block[together.index(src_name)] if src_name in together else \
-                    torch.empty(n, k, dtype=src.dtype, device=dev)
-                _lib.check(lib.et_transpose_weight(h, _lib.ET_FP16, _p(src), _p(dst), k, n, _stream()), h)
+                    torch.empty(n, width * k, dtype=dt, device=dev)
+                _lib.check(lib.et_transpose_weight(h, _dtype_code(src.dtype), _p(src), _p(dst), k, n, _stream()), h)
                 self._prepared_tensors.append(dst)
                 setattr(prep, field, dst.data_ptr())
         self.prepared = prep

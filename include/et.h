@@ -139,9 +139,9 @@ et_status et_layer(et_handle h, et_dtype dtype, const et_layer_weights* weights,
 /* What a caller that keeps a layer's weights constant can prepare once instead of having et_layer redo it on every
  * call.  No counterpart in the reference, whose op receives the weights as inputs of every call (tf_op/
  * bert_transformer_op.cc:44-77) and rebuilds nothing across calls either.  Every member may be NULL.
- *   *_t: the dense kernel handed over [out,in] (k-contiguous), i.e. et_transpose_weight of the [in,out] tensor, fp16
- *        only.  Used where et_layer would run its large-M GEMM (it then skips its per-call transposition; Q, K and V
- *        go together); ignored for batches that run the small-M kernels, which read the [in,out] tensors.
+ *   *_t: the dense kernel as et_transpose_weight leaves it: [out,in] (k-contiguous) in fp16, split rows in fp32.  The
+ *        call then skips making that copy itself; Q, K and V go together.  Ignored for hidden sizes whose GEMMs read the
+ *        [in,out] tensors (no multiple of 64 in fp16, of 32 in fp32).
  *   seq_start, seq_start_bytes: the sequence table et_sequence_starts wrote for THIS batch and the size of its buffer
  *        (at least et_seq_workspace_bytes(batch_size), ET_WORKSPACE_TOO_SMALL below); the same table serves every
  *        layer of the batch.
@@ -319,8 +319,9 @@ et_status et_gemm(et_handle h, et_dtype dtype, const void* A, const void* B, voi
 et_status et_gemm_bias_gelu(et_handle h, et_dtype dtype, const void* A, const void* B, void* C, const void* bias,
                             int m, int n, int k, const int32_t* m_dev, void* stream);
 
-/* dst[n][k] = transpose of src[k][n] (both row-major), fp16 only.  No counterpart in the reference, which hands the
- * TF dense kernels [in,out] to cuBLAS as they are; et_layer does this internally for its large-M GEMMs. */
+/* fp16: dst[n][k] = transpose of src[k][n] (both row-major).  fp32: dst = the n split rows of the transpose (see
+ * et_gemm_split), 6 k n bytes; k % 32 == 0, n % 4 == 0.  No counterpart in the reference, which hands the TF dense kernels
+ * [in,out] to cuBLAS as they are; et_layer does this internally for its GEMMs. */
 et_status et_transpose_weight(et_handle h, et_dtype dtype, const void* src, void* dst, int k, int n, void* stream);
 
 /* et_gemm with the second operand k-contiguous: C[m,n] = A[m,k] . Bt[n,k]^T (+ bias), fp16 only.  This is the kernel
@@ -337,6 +338,18 @@ et_status et_gemm_bt(et_handle h, et_dtype dtype, const void* A, const void* Bt,
  * bias required; shapes as for et_gemm_bt. */
 et_status et_gemm_bt_bias_gelu(et_handle h, et_dtype dtype, const void* A, const void* Bt, void* C, const void* bias,
                                int m, int n, int k, const int32_t* m_dev, void* stream);
+
+/* The fp32 product of the layer on the 16-bit matrix cores: C[m,n] = A[m,k] . Bt[n,k]^T (+ bias).  Both operands are
+ * split rows, [row][k / 32][3][32] bfloat16: every float is the exact sum of three bfloat16 pieces (h, m, l, each the rest
+ * of the ones before it rounded to nearest), kept side by side for every 32 values.  The six products of pieces that
+ * reach into the float result are summed in float, leading ones and corrections apart; against float64 the result is
+ * closer than that of the fp32 matrix instructions et_gemm runs on.  k % 32 == 0, n % 4 == 0.  C is float [m,n]; with
+ * gelu it holds the split rows of gelu(A.Bt^T + bias) instead (6 n bytes per row, n % 32 == 0, bias required).  Bt comes
+ * from et_transpose_weight(ET_FP32), A from et_split_rows: dst = the split rows of the first m (or *m_dev) rows of
+ * src[m][k]. */
+et_status et_split_rows(et_handle h, const void* src, void* dst, int m, int k, const int32_t* m_dev, void* stream);
+et_status et_gemm_split(et_handle h, const void* A, const void* Bt, void* C, const void* bias, int gelu, int m, int n,
+                        int k, const int32_t* m_dev, void* stream);
 
 /* Measurement aid, no counterpart in the reference and no part of the encoder path: one launch of `iters` k-steps of
  * the large fp16 GEMM's inner loop (per wavefront 32 v_mfma_f32_16x16x32_f16 and 12 16-byte LDS operand reads, 8
