@@ -41,6 +41,13 @@ class EmbeddingWeights(C.Structure):
                 ("vocab_size", C.c_int), ("type_vocab_size", C.c_int), ("max_position_embeddings", C.c_int)]
 
 
+class EncoderBatch(C.Structure):
+    _fields_ = [("from_tensor", C.c_void_p), ("embeddings", C.POINTER(EmbeddingWeights)), ("input_ids", C.c_void_p),
+                ("token_type_ids", C.c_void_p), ("mask", C.c_void_p), ("attr_mask", C.c_void_p), ("out", C.c_void_p),
+                ("batch_size", C.c_int), ("seq_len", C.c_int), ("rows_bound", C.c_int), ("count_word", C.c_void_p),
+                ("valid_word_num", C.POINTER(C.c_int32))]
+
+
 class EtError(RuntimeError):
     def __init__(self, status: int, message: str):
         super().__init__("%s: %s" % (STATUS_NAMES.get(status, str(status)), message))
@@ -68,6 +75,9 @@ SIGNATURES = {
     "et_sequence_starts": (_i, [_vp, _vp, _vp, _i, _i, _vp, _sz, _vp]),
     "et_layer_with_prepared": (_i, [_vp, _i, C.POINTER(LayerWeights), C.POINTER(LayerPrepared), _vp, _vp, _vp, _vp, _vp,
                                     _vp, _vp, _i, _i, _i, _i, _i, _i, _vp, _sz, _vp]),
+    "et_encoder_workspace_bytes": (_sz, [_i, _i, _i, _i, _i]),
+    "et_encoder": (_i, [_vp, _i, _i, C.POINTER(LayerWeights), C.POINTER(LayerPrepared), C.POINTER(EncoderBatch), _i, _i, _vp,
+                        _sz, _vp]),
     "et_first_token": (_i, [_vp, _i, _vp, _vp, _vp, _vp, _vp, _i, _i, _i, _vp]),
     "et_output": (_i, [_vp, _i, _vp, _vp, _vp, _vp, _vp, _i, _i, _i, _i, _vp]),
     "et_exclusive_scan": (_i, [_vp, _vp, _vp, _i, _vp, _sz, _vp]),

@@ -6,6 +6,8 @@
 
 #include <hip/hip_runtime.h>
 
+#include <algorithm>
+#include <atomic>
 #include <cmath>
 #include <cstdio>
 #include <cstring>
@@ -231,6 +233,21 @@ float softmax_scaler(et_dtype dtype, int d) {
   float s = 1.0f / sqrtf((float)d);
   if (dtype == ET_FP16) s = (float)(_Float16)s;   // the reference holds the scaler in the element type
   return s;
+}
+
+et_status embedding_args_ok(et_handle h, et_dtype dtype, const et_embedding_weights* emb, const int32_t* token_type_ids,
+                            int seq_len, int H) {
+  ET_REQUIRE(h, emb != nullptr, "null embeddings");
+  ET_REQUIRE(h, emb->word_embeddings && emb->layernorm_gamma && emb->layernorm_beta, "null embedding table or LayerNorm weight");
+  ET_REQUIRE(h, emb->vocab_size >= 1, "vocab_size must be >= 1");
+  ET_REQUIRE(h, (emb->token_type_embeddings == nullptr) == (token_type_ids == nullptr),
+             "token_type_ids and token_type_embeddings go together");
+  ET_REQUIRE(h, emb->token_type_embeddings == nullptr || emb->type_vocab_size >= 1, "type_vocab_size must be >= 1");
+  ET_REQUIRE(h, emb->position_embeddings == nullptr || seq_len <= emb->max_position_embeddings,
+             "seq_len exceeds max_position_embeddings");
+  if (!et::layernorm_row_in_registers(to_dt(dtype), H))
+    return fail(h, ET_UNSUPPORTED, "hidden size not supported by the embedding kernel (even, at most 4096)");
+  return ET_OK;
 }
 
 // What a layer asks of its arguments whoever calls it; the tensors and the entry are the caller's to check.
@@ -600,21 +617,12 @@ et_status et_embedding_input(et_handle h, et_dtype dtype, const et_embedding_wei
   if (s != ET_OK) return s;
   ET_REQUIRE(h, dtype_ok(dtype), "dtype must be ET_FP32 or ET_FP16");
   if ((s = dims_ok(h, batch_size, seq_len, head_num, size_per_head)) != ET_OK) return s;
-  ET_REQUIRE(h, emb != nullptr, "null embeddings");
-  ET_REQUIRE(h, emb->word_embeddings && emb->layernorm_gamma && emb->layernorm_beta, "null embedding table or LayerNorm weight");
-  ET_REQUIRE(h, emb->vocab_size >= 1, "vocab_size must be >= 1");
-  ET_REQUIRE(h, (emb->token_type_embeddings == nullptr) == (token_type_ids == nullptr),
-             "token_type_ids and token_type_embeddings go together");
-  ET_REQUIRE(h, emb->token_type_embeddings == nullptr || emb->type_vocab_size >= 1, "type_vocab_size must be >= 1");
-  ET_REQUIRE(h, emb->position_embeddings == nullptr || seq_len <= emb->max_position_embeddings,
-             "seq_len exceeds max_position_embeddings");
+  if ((s = embedding_args_ok(h, dtype, emb, token_type_ids, seq_len, head_num * size_per_head)) != ET_OK) return s;
   ET_REQUIRE(h, input_ids && mask && to_tensor && valid_word_num_dev && batch_idx && word_idx, "null tensor pointer");
   ET_REQUIRE(h, workspace != nullptr, "null workspace");
   if (workspace_bytes < et_input_workspace_bytes(batch_size, seq_len))
     return fail(h, ET_WORKSPACE_TOO_SMALL, "et_embedding_input needs et_input_workspace_bytes(batch_size, seq_len)");
   const int H = head_num * size_per_head;
-  if (!et::layernorm_row_in_registers(to_dt(dtype), H))
-    return fail(h, ET_UNSUPPORTED, "hidden size not supported by the embedding kernel (even, at most 4096)");
   hipStream_t st = (hipStream_t)stream;
   et::launch_scan_index(mask, batch_size * seq_len, nullptr, batch_idx, word_idx, valid_word_num_dev, seq_len,
                         (int32_t*)workspace, st);
@@ -687,6 +695,189 @@ et_status et_layer_with_prepared(et_handle h, et_dtype dtype, const et_layer_wei
   c.workspace = (char*)workspace;
   c.stream = (hipStream_t)stream;
   return run_layer(h, c);
+}
+
+// ---- the encoder in one call ------------------------------------------------------------------------------------
+
+namespace {
+
+struct EncoderWs {
+  size_t x[2], batch_idx, word_idx, count, seq, scan, layer, total;
+};
+
+EncoderWs encoder_ws(et_dtype dtype, int B, int S, int heads, int d) {
+  const size_t e = dtype == ET_FP32 ? 4 : 2;
+  const size_t rows = (size_t)B * S, H = (size_t)heads * d;
+  EncoderWs w;
+  size_t off = 0;
+  auto take = [&](size_t bytes) {
+    const size_t at = off;
+    off += align_up(bytes, 256);
+    return at;
+  };
+  w.x[0] = take(rows * H * e);
+  w.x[1] = take(rows * H * e);
+  w.batch_idx = take(rows * sizeof(int32_t));
+  w.word_idx = take(rows * sizeof(int32_t));
+  w.count = take(sizeof(int32_t));
+  w.seq = take(et_seq_workspace_bytes(B));
+  w.scan = take(et_input_workspace_bytes(B, S));
+  w.layer = take(et_layer_workspace_bytes(dtype, B, S, heads, d));
+  w.total = off;
+  return w;
+}
+
+// Waits until the scan of this call has stored its count (upper half = tag).  The word is written by the GPU in the
+// middle of the stream's work, so the host spins on it; now and then the stream is asked whether it has failed or run dry.
+et_status wait_for_count(et_handle h, const uint64_t* word, uint32_t tag, const int32_t* count_dev, hipStream_t st, int* T) {
+  for (unsigned spin = 1;; ++spin) {
+    const uint64_t v = __atomic_load_n(word, __ATOMIC_ACQUIRE);
+    if ((uint32_t)(v >> 32) == tag) {
+      *T = (int32_t)(uint32_t)v;
+      return ET_OK;
+    }
+    if (spin % 4096 != 0) {
+#if !defined(__HIP_DEVICE_COMPILE__)
+      __builtin_ia32_pause();
+#endif
+      continue;
+    }
+    const hipError_t q = hipStreamQuery(st);
+    if (q == hipErrorNotReady) {
+      (void)hipGetLastError();
+      continue;
+    }
+    ET_HIP(h, q);
+    // everything has run and the word is not there (memory the GPU's store does not reach): read the count itself
+    int32_t value = 0;
+    ET_HIP(h, hipMemcpyAsync(&value, count_dev, sizeof value, hipMemcpyDeviceToHost, st));
+    ET_HIP(h, hipStreamSynchronize(st));
+    *T = value;
+    return ET_OK;
+  }
+}
+
+// Batches of at most this many padded positions are launched for all of them without waiting for the count: the launches
+// of fewer rows would hardly be smaller (a handful of 32-row tiles), and the host may run ahead.
+constexpr int kWaitForCountRows = 256;
+
+}  // namespace
+
+size_t et_encoder_workspace_bytes(et_dtype dtype, int batch_size, int seq_len, int head_num, int size_per_head) {
+  if (batch_size < 1 || seq_len < 1 || head_num < 1 || size_per_head < 1 || !dtype_ok(dtype)) return 0;
+  return encoder_ws(dtype, batch_size, seq_len, head_num, size_per_head).total;
+}
+
+et_status et_encoder(et_handle h, et_dtype dtype, int num_layers, const et_layer_weights* weights,
+                     const et_layer_prepared* prepared, const et_encoder_batch* b, int head_num, int size_per_head,
+                     void* workspace, size_t workspace_bytes, void* stream) {
+  Entry entry(h);
+  et_status s = entry.status;
+  if (s != ET_OK) return s;
+  ET_REQUIRE(h, dtype_ok(dtype), "dtype must be ET_FP32 or ET_FP16");
+  ET_REQUIRE(h, b != nullptr, "null batch");
+  const int B = b->batch_size, S = b->seq_len, H = head_num * size_per_head;
+  if ((s = dims_ok(h, B, S, head_num, size_per_head)) != ET_OK) return s;
+  ET_REQUIRE(h, num_layers >= 1 && weights != nullptr, "an encoder has at least one layer");
+  ET_REQUIRE(h, (b->from_tensor != nullptr) != (b->embeddings != nullptr), "either from_tensor or embeddings");
+  ET_REQUIRE(h, b->mask && b->attr_mask && b->out && (b->from_tensor || b->input_ids), "null tensor pointer");
+  ET_REQUIRE(h, b->rows_bound >= 0 && b->rows_bound <= B * S, "rows_bound out of range");
+  if (b->embeddings && (s = embedding_args_ok(h, dtype, b->embeddings, b->token_type_ids, S, H)) != ET_OK) return s;
+  for (int l = 0; l < num_layers; ++l)
+    if ((s = layer_args_ok(h, dtype, weights + l, prepared ? prepared + l : nullptr, B, S, head_num, size_per_head)) != ET_OK)
+      return s;
+  ET_REQUIRE(h, workspace != nullptr, "null workspace");
+  const EncoderWs ws = encoder_ws(dtype, B, S, head_num, size_per_head);
+  if (workspace_bytes < ws.total) return fail(h, ET_WORKSPACE_TOO_SMALL, "et_encoder needs et_encoder_workspace_bytes(...)");
+  const et::DType dt = to_dt(dtype);
+  const size_t row_bytes = (size_t)H * et::elem_size(dt);
+  if (et::move_chunks(B * S, (int)row_bytes) >= (1ull << 31))
+    return fail(h, ET_UNSUPPORTED, "tensor too large for one launch");
+
+  char* base = (char*)workspace;
+  void* x[2] = {base + ws.x[0], base + ws.x[1]};
+  int32_t *batch_idx = (int32_t*)(base + ws.batch_idx), *word_idx = (int32_t*)(base + ws.word_idx);
+  int32_t *count = (int32_t*)(base + ws.count), *seq = (int32_t*)(base + ws.seq);
+  char* layer_base = base + ws.layer;
+  hipStream_t st = (hipStream_t)stream;
+
+  // The count comes back through the caller's pinned word, stored by the scan itself: no copy on the stream, no event.
+  // Every call has a tag of its own, so a word left by an earlier batch is never taken for this one's.
+  static std::atomic<uint32_t> next_tag{1};
+  const bool wait_for_layers = b->rows_bound == 0 && num_layers > 1 && B * S > kWaitForCountRows;
+  et::ScanExtras scan;
+  scan.seq_start = seq;
+  if (b->count_word && (wait_for_layers || b->valid_word_num)) {
+    scan.host_word = b->count_word;
+    scan.host_tag = next_tag.fetch_add(1, std::memory_order_relaxed);
+    if (scan.host_tag == 0) scan.host_tag = next_tag.fetch_add(1, std::memory_order_relaxed);
+  }
+  et::launch_scan_index(b->mask, B * S, nullptr, batch_idx, word_idx, count, S, (int32_t*)(base + ws.scan), st, scan);
+  if ((s = check_launch(h, "mask scan")) != ET_OK) return s;
+  const bool split = layer_splits(dtype, H);
+  et::CompressExtras extras;
+  extras.seq_table = seq;
+  // (split layers read their first input from the room of the layer workspace's intermediate)
+  const size_t split_off = layer_ws(dtype, B, S, head_num, size_per_head).inter;
+  if (split) extras.split = (uint16_t*)(layer_base + split_off);
+  if (b->embeddings) {
+    const et_embedding_weights& emb = *b->embeddings;
+    et::launch_embed_layernorm(dt, x[0], b->input_ids, b->token_type_ids, batch_idx, word_idx, emb.word_embeddings,
+                               emb.vocab_size, emb.token_type_embeddings, emb.type_vocab_size, emb.position_embeddings,
+                               emb.max_position_embeddings, emb.layernorm_gamma, emb.layernorm_beta, B * S, H, S, count, st,
+                               extras, B);
+  } else {
+    et::launch_compress_rows(b->from_tensor, x[0], batch_idx, word_idx, count, nullptr, nullptr, B, S, (int)row_bytes, st,
+                             extras);
+  }
+  if ((s = check_launch(h, "input")) != ET_OK) return s;
+
+  LayerCall c;
+  c.dtype = dtype;
+  c.attr_mask = b->attr_mask;
+  c.count = count; c.batch_idx = batch_idx; c.word_idx = word_idx;
+  c.seq_start = seq;
+  c.B = B; c.S = S; c.heads = head_num; c.d = size_per_head;
+  c.rows = b->rows_bound > 0 ? b->rows_bound : B * S;
+  c.workspace = layer_base;
+  c.stream = st;
+  int T = -1;
+  int cur = 0;
+  for (int l = 0; l < num_layers && c.rows > 0; ++l) {
+    if (l == 1 && wait_for_layers && scan.host_word) {
+      // the first layer, sized for every position, is in the queue: the GPU has work while the host waits for the count
+      // (other threads may use the handle meanwhile)
+      entry.lock.unlock();
+      s = wait_for_count(h, scan.host_word, scan.host_tag, count, st, &T);
+      entry.lock.lock();
+      if (s != ET_OK) return s;
+      c.rows = std::min(std::max(T, 0), B * S);
+      if (c.rows == 0) break;
+    }
+    c.w = weights + l;
+    c.prep = prepared ? prepared + l : nullptr;
+    c.from = c.to = x[cur];
+    c.out = x[cur ^ 1];
+    c.from_split_ready = split;
+    c.write_out_split = l + 1 < num_layers;
+    if ((s = run_layer(h, c)) != ET_OK) return s;
+    cur ^= 1;
+  }
+  et::launch_restore_rows(b->out, x[cur], batch_idx, word_idx, count, B, S, (int)row_bytes, st);
+  if ((s = check_launch(h, "restore")) != ET_OK) return s;
+  if (b->valid_word_num) {
+    if (T < 0 && scan.host_word) {
+      entry.lock.unlock();
+      s = wait_for_count(h, scan.host_word, scan.host_tag, count, st, &T);
+      entry.lock.lock();
+      if (s != ET_OK) return s;
+    } else if (T < 0) {
+      ET_HIP(h, hipMemcpyAsync(&T, count, sizeof T, hipMemcpyDeviceToHost, st));
+      ET_HIP(h, hipStreamSynchronize(st));
+    }
+    *b->valid_word_num = T;
+  }
+  return ET_OK;
 }
 
 et_status et_output(et_handle h, et_dtype dtype, const void* from_tensor, const int32_t* valid_word_num_dev,

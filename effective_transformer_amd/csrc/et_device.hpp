@@ -179,4 +179,30 @@ __device__ __forceinline__ void seq_start_for_row(const int32_t* __restrict__ ba
   for (int b = prev + 1; b <= last; ++b) seq_start[b] = t;
 }
 
+// order[0..batch) = the sequences sorted by length, longest first (buckets of 16 tokens; the order inside a bucket is
+// whatever the atomics give: it only decides which workgroup of the attention kernel starts first).  All THREADS threads
+// of one workgroup.
+constexpr int kOrderBuckets = 65;             // lengths up to 1024
+template <int THREADS>
+__device__ __forceinline__ void sort_sequences(const int32_t* __restrict__ seq_start, int batch, int32_t* __restrict__ order) {
+  __shared__ int hist[kOrderBuckets], base[kOrderBuckets];
+  for (int i = threadIdx.x; i < kOrderBuckets; i += THREADS) hist[i] = 0;
+  __syncthreads();
+  auto bucket_of = [&](int b) {
+    const int len = seq_start[b + 1] - seq_start[b];
+    return kOrderBuckets - 1 - min(max(len, 0) >> 4, kOrderBuckets - 1);      // longest first
+  };
+  for (int b = threadIdx.x; b < batch; b += THREADS) atomicAdd(&hist[bucket_of(b)], 1);
+  __syncthreads();
+  if (threadIdx.x == 0) {
+    int run = 0;
+    for (int i = 0; i < kOrderBuckets; ++i) {
+      base[i] = run;
+      run += hist[i];
+    }
+  }
+  __syncthreads();
+  for (int b = threadIdx.x; b < batch; b += THREADS) order[atomicAdd(&base[bucket_of(b)], 1)] = b;
+}
+
 }  // namespace et

@@ -57,7 +57,8 @@ __global__ __launch_bounds__(kScanThreads) void scan_index_kernel(const int32_t*
                                                                    int32_t* __restrict__ prefix_out,
                                                                    int32_t* __restrict__ batch_idx,
                                                                    int32_t* __restrict__ word_idx,
-                                                                   int32_t* __restrict__ valid_word_num, int seq_len) {
+                                                                   int32_t* __restrict__ valid_word_num, int seq_len,
+                                                                   ScanExtras extras) {
   __shared__ int lds[kScanWaves];
   __shared__ int wave_tot[kScanWaves];
   int part = 0;
@@ -109,8 +110,20 @@ __global__ __launch_bounds__(kScanThreads) void scan_index_kernel(const int32_t*
           batch_idx[excl] = b;
           word_idx[excl] = idx - b * seq_len;
         }
+        // the first half of the sequence table: the prefix where a sequence begins is its first packed row
+        if (extras.seq_start) {
+          const int b = idx / seq_len;
+          if (idx == b * seq_len) extras.seq_start[b] = min(max(excl, 0), n);
+        }
         // T = prefix[last] + (mask[last] == 1)   (bert_transformer_op.cu.cc:306-315)
-        if (idx == n - 1) *valid_word_num = excl + (v == 1 ? 1 : 0);
+        if (idx == n - 1) {
+          const int T = excl + (v == 1 ? 1 : 0);
+          *valid_word_num = T;
+          if (extras.seq_start) extras.seq_start[n / seq_len] = min(max(T, 0), n);
+          if (extras.host_word)
+            __hip_atomic_store(extras.host_word, ((uint64_t)extras.host_tag << 32) | (uint32_t)T, __ATOMIC_RELEASE,
+                               __HIP_MEMORY_SCOPE_SYSTEM);
+        }
       }
     }
     carry += chunk;
@@ -142,7 +155,17 @@ template <typename CH>
 __global__ __launch_bounds__(kMoveThreads) void compress_rows_kernel(
     const CH* __restrict__ from, CH* __restrict__ to, const int32_t* __restrict__ batch_idx,
     const int32_t* __restrict__ word_idx, const int32_t* __restrict__ rows_dev, const int32_t* __restrict__ prefix,
-    const int32_t* __restrict__ mask, int n_pos, int seq_len, fastdiv cpr) {
+    const int32_t* __restrict__ mask, int n_pos, int seq_len, fastdiv cpr, CompressExtras extras) {
+  // the first workgroup sorts the sequence table whose first half the scan wrote, where that is asked for
+  uint32_t block = blockIdx.x;
+  if (extras.seq_table) {
+    if (block == 0) {
+      const int batch = n_pos / seq_len;
+      sort_sequences<kMoveThreads>(extras.seq_table, batch, extras.seq_table + batch + 1);
+      return;
+    }
+    --block;
+  }
   int T;
   if (rows_dev) {
     T = *rows_dev;
@@ -151,8 +174,8 @@ __global__ __launch_bounds__(kMoveThreads) void compress_rows_kernel(
   }
   T = min(T, n_pos);
   const uint32_t total = (uint32_t)T * cpr.d;
-  const uint32_t base = blockIdx.x * (kMoveThreads * kMoveUnroll) + threadIdx.x;
-  if (blockIdx.x * (kMoveThreads * kMoveUnroll) >= total) return;
+  const uint32_t base = block * (kMoveThreads * kMoveUnroll) + threadIdx.x;
+  if (block * (kMoveThreads * kMoveUnroll) >= total) return;
   // No predication at all: lanes past the end repeat the last chunk (load and store of identical data), so that
   // all index loads, then all data loads, then all stores are issued back to back.
   const uint32_t last = total - 1;
@@ -175,6 +198,13 @@ __global__ __launch_bounds__(kMoveThreads) void compress_rows_kernel(
   }
 #pragma unroll
   for (int u = 0; u < kMoveUnroll; ++u) to[idx[u]] = val[u];
+  // float rows once more as split rows, the form the first layer's products read
+  if constexpr (sizeof(CH) == 16)
+    if (extras.split) {
+#pragma unroll
+      for (int u = 0; u < kMoveUnroll; ++u)
+        store_split<4>(extras.split + (size_t)row[u] * cpr.d * 12, (int)chunk[u] * 4, __builtin_bit_cast(float4v, val[u]));
+    }
 }
 
 constexpr int kRestorePos = 32;   // padded positions per workgroup
@@ -254,29 +284,10 @@ __global__ __launch_bounds__(256) void seq_start_kernel(const int32_t* __restric
   seq_start_for_row(batch_idx, T, blockIdx.x * 256 + threadIdx.x, batch, seq_start);
 }
 
-// order[0..batch) = the sequences sorted by length, longest first (buckets of 16 tokens; the order inside a bucket is
-// whatever the atomics give: it only decides which workgroup of the attention kernel starts first).  One workgroup.
-constexpr int kOrderBuckets = 65;             // lengths up to 1024
+// order[0..batch) = the sequences sorted by length, longest first.  One workgroup.
 __global__ __launch_bounds__(1024) void seq_order_kernel(const int32_t* __restrict__ seq_start, int batch,
                                                          int32_t* __restrict__ order) {
-  __shared__ int hist[kOrderBuckets], base[kOrderBuckets];
-  for (int i = threadIdx.x; i < kOrderBuckets; i += 1024) hist[i] = 0;
-  __syncthreads();
-  auto bucket_of = [&](int b) {
-    const int len = seq_start[b + 1] - seq_start[b];
-    return kOrderBuckets - 1 - min(max(len, 0) >> 4, kOrderBuckets - 1);      // longest first
-  };
-  for (int b = threadIdx.x; b < batch; b += 1024) atomicAdd(&hist[bucket_of(b)], 1);
-  __syncthreads();
-  if (threadIdx.x == 0) {
-    int run = 0;
-    for (int i = 0; i < kOrderBuckets; ++i) {
-      base[i] = run;
-      run += hist[i];
-    }
-  }
-  __syncthreads();
-  for (int b = threadIdx.x; b < batch; b += 1024) order[atomicAdd(&base[bucket_of(b)], 1)] = b;
+  sort_sequences<1024>(seq_start, batch, order);
 }
 
 // to[b,:] = row of the packed matrix that sits at position 0 of sequence b, zeros where sequence b has no token
@@ -329,7 +340,8 @@ size_t scan_scratch_words(int length) {
 }
 
 void launch_scan_index(const int32_t* in, int length, int32_t* prefix_out, int32_t* batch_idx, int32_t* word_idx,
-                       int32_t* valid_word_num, int seq_len, int32_t* scratch, hipStream_t stream) {
+                       int32_t* valid_word_num, int seq_len, int32_t* scratch, hipStream_t stream,
+                       const ScanExtras& extras) {
   const int tile = scan_tile_for(length);
   const int tiles = (length + tile - 1) / tile;
   // up to 128 tiles every workgroup re-adds the elements in front of its tile itself (at most 508 KB of L2 reads);
@@ -337,7 +349,7 @@ void launch_scan_index(const int32_t* in, int length, int32_t* prefix_out, int32
   const bool direct = tiles <= 128 && (reinterpret_cast<uintptr_t>(in) & 15) == 0;
   if (!direct) scan_tile_sums_kernel<<<tiles, kScanThreads, 0, stream>>>(in, length, tile, scratch);
   scan_index_kernel<<<tiles, kScanThreads, 0, stream>>>(in, length, tile, direct ? nullptr : scratch, prefix_out,
-                                                         batch_idx, word_idx, valid_word_num, seq_len);
+                                                         batch_idx, word_idx, valid_word_num, seq_len, extras);
 }
 
 void launch_index_from_prefix(const int32_t* mask, const int32_t* prefix, int32_t* batch_idx, int32_t* word_idx,
@@ -355,24 +367,25 @@ size_t move_chunks(int n_pos, int row_bytes) { return (size_t)n_pos * (size_t)(r
 
 void launch_compress_rows(const void* from, void* to, const int32_t* batch_idx, const int32_t* word_idx,
                           const int32_t* rows_dev, const int32_t* prefix, const int32_t* mask, int batch, int seq_len,
-                          int row_bytes, hipStream_t stream) {
+                          int row_bytes, hipStream_t stream, const CompressExtras& extras) {
   const int n_pos = batch * seq_len;
   const int cb = move_chunk_bytes(row_bytes);
   const uint32_t cpr = (uint32_t)row_bytes / (uint32_t)cb;
   const uint64_t chunks = (uint64_t)n_pos * cpr;
   const uint32_t per_wg = kMoveThreads * kMoveUnroll;
-  const uint32_t grid = (uint32_t)((chunks + per_wg - 1) / per_wg);
+  const uint32_t grid = (uint32_t)((chunks + per_wg - 1) / per_wg) + (extras.seq_table ? 1 : 0);
   if (cb == 16)
     compress_rows_kernel<u32x4><<<grid, kMoveThreads, 0, stream>>>((const u32x4*)from, (u32x4*)to, batch_idx, word_idx,
-                                                                   rows_dev, prefix, mask, n_pos, seq_len, make_fastdiv(cpr));
+                                                                   rows_dev, prefix, mask, n_pos, seq_len, make_fastdiv(cpr),
+                                                                   extras);
   else if (cb == 4)
     compress_rows_kernel<uint32_t><<<grid, kMoveThreads, 0, stream>>>((const uint32_t*)from, (uint32_t*)to, batch_idx,
                                                                       word_idx, rows_dev, prefix, mask, n_pos, seq_len,
-                                                                      make_fastdiv(cpr));
+                                                                      make_fastdiv(cpr), extras);
   else
     compress_rows_kernel<uint16_t><<<grid, kMoveThreads, 0, stream>>>((const uint16_t*)from, (uint16_t*)to, batch_idx,
                                                                       word_idx, rows_dev, prefix, mask, n_pos, seq_len,
-                                                                      make_fastdiv(cpr));
+                                                                      make_fastdiv(cpr), extras);
 }
 
 void launch_restore_rows(void* to, const void* from, const int32_t* batch_idx, const int32_t* word_idx,

@@ -21,11 +21,21 @@ hipError_t take_attribute_error();
 // ---- input_output.hip --------------------------------------------------------------------
 // Number of int32 words of scratch the scan needs for `length` elements.
 size_t scan_scratch_words(int length);
+// What the scan of a mask can leave behind on its way, and what the compress launch behind it can (each nullable).
+struct ScanExtras {
+  int32_t* seq_start = nullptr;      // first half of the batch's sequence table (see launch_seq_start)
+  uint64_t* host_word = nullptr;     // pinned host memory: host_tag << 32 | valid-token count, one 8-byte store
+  uint32_t host_tag = 0;
+};
+struct CompressExtras {
+  int32_t* seq_table = nullptr;      // the table whose first half the scan wrote: its second half is filled in
+  uint16_t* split = nullptr;         // float rows of a multiple of 32 values: the packed rows once more as split rows
+};
 // Exclusive prefix sum of `in`; optionally (seq_len > 0) also writes batch_idx / word_idx for
 // every element > 0 and the valid-token count.  prefix_out may be null.
 void launch_scan_index(const int32_t* in, int length, int32_t* prefix_out, int32_t* batch_idx,
                        int32_t* word_idx, int32_t* valid_word_num, int seq_len, int32_t* scratch,
-                       hipStream_t stream);
+                       hipStream_t stream, const ScanExtras& extras = ScanExtras());
 // batch_idx / word_idx from mask + an existing prefix sum.
 void launch_index_from_prefix(const int32_t* mask, const int32_t* prefix, int32_t* batch_idx,
                               int32_t* word_idx, int batch, int seq_len, hipStream_t stream);
@@ -33,7 +43,8 @@ void launch_index_from_prefix(const int32_t* mask, const int32_t* prefix, int32_
 // otherwise from prefix[last] + (mask[last] == 1).
 void launch_compress_rows(const void* from, void* to, const int32_t* batch_idx, const int32_t* word_idx,
                           const int32_t* rows_dev, const int32_t* prefix, const int32_t* mask,
-                          int batch, int seq_len, int row_bytes, hipStream_t stream);
+                          int batch, int seq_len, int row_bytes, hipStream_t stream,
+                          const CompressExtras& extras = CompressExtras());
 // Chunks (16, 4 or 2 bytes: the widest piece row_bytes is a whole number of) the two movers below index for n_pos rows;
 // must stay below 2^31.
 size_t move_chunks(int n_pos, int row_bytes);
@@ -79,7 +90,8 @@ void launch_bias_residual_layernorm(DType t, void* out, const void* input, const
 void launch_embed_layernorm(DType t, void* out, const int32_t* ids, const int32_t* type_ids, const int32_t* batch_idx,
                             const int32_t* word_idx, const void* word_table, int vocab, const void* type_table,
                             int type_vocab, const void* pos_table, int max_pos, const void* gamma, const void* beta,
-                            int m, int n, int seq_len, const int32_t* rows_dev, hipStream_t stream);
+                            int m, int n, int seq_len, const int32_t* rows_dev, hipStream_t stream,
+                            const CompressExtras& extras = CompressExtras(), int batch = 0);
 
 // ---- attention.hip -----------------------------------------------------------------------
 void launch_qkv_bias_pad(DType t, const void* Q, const void* bQ, const void* K, const void* bK,

@@ -192,12 +192,18 @@ __global__ __launch_bounds__(kLnThreads) void embed_layernorm_kernel(
     const int32_t* __restrict__ batch_idx, const int32_t* __restrict__ word_idx, const T* __restrict__ word_table,
     int vocab, const T* __restrict__ type_table, int type_vocab, const T* __restrict__ pos_table, int max_pos,
     const T* __restrict__ gamma, const T* __restrict__ beta, int m, int n, int seq_len,
-    const int32_t* __restrict__ rows_dev) {
+    const int32_t* __restrict__ rows_dev, CompressExtras extras, int batch) {
   using V = typename RowVec<T, VEC>::type;
+  // the first workgroup sorts the sequence table whose first half the scan wrote, where that is asked for
+  const int first = extras.seq_table ? 1 : 0;
+  if (first && blockIdx.x == 0) {
+    sort_sequences<kLnThreads>(extras.seq_table, batch, extras.seq_table + batch + 1);
+    return;
+  }
   const int rows = rows_dev ? min(*rows_dev, m) : m;
   const int lane = threadIdx.x & (kWave - 1);
-  const int wave = blockIdx.x * kLnWaves + threadIdx.x / kWave;
-  const int nwaves = gridDim.x * kLnWaves;
+  const int wave = ((int)blockIdx.x - first) * kLnWaves + threadIdx.x / kWave;
+  const int nwaves = ((int)gridDim.x - first) * kLnWaves;
   const int vpr = n / VEC;
 
   V g[ITERS], be[ITERS];
@@ -262,6 +268,8 @@ __global__ __launch_bounds__(kLnThreads) void embed_layernorm_kernel(
 #pragma unroll
         for (int j = 0; j < VEC; ++j) y[j] = (T)(((x[i][j] - mean) * rstd) * (float)g[i][j] + (float)be[i][j]);
         orow[c] = y;
+        if constexpr (sizeof(T) == 4 && VEC == 4)
+          if (extras.split) store_split<4>(extras.split + (size_t)r * 3 * n, c * VEC, y);
       }
     }
   }
@@ -327,6 +335,8 @@ struct EmbedArgs {
   const void *word_table, *type_table, *pos_table, *gamma, *beta;
   int vocab, type_vocab, max_pos, m, n, seq_len;
   const int32_t* rows_dev;
+  CompressExtras extras;
+  int batch;
 };
 
 template <typename T, int VEC>
@@ -336,7 +346,7 @@ void embed_launch_iters(int iters, int grid, hipStream_t stream, const EmbedArgs
     embed_layernorm_kernel<T, VEC, I><<<grid, kLnThreads, 0, stream>>>(                                             \
         (T*)a.out, a.ids, a.type_ids, a.batch_idx, a.word_idx, (const T*)a.word_table, a.vocab,                     \
         (const T*)a.type_table, a.type_vocab, (const T*)a.pos_table, a.max_pos, (const T*)a.gamma, (const T*)a.beta, \
-        a.m, a.n, a.seq_len, a.rows_dev);                                                                           \
+        a.m, a.n, a.seq_len, a.rows_dev, a.extras, a.batch);                                                                           \
     break;
   switch (iters) {
     ET_EMB_CASE(1)
@@ -355,7 +365,7 @@ template <typename T>
 void embed_launch(const EmbedArgs& a, hipStream_t stream) {
   int vec = 0, iters = 0;
   if (!ln_pick<T>(a.n, vec, iters)) return;
-  const int grid = (int)min((long)(a.m + kLnWaves - 1) / kLnWaves, 256L * 8);
+  const int grid = (int)min((long)(a.m + kLnWaves - 1) / kLnWaves, 256L * 8) + (a.extras.seq_table ? 1 : 0);
   constexpr int MV = 16 / (int)sizeof(T);
   if (vec == MV)
     embed_launch_iters<T, MV>(iters, grid, stream, a);
@@ -370,10 +380,11 @@ void embed_launch(const EmbedArgs& a, hipStream_t stream) {
 void launch_embed_layernorm(DType t, void* out, const int32_t* ids, const int32_t* type_ids, const int32_t* batch_idx,
                             const int32_t* word_idx, const void* word_table, int vocab, const void* type_table,
                             int type_vocab, const void* pos_table, int max_pos, const void* gamma, const void* beta,
-                            int m, int n, int seq_len, const int32_t* rows_dev, hipStream_t stream) {
+                            int m, int n, int seq_len, const int32_t* rows_dev, hipStream_t stream,
+                            const CompressExtras& extras, int batch) {
   if (m <= 0) return;
   EmbedArgs a{out, ids, type_ids, batch_idx, word_idx, word_table, type_table, pos_table, gamma, beta,
-              vocab, type_vocab, max_pos, m, n, seq_len, rows_dev};
+              vocab, type_vocab, max_pos, m, n, seq_len, rows_dev, extras, batch};
   if (t == DType::F32)
     embed_launch<float>(a, stream);
   else

@@ -374,10 +374,29 @@ class EffectiveTransformerEncoder:
                     w.prepared.warm = nxt.warm_block.data_ptr()
                     w.prepared.warm_bytes = nxt.warm_block.numel() * 2
                     self._warm_refs.append(nxt.warm_block)
-        # ping-pong activations, sequence table and the pinned count, per (activation shape, stream, host thread): two
-        # threads or streams that run this encoder at the same time each have their own
-        self._bufs: Dict[tuple, list] = {}
-        self._bufs_lock = threading.Lock()
+        # what a call needs besides its workspace, per (stream, host thread): the pinned word its count comes back in
+        self._count_words: Dict[tuple, torch.Tensor] = {}
+        self._lock = threading.Lock()
+        self._table: Optional[tuple] = None
+
+    def _layer_table(self):
+        """The layers' weight and prepared structs as the arrays et_encoder takes.  Every prepared struct is made a view of
+        its array element, so that changes to one reach the next call; a layer that has been prepared anew since, or
+        replaced, has the table made again."""
+        t = self._table
+        if t is not None and len(t[0]) == len(self.layers) and \
+                all(w is ref and w.prepared is p for w, ref, p in zip(self.layers, t[0], t[1])):
+            return t
+        with self._lock:
+            n = len(self.layers)
+            weights, prepared = (_lib.LayerWeights * n)(), (_lib.LayerPrepared * n)()
+            for l, w in enumerate(self.layers):
+                weights[l] = w.struct
+                if w.prepared is not None:
+                    prepared[l] = w.prepared
+                    w.prepared = prepared[l]
+            self._table = t = (list(self.layers), [w.prepared for w in self.layers], weights, prepared)
+            return t
 
     @classmethod
     def from_checkpoint(cls, path: str, head_num: int, size_per_head: int, dtype: torch.dtype, device="cuda",
@@ -392,57 +411,65 @@ class EffectiveTransformerEncoder:
                  sync_count: bool = True, rows_bound: Optional[int] = None) -> torch.Tensor:
         """rows_bound (with sync_count=False): an upper bound of the valid-token count that the caller vouches for;
         the launches are sized for that many rows instead of B*S (rows beyond it would not be computed)."""
-        B, S = input_mask.shape
-        hn, d = self.head_num, self.size_per_head
-        x, vwn, bidx, widx = effective_transformer_input(from_tensor, input_mask, B, S, S, hn, d)
-        return self._layers_and_output(x, vwn, bidx, widx, sync_count, attention_mask, B, S, rows_bound)
+        _require_cuda(from_tensor)
+        if from_tensor.dtype != self.dtype:
+            raise TypeError("from_tensor must have the dtype of the weights")
+        batch = _lib.EncoderBatch()
+        batch.from_tensor = from_tensor.data_ptr()
+        return self._run(batch, from_tensor.shape, input_mask, attention_mask, sync_count, rows_bound)
 
     def forward_ids(self, input_ids, token_type_ids, input_mask, attention_mask, embeddings: "EmbeddingWeights",
                     sync_count: bool = True) -> torch.Tensor:
         """Embedding block + encoder from token ids: the packed token matrix is produced directly."""
-        B, S = input_mask.shape
-        hn, d = self.head_num, self.size_per_head
-        r = effective_transformer_embedding_input(input_ids, token_type_ids, input_mask, embeddings, hn, d)
-        x, vwn, bidx, widx = r[:4]
-        return self._layers_and_output(x, vwn, bidx, widx, sync_count, attention_mask, B, S)
+        _require_cuda(input_ids)
+        if input_ids.dtype != torch.int32 or (token_type_ids is not None and token_type_ids.dtype != torch.int32):
+            raise TypeError("ids and mask must be int32")
+        if embeddings.dtype != self.dtype:
+            raise TypeError("the embeddings must have the dtype of the weights")
+        batch = _lib.EncoderBatch()
+        batch.embeddings = C.pointer(embeddings.struct)
+        batch.input_ids = input_ids.data_ptr()
+        if token_type_ids is not None:
+            _require_cuda(token_type_ids)
+            batch.token_type_ids = token_type_ids.data_ptr()
+        return self._run(batch, (*input_mask.shape, embeddings.hidden), input_mask, attention_mask, sync_count, None)
 
-    def _layers_and_output(self, x, vwn, bidx, widx, sync_count, attention_mask, B, S, rows_bound=None):
-        """sync_count: read the valid-token count back once per batch, so that the launches of layers 2 .. L are sized
-        exactly (the reference reads it back in every layer).  The copy is asynchronous and the host waits for it
-        behind the launches of the first layer, which is sized for B*S rows and bounded on the device: the GPU never
-        idles for the read-back (waiting right after the input op left it without work for 0.13-0.19 ms per batch)."""
-        hn, d = self.head_num, self.size_per_head
-        key = (tuple(x.shape), torch.cuda.current_stream(x.device).cuda_stream, threading.get_ident(),
-               getattr(_scope, "owner", None))
-        with self._bufs_lock:
-            bufs = self._bufs.get(key)
-        if bufs is None:
-            # (the pinned word for the count is made on first use: a pass under graph capture never reads the count back)
-            bufs = [torch.empty_like(x), torch.empty_like(x),
-                    torch.empty(_lib.load().et_seq_workspace_bytes(B) // 4, dtype=torch.int32, device=x.device), None]
-            with self._bufs_lock:
-                self._bufs[key] = bufs
-        T, copied = -1, None
+    def _run(self, batch, shape, input_mask, attention_mask, sync_count, rows_bound):
+        """One et_encoder call.  sync_count: the valid-token count is read back once per batch, so that the launches of
+        layers 2 .. L are sized exactly (the reference reads it back in every layer); the host waits for it behind the
+        launches of the first layer, which is sized for B*S rows and bounded on the device, so the GPU never idles for it."""
+        lib = _lib.load()
+        _require_cuda(input_mask, attention_mask)
+        if input_mask.dtype != torch.int32:
+            raise TypeError("mask must be int32")
+        if attention_mask.dtype != self.dtype:
+            raise TypeError("attr_mask must have the dtype of from_tensor")
+        B, S = input_mask.shape
+        dev = input_mask.device
+        out = torch.empty(shape, dtype=self.dtype, device=dev)
+        code = _dtype_code(self.dtype)
+        stream = torch.cuda.current_stream().cuda_stream
         if not sync_count and rows_bound is not None:
             if not 0 < rows_bound <= B * S:
                 raise ValueError("rows_bound must be in 1 .. batch * seq_len")
-            T = int(rows_bound)
-        if sync_count and len(self.layers) > 1:
-            if bufs[3] is None:
-                bufs[3] = torch.empty(1, dtype=torch.int32, pin_memory=True)
-            bufs[3].copy_(vwn, non_blocking=True)
-            copied = torch.cuda.Event()
-            copied.record()
-        starts = sequence_starts(vwn, bidx, B, S, out=bufs[2])       # one table for all layers of the batch
-        for l, w in enumerate(self.layers):
-            out = bufs[l & 1]
-            if l == 1 and copied is not None:
-                copied.synchronize()
-                T = int(bufs[3].item())
-            effective_transformer(x, x, attention_mask, vwn, bidx, widx, w, B, S, S, hn, d, valid_word_num_hint=T,
-                                  out=out, seq_start=starts)
-            x = out
-        return effective_transformer_output(x, vwn, bidx, widx, B, S, S, hn, d)
+            batch.rows_bound = int(rows_bound)
+        if sync_count:
+            key = (stream, threading.get_ident())
+            word = self._count_words.get(key)
+            if word is None:
+                word = torch.zeros(1, dtype=torch.int64, pin_memory=True)
+                with self._lock:
+                    self._count_words[key] = word
+            batch.count_word = word.data_ptr()
+        batch.mask, batch.attr_mask, batch.out = input_mask.data_ptr(), attention_mask.data_ptr(), out.data_ptr()
+        batch.batch_size, batch.seq_len = B, S
+        nbytes = lib.et_encoder_workspace_bytes(code, B, S, self.head_num, self.size_per_head)
+        ws = _workspace(dev, "encoder", nbytes)
+        _, _, weights, prepared = self._layer_table()
+        h = handle(dev)
+        _lib.check(lib.et_encoder(h, code, len(self.layers), weights, prepared, C.byref(batch), self.head_num,
+                                  self.size_per_head, ws.data_ptr(), ws.numel(), stream), h)
+        return out
 
     def make_graph(self, from_tensor, input_mask, attention_mask,
                    max_valid_tokens: Optional[int] = None) -> "GraphedEncoder":
@@ -470,14 +497,11 @@ class GraphedEncoder:
         self.mask = input_mask.clone()
         self.attn = attention_mask.clone()
         # warm-up outside the capture (kernel attributes, allocator pools), on a side stream; its buffers are dropped
-        # again.  The workspaces and the encoder's ping-pong buffers made under this owner during the capture come from
-        # the graph's own memory pool, belong to this graph alone and are kept alive with it.
+        # again.  The workspace made under this owner during the capture comes from the graph's own memory pool, belongs
+        # to this graph alone and is kept alive with it.
         _scope.owner = id(self)
 
         def drop_owned():
-            with enc._bufs_lock:
-                for key in [k for k in enc._bufs if k[3] == id(self)]:
-                    del enc._bufs[key]
             with _lock:
                 for key in [k for k in _workspaces if k[3] == id(self)]:
                     del _workspaces[key]
@@ -496,8 +520,6 @@ class GraphedEncoder:
                 self.out = enc(self.x, self.mask, self.attn, sync_count=False, rows_bound=max_valid_tokens)
             with _lock:
                 self._held = [ws for key, ws in _workspaces.items() if key[3] == id(self)]
-            with enc._bufs_lock:
-                self._held += [t for key, bufs in enc._bufs.items() if key[3] == id(self) for t in bufs if t is not None]
         finally:
             _scope.owner = None
             drop_owned()

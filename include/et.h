@@ -214,6 +214,35 @@ et_status et_embedding_input(et_handle h, et_dtype dtype, const et_embedding_wei
                              int batch_size, int seq_len, int head_num, int size_per_head,
                              void* workspace, size_t workspace_bytes, void* stream, int32_t* valid_word_num_host);
 
+/* One batch of et_encoder.  Zero-initialise it and set what applies. */
+typedef struct et_encoder_batch {
+  const void* from_tensor;                 /* [B,S,H] in dtype, or NULL when the batch comes as token ids: */
+  const et_embedding_weights* embeddings;  /* the tables, and */
+  const int32_t* input_ids;                /* int32 [B,S] */
+  const int32_t* token_type_ids;           /* int32 [B,S], or NULL without a token-type table */
+  const int32_t* mask;                     /* int32 [B,S], 0/1 */
+  const void* attr_mask;                   /* [B,S,S] in dtype, 1 = attend */
+  void* out;                               /* [B,S,H] in dtype, zeros at padding */
+  int batch_size, seq_len;
+  int rows_bound;                          /* > 0: upper bound of the valid tokens that the caller vouches for (launches are
+                                              sized for it); 0: not known */
+  uint64_t* count_word;                    /* optional: 8 bytes of pinned host memory the GPU can write, one word for each
+                                              stream that may have calls in flight */
+  int32_t* valid_word_num;                 /* optional: receives the valid-token count; the call then waits for it */
+} et_encoder_batch;
+
+/* Input -> num_layers x Layer -> Output in one call: what python/effective_transformer/__init__.py:40-84 strings together
+ * from the three ops, with the index arrays, the sequence table and the activations in the workspace
+ * (et_encoder_workspace_bytes).  weights, prepared (may be NULL; its seq_start members are not used): one per layer.  Same
+ * results as the ops called one by one, bit for bit.
+ * With count_word (and rows_bound 0) the host waits for the valid-token count behind the launches of the first layer where
+ * that makes the launches of the others smaller; without it nothing is waited for and every launch is sized for B*S rows
+ * and bounded on the device (what a call under graph capture needs). */
+size_t et_encoder_workspace_bytes(et_dtype dtype, int batch_size, int seq_len, int head_num, int size_per_head);
+et_status et_encoder(et_handle h, et_dtype dtype, int num_layers, const et_layer_weights* weights,
+                     const et_layer_prepared* prepared, const et_encoder_batch* batch, int head_num, int size_per_head,
+                     void* workspace, size_t workspace_bytes, void* stream);
+
 /* The consumer side of the same fusion: the first token of every sequence straight from the packed matrix, i.e.
  * what `sequence_output[:, 0:1, :]` (the pooler's input, sample/tensorflow/modeling.py:224-232) reads after
  * EffectiveTransformerOutput, without materialising the padded [B,S,H] tensor.

@@ -112,67 +112,36 @@ class Encoder {
   }
 
   ~Encoder() {
-    if (host_count_) (void)hipHostFree(host_count_);
-    if (copied_) (void)hipEventDestroy(copied_);
+    if (count_word_) (void)hipHostFree(count_word_);
   }
   Encoder(const Encoder&) = delete;
   Encoder& operator=(const Encoder&) = delete;
 
   // from_tensor [B,S,H], mask int32 [B,S], attr_mask [B,S,S] in dtype -> out [B,S,H] (zeros at padding).
-  // sync_count: read the valid-token count back once per batch, so that the launches of layers 2 .. L are sized
-  // exactly (the reference reads it back in every layer), or leave it on the device (launches sized for B*S rows).
-  // The copy is asynchronous and the host waits for it behind the launches of the first layer, which is sized for
-  // B*S rows and bounded on the device, so the GPU never idles for the read-back.
+  // sync_count: the valid-token count is read back once per batch, so that the launches of layers 2 .. L are sized
+  // exactly (the reference reads it back in every layer), or left on the device (launches sized for B*S rows); the host
+  // waits for it behind the launches of the first layer, so the GPU never idles for the read-back.
   // Returns the valid-token count, or -1 when it was not read back.
   int forward(const void* from_tensor, const int32_t* mask, const void* attr_mask, void* out, int batch, int seq_len,
               hipStream_t stream, bool sync_count = true) {
-    const size_t e = dtype_ == ET_FP32 ? 4 : 2;
-    const size_t H = (size_t)heads_ * d_, rows = (size_t)batch * seq_len;
-    char* act = (char*)act_.reserve(3 * rows * H * e);                 // packed input + two layer outputs
-    // batch_idx, word_idx, the count, then the sequence table (2 B + 1 words)
-    int32_t* idx = (int32_t*)idx_.reserve((2 * rows + 1) * sizeof(int32_t) + et_seq_workspace_bytes(batch));
-    int32_t *batch_idx = idx, *word_idx = idx + rows, *count = idx + 2 * rows, *starts = idx + 2 * rows + 1;
-    const size_t in_ws = et_input_workspace_bytes(batch, seq_len);
-    const size_t layer_ws = et_layer_workspace_bytes(dtype_, batch, seq_len, heads_, d_);
-    void* ws = ws_.reserve(in_ws > layer_ws ? in_ws : layer_ws);
-    int32_t host_count = -1;
-    check(et_input(handle_.get(), dtype_, from_tensor, mask, act, count, batch_idx, word_idx, batch, seq_len, heads_, d_, ws,
-                   ws_.capacity(), stream, nullptr),
-          handle_.get());
-    bool pending = false;
+    et_encoder_batch b = {};
+    b.from_tensor = from_tensor;
+    b.mask = mask;
+    b.attr_mask = attr_mask;
+    b.out = out;
+    b.batch_size = batch;
+    b.seq_len = seq_len;
+    int32_t count = -1;
     if (sync_count) {
-      if (!host_count_) check_hip(hipHostMalloc((void**)&host_count_, sizeof(int32_t), hipHostMallocDefault), "hipHostMalloc");
-      if (!copied_) check_hip(hipEventCreateWithFlags(&copied_, hipEventDisableTiming), "hipEventCreate");
-      check_hip(hipMemcpyAsync(host_count_, count, sizeof(int32_t), hipMemcpyDeviceToHost, stream), "hipMemcpyAsync");
-      check_hip(hipEventRecord(copied_, stream), "hipEventRecord");
-      pending = true;
+      if (!count_word_) check_hip(hipHostMalloc((void**)&count_word_, sizeof(uint64_t), hipHostMallocDefault), "hipHostMalloc");
+      b.count_word = count_word_;
+      b.valid_word_num = &count;
     }
-    // one sequence start table serves every layer of the batch
-    check(et_sequence_starts(handle_.get(), batch_idx, count, batch, seq_len, starts, et_seq_workspace_bytes(batch), stream),
+    void* ws = ws_.reserve(et_encoder_workspace_bytes(dtype_, batch, seq_len, heads_, d_));
+    check(et_encoder(handle_.get(), dtype_, (int)layers_.size(), layers_.data(), prepared_.data(), &b, heads_, d_, ws,
+                     ws_.capacity(), stream),
           handle_.get());
-    const char* x = act;
-    for (size_t l = 0; l < layers_.size(); ++l) {
-      if (l == 1 && pending) {       // the first layer is in the queue: waiting here leaves the GPU with work
-        check_hip(hipEventSynchronize(copied_), "hipEventSynchronize");
-        host_count = *host_count_;
-        pending = false;
-      }
-      char* y = act + (1 + (l & 1)) * rows * H * e;
-      et_layer_prepared prep = prepared_[l];
-      prep.seq_start = starts;
-      prep.seq_start_bytes = et_seq_workspace_bytes(batch);
-      check(et_layer_with_prepared(handle_.get(), dtype_, &layers_[l], &prep, x, x, attr_mask, count, batch_idx, word_idx, y,
-                                   batch, seq_len, seq_len, heads_, d_, host_count, ws, ws_.capacity(), stream),
-            handle_.get());
-      x = y;
-    }
-    check(et_output(handle_.get(), dtype_, x, count, batch_idx, word_idx, out, batch, seq_len, heads_, d_, stream),
-          handle_.get());
-    if (pending) {                   // a single layer: nothing needed the count, the caller still gets it
-      check_hip(hipEventSynchronize(copied_), "hipEventSynchronize");
-      host_count = *host_count_;
-    }
-    return host_count;
+    return count;
   }
 
  private:
@@ -181,9 +150,8 @@ class Encoder {
   int heads_, d_;
   std::vector<et_layer_weights> layers_;
   std::vector<et_layer_prepared> prepared_;
-  DeviceBuffer act_, idx_, ws_, wt_;
-  int32_t* host_count_ = nullptr;      // pinned
-  hipEvent_t copied_ = nullptr;
+  DeviceBuffer ws_, wt_;
+  uint64_t* count_word_ = nullptr;     // pinned
 };
 
 }  // namespace et
