@@ -403,20 +403,19 @@ et_status run_layer(et_handle h, const LayerCall& c) {
   g1.b_transposed = t_o;
   gemm(g1, attn, H, H, H);
   // Every weight matrix was last read a whole batch ago, and a GEMM's first round of tiles waits for each cold slice of
-  // it (13000 rows: FFN-down 63 us with cold weights, 53 with the weights in the last-level cache; 2 .. 3 us for the
-  // other projections).  The two LayerNorm kernels request the matrices that come next on their way, for batches in
-  // which those are small beside what the kernel moves anyway: this one the FFN-up weights and, while the layer's
-  // matrices are small enough for them to survive FFN-up, the FFN-down weights (12-layer BERT-base: -3 % at 4000
-  // tokens, -4.4 % at 8000 and 12000, -1 % at 16000); the last one the region the caller names, the next layer's
-  // attention weights (another -0.7 .. -1.6 % from 4000 to 40000 tokens, FFN-up included).
+  // it (13000 rows: FFN-down 63 us with cold weights, 53 with the weights in the last-level cache; 2000 rows: 20 and
+  // 15.6 us).  The two LayerNorm kernels request the matrices that come next on their way: this one the FFN-up weights
+  // and, while the layer's matrices are small enough for them to survive FFN-up, the FFN-down weights; the last one the
+  // region the caller names, the next layer's attention weights (12-layer BERT-base on three models' weights in turn:
+  // -5 % at 700 tokens, -11 % at 2000, -4 % at 8000, -1 % at 16000).
   const bool warm_fits = (double)rows * (7.0 * H + F) * (double)e <= kWarmLayerBytes;
   et::WarmList warm1, warm2;
   // (whichever copy the GEMM reads, unless this call has just written it)
   const void* b_up = t_up ? wt_up : w->inter_kernel;
   const void* b_down = t_down ? wt_down : w->output_kernel;
-  if (rows >= F && !(t_up && !pp.inter_kernel_t)) warm1.add(b_up, (size_t)H * F * (split ? 6 : e));
-  if (rows >= F && warm_fits && !(t_down && !pp.output_kernel_t)) warm1.add(b_down, (size_t)H * F * (split ? 6 : e));
-  if (rows >= F) warm2.add(pp.warm, pp.warm_bytes);
+  if (!(t_up && !pp.inter_kernel_t)) warm1.add(b_up, (size_t)H * F * (split ? 6 : e));
+  if (warm_fits && !(t_down && !pp.output_kernel_t)) warm1.add(b_down, (size_t)H * F * (split ? 6 : e));
+  warm2.add(pp.warm, pp.warm_bytes);
   // (split layers: the row kernel leaves its output as split rows too; rows it cannot hold in registers take a pass)
   const bool ln_split = split && et::layernorm_row_in_registers(dt, H);
   uint16_t* attn_split = (uint16_t*)(base + ws.attn_split);

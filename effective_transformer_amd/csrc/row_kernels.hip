@@ -316,8 +316,10 @@ void ln_launch(void* out, const void* input, const void* bias, const void* gamma
                const int32_t* rows_dev, hipStream_t stream, const WarmList& warm, uint16_t* split) {
   int vec = 0, iters = 0;
   if (!ln_pick<T>(n, vec, iters)) return;
-  // enough wavefronts to fill 256 CUs several times over; rows beyond that are looped
-  const int grid = (int)min((long)(m + kLnWaves - 1) / kLnWaves, 256L * 8);
+  // enough wavefronts to fill 256 CUs several times over; rows beyond that are looped.  A list of lines to request brings
+  // as many threads as it has lines (up to the same bound): few rows must not be held up by a long list.
+  const long lines = (warm.total + kLnThreads - 1) / kLnThreads;
+  const int grid = (int)min(max((long)(m + kLnWaves - 1) / kLnWaves, lines), 256L * 8);
   T* o = (T*)out;
   const T *i = (const T*)input, *b = (const T*)bias, *g = (const T*)gamma, *be = (const T*)beta;
   constexpr int MV = 16 / (int)sizeof(T);
