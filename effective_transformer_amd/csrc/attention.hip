@@ -10,6 +10,8 @@
 // Softmax semantics (both kernels): t = qk*scale + (1-mask)*(-10000); m = max(max_k t, 0);
 // e = exp(t-m); p = e / (sum e + 1e-6).  In fp16 the score is rounded to half before the softmax
 // and the probability after it, as the reference stores both in half.
+#include <type_traits>
+
 #include "et_device.hpp"
 #include "kernels.hpp"
 
@@ -570,35 +572,34 @@ void attention_launch(const void* q, const void* k, const void* v, int layout, i
 
 
 // ------------------------------------------------------------------------------------------
-// fused attention for 128 < seq_len <= 512: one workgroup (4 wavefronts) per (64 queries, head, sequence).
+// fp32 fused attention for 128 < seq_len <= 512: one workgroup (4 wavefronts) per (64 queries, head, sequence).
 // The scores of a wavefront's 16 queries against all keys stay in registers (4 per lane and 16-key tile); K and
 // V pass through LDS in chunks of 128 keys (K chunks first, the softmax over the registers, then V chunks), so the
 // LDS footprint does not grow with the sequence.  Q comes straight from global memory: the MFMA operand of a lane
-// is 16 (fp16) or 64 (fp32) contiguous bytes of its query's row.  Arithmetic and rounding points are those of
+// is 64 contiguous bytes of its query's row.  Arithmetic and rounding points are those of
 // the kernel above; key tiles beyond the last token skip their MFMAs (score 0, value 0).
 // ------------------------------------------------------------------------------------------
 constexpr int kLongChunkTiles = 8;                 // 128 keys per LDS chunk
 constexpr int kLongChunk = kLongChunkTiles * 16;
 
-template <typename T>
 struct LongSmem {
-  static constexpr int kQS = AttnCfg<T>::kQkStride;
-  static constexpr int kVR = AttnCfg<_Float16>::kVStride;              // fp16 V rows
-  static constexpr int kVS = kLongChunk + AttnCfg<T>::kVtPad;          // fp32 V^T rows
-  static constexpr size_t kKBytes = (size_t)kLongChunk * kQS * sizeof(T);
-  static constexpr size_t kVBytes = sizeof(T) == 2 ? (size_t)kLongChunk * kVR * sizeof(T) : (size_t)kD * kVS * sizeof(T);
+  static constexpr int kQS = AttnCfg<float>::kQkStride;
+  static constexpr int kVS = kLongChunk + AttnCfg<float>::kVtPad;      // V^T rows
+  static constexpr size_t kKBytes = (size_t)kLongChunk * kQS * sizeof(float);
+  static constexpr size_t kVBytes = (size_t)kD * kVS * sizeof(float);
   static constexpr size_t kTileBytes = kKBytes > kVBytes ? kKBytes : kVBytes;   // K and V chunks take turns
 };
 
-template <typename T, int NKT>
+template <int NKT>
 __global__ __launch_bounds__(kAttnThreads) void attention_long_kernel(
-    const T* __restrict__ q_src, const T* __restrict__ k_src, const T* __restrict__ v_src, int layout, int packed_ld,
-    const T* __restrict__ attr_mask, T* __restrict__ dst, const int32_t* __restrict__ seq_start,
+    const float* __restrict__ q_src, const float* __restrict__ k_src, const float* __restrict__ v_src, int layout,
+    int packed_ld, const float* __restrict__ attr_mask, float* __restrict__ dst, const int32_t* __restrict__ seq_start,
     const int32_t* __restrict__ word_idx, int batch, int seq_len, int heads, float scaler, int split_out) {
-  using Sm = LongSmem<T>;
+  using T = float;
+  using Sm = LongSmem;
   using C = Chunk16<T>;
   using V16 = typename C::vec;
-  constexpr int kQS = Sm::kQS, kVR = Sm::kVR, kVS = Sm::kVS;
+  constexpr int kQS = Sm::kQS, kVS = Sm::kVS;
   constexpr int kSp = NKT * 16;
   constexpr int kCpr = kD / C::kElems;
   constexpr int kChunks = NKT / kLongChunkTiles;
@@ -664,23 +665,13 @@ __global__ __launch_bounds__(kAttnThreads) void attention_long_kernel(
   const bool vec_mask = (seq_len & 3) == 0;
 
   // Q operand of this lane (zeros for a query position without a token: its result is never stored)
-  half8 bqh[2];
   float bqf[16];
-  if constexpr (sizeof(T) == 2) {
 #pragma unroll
-    for (int ks = 0; ks < 2; ++ks) {
+  for (int i = 0; i < 4; ++i) {
+    float4v v4 = {0.f, 0.f, 0.f, 0.f};
+    if (tq >= 0) v4 = *reinterpret_cast<const float4v*>(q_src + src_off(tq, q) + g * 16 + i * 4);
 #pragma unroll
-      for (int j = 0; j < 8; ++j) bqh[ks][j] = (_Float16)0;
-      if (tq >= 0) bqh[ks] = *reinterpret_cast<const half8*>(q_src + src_off(tq, q) + ks * 32 + g * 8);
-    }
-  } else {
-#pragma unroll
-    for (int i = 0; i < 4; ++i) {
-      float4v v4 = {0.f, 0.f, 0.f, 0.f};
-      if (tq >= 0) v4 = *reinterpret_cast<const float4v*>(q_src + src_off(tq, q) + g * 16 + i * 4);
-#pragma unroll
-      for (int j = 0; j < 4; ++j) bqf[i * 4 + j] = v4[j];
-    }
+    for (int j = 0; j < 4; ++j) bqf[i * 4 + j] = v4[j];
   }
 
   // ---- S^T = K Q^T chunk by chunk, bias added on the way ------------------------------------------
@@ -699,19 +690,11 @@ __global__ __launch_bounds__(kAttnThreads) void attention_long_kernel(
         const int kt = ch * kLongChunkTiles + kc;
         float4v acc = {0.f, 0.f, 0.f, 0.f};
         if (kt < n_tiles) {
-          if constexpr (sizeof(T) == 2) {
 #pragma unroll
-            for (int ks = 0; ks < 2; ++ks) {
-              const half8 a = *reinterpret_cast<const half8*>(Ks + (kc * 16 + l16) * kQS + ks * 32 + g * 8);
-              acc = __builtin_amdgcn_mfma_f32_16x16x32_f16(a, bqh[ks], acc, 0, 0, 0);
-            }
-          } else {
+          for (int i = 0; i < 4; ++i) {
+            const float4v a4 = *reinterpret_cast<const float4v*>(Ks + (kc * 16 + l16) * kQS + g * 16 + i * 4);
 #pragma unroll
-            for (int i = 0; i < 4; ++i) {
-              const float4v a4 = *reinterpret_cast<const float4v*>(Ks + (kc * 16 + l16) * kQS + g * 16 + i * 4);
-#pragma unroll
-              for (int j = 0; j < 4; ++j) acc = __builtin_amdgcn_mfma_f32_16x16x4f32(a4[j], bqf[i * 4 + j], acc, 0, 0, 0);
-            }
+            for (int j = 0; j < 4; ++j) acc = __builtin_amdgcn_mfma_f32_16x16x4f32(a4[j], bqf[i * 4 + j], acc, 0, 0, 0);
           }
         }
         const int key0 = kt * 16 + g * 4;
@@ -725,8 +708,7 @@ __global__ __launch_bounds__(kAttnThreads) void attention_long_kernel(
         }
 #pragma unroll
         for (int r = 0; r < 4; ++r) {
-          const float sc = sizeof(T) == 2 ? h2f(f2h(acc[r])) : acc[r];      // the score is stored in the element type
-          s[kt][r] = key0 + r < seq_len ? sc * scaler + (1.0f - (float)m4[r]) * -10000.0f : -INFINITY;
+          s[kt][r] = key0 + r < seq_len ? acc[r] * scaler + (1.0f - (float)m4[r]) * -10000.0f : -INFINITY;
         }
       }
     }
@@ -764,113 +746,61 @@ __global__ __launch_bounds__(kAttnThreads) void attention_long_kernel(
   for (int ch = 0; ch < kChunks; ++ch) {
     if (ch * kLongChunkTiles >= n_tiles) break;                         // workgroup-uniform: no token, value 0
     __syncthreads();
-    if constexpr (sizeof(T) == 2) {
-      stage_rows(v_src, Vs, kVR, ch * kLongChunk);
-    } else {
-      // fp32 keeps V^T: feature rows, key columns
+    // fp32 keeps V^T: feature rows, key columns
 #pragma unroll
-      for (int k = 0; k < CPT; ++k) {
-        const int i = threadIdx.x + k * kAttnThreads;
-        const int row = i / kCpr, c = i - row * kCpr;
-        const int pos = ch * kLongChunk + row;
-        const int tk = pos < kSp ? tok_of_pos[pos] : -1;
-        V16 r = {0.f, 0.f, 0.f, 0.f};
-        if (tk >= 0) r = *reinterpret_cast<const V16*>(v_src + src_off(tk, pos) + c * C::kElems);
+    for (int k = 0; k < CPT; ++k) {
+      const int i = threadIdx.x + k * kAttnThreads;
+      const int row = i / kCpr, c = i - row * kCpr;
+      const int pos = ch * kLongChunk + row;
+      const int tk = pos < kSp ? tok_of_pos[pos] : -1;
+      V16 r = {0.f, 0.f, 0.f, 0.f};
+      if (tk >= 0) r = *reinterpret_cast<const V16*>(v_src + src_off(tk, pos) + c * C::kElems);
 #pragma unroll
-        for (int j = 0; j < C::kElems; ++j) Vs[(c * C::kElems + j) * kVS + row] = r[j];
-      }
+      for (int j = 0; j < C::kElems; ++j) Vs[(c * C::kElems + j) * kVS + row] = r[j];
     }
     __syncthreads();
     if (!active) continue;
-    if constexpr (sizeof(T) == 2) {
 #pragma unroll
-      for (int kp = 0; kp < kLongChunkTiles / 2; ++kp) {
-        const int kt = ch * kLongChunkTiles + 2 * kp;
-        if (kt < n_tiles) {
-          half8 p;
+    for (int kc = 0; kc < kLongChunkTiles; ++kc) {
+      const int kt = ch * kLongChunkTiles + kc;
+      if (kt < n_tiles) {
 #pragma unroll
-          for (int r = 0; r < 4; ++r) {
-            p[r] = f2h(s[kt][r]);
-            p[4 + r] = f2h(s[kt + 1][r]);
-          }
-          typedef uint32_t u2 __attribute__((ext_vector_type(2)));
-          typedef uint32_t u4 __attribute__((ext_vector_type(4)));
-          u2 raw[8];
+        for (int dt = 0; dt < 4; ++dt) {
+          const float4v a4 = *reinterpret_cast<const float4v*>(Vs + (dt * 16 + l16) * kVS + kc * 16 + g * 4);
 #pragma unroll
-          for (int kk = 0; kk < 8; ++kk) {
-            const int key = kp * 32 + (kk >> 2) * 16 + g * 4 + (kk & 3);
-            raw[kk] = *reinterpret_cast<const u2*>(Vs + key * kVR + l16 * 4);
-          }
-#pragma unroll
-          for (int jj = 0; jj < 2; ++jj) {
-            u4 lo, hi;
-#pragma unroll
-            for (int q4 = 0; q4 < 4; ++q4) {
-              lo[q4] = __builtin_amdgcn_perm(raw[2 * q4 + 1][jj], raw[2 * q4][jj], 0x05040100u);
-              hi[q4] = __builtin_amdgcn_perm(raw[2 * q4 + 1][jj], raw[2 * q4][jj], 0x07060302u);
-            }
-            o[2 * jj] = __builtin_amdgcn_mfma_f32_16x16x32_f16(__builtin_bit_cast(half8, lo), p, o[2 * jj], 0, 0, 0);
-            o[2 * jj + 1] = __builtin_amdgcn_mfma_f32_16x16x32_f16(__builtin_bit_cast(half8, hi), p, o[2 * jj + 1], 0, 0, 0);
-          }
-        }
-      }
-    } else {
-#pragma unroll
-      for (int kc = 0; kc < kLongChunkTiles; ++kc) {
-        const int kt = ch * kLongChunkTiles + kc;
-        if (kt < n_tiles) {
-#pragma unroll
-          for (int dt = 0; dt < 4; ++dt) {
-            const float4v a4 = *reinterpret_cast<const float4v*>(Vs + (dt * 16 + l16) * kVS + kc * 16 + g * 4);
-#pragma unroll
-            for (int r = 0; r < 4; ++r) o[dt] = __builtin_amdgcn_mfma_f32_16x16x4f32(a4[r], s[kt][r], o[dt], 0, 0, 0);
-          }
+          for (int r = 0; r < 4; ++r) o[dt] = __builtin_amdgcn_mfma_f32_16x16x4f32(a4[r], s[kt][r], o[dt], 0, 0, 0);
         }
       }
     }
   }
 
   if (tq >= 0) {
-    if constexpr (sizeof(T) == 2) {
-      half8 v0, v1;
+    T* orow = dst + (size_t)tq * H + head * kD + g * 4;
 #pragma unroll
-      for (int r = 0; r < 2; ++r)
+    for (int dt = 0; dt < 4; ++dt) {
+      float4v v;
 #pragma unroll
-        for (int j = 0; j < 4; ++j) {
-          v0[4 * r + j] = f2h(o[j][r]);
-          v1[4 * r + j] = f2h(o[j][2 + r]);
-        }
-      T* orow = dst + (size_t)tq * H + head * kD + g * 16;
-      *reinterpret_cast<half8*>(orow) = v0;
-      *reinterpret_cast<half8*>(orow + 8) = v1;
-    } else {
-      T* orow = dst + (size_t)tq * H + head * kD + g * 4;
-#pragma unroll
-      for (int dt = 0; dt < 4; ++dt) {
-        float4v v;
-#pragma unroll
-        for (int r = 0; r < 4; ++r) v[r] = o[dt][r];
-        if (split_out) store_split<4>(reinterpret_cast<uint16_t*>(dst) + (size_t)tq * 3 * H, head * kD + dt * 16 + g * 4, v);
-        else *reinterpret_cast<float4v*>(orow + dt * 16) = v;
-      }
+      for (int r = 0; r < 4; ++r) v[r] = o[dt][r];
+      if (split_out) store_split<4>(reinterpret_cast<uint16_t*>(dst) + (size_t)tq * 3 * H, head * kD + dt * 16 + g * 4, v);
+      else *reinterpret_cast<float4v*>(orow + dt * 16) = v;
     }
   }
 }
 
-template <typename T, int NKT>
+template <int NKT>
 void attention_long_launch(const void* q, const void* k, const void* v, int layout, int packed_ld, const void* attr_mask,
                            void* dst, const int32_t* seq_start, const int32_t* word_idx, int batch, int seq_len, int heads,
                            float scaler, bool split_out, hipStream_t stream) {
-  const size_t smem = LongSmem<T>::kTileBytes + (size_t)NKT * 16 * sizeof(int);
-  auto kern = attention_long_kernel<T, NKT>;
+  const size_t smem = LongSmem::kTileBytes + (size_t)NKT * 16 * sizeof(int);
+  auto kern = attention_long_kernel<NKT>;
   dim3 grid((seq_len + 63) / 64, heads, batch);               // blocks of 64 queries that can hold a token
-  kern<<<grid, kAttnThreads, smem, stream>>>((const T*)q, (const T*)k, (const T*)v, layout, packed_ld, (const T*)attr_mask,
-                                             (T*)dst, seq_start, word_idx, batch, seq_len, heads, scaler,
+  kern<<<grid, kAttnThreads, smem, stream>>>((const float*)q, (const float*)k, (const float*)v, layout, packed_ld, (const float*)attr_mask,
+                                             (float*)dst, seq_start, word_idx, batch, seq_len, heads, scaler,
                                              split_out ? 1 : 0);
 }
 
 // ------------------------------------------------------------------------------------------
-// K / V rows brought into LDS by DMA (the resident-key kernels below): rows of 128 bytes without padding, one
+// K / V rows brought into LDS by DMA (the streaming kernel below): rows of 128 bytes without padding, one
 // `buffer_load ... lds` instruction fills eight of them (lane -> row lane / 8, 16-byte chunk lane & 7).  A row without
 // a token is requested beyond its buffer descriptor's range and arrives as zeros.
 // Which key a row of an MFMA tile stands for is free as long as K, the mask and V agree: row m of the first tile of a
@@ -885,261 +815,8 @@ __device__ __forceinline__ int wide_slot(int key) { return key ^ ((key >> 3) & 1
 __device__ __forceinline__ int wide_swizzle(int slot) { return ((slot >> 1) & 1) | ((slot >> 2) & 6); }
 // s_waitcnt immediates of gfx9: vmcnt[3:0] | expcnt[6:4] | lgkmcnt[11:8] | vmcnt[5:4] at [15:14]
 __device__ __forceinline__ void wide_wait_dma() { __builtin_amdgcn_s_waitcnt(0 | (7 << 4) | (15 << 8) | (0 << 14)); }
-__device__ __forceinline__ void wide_wait_lds() { __builtin_amdgcn_s_waitcnt(15 | (7 << 4) | (0 << 8) | (3 << 14)); }
 // barrier without the fence of __syncthreads(), which would wait for every DMA in flight
 __device__ __forceinline__ void wide_barrier() { asm volatile("s_barrier" ::: "memory"); }
-
-// ------------------------------------------------------------------------------------------
-// fp16 fused attention for 128 < seq_len <= 512 with K and V of the whole sequence resident in LDS: one workgroup of
-// 8 wavefronts per (head, sequence) (or per share of its query tiles, see `qsplit`).  K and V arrive once by DMA (64 +
-// 64 KB at 512 keys, all requests in flight at once, layout above) instead of once per block of 64 queries, and after
-// that one barrier the wavefronts run their 16-query tiles independently: S^T = K Q^T over all key tiles, the softmax
-// over the registers, O^T = V^T P^T.  Arithmetic and rounding points per element are those of attention_long_kernel.
-// ------------------------------------------------------------------------------------------
-constexpr int kResThreads = 512;
-[[maybe_unused]] constexpr int kResWaves = kResThreads / kWave;
-
-template <int NKT>
-struct ResSmem {
-  static constexpr int kSp = NKT * 16;
-  static constexpr size_t kKBytes = (size_t)kSp * 128;
-  static constexpr size_t kVBytes = (size_t)kSp * 128;
-  static constexpr size_t kBytes = kKBytes + kVBytes + (size_t)kSp * sizeof(int);
-};
-
-template <int NKT>
-__global__ __launch_bounds__(kResThreads) __attribute__((amdgpu_waves_per_eu(NKT <= 16 ? 4 : 2, NKT <= 16 ? 4 : 2)))
-void attention_resident_kernel(
-    const _Float16* __restrict__ q_src, const _Float16* __restrict__ k_src, const _Float16* __restrict__ v_src, int layout,
-    int packed_ld, const _Float16* __restrict__ attr_mask, _Float16* __restrict__ dst,
-    const int32_t* __restrict__ seq_start, const int32_t* __restrict__ word_idx, int batch, int seq_len, int heads,
-    int qsplit, float scaler) {
-#if defined(__HIP_DEVICE_COMPILE__)   // device-only types in the body; the host pass only needs the stub
-  using T = _Float16;
-  using Sm = ResSmem<NKT>;
-  constexpr int kSp = Sm::kSp;
-
-  extern __shared__ __attribute__((aligned(1024))) unsigned char smem_raw[];
-  unsigned char* ks = smem_raw;
-  unsigned char* vs = smem_raw + Sm::kKBytes;
-  int* tok_of_pos = reinterpret_cast<int*>(smem_raw + Sm::kKBytes + Sm::kVBytes);
-
-  const int b = min(max(seq_start[batch + 1 + blockIdx.y], 0), batch - 1);
-  const int head = blockIdx.x / qsplit, part = blockIdx.x - head * qsplit;
-  const int t0 = seq_start[b], t1 = seq_start[b + 1];
-  const int len = t1 - t0;
-  if (len <= 0) return;
-  const int H = heads * kD;
-  const int lane = threadIdx.x & (kWave - 1);
-  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x / kWave);
-  const int l16 = lane & 15, g = lane >> 4;
-
-  const int last_pos = min(max(word_idx[t1 - 1], 0), seq_len - 1);
-  const int n_tiles = last_pos / 16 + 1;                     // 16-row tiles that hold at least one token
-  if (part >= n_tiles) return;                               // no query tile for this share (workgroup-uniform)
-  for (int i = threadIdx.x; i < kSp; i += kResThreads) tok_of_pos[i] = -1;
-  __syncthreads();
-  for (int tt = threadIdx.x; tt < len; tt += kResThreads) {
-    const int pos = word_idx[t0 + tt];
-    if (pos >= 0 && pos < seq_len) tok_of_pos[pos] = tt;     // relative to the sequence's first packed row
-  }
-  __syncthreads();
-
-  // K and V rows of every group of four key tiles that holds a token (the loops below run over such groups)
-  const int n_groups = (n_tiles + 3) / 4;
-  {
-    const int rows_in = min(kSp, n_groups * 64);
-    const T* kbase = layout == 1 ? k_src + (size_t)t0 * packed_ld + head * kD : k_src + ((size_t)b * heads + head) * seq_len * kD;
-    const T* vbase = layout == 1 ? v_src + (size_t)t0 * packed_ld + head * kD : v_src + ((size_t)b * heads + head) * seq_len * kD;
-    const uint32_t bytes = layout == 1 ? ((uint32_t)(len - 1) * (uint32_t)packed_ld + kD) * 2u : (uint32_t)seq_len * kD * 2u;
-    const __amdgpu_buffer_rsrc_t rk = __builtin_amdgcn_make_buffer_rsrc(const_cast<T*>(kbase), 0, (int)bytes, 0x00020000);
-    const __amdgpu_buffer_rsrc_t rv = __builtin_amdgcn_make_buffer_rsrc(const_cast<T*>(vbase), 0, (int)bytes, 0x00020000);
-    for (int i = wave; i < rows_in / 8; i += kResWaves) {
-      const int slot = i * 8 + (lane >> 3);
-      const int key = wide_slot(slot);
-      const int c = (lane & 7) ^ wide_swizzle(slot);
-      const int tk = tok_of_pos[key];
-      const uint32_t row_off = layout == 1 ? (uint32_t)tk * (uint32_t)packed_ld : (uint32_t)key * kD;
-      const uint32_t voff = tk >= 0 ? (row_off + (uint32_t)c * 8u) * 2u : 0x80000000u;      // out of range: zeros
-      __builtin_amdgcn_raw_ptr_buffer_load_lds(rk, ET_ATTN_LDS_PTR(ks + i * 1024), 16, voff, 0, 0, 0);
-      __builtin_amdgcn_raw_ptr_buffer_load_lds(rv, ET_ATTN_LDS_PTR(vs + i * 1024), 16, voff, 0, 0, 0);
-    }
-  }
-  wide_wait_dma();
-  __syncthreads();
-
-  // Operand addresses: a lane-dependent base plus a compile-time offset per tile.  The slot flip touches bit 0 of the
-  // row and the swizzle bits 1, 3, 4, none of which the tile's part of the row number (multiples of 32, +4 for the
-  // second tile of a pair) reaches, so both are constants of the lane.
-  //   K, row l16 of a tile: key row L = (l16 >> 2) * 8 + (l16 & 3) within the pair, chunk ks * 4 + g
-  const unsigned char* kbase_ks[2];
-  {
-    const int L = wide_slot((l16 >> 2) * 8 + (l16 & 3));
-    const int sw = wide_swizzle(L);
-#pragma unroll
-    for (int ks2 = 0; ks2 < 2; ++ks2) kbase_ks[ks2] = ks + L * 128 + (((ks2 * 4 + g) ^ sw) * 16);
-  }
-  //   V, key g * 8 + kk of a pair (kk = 4 a + 2 b + c), features 4 l16 ..: base by (b, c), offset 512 a
-  const unsigned char* vbase_bc[2][2];
-#pragma unroll
-  for (int bb = 0; bb < 2; ++bb)
-#pragma unroll
-    for (int cc = 0; cc < 2; ++cc) {
-      const int slot = wide_slot(g * 8 + 2 * bb + cc);
-      vbase_bc[bb][cc] = vs + slot * 128 + (((l16 >> 1) ^ wide_swizzle(slot)) * 16) + (l16 & 1) * 8;
-    }
-
-  const bool vec_mask = (seq_len & 7) == 0;                  // mask rows start at multiples of 16 bytes
-  for (int qt = part + qsplit * wave; qt < n_tiles; qt += qsplit * kResWaves) {
-    const int q = qt * 16 + l16;
-    const int tq = tok_of_pos[q];
-    const T* mrow = attr_mask + ((size_t)b * seq_len + min(q, seq_len - 1)) * seq_len;
-    // Q operand of this lane (zeros for a query position without a token: its result is never stored)
-    half8 bqh[2];
-#pragma unroll
-    for (int ks2 = 0; ks2 < 2; ++ks2) {
-#pragma unroll
-      for (int j = 0; j < 8; ++j) bqh[ks2][j] = (_Float16)0;
-      if (tq >= 0) {
-        const size_t qo = layout == 1 ? (size_t)(t0 + tq) * packed_ld + head * kD
-                                      : (((size_t)b * heads + head) * seq_len + q) * kD;
-        bqh[ks2] = *reinterpret_cast<const half8*>(q_src + qo + ks2 * 32 + g * 8);
-      }
-    }
-
-    // ---- the additive bias of the mask row first: the whole row requested before any of it is converted --------
-    float s[NKT][4];                                         // s[2 P], s[2 P + 1]: keys 32 P + 8 g + 0..3, + 4..7
-    // (opaque to the compiler, or it would keep the clamped offsets of all pairs in registers across query tiles)
-    int g8 = g * 8;
-    asm volatile("" : "+v"(g8));
-    // (1 - m) * -10000 as one fma: 1 - m is exact in float for a half m, so both forms round the same real number once
-    if (vec_mask) {
-      half8 m8[NKT / 2];
-#pragma unroll
-      for (int kp = 0; kp < NKT / 2; ++kp) m8[kp] = *reinterpret_cast<const half8*>(mrow + min(kp * 32 + g8, seq_len - 8));
-      __builtin_amdgcn_sched_barrier(0);
-#pragma unroll
-      for (int kp = 0; kp < NKT / 2; ++kp) {
-        const int key0 = kp * 32 + g8;
-        if ((kp + 1) * 32 <= seq_len) {                      // wave-uniform: every key of the pair exists
-#pragma unroll
-          for (int j = 0; j < 8; ++j) s[2 * kp + (j >> 2)][j & 3] = __builtin_fmaf((float)m8[kp][j], 10000.0f, -10000.0f);
-        } else {
-#pragma unroll
-          for (int j = 0; j < 8; ++j)
-            s[2 * kp + (j >> 2)][j & 3] = key0 < seq_len ? __builtin_fmaf((float)m8[kp][j], 10000.0f, -10000.0f) : -INFINITY;
-        }
-      }
-    } else {
-#pragma unroll
-      for (int kp = 0; kp < NKT / 2; ++kp) {
-        const int key0 = kp * 32 + g8;
-#pragma unroll
-        for (int j = 0; j < 8; ++j) {
-          const T m = mrow[min(key0 + j, seq_len - 1)];
-          s[2 * kp + (j >> 2)][j & 3] = key0 + j < seq_len ? __builtin_fmaf((float)m, 10000.0f, -10000.0f) : -INFINITY;
-        }
-        if (kp % 2 == 1) __builtin_amdgcn_sched_barrier(0);
-      }
-    }
-    // ---- S^T = K Q^T, four key tiles at a time (rows without a token are zero: score 0) ---------------------
-#pragma unroll
-    for (int kg = 0; kg < NKT / 4; ++kg) {
-      if (kg < n_groups) {
-#pragma unroll
-        for (int kc = 0; kc < 4; ++kc) {
-          const int kt = kg * 4 + kc;
-          // row l16 of tile kt: pair kt >> 1, first or second tile kt & 1 (4 rows further)
-          float4v acc = {0.f, 0.f, 0.f, 0.f};
-#pragma unroll
-          for (int ks2 = 0; ks2 < 2; ++ks2) {
-            const half8 a = *reinterpret_cast<const half8*>(kbase_ks[ks2] + ((kt & ~1) * 16 + (kt & 1) * 4) * 128);
-            acc = __builtin_amdgcn_mfma_f32_16x16x32_f16(a, bqh[ks2], acc, 0, 0, 0);
-          }
-#pragma unroll
-          for (int r = 0; r < 4; ++r) {
-            const float sc = h2f(f2h(acc[r]));                         // the score is stored in half
-            s[kt][r] = sc * scaler + s[kt][r];                         // -inf stays -inf for keys that do not exist
-          }
-        }
-      }
-    }
-
-    // ---- masked softmax over the registers ------------------------------------------------------------
-    {
-      float mx = 0.f;
-#pragma unroll
-      for (int kt = 0; kt < NKT; ++kt)
-#pragma unroll
-        for (int r = 0; r < 4; ++r) mx = fmaxf(mx, s[kt][r]);
-      mx = xor_lanes_16_32_max(mx) * kLog2e;
-      float sum = 0.f;
-#pragma unroll
-      for (int kt = 0; kt < NKT; ++kt)
-#pragma unroll
-        for (int r = 0; r < 4; ++r) {
-          s[kt][r] = __builtin_amdgcn_exp2f(s[kt][r] * kLog2e - mx);
-          sum += s[kt][r];
-        }
-      sum = xor_lanes_16_32_sum(sum) + 1e-6f;
-      const float inv = 1.0f / sum;
-#pragma unroll
-      for (int kt = 0; kt < NKT; ++kt)
-#pragma unroll
-        for (int r = 0; r < 4; ++r) s[kt][r] *= inv;
-    }
-
-    // ---- O^T = V^T P^T over pairs of key tiles ----------------------------------------------------------
-    float4v o[4];
-#pragma unroll
-    for (int dt = 0; dt < 4; ++dt) o[dt] = float4v{0.f, 0.f, 0.f, 0.f};
-#pragma unroll
-    for (int kp = 0; kp < NKT / 2; ++kp) {
-      const int kt = 2 * kp;
-      if (kp / 2 < n_groups) {
-        half8 p;
-#pragma unroll
-        for (int r = 0; r < 4; ++r) {
-          p[r] = f2h(s[kt][r]);
-          p[4 + r] = f2h(s[kt + 1][r]);
-        }
-        typedef uint32_t u2 __attribute__((ext_vector_type(2)));
-        typedef uint32_t u4 __attribute__((ext_vector_type(4)));
-        u2 raw[8];
-#pragma unroll
-        for (int kk = 0; kk < 8; ++kk) {
-          raw[kk] = *reinterpret_cast<const u2*>(vbase_bc[(kk >> 1) & 1][kk & 1] + (kp * 32 + (kk & 4)) * 128);
-        }
-#pragma unroll
-        for (int jj = 0; jj < 2; ++jj) {
-          u4 lo, hi;
-#pragma unroll
-          for (int q4 = 0; q4 < 4; ++q4) {
-            lo[q4] = __builtin_amdgcn_perm(raw[2 * q4 + 1][jj], raw[2 * q4][jj], 0x05040100u);
-            hi[q4] = __builtin_amdgcn_perm(raw[2 * q4 + 1][jj], raw[2 * q4][jj], 0x07060302u);
-          }
-          o[2 * jj] = __builtin_amdgcn_mfma_f32_16x16x32_f16(__builtin_bit_cast(half8, lo), p, o[2 * jj], 0, 0, 0);
-          o[2 * jj + 1] = __builtin_amdgcn_mfma_f32_16x16x32_f16(__builtin_bit_cast(half8, hi), p, o[2 * jj + 1], 0, 0, 0);
-        }
-      }
-    }
-
-    if (tq >= 0) {
-      half8 v0, v1;
-#pragma unroll
-      for (int r = 0; r < 2; ++r)
-#pragma unroll
-        for (int j = 0; j < 4; ++j) {
-          v0[4 * r + j] = f2h(o[j][r]);
-          v1[4 * r + j] = f2h(o[j][2 + r]);
-        }
-      T* orow = dst + (size_t)(t0 + tq) * H + head * kD + g * 16;
-      *reinterpret_cast<half8*>(orow) = v0;
-      *reinterpret_cast<half8*>(orow + 8) = v1;
-    }
-  }
-#endif
-}
 
 inline int attention_cu_count() {
   int dev = 0, n = 0;
@@ -1149,25 +826,407 @@ inline int attention_cu_count() {
   return n;
 }
 
-template <int NKT>
-void attention_resident_launch(const void* q, const void* k, const void* v, int layout, int packed_ld,
-                               const void* attr_mask, void* dst, const int32_t* seq_start, const int32_t* word_idx,
-                               int batch, int seq_len, int heads, float scaler, hipStream_t stream) {
-  using Sm = ResSmem<NKT>;
-  auto kern = attention_resident_kernel<NKT>;
-  allow_dynamic_lds(reinterpret_cast<const void*>(kern), (int)Sm::kBytes);
-  // few (head, sequence) pairs: the query tiles of a pair are dealt to 2 or 4 workgroups, each staging K and V itself
-  const long pairs = (long)heads * batch;
-  const int cus = attention_cu_count();
-  const int qsplit = pairs >= cus ? 1 : (2 * pairs >= cus ? 2 : 4);
-  dim3 grid(heads * qsplit, batch);
-  kern<<<grid, kResThreads, Sm::kBytes, stream>>>((const _Float16*)q, (const _Float16*)k, (const _Float16*)v, layout,
-                                                 packed_ld, (const _Float16*)attr_mask, (_Float16*)dst, seq_start,
-                                                 word_idx, batch, seq_len, heads, qsplit, scaler);
+// ------------------------------------------------------------------------------------------
+// fp16 fused attention for 128 < seq_len <= 1024: one workgroup of 4 wavefronts per (64 QSUB queries, head, sequence),
+// a wavefront serves QSUB tiles of 16 queries.  K and V stream through LDS in stages of 64 keys (two stages of 16 KB, the
+// next one arriving by DMA under the work on this one), and the softmax runs along with them: per query the maximum so
+// far, the sum and the output so far, rescaled where the maximum moves.  Nothing grows with the sequence, so several
+// workgroups share a CU and fill each other's waits, and a stage's K and V operands serve all queries of a wavefront.
+// Bound: VALU issue while it runs (a wavefront and stage of 64 keys x 32 queries: about 1060 cycles of VALU, exp2 at a quarter
+// of the rate, against 576 of MFMA), and the start of a workgroup (order -> start table -> rows, then the first stage) over
+// the one and a half rounds its grid takes: the kernel without its arithmetic takes 23 of the 53 us.  Measured per launch,
+// 12 heads: 16 x 1024 positions / 10700 tokens 53 us (172 us with K or V of a whole sequence in 128 KB of LDS, one workgroup
+// per CU and the scores of a query in registers), 32 x 512 positions 39 us (60 us).  Deeper rings of stages, 8 wavefronts
+// per workgroup or a bound of 3 wavefronts per SIMD: 1 to 5 % slower.
+// Rounding points are those of the other kernels (score rounded to half, softmax in float, probabilities rounded to half
+// for P.V, here before the division by the sum instead of after it).
+//
+// A block of 16 queries whose mask rows are 1 up to the sequence's last token and 0 from there on (`mask_class`, see
+// mask_class_kernel) needs no mask: keys behind the last token have weight exp(-10000 - maximum) = 0 and are not visited.
+// Any other block reads its mask rows and visits every key.
+// ------------------------------------------------------------------------------------------
+constexpr int kFlKeys = 64;                                  // keys per stage
+constexpr int kFlStage = kFlKeys * 128;                      // bytes of K (and of V) per stage
+constexpr int kFlRing = 2;                                   // stages in LDS
+constexpr int kFlMaxKeys = 1024;
+typedef __fp16 half4_fp16 __attribute__((ext_vector_type(4)));
+constexpr int kFlSmem = kFlRing * 2 * kFlStage + kFlMaxKeys * (int)sizeof(int);
+
+// class of every block of 16 query positions: 1 = the rows of the mask are 1 for keys up to the last token's and 0 beyond
+__global__ __launch_bounds__(256) void mask_class_kernel(const _Float16* __restrict__ attr_mask,
+                                                         const int32_t* __restrict__ seq_start,
+                                                         const int32_t* __restrict__ word_idx, int seq_len, int blocks,
+                                                         uint8_t* __restrict__ cls) {
+  const int b = blockIdx.y, qb = blockIdx.x;
+  const int t0 = seq_start[b], t1 = seq_start[b + 1];
+  if (t1 <= t0) return;
+  const int n = min(max(word_idx[t1 - 1], 0), seq_len - 1) + 1;
+  if (qb * 16 >= n) return;                                  // never looked at
+  const int rows = min(16, n - qb * 16);
+  const _Float16* m = attr_mask + ((size_t)b * seq_len + qb * 16) * seq_len;
+  bool plain = true;
+  if ((seq_len & 7) == 0) {
+    const int cpr = seq_len / 8;
+    for (int i = threadIdx.x; i < rows * cpr; i += 256) {
+      const int k0 = (i % cpr) * 8;
+      const half8 v = reinterpret_cast<const half8*>(m)[i];
+#pragma unroll
+      for (int j = 0; j < 8; ++j) plain = plain && v[j] == (k0 + j < n ? (_Float16)1.0f : (_Float16)0.0f);
+    }
+  } else {
+    for (int i = threadIdx.x; i < rows * seq_len; i += 256)
+      plain = plain && m[i] == (i % seq_len < n ? (_Float16)1.0f : (_Float16)0.0f);
+  }
+  const int all = __syncthreads_and(plain);
+  if (threadIdx.x == 0) cls[(size_t)b * blocks + qb] = all ? 1 : 0;
+}
+
+__device__ __forceinline__ int v_swizzle(int key) { return (((key >> 1) & 1) | ((key >> 2) & 2)) * 2; }
+// 16 lanes read four rows of 16 halves (lane i: 8 bytes at row i / 4, halves 4 (i & 3) ..) and each gets one column
+__device__ __forceinline__ half4 read_transposed(const unsigned char* p) {
+#if defined(__HIP_DEVICE_COMPILE__)
+  return __builtin_bit_cast(half4, __builtin_amdgcn_ds_read_tr16_b64_v4f16(
+                                       (__attribute__((address_space(3))) half4_fp16*)(p)));
+#else
+  return half4{};
+#endif
+}
+
+template <int QSUB, int WAVES, int OCC>
+__global__ __launch_bounds__(WAVES * kWave, OCC) void attention_flash_kernel(
+    const _Float16* __restrict__ q_src, const _Float16* __restrict__ k_src, const _Float16* __restrict__ v_src, int layout,
+    int packed_ld, const _Float16* __restrict__ attr_mask, const uint8_t* __restrict__ mask_class,
+    _Float16* __restrict__ dst, const int32_t* __restrict__ seq_start, const int32_t* __restrict__ word_idx, int batch,
+    int seq_len, int heads, int q_blocks, float scaler) {
+#if defined(__HIP_DEVICE_COMPILE__)   // device-only types in the body; the host pass only needs the stub
+  using T = _Float16;
+  typedef _Float16 half2x __attribute__((ext_vector_type(2)));
+  extern __shared__ __attribute__((aligned(1024))) unsigned char smem_raw[];
+  unsigned char* kv = smem_raw;                                        // [stage][K, V]
+  int* tok_of_pos = reinterpret_cast<int*>(smem_raw + kFlRing * 2 * kFlStage);
+
+  // The query blocks of one (head, sequence) go to one XCD, whose L2 then fetches their K and V once: workgroup ids are
+  // dealt round-robin to the XCDs, pair p = 8 * (slot / q_blocks) + xcd.
+  const int xcd = blockIdx.x & 7, slot_id = blockIdx.x >> 3;
+  const int pair = (slot_id / q_blocks) * 8 + xcd, qblock = slot_id % q_blocks;
+  if (pair >= batch * heads) return;
+  const int head = pair % heads;
+  const int b = min(max(seq_start[batch + 1 + pair / heads], 0), batch - 1);
+  const int t0 = seq_start[b], t1 = seq_start[b + 1];
+  const int len = t1 - t0;
+  if (len <= 0) return;
+  const int H = heads * kD;
+  const int lane = threadIdx.x & (kWave - 1);
+  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x / kWave);
+  const int l16 = lane & 15, g = lane >> 4;
+
+  const int first_q = qblock * 16 * WAVES * QSUB;
+  const int q0 = first_q + wave * 16 * QSUB;                           // this wavefront's: tile u holds q0 + 16 u + l16
+
+  // K / V rows of a stage by DMA: one instruction fills eight slots (lane -> slot 8 i + lane / 8, 16-byte chunk
+  // (lane & 7) ^ swizzle).  A row without a token is requested beyond the descriptor's range and arrives as zeros.
+  const T* kb = layout == 1 ? k_src + (size_t)t0 * packed_ld + head * kD : k_src + ((size_t)b * heads + head) * seq_len * kD;
+  const T* vb = layout == 1 ? v_src + (size_t)t0 * packed_ld + head * kD : v_src + ((size_t)b * heads + head) * seq_len * kD;
+  const T* qb = layout == 1 ? q_src + (size_t)t0 * packed_ld + head * kD : q_src + ((size_t)b * heads + head) * seq_len * kD;
+  const uint32_t ld = layout == 1 ? (uint32_t)packed_ld : (uint32_t)kD;
+  constexpr int kPer = 8 / WAVES;                                      // requests of a wavefront for K (and for V) per stage
+  uint32_t voff[kPer], voff_v[kPer];
+  int dma_key[kPer];
+#pragma unroll
+  for (int i = 0; i < kPer; ++i) {
+    const int slot = (wave * kPer + i) * 8 + (lane >> 3);
+    dma_key[i] = wide_slot(slot);
+    voff[i] = ((uint32_t)dma_key[i] * ld + (uint32_t)((lane & 7) ^ wide_swizzle(slot)) * 8u) * 2u;
+    // V is read transposed, four rows x 32 bytes by 16 lanes: rows in key order, pairs of chunks XORed with key bits 1 and 3
+    voff_v[i] = ((uint32_t)slot * ld + (uint32_t)((lane & 7) ^ v_swizzle(slot)) * 8u) * 2u;
+  }
+  // `rows`: of the matrices behind kb, vb that exist
+  auto issue = [&](int slot, int st, bool dense, int rows) {
+    unsigned char* base = kv + slot * 2 * kFlStage;
+    const int bytes = (int)(((uint32_t)(rows - 1) * ld + kD) * 2u);
+    const __amdgpu_buffer_rsrc_t rk = __builtin_amdgcn_make_buffer_rsrc(const_cast<T*>(kb), 0, bytes, 0x00020000);
+    const __amdgpu_buffer_rsrc_t rv = __builtin_amdgcn_make_buffer_rsrc(const_cast<T*>(vb), 0, bytes, 0x00020000);
+#pragma unroll
+    for (int i = 0; i < kPer; ++i) {
+      uint32_t off = voff[i], off_v = voff_v[i];
+      uint32_t stage_off = (uint32_t)st * kFlKeys * ld * 2u;
+      if (!dense) {
+        auto place = [&](uint32_t o, int in_stage) -> uint32_t {       // the row of key `in_stage` of the stage, or nowhere
+          const int key = st * kFlKeys + in_stage;
+          const int tk = key < kFlMaxKeys ? tok_of_pos[key] : -1;
+          const uint32_t row = layout == 1 ? (uint32_t)tk : (uint32_t)key;
+          return tk >= 0 ? o + (row - (uint32_t)in_stage) * ld * 2u : 0x80000000u;
+        };
+        off = place(off, dma_key[i]);
+        off_v = place(off_v, (wave * kPer + i) * 8 + (lane >> 3));
+        stage_off = 0;
+      }
+      __builtin_amdgcn_raw_ptr_buffer_load_lds(rk, ET_ATTN_LDS_PTR(base + (wave * kPer + i) * 1024), 16, off, stage_off, 0, 0);
+      __builtin_amdgcn_raw_ptr_buffer_load_lds(rv, ET_ATTN_LDS_PTR(base + kFlStage + (wave * kPer + i) * 1024), 16, off_v, stage_off, 0, 0);
+    }
+  };
+  int tq[QSUB];
+  half8 bq[QSUB][2];
+  auto load_q = [&](bool dense, int n) {
+#pragma unroll
+    for (int u = 0; u < QSUB; ++u) {
+      const int q = q0 + u * 16 + l16;
+      tq[u] = q < n ? (dense ? q : tok_of_pos[q]) : -1;
+#pragma unroll
+      for (int ks = 0; ks < 2; ++ks) {
+#pragma unroll
+        for (int j = 0; j < 8; ++j) bq[u][ks][j] = (_Float16)0;
+        if (tq[u] >= 0)
+          bq[u][ks] = *reinterpret_cast<const half8*>(qb + (size_t)(layout == 1 ? tq[u] : q) * ld + ks * 32 + g * 8);
+      }
+    }
+  };
+
+  // Without a hole in the sequence, position p holds token p: the first stage and the queries are requested on that
+  // assumption, in one step of the chain of dependent loads with what decides it.
+  if (first_q < len) {
+    issue(0, 0, true, len);
+    load_q(true, len);
+  }
+  const int n = min(max(word_idx[t1 - 1], 0), seq_len - 1) + 1;        // positions up to the last token
+  // the workgroup's blocks of 16 queries all plain: uniform over the workgroup, as the stages are
+  const int cblocks = (seq_len + 15) / 16;
+  bool plain = mask_class != nullptr;
+  if (plain) {
+    const int c = first_q / 16 + lane;                                 // one class per lane, all of them in one request
+    const bool mine = lane < WAVES * QSUB && c * 16 < n;
+    plain = __all(!mine || mask_class[(size_t)b * cblocks + min(c, cblocks - 1)] != 0);
+  }
+  const bool dense = n == len;
+  const bool active = q0 < n;                                          // wave-uniform
+  const int stages = ((plain ? n : seq_len) + kFlKeys - 1) / kFlKeys;
+  if (!dense) {
+    wide_wait_dma();
+    __syncthreads();
+    if (first_q >= n) return;                                          // no token among this workgroup's queries
+    for (int i = threadIdx.x; i < kFlMaxKeys; i += WAVES * kWave) tok_of_pos[i] = -1;
+    __syncthreads();
+    for (int tt = threadIdx.x; tt < len; tt += WAVES * kWave) {
+      const int pos = word_idx[t0 + tt];
+      if (pos >= 0 && pos < seq_len) tok_of_pos[pos] = tt;             // relative to the sequence's first packed row
+    }
+    __syncthreads();
+    issue(0, 0, false, layout == 1 ? len : n);
+    load_q(false, n);
+  } else if (first_q >= n) {
+    return;                                                            // (nothing has been requested)
+  }
+#pragma unroll
+  for (int i = 1; i < kFlRing - 1; ++i) issue(i, min(i, stages - 1), dense, layout == 1 ? len : n);
+
+  // the queries are waited for here: left pending, they would have the compiler put a wait for every outstanding request,
+  // the DMA included, into the stage loop
+#pragma unroll
+  for (int u = 0; u < QSUB; ++u)
+#pragma unroll
+    for (int ks = 0; ks < 2; ++ks) asm volatile("" : "+v"(bq[u][ks]));
+
+  // operand addresses (see above): a lane constant plus a compile-time offset per pair of key tiles
+  int k_rd[2], v_rd[4];
+  {
+    const int L = wide_slot((l16 >> 2) * 8 + (l16 & 3));
+    const int sw = wide_swizzle(L);
+#pragma unroll
+    for (int ks = 0; ks < 2; ++ks) k_rd[ks] = L * 128 + (((ks * 4 + g) ^ sw) * 16);
+    // V, transposed read of feature tile dt: the lane's 8 bytes are key g * 8 + l16 / 4, features dt * 16 + (l16 & 3) * 4
+    const int key = g * 8 + (l16 >> 2);
+#pragma unroll
+    for (int dt = 0; dt < 4; ++dt)
+      v_rd[dt] = kFlStage + key * 128 + (((dt * 2 + ((l16 >> 1) & 1)) ^ v_swizzle(key)) * 16) + (l16 & 1) * 8;
+  }
+
+  // Per query: `ref`, the exponent (log2) its probabilities are taken against, is the maximum of the first stage, moved up
+  // only when a score exceeds it by more than kFlSlack (a probability may then reach 2^kFlSlack, far inside half's range,
+  // with the same relative precision); `top` is this lane's share of the true maximum.  The sum of the probabilities is
+  // one more row of the P.V product (a V^T row of ones).
+  constexpr float kFlSlack = 10.f;
+  float ref[QSUB], top[QSUB];
+  float4v o[QSUB][4], l[QSUB];
+#pragma unroll
+  for (int u = 0; u < QSUB; ++u) {
+    ref[u] = top[u] = -INFINITY;
+    l[u] = float4v{0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+    for (int dt = 0; dt < 4; ++dt) o[u][dt] = float4v{0.f, 0.f, 0.f, 0.f};
+  }
+  const float c_exp = scaler * kLog2e;
+  const __amdgpu_buffer_rsrc_t rm = __builtin_amdgcn_make_buffer_rsrc(
+      const_cast<T*>(attr_mask + (size_t)b * seq_len * seq_len), 0, seq_len * seq_len * 2, 0x00020000);
+  uint32_t mask_row[QSUB];
+#pragma unroll
+  for (int u = 0; u < QSUB; ++u) mask_row[u] = (uint32_t)min(q0 + u * 16 + l16, seq_len - 1) * (uint32_t)seq_len * 2u;
+  half8 ones;
+#pragma unroll
+  for (int j = 0; j < 8; ++j) ones[j] = (_Float16)1.0f;
+
+  auto stage = [&](auto PLAINc, int st, int slot) {
+    constexpr bool PLAIN = decltype(PLAINc)::value;
+    const unsigned char* base = kv + slot * 2 * kFlStage;
+    const int key_base = st * kFlKeys + g * 8;                         // this lane's keys: + 32 pair + 0 .. 7
+    // ---- S^T = K Q^T: the lane gets 8 consecutive keys per pair of key tiles, rounded to half ----------------------
+    half8 sc[QSUB][2];
+#pragma unroll
+    for (int pr = 0; pr < 2; ++pr)
+#pragma unroll
+      for (int t = 0; t < 2; ++t) {
+        half8 a[2];
+#pragma unroll
+        for (int ks = 0; ks < 2; ++ks) a[ks] = *reinterpret_cast<const half8*>(base + k_rd[ks] + (pr * 32 + t * 4) * 128);
+#pragma unroll
+        for (int u = 0; u < QSUB; ++u) {
+          float4v acc = {0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+          for (int ks = 0; ks < 2; ++ks) acc = __builtin_amdgcn_mfma_f32_16x16x32_f16(a[ks], bq[u][ks], acc, 0, 0, 0);
+          const half4 h = __builtin_convertvector(acc, half4);
+#pragma unroll
+          for (int r = 0; r < 4; ++r) sc[u][pr][t * 4 + r] = h[r];
+        }
+      }
+    half8 p[QSUB][2];
+#pragma unroll
+    for (int u = 0; u < QSUB; ++u) {
+      float mx, e[2][8];                                               // mx: of this lane's keys, in log2 units
+      if constexpr (PLAIN) {
+        if ((st + 1) * kFlKeys > n) {                                  // workgroup-uniform: the last, partial stage
+          int key_base = st * kFlKeys + g * 8;
+          asm volatile("" : "+v"(key_base));                           // (keeps the comparisons in this block)
+#pragma unroll
+          for (int pr = 0; pr < 2; ++pr)
+#pragma unroll
+            for (int j = 0; j < 8; ++j)
+              if (key_base + pr * 32 + j >= n) sc[u][pr][j] = (_Float16)-INFINITY;
+        }
+        const half8 m8 = __builtin_elementwise_max(sc[u][0], sc[u][1]);
+        const half2x m2 = __builtin_elementwise_max(__builtin_elementwise_max(half2x{m8[0], m8[1]}, half2x{m8[2], m8[3]}),
+                                                    __builtin_elementwise_max(half2x{m8[4], m8[5]}, half2x{m8[6], m8[7]}));
+        mx = fmaxf((float)m2[0], (float)m2[1]) * c_exp;
+      } else {
+        // additive bias of the mask row: (1 - m) * -10000 as one fma (1 - m is exact in float for a half m)
+        mx = -INFINITY;
+#pragma unroll
+        for (int pr = 0; pr < 2; ++pr) {
+          const int k0 = key_base + pr * 32;
+          const uint32_t off = mask_row[u] + (uint32_t)k0 * 2u;        // bytes; reads behind the mask give 0
+          half8 mk;
+          if ((seq_len & 7) == 0) {
+            mk = __builtin_bit_cast(half8, __builtin_amdgcn_raw_buffer_load_b128(rm, off, 0, 0));
+          } else {
+#pragma unroll
+            for (int j = 0; j < 8; ++j) mk[j] = __builtin_bit_cast(T, __builtin_amdgcn_raw_buffer_load_b16(rm, off + 2u * j, 0, 0));
+          }
+#pragma unroll
+          for (int j = 0; j < 8; ++j) {
+            e[pr][j] = k0 + j < seq_len ? h2f(sc[u][pr][j]) * scaler + __builtin_fmaf((float)mk[j], 10000.0f, -10000.0f) : -INFINITY;
+            mx = fmaxf(mx, e[pr][j]);
+          }
+        }
+        mx *= kLog2e;
+      }
+      top[u] = fmaxf(top[u], mx);
+      if (__any(mx > ref[u] + kFlSlack)) {                             // the first stage, and seldom after it
+        const float up = xor_lanes_16_32_max(mx);
+        const float next = up > ref[u] + kFlSlack ? up : ref[u];       // the same in all lanes of a query
+        float alpha = __builtin_amdgcn_exp2f(ref[u] - next);
+        ref[u] = next;
+        asm volatile("s_nop 7" : "+v"(alpha));      // wait states the compiler does not add for the instructions below
+        // (in place by hand: the compiler would give the products registers of their own and copy all of them on the way
+        // around this block)
+        auto scale = [&](float4v& v) {
+#pragma unroll
+          for (int r = 0; r < 4; ++r) {
+            float x = v[r];
+            asm volatile("v_mul_f32 %0, %1, %0" : "+v"(x) : "v"(alpha));
+            v[r] = x;
+          }
+        };
+        scale(l[u]);
+#pragma unroll
+        for (int dt = 0; dt < 4; ++dt) scale(o[u][dt]);
+      }
+#pragma unroll
+      for (int pr = 0; pr < 2; ++pr)
+#pragma unroll
+        for (int j = 0; j < 8; j += 2) {
+          float2v w;
+#pragma unroll
+          for (int i = 0; i < 2; ++i)
+            w[i] = __builtin_amdgcn_exp2f(PLAIN ? __builtin_fmaf(h2f(sc[u][pr][j + i]), c_exp, -ref[u])
+                                                : __builtin_fmaf(e[pr][j + i], kLog2e, -ref[u]));
+          const half2x h = __builtin_convertvector(w, half2x);
+          p[u][pr][j] = h[0];
+          p[u][pr][j + 1] = h[1];
+        }
+    }
+    // ---- O^T += V^T P^T, a pair of key tiles (one MFMA k range) at a time: the transposed reads give the lane features
+    // dt * 16 + l16 of keys g * 8 .. + 3 and + 4 .. + 7 ------------------------------------------------------------
+#pragma unroll
+    for (int pr = 0; pr < 2; ++pr) {
+#pragma unroll
+      for (int u = 0; u < QSUB; ++u) l[u] = __builtin_amdgcn_mfma_f32_16x16x32_f16(ones, p[u][pr], l[u], 0, 0, 0);
+#pragma unroll
+      for (int dt = 0; dt < 4; ++dt) {
+        const half4 lo = read_transposed(base + v_rd[dt] + pr * 32 * 128), hi = read_transposed(base + v_rd[dt] + (pr * 32 + 4) * 128);
+        const half8 vt = __builtin_shufflevector(lo, hi, 0, 1, 2, 3, 4, 5, 6, 7);
+#pragma unroll
+        for (int u = 0; u < QSUB; ++u) o[u][dt] = __builtin_amdgcn_mfma_f32_16x16x32_f16(vt, p[u][pr], o[u][dt], 0, 0, 0);
+      }
+    }
+  };
+
+  auto run = [&](auto PLAINc) {
+    int slot = 0;
+    for (int st = 0; st < stages; ++st) {
+      constexpr int kFly = 2 * kPer * (kFlRing - 2);                   // this wavefront's share of the stage has landed; those
+      __builtin_amdgcn_s_waitcnt((kFly & 15) | (7 << 4) | (15 << 8) | ((kFly >> 4) << 14));      // behind it may fly
+      wide_barrier();                                                  // everybody's has, and the slot before this one is free
+      // (stages past the end re-load the last one, which keeps the count of requests in flight uniform)
+      issue(slot == 0 ? kFlRing - 1 : slot - 1, min(st + kFlRing - 1, stages - 1), dense, layout == 1 ? len : n);
+      if (active) stage(PLAINc, st, slot);
+      slot = slot + 1 == kFlRing ? 0 : slot + 1;
+    }
+  };
+  if (plain) run(std::true_type{});
+  else run(std::false_type{});
+  wide_wait_dma();                                                     // no DMA may still target this workgroup's LDS when it ends
+
+#pragma unroll
+  for (int u = 0; u < QSUB; ++u) {
+    // the reference divides by (sum of exp(score - maximum)) + 1e-6, its maximum clamped at 0 below 1024 keys: in units of
+    // 2^ref that is the sum here + 1e-6 * 2^(maximum - ref)
+    const float mx = fmaxf(xor_lanes_16_32_max(top[u]), seq_len < kFlMaxKeys ? 0.f : -INFINITY);
+    const float inv = 1.0f / (l[u][0] + 1e-6f * __builtin_amdgcn_exp2f(mx - ref[u]));
+    if (tq[u] < 0) continue;
+    T* orow = dst + (size_t)(t0 + tq[u]) * H + head * kD + g * 4;
+#pragma unroll
+    for (int dt = 0; dt < 4; ++dt) *reinterpret_cast<half4*>(orow + dt * 16) = __builtin_convertvector(o[u][dt] * inv, half4);
+  }
+#endif
+}
+
+void attention_flash_launch(const void* q, const void* k, const void* v, int layout, int packed_ld, const void* attr_mask,
+                            const uint8_t* mask_class, void* dst, const int32_t* seq_start, const int32_t* word_idx,
+                            int batch, int seq_len, int heads, float scaler, hipStream_t stream) {
+  const int pairs8 = (batch * heads + 7) / 8 * 8;
+  auto go = [&](auto kern, int waves, int queries) {
+    const int q_blocks = (seq_len + queries - 1) / queries;
+    allow_dynamic_lds(reinterpret_cast<const void*>(kern), kFlSmem);
+    kern<<<pairs8 * q_blocks, waves * kWave, kFlSmem, stream>>>(
+        (const _Float16*)q, (const _Float16*)k, (const _Float16*)v, layout, packed_ld, (const _Float16*)attr_mask, mask_class,
+        (_Float16*)dst, seq_start, word_idx, batch, seq_len, heads, q_blocks, scaler);
+  };
+  // Two query tiles per wavefront halve the LDS reads per score; with few workgroups the CUs are better filled by twice as
+  // many of one tile.
+  if ((long)batch * heads * ((seq_len + 127) / 128) >= 2L * attention_cu_count()) go(attention_flash_kernel<2, 4, 4>, 4, 128);
+  else go(attention_flash_kernel<1, 4, 4>, 4, 64);
 }
 
 // ------------------------------------------------------------------------------------------
-// fused attention for 512 < seq_len <= 1024: the chunked kernel above with the keys of a query tile split over two
+// fp32 fused attention for 512 < seq_len <= 1024: the chunked kernel above with the keys of a query tile split over two
 // wavefronts.  One workgroup of 8 wavefronts per (64 queries, head, sequence): wavefront w serves query tile w & 3 and
 // the key half w >> 2 (512 keys: 4 scores per lane and key tile, 128 VGPRs).  K and V pass through LDS in chunks of
 // 128 keys per half, both halves in the same step.  The two halves of a query tile exchange their maxima and their
@@ -1179,13 +1238,12 @@ constexpr int kSplitThreads = 512;
 constexpr int kSplitHalfTiles = 32;               // key tiles per wavefront
 constexpr int kSplitKeys = 2 * kSplitHalfTiles * 16;
 
-template <typename T>
 __global__ __launch_bounds__(kSplitThreads) void attention_split_kernel(
-    const T* __restrict__ q_src, const T* __restrict__ k_src, const T* __restrict__ v_src, int layout, int packed_ld,
-    const T* __restrict__ attr_mask, T* __restrict__ dst, const int32_t* __restrict__ seq_start,
+    const float* __restrict__ q_src, const float* __restrict__ k_src, const float* __restrict__ v_src, int layout,
+    int packed_ld, const float* __restrict__ attr_mask, float* __restrict__ dst, const int32_t* __restrict__ seq_start,
     const int32_t* __restrict__ word_idx, int batch, int seq_len, int heads, float scaler, int split_out) {
-  static_assert(sizeof(T) == 4, "fp32 only: fp16 beyond 512 positions runs attention_wide_kernel");
-  using Sm = LongSmem<T>;
+  using T = float;
+  using Sm = LongSmem;
   using C = Chunk16<T>;
   using V16 = typename C::vec;
   constexpr int kQS = Sm::kQS, kVS = Sm::kVS;
@@ -1420,303 +1478,15 @@ __global__ __launch_bounds__(kSplitThreads) void attention_split_kernel(
   }
 }
 
-// ------------------------------------------------------------------------------------------
-// fp16, 512 < seq_len <= 1024: the split kernel above with K of the whole sequence in LDS at once, then V in its place.
-// The score registers allow one workgroup per CU either way, so the workgroup takes 128 KB of LDS: every K row (128
-// bytes) arrives by DMA, all requests in flight together with the mask row and Q, instead of chunk after chunk through
-// registers with a fetch latency each; V follows into the same rows while the softmax runs.  A row without a token is
-// requested beyond its buffer descriptor's range and arrives as zeros.
-// Rows, key order and swizzle as described above the resident-key kernel.  Arithmetic and rounding points per element
-// are those of the split kernel.
-// ------------------------------------------------------------------------------------------
-constexpr int kWideKvBytes = kSplitKeys * 128;
-constexpr int kWideSmem = kWideKvBytes + kSplitKeys * (int)sizeof(int) + 2 * 4 * 2 * 16 * (int)sizeof(float);
-
-__global__ __launch_bounds__(kSplitThreads) void attention_wide_kernel(
-    const _Float16* __restrict__ q_src, const _Float16* __restrict__ k_src, const _Float16* __restrict__ v_src, int layout,
-    int packed_ld, const _Float16* __restrict__ attr_mask, _Float16* __restrict__ dst, const int32_t* __restrict__ seq_start,
-    const int32_t* __restrict__ word_idx, int batch, int seq_len, int heads, float scaler) {
-#if defined(__HIP_DEVICE_COMPILE__)   // device-only types in the body; the host pass only needs the stub
-  using T = _Float16;
-  constexpr int NKT = kSplitHalfTiles;
-
-  extern __shared__ __attribute__((aligned(1024))) unsigned char smem_raw[];
-  unsigned char* kv = smem_raw;
-  int* tok_of_pos = reinterpret_cast<int*>(smem_raw + kWideKvBytes);
-  float* red = reinterpret_cast<float*>(smem_raw + kWideKvBytes + kSplitKeys * sizeof(int));   // [2][4 tiles][2 halves][16]
-
-  const int b = min(max(seq_start[batch + 1 + blockIdx.z], 0), batch - 1), head = blockIdx.y, qblock = blockIdx.x;
-  const int t0 = seq_start[b], t1 = seq_start[b + 1];
-  const int len = t1 - t0;
-  if (len <= 0) return;
-  const int H = heads * kD;
-  const int lane = threadIdx.x & (kWave - 1);
-  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x / kWave);
-  const int tile_w = wave & 3, half = wave >> 2;
-  const int l16 = lane & 15, g = lane >> 4;
-  const int kt_base = half * NKT;                            // first key tile of this half
-
-  const int last_pos = min(max(word_idx[t1 - 1], 0), seq_len - 1);
-  const int n_tiles = last_pos / 16 + 1;                     // 16-row tiles that hold at least one token
-  if (qblock * 4 >= n_tiles) return;                         // no token among this workgroup's queries
-  for (int i = threadIdx.x; i < kSplitKeys; i += kSplitThreads) tok_of_pos[i] = -1;
-  __syncthreads();
-  for (int tt = threadIdx.x; tt < len; tt += kSplitThreads) {
-    const int pos = word_idx[t0 + tt];
-    if (pos >= 0 && pos < seq_len) tok_of_pos[pos] = tt;     // relative to the sequence's first packed row
-  }
-  __syncthreads();
-
-  // Rows come in whole groups of four key tiles (what a step of the QK loop reads).  One DMA instruction fills eight
-  // slots; lane -> slot 8 i + lane / 8, 16-byte chunk (lane & 7) ^ swizzle.
-  const int rows_in = min((n_tiles + 3) / 4 * 64, kSplitKeys);
-  auto stage = [&](const T* __restrict__ src) {
-    const T* base = layout == 1 ? src + (size_t)t0 * packed_ld + head * kD : src + ((size_t)b * heads + head) * seq_len * kD;
-    const uint32_t bytes = layout == 1 ? ((uint32_t)(len - 1) * (uint32_t)packed_ld + kD) * 2u : (uint32_t)seq_len * kD * 2u;
-    const __amdgpu_buffer_rsrc_t rsrc = __builtin_amdgcn_make_buffer_rsrc(const_cast<T*>(base), 0, (int)bytes, 0x00020000);
-    for (int i = wave; i < rows_in / 8; i += kSplitThreads / kWave) {
-      const int slot = i * 8 + (lane >> 3);
-      const int key = wide_slot(slot);
-      const int c = (lane & 7) ^ wide_swizzle(slot);
-      const int tk = tok_of_pos[key];
-      const uint32_t row_off = layout == 1 ? (uint32_t)tk * (uint32_t)packed_ld : (uint32_t)key * kD;
-      const uint32_t voff = tk >= 0 ? (row_off + (uint32_t)c * 8u) * 2u : 0x80000000u;      // out of range: zeros
-      __builtin_amdgcn_raw_ptr_buffer_load_lds(rsrc, ET_ATTN_LDS_PTR(kv + i * 1024), 16, voff, 0, 0, 0);
-    }
-  };
-  stage(k_src);
-
-  const int qt = qblock * 4 + tile_w;                        // this wavefront's 16-query tile
-  const bool active = qt < n_tiles;                          // wave-uniform
-  const int q = qt * 16 + l16;
-  const int tq = (active && q < kSplitKeys) ? tok_of_pos[q] : -1;
-  const T* mrow = attr_mask + ((size_t)b * seq_len + min(q, seq_len - 1)) * seq_len;
-  const bool vec_mask = (seq_len & 7) == 0;                  // mask rows start at multiples of 16 bytes
-  auto q_off = [&](int tk, int pos) -> size_t {
-    return layout == 1 ? (size_t)(t0 + tk) * packed_ld + head * kD : (((size_t)b * heads + head) * seq_len + pos) * kD;
-  };
-
-  // Q operand of this lane (zeros for a query position without a token: its result is never stored)
-  half8 bqh[2];
-#pragma unroll
-  for (int ks = 0; ks < 2; ++ks) {
-#pragma unroll
-    for (int j = 0; j < 8; ++j) bqh[ks][j] = (_Float16)0;
-    if (tq >= 0) bqh[ks] = *reinterpret_cast<const half8*>(q_src + q_off(tq, q) + ks * 32 + g * 8);
-  }
-
-  // ---- the additive bias of this half of the mask row: all loads of the row in flight before the first use -------
-  float s[NKT][4];                                           // s[2 P], s[2 P + 1]: keys base + 8 g + 0..3, + 4..7 of pair P
-  // (1 - m) * -10000 as one fma: 1 - m is exact in float for a half m, so both forms round the same real number once
-  {
-    int g8 = g * 8;
-    asm volatile("" : "+v"(g8));       // opaque: the clamped offsets are recomputed, not kept in registers
-    if (vec_mask) {
-      half8 m8[NKT / 2];
-#pragma unroll
-      for (int kp = 0; kp < NKT / 2; ++kp)
-        m8[kp] = *reinterpret_cast<const half8*>(mrow + min((kt_base + 2 * kp) * 16 + g8, seq_len - 8));
-      __builtin_amdgcn_sched_barrier(0);
-#pragma unroll
-      for (int kp = 0; kp < NKT / 2; ++kp) {
-        const int key0 = (kt_base + 2 * kp) * 16 + g8;
-        if ((kt_base + 2 * kp + 2) * 16 <= seq_len) {        // wave-uniform: every key of the pair exists
-#pragma unroll
-          for (int j = 0; j < 8; ++j) s[2 * kp + (j >> 2)][j & 3] = __builtin_fmaf((float)m8[kp][j], 10000.0f, -10000.0f);
-        } else {
-#pragma unroll
-          for (int j = 0; j < 8; ++j)
-            s[2 * kp + (j >> 2)][j & 3] = key0 < seq_len ? __builtin_fmaf((float)m8[kp][j], 10000.0f, -10000.0f) : -INFINITY;
-        }
-      }
-    } else {
-#pragma unroll
-      for (int kp = 0; kp < NKT / 2; ++kp) {
-        const int key0 = (kt_base + 2 * kp) * 16 + g8;
-#pragma unroll
-        for (int j = 0; j < 8; ++j) {
-          const T m = mrow[min(key0 + j, seq_len - 1)];
-          s[2 * kp + (j >> 2)][j & 3] = key0 + j < seq_len ? __builtin_fmaf((float)m, 10000.0f, -10000.0f) : -INFINITY;
-        }
-        if (kp % 4 == 3) __builtin_amdgcn_sched_barrier(0);
-      }
-    }
-  }
-
-  // operand addresses: a lane-dependent base (this half's first row included) plus a compile-time offset per tile
-  const unsigned char* kbase_ks[2];
-  const unsigned char* vbase_bc[2][2];
-  {
-    const int L = wide_slot((l16 >> 2) * 8 + (l16 & 3));
-    const int sw = wide_swizzle(L);
-#pragma unroll
-    for (int ks = 0; ks < 2; ++ks) kbase_ks[ks] = kv + (kt_base * 16 + L) * 128 + (((ks * 4 + g) ^ sw) * 16);
-#pragma unroll
-    for (int bb = 0; bb < 2; ++bb)
-#pragma unroll
-      for (int cc = 0; cc < 2; ++cc) {
-        const int slot = wide_slot(g * 8 + 2 * bb + cc);
-        vbase_bc[bb][cc] = kv + (kt_base * 16 + slot) * 128 + (((l16 >> 1) ^ wide_swizzle(slot)) * 16) + (l16 & 1) * 8;
-      }
-  }
-  wide_wait_dma();
-  __syncthreads();                                           // K is in place
-
-  // ---- S^T = K Q^T, four key tiles at a time -----------------------------------------------------------------------
-  if (active) {
-#pragma unroll
-    for (int kg = 0; kg < NKT / 4; ++kg) {
-      if (kt_base + kg * 4 < n_tiles) {                      // wave-uniform; the rows of a started group are all staged
-        half8 a[4][2];
-#pragma unroll
-        for (int t = 0; t < 4; ++t) {
-          // row l16 of tile t of the group: pair t >> 1, first or second tile t & 1 (4 rows further)
-#pragma unroll
-          for (int ks = 0; ks < 2; ++ks)
-            a[t][ks] = *reinterpret_cast<const half8*>(kbase_ks[ks] + ((kg * 4 + (t & ~1)) * 16 + (t & 1) * 4) * 128);
-        }
-#pragma unroll
-        for (int t = 0; t < 4; ++t) {
-          float4v acc = {0.f, 0.f, 0.f, 0.f};
-#pragma unroll
-          for (int ks = 0; ks < 2; ++ks) acc = __builtin_amdgcn_mfma_f32_16x16x32_f16(a[t][ks], bqh[ks], acc, 0, 0, 0);
-#pragma unroll
-          for (int r = 0; r < 4; ++r) {
-            const float sc = h2f(f2h(acc[r]));                 // the score is stored in half
-            s[kg * 4 + t][r] = sc * scaler + s[kg * 4 + t][r];
-          }
-        }
-      }
-    }
-  }
-  __syncthreads();                                           // every wavefront has read K for the last time
-  stage(v_src);                                              // arrives while the softmax runs
-
-  // ---- masked softmax: each half over its registers, maxima and sums exchanged through LDS --------------------
-  float* red_max = red;
-  float* red_sum = red + 4 * 2 * 16;
-  {
-    float mx = seq_len < kSplitKeys ? 0.f : -INFINITY;       // the clamp at 0 holds below 1024 keys
-#pragma unroll
-    for (int kt = 0; kt < NKT; ++kt)
-#pragma unroll
-      for (int r = 0; r < 4; ++r) mx = fmaxf(mx, s[kt][r]);
-    mx = xor_lanes_16_32_max(mx);
-    if (g == 0) red_max[(tile_w * 2 + half) * 16 + l16] = mx;
-  }
-  wide_wait_lds();
-  wide_barrier();
-  {
-    const float mx = fmaxf(red_max[(tile_w * 2) * 16 + l16], red_max[(tile_w * 2 + 1) * 16 + l16]) * kLog2e;
-    float sum = 0.f;
-#pragma unroll
-    for (int kt = 0; kt < NKT; ++kt)
-#pragma unroll
-      for (int r = 0; r < 4; ++r) {
-        s[kt][r] = __builtin_amdgcn_exp2f(s[kt][r] * kLog2e - mx);
-        sum += s[kt][r];
-      }
-    sum = xor_lanes_16_32_sum(sum);
-    if (g == 0) red_sum[(tile_w * 2 + half) * 16 + l16] = sum;
-  }
-  wide_wait_lds();
-  wide_barrier();
-  {
-    const float sum = red_sum[(tile_w * 2) * 16 + l16] + red_sum[(tile_w * 2 + 1) * 16 + l16] + 1e-6f;
-    const float inv = 1.0f / sum;
-#pragma unroll
-    for (int kt = 0; kt < NKT; ++kt)
-#pragma unroll
-      for (int r = 0; r < 4; ++r) s[kt][r] *= inv;
-  }
-  wide_wait_dma();
-  __syncthreads();                                           // V is in place
-
-  // ---- O^T = V^T P^T, each half over its keys, two key tiles (one MFMA k range) at a time ------------------------
-  float4v o[4];
-#pragma unroll
-  for (int dt = 0; dt < 4; ++dt) o[dt] = float4v{0.f, 0.f, 0.f, 0.f};
-  if (active) {
-#pragma unroll
-    for (int kp = 0; kp < NKT / 2; ++kp) {
-      if (kt_base + 2 * kp < n_tiles) {                      // wave-uniform
-        half8 p;
-#pragma unroll
-        for (int r = 0; r < 4; ++r) {
-          p[r] = f2h(s[2 * kp][r]);
-          p[4 + r] = f2h(s[2 * kp + 1][r]);
-        }
-        typedef uint32_t u2 __attribute__((ext_vector_type(2)));
-        typedef uint32_t u4 __attribute__((ext_vector_type(4)));
-        u2 raw[8];
-#pragma unroll
-        for (int kk = 0; kk < 8; ++kk) {
-          raw[kk] = *reinterpret_cast<const u2*>(vbase_bc[(kk >> 1) & 1][kk & 1] + (kp * 32 + (kk & 4)) * 128);
-        }
-#pragma unroll
-        for (int jj = 0; jj < 2; ++jj) {
-          u4 lo, hi;
-#pragma unroll
-          for (int q4 = 0; q4 < 4; ++q4) {
-            lo[q4] = __builtin_amdgcn_perm(raw[2 * q4 + 1][jj], raw[2 * q4][jj], 0x05040100u);
-            hi[q4] = __builtin_amdgcn_perm(raw[2 * q4 + 1][jj], raw[2 * q4][jj], 0x07060302u);
-          }
-          o[2 * jj] = __builtin_amdgcn_mfma_f32_16x16x32_f16(__builtin_bit_cast(half8, lo), p, o[2 * jj], 0, 0, 0);
-          o[2 * jj + 1] = __builtin_amdgcn_mfma_f32_16x16x32_f16(__builtin_bit_cast(half8, hi), p, o[2 * jj + 1], 0, 0, 0);
-        }
-      }
-    }
-  }
-
-  // ---- the second half hands its part of O over (through the K/V rows, free now), the first adds and stores ------
-  __syncthreads();
-  float4v* xo = reinterpret_cast<float4v*>(smem_raw);        // [4 tiles][64 lanes][4]
-  if (half == 1) {
-#pragma unroll
-    for (int dt = 0; dt < 4; ++dt) xo[(tile_w * kWave + lane) * 4 + dt] = o[dt];
-  }
-  __syncthreads();
-  if (half == 0 && tq >= 0) {
-#pragma unroll
-    for (int dt = 0; dt < 4; ++dt) {
-      const float4v other = xo[(tile_w * kWave + lane) * 4 + dt];
-#pragma unroll
-      for (int r = 0; r < 4; ++r) o[dt][r] += other[r];
-    }
-    half8 v0, v1;
-#pragma unroll
-    for (int r = 0; r < 2; ++r)
-#pragma unroll
-      for (int j = 0; j < 4; ++j) {
-        v0[4 * r + j] = f2h(o[j][r]);
-        v1[4 * r + j] = f2h(o[j][2 + r]);
-      }
-    T* orow = dst + (size_t)(t0 + tq) * H + head * kD + g * 16;
-    *reinterpret_cast<half8*>(orow) = v0;
-    *reinterpret_cast<half8*>(orow + 8) = v1;
-  }
-#endif
-}
-
-// 512 < seq_len <= 1024, head size 64: fp32 runs the chunked split kernel, fp16 the kernel with the whole sequence in LDS
-template <typename T>
 void attention_split_launch(const void* q, const void* k, const void* v, int layout, int packed_ld, const void* attr_mask,
                             void* dst, const int32_t* seq_start, const int32_t* word_idx, int batch, int seq_len, int heads,
                             float scaler, bool split_out, hipStream_t stream) {
   dim3 grid((seq_len + 63) / 64, heads, batch);              // blocks of 64 queries that can hold a token
-  if constexpr (sizeof(T) == 2) {
-    allow_dynamic_lds(reinterpret_cast<const void*>(attention_wide_kernel), kWideSmem);
-    attention_wide_kernel<<<grid, kSplitThreads, kWideSmem, stream>>>(
-        (const _Float16*)q, (const _Float16*)k, (const _Float16*)v, layout, packed_ld, (const _Float16*)attr_mask,
-        (_Float16*)dst, seq_start, word_idx, batch, seq_len, heads, scaler);
-  } else {
-    const size_t smem = 2 * LongSmem<T>::kTileBytes + (size_t)kSplitKeys * sizeof(int) + 2 * 4 * 2 * 16 * sizeof(float);
-    auto kern = attention_split_kernel<T>;
-    allow_dynamic_lds(reinterpret_cast<const void*>(kern), (int)smem);
-    kern<<<grid, kSplitThreads, smem, stream>>>((const T*)q, (const T*)k, (const T*)v, layout, packed_ld,
-                                                (const T*)attr_mask, (T*)dst, seq_start, word_idx, batch, seq_len, heads,
-                                                scaler, split_out ? 1 : 0);
-  }
+  const size_t smem = 2 * LongSmem::kTileBytes + (size_t)kSplitKeys * sizeof(int) + 2 * 4 * 2 * 16 * sizeof(float);
+  allow_dynamic_lds(reinterpret_cast<const void*>(attention_split_kernel), (int)smem);
+  attention_split_kernel<<<grid, kSplitThreads, smem, stream>>>((const float*)q, (const float*)k, (const float*)v, layout,
+                                                                packed_ld, (const float*)attr_mask, (float*)dst, seq_start,
+                                                                word_idx, batch, seq_len, heads, scaler, split_out ? 1 : 0);
 }
 
 // ------------------------------------------------------------------------------------------
@@ -1861,28 +1631,22 @@ void attention_generic_launch(const void* q, const void* k, const void* v, int l
 template <typename T>
 void attention_dispatch(const void* q, const void* k, const void* v, int layout, int packed_ld, const void* attr_mask,
                         void* dst, const int32_t* seq_start, const int32_t* word_idx, int batch, int seq_len, int heads,
-                        int d, float scaler, bool split_out, hipStream_t stream) {
+                        int d, float scaler, bool split_out, const uint8_t* mask_class, hipStream_t stream) {
   if (d != kD || !head_rows_16b<T>(q, k, v, layout, packed_ld, d))
     attention_generic_launch<T>(q, k, v, layout, packed_ld, attr_mask, dst, seq_start, word_idx, batch, seq_len, heads, d,
                                 scaler, stream);
-  else if (seq_len > 512)
-    attention_split_launch<T>(q, k, v, layout, packed_ld, attr_mask, dst, seq_start, word_idx, batch, seq_len, heads,
-                              scaler, split_out, stream);
-  else if (sizeof(T) == 2 && seq_len > 384)
-    attention_resident_launch<32>(q, k, v, layout, packed_ld, attr_mask, dst, seq_start, word_idx, batch, seq_len, heads,
-                                  scaler, stream);
-  else if (sizeof(T) == 2 && seq_len > 256)
-    attention_resident_launch<24>(q, k, v, layout, packed_ld, attr_mask, dst, seq_start, word_idx, batch, seq_len, heads,
-                                  scaler, stream);
   else if (sizeof(T) == 2 && seq_len > 128)
-    attention_resident_launch<16>(q, k, v, layout, packed_ld, attr_mask, dst, seq_start, word_idx, batch, seq_len, heads,
-                                  scaler, stream);
+    attention_flash_launch(q, k, v, layout, packed_ld, attr_mask, mask_class, dst, seq_start, word_idx, batch, seq_len, heads,
+                           scaler, stream);
+  else if (seq_len > 512)
+    attention_split_launch(q, k, v, layout, packed_ld, attr_mask, dst, seq_start, word_idx, batch, seq_len, heads, scaler,
+                           split_out, stream);
   else if (seq_len > 256)
-    attention_long_launch<T, 32>(q, k, v, layout, packed_ld, attr_mask, dst, seq_start, word_idx, batch, seq_len, heads,
-                                 scaler, split_out, stream);
+    attention_long_launch<32>(q, k, v, layout, packed_ld, attr_mask, dst, seq_start, word_idx, batch, seq_len, heads, scaler,
+                              split_out, stream);
   else if (seq_len > 128)
-    attention_long_launch<T, 16>(q, k, v, layout, packed_ld, attr_mask, dst, seq_start, word_idx, batch, seq_len, heads,
-                                 scaler, split_out, stream);
+    attention_long_launch<16>(q, k, v, layout, packed_ld, attr_mask, dst, seq_start, word_idx, batch, seq_len, heads, scaler,
+                              split_out, stream);
   else if (seq_len <= 32)
     attention_launch<T, 2>(q, k, v, layout, packed_ld, attr_mask, dst, seq_start, word_idx, batch, seq_len, heads,
                            scaler, split_out, stream);
@@ -1954,6 +1718,16 @@ bool attention_supported(DType t, int seq_len, int d) {
   return d >= 1 && d <= kGenMaxD && seq_len >= 1 && seq_len <= kGenMaxSeq;
 }
 
+size_t mask_class_bytes(DType t, int batch, int seq_len, int d) {
+  return t == DType::F16 && d == kD && seq_len > 128 && seq_len <= kFlMaxKeys ? (size_t)batch * ((seq_len + 15) / 16) : 0;
+}
+
+void launch_mask_class(const void* attr_mask, const int32_t* seq_start, const int32_t* word_idx, int batch, int seq_len,
+                       uint8_t* cls, hipStream_t stream) {
+  const int blocks = (seq_len + 15) / 16;
+  mask_class_kernel<<<dim3(blocks, batch), 256, 0, stream>>>((const _Float16*)attr_mask, seq_start, word_idx, seq_len, blocks, cls);
+}
+
 bool attention_writes_split(const void* q, const void* k, const void* v, int layout, int packed_ld, int d) {
   return d == kD && head_rows_16b<float>(q, k, v, layout, packed_ld, d);
 }
@@ -1961,13 +1735,13 @@ bool attention_writes_split(const void* q, const void* k, const void* v, int lay
 void launch_attention(DType t, const void* q, const void* k, const void* v, int layout, int packed_ld,
                       const void* attr_mask, void* dst, const int32_t* seq_start, const int32_t* word_idx, int batch,
                       int seq_len, int heads, int d, float scaler, hipStream_t stream,
-                      bool split_out) {
+                      bool split_out, const uint8_t* mask_class) {
   if (t == DType::F32)
     attention_dispatch<float>(q, k, v, layout, packed_ld, attr_mask, dst, seq_start, word_idx, batch, seq_len, heads, d,
-                              scaler, split_out, stream);
+                              scaler, split_out, nullptr, stream);
   else
     attention_dispatch<_Float16>(q, k, v, layout, packed_ld, attr_mask, dst, seq_start, word_idx, batch, seq_len,
-                                 heads, d, scaler, false, stream);
+                                 heads, d, scaler, false, mask_class, stream);
 }
 
 }  // namespace et

@@ -174,7 +174,7 @@ et::DType to_dt(et_dtype d) { return d == ET_FP32 ? et::DType::F32 : et::DType::
 bool layer_splits(et_dtype dtype, int H) { return dtype == ET_FP32 && H % 32 == 0 && et::gemm_split_supported(H, 4 * H); }
 
 struct LayerWs {
-  size_t qkv, ctx, attn, attn_split, inter, seq, wt, total;
+  size_t qkv, ctx, attn, attn_split, inter, seq, cls, wt, total;
 };
 
 LayerWs layer_ws(et_dtype dtype, int B, int S, int heads, int d) {
@@ -193,6 +193,7 @@ LayerWs layer_ws(et_dtype dtype, int B, int S, int heads, int d) {
   // the intermediate has been consumed.
   w.inter = off; off += align_up(align_up(rows, 256) * 4 * H * ea, 256);
   w.seq = off;   off += align_up(et::seq_table_words(B) * sizeof(int32_t), 256);
+  w.cls = off;   off += align_up(et::mask_class_bytes(dtype == ET_FP32 ? et::DType::F32 : et::DType::F16, B, S, d), 256);
   // k-contiguous copies (fp32: split rows) of the six dense kernels (3 H^2 + H^2 + 4 H^2 + 4 H^2 elements)
   w.wt = off;    off += dtype == ET_FP16 || split ? align_up(12 * H * H * ea, 256) : 0;
   w.total = off;
@@ -289,6 +290,7 @@ struct LayerCall {
   const void *from, *to, *attr_mask;
   const int32_t *count, *batch_idx, *word_idx;
   const int32_t* seq_start;           // the batch's sequence table, or null: built here
+  const uint8_t* mask_class = nullptr;   // the classes of the batch's mask rows, or null: made here where they are used
   void* out;
   int B, S, heads, d;
   int rows;                           // launches are sized for this many rows
@@ -390,9 +392,14 @@ et_status run_layer(et_handle h, const LayerCall& c) {
   // QK^T, softmax, PV, un-pad (:159-192)
   const char *q = (const char*)qkv, *k = q + (size_t)H * e, *v = k + (size_t)H * e;
   const bool ctx_split = split && et::attention_writes_split(q, k, v, 1, 3 * H, c.d);
+  const uint8_t* cls = c.mask_class;
+  if (!cls && et::mask_class_bytes(dt, B, S, c.d)) {
+    et::launch_mask_class(c.attr_mask, seq_start, c.word_idx, B, S, (uint8_t*)(base + ws.cls), st);
+    cls = (const uint8_t*)(base + ws.cls);
+  }
   // (where the attention kernel writes floats only, they take the attention output's place until they are split)
   et::launch_attention(dt, q, k, v, 1, 3 * H, c.attr_mask, split && !ctx_split ? attn : ctx, seq_start, c.word_idx, B, S,
-                       c.heads, c.d, softmax_scaler(c.dtype, c.d), st, ctx_split);
+                       c.heads, c.d, softmax_scaler(c.dtype, c.d), st, ctx_split, cls);
   if (split && !ctx_split) et::launch_split_rows((const float*)attn, (uint16_t*)ctx, rows, H, T, st);
   if ((s = check_launch(h, "attention")) != ET_OK) return s;
   // attention output projection + bias + residual(from_tensor) + LayerNorm (:195-213)
@@ -832,6 +839,11 @@ et_status et_encoder(et_handle h, et_dtype dtype, int num_layers, const et_layer
   if ((s = check_launch(h, "input")) != ET_OK) return s;
 
   LayerCall c;
+  if (et::mask_class_bytes(dt, B, S, size_per_head)) {      // once for all layers, in the first one's place for them
+    uint8_t* cls = (uint8_t*)(layer_base + layer_ws(dtype, B, S, head_num, size_per_head).cls);
+    et::launch_mask_class(b->attr_mask, seq, word_idx, B, S, cls, st);
+    c.mask_class = cls;
+  }
   c.dtype = dtype;
   c.attr_mask = b->attr_mask;
   c.count = count; c.batch_idx = batch_idx; c.word_idx = word_idx;
