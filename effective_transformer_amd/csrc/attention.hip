@@ -148,7 +148,7 @@ __global__ __launch_bounds__(256) void transpose_rm_padding_kernel(
 }
 
 // ------------------------------------------------------------------------------------------
-// fused attention, size_per_head = 64, seq_len <= 128 (longer sequences: attention_long_kernel below).
+// fused attention, size_per_head = 64, seq_len <= 64 in fp16 and <= 128 in fp32 (longer sequences: the kernels below).
 //
 // One workgroup (4 wavefronts) per (sequence, group of heads).  What does not depend on the
 // head is done once: token positions, the zero fill of key/value slots without a token (so that a
@@ -546,8 +546,6 @@ void attention_launch(const void* q, const void* k, const void* v, int layout, i
                       float scaler, bool split_out, hipStream_t stream) {
   using Sm = AttnSmem<T, NKT>;
   constexpr int kCpr = kD * (int)sizeof(T) / 16;
-  // Four wavefronts.  Eight at 128 keys in fp16 (one query tile per wavefront, 128 registers, two workgroups per CU)
-  // run the kernel alone 6 % faster on a batch with few long sequences and no faster inside the layer.
   constexpr int WAVES = 4;
   constexpr int kThreads = WAVES * kWave;
   constexpr int CPT = (NKT * 16 * kCpr + kThreads - 1) / kThreads;
@@ -827,7 +825,7 @@ inline int attention_cu_count() {
 }
 
 // ------------------------------------------------------------------------------------------
-// fp16 fused attention for 128 < seq_len <= 1024: one workgroup of 4 wavefronts per (64 QSUB queries, head, sequence),
+// fp16 fused attention for 64 < seq_len <= 1024: one workgroup of 4 wavefronts per (64 QSUB queries, head, sequence),
 // a wavefront serves QSUB tiles of 16 queries.  K and V stream through LDS in stages of 64 keys (two stages of 16 KB, the
 // next one arriving by DMA under the work on this one), and the softmax runs along with them: per query the maximum so
 // far, the sum and the output so far, rescaled where the maximum moves.  Nothing grows with the sequence, so several
@@ -835,7 +833,8 @@ inline int attention_cu_count() {
 // Bound: VALU issue while it runs (a wavefront and stage of 64 keys x 32 queries: about 1060 cycles of VALU, exp2 at a quarter
 // of the rate, against 576 of MFMA), and the start of a workgroup (order -> start table -> rows, then the first stage) over
 // the one and a half rounds its grid takes: the kernel without its arithmetic takes 23 of the 53 us.  Measured per launch,
-// 12 heads: 16 x 1024 positions / 10700 tokens 53 us (172 us with K or V of a whole sequence in 128 KB of LDS, one workgroup
+// 12 heads: 8 x 128 positions / 580 tokens 5.1 us (11.3 us with one workgroup's four wavefronts serving a whole head, two
+// query tiles each, and scores, mask and next rows in registers), 16 heads and 256 x 128 skewed 30 us (40 us), 16 x 1024 positions / 10700 tokens 53 us (172 us with K or V of a whole sequence in 128 KB of LDS, one workgroup
 // per CU and the scores of a query in registers), 32 x 512 positions 39 us (60 us).  Deeper rings of stages, 8 wavefronts
 // per workgroup or a bound of 3 wavefronts per SIMD: 1 to 5 % slower.
 // Rounding points are those of the other kernels (score rounded to half, softmax in float, probabilities rounded to half
@@ -849,6 +848,11 @@ constexpr int kFlKeys = 64;                                  // keys per stage
 constexpr int kFlStage = kFlKeys * 128;                      // bytes of K (and of V) per stage
 constexpr int kFlRing = 2;                                   // stages in LDS
 constexpr int kFlMaxKeys = 1024;
+// Up to 64 positions attention_kernel is the faster one: a head is a single stage there, so nothing streams, and its
+// workgroups serve six heads for one start (12 layers, 1000 x 64: 7.79 ms with it, 7.98 ms with this kernel; 217 x 53 in
+// single layer calls 2.24 and 2.32 ms).  Beyond, this kernel (12 layers: 8 x 128 from ids 0.67 -> 0.61 ms, 60 x 101
+// 1.54 -> 1.25 ms, 300 x 128 7.08 -> 6.87 ms, 500 x 80 5.50 -> 5.47 ms; 24 layers, 256 x 128 skewed 8.63 -> 8.36 ms).
+constexpr int kFlMinKeys = 64;
 typedef __fp16 half4_fp16 __attribute__((ext_vector_type(4)));
 constexpr int kFlSmem = kFlRing * 2 * kFlStage + kFlMaxKeys * (int)sizeof(int);
 
@@ -1635,7 +1639,7 @@ void attention_dispatch(const void* q, const void* k, const void* v, int layout,
   if (d != kD || !head_rows_16b<T>(q, k, v, layout, packed_ld, d))
     attention_generic_launch<T>(q, k, v, layout, packed_ld, attr_mask, dst, seq_start, word_idx, batch, seq_len, heads, d,
                                 scaler, stream);
-  else if (sizeof(T) == 2 && seq_len > 128)
+  else if (sizeof(T) == 2 && seq_len > kFlMinKeys)
     attention_flash_launch(q, k, v, layout, packed_ld, attr_mask, mask_class, dst, seq_start, word_idx, batch, seq_len, heads,
                            scaler, stream);
   else if (seq_len > 512)
@@ -1653,7 +1657,7 @@ void attention_dispatch(const void* q, const void* k, const void* v, int layout,
   else if (seq_len <= 64)
     attention_launch<T, 4>(q, k, v, layout, packed_ld, attr_mask, dst, seq_start, word_idx, batch, seq_len, heads,
                            scaler, split_out, stream);
-  else
+  else if constexpr (sizeof(T) == 4)
     attention_launch<T, 8>(q, k, v, layout, packed_ld, attr_mask, dst, seq_start, word_idx, batch, seq_len, heads,
                            scaler, split_out, stream);
 }
@@ -1719,7 +1723,7 @@ bool attention_supported(DType t, int seq_len, int d) {
 }
 
 size_t mask_class_bytes(DType t, int batch, int seq_len, int d) {
-  return t == DType::F16 && d == kD && seq_len > 128 && seq_len <= kFlMaxKeys ? (size_t)batch * ((seq_len + 15) / 16) : 0;
+  return t == DType::F16 && d == kD && seq_len > kFlMinKeys && seq_len <= kFlMaxKeys ? (size_t)batch * ((seq_len + 15) / 16) : 0;
 }
 
 void launch_mask_class(const void* attr_mask, const int32_t* seq_start, const int32_t* word_idx, int batch, int seq_len,
