@@ -570,234 +570,6 @@ void attention_launch(const void* q, const void* k, const void* v, int layout, i
 
 
 // ------------------------------------------------------------------------------------------
-// fp32 fused attention for 128 < seq_len <= 512: one workgroup (4 wavefronts) per (64 queries, head, sequence).
-// The scores of a wavefront's 16 queries against all keys stay in registers (4 per lane and 16-key tile); K and
-// V pass through LDS in chunks of 128 keys (K chunks first, the softmax over the registers, then V chunks), so the
-// LDS footprint does not grow with the sequence.  Q comes straight from global memory: the MFMA operand of a lane
-// is 64 contiguous bytes of its query's row.  Arithmetic and rounding points are those of
-// the kernel above; key tiles beyond the last token skip their MFMAs (score 0, value 0).
-// ------------------------------------------------------------------------------------------
-constexpr int kLongChunkTiles = 8;                 // 128 keys per LDS chunk
-constexpr int kLongChunk = kLongChunkTiles * 16;
-
-struct LongSmem {
-  static constexpr int kQS = AttnCfg<float>::kQkStride;
-  static constexpr int kVS = kLongChunk + AttnCfg<float>::kVtPad;      // V^T rows
-  static constexpr size_t kKBytes = (size_t)kLongChunk * kQS * sizeof(float);
-  static constexpr size_t kVBytes = (size_t)kD * kVS * sizeof(float);
-  static constexpr size_t kTileBytes = kKBytes > kVBytes ? kKBytes : kVBytes;   // K and V chunks take turns
-};
-
-template <int NKT>
-__global__ __launch_bounds__(kAttnThreads) void attention_long_kernel(
-    const float* __restrict__ q_src, const float* __restrict__ k_src, const float* __restrict__ v_src, int layout,
-    int packed_ld, const float* __restrict__ attr_mask, float* __restrict__ dst, const int32_t* __restrict__ seq_start,
-    const int32_t* __restrict__ word_idx, int batch, int seq_len, int heads, float scaler, int split_out) {
-  using T = float;
-  using Sm = LongSmem;
-  using C = Chunk16<T>;
-  using V16 = typename C::vec;
-  constexpr int kQS = Sm::kQS, kVS = Sm::kVS;
-  constexpr int kSp = NKT * 16;
-  constexpr int kCpr = kD / C::kElems;
-  constexpr int kChunks = NKT / kLongChunkTiles;
-  constexpr int CPT = kLongChunk * kCpr / kAttnThreads;      // 16-byte pieces of a chunk per thread
-  typedef T mask4 __attribute__((ext_vector_type(4)));
-
-  extern __shared__ __attribute__((aligned(16))) unsigned char smem_raw[];
-  T* Ks = reinterpret_cast<T*>(smem_raw);                    // K chunk, later V chunk
-  T* Vs = Ks;
-  int* tok_of_pos = reinterpret_cast<int*>(smem_raw + Sm::kTileBytes);
-
-  const int b = min(max(seq_start[batch + 1 + blockIdx.z], 0), batch - 1), head = blockIdx.y, qblock = blockIdx.x;
-  const int t0 = seq_start[b], t1 = seq_start[b + 1];
-  const int len = t1 - t0;
-  if (len <= 0) return;
-  const int H = heads * kD;
-  const int lane = threadIdx.x & (kWave - 1);
-  const int wave = threadIdx.x / kWave;
-  const int l16 = lane & 15, g = lane >> 4;
-
-  const int last_pos = min(max(word_idx[t1 - 1], 0), seq_len - 1);
-  const int n_tiles = last_pos / 16 + 1;                     // 16-row tiles that hold at least one token
-  if (qblock * 4 >= n_tiles) return;                         // no token among this workgroup's queries
-  for (int i = threadIdx.x; i < kSp; i += kAttnThreads) tok_of_pos[i] = -1;
-  __syncthreads();
-  for (int tt = threadIdx.x; tt < len; tt += kAttnThreads) {
-    const int pos = word_idx[t0 + tt];
-    if (pos >= 0 && pos < seq_len) tok_of_pos[pos] = t0 + tt;
-  }
-  __syncthreads();
-
-  // element offset of (token t / position pos, this head) in the source matrices
-  auto src_off = [&](int t, int pos) -> size_t {
-    return layout == 1 ? (size_t)t * packed_ld + head * kD : (((size_t)b * heads + head) * seq_len + pos) * kD;
-  };
-  // stage rows [c0, c0 + 128) of `src` row-major (stride `stride` elements) into LDS, zeros where no token sits
-  auto stage_rows = [&](const T* __restrict__ src, T* lds, int stride, int c0) {
-    V16 r[CPT];
-    int tk[CPT];
-#pragma unroll
-    for (int k = 0; k < CPT; ++k) {
-      const int i = threadIdx.x + k * kAttnThreads;
-      const int row = i / kCpr, c = i - row * kCpr;
-      const int pos = c0 + row;
-      tk[k] = pos < kSp ? tok_of_pos[pos] : -1;
-#pragma unroll
-      for (int j = 0; j < C::kElems; ++j) r[k][j] = (T)0;
-      if (tk[k] >= 0) r[k] = *reinterpret_cast<const V16*>(src + src_off(tk[k], pos) + c * C::kElems);
-    }
-#pragma unroll
-    for (int k = 0; k < CPT; ++k) {
-      const int i = threadIdx.x + k * kAttnThreads;
-      const int row = i / kCpr, c = i - row * kCpr;
-      *reinterpret_cast<V16*>(lds + row * stride + c * C::kElems) = r[k];
-    }
-  };
-
-  const int qt = qblock * 4 + wave;                          // this wavefront's 16-query tile
-  const bool active = qt < n_tiles;                          // wave-uniform
-  const int q = qt * 16 + l16;
-  const int tq = (active && q < kSp) ? tok_of_pos[q] : -1;
-  const T* mrow = attr_mask + ((size_t)b * seq_len + min(q, seq_len - 1)) * seq_len;
-  const bool vec_mask = (seq_len & 3) == 0;
-
-  // Q operand of this lane (zeros for a query position without a token: its result is never stored)
-  float bqf[16];
-#pragma unroll
-  for (int i = 0; i < 4; ++i) {
-    float4v v4 = {0.f, 0.f, 0.f, 0.f};
-    if (tq >= 0) v4 = *reinterpret_cast<const float4v*>(q_src + src_off(tq, q) + g * 16 + i * 4);
-#pragma unroll
-    for (int j = 0; j < 4; ++j) bqf[i * 4 + j] = v4[j];
-  }
-
-  // ---- S^T = K Q^T chunk by chunk, bias added on the way ------------------------------------------
-  float s[NKT][4];
-#pragma unroll
-  for (int ch = 0; ch < kChunks; ++ch) {
-    const bool chunk_has_tokens = ch * kLongChunkTiles < n_tiles;       // workgroup-uniform
-    if (chunk_has_tokens) {
-      __syncthreads();                                                  // previous chunk fully consumed
-      stage_rows(k_src, Ks, kQS, ch * kLongChunk);
-      __syncthreads();
-    }
-    if (active) {
-#pragma unroll
-      for (int kc = 0; kc < kLongChunkTiles; ++kc) {
-        const int kt = ch * kLongChunkTiles + kc;
-        float4v acc = {0.f, 0.f, 0.f, 0.f};
-        if (kt < n_tiles) {
-#pragma unroll
-          for (int i = 0; i < 4; ++i) {
-            const float4v a4 = *reinterpret_cast<const float4v*>(Ks + (kc * 16 + l16) * kQS + g * 16 + i * 4);
-#pragma unroll
-            for (int j = 0; j < 4; ++j) acc = __builtin_amdgcn_mfma_f32_16x16x4f32(a4[j], bqf[i * 4 + j], acc, 0, 0, 0);
-          }
-        }
-        const int key0 = kt * 16 + g * 4;
-        mask4 m4 = {(T)0, (T)0, (T)0, (T)0};
-        if (vec_mask) {
-          if (key0 < seq_len) m4 = *reinterpret_cast<const mask4*>(mrow + key0);
-        } else {
-#pragma unroll
-          for (int r = 0; r < 4; ++r)
-            if (key0 + r < seq_len) m4[r] = mrow[key0 + r];
-        }
-#pragma unroll
-        for (int r = 0; r < 4; ++r) {
-          s[kt][r] = key0 + r < seq_len ? acc[r] * scaler + (1.0f - (float)m4[r]) * -10000.0f : -INFINITY;
-        }
-      }
-    }
-  }
-
-  // ---- masked softmax over the registers ---------------------------------------------------------------
-  if (active) {
-    float mx = 0.f;
-#pragma unroll
-    for (int kt = 0; kt < NKT; ++kt)
-#pragma unroll
-      for (int r = 0; r < 4; ++r) mx = fmaxf(mx, s[kt][r]);
-    mx = xor_lanes_16_32_max(mx) * kLog2e;
-    float sum = 0.f;
-#pragma unroll
-    for (int kt = 0; kt < NKT; ++kt)
-#pragma unroll
-      for (int r = 0; r < 4; ++r) {
-        s[kt][r] = __builtin_amdgcn_exp2f(s[kt][r] * kLog2e - mx);
-        sum += s[kt][r];
-      }
-    sum = xor_lanes_16_32_sum(sum) + 1e-6f;
-    const float inv = 1.0f / sum;
-#pragma unroll
-    for (int kt = 0; kt < NKT; ++kt)
-#pragma unroll
-      for (int r = 0; r < 4; ++r) s[kt][r] *= inv;
-  }
-
-  // ---- O^T = V^T P^T chunk by chunk ----------------------------------------------------------------------
-  float4v o[4];
-#pragma unroll
-  for (int dt = 0; dt < 4; ++dt) o[dt] = float4v{0.f, 0.f, 0.f, 0.f};
-#pragma unroll
-  for (int ch = 0; ch < kChunks; ++ch) {
-    if (ch * kLongChunkTiles >= n_tiles) break;                         // workgroup-uniform: no token, value 0
-    __syncthreads();
-    // fp32 keeps V^T: feature rows, key columns
-#pragma unroll
-    for (int k = 0; k < CPT; ++k) {
-      const int i = threadIdx.x + k * kAttnThreads;
-      const int row = i / kCpr, c = i - row * kCpr;
-      const int pos = ch * kLongChunk + row;
-      const int tk = pos < kSp ? tok_of_pos[pos] : -1;
-      V16 r = {0.f, 0.f, 0.f, 0.f};
-      if (tk >= 0) r = *reinterpret_cast<const V16*>(v_src + src_off(tk, pos) + c * C::kElems);
-#pragma unroll
-      for (int j = 0; j < C::kElems; ++j) Vs[(c * C::kElems + j) * kVS + row] = r[j];
-    }
-    __syncthreads();
-    if (!active) continue;
-#pragma unroll
-    for (int kc = 0; kc < kLongChunkTiles; ++kc) {
-      const int kt = ch * kLongChunkTiles + kc;
-      if (kt < n_tiles) {
-#pragma unroll
-        for (int dt = 0; dt < 4; ++dt) {
-          const float4v a4 = *reinterpret_cast<const float4v*>(Vs + (dt * 16 + l16) * kVS + kc * 16 + g * 4);
-#pragma unroll
-          for (int r = 0; r < 4; ++r) o[dt] = __builtin_amdgcn_mfma_f32_16x16x4f32(a4[r], s[kt][r], o[dt], 0, 0, 0);
-        }
-      }
-    }
-  }
-
-  if (tq >= 0) {
-    T* orow = dst + (size_t)tq * H + head * kD + g * 4;
-#pragma unroll
-    for (int dt = 0; dt < 4; ++dt) {
-      float4v v;
-#pragma unroll
-      for (int r = 0; r < 4; ++r) v[r] = o[dt][r];
-      if (split_out) store_split<4>(reinterpret_cast<uint16_t*>(dst) + (size_t)tq * 3 * H, head * kD + dt * 16 + g * 4, v);
-      else *reinterpret_cast<float4v*>(orow + dt * 16) = v;
-    }
-  }
-}
-
-template <int NKT>
-void attention_long_launch(const void* q, const void* k, const void* v, int layout, int packed_ld, const void* attr_mask,
-                           void* dst, const int32_t* seq_start, const int32_t* word_idx, int batch, int seq_len, int heads,
-                           float scaler, bool split_out, hipStream_t stream) {
-  const size_t smem = LongSmem::kTileBytes + (size_t)NKT * 16 * sizeof(int);
-  auto kern = attention_long_kernel<NKT>;
-  dim3 grid((seq_len + 63) / 64, heads, batch);               // blocks of 64 queries that can hold a token
-  kern<<<grid, kAttnThreads, smem, stream>>>((const float*)q, (const float*)k, (const float*)v, layout, packed_ld, (const float*)attr_mask,
-                                             (float*)dst, seq_start, word_idx, batch, seq_len, heads, scaler,
-                                             split_out ? 1 : 0);
-}
-
-// ------------------------------------------------------------------------------------------
 // K / V rows brought into LDS by DMA (the streaming kernel below): rows of 128 bytes without padding, one
 // `buffer_load ... lds` instruction fills eight of them (lane -> row lane / 8, 16-byte chunk lane & 7).  A row without
 // a token is requested beyond its buffer descriptor's range and arrives as zeros.
@@ -853,33 +625,38 @@ constexpr int kFlMaxKeys = 1024;
 // single layer calls 2.24 and 2.32 ms).  Beyond, this kernel (12 layers: 8 x 128 from ids 0.67 -> 0.61 ms, 60 x 101
 // 1.54 -> 1.25 ms, 300 x 128 7.08 -> 6.87 ms, 500 x 80 5.50 -> 5.47 ms; 24 layers, 256 x 128 skewed 8.63 -> 8.36 ms).
 constexpr int kFlMinKeys = 64;
+[[maybe_unused]] constexpr float kFlSlack = 10.f;                             // how far (log2) a score may exceed the exponents' reference
+[[maybe_unused]] constexpr float kFlLowest = -3e38f;                          // the reference before the first stage; finite, so that scores of
+                                                             // -infinity weigh nothing against it
 typedef __fp16 half4_fp16 __attribute__((ext_vector_type(4)));
 constexpr int kFlSmem = kFlRing * 2 * kFlStage + kFlMaxKeys * (int)sizeof(int);
 
 // class of every block of 16 query positions: 1 = the rows of the mask are 1 for keys up to the last token's and 0 beyond
-__global__ __launch_bounds__(256) void mask_class_kernel(const _Float16* __restrict__ attr_mask,
-                                                         const int32_t* __restrict__ seq_start,
+template <typename T>
+__global__ __launch_bounds__(256) void mask_class_kernel(const T* __restrict__ attr_mask, const int32_t* __restrict__ seq_start,
                                                          const int32_t* __restrict__ word_idx, int seq_len, int blocks,
                                                          uint8_t* __restrict__ cls) {
+  using V = typename Chunk16<T>::vec;
+  constexpr int kElems = Chunk16<T>::kElems;
   const int b = blockIdx.y, qb = blockIdx.x;
   const int t0 = seq_start[b], t1 = seq_start[b + 1];
   if (t1 <= t0) return;
   const int n = min(max(word_idx[t1 - 1], 0), seq_len - 1) + 1;
   if (qb * 16 >= n) return;                                  // never looked at
   const int rows = min(16, n - qb * 16);
-  const _Float16* m = attr_mask + ((size_t)b * seq_len + qb * 16) * seq_len;
+  const T* m = attr_mask + ((size_t)b * seq_len + qb * 16) * seq_len;
   bool plain = true;
-  if ((seq_len & 7) == 0) {
-    const int cpr = seq_len / 8;
+  if (seq_len % kElems == 0) {
+    const int cpr = seq_len / kElems;
     for (int i = threadIdx.x; i < rows * cpr; i += 256) {
-      const int k0 = (i % cpr) * 8;
-      const half8 v = reinterpret_cast<const half8*>(m)[i];
+      const int k0 = (i % cpr) * kElems;
+      const V v = reinterpret_cast<const V*>(m)[i];
 #pragma unroll
-      for (int j = 0; j < 8; ++j) plain = plain && v[j] == (k0 + j < n ? (_Float16)1.0f : (_Float16)0.0f);
+      for (int j = 0; j < kElems; ++j) plain = plain && v[j] == (k0 + j < n ? (T)1.0f : (T)0.0f);
     }
   } else {
     for (int i = threadIdx.x; i < rows * seq_len; i += 256)
-      plain = plain && m[i] == (i % seq_len < n ? (_Float16)1.0f : (_Float16)0.0f);
+      plain = plain && m[i] == (i % seq_len < n ? (T)1.0f : (T)0.0f);
   }
   const int all = __syncthreads_and(plain);
   if (threadIdx.x == 0) cls[(size_t)b * blocks + qb] = all ? 1 : 0;
@@ -1048,12 +825,12 @@ __global__ __launch_bounds__(WAVES * kWave, OCC) void attention_flash_kernel(
   // only when a score exceeds it by more than kFlSlack (a probability may then reach 2^kFlSlack, far inside half's range,
   // with the same relative precision); `top` is this lane's share of the true maximum.  The sum of the probabilities is
   // one more row of the P.V product (a V^T row of ones).
-  constexpr float kFlSlack = 10.f;
   float ref[QSUB], top[QSUB];
   float4v o[QSUB][4], l[QSUB];
 #pragma unroll
   for (int u = 0; u < QSUB; ++u) {
-    ref[u] = top[u] = -INFINITY;
+    ref[u] = kFlLowest;
+    top[u] = -INFINITY;
     l[u] = float4v{0.f, 0.f, 0.f, 0.f};
 #pragma unroll
     for (int dt = 0; dt < 4; ++dt) o[u][dt] = float4v{0.f, 0.f, 0.f, 0.f};
@@ -1230,267 +1007,244 @@ void attention_flash_launch(const void* q, const void* k, const void* v, int lay
 }
 
 // ------------------------------------------------------------------------------------------
-// fp32 fused attention for 512 < seq_len <= 1024: the chunked kernel above with the keys of a query tile split over two
-// wavefronts.  One workgroup of 8 wavefronts per (64 queries, head, sequence): wavefront w serves query tile w & 3 and
-// the key half w >> 2 (512 keys: 4 scores per lane and key tile, 128 VGPRs).  K and V pass through LDS in chunks of
-// 128 keys per half, both halves in the same step.  The two halves of a query tile exchange their maxima and their
-// sums through LDS (sum = first half + second half, the same on both sides), and the second half hands its part of
-// O over for the first to add and store.  Arithmetic and rounding points per element are those of the other kernels;
-// at 1024 keys the maximum is not clamped at 0 (see attention_generic_kernel).
+// fp32 fused attention for 128 < seq_len <= 1024, built like the kernel above: one workgroup of 4 wavefronts per (64 queries,
+// head, sequence), 16 queries per wavefront, K and V by DMA in stages of 32 keys (two stages of 16 KB), the softmax along
+// with them, everything in float on v_mfma_f32_16x16x4_f32.  A lane's 16-byte V read is four features of one key, one for
+// each of the four feature tiles (row l16 of tile dt is feature 4 l16 + dt), so V needs no transpose and a lane ends up
+// with 16 consecutive features of its query; K's chunks are XOR-swizzled with the key, which spreads an operand read (16
+// rows x one chunk) over all banks.
+// Bound: the fp32 matrix instructions (a wavefront and stage: 2048 cycles of MFMA, about 400 of VALU, 16 LDS reads) over the
+// rounds of workgroups, long sequences first.  15 x 379 positions / 3850 tokens, 12 heads: 48 us per launch, 104 us with K
+// and V in chunks of 128 keys behind barriers and the scores of a query against all keys in registers.
 // ------------------------------------------------------------------------------------------
-constexpr int kSplitThreads = 512;
-constexpr int kSplitHalfTiles = 32;               // key tiles per wavefront
-constexpr int kSplitKeys = 2 * kSplitHalfTiles * 16;
+constexpr int kF32Keys = 32;                                 // keys per stage
+constexpr int kF32Stage = kF32Keys * kD * 4;                 // bytes of K (and of V) per stage
+constexpr int kF32MinKeys = 128;
+constexpr int kF32Smem = 2 * 2 * kF32Stage + kFlMaxKeys * (int)sizeof(int);
 
-__global__ __launch_bounds__(kSplitThreads) void attention_split_kernel(
-    const float* __restrict__ q_src, const float* __restrict__ k_src, const float* __restrict__ v_src, int layout,
-    int packed_ld, const float* __restrict__ attr_mask, float* __restrict__ dst, const int32_t* __restrict__ seq_start,
-    const int32_t* __restrict__ word_idx, int batch, int seq_len, int heads, float scaler, int split_out) {
-  using T = float;
-  using Sm = LongSmem;
-  using C = Chunk16<T>;
-  using V16 = typename C::vec;
-  constexpr int kQS = Sm::kQS, kVS = Sm::kVS;
-  constexpr int kCpr = kD / C::kElems;
-  constexpr int NKT = kSplitHalfTiles;
-  constexpr int kChunks = NKT / kLongChunkTiles;             // 4 steps of 128 keys per half
-  constexpr int CPT = kLongChunk * kCpr / kAttnThreads;      // 16-byte pieces of a chunk per thread of a half
-  typedef T mask4 __attribute__((ext_vector_type(4)));
+__global__ __launch_bounds__(kAttnThreads, 4) void attention_flash_f32_kernel(
+    const float* __restrict__ q_src, const float* __restrict__ k_src, const float* __restrict__ v_src, int layout, int packed_ld,
+    const float* __restrict__ attr_mask, const uint8_t* __restrict__ mask_class, float* __restrict__ dst,
+    const int32_t* __restrict__ seq_start, const int32_t* __restrict__ word_idx, int batch, int seq_len, int heads, int q_blocks,
+    float scaler, int split_out) {
+#if defined(__HIP_DEVICE_COMPILE__)   // device-only types in the body; the host pass only needs the stub
+  extern __shared__ __attribute__((aligned(1024))) unsigned char smem_raw[];
+  unsigned char* kv = smem_raw;                                        // [stage][K, V]
+  int* tok_of_pos = reinterpret_cast<int*>(smem_raw + 2 * 2 * kF32Stage);
 
-  extern __shared__ __attribute__((aligned(16))) unsigned char smem_raw[];
-  int* tok_of_pos = reinterpret_cast<int*>(smem_raw + 2 * Sm::kTileBytes);
-  float* red = reinterpret_cast<float*>(smem_raw + 2 * Sm::kTileBytes + kSplitKeys * sizeof(int));   // [2][4 tiles][2 halves][16]
-
-  const int b = min(max(seq_start[batch + 1 + blockIdx.z], 0), batch - 1), head = blockIdx.y, qblock = blockIdx.x;
+  // the query blocks of one (head, sequence) go to one XCD, as above
+  const int xcd = blockIdx.x & 7, slot_id = blockIdx.x >> 3;
+  const int pair = (slot_id / q_blocks) * 8 + xcd, qblock = slot_id % q_blocks;
+  if (pair >= batch * heads) return;
+  const int head = pair % heads;
+  const int b = min(max(seq_start[batch + 1 + pair / heads], 0), batch - 1);
   const int t0 = seq_start[b], t1 = seq_start[b + 1];
   const int len = t1 - t0;
   if (len <= 0) return;
   const int H = heads * kD;
   const int lane = threadIdx.x & (kWave - 1);
-  const int wave = threadIdx.x / kWave;
-  const int tile_w = wave & 3, half = wave >> 2;
+  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x / kWave);
   const int l16 = lane & 15, g = lane >> 4;
-  // this half's staging threads (256 per half) and its chunk buffer
-  const int tid_h = threadIdx.x & (kAttnThreads - 1);
-  T* Ks = reinterpret_cast<T*>(smem_raw + half * Sm::kTileBytes);
-  T* Vs = Ks;
-  const int kt_base = half * NKT;                            // first key tile of this half
+  const int first_q = qblock * 64, q = first_q + wave * 16 + l16;
 
-  const int last_pos = min(max(word_idx[t1 - 1], 0), seq_len - 1);
-  const int n_tiles = last_pos / 16 + 1;                     // 16-row tiles that hold at least one token
-  if (qblock * 4 >= n_tiles) return;                         // no token among this workgroup's queries
-  for (int i = threadIdx.x; i < kSplitKeys; i += kSplitThreads) tok_of_pos[i] = -1;
-  __syncthreads();
-  for (int tt = threadIdx.x; tt < len; tt += kSplitThreads) {
-    const int pos = word_idx[t0 + tt];
-    if (pos >= 0 && pos < seq_len) tok_of_pos[pos] = t0 + tt;
+  const size_t first = layout == 1 ? (size_t)t0 * packed_ld + head * kD : ((size_t)b * heads + head) * seq_len * kD;
+  const float *kb = k_src + first, *vb = v_src + first, *qb = q_src + first;
+  const uint32_t ld = layout == 1 ? (uint32_t)packed_ld : (uint32_t)kD;
+
+  // DMA: one instruction fills four rows of 256 bytes (lane -> row lane / 16, 16-byte chunk l16, K's swizzled); a
+  // wavefront's share of a stage is eight keys of K and of V
+  uint32_t voff_k[2], voff_v[2];
+  int dma_key[2];
+#pragma unroll
+  for (int i = 0; i < 2; ++i) {
+    dma_key[i] = (wave * 2 + i) * 4 + g;
+    voff_k[i] = ((uint32_t)dma_key[i] * ld + (uint32_t)(l16 ^ (dma_key[i] & 15)) * 4u) * 4u;
+    voff_v[i] = ((uint32_t)dma_key[i] * ld + (uint32_t)l16 * 4u) * 4u;
   }
-  __syncthreads();
-
-  auto src_off = [&](int t, int pos) -> size_t {
-    return layout == 1 ? (size_t)t * packed_ld + head * kD : (((size_t)b * heads + head) * seq_len + pos) * kD;
-  };
-  // rows [c0, c0 + 128) of `src`, zeros where no token sits: global memory -> registers -> this half's buffer
-  // (row-major, stride `stride` elements)
-  auto stage_rows = [&](const T* __restrict__ src, T* lds, int stride, int c0) {
-    V16 r[CPT];
+  auto issue = [&](int slot, int st, bool dense, int rows) {
+    unsigned char* base = kv + slot * 2 * kF32Stage;
+    const int bytes = (int)(((uint32_t)(rows - 1) * ld + kD) * 4u);
+    const __amdgpu_buffer_rsrc_t rk = __builtin_amdgcn_make_buffer_rsrc(const_cast<float*>(kb), 0, bytes, 0x00020000);
+    const __amdgpu_buffer_rsrc_t rv = __builtin_amdgcn_make_buffer_rsrc(const_cast<float*>(vb), 0, bytes, 0x00020000);
 #pragma unroll
-    for (int k = 0; k < CPT; ++k) {
-      const int i = tid_h + k * kAttnThreads;
-      const int row = i / kCpr, c = i - row * kCpr;
-      const int pos = c0 + row;
-      const int tk = pos < kSplitKeys ? tok_of_pos[pos] : -1;
-#pragma unroll
-      for (int j = 0; j < C::kElems; ++j) r[k][j] = (T)0;
-      if (tk >= 0) r[k] = *reinterpret_cast<const V16*>(src + src_off(tk, pos) + c * C::kElems);
-    }
-#pragma unroll
-    for (int k = 0; k < CPT; ++k) {
-      const int i = tid_h + k * kAttnThreads;
-      const int row = i / kCpr, c = i - row * kCpr;
-      *reinterpret_cast<V16*>(lds + row * stride + c * C::kElems) = r[k];
-    }
-  };
-
-  const int qt = qblock * 4 + tile_w;                        // this wavefront's 16-query tile
-  const bool active = qt < n_tiles;                          // wave-uniform
-  const int q = qt * 16 + l16;
-  const int tq = (active && q < kSplitKeys) ? tok_of_pos[q] : -1;
-  const T* mrow = attr_mask + ((size_t)b * seq_len + min(q, seq_len - 1)) * seq_len;
-  const bool vec_mask = (seq_len & 3) == 0;
-
-  // Q operand of this lane (zeros for a query position without a token: its result is never stored)
-  float bqf[16];
-#pragma unroll
-  for (int i = 0; i < 4; ++i) {
-    float4v v4 = {0.f, 0.f, 0.f, 0.f};
-    if (tq >= 0) v4 = *reinterpret_cast<const float4v*>(q_src + src_off(tq, q) + g * 16 + i * 4);
-#pragma unroll
-    for (int j = 0; j < 4; ++j) bqf[i * 4 + j] = v4[j];
-  }
-
-  // ---- the additive bias of this half of the mask row (no branch between the loads) -------------------------
-  float s[NKT][4];
-  {
-    int g4 = g * 4;
-    asm volatile("" : "+v"(g4));       // opaque: the clamped offsets are recomputed, not kept in registers
-#pragma unroll
-    for (int kt = 0; kt < NKT; ++kt) {
-      const int key0 = (kt_base + kt) * 16 + g4;
-      if (vec_mask) {
-        const mask4 m4 = *reinterpret_cast<const mask4*>(mrow + min(key0, seq_len - 4));
-#pragma unroll
-        for (int r = 0; r < 4; ++r) s[kt][r] = key0 < seq_len ? (1.0f - (float)m4[r]) * -10000.0f : -INFINITY;
-      } else {
-#pragma unroll
-        for (int r = 0; r < 4; ++r) {
-          const T m = mrow[min(key0 + r, seq_len - 1)];
-          s[kt][r] = key0 + r < seq_len ? (1.0f - (float)m) * -10000.0f : -INFINITY;
-        }
+    for (int i = 0; i < 2; ++i) {
+      uint32_t off_k = voff_k[i], off_v = voff_v[i];
+      uint32_t stage_off = (uint32_t)st * kF32Keys * ld * 4u;
+      if (!dense) {                                                    // the row of the key, or nowhere
+        const int key = st * kF32Keys + dma_key[i];
+        const int tk = key < kFlMaxKeys ? tok_of_pos[key] : -1;
+        const uint32_t row = layout == 1 ? (uint32_t)tk : (uint32_t)key;
+        const uint32_t by = (row - (uint32_t)dma_key[i]) * ld * 4u;
+        off_k = tk >= 0 ? off_k + by : 0x80000000u;
+        off_v = tk >= 0 ? off_v + by : 0x80000000u;
+        stage_off = 0;
       }
-      if (kt % 4 == 3) __builtin_amdgcn_sched_barrier(0);
+      __builtin_amdgcn_raw_ptr_buffer_load_lds(rk, ET_ATTN_LDS_PTR(base + (wave * 2 + i) * 1024), 16, off_k, stage_off, 0, 0);
+      __builtin_amdgcn_raw_ptr_buffer_load_lds(rv, ET_ATTN_LDS_PTR(base + kF32Stage + (wave * 2 + i) * 1024), 16, off_v, stage_off, 0, 0);
     }
-  }
-
-  // ---- S^T = K Q^T chunk by chunk -------------------------------------------------------------------------
+  };
+  int tq;
+  float4v bq[4];                                                       // features 16 g .. 16 g + 15 of the lane's query
+  auto load_q = [&](bool dense, int n) {
+    tq = q < n ? (dense ? q : tok_of_pos[q]) : -1;
 #pragma unroll
-  for (int ch = 0; ch < kChunks; ++ch) {
-    if (ch * kLongChunkTiles >= n_tiles) break;                          // workgroup-uniform: no token in either half
-    const bool chunk_has_tokens = kt_base + ch * kLongChunkTiles < n_tiles;   // uniform over this half's 4 wavefronts
-    __syncthreads();                                                     // previous chunks fully consumed
-    if (chunk_has_tokens) stage_rows(k_src, Ks, kQS, (kt_base + ch * kLongChunkTiles) * 16);
+    for (int i = 0; i < 4; ++i) {
+      bq[i] = float4v{0.f, 0.f, 0.f, 0.f};
+      if (tq >= 0) bq[i] = *reinterpret_cast<const float4v*>(qb + (size_t)(layout == 1 ? tq : q) * ld + g * 16 + i * 4);
+    }
+  };
+
+  // without a hole in the sequence position p holds token p: requested on that assumption beside what decides it
+  if (first_q < len) {
+    issue(0, 0, true, len);
+    load_q(true, len);
+  }
+  const int n = min(max(word_idx[t1 - 1], 0), seq_len - 1) + 1;        // positions up to the last token
+  const int cblocks = (seq_len + 15) / 16;
+  bool plain = mask_class != nullptr;
+  if (plain) {                                                         // uniform over the workgroup, as the stages are
+    const int c = first_q / 16 + (lane & 3);
+    plain = __all(c * 16 >= n || mask_class[(size_t)b * cblocks + min(c, cblocks - 1)] != 0);
+  }
+  const bool dense = n == len;
+  const bool active = first_q + wave * 16 < n;                         // wave-uniform
+  const int stages = ((plain ? n : seq_len) + kF32Keys - 1) / kF32Keys;
+  if (!dense) {
+    wide_wait_dma();
     __syncthreads();
-    if (active && chunk_has_tokens) {
-#pragma unroll
-      for (int kc = 0; kc < kLongChunkTiles; ++kc) {
-        const int ktl = ch * kLongChunkTiles + kc;
-        if (kt_base + ktl < n_tiles) {
-          float4v acc = {0.f, 0.f, 0.f, 0.f};
-#pragma unroll
-          for (int i = 0; i < 4; ++i) {
-            const float4v a4 = *reinterpret_cast<const float4v*>(Ks + (kc * 16 + l16) * kQS + g * 16 + i * 4);
-#pragma unroll
-            for (int j = 0; j < 4; ++j) acc = __builtin_amdgcn_mfma_f32_16x16x4f32(a4[j], bqf[i * 4 + j], acc, 0, 0, 0);
-          }
-#pragma unroll
-          for (int r = 0; r < 4; ++r) s[ktl][r] = acc[r] * scaler + s[ktl][r];
-        }
-      }
+    if (first_q >= n) return;                                          // no token among this workgroup's queries
+    for (int i = threadIdx.x; i < kFlMaxKeys; i += kAttnThreads) tok_of_pos[i] = -1;
+    __syncthreads();
+    for (int tt = threadIdx.x; tt < len; tt += kAttnThreads) {
+      const int pos = word_idx[t0 + tt];
+      if (pos >= 0 && pos < seq_len) tok_of_pos[pos] = tt;             // relative to the sequence's first packed row
     }
+    __syncthreads();
+    issue(0, 0, false, layout == 1 ? len : n);
+    load_q(false, n);
+  } else if (first_q >= n) {
+    return;                                                            // (nothing has been requested)
   }
+  // (the queries are waited for here and not in the stage loop, where the wait would cover the DMA)
+#pragma unroll
+  for (int i = 0; i < 4; ++i) asm volatile("" : "+v"(bq[i]));
 
-  // ---- masked softmax: each half over its registers, maxima and sums exchanged through LDS --------------------
-  float* red_max = red;
-  float* red_sum = red + 4 * 2 * 16;
-  {
-    float mx = seq_len < kSplitKeys ? 0.f : -INFINITY;       // the clamp at 0 holds below 1024 keys
-#pragma unroll
-    for (int kt = 0; kt < NKT; ++kt)
-#pragma unroll
-      for (int r = 0; r < 4; ++r) mx = fmaxf(mx, s[kt][r]);
-    mx = xor_lanes_16_32_max(mx);
-    if (g == 0) red_max[(tile_w * 2 + half) * 16 + l16] = mx;
-  }
-  __syncthreads();
-  float inv;
-  {
-    const float mx = fmaxf(red_max[(tile_w * 2) * 16 + l16], red_max[(tile_w * 2 + 1) * 16 + l16]) * kLog2e;
-    float sum = 0.f;
-#pragma unroll
-    for (int kt = 0; kt < NKT; ++kt)
-#pragma unroll
-      for (int r = 0; r < 4; ++r) {
-        s[kt][r] = __builtin_amdgcn_exp2f(s[kt][r] * kLog2e - mx);
-        sum += s[kt][r];
-      }
-    sum = xor_lanes_16_32_sum(sum);
-    if (g == 0) red_sum[(tile_w * 2 + half) * 16 + l16] = sum;
-  }
-  __syncthreads();
-  {
-    const float sum = red_sum[(tile_w * 2) * 16 + l16] + red_sum[(tile_w * 2 + 1) * 16 + l16] + 1e-6f;
-    inv = 1.0f / sum;
-#pragma unroll
-    for (int kt = 0; kt < NKT; ++kt)
-#pragma unroll
-      for (int r = 0; r < 4; ++r) s[kt][r] *= inv;
-  }
-
-  // ---- O^T = V^T P^T chunk by chunk, each half over its keys ---------------------------------------------------
+  float ref = kFlLowest, top = -INFINITY, l = 0.f;                     // as above; l: of this lane's keys
   float4v o[4];
 #pragma unroll
   for (int dt = 0; dt < 4; ++dt) o[dt] = float4v{0.f, 0.f, 0.f, 0.f};
-#pragma unroll
-  for (int ch = 0; ch < kChunks; ++ch) {
-    if (ch * kLongChunkTiles >= n_tiles) break;                         // workgroup-uniform
-    const bool chunk_has_tokens = kt_base + ch * kLongChunkTiles < n_tiles;
-    __syncthreads();
-    if (chunk_has_tokens) {
-      // V^T in LDS: feature rows, key columns
-#pragma unroll
-      for (int k = 0; k < CPT; ++k) {
-        const int i = tid_h + k * kAttnThreads;
-        const int row = i / kCpr, c = i - row * kCpr;
-        const int pos = (kt_base + ch * kLongChunkTiles) * 16 + row;
-        const int tk = pos < kSplitKeys ? tok_of_pos[pos] : -1;
-        V16 r = {0.f, 0.f, 0.f, 0.f};
-        if (tk >= 0) r = *reinterpret_cast<const V16*>(v_src + src_off(tk, pos) + c * C::kElems);
-#pragma unroll
-        for (int j = 0; j < C::kElems; ++j) Vs[(c * C::kElems + j) * kVS + row] = r[j];
-      }
-    }
-    __syncthreads();
-    if (!active || !chunk_has_tokens) continue;
-#pragma unroll
-    for (int kc = 0; kc < kLongChunkTiles; ++kc) {
-      const int ktl = ch * kLongChunkTiles + kc;
-      if (kt_base + ktl < n_tiles) {
-#pragma unroll
-        for (int dt = 0; dt < 4; ++dt) {
-          const float4v a4 = *reinterpret_cast<const float4v*>(Vs + (dt * 16 + l16) * kVS + kc * 16 + g * 4);
-#pragma unroll
-          for (int r = 0; r < 4; ++r) o[dt] = __builtin_amdgcn_mfma_f32_16x16x4f32(a4[r], s[ktl][r], o[dt], 0, 0, 0);
-        }
-      }
-    }
-  }
+  const float c_exp = scaler * kLog2e;
+  const float* mrow = attr_mask + ((size_t)b * seq_len + min(q, seq_len - 1)) * seq_len;
 
-  // ---- the second half hands its part of O over (through the chunk buffers, free now), the first adds and stores --
-  __syncthreads();
-  float4v* xo = reinterpret_cast<float4v*>(smem_raw);        // [4 tiles][64 lanes][4]
-  if (half == 1) {
+  auto stage = [&](auto PLAINc, int st, int slot) {
+    constexpr bool PLAIN = decltype(PLAINc)::value;
+    const unsigned char* base = kv + slot * 2 * kF32Stage;
+    float s[2][4];                                                     // keys 32 st + 16 kt + 4 g + r
 #pragma unroll
-    for (int dt = 0; dt < 4; ++dt) xo[(tile_w * kWave + lane) * 4 + dt] = o[dt];
-  }
-  __syncthreads();
-  if (half == 0 && tq >= 0) {
+    for (int kt = 0; kt < 2; ++kt) {
+      float4v acc = {0.f, 0.f, 0.f, 0.f};
 #pragma unroll
-    for (int dt = 0; dt < 4; ++dt) {
-      const float4v other = xo[(tile_w * kWave + lane) * 4 + dt];
+      for (int i = 0; i < 4; ++i) {
+        const float4v a = *reinterpret_cast<const float4v*>(base + (kt * 16 + l16) * 256 + (((g * 4 + i) ^ l16) * 16));
 #pragma unroll
-      for (int r = 0; r < 4; ++r) o[dt][r] += other[r];
+        for (int j = 0; j < 4; ++j) acc = __builtin_amdgcn_mfma_f32_16x16x4f32(a[j], bq[i][j], acc, 0, 0, 0);
+      }
+#pragma unroll
+      for (int r = 0; r < 4; ++r) s[kt][r] = acc[r];
     }
-    T* orow = dst + (size_t)tq * H + head * kD + g * 4;
+    // the exponents' factor: log2 units of the plain scores, of the masked ones otherwise
+    const float unit = PLAIN ? c_exp : kLog2e;
+    const int key0 = st * kF32Keys + g * 4;
+    float mx = -INFINITY;
+    if constexpr (PLAIN) {
+      if ((st + 1) * kF32Keys > n) {                                   // workgroup-uniform: the last, partial stage
 #pragma unroll
-    for (int dt = 0; dt < 4; ++dt) {
-      float4v v;
+        for (int kt = 0; kt < 2; ++kt)
 #pragma unroll
-      for (int r = 0; r < 4; ++r) v[r] = o[dt][r];
-      if (split_out) store_split<4>(reinterpret_cast<uint16_t*>(dst) + (size_t)tq * 3 * H, head * kD + dt * 16 + g * 4, v);
-      else *reinterpret_cast<float4v*>(orow + dt * 16) = v;
+          for (int r = 0; r < 4; ++r)
+            if (key0 + kt * 16 + r >= n) s[kt][r] = -INFINITY;
+      }
+    } else {
+#pragma unroll
+      for (int kt = 0; kt < 2; ++kt) {
+        const int k0 = key0 + kt * 16;
+        float4v m4 = {0.f, 0.f, 0.f, 0.f};
+        if ((seq_len & 3) == 0) {
+          if (k0 < seq_len) m4 = *reinterpret_cast<const float4v*>(mrow + k0);
+        } else {
+#pragma unroll
+          for (int r = 0; r < 4; ++r)
+            if (k0 + r < seq_len) m4[r] = mrow[k0 + r];
+        }
+#pragma unroll
+        for (int r = 0; r < 4; ++r) s[kt][r] = k0 + r < seq_len ? s[kt][r] * scaler + (1.0f - m4[r]) * -10000.0f : -INFINITY;
+      }
     }
+#pragma unroll
+    for (int kt = 0; kt < 2; ++kt)
+#pragma unroll
+      for (int r = 0; r < 4; ++r) mx = fmaxf(mx, s[kt][r]);
+    mx *= unit;
+    top = fmaxf(top, mx);
+    if (__any(mx > ref + kFlSlack)) {                                  // the first stage, and seldom after it
+      const float up = xor_lanes_16_32_max(mx);
+      const float next = up > ref + kFlSlack ? up : ref;               // the same in all lanes of a query
+      const float alpha = __builtin_amdgcn_exp2f(ref - next);
+      ref = next;
+      l *= alpha;
+#pragma unroll
+      for (int dt = 0; dt < 4; ++dt) o[dt] *= alpha;
+    }
+#pragma unroll
+    for (int kt = 0; kt < 2; ++kt)
+#pragma unroll
+      for (int r = 0; r < 4; ++r) {
+        s[kt][r] = __builtin_amdgcn_exp2f(__builtin_fmaf(s[kt][r], unit, -ref));
+        l += s[kt][r];
+      }
+#pragma unroll
+    for (int kt = 0; kt < 2; ++kt)
+#pragma unroll
+      for (int r = 0; r < 4; ++r) {
+        const float4v v = *reinterpret_cast<const float4v*>(base + kF32Stage + (kt * 16 + g * 4 + r) * 256 + l16 * 16);
+#pragma unroll
+        for (int dt = 0; dt < 4; ++dt) o[dt] = __builtin_amdgcn_mfma_f32_16x16x4f32(v[dt], s[kt][r], o[dt], 0, 0, 0);
+      }
+  };
+  auto run = [&](auto PLAINc) {
+    for (int st = 0; st < stages; ++st) {
+      wide_wait_dma();                                                 // this wavefront's share of the stage has landed,
+      wide_barrier();                                                  // everybody's has, and the other slot is free
+      if (st + 1 < stages) issue((st + 1) & 1, st + 1, dense, layout == 1 ? len : n);
+      if (active) stage(PLAINc, st, st & 1);
+    }
+  };
+  if (plain) run(std::true_type{});
+  else run(std::false_type{});
+
+  const float mx = fmaxf(xor_lanes_16_32_max(top), seq_len < kFlMaxKeys ? 0.f : -INFINITY);
+  const float sum = xor_lanes_16_32_sum(l);
+  if (tq < 0) return;
+  const float inv = 1.0f / (sum + 1e-6f * __builtin_amdgcn_exp2f(mx - ref));
+  // o[dt][r] is feature 16 g + 4 r + dt
+#pragma unroll
+  for (int r = 0; r < 4; ++r) {
+    const float4v v = {o[0][r] * inv, o[1][r] * inv, o[2][r] * inv, o[3][r] * inv};
+    const int col = head * kD + g * 16 + r * 4;
+    if (split_out) store_split<4>(reinterpret_cast<uint16_t*>(dst) + (size_t)(t0 + tq) * 3 * H, col, v);
+    else *reinterpret_cast<float4v*>(dst + (size_t)(t0 + tq) * H + col) = v;
   }
+#endif
 }
 
-void attention_split_launch(const void* q, const void* k, const void* v, int layout, int packed_ld, const void* attr_mask,
-                            void* dst, const int32_t* seq_start, const int32_t* word_idx, int batch, int seq_len, int heads,
-                            float scaler, bool split_out, hipStream_t stream) {
-  dim3 grid((seq_len + 63) / 64, heads, batch);              // blocks of 64 queries that can hold a token
-  const size_t smem = 2 * LongSmem::kTileBytes + (size_t)kSplitKeys * sizeof(int) + 2 * 4 * 2 * 16 * sizeof(float);
-  allow_dynamic_lds(reinterpret_cast<const void*>(attention_split_kernel), (int)smem);
-  attention_split_kernel<<<grid, kSplitThreads, smem, stream>>>((const float*)q, (const float*)k, (const float*)v, layout,
-                                                                packed_ld, (const float*)attr_mask, (float*)dst, seq_start,
-                                                                word_idx, batch, seq_len, heads, scaler, split_out ? 1 : 0);
+void attention_flash_f32_launch(const void* q, const void* k, const void* v, int layout, int packed_ld, const void* attr_mask,
+                                const uint8_t* mask_class, void* dst, const int32_t* seq_start, const int32_t* word_idx,
+                                int batch, int seq_len, int heads, float scaler, bool split_out, hipStream_t stream) {
+  const int q_blocks = (seq_len + 63) / 64;
+  const int grid = (batch * heads + 7) / 8 * 8 * q_blocks;
+  attention_flash_f32_kernel<<<grid, kAttnThreads, kF32Smem, stream>>>(
+      (const float*)q, (const float*)k, (const float*)v, layout, packed_ld, (const float*)attr_mask, mask_class, (float*)dst,
+      seq_start, word_idx, batch, seq_len, heads, q_blocks, scaler, split_out ? 1 : 0);
 }
 
 // ------------------------------------------------------------------------------------------
@@ -1636,21 +1390,17 @@ template <typename T>
 void attention_dispatch(const void* q, const void* k, const void* v, int layout, int packed_ld, const void* attr_mask,
                         void* dst, const int32_t* seq_start, const int32_t* word_idx, int batch, int seq_len, int heads,
                         int d, float scaler, bool split_out, const uint8_t* mask_class, hipStream_t stream) {
-  if (d != kD || !head_rows_16b<T>(q, k, v, layout, packed_ld, d))
+  // (the streaming kernels address the rows of a sequence with 31 bits)
+  const bool far = (uint64_t)seq_len * (uint64_t)(layout == 1 ? packed_ld : kD) * sizeof(T) >= 0x80000000ull;
+  if (d != kD || !head_rows_16b<T>(q, k, v, layout, packed_ld, d) || (far && seq_len > kFlMinKeys))
     attention_generic_launch<T>(q, k, v, layout, packed_ld, attr_mask, dst, seq_start, word_idx, batch, seq_len, heads, d,
                                 scaler, stream);
   else if (sizeof(T) == 2 && seq_len > kFlMinKeys)
     attention_flash_launch(q, k, v, layout, packed_ld, attr_mask, mask_class, dst, seq_start, word_idx, batch, seq_len, heads,
                            scaler, stream);
-  else if (seq_len > 512)
-    attention_split_launch(q, k, v, layout, packed_ld, attr_mask, dst, seq_start, word_idx, batch, seq_len, heads, scaler,
-                           split_out, stream);
-  else if (seq_len > 256)
-    attention_long_launch<32>(q, k, v, layout, packed_ld, attr_mask, dst, seq_start, word_idx, batch, seq_len, heads, scaler,
-                              split_out, stream);
-  else if (seq_len > 128)
-    attention_long_launch<16>(q, k, v, layout, packed_ld, attr_mask, dst, seq_start, word_idx, batch, seq_len, heads, scaler,
-                              split_out, stream);
+  else if (sizeof(T) == 4 && seq_len > kF32MinKeys)
+    attention_flash_f32_launch(q, k, v, layout, packed_ld, attr_mask, mask_class, dst, seq_start, word_idx, batch, seq_len,
+                               heads, scaler, split_out, stream);
   else if (seq_len <= 32)
     attention_launch<T, 2>(q, k, v, layout, packed_ld, attr_mask, dst, seq_start, word_idx, batch, seq_len, heads,
                            scaler, split_out, stream);
@@ -1723,13 +1473,17 @@ bool attention_supported(DType t, int seq_len, int d) {
 }
 
 size_t mask_class_bytes(DType t, int batch, int seq_len, int d) {
-  return t == DType::F16 && d == kD && seq_len > kFlMinKeys && seq_len <= kFlMaxKeys ? (size_t)batch * ((seq_len + 15) / 16) : 0;
+  return d == kD && seq_len > (t == DType::F16 ? kFlMinKeys : kF32MinKeys) && seq_len <= kFlMaxKeys ? (size_t)batch * ((seq_len + 15) / 16) : 0;
 }
 
-void launch_mask_class(const void* attr_mask, const int32_t* seq_start, const int32_t* word_idx, int batch, int seq_len,
+void launch_mask_class(DType t, const void* attr_mask, const int32_t* seq_start, const int32_t* word_idx, int batch, int seq_len,
                        uint8_t* cls, hipStream_t stream) {
   const int blocks = (seq_len + 15) / 16;
-  mask_class_kernel<<<dim3(blocks, batch), 256, 0, stream>>>((const _Float16*)attr_mask, seq_start, word_idx, seq_len, blocks, cls);
+  const dim3 grid(blocks, batch);
+  if (t == DType::F32)
+    mask_class_kernel<<<grid, 256, 0, stream>>>((const float*)attr_mask, seq_start, word_idx, seq_len, blocks, cls);
+  else
+    mask_class_kernel<<<grid, 256, 0, stream>>>((const _Float16*)attr_mask, seq_start, word_idx, seq_len, blocks, cls);
 }
 
 bool attention_writes_split(const void* q, const void* k, const void* v, int layout, int packed_ld, int d) {
@@ -1742,7 +1496,7 @@ void launch_attention(DType t, const void* q, const void* k, const void* v, int 
                       bool split_out, const uint8_t* mask_class) {
   if (t == DType::F32)
     attention_dispatch<float>(q, k, v, layout, packed_ld, attr_mask, dst, seq_start, word_idx, batch, seq_len, heads, d,
-                              scaler, split_out, nullptr, stream);
+                              scaler, split_out, mask_class, stream);
   else
     attention_dispatch<_Float16>(q, k, v, layout, packed_ld, attr_mask, dst, seq_start, word_idx, batch, seq_len,
                                  heads, d, scaler, false, mask_class, stream);

@@ -394,7 +394,7 @@ et_status run_layer(et_handle h, const LayerCall& c) {
   const bool ctx_split = split && et::attention_writes_split(q, k, v, 1, 3 * H, c.d);
   const uint8_t* cls = c.mask_class;
   if (!cls && et::mask_class_bytes(dt, B, S, c.d)) {
-    et::launch_mask_class(c.attr_mask, seq_start, c.word_idx, B, S, (uint8_t*)(base + ws.cls), st);
+    et::launch_mask_class(dt, c.attr_mask, seq_start, c.word_idx, B, S, (uint8_t*)(base + ws.cls), st);
     cls = (const uint8_t*)(base + ws.cls);
   }
   // (where the attention kernel writes floats only, they take the attention output's place until they are split)
@@ -841,7 +841,7 @@ et_status et_encoder(et_handle h, et_dtype dtype, int num_layers, const et_layer
   LayerCall c;
   if (et::mask_class_bytes(dt, B, S, size_per_head)) {      // once for all layers, in the first one's place for them
     uint8_t* cls = (uint8_t*)(layer_base + layer_ws(dtype, B, S, head_num, size_per_head).cls);
-    et::launch_mask_class(b->attr_mask, seq, word_idx, B, S, cls, st);
+    et::launch_mask_class(dt, b->attr_mask, seq, word_idx, B, S, cls, st);
     c.mask_class = cls;
   }
   c.dtype = dtype;

@@ -1,4 +1,4 @@
-"""fp16 layers of more than 64 positions: blocks of queries whose mask rows simply end with the sequence take a way of
+"""Layers of more than 64 (fp16) or 128 (fp32) positions: blocks of queries whose mask rows simply end with the sequence take a way of
 their own through the attention kernel, decided on the device from the mask."""
 import numpy as np
 import pytest
@@ -12,7 +12,8 @@ pytestmark = pytest.mark.gpu
 
 # around a block of 16 queries, a stage of 64 keys and a workgroup's 64 or 128 queries; a length that is no multiple of 8
 @pytest.mark.parametrize("S,B,dtype", [(S, B, "fp16") for S, B in [(65, 6), (80, 300), (101, 64), (127, 6), (128, 6), (129, 6),
-                                                                    (150, 64), (192, 7), (257, 130), (1023, 6), (1024, 6)]])
+                                                                    (150, 64), (192, 7), (257, 130), (1023, 6), (1024, 6)]] +
+                         [(S, B, "fp32") for S, B in [(129, 6), (150, 40), (160, 6), (255, 6), (513, 6), (1023, 6), (1024, 6)]])
 def test_masks_of_every_kind(S, B, dtype):
     print("long masks", S, B, dtype, flush=True)
     el = np.float16 if dtype == "fp16" else np.float32
