@@ -148,7 +148,7 @@ __global__ __launch_bounds__(256) void transpose_rm_padding_kernel(
 }
 
 // ------------------------------------------------------------------------------------------
-// fused attention, size_per_head = 64, seq_len <= 64 in fp16 and <= 128 in fp32 (longer sequences: the kernels below).
+// fused attention, size_per_head = 64, seq_len <= 64 in fp16 and <= 32 in fp32 (longer sequences: the kernels below).
 //
 // One workgroup (4 wavefronts) per (sequence, group of heads).  What does not depend on the
 // head is done once: token positions, the zero fill of key/value slots without a token (so that a
@@ -218,7 +218,7 @@ __device__ __forceinline__ float xor_lanes_16_32_sum(float v) {
   return a + b;
 }
 
-// WAVES: wavefronts per workgroup (4; a wavefront serves NKT / WAVES query tiles at 128 keys).  CPT = 16-byte chunks of
+// WAVES: wavefronts per workgroup, one 16-query tile each.  CPT = 16-byte chunks of
 // one matrix a thread moves per head (ceil(seq rows * chunks per row / threads)).
 // PF: keep the next head's Q/K/V chunks in registers while the current head is computed.
 template <typename T, int NKT, int WAVES, int CPT, bool PF>
@@ -236,7 +236,7 @@ __global__ __launch_bounds__(WAVES * kWave) void attention_kernel(
   constexpr int kSp = Sm::kSp;
   constexpr int kCpr = kD / C::kElems;       // 16-byte chunks per head row
   constexpr int kThreads = WAVES * kWave;
-  constexpr int QPW = NKT > WAVES ? NKT / WAVES : 1;   // query tiles per wavefront
+  static_assert(NKT <= WAVES, "a wavefront serves one query tile");
   typedef T mask4 __attribute__((ext_vector_type(4)));
 
   extern __shared__ __attribute__((aligned(16))) unsigned char smem_raw[];
@@ -272,11 +272,10 @@ __global__ __launch_bounds__(WAVES * kWave) void attention_kernel(
     my_pos[k] = tt < len ? word_idx[t0 + tt] : -1;
   }
   // the mask rows of this wavefront's queries stay in registers for all heads
-  mask4 mreg[QPW][NKT];
+  mask4 mreg[NKT];
   const bool vec_mask = (seq_len & 3) == 0;
-#pragma unroll
-  for (int qi = 0; qi < QPW; ++qi) {
-    const int q = (wave + qi * WAVES) * 16 + l16;
+  {
+    const int q = wave * 16 + l16;
     const T* mrow = attr_mask + ((size_t)b * seq_len + min(q, seq_len - 1)) * seq_len;
 #pragma unroll
     for (int kt = 0; kt < NKT; ++kt) {
@@ -289,7 +288,7 @@ __global__ __launch_bounds__(WAVES * kWave) void attention_kernel(
         for (int r = 0; r < 4; ++r)
           if (key0 + r < seq_len) m4[r] = mrow[key0 + r];
       }
-      mreg[qi][kt] = m4;
+      mreg[kt] = m4;
     }
   }
   using V16 = typename C::vec;
@@ -317,12 +316,10 @@ __global__ __launch_bounds__(WAVES * kWave) void attention_kernel(
   // mask value -> additive bias, once for all heads: (1 - m) * -10000 in float as the reference computes it, kept in
   // the element type (exact for 0/1 masks); keys beyond seq_len do not exist
 #pragma unroll
-  for (int qi = 0; qi < QPW; ++qi)
+  for (int kt = 0; kt < NKT; ++kt)
 #pragma unroll
-    for (int kt = 0; kt < NKT; ++kt)
-#pragma unroll
-      for (int r = 0; r < 4; ++r)
-        mreg[qi][kt][r] = kt * 16 + g * 4 + r < seq_len ? (T)((1.0f - (float)mreg[qi][kt][r]) * -10000.0f) : (T)-INFINITY;
+    for (int r = 0; r < 4; ++r)
+      mreg[kt][r] = kt * 16 + g * 4 + r < seq_len ? (T)((1.0f - (float)mreg[kt][r]) * -10000.0f) : (T)-INFINITY;
 
   // ---- position table, then zero the key / value slots that hold no token (once: heads only overwrite tokens) ----
   for (int i = threadIdx.x; i < kSp; i += kThreads) tok_of_pos[i] = -1;
@@ -350,16 +347,11 @@ __global__ __launch_bounds__(WAVES * kWave) void attention_kernel(
     }
   }
 
-  // where each of this lane's queries writes its output row (head 0; null without a token): the same for every head
-  T* out_row[QPW];
-#pragma unroll
-  for (int qi = 0; qi < QPW; ++qi) {
-    const int qt = wave + qi * WAVES;
-    const int tq = qt < n_tiles ? tok_of_pos[qt * 16 + l16] : -1;
-    out_row[qi] = tq >= 0 ? dst + (size_t)tq * H + g * (sizeof(T) == 2 ? 16 : 4) : nullptr;
-    if (sizeof(T) == 4 && split_out && tq >= 0)
-      out_row[qi] = reinterpret_cast<T*>(reinterpret_cast<uint16_t*>(dst) + (size_t)tq * 3 * H);
-  }
+  // where this lane's query writes its output row (head 0; null without a token): the same for every head
+  const int tq = wave < n_tiles && wave < NKT ? tok_of_pos[wave * 16 + l16] : -1;
+  T* out_row = tq >= 0 ? dst + (size_t)tq * H + g * (sizeof(T) == 2 ? 16 : 4) : nullptr;
+  if (sizeof(T) == 4 && split_out && tq >= 0)
+    out_row = reinterpret_cast<T*>(reinterpret_cast<uint16_t*>(dst) + (size_t)tq * 3 * H);
 
   for (int head = h_begin; head < h_end; ++head) {
     if (!PF) { ET_ATTN_LOAD_HEAD(head) }
@@ -382,11 +374,8 @@ __global__ __launch_bounds__(WAVES * kWave) void attention_kernel(
     __syncthreads();
     if (PF && head + 1 < h_end) { ET_ATTN_LOAD_HEAD(head + 1) }   // flies while this head is computed
 
-#pragma unroll
-    for (int qi = 0; qi < QPW; ++qi) {
-      const int qt = wave + qi * WAVES;
-      if (qt >= n_tiles) break;               // wave-uniform
-      const int q = qt * 16 + l16;            // this lane's query position
+    if (wave < n_tiles) {                     // wave-uniform
+      const int q = wave * 16 + l16;          // this lane's query position
       float s[NKT][4];
       // ---- S^T = K Q^T -------------------------------------------------------------------
       if constexpr (sizeof(T) == 2) {
@@ -436,7 +425,7 @@ __global__ __launch_bounds__(WAVES * kWave) void attention_kernel(
       for (int kt = 0; kt < NKT; ++kt)
 #pragma unroll
         for (int r = 0; r < 4; ++r) {
-          const float tv = s[kt][r] * scaler + (float)mreg[qi][kt][r];   // mreg: (1 - mask) * -10000, -inf beyond seq_len
+          const float tv = s[kt][r] * scaler + (float)mreg[kt][r];   // mreg: (1 - mask) * -10000, -inf beyond seq_len
           s[kt][r] = tv;
           mx = fmaxf(mx, tv);
         }
@@ -507,7 +496,7 @@ __global__ __launch_bounds__(WAVES * kWave) void attention_kernel(
         }
       }
       // ---- write the lane's 16 features of its query's packed row --------------------------
-      if (out_row[qi] != nullptr) {
+      if (out_row != nullptr) {
         if constexpr (sizeof(T) == 2) {
           // o[j][r] is feature 16*g + 4*r + j: 16 consecutive features
           half8 v0, v1;
@@ -518,18 +507,18 @@ __global__ __launch_bounds__(WAVES * kWave) void attention_kernel(
               v0[4 * r + j] = f2h(o[j][r]);
               v1[4 * r + j] = f2h(o[j][2 + r]);
             }
-          T* orow = out_row[qi] + head * kD;
+          T* orow = out_row + head * kD;
           *reinterpret_cast<half8*>(orow) = v0;
           *reinterpret_cast<half8*>(orow + 8) = v1;
         } else {
-          T* orow = out_row[qi] + head * kD;
+          T* orow = out_row + head * kD;
 #pragma unroll
           for (int dt = 0; dt < 4; ++dt) {
             typedef T out4 __attribute__((ext_vector_type(4)));
             out4 v;
 #pragma unroll
             for (int r = 0; r < 4; ++r) v[r] = (T)o[dt][r];
-            if (split_out) store_split<4>(reinterpret_cast<uint16_t*>(out_row[qi]), head * kD + dt * 16 + g * 4, v);
+            if (split_out) store_split<4>(reinterpret_cast<uint16_t*>(out_row), head * kD + dt * 16 + g * 4, v);
             else *reinterpret_cast<out4*>(orow + dt * 16) = v;
           }
         }
@@ -554,10 +543,10 @@ void attention_launch(const void* q, const void* k, const void* v, int layout, i
   allow_dynamic_lds(reinterpret_cast<const void*>(kern), (int)Sm::kBytes);
   // A workgroup serves several heads of one sequence: mask rows, positions and zero fill are shared by them, and the
   // chain of dependent loads a workgroup starts with (sequence start, positions, rows) is paid once.  Up to 6 heads
-  // (4 in fp32; 8 for the 128-key kernel, whose start is the longest), in equal groups, as long as about two workgroups per CU
-  // remain: measured best on batches of 100 x 32, 1000 x 64 and 256 x 128 tokens.
+  // (4 in fp32), in equal groups, as long as about two workgroups per CU remain: measured best on batches of 100 x 32 and
+  // 1000 x 64 tokens.
   int hpw = 1;
-  for (int h = NKT >= 8 ? 8 : (sizeof(T) == 2 ? 6 : 4); h > 1; --h)
+  for (int h = sizeof(T) == 2 ? 6 : 4; h > 1; --h)
     if (heads % h == 0 && (long)batch * (heads / h) >= 512) {
       hpw = h;
       break;
@@ -1007,7 +996,7 @@ void attention_flash_launch(const void* q, const void* k, const void* v, int lay
 }
 
 // ------------------------------------------------------------------------------------------
-// fp32 fused attention for 128 < seq_len <= 1024, built like the kernel above: one workgroup of 4 wavefronts per (64 queries,
+// fp32 fused attention for 32 < seq_len <= 1024, built like the kernel above: one workgroup of 4 wavefronts per (64 queries,
 // head, sequence), 16 queries per wavefront, K and V by DMA in stages of 32 keys (two stages of 16 KB), the softmax along
 // with them, everything in float on v_mfma_f32_16x16x4_f32.  A lane's 16-byte V read is four features of one key, one for
 // each of the four feature tiles (row l16 of tile dt is feature 4 l16 + dt), so V needs no transpose and a lane ends up
@@ -1019,7 +1008,10 @@ void attention_flash_launch(const void* q, const void* k, const void* v, int lay
 // ------------------------------------------------------------------------------------------
 constexpr int kF32Keys = 32;                                 // keys per stage
 constexpr int kF32Stage = kF32Keys * kD * 4;                 // bytes of K (and of V) per stage
-constexpr int kF32MinKeys = 128;
+// Up to 32 positions attention_kernel is level or ahead (12 layers, 200 x 32: 4.41 ms either way; one layer, 8 x 32: 90.4 and
+// 91.7 us); beyond, this kernel (12 layers: 7 x 50 1.056 -> 1.025 ms, 500 x 64 17.76 -> 17.61 ms, 9 x 101 1.59 -> 1.39 ms,
+// 40 x 128 4.16 -> 3.91 ms; single layer calls with their masks looked at each time, 200 x 64: 8.30 -> 8.18 ms).
+constexpr int kF32MinKeys = 32;
 constexpr int kF32Smem = 2 * 2 * kF32Stage + kFlMaxKeys * (int)sizeof(int);
 
 __global__ __launch_bounds__(kAttnThreads, 4) void attention_flash_f32_kernel(
@@ -1392,7 +1384,7 @@ void attention_dispatch(const void* q, const void* k, const void* v, int layout,
                         int d, float scaler, bool split_out, const uint8_t* mask_class, hipStream_t stream) {
   // (the streaming kernels address the rows of a sequence with 31 bits)
   const bool far = (uint64_t)seq_len * (uint64_t)(layout == 1 ? packed_ld : kD) * sizeof(T) >= 0x80000000ull;
-  if (d != kD || !head_rows_16b<T>(q, k, v, layout, packed_ld, d) || (far && seq_len > kFlMinKeys))
+  if (d != kD || !head_rows_16b<T>(q, k, v, layout, packed_ld, d) || (far && seq_len > kF32MinKeys))
     attention_generic_launch<T>(q, k, v, layout, packed_ld, attr_mask, dst, seq_start, word_idx, batch, seq_len, heads, d,
                                 scaler, stream);
   else if (sizeof(T) == 2 && seq_len > kFlMinKeys)
@@ -1404,11 +1396,8 @@ void attention_dispatch(const void* q, const void* k, const void* v, int layout,
   else if (seq_len <= 32)
     attention_launch<T, 2>(q, k, v, layout, packed_ld, attr_mask, dst, seq_start, word_idx, batch, seq_len, heads,
                            scaler, split_out, stream);
-  else if (seq_len <= 64)
+  else if constexpr (sizeof(T) == 2)
     attention_launch<T, 4>(q, k, v, layout, packed_ld, attr_mask, dst, seq_start, word_idx, batch, seq_len, heads,
-                           scaler, split_out, stream);
-  else if constexpr (sizeof(T) == 4)
-    attention_launch<T, 8>(q, k, v, layout, packed_ld, attr_mask, dst, seq_start, word_idx, batch, seq_len, heads,
                            scaler, split_out, stream);
 }
 
