@@ -18,6 +18,7 @@
 // 14, 10, 15, 21 us against 17, 17, 19, 59).
 #include <algorithm>
 #include <atomic>
+#include <iterator>
 #include <type_traits>
 
 #include "et_device.hpp"
@@ -74,7 +75,7 @@ __global__ __launch_bounds__(WM * WN * kWave) void gemm_split_kernel(SplitGemmAr
 #if defined(__HIP_DEVICE_COMPILE__)   // device-only types in the body; the host pass only needs the stub
   using Tile = SplitTile<WM, WN, MI, NJ, ST>;
   constexpr int BM = Tile::BM, BN = Tile::BN;
-  constexpr bool kTwoPerSimd = Tile::WAVES == 8 && MI * NJ == 16;
+  constexpr bool kTwoPerSimd = Tile::WAVES == 8 && MI * NJ >= 12;
   typedef __bf16 bf16x8 __attribute__((ext_vector_type(8)));
   extern __shared__ __attribute__((aligned(1024))) unsigned char smem[];
 
@@ -349,15 +350,17 @@ int device_cu_count() {
 // Tile of a launch.  Below a round of the chip a launch takes the k loop of one tile, so small problems want small tiles;
 // large ones want the tile with the fewest operand bytes per product.  A launch takes rounds of tiles over the CUs, each
 // as long as its k-steps (microseconds per k-step below: measured with few workgroups, K = 768 .. 3072) and about 3 us
-// for filling the ring and storing C.
-enum SplitPick { k256x128, k128x128, k64x128, k64x64, k32x64, k32x32 };
+// for filling the ring and storing C.  (The heights of 192 and 96 rows are there for the part-filled last round: 3850 rows,
+// n = 2304 / 768 at k = 768, 3072 + GELU, and 768 at k = 3072: 84, 32, 90, 102 us without them, 70, 28, 84, 90 with; 5500
+// rows: 95, 47, 147, 164 and 95, 40, 120, 133.)
+enum SplitPick { k256x128, k192x128, k128x128, k96x128, k64x128, k64x64, k32x64, k32x32 };
 SplitPick pick_split_tile(int m, int n, int k, int groups) {
-  static constexpr struct { int bm, bn; float step; } kTiles[] = {{256, 128, 1.58f}, {128, 128, 0.97f}, {64, 128, 0.6f},
-                                                                   {64, 64, 0.38f},   {32, 64, 0.26f},   {32, 32, 0.15f}};
+  static constexpr struct { int bm, bn; float step; } kTiles[] = {
+      {256, 128, 1.58f}, {192, 128, 1.33f}, {128, 128, 0.97f}, {96, 128, 0.79f}, {64, 128, 0.6f}, {64, 64, 0.38f}, {32, 64, 0.26f}, {32, 32, 0.15f}};
   const long cus = device_cu_count();
   int best = 0;
   float best_cost = 0.f;
-  for (int i = 0; i < 6; ++i) {
+  for (int i = 0; i < (int)std::size(kTiles); ++i) {
     const long tiles = (long)((m + kTiles[i].bm - 1) / kTiles[i].bm) * ((n + kTiles[i].bn - 1) / kTiles[i].bn) * groups;
     const float cost = (float)((tiles + cus - 1) / cus) * (kTiles[i].step * (float)(k / 32) + 3.f);
     if (i == 0 || cost < best_cost) {
@@ -483,7 +486,9 @@ void launch_gemm_split(const GemmGroups& g, void* C, int ldc, int m_bound, int n
   a.k = k;
   switch (pick_split_tile(m_bound, n, k, g.groups)) {
     case k256x128: return launch_tile<4, 2, 4, 4, 2>(a, g.gelu, g.groups, stream);
+    case k192x128: return launch_tile<4, 2, 3, 4, 2>(a, g.gelu, g.groups, stream);
     case k128x128: return launch_tile<2, 4, 4, 2, 3>(a, g.gelu, g.groups, stream);
+    case k96x128: return launch_tile<2, 4, 3, 2, 3>(a, g.gelu, g.groups, stream);
     case k64x128: return launch_tile<2, 4, 2, 2, 4>(a, g.gelu, g.groups, stream);
     case k64x64: return launch_tile<4, 2, 1, 2, 6>(a, g.gelu, g.groups, stream);
     case k32x64: return launch_tile<2, 4, 1, 1, 8>(a, g.gelu, g.groups, stream);

@@ -20,11 +20,14 @@ def _operands(m, n, kk, positive=False):
     return (a.abs(), b.abs(), bias) if positive else (a, b, bias)
 
 
-# rows and columns around 32, 64, 128 and 256 (the tiles' sides), one and an odd number of k-steps of 32, fewer k-steps
+# rows and columns around 32, 64, 128 and 256 (tiles' sides), one and an odd number of k-steps of 32, fewer k-steps
 # than the LDS ring of the small tiles holds, and grids of one to several rounds of the chip
 @pytest.mark.parametrize("m,n,kk", [(1, 4, 32), (31, 36, 32), (33, 64, 96), (64, 100, 160), (65, 768, 768), (127, 132, 64),
                                     (160, 768, 3072), (257, 136, 96), (700, 768, 3072), (1025, 2304, 768),
-                                    (4200, 768, 768), (9000, 1536, 128)])
+                                    (4200, 768, 768), (9000, 1536, 128),
+                                    # tiles of 192 and of 96 rows: last row of a tile, one behind it, one and several rounds
+                                    (7872, 768, 768), (5761, 772, 768), (7999, 768, 3072), (8000, 2304, 96), (3072, 768, 768), (3073, 768, 3072),
+                                    (1000, 2304, 768)])
 @pytest.mark.parametrize("positive", [False, True])
 def test_gemm_split(m, n, kk, positive):
     print("gemm_split", m, n, kk, positive, flush=True)
