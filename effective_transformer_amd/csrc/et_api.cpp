@@ -294,6 +294,7 @@ struct LayerCall {
   void* out;
   int B, S, heads, d;
   int rows;                           // launches are sized for this many rows
+  bool rows_exact = false;            //   ... which is the count itself: no kernel asks the device for it
   char* workspace;
   bool from_split_ready = false;      // split layers: the split rows of `from` are in the workspace's intermediate already
   bool write_out_split = false;       //   ... and those of `out` are to be left there
@@ -306,7 +307,7 @@ et_status run_layer(et_handle h, const LayerCall& c) {
   const int B = c.B, S = c.S, H = c.heads * c.d, F = 4 * H, rows = c.rows;
   const LayerWs ws = layer_ws(c.dtype, B, S, c.heads, c.d);
   const et::DType dt = to_dt(c.dtype);
-  const int32_t* T = c.count;
+  const int32_t* T = c.rows_exact ? nullptr : c.count;
   hipStream_t st = c.stream;
   et_status s;
   const size_t e = et::elem_size(dt);
@@ -853,18 +854,18 @@ et_status et_encoder(et_handle h, et_dtype dtype, int num_layers, const et_layer
   c.workspace = layer_base;
   c.stream = st;
   int T = -1;
+  if (wait_for_layers && scan.host_word) {
+    // The count is there when the scan ends and the host has it while the input rows are still being moved: the layers
+    // are launched for exactly that many rows (other threads may use the handle meanwhile).
+    entry.lock.unlock();
+    s = wait_for_count(h, scan.host_word, scan.host_tag, count, st, &T);
+    entry.lock.lock();
+    if (s != ET_OK) return s;
+    c.rows = std::min(std::max(T, 0), B * S);
+    c.rows_exact = true;
+  }
   int cur = 0;
   for (int l = 0; l < num_layers && c.rows > 0; ++l) {
-    if (l == 1 && wait_for_layers && scan.host_word) {
-      // the first layer, sized for every position, is in the queue: the GPU has work while the host waits for the count
-      // (other threads may use the handle meanwhile)
-      entry.lock.unlock();
-      s = wait_for_count(h, scan.host_word, scan.host_tag, count, st, &T);
-      entry.lock.lock();
-      if (s != ET_OK) return s;
-      c.rows = std::min(std::max(T, 0), B * S);
-      if (c.rows == 0) break;
-    }
     c.w = weights + l;
     c.prep = prepared ? prepared + l : nullptr;
     c.from = c.to = x[cur];
