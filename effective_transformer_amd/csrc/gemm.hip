@@ -856,7 +856,7 @@ __global__ __launch_bounds__(kPThreads) void gemm_f16_pair_kernel(GemmArgs args)
 // ------------------------------------------------------------------------------------------
 // fp16, problems below the persistent regime, B k-contiguous ([n][k]): one (32 MI) x (32 NJ) tile per workgroup,
 // 4 wavefronts (2 x 2), LDS slots of two k-steps like the persistent kernel above.  MI = 1 .. 4 blocks of 32 rows,
-// NJ = 2, 4, 6 or 8 blocks of 32 columns.
+// NJ = 1, 2, 4, 6 or 8 blocks of 32 columns.
 //
 // With the weights in TF's [k][n] order a small tile reads its B operands with 8-byte LDS reads (half the rate of
 // 16-byte ones) and transposes them in registers, and its A rows arrive in 64-byte pieces; a 64 x 128 tile then spends
@@ -879,7 +879,9 @@ __global__ __launch_bounds__(kHThreads) __attribute__((amdgpu_waves_per_eu(2))) 
 #if defined(__HIP_DEVICE_COMPILE__)   // device-only types in the body; the host pass only needs the stub
   using Tile = BtTile<MI, NJ, ST>;
   static_assert(Tile::DMA * (ST - 1) < 64, "the DMA instructions in flight must fit the 6-bit vmcnt");
-  using HalfN = typename std::conditional<NJ == 8, half8, typename std::conditional<NJ == 4, half4, half2v>::type>::type;
+  typedef _Float16 half1v __attribute__((ext_vector_type(1)));
+  using HalfN = typename std::conditional<NJ == 8, half8, typename std::conditional<NJ == 4, half4,
+                                          typename std::conditional<NJ == 1, half1v, half2v>::type>::type>::type;
   constexpr int BM = Tile::BM, BN = Tile::BN, WC = 16 * NJ;       // WC: columns of a wave tile
   extern __shared__ __attribute__((aligned(1024))) unsigned char smem[];
 
@@ -1006,7 +1008,7 @@ __global__ __launch_bounds__(kHThreads) __attribute__((amdgpu_waves_per_eu(2))) 
   const int col = n0 + wn * WC + l16 * (NJ == 6 ? 4 : NJ);
   if (col < N) {
     _Float16* C = (_Float16*)args.C + (size_t)grp * N + col;
-    if constexpr (NJ == 2 || NJ == 4 || NJ == 8) {
+    if constexpr (NJ == 1 || NJ == 2 || NJ == 4 || NJ == 8) {
       // bias added in half on the rounded product, as the reference's next kernel does; without a bias the addend is
       // -0, which leaves every value (and the sign of a zero) as it is
       HalfN biasv;
@@ -1354,6 +1356,8 @@ void launch_f16_persistent(GemmArgs a, hipStream_t stream, bool b_transposed) {
 // CU's units: the smallest tile that still gives every workgroup a CU to itself ("solo", ring of 3 to 5 slots), or
 // two workgroups per CU ("duo", rings that fit twice into the LDS) where 2 (MI + NJ) / 1.3 is less: two resident
 // workgroups draw 1.3 times the rows of one.  A 96-column wave tile stores in two pieces and counts one unit more.
+// 32 x 32 is for launches that stay within a round with it (320 rows at n = 768; up to 32 rows: k = 768 / 3072 5.1 / 9.7 us
+// on 32 x 64, 4.5 / 8.3 us on it; 12 layers on one query 469 -> 439 us, on 180 rows 539 -> 518 us).
 // Ties go to the tile whose XCD bands touch fewer distinct operand rows.  (Timed for n = 768 .. 4096, k = 768 .. 4096,
 // 250 .. 16000 rows with the weights of twelve layers taking turns: within 2 % of the best tile on average.)
 struct BtPick {
@@ -1366,7 +1370,7 @@ BtPick pick_bt_tile(int m_bound, int n, int groups, int cus, bool proven_only) {
   float best_cost = 0.f;
   long best_band = 0;
   // (the other combinations of 1 .. 4 row blocks and 2 .. 8 column blocks never come out ahead of these)
-  static constexpr struct { int mi, nj; bool duo; } kTiles[] = {{1, 2, true}, {2, 2, true}, {2, 4, true}, {3, 2, true},
+  static constexpr struct { int mi, nj; bool duo; } kTiles[] = {{1, 1, false}, {1, 2, true}, {2, 2, true}, {2, 4, true}, {3, 2, true},
                                                                  {3, 4, true}, {3, 6, true}, {4, 2, true}, {4, 4, true},
                                                                  {4, 6, true}, {4, 8, false}};
   for (const auto& tile : kTiles) {
@@ -1401,6 +1405,7 @@ BtPick pick_bt_tile(int m_bound, int n, int groups, int cus, bool proven_only) {
 
 void launch_bt_tile(BtPick p, const GemmArgs& a, hipStream_t stream) {
   switch (p.mi * 100 + p.nj * 10 + (p.duo ? 1 : 0)) {
+    case 110: return launch_f16_bt<1, 1, 5>(a, stream);
     case 120: return launch_f16_bt<1, 2, 5>(a, stream);
     case 121: return launch_f16_bt<1, 2, 3>(a, stream);
     case 220: return launch_f16_bt<2, 2, 4>(a, stream);
