@@ -874,7 +874,9 @@ struct BtTile {
   static constexpr int DMA = MI + NJ;                         // instructions per wavefront and pair: MI for A, NJ for B^T
 };
 
-template <int MI, int NJ, int ST>
+// COLUMNS: the tile order runs down the columns of tiles instead of along the rows (see band_rows); a template parameter,
+// because the choice at run time would put 0.3 us in front of the first request of every launch.
+template <int MI, int NJ, int ST, bool COLUMNS>
 __global__ __launch_bounds__(kHThreads) __attribute__((amdgpu_waves_per_eu(2))) void gemm_f16_bt_kernel(GemmArgs args) {
 #if defined(__HIP_DEVICE_COMPILE__)   // device-only types in the body; the host pass only needs the stub
   using Tile = BtTile<MI, NJ, ST>;
@@ -889,8 +891,15 @@ __global__ __launch_bounds__(kHThreads) __attribute__((amdgpu_waves_per_eu(2))) 
   const int tiles_n_all = args.tiles_n * args.groups;
   const int tile = remap_valid_tile(blockIdx.x, ((rows + BM - 1) / BM) * tiles_n_all);
   if (tile < 0) return;
-  const int tm = tile / tiles_n_all;
-  const int tn_all = tile - tm * tiles_n_all;
+  int tm, tn_all;
+  if constexpr (COLUMNS) {
+    const int tiles_m = (rows + BM - 1) / BM;
+    tn_all = tile / tiles_m;
+    tm = tile - tn_all * tiles_m;
+  } else {
+    tm = tile / tiles_n_all;
+    tn_all = tile - tm * tiles_n_all;
+  }
   const int grp = tn_all / args.tiles_n;
   const int m0 = tm * BM;
   const int n0 = (tn_all - grp * args.tiles_n) * BN;
@@ -1225,16 +1234,37 @@ void launch_f16(GemmArgs a, hipStream_t stream) {
   kern<<<a.per_xcd * kXcds, kHThreads, Tile::SMEM_BYTES, stream>>>(a);
 }
 
+// Distinct operand rows (of A and of B^T) that the tiles of one XCD's band touch, which is what its L2 has to fetch, with
+// the tile order running along the rows of tiles or down the columns.
+constexpr int kColumnRows = 1024;
+struct BandRows {
+  long along, down;
+};
+BandRows band_rows(long tiles_m, long tiles_n, int bm, int bn) {
+  const long band = (tiles_m * tiles_n + kXcds - 1) / kXcds;
+  auto rows = [&](long inner, int b_inner, int b_outer) {
+    return std::min(band, inner) * b_inner + (band + inner - 1) / inner * b_outer;
+  };
+  return {rows(tiles_n, bn, bm), rows(tiles_m, bm, bn)};
+}
+
 template <int MI, int NJ, int ST>
 void launch_f16_bt(GemmArgs a, hipStream_t stream) {
   using Tile = BtTile<MI, NJ, ST>;
-  auto kern = gemm_f16_bt_kernel<MI, NJ, ST>;
-  allow_dynamic_lds(reinterpret_cast<const void*>(kern), (int)Tile::SMEM_BYTES);
   a.tiles_m = (a.m_bound + Tile::BM - 1) / Tile::BM;
   a.tiles_n = (a.n + Tile::BN - 1) / Tile::BN;
   const int total = a.tiles_m * a.tiles_n * a.groups;
   a.per_xcd = (total + kXcds - 1) / kXcds;
-  kern<<<a.per_xcd * kXcds, kHThreads, Tile::SMEM_BYTES, stream>>>(a);
+  auto go = [&](auto kern) {
+    allow_dynamic_lds(reinterpret_cast<const void*>(kern), (int)Tile::SMEM_BYTES);
+    kern<<<a.per_xcd * kXcds, kHThreads, Tile::SMEM_BYTES, stream>>>(a);
+  };
+  // Few rows want the columns: the weights are then spread over the XCDs instead of read by each of them (12 layers on 580
+  // rows of BERT-base 594 -> 572 us, on 300 rows of BERT-large 633 -> 575 us).  Where the two orders fetch about the same
+  // they take the same time, and from about 1000 rows on the columns lose up to 1 %.
+  const BandRows band = band_rows(a.tiles_m, (long)a.tiles_n * a.groups, Tile::BM, Tile::BN);
+  if (a.m_bound <= kColumnRows && 4 * band.down <= 3 * band.along) go(gemm_f16_bt_kernel<MI, NJ, ST, true>);
+  else go(gemm_f16_bt_kernel<MI, NJ, ST, false>);
 }
 
 int device_cu_count() {
@@ -1388,10 +1418,7 @@ BtPick pick_bt_tile(int m_bound, int n, int groups, int cus, bool proven_only) {
     } else {
       continue;
     }
-    // distinct operand rows (of A and of B^T) that the tiles of one XCD's band touch: what its L2 has to fetch
-    const long per_band = (wgs + kXcds - 1) / kXcds;
-    const long band = (per_band >= tiles_n ? (per_band + tiles_n - 1) / tiles_n : 1) * 32 * mi +
-                      std::min(per_band, tiles_n) * 32 * nj;
+    const long band = band_rows((m_bound + 32 * mi - 1) / (32 * mi), tiles_n, 32 * mi, 32 * nj).along;
     if (best.mi == 0 || cost < best_cost || (cost == best_cost && band < best_band)) {
       best.mi = mi;
       best.nj = nj;
