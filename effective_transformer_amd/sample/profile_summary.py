@@ -22,9 +22,9 @@ import sys
 from .workloads import WORKLOADS
 
 ROLES = ["QKV", "attention", "attention out", "LayerNorm 1", "FFN up + GELU", "FFN down", "LayerNorm 2"]
-SIDE = ("scan_index", "compress_rows", "embed_layernorm", "seq_start", "seq_order", "restore_rows")
+SIDE = ("scan_index", "compress_rows", "embed_layernorm", "seq_start", "seq_order", "mask_class", "restore_rows")
 LAYER_KINDS = ("attention", "bias_residual_layernorm", "gemm_f16_pair", "gemm_f16_bt", "gemm_f16_persistent", "gemm_f16_kernel",
-               "gemm_f32")
+               "gemm_f32", "gemm_split")
 
 
 def describe(workload: str) -> str:
@@ -45,7 +45,7 @@ def short(name: str) -> str:
 def kind(name: str) -> str:
     """What a dispatch is, by its kernel name."""
     for k in SIDE + ("attention", "bias_residual_layernorm", "bias_gelu", "layer_prologue", "gemm_f16_pair", "gemm_f16_bt",
-                     "gemm_f16_persistent", "gemm_f16_kernel", "gemm_f32", "mfma_ceiling", "copyBuffer"):
+                     "gemm_f16_persistent", "gemm_f16_kernel", "gemm_f32", "gemm_split", "mfma_ceiling", "copyBuffer"):
         if k in name:
             return k
     return name[:30]
