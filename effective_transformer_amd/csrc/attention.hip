@@ -602,8 +602,10 @@ inline int attention_cu_count() {
 // for P.V, here before the division by the sum instead of after it).
 //
 // A block of 16 queries whose mask rows are 1 up to the sequence's last token and 0 from there on (`mask_class`, see
-// mask_class_kernel) needs no mask: keys behind the last token have weight exp(-10000 - maximum) = 0 and are not visited.
-// Any other block reads its mask rows and visits every key.
+// mask_class_kernel) needs no mask and visits no key behind the last token.  Such a key has score -10000 and value 0.  Below
+// 1024 positions its weight exp(-10000 - maximum) is 0, as the maximum is clamped at 0; at 1024 there is no clamp, and the
+// unvisited keys enter the maximum and the sum at the end (`unseen`).  Any other block reads its mask rows and visits every
+// key.
 // ------------------------------------------------------------------------------------------
 constexpr int kFlKeys = 64;                                  // keys per stage
 constexpr int kFlStage = kFlKeys * 128;                      // bytes of K (and of V) per stage
@@ -619,6 +621,17 @@ constexpr int kFlMinKeys = 64;
                                                              // -infinity weigh nothing against it
 typedef __fp16 half4_fp16 __attribute__((ext_vector_type(4)));
 constexpr int kFlSmem = kFlRing * 2 * kFlStage + kFlMaxKeys * (int)sizeof(int);
+
+// Keys of score -10000 and value 0 that a block at 1024 positions has not visited (0 below, where they weigh nothing): what the
+// maximum (log2 units) is at least, and what they add to a sum taken against the exponent `ref` (infinity where they leave
+// nothing to the visited keys).
+__device__ __forceinline__ int unseen_keys(bool plain, int seq_len, int n) { return plain && seq_len == kFlMaxKeys ? seq_len - n : 0; }
+__device__ __forceinline__ float lowest_maximum(int seq_len, int unseen) {
+  return seq_len < kFlMaxKeys ? 0.f : unseen > 0 ? -10000.0f * kLog2e : -INFINITY;
+}
+__device__ __forceinline__ float unseen_weight(int unseen, float ref) {
+  return unseen > 0 ? (float)unseen * __builtin_amdgcn_exp2f(__builtin_fmaf(-10000.0f, kLog2e, -ref)) : 0.f;
+}
 
 // class of every block of 16 query positions: 1 = the rows of the mask are 1 for keys up to the last token's and 0 beyond
 template <typename T>
@@ -964,12 +977,14 @@ __global__ __launch_bounds__(WAVES * kWave, OCC) void attention_flash_kernel(
   else run(std::false_type{});
   wide_wait_dma();                                                     // no DMA may still target this workgroup's LDS when it ends
 
+  const int unseen = unseen_keys(plain, seq_len, n);
+  const float lowest = lowest_maximum(seq_len, unseen);
 #pragma unroll
   for (int u = 0; u < QSUB; ++u) {
     // the reference divides by (sum of exp(score - maximum)) + 1e-6, its maximum clamped at 0 below 1024 keys: in units of
     // 2^ref that is the sum here + 1e-6 * 2^(maximum - ref)
-    const float mx = fmaxf(xor_lanes_16_32_max(top[u]), seq_len < kFlMaxKeys ? 0.f : -INFINITY);
-    const float inv = 1.0f / (l[u][0] + 1e-6f * __builtin_amdgcn_exp2f(mx - ref[u]));
+    const float mx = fmaxf(xor_lanes_16_32_max(top[u]), lowest);
+    const float inv = 1.0f / (l[u][0] + unseen_weight(unseen, ref[u]) + 1e-6f * __builtin_amdgcn_exp2f(mx - ref[u]));
     if (tq[u] < 0) continue;
     T* orow = dst + (size_t)(t0 + tq[u]) * H + head * kD + g * 4;
 #pragma unroll
@@ -1214,8 +1229,9 @@ __global__ __launch_bounds__(kAttnThreads, 4) void attention_flash_f32_kernel(
   if (plain) run(std::true_type{});
   else run(std::false_type{});
 
-  const float mx = fmaxf(xor_lanes_16_32_max(top), seq_len < kFlMaxKeys ? 0.f : -INFINITY);
-  const float sum = xor_lanes_16_32_sum(l);
+  const int unseen = unseen_keys(plain, seq_len, n);
+  const float mx = fmaxf(xor_lanes_16_32_max(top), lowest_maximum(seq_len, unseen));
+  const float sum = xor_lanes_16_32_sum(l) + unseen_weight(unseen, ref);
   if (tq < 0) return;
   const float inv = 1.0f / (sum + 1e-6f * __builtin_amdgcn_exp2f(mx - ref));
   // o[dt][r] is feature 16 g + 4 r + dt

@@ -45,3 +45,37 @@ def test_masks_of_every_kind(S, B, dtype):
     err = np.abs(got[valid].astype(np.float64) - want[valid].astype(np.float64)).max()
     print("  max abs diff", err, flush=True)
     assert err < (2e-2 if dtype == "fp16" else 1e-4)
+
+
+# At 1024 positions the maximum is not clamped at 0: keys behind the last token (score -10000, value 0) take weight where every
+# score of a query lies about as low.  Q and K are their biases here, so that a head's scores are one number, exactly: fp32
+# -20000 and -9999 after scaling, fp16 -infinity (the score is stored in half) and an ordinary one.  The tolerances are those of
+# the layer (fp32 1e-4, fp16 2e-2): a wrong weight moves the attention's output by its own size.
+@pytest.mark.parametrize("dtype", ["fp32", "fp16"])
+@pytest.mark.parametrize("S", [1024, 1023])
+def test_scores_below_the_mask_bias(S, dtype):
+    print("scores below the mask bias", S, dtype, flush=True)
+    el = np.float16 if dtype == "fp16" else np.float32
+    lens = np.array([1, 40, 700, 1000, S - 1])
+    B = len(lens)
+    wl = Workload("low_scores", S, dtype, 1, B, S, 2, 64, 512)
+    rng = np.random.RandomState(S)
+    weights = make_layer_weights(wl, rng, random_affine=True)
+    for slot in (0, 1, 2, 3):
+        weights[slot] = np.zeros_like(weights[slot])
+    q, k = weights[1].reshape(2, 64), weights[3].reshape(2, 64)
+    q[:] = 0
+    q[:, 0], k[:, 0] = (16, (-10000, -4999.5)) if dtype == "fp32" else ((1000, 1), (-1000, 1))
+    mask = (np.arange(S)[None] < lens[:, None]).astype(np.int32)
+    mask[2, 20:90] = 0                                       # a hole: keys that the mask does not hide, score and value 0
+    attr = np.ascontiguousarray(np.broadcast_to(mask[:, None], (B, S, S))).astype(el)
+    attr[2, :, 20:90] = 1
+    # (the last query's row is not of the plain form: its block takes the general path, the others are as they were)
+    attr[3, 999, 1] = 0
+    w = dict(wl=wl, x=rng.randn(B, S, wl.H).astype(el), weights=weights, mask=mask, attr_mask=attr)
+    got, want = run_encoder(w), o.encoder(w["x"], mask, attr, weights, wl.heads, wl.d, dtype)
+    valid = mask.astype(bool)
+    assert np.isfinite(want[valid]).all()
+    err = np.abs(got[valid].astype(np.float64) - want[valid].astype(np.float64)).max()
+    print("  max abs diff", err, flush=True)
+    assert err < (2e-2 if dtype == "fp16" else 1e-4)
