@@ -347,6 +347,14 @@ def effective_transformer_first_token(from_tensor: torch.Tensor, valid_word_num:
 
 # --------------------------------------------------------------------------- the glue
 
+def _require_masks(B: int, S: int, input_mask: torch.Tensor, attention_mask: torch.Tensor) -> None:
+    """The masks of B sequences of S positions, in full: the kernels read that much of them."""
+    if input_mask.dim() != 2 or input_mask.shape[0] < B or input_mask.shape[1] != S:
+        raise ValueError("mask %s must be [%d, %d]" % (tuple(input_mask.shape), B, S))
+    if attention_mask.shape[-1] != S or attention_mask.numel() < B * S * S:
+        raise ValueError("attention mask %s must be [%d, %d, %d]" % (tuple(attention_mask.shape), B, S, S))
+
+
 class EffectiveTransformerEncoder:
     """Input -> L x Layer -> Output with the weights resident on the device (the reference bakes
     them into op attributes at graph build, python/effective_transformer/__init__.py:48-76)."""
@@ -409,18 +417,33 @@ class EffectiveTransformerEncoder:
 
     def __call__(self, from_tensor: torch.Tensor, input_mask: torch.Tensor, attention_mask: torch.Tensor,
                  sync_count: bool = True, rows_bound: Optional[int] = None) -> torch.Tensor:
-        """rows_bound (with sync_count=False): an upper bound of the valid-token count that the caller vouches for;
+        """from_tensor [B,S,H]; input_mask [B,S] and attention_mask [B,S,S], or more sequences than B (the first B count).
+        rows_bound (with sync_count=False): an upper bound of the valid-token count that the caller vouches for;
         the launches are sized for that many rows instead of B*S (rows beyond it would not be computed)."""
+        B, S = from_tensor.shape[0], input_mask.shape[1]
+        if from_tensor.numel() != B * S * self.head_num * self.size_per_head:
+            raise ValueError("from_tensor %s must be [batch, %d, %d] (mask, heads * size)" %
+                             (tuple(from_tensor.shape), S, self.head_num * self.size_per_head))
+        _require_masks(B, S, input_mask, attention_mask)
         _require_cuda(from_tensor)
         if from_tensor.dtype != self.dtype:
             raise TypeError("from_tensor must have the dtype of the weights")
         batch = _lib.EncoderBatch()
         batch.from_tensor = from_tensor.data_ptr()
-        return self._run(batch, from_tensor.shape, input_mask, attention_mask, sync_count, rows_bound)
+        return self._run(batch, B, S, from_tensor.shape, input_mask, attention_mask, sync_count, rows_bound)
 
     def forward_ids(self, input_ids, token_type_ids, input_mask, attention_mask, embeddings: "EmbeddingWeights",
                     sync_count: bool = True) -> torch.Tensor:
-        """Embedding block + encoder from token ids: the packed token matrix is produced directly."""
+        """Embedding block + encoder from token ids: the packed token matrix is produced directly.  The batch is that of
+        input_mask [B,S]; the other tensors may hold more sequences."""
+        B, S = input_mask.shape
+        for ids in (input_ids,) if token_type_ids is None else (input_ids, token_type_ids):
+            if ids.shape[-1] != S or ids.numel() < B * S:
+                raise ValueError("ids %s must be [%d, %d] (mask)" % (tuple(ids.shape), B, S))
+        if embeddings.hidden != self.head_num * self.size_per_head:
+            raise ValueError("embeddings of %d columns for a hidden size of %d" %
+                             (embeddings.hidden, self.head_num * self.size_per_head))
+        _require_masks(B, S, input_mask, attention_mask)
         _require_cuda(input_ids)
         if input_ids.dtype != torch.int32 or (token_type_ids is not None and token_type_ids.dtype != torch.int32):
             raise TypeError("ids and mask must be int32")
@@ -432,9 +455,9 @@ class EffectiveTransformerEncoder:
         if token_type_ids is not None:
             _require_cuda(token_type_ids)
             batch.token_type_ids = token_type_ids.data_ptr()
-        return self._run(batch, (*input_mask.shape, embeddings.hidden), input_mask, attention_mask, sync_count, None)
+        return self._run(batch, B, S, (B, S, embeddings.hidden), input_mask, attention_mask, sync_count, None)
 
-    def _run(self, batch, shape, input_mask, attention_mask, sync_count, rows_bound):
+    def _run(self, batch, B, S, shape, input_mask, attention_mask, sync_count, rows_bound):
         """One et_encoder call.  sync_count: the valid-token count is read back once per batch, so that the launches of
         layers 2 .. L are sized exactly (the reference reads it back in every layer); the host waits for it behind the
         launches of the first layer, which is sized for B*S rows and bounded on the device, so the GPU never idles for it."""
@@ -444,7 +467,6 @@ class EffectiveTransformerEncoder:
             raise TypeError("mask must be int32")
         if attention_mask.dtype != self.dtype:
             raise TypeError("attr_mask must have the dtype of from_tensor")
-        B, S = input_mask.shape
         dev = input_mask.device
         out = torch.empty(shape, dtype=self.dtype, device=dev)
         code = _dtype_code(self.dtype)
