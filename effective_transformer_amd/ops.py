@@ -203,13 +203,15 @@ class LayerWeights:
         self._prepared_tensors: List[torch.Tensor] = []
 
     def prepare(self, every_kernel: bool = True) -> "LayerWeights":
-        """For weights that stay as they are: the copies of the dense kernels that the layer op's GEMMs read, made once
-        instead of on every call.  fp16: k-contiguous ([out,in]); fp32: k-contiguous split rows (et_gemm_split in et.h).
+        """For weights that stay as they are: k-contiguous ([out,in]) copies of the dense kernels, which the layer op's GEMMs
+        then read instead of making them on every call (fp16 only).  A no-op for fp32, whose weights are read on every call
+        and may change in place between calls.
         every_kernel=False: only the kernels of the wide projections (Q, K, V, FFN up)."""
-        # hidden sizes the tuned GEMMs do not take have no copies: k in multiples of 64 in fp16, of 32 in fp32
+        if self.t["attr_kernel_q"].dtype != torch.float16:
+            return self
+        # the k-contiguous kernels take k in multiples of 64; other hidden sizes run the [k][n] kernels
         hq = self.t["attr_kernel_q"].shape[0]
-        half = self.t["attr_kernel_q"].dtype == torch.float16
-        if hq % (64 if half else 32) != 0:
+        if hq % 64 != 0:
             return self
         lib = _lib.load()
         dev = self.t["attr_kernel_q"].device
@@ -224,15 +226,14 @@ class LayerWeights:
             # the copies of Q, K, V and the attention output kernel lie one behind the other: one region for the layer in
             # front of this one to request (et_layer_prepared.warm)
             together = [nm for nm, _ in names if nm.startswith("attr_") and tuple(self.t[nm].shape) == (hq, hq)]
-            width, dt = (1, torch.float16) if half else (3, torch.bfloat16)
-            block = torch.empty(len(together), hq, width * hq, dtype=dt, device=dev)
+            block = torch.empty(len(together), hq, hq, dtype=torch.float16, device=dev)
             self.warm_block = block if len(together) >= 3 else None
             for src_name, field in names:
                 src = self.t[src_name]
                 k, n = src.shape
                 dst = block[together.index(src_name)] if src_name in together else \
-                    torch.empty(n, width * k, dtype=dt, device=dev)
-                _lib.check(lib.et_transpose_weight(h, _dtype_code(src.dtype), _p(src), _p(dst), k, n, _stream()), h)
+                    torch.empty(n, k, dtype=src.dtype, device=dev)
+                _lib.check(lib.et_transpose_weight(h, _lib.ET_FP16, _p(src), _p(dst), k, n, _stream()), h)
                 self._prepared_tensors.append(dst)
                 setattr(prep, field, dst.data_ptr())
         self.prepared = prep
@@ -361,8 +362,9 @@ class EffectiveTransformerEncoder:
 
     def __init__(self, num_layers: int, head_num: int, size_per_head: int, weights_value: Sequence, dtype: torch.dtype,
                  device="cuda", prepare: bool = True):
-        """prepare: the weights are constants of this object, so the k-contiguous copies the large-M GEMMs want are
-        made here once (fp16) instead of in every layer call."""
+        """prepare (fp16): the weights are constants of this object, so the k-contiguous copies the GEMMs read are made here
+        once instead of in every layer call; tensors handed in and changed in place afterwards are not seen.  fp32 weights
+        are read anew by every call."""
         if len(weights_value) != 16 * num_layers:
             raise ValueError("expected %d weight tensors, got %d" % (16 * num_layers, len(weights_value)))
         self.device = torch.device(device)

@@ -72,24 +72,23 @@ class DeviceBuffer {
 // object owns only its scratch: packed activations, index arrays, workspaces.  Not thread-safe; one object per stream.
 class Encoder {
  public:
-  // prepare: the weights stay as they are for the life of this object, so the copies of the dense kernels that the GEMMs
-  // read (k-contiguous; fp32: as split rows) are made here once (on the device's default stream, waited for) instead of in
-  // every layer call.
+  // prepare (fp16): the weights stay as they are for the life of this object, so the k-contiguous copies of the dense kernels
+  // that the GEMMs read are made here once (on the device's default stream, waited for) instead of in every layer call.
+  // fp32 weights are read anew by every call.
   Encoder(int device, et_dtype dtype, int head_num, int size_per_head, std::vector<et_layer_weights> layers,
           bool prepare = true)
       : handle_(device), dtype_(dtype), heads_(head_num), d_(size_per_head), layers_(std::move(layers)) {
     prepared_.assign(layers_.size(),
                      et_layer_prepared{nullptr, nullptr, nullptr, nullptr, nullptr, nullptr, nullptr, nullptr, 0, 0});
-    // (hidden sizes in multiples of 64, fp32 of 32; others run on the weights as they are)
-    if (!prepare || ((size_t)head_num * size_per_head) % (dtype == ET_FP16 ? 64 : 32) != 0) return;
+    // (the k-contiguous kernels take hidden sizes in multiples of 64; others run on the weights as they are)
+    if (!prepare || dtype != ET_FP16 || ((size_t)head_num * size_per_head) % 64 != 0) return;
     check_hip(hipSetDevice(device), "hipSetDevice");
     const size_t H = (size_t)head_num * size_per_head;
-    const size_t e = dtype == ET_FP16 ? 2 : 6;             // bytes per value of a copy
-    char* dst = (char*)wt_.reserve(layers_.size() * 12 * H * H * e);
+    char* dst = (char*)wt_.reserve(layers_.size() * 12 * H * H * 2);
     auto transposed = [&](const void* src, int k, int n) {
       void* out = dst;
-      check(et_transpose_weight(handle_.get(), dtype, src, out, k, n, nullptr), handle_.get());
-      dst += (size_t)k * n * e;
+      check(et_transpose_weight(handle_.get(), ET_FP16, src, out, k, n, nullptr), handle_.get());
+      dst += (size_t)k * n * 2;
       return (const void*)out;
     };
     for (size_t l = 0; l < layers_.size(); ++l) {
@@ -106,7 +105,7 @@ class Encoder {
     // would otherwise be read cold
     for (size_t l = 0; l + 1 < layers_.size(); ++l) {
       prepared_[l].warm = prepared_[l + 1].attr_kernel_Q_t;
-      prepared_[l].warm_bytes = 4 * H * H * e;
+      prepared_[l].warm_bytes = 4 * H * H * 2;
     }
     check_hip(hipStreamSynchronize(nullptr), "hipStreamSynchronize");
   }
