@@ -390,22 +390,25 @@ class EffectiveTransformerEncoder:
         self._table: Optional[tuple] = None
 
     def _layer_table(self):
-        """The layers' weight and prepared structs as the arrays et_encoder takes.  Every prepared struct is made a view of
-        its array element, so that changes to one reach the next call; a layer that has been prepared anew since, or
-        replaced, has the table made again."""
+        """The layers' weight and prepared structs as the arrays et_encoder takes.  Every struct is made a view of its array
+        element, so that changes to its members reach the next call; a layer whose structs have been replaced since (prepared
+        anew, or taken into another encoder's table), or that has been replaced itself, has the table made again."""
         t = self._table
         if t is not None and len(t[0]) == len(self.layers) and \
-                all(w is ref and w.prepared is p for w, ref, p in zip(self.layers, t[0], t[1])):
+                all(w is ref and w.struct is s and w.prepared is p for w, (ref, s, p) in zip(self.layers, t[0])):
             return t
         with self._lock:
             n = len(self.layers)
             weights, prepared = (_lib.LayerWeights * n)(), (_lib.LayerPrepared * n)()
             for l, w in enumerate(self.layers):
                 weights[l] = w.struct
+                w.struct = weights[l]
                 if w.prepared is not None:
                     prepared[l] = w.prepared
                     w.prepared = prepared[l]
-            self._table = t = (list(self.layers), [w.prepared for w in self.layers], weights, prepared)
+            t = ([(w, w.struct, w.prepared) for w in self.layers], weights, prepared)
+            # (a layer used more than once has several elements and one view: its table is made for every call)
+            self._table = t if len(set(map(id, self.layers))) == n else None
             return t
 
     @classmethod
@@ -489,7 +492,7 @@ class EffectiveTransformerEncoder:
         batch.batch_size, batch.seq_len = B, S
         nbytes = lib.et_encoder_workspace_bytes(code, B, S, self.head_num, self.size_per_head)
         ws = _workspace(dev, "encoder", nbytes)
-        _, _, weights, prepared = self._layer_table()
+        _, weights, prepared = self._layer_table()
         h = handle(dev)
         _lib.check(lib.et_encoder(h, code, len(self.layers), weights, prepared, C.byref(batch), self.head_num,
                                   self.size_per_head, ws.data_ptr(), ws.numel(), stream), h)

@@ -1,10 +1,12 @@
 """Tensors that do not fit each other are refused by the host before anything is launched; a batch of fewer sequences than its
 masks hold is not one of them."""
+import threading
+
 import numpy as np
 import pytest
 import torch
 
-from effective_transformer_amd import ops
+from effective_transformer_amd import _lib, ops
 
 
 def _encoder(heads=2, d=64, dtype=torch.float32):
@@ -50,3 +52,36 @@ def test_fewer_sequences_than_the_masks_hold(dtype):
     assert got.shape == x[:3].shape and torch.equal(got, want)
     assert torch.equal(enc(x[:3], mask, attr, sync_count=False), want)
     assert torch.equal(enc(x[:3], mask, attr[:, None]), want)        # [B,1,S,S]
+
+
+def _layer(n):
+    slots = [torch.full((4, 4), float(n)) for _ in range(16)]
+    return ops.LayerWeights.from_slots(torch.device("cpu"), torch.float32, slots)
+
+
+def test_weight_structs_changed_after_a_call():
+    """The structs a layer carries are what the next call hands over, also once an earlier call has put them into a table."""
+    enc, other = _encoder(), _encoder()
+    for e in (enc, other):
+        e.layers, e._table, e._lock = [_layer(0), _layer(1)], None, threading.Lock()
+    enc._layer_table()
+    bias = torch.ones(4)
+    enc.layers[1].struct.inter_bias = bias.data_ptr()                   # a member
+    assert enc._layer_table()[1][1].inter_bias == bias.data_ptr()
+    enc.layers[0].struct = _lib.LayerWeights()                          # the whole struct
+    assert not enc._layer_table()[1][0].inter_bias
+    enc.layers[0].struct.inter_bias = bias.data_ptr()
+    other.layers[1] = enc.layers[0]                                     # a layer in two encoders' tables
+    for e, l in ((other, 1), (enc, 0)):
+        assert e._layer_table()[1][l].inter_bias == bias.data_ptr()
+    enc.layers[0].struct.inter_bias = None
+    for e, l in ((other, 1), (enc, 0)):
+        assert not e._layer_table()[1][l].inter_bias
+    enc.layers[1].prepared = _lib.LayerPrepared()
+    enc.layers[1].prepared.inter_kernel_t = bias.data_ptr()
+    assert enc._layer_table()[2][1].inter_kernel_t == bias.data_ptr()
+    enc.layers = [enc.layers[0], enc.layers[1], enc.layers[0]]          # one layer twice
+    enc._layer_table()
+    enc.layers[0].struct.inter_bias = bias.data_ptr()
+    t = enc._layer_table()[1]
+    assert t[0].inter_bias == t[2].inter_bias == bias.data_ptr() != t[1].inter_bias
