@@ -601,11 +601,12 @@ inline int attention_cu_count() {
 // Rounding points are those of the other kernels (score rounded to half, softmax in float, probabilities rounded to half
 // for P.V, here before the division by the sum instead of after it).
 //
-// A block of 16 queries whose mask rows are 1 up to the sequence's last token and 0 from there on (`mask_class`, see
-// mask_class_kernel) needs no mask and visits no key behind the last token.  Such a key has score -10000 and value 0.  Below
-// 1024 positions its weight exp(-10000 - maximum) is 0, as the maximum is clamped at 0; at 1024 there is no clamp, and the
-// unvisited keys enter the maximum and the sum at the end (`unseen`).  Any other block reads its mask rows and visits every
-// key.
+// Behind the stage of the last token K and V are zero, so nothing streams there: a score is the mask's bias alone, and a key
+// without a value only enters the maximum and the sum (`Unseen`).  `mask_class` says of every block of 16 queries whether its
+// mask rows are plain (1 up to the sequence's last token and 0 from there on: then no mask is read), and whether they are all 0
+// or all 1 behind the last token; other rows, and those of a caller without classes, are read 64 keys at a time.  Per launch, 12
+// heads, fp16, sequences of 16 .. 128 tokens in 32 x 512 positions: plain 13.8 us, causal 17.4, all ones 17.7, random behind
+// the tokens 38 (47 each but the first with the stages run over all positions); 64 .. 384 tokens in 64 x 384, causal: 46 (56).
 // ------------------------------------------------------------------------------------------
 constexpr int kFlKeys = 64;                                  // keys per stage
 constexpr int kFlStage = kFlKeys * 128;                      // bytes of K (and of V) per stage
@@ -622,23 +623,34 @@ constexpr int kFlMinKeys = 64;
 typedef __fp16 half4_fp16 __attribute__((ext_vector_type(4)));
 constexpr int kFlSmem = kFlRing * 2 * kFlStage + kFlMaxKeys * (int)sizeof(int);
 
-// Keys of score -10000 and value 0 that a block at 1024 positions has not visited (0 below, where they weigh nothing): what the
-// maximum (log2 units) is at least, and what they add to a sum taken against the exponent `ref` (infinity where they leave
-// nothing to the visited keys).
-__device__ __forceinline__ int unseen_keys(bool plain, int seq_len, int n) { return plain && seq_len == kFlMaxKeys ? seq_len - n : 0; }
-__device__ __forceinline__ float lowest_maximum(int seq_len, int unseen) {
-  return seq_len < kFlMaxKeys ? 0.f : unseen > 0 ? -10000.0f * kLog2e : -INFINITY;
-}
-__device__ __forceinline__ float unseen_weight(int unseen, float ref) {
-  return unseen > 0 ? (float)unseen * __builtin_amdgcn_exp2f(__builtin_fmaf(-10000.0f, kLog2e, -ref)) : 0.f;
-}
+// Keys without a value that have not been visited one by one enter the maximum (`lowest`, log2 units: what it is at least) and
+// the sum against the exponent `ref` (`extra`; infinity where they leave nothing to the visited keys).  Masked with 0 their score
+// is -10000: below 1024 positions, where the maximum is clamped at 0, they weigh exp(-10000 - maximum) = 0; at 1024 there is no
+// clamp.  Masked with 1 their score is 0.
+struct Unseen {
+  float lowest, extra = 0.f;
+  __device__ __forceinline__ explicit Unseen(int seq_len) : lowest(seq_len < kFlMaxKeys ? 0.f : -INFINITY) {}
+  __device__ __forceinline__ void add_zeros(int seq_len, int keys, float ref) {
+    if (seq_len < kFlMaxKeys || keys <= 0) return;
+    lowest = fmaxf(lowest, -10000.0f * kLog2e);
+    extra += (float)keys * __builtin_amdgcn_exp2f(__builtin_fmaf(-10000.0f, kLog2e, -ref));
+  }
+  __device__ __forceinline__ void add_ones(int keys, float ref) {
+    if (keys <= 0) return;
+    lowest = fmaxf(lowest, 0.f);
+    extra += (float)keys * __builtin_amdgcn_exp2f(-ref);
+  }
+};
+// what is known of a block's mask rows behind the last token
+constexpr int kMaskPlain = 1, kMaskZeros = 2, kMaskOnes = 4;
+typedef uint32_t uint4x __attribute__((ext_vector_type(4)));
 
-// class of every block of 16 query positions: 1 = the rows of the mask are 1 for keys up to the last token's and 0 beyond
+// class of every block of 16 query positions: kMaskPlain = the rows of the mask are 1 for keys up to the last token's and 0
+// beyond, kMaskZeros / kMaskOnes = they are all 0 / all 1 beyond it
 template <typename T>
 __global__ __launch_bounds__(256) void mask_class_kernel(const T* __restrict__ attr_mask, const int32_t* __restrict__ seq_start,
                                                          const int32_t* __restrict__ word_idx, int seq_len, int blocks,
                                                          uint8_t* __restrict__ cls) {
-  using V = typename Chunk16<T>::vec;
   constexpr int kElems = Chunk16<T>::kElems;
   const int b = blockIdx.y, qb = blockIdx.x;
   const int t0 = seq_start[b], t1 = seq_start[b + 1];
@@ -647,21 +659,42 @@ __global__ __launch_bounds__(256) void mask_class_kernel(const T* __restrict__ a
   if (qb * 16 >= n) return;                                  // never looked at
   const int rows = min(16, n - qb * 16);
   const T* m = attr_mask + ((size_t)b * seq_len + qb * 16) * seq_len;
-  bool plain = true;
+  // what differs from 1 up to the last token, from 0 behind it, from 1 behind it (bit patterns)
+  uint32_t no_token = 0, no_zero = 0, no_one = 0;
   if (seq_len % kElems == 0) {
+    constexpr uint32_t kOne = sizeof(T) == 2 ? 0x3c003c00u : 0x3f800000u;
     const int cpr = seq_len / kElems;
+#pragma unroll 4
     for (int i = threadIdx.x; i < rows * cpr; i += 256) {
-      const int k0 = (i % cpr) * kElems;
-      const V v = reinterpret_cast<const V*>(m)[i];
+      const uint4x w = reinterpret_cast<const uint4x*>(m)[i];
+      const int bits = (n - (i % cpr) * kElems) * (int)sizeof(T) * 8;       // of the 128 here, those up to the last token
 #pragma unroll
-      for (int j = 0; j < kElems; ++j) plain = plain && v[j] == (k0 + j < n ? (T)1.0f : (T)0.0f);
+      for (int j = 0; j < 4; ++j) {
+        const int t = min(max(bits - j * 32, 0), 32);
+        const uint32_t token = (uint32_t)((1ull << t) - 1), one = w[j] ^ kOne;
+        no_token |= one & token;
+        no_zero |= w[j] & ~token;
+        no_one |= one & ~token;
+      }
     }
   } else {
-    for (int i = threadIdx.x; i < rows * seq_len; i += 256)
-      plain = plain && m[i] == (i % seq_len < n ? (T)1.0f : (T)0.0f);
+    for (int i = threadIdx.x; i < rows * seq_len; i += 256) {
+      const T v = m[i];
+      const uint32_t zero = v == (T)0.0f ? 0u : 1u, one = v == (T)1.0f ? 0u : 1u;
+      if (i % seq_len < n) {
+        no_token |= one;
+      } else {
+        no_zero |= zero;
+        no_one |= one;
+      }
+    }
   }
-  const int all = __syncthreads_and(plain);
-  if (threadIdx.x == 0) cls[(size_t)b * blocks + qb] = all ? 1 : 0;
+  __shared__ int found[4];
+  const bool plain = !__any(no_token != 0), zeros = !__any(no_zero != 0), ones = !__any(no_one != 0);
+  if ((threadIdx.x & (kWave - 1)) == 0)
+    found[threadIdx.x / kWave] = (plain && zeros ? kMaskPlain : 0) | (zeros ? kMaskZeros : 0) | (ones ? kMaskOnes : 0);
+  __syncthreads();
+  if (threadIdx.x == 0) cls[(size_t)b * blocks + qb] = (uint8_t)(found[0] & found[1] & found[2] & found[3]);
 }
 
 __device__ __forceinline__ int v_swizzle(int key) { return (((key >> 1) & 1) | ((key >> 2) & 2)) * 2; }
@@ -748,19 +781,18 @@ __global__ __launch_bounds__(WAVES * kWave, OCC) void attention_flash_kernel(
       __builtin_amdgcn_raw_ptr_buffer_load_lds(rv, ET_ATTN_LDS_PTR(base + kFlStage + (wave * kPer + i) * 1024), 16, off_v, stage_off, 0, 0);
     }
   };
-  int tq[QSUB];
   half8 bq[QSUB][2];
   auto load_q = [&](bool dense, int n) {
 #pragma unroll
     for (int u = 0; u < QSUB; ++u) {
       const int q = q0 + u * 16 + l16;
-      tq[u] = q < n ? (dense ? q : tok_of_pos[q]) : -1;
+      const int tq = q < n ? (dense ? q : tok_of_pos[q]) : -1;
 #pragma unroll
       for (int ks = 0; ks < 2; ++ks) {
 #pragma unroll
         for (int j = 0; j < 8; ++j) bq[u][ks][j] = (_Float16)0;
-        if (tq[u] >= 0)
-          bq[u][ks] = *reinterpret_cast<const half8*>(qb + (size_t)(layout == 1 ? tq[u] : q) * ld + ks * 32 + g * 8);
+        if (tq >= 0)
+          bq[u][ks] = *reinterpret_cast<const half8*>(qb + (size_t)(layout == 1 ? tq : q) * ld + ks * 32 + g * 8);
       }
     }
   };
@@ -772,17 +804,21 @@ __global__ __launch_bounds__(WAVES * kWave, OCC) void attention_flash_kernel(
     load_q(true, len);
   }
   const int n = min(max(word_idx[t1 - 1], 0), seq_len - 1) + 1;        // positions up to the last token
-  // the workgroup's blocks of 16 queries all plain: uniform over the workgroup, as the stages are
+  // the workgroup's blocks of 16 queries all plain: uniform over the workgroup
   const int cblocks = (seq_len + 15) / 16;
-  bool plain = mask_class != nullptr;
-  if (plain) {
+  bool plain = false;
+  uint32_t zeros_behind = 0, ones_behind = 0;                          // bit i: its block i
+  if (mask_class != nullptr) {
     const int c = first_q / 16 + lane;                                 // one class per lane, all of them in one request
-    const bool mine = lane < WAVES * QSUB && c * 16 < n;
-    plain = __all(!mine || mask_class[(size_t)b * cblocks + min(c, cblocks - 1)] != 0);
+    const int got = mask_class[(size_t)b * cblocks + min(c, cblocks - 1)];     // (which does not wait for n)
+    const int cl = lane < WAVES * QSUB && c * 16 < n ? got : kMaskPlain | kMaskZeros;
+    plain = __all(cl & kMaskPlain);
+    zeros_behind = (uint32_t)__ballot(cl & kMaskZeros);
+    ones_behind = (uint32_t)__ballot(cl & kMaskOnes);
   }
   const bool dense = n == len;
   const bool active = q0 < n;                                          // wave-uniform
-  const int stages = ((plain ? n : seq_len) + kFlKeys - 1) / kFlKeys;
+  const int stages = (n + kFlKeys - 1) / kFlKeys;
   if (!dense) {
     wide_wait_dma();
     __syncthreads();
@@ -847,6 +883,41 @@ __global__ __launch_bounds__(WAVES * kWave, OCC) void attention_flash_kernel(
 #pragma unroll
   for (int j = 0; j < 8; ++j) ones[j] = (_Float16)1.0f;
 
+  // eight mask values from byte `off` of the sequence's mask; 0 behind the mask
+  auto load_mask = [&](uint32_t off) -> half8 {
+    half8 mk;
+    if ((seq_len & 7) == 0) {
+      mk = __builtin_bit_cast(half8, __builtin_amdgcn_raw_buffer_load_b128(rm, off, 0, 0));
+    } else {
+#pragma unroll
+      for (int j = 0; j < 8; ++j) mk[j] = __builtin_bit_cast(T, __builtin_amdgcn_raw_buffer_load_b16(rm, off + 2u * j, 0, 0));
+    }
+    return mk;
+  };
+  // moves a query's reference up to its lanes' maximum `mx`, where that is far enough above it; returns the factor of what has
+  // been summed against the old one
+  auto move_ref = [&](int u, float mx) -> float {
+    const float up = xor_lanes_16_32_max(mx);
+    const float next = up > ref[u] + kFlSlack ? up : ref[u];           // the same in all lanes of a query
+    float alpha = __builtin_amdgcn_exp2f(ref[u] - next);
+    ref[u] = next;
+    asm volatile("s_nop 7" : "+v"(alpha));          // wait states the compiler does not add for the instructions below
+    // (in place by hand: the compiler would give the products registers of their own and copy all of them on the way
+    // around this block)
+    auto scale = [&](float4v& v) {
+#pragma unroll
+      for (int r = 0; r < 4; ++r) {
+        float x = v[r];
+        asm volatile("v_mul_f32 %0, %1, %0" : "+v"(x) : "v"(alpha));
+        v[r] = x;
+      }
+    };
+    scale(l[u]);
+#pragma unroll
+    for (int dt = 0; dt < 4; ++dt) scale(o[u][dt]);
+    return alpha;
+  };
+
   auto stage = [&](auto PLAINc, int st, int slot) {
     constexpr bool PLAIN = decltype(PLAINc)::value;
     const unsigned char* base = kv + slot * 2 * kFlStage;
@@ -894,14 +965,7 @@ __global__ __launch_bounds__(WAVES * kWave, OCC) void attention_flash_kernel(
 #pragma unroll
         for (int pr = 0; pr < 2; ++pr) {
           const int k0 = key_base + pr * 32;
-          const uint32_t off = mask_row[u] + (uint32_t)k0 * 2u;        // bytes; reads behind the mask give 0
-          half8 mk;
-          if ((seq_len & 7) == 0) {
-            mk = __builtin_bit_cast(half8, __builtin_amdgcn_raw_buffer_load_b128(rm, off, 0, 0));
-          } else {
-#pragma unroll
-            for (int j = 0; j < 8; ++j) mk[j] = __builtin_bit_cast(T, __builtin_amdgcn_raw_buffer_load_b16(rm, off + 2u * j, 0, 0));
-          }
+          const half8 mk = load_mask(mask_row[u] + (uint32_t)k0 * 2u);
 #pragma unroll
           for (int j = 0; j < 8; ++j) {
             e[pr][j] = k0 + j < seq_len ? h2f(sc[u][pr][j]) * scaler + __builtin_fmaf((float)mk[j], 10000.0f, -10000.0f) : -INFINITY;
@@ -911,26 +975,7 @@ __global__ __launch_bounds__(WAVES * kWave, OCC) void attention_flash_kernel(
         mx *= kLog2e;
       }
       top[u] = fmaxf(top[u], mx);
-      if (__any(mx > ref[u] + kFlSlack)) {                             // the first stage, and seldom after it
-        const float up = xor_lanes_16_32_max(mx);
-        const float next = up > ref[u] + kFlSlack ? up : ref[u];       // the same in all lanes of a query
-        float alpha = __builtin_amdgcn_exp2f(ref[u] - next);
-        ref[u] = next;
-        asm volatile("s_nop 7" : "+v"(alpha));      // wait states the compiler does not add for the instructions below
-        // (in place by hand: the compiler would give the products registers of their own and copy all of them on the way
-        // around this block)
-        auto scale = [&](float4v& v) {
-#pragma unroll
-          for (int r = 0; r < 4; ++r) {
-            float x = v[r];
-            asm volatile("v_mul_f32 %0, %1, %0" : "+v"(x) : "v"(alpha));
-            v[r] = x;
-          }
-        };
-        scale(l[u]);
-#pragma unroll
-        for (int dt = 0; dt < 4; ++dt) scale(o[u][dt]);
-      }
+      if (__any(mx > ref[u] + kFlSlack)) move_ref(u, mx);              // the first stage, and seldom after it
 #pragma unroll
       for (int pr = 0; pr < 2; ++pr)
 #pragma unroll
@@ -977,16 +1022,62 @@ __global__ __launch_bounds__(WAVES * kWave, OCC) void attention_flash_kernel(
   else run(std::false_type{});
   wide_wait_dma();                                                     // no DMA may still target this workgroup's LDS when it ends
 
-  const int unseen = unseen_keys(plain, seq_len, n);
-  const float lowest = lowest_maximum(seq_len, unseen);
+  // What follows starts from the lane number once more, hidden from the compiler: a register that lives through the stage loop
+  // for it would be spilled, and its reload waited for at the end of every workgroup (0.7 us).
+  int ln = lane_id();
+  asm volatile("" : "+v"(ln));
 #pragma unroll
   for (int u = 0; u < QSUB; ++u) {
+    const int q = q0 + u * 16 + (ln & 15), g = ln >> 4;
+    const int tq = q < n ? (dense ? q : tok_of_pos[q]) : -1;
+    // the keys behind the last token's stage: no rows, the mask alone
+    Unseen unseen(seq_len);
+    const int keys = seq_len - stages * kFlKeys;
+    if (plain) {
+      unseen.add_zeros(seq_len, seq_len - n, ref[u]);
+    } else if (zeros_behind >> (wave * QSUB + u) & 1) {
+      unseen.add_zeros(seq_len, keys, ref[u]);
+    } else if (ones_behind >> (wave * QSUB + u) & 1) {
+      unseen.add_ones(keys, ref[u]);
+    } else if (active) {
+      const uint32_t mask_row = (uint32_t)min(q, seq_len - 1) * (uint32_t)seq_len * 2u;
+      int zeros = 0;
+      float sum = 0.f;                                                 // of this lane's keys
+#pragma unroll 1
+      for (int first = stages * kFlKeys; first < seq_len; first += kFlKeys) {
+        half8 mk[2];
+        uint32_t not_zero = 0;
+#pragma unroll
+        for (int pr = 0; pr < 2; ++pr) {
+          mk[pr] = load_mask(mask_row + (uint32_t)(first + pr * 32 + g * 8) * 2u);
+          const uint4x w = __builtin_bit_cast(uint4x, mk[pr]);
+          not_zero |= first + pr * 32 + g * 8 < seq_len ? w[0] | w[1] | w[2] | w[3] : 0;
+        }
+        if (!__any(not_zero != 0)) {
+          zeros += min(kFlKeys, seq_len - first);
+          continue;
+        }
+        float mx = -INFINITY;
+        auto bias = [&](int pr, int j) {
+          return first + pr * 32 + g * 8 + j < seq_len ? __builtin_fmaf((float)mk[pr][j], 10000.0f, -10000.0f) : -INFINITY;
+        };
+#pragma unroll
+        for (int j = 0; j < 16; ++j) mx = fmaxf(mx, bias(j >> 3, j & 7));
+        mx *= kLog2e;
+        top[u] = fmaxf(top[u], mx);
+        if (__any(mx > ref[u] + kFlSlack)) sum *= move_ref(u, mx);
+#pragma unroll
+        for (int j = 0; j < 16; ++j) sum += __builtin_amdgcn_exp2f(__builtin_fmaf(bias(j >> 3, j & 7), kLog2e, -ref[u]));
+      }
+      unseen.extra = xor_lanes_16_32_sum(sum);
+      unseen.add_zeros(seq_len, zeros, ref[u]);
+    }
     // the reference divides by (sum of exp(score - maximum)) + 1e-6, its maximum clamped at 0 below 1024 keys: in units of
     // 2^ref that is the sum here + 1e-6 * 2^(maximum - ref)
-    const float mx = fmaxf(xor_lanes_16_32_max(top[u]), lowest);
-    const float inv = 1.0f / (l[u][0] + unseen_weight(unseen, ref[u]) + 1e-6f * __builtin_amdgcn_exp2f(mx - ref[u]));
-    if (tq[u] < 0) continue;
-    T* orow = dst + (size_t)(t0 + tq[u]) * H + head * kD + g * 4;
+    const float mx = fmaxf(xor_lanes_16_32_max(top[u]), unseen.lowest);
+    const float inv = 1.0f / (l[u][0] + unseen.extra + 1e-6f * __builtin_amdgcn_exp2f(mx - ref[u]));
+    if (tq < 0) continue;
+    T* orow = dst + (size_t)(t0 + tq) * H + head * kD + g * 4;
 #pragma unroll
     for (int dt = 0; dt < 4; ++dt) *reinterpret_cast<half4*>(orow + dt * 16) = __builtin_convertvector(o[u][dt] * inv, half4);
   }
@@ -1108,14 +1199,19 @@ __global__ __launch_bounds__(kAttnThreads, 4) void attention_flash_f32_kernel(
   }
   const int n = min(max(word_idx[t1 - 1], 0), seq_len - 1) + 1;        // positions up to the last token
   const int cblocks = (seq_len + 15) / 16;
-  bool plain = mask_class != nullptr;
-  if (plain) {                                                         // uniform over the workgroup, as the stages are
+  bool plain = false;
+  uint32_t zeros_behind = 0, ones_behind = 0;                          // as above
+  if (mask_class != nullptr) {
     const int c = first_q / 16 + (lane & 3);
-    plain = __all(c * 16 >= n || mask_class[(size_t)b * cblocks + min(c, cblocks - 1)] != 0);
+    const int got = mask_class[(size_t)b * cblocks + min(c, cblocks - 1)];
+    const int cl = c * 16 < n ? got : kMaskPlain | kMaskZeros;
+    plain = __all(cl & kMaskPlain);
+    zeros_behind = (uint32_t)__ballot(cl & kMaskZeros);
+    ones_behind = (uint32_t)__ballot(cl & kMaskOnes);
   }
   const bool dense = n == len;
   const bool active = first_q + wave * 16 < n;                         // wave-uniform
-  const int stages = ((plain ? n : seq_len) + kF32Keys - 1) / kF32Keys;
+  const int stages = (n + kF32Keys - 1) / kF32Keys;
   if (!dense) {
     wide_wait_dma();
     __syncthreads();
@@ -1142,6 +1238,27 @@ __global__ __launch_bounds__(kAttnThreads, 4) void attention_flash_f32_kernel(
   for (int dt = 0; dt < 4; ++dt) o[dt] = float4v{0.f, 0.f, 0.f, 0.f};
   const float c_exp = scaler * kLog2e;
   const float* mrow = attr_mask + ((size_t)b * seq_len + min(q, seq_len - 1)) * seq_len;
+
+  auto load_mask = [&](int k0) -> float4v {                            // of keys k0 .. k0 + 3, 0 beyond the row
+    float4v m4 = {0.f, 0.f, 0.f, 0.f};
+    if ((seq_len & 3) == 0) {
+      if (k0 < seq_len) m4 = *reinterpret_cast<const float4v*>(mrow + k0);
+    } else {
+#pragma unroll
+      for (int r = 0; r < 4; ++r)
+        if (k0 + r < seq_len) m4[r] = mrow[k0 + r];
+    }
+    return m4;
+  };
+  auto move_ref = [&](float mx) {                                      // as above
+    const float up = xor_lanes_16_32_max(mx);
+    const float next = up > ref + kFlSlack ? up : ref;                 // the same in all lanes of a query
+    const float alpha = __builtin_amdgcn_exp2f(ref - next);
+    ref = next;
+    l *= alpha;
+#pragma unroll
+    for (int dt = 0; dt < 4; ++dt) o[dt] *= alpha;
+  };
 
   auto stage = [&](auto PLAINc, int st, int slot) {
     constexpr bool PLAIN = decltype(PLAINc)::value;
@@ -1175,14 +1292,7 @@ __global__ __launch_bounds__(kAttnThreads, 4) void attention_flash_f32_kernel(
 #pragma unroll
       for (int kt = 0; kt < 2; ++kt) {
         const int k0 = key0 + kt * 16;
-        float4v m4 = {0.f, 0.f, 0.f, 0.f};
-        if ((seq_len & 3) == 0) {
-          if (k0 < seq_len) m4 = *reinterpret_cast<const float4v*>(mrow + k0);
-        } else {
-#pragma unroll
-          for (int r = 0; r < 4; ++r)
-            if (k0 + r < seq_len) m4[r] = mrow[k0 + r];
-        }
+        const float4v m4 = load_mask(k0);
 #pragma unroll
         for (int r = 0; r < 4; ++r) s[kt][r] = k0 + r < seq_len ? s[kt][r] * scaler + (1.0f - m4[r]) * -10000.0f : -INFINITY;
       }
@@ -1193,15 +1303,7 @@ __global__ __launch_bounds__(kAttnThreads, 4) void attention_flash_f32_kernel(
       for (int r = 0; r < 4; ++r) mx = fmaxf(mx, s[kt][r]);
     mx *= unit;
     top = fmaxf(top, mx);
-    if (__any(mx > ref + kFlSlack)) {                                  // the first stage, and seldom after it
-      const float up = xor_lanes_16_32_max(mx);
-      const float next = up > ref + kFlSlack ? up : ref;               // the same in all lanes of a query
-      const float alpha = __builtin_amdgcn_exp2f(ref - next);
-      ref = next;
-      l *= alpha;
-#pragma unroll
-      for (int dt = 0; dt < 4; ++dt) o[dt] *= alpha;
-    }
+    if (__any(mx > ref + kFlSlack)) move_ref(mx);                      // the first stage, and seldom after it
 #pragma unroll
     for (int kt = 0; kt < 2; ++kt)
 #pragma unroll
@@ -1229,9 +1331,48 @@ __global__ __launch_bounds__(kAttnThreads, 4) void attention_flash_f32_kernel(
   if (plain) run(std::true_type{});
   else run(std::false_type{});
 
-  const int unseen = unseen_keys(plain, seq_len, n);
-  const float mx = fmaxf(xor_lanes_16_32_max(top), lowest_maximum(seq_len, unseen));
-  const float sum = xor_lanes_16_32_sum(l) + unseen_weight(unseen, ref);
+  // the keys behind the last token's stage, as above
+  Unseen unseen(seq_len);
+  {
+    const int keys = seq_len - stages * kF32Keys;
+    if (plain) {
+      unseen.add_zeros(seq_len, seq_len - n, ref);
+    } else if (zeros_behind >> wave & 1) {
+      unseen.add_zeros(seq_len, keys, ref);
+    } else if (ones_behind >> wave & 1) {
+      unseen.add_ones(keys, ref);
+    } else if (active) {
+      int zeros = 0;
+#pragma unroll 1
+      for (int first = stages * kF32Keys; first < seq_len; first += 64) {
+        float4v m4[4];
+        uint32_t not_zero = 0;
+#pragma unroll
+        for (int i = 0; i < 4; ++i) {
+          m4[i] = load_mask(first + i * 16 + g * 4);
+          const uint4x w = __builtin_bit_cast(uint4x, m4[i]);
+          not_zero |= w[0] | w[1] | w[2] | w[3];
+        }
+        if (!__any(not_zero != 0)) {
+          zeros += min(64, seq_len - first);
+          continue;
+        }
+        float high = -INFINITY;
+        auto bias = [&](int i, int r) { return first + i * 16 + g * 4 + r < seq_len ? (1.0f - m4[i][r]) * -10000.0f : -INFINITY; };
+#pragma unroll
+        for (int j = 0; j < 16; ++j) high = fmaxf(high, bias(j >> 2, j & 3));
+        high *= kLog2e;
+        top = fmaxf(top, high);
+        if (__any(high > ref + kFlSlack)) move_ref(high);
+#pragma unroll
+        for (int j = 0; j < 16; ++j) l += __builtin_amdgcn_exp2f(__builtin_fmaf(bias(j >> 2, j & 3), kLog2e, -ref));
+      }
+      unseen.add_zeros(seq_len, zeros, ref);
+    }
+  }
+
+  const float mx = fmaxf(xor_lanes_16_32_max(top), unseen.lowest);
+  const float sum = xor_lanes_16_32_sum(l) + unseen.extra;
   if (tq < 0) return;
   const float inv = 1.0f / (sum + 1e-6f * __builtin_amdgcn_exp2f(mx - ref));
   // o[dt][r] is feature 16 g + 4 r + dt
@@ -1480,6 +1621,8 @@ bool attention_supported(DType t, int seq_len, int d) {
 size_t mask_class_bytes(DType t, int batch, int seq_len, int d) {
   return d == kD && seq_len > (t == DType::F16 ? kFlMinKeys : kF32MinKeys) && seq_len <= kFlMaxKeys ? (size_t)batch * ((seq_len + 15) / 16) : 0;
 }
+
+size_t mask_class_bytes_max(int batch) { return (size_t)batch * (kFlMaxKeys / 16); }
 
 void launch_mask_class(DType t, const void* attr_mask, const int32_t* seq_start, const int32_t* word_idx, int batch, int seq_len,
                        uint8_t* cls, hipStream_t stream) {

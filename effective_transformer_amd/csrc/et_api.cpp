@@ -128,6 +128,10 @@ thread_local std::string tls_error_copy;      // et_last_error's copy of another
 
 inline size_t align_up(size_t v, size_t a) { return (v + a - 1) / a * a; }
 
+// The smallest buffer a sequence table is taken in.  et_seq_workspace_bytes asks for more: et_attention has the classes of the
+// mask rows made behind the table where there is room for them.
+inline size_t seq_table_bytes_min(int batch) { return align_up(et::seq_table_words(batch) * sizeof(int32_t), 256); }
+
 et_status fail(et_handle h, et_status s, const std::string& msg) {
   std::string full = std::string("[ET][ERROR] ") + et_status_string(s) + ": " + msg;
   if (h) {
@@ -273,7 +277,7 @@ et_status layer_args_ok(et_handle h, et_dtype dtype, const et_layer_weights* w, 
   if (!et::bias_gelu_supported(dt, F) || !et::bias_residual_layernorm_supported(dt, H))
     return fail(h, ET_UNSUPPORTED, "hidden size not supported by the row kernels");
   if (prep) {
-    if (prep->seq_start && prep->seq_start_bytes < et_seq_workspace_bytes(B))
+    if (prep->seq_start && prep->seq_start_bytes < seq_table_bytes_min(B))
       return fail(h, ET_WORKSPACE_TOO_SMALL, "et_layer_prepared.seq_start needs et_seq_workspace_bytes(batch_size) bytes");
     ET_REQUIRE(h, (prep->attr_kernel_Q_t != nullptr) == (prep->attr_kernel_K_t != nullptr) &&
                       (prep->attr_kernel_Q_t != nullptr) == (prep->attr_kernel_V_t != nullptr),
@@ -534,7 +538,7 @@ size_t et_layer_workspace_bytes(et_dtype dtype, int batch_size, int seq_len, int
 
 size_t et_seq_workspace_bytes(int batch_size) {
   if (batch_size < 1) return 0;
-  return align_up(et::seq_table_words(batch_size) * sizeof(int32_t), 256);
+  return seq_table_bytes_min(batch_size) + et::mask_class_bytes_max(batch_size);
 }
 
 et_status et_input(et_handle h, et_dtype dtype, const void* from_tensor, const int32_t* mask, void* to_tensor,
@@ -663,7 +667,7 @@ et_status et_sequence_starts(et_handle h, const int32_t* batch_idx, const int32_
   if (s != ET_OK) return s;
   if ((s = dims_ok(h, batch_size, seq_len, 1, 1)) != ET_OK) return s;
   ET_REQUIRE(h, batch_idx && valid_word_num_dev && seq_start, "null tensor pointer");
-  if (seq_start_bytes < et_seq_workspace_bytes(batch_size))
+  if (seq_start_bytes < seq_table_bytes_min(batch_size))
     return fail(h, ET_WORKSPACE_TOO_SMALL, "the sequence table needs et_seq_workspace_bytes(batch_size)");
   et::launch_seq_start(batch_idx, valid_word_num_dev, batch_size * seq_len, batch_size, seq_start, (hipStream_t)stream);
   return check_launch(h, "sequence starts");
@@ -727,7 +731,7 @@ EncoderWs encoder_ws(et_dtype dtype, int B, int S, int heads, int d) {
   w.batch_idx = take(rows * sizeof(int32_t));
   w.word_idx = take(rows * sizeof(int32_t));
   w.count = take(sizeof(int32_t));
-  w.seq = take(et_seq_workspace_bytes(B));
+  w.seq = take(seq_table_bytes_min(B));
   w.scan = take(et_input_workspace_bytes(B, S));
   w.layer = take(et_layer_workspace_bytes(dtype, B, S, heads, d));
   w.total = off;
@@ -1010,7 +1014,7 @@ et_status et_add_qkv_bias_padding(et_handle h, et_dtype dtype, const void* Q, co
                     batch_idx && word_idx,
              "null tensor pointer");
   ET_REQUIRE(h, workspace != nullptr, "null workspace");
-  if (workspace_bytes < et_seq_workspace_bytes(batch_size))
+  if (workspace_bytes < seq_table_bytes_min(batch_size))
     return fail(h, ET_WORKSPACE_TOO_SMALL, "needs et_seq_workspace_bytes(batch_size)");
   if (seq_len > 1024) return fail(h, ET_UNSUPPORTED, "seq_len <= 1024");
   hipStream_t st = (hipStream_t)stream;
@@ -1053,7 +1057,7 @@ et_status et_attention(et_handle h, et_dtype dtype, const void* q, const void* k
                        const int32_t* word_idx, void* workspace, size_t workspace_bytes, void* stream) {
   if (h) {
     ET_REQUIRE(h, workspace != nullptr, "null workspace");
-    if (workspace_bytes < et_seq_workspace_bytes(batch_size))
+    if (workspace_bytes < seq_table_bytes_min(batch_size))
       return fail(h, ET_WORKSPACE_TOO_SMALL, "needs et_seq_workspace_bytes(batch_size)");
   }
   return et_attention_with_starts(h, dtype, q, k, v, qkv_layout, packed_ld, attr_mask, dst, valid_word_num_dev,
@@ -1076,18 +1080,24 @@ et_status et_attention_with_starts(et_handle h, et_dtype dtype, const void* q, c
   ET_REQUIRE(h, qkv_layout == 0 || qkv_layout == 1, "qkv_layout must be 0 (padded) or 1 (packed)");
   ET_REQUIRE(h, qkv_layout == 0 || packed_ld >= head_num * size_per_head, "packed_ld smaller than the hidden size");
   ET_REQUIRE(h, seq_start != nullptr || seq_start_scratch != nullptr, "null sequence start table");
-  if (seq_table_bytes < et_seq_workspace_bytes(batch_size))
+  if (seq_table_bytes < seq_table_bytes_min(batch_size))
     return fail(h, ET_WORKSPACE_TOO_SMALL, "the sequence table needs et_seq_workspace_bytes(batch_size)");
   if ((s = batch_fits_grid(h, batch_size)) != ET_OK) return s;
   if (!et::attention_supported(to_dt(dtype), seq_len, size_per_head))
     return fail(h, ET_UNSUPPORTED, "attention needs size_per_head <= 256 and seq_len <= 1024");
   hipStream_t st = (hipStream_t)stream;
+  uint8_t* cls = nullptr;
   if (!seq_start) {
     et::launch_seq_start(batch_idx, valid_word_num_dev, batch_size * seq_len, batch_size, seq_start_scratch, st);
     seq_start = seq_start_scratch;
+    const size_t table = seq_table_bytes_min(batch_size), bytes = et::mask_class_bytes(to_dt(dtype), batch_size, seq_len, size_per_head);
+    if (bytes > 0 && seq_table_bytes >= table + bytes) {
+      cls = (uint8_t*)seq_start_scratch + table;
+      et::launch_mask_class(to_dt(dtype), attr_mask, seq_start, word_idx, batch_size, seq_len, cls, st);
+    }
   }
   et::launch_attention(to_dt(dtype), q, k, v, qkv_layout, packed_ld, attr_mask, dst, seq_start, word_idx, batch_size,
-                       seq_len, head_num, size_per_head, softmax_scaler(dtype, size_per_head), st);
+                       seq_len, head_num, size_per_head, softmax_scaler(dtype, size_per_head), st, false, cls);
   return check_launch(h, "attention");
 }
 

@@ -112,6 +112,7 @@ void launch_attention(DType t, const void* q, const void* k, const void* v, int 
 // Classes of the mask rows (one byte per 16 query positions of a sequence) for the kernel that makes use of them; the same
 // array serves every layer of a batch.  0 bytes: the kernel of this shape has no use for them.
 size_t mask_class_bytes(DType t, int batch, int seq_len, int d);
+size_t mask_class_bytes_max(int batch);                // at any length
 void launch_mask_class(DType t, const void* attr_mask, const int32_t* seq_start, const int32_t* word_idx, int batch, int seq_len,
                        uint8_t* cls, hipStream_t stream);
 // split_out (fp32): dst gets split rows (see gemm_split.hip) instead of float rows; only where this says so

@@ -84,7 +84,8 @@ typedef struct et_layer_weights {
 size_t et_input_workspace_bytes(int batch_size, int seq_len);
 size_t et_layer_workspace_bytes(et_dtype dtype, int batch_size, int seq_len, int head_num, int size_per_head);
 /* size of the sequence table of a batch (et_sequence_starts; also the scratch of the kernel-level entry points that
- * build one): 2 * batch_size + 1 int32, rounded up to 256 bytes */
+ * build one): 2 * batch_size + 1 int32, rounded up to 256 bytes, and 64 bytes a sequence in which et_attention notes what
+ * its mask rows look like.  A buffer for the table alone (the first of the two) is taken everywhere. */
 size_t et_seq_workspace_bytes(int batch_size);
 
 /* ---- the three ops ------------------------------------------------------------------ */
