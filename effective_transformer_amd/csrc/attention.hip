@@ -220,8 +220,7 @@ __device__ __forceinline__ float xor_lanes_16_32_sum(float v) {
 
 // WAVES: wavefronts per workgroup, one 16-query tile each.  CPT = 16-byte chunks of
 // one matrix a thread moves per head (ceil(seq rows * chunks per row / threads)).
-// PF: keep the next head's Q/K/V chunks in registers while the current head is computed.
-template <typename T, int NKT, int WAVES, int CPT, bool PF>
+template <typename T, int NKT, int WAVES, int CPT>
 __global__ __launch_bounds__(WAVES * kWave) void attention_kernel(
     const T* __restrict__ q_src, const T* __restrict__ k_src, const T* __restrict__ v_src, int layout, int packed_ld,
     const T* __restrict__ attr_mask, T* __restrict__ dst, const int32_t* __restrict__ seq_start,
@@ -308,7 +307,7 @@ __global__ __launch_bounds__(WAVES * kWave) void attention_kernel(
       rv[k] = *reinterpret_cast<const V16*>(v_src + off);                                                   \
     }                                                                                                       \
   }
-  if (PF) { ET_ATTN_LOAD_HEAD(h_begin) }
+  ET_ATTN_LOAD_HEAD(h_begin)
 
   const int last_pos = min(max(last_pos_raw, 0), seq_len - 1);
   const int n_tiles = last_pos / 16 + 1;    // 16-row tiles that hold at least one token (queries and keys)
@@ -354,7 +353,6 @@ __global__ __launch_bounds__(WAVES * kWave) void attention_kernel(
     out_row = reinterpret_cast<T*>(reinterpret_cast<uint16_t*>(dst) + (size_t)tq * 3 * H);
 
   for (int head = h_begin; head < h_end; ++head) {
-    if (!PF) { ET_ATTN_LOAD_HEAD(head) }
     if (head != h_begin) __syncthreads();      // every wavefront is done with the previous head's tiles
 #pragma unroll
     for (int k = 0; k < CPT; ++k) {
@@ -372,7 +370,7 @@ __global__ __launch_bounds__(WAVES * kWave) void attention_kernel(
       }
     }
     __syncthreads();
-    if (PF && head + 1 < h_end) { ET_ATTN_LOAD_HEAD(head + 1) }   // flies while this head is computed
+    if (head + 1 < h_end) { ET_ATTN_LOAD_HEAD(head + 1) }         // flies while this head is computed
 
     if (wave < n_tiles) {                     // wave-uniform
       const int q = wave * 16 + l16;          // this lane's query position
@@ -538,8 +536,8 @@ void attention_launch(const void* q, const void* k, const void* v, int layout, i
   constexpr int WAVES = 4;
   constexpr int kThreads = WAVES * kWave;
   constexpr int CPT = (NKT * 16 * kCpr + kThreads - 1) / kThreads;
-  constexpr bool PF = CPT <= 4;                // more than 4 chunks x 3 matrices in flight would not fit the registers
-  auto kern = attention_kernel<T, NKT, WAVES, CPT, PF>;
+  static_assert(CPT <= 4, "the next head's chunks, 3 matrices of them, are kept in registers");
+  auto kern = attention_kernel<T, NKT, WAVES, CPT>;
   allow_dynamic_lds(reinterpret_cast<const void*>(kern), (int)Sm::kBytes);
   // A workgroup serves several heads of one sequence: mask rows, positions and zero fill are shared by them, and the
   // chain of dependent loads a workgroup starts with (sequence start, positions, rows) is paid once.  Up to 6 heads
@@ -610,7 +608,7 @@ inline int attention_cu_count() {
 // ------------------------------------------------------------------------------------------
 constexpr int kFlKeys = 64;                                  // keys per stage
 constexpr int kFlStage = kFlKeys * 128;                      // bytes of K (and of V) per stage
-constexpr int kFlRing = 2;                                   // stages in LDS
+constexpr int kFlWaves = 4;                                  // wavefronts of a workgroup, and per SIMD
 constexpr int kFlMaxKeys = 1024;
 // Up to 64 positions attention_kernel is the faster one: a head is a single stage there, so nothing streams, and its
 // workgroups serve six heads for one start (12 layers, 1000 x 64: 7.79 ms with it, 7.98 ms with this kernel; 217 x 53 in
@@ -621,7 +619,7 @@ constexpr int kFlMinKeys = 64;
 [[maybe_unused]] constexpr float kFlLowest = -3e38f;                          // the reference before the first stage; finite, so that scores of
                                                              // -infinity weigh nothing against it
 typedef __fp16 half4_fp16 __attribute__((ext_vector_type(4)));
-constexpr int kFlSmem = kFlRing * 2 * kFlStage + kFlMaxKeys * (int)sizeof(int);
+constexpr int kFlSmem = 2 * 2 * kFlStage + kFlMaxKeys * (int)sizeof(int);
 
 // Keys without a value that have not been visited one by one enter the maximum (`lowest`, log2 units: what it is at least) and
 // the sum against the exponent `ref` (`extra`; infinity where they leave nothing to the visited keys).  Masked with 0 their score
@@ -708,8 +706,8 @@ __device__ __forceinline__ half4 read_transposed(const unsigned char* p) {
 #endif
 }
 
-template <int QSUB, int WAVES, int OCC>
-__global__ __launch_bounds__(WAVES * kWave, OCC) void attention_flash_kernel(
+template <int QSUB>
+__global__ __launch_bounds__(kFlWaves * kWave, 4) void attention_flash_kernel(
     const _Float16* __restrict__ q_src, const _Float16* __restrict__ k_src, const _Float16* __restrict__ v_src, int layout,
     int packed_ld, const _Float16* __restrict__ attr_mask, const uint8_t* __restrict__ mask_class,
     _Float16* __restrict__ dst, const int32_t* __restrict__ seq_start, const int32_t* __restrict__ word_idx, int batch,
@@ -719,7 +717,7 @@ __global__ __launch_bounds__(WAVES * kWave, OCC) void attention_flash_kernel(
   typedef _Float16 half2x __attribute__((ext_vector_type(2)));
   extern __shared__ __attribute__((aligned(1024))) unsigned char smem_raw[];
   unsigned char* kv = smem_raw;                                        // [stage][K, V]
-  int* tok_of_pos = reinterpret_cast<int*>(smem_raw + kFlRing * 2 * kFlStage);
+  int* tok_of_pos = reinterpret_cast<int*>(smem_raw + 2 * 2 * kFlStage);
 
   // The query blocks of one (head, sequence) go to one XCD, whose L2 then fetches their K and V once: workgroup ids are
   // dealt round-robin to the XCDs, pair p = 8 * (slot / q_blocks) + xcd.
@@ -736,7 +734,7 @@ __global__ __launch_bounds__(WAVES * kWave, OCC) void attention_flash_kernel(
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x / kWave);
   const int l16 = lane & 15, g = lane >> 4;
 
-  const int first_q = qblock * 16 * WAVES * QSUB;
+  const int first_q = qblock * 16 * kFlWaves * QSUB;
   const int q0 = first_q + wave * 16 * QSUB;                           // this wavefront's: tile u holds q0 + 16 u + l16
 
   // K / V rows of a stage by DMA: one instruction fills eight slots (lane -> slot 8 i + lane / 8, 16-byte chunk
@@ -745,7 +743,7 @@ __global__ __launch_bounds__(WAVES * kWave, OCC) void attention_flash_kernel(
   const T* vb = layout == 1 ? v_src + (size_t)t0 * packed_ld + head * kD : v_src + ((size_t)b * heads + head) * seq_len * kD;
   const T* qb = layout == 1 ? q_src + (size_t)t0 * packed_ld + head * kD : q_src + ((size_t)b * heads + head) * seq_len * kD;
   const uint32_t ld = layout == 1 ? (uint32_t)packed_ld : (uint32_t)kD;
-  constexpr int kPer = 8 / WAVES;                                      // requests of a wavefront for K (and for V) per stage
+  constexpr int kPer = 8 / kFlWaves;                                   // requests of a wavefront for K (and for V) per stage
   uint32_t voff[kPer], voff_v[kPer];
   int dma_key[kPer];
 #pragma unroll
@@ -811,7 +809,7 @@ __global__ __launch_bounds__(WAVES * kWave, OCC) void attention_flash_kernel(
   if (mask_class != nullptr) {
     const int c = first_q / 16 + lane;                                 // one class per lane, all of them in one request
     const int got = mask_class[(size_t)b * cblocks + min(c, cblocks - 1)];     // (which does not wait for n)
-    const int cl = lane < WAVES * QSUB && c * 16 < n ? got : kMaskPlain | kMaskZeros;
+    const int cl = lane < kFlWaves * QSUB && c * 16 < n ? got : kMaskPlain | kMaskZeros;
     plain = __all(cl & kMaskPlain);
     zeros_behind = (uint32_t)__ballot(cl & kMaskZeros);
     ones_behind = (uint32_t)__ballot(cl & kMaskOnes);
@@ -823,9 +821,9 @@ __global__ __launch_bounds__(WAVES * kWave, OCC) void attention_flash_kernel(
     wide_wait_dma();
     __syncthreads();
     if (first_q >= n) return;                                          // no token among this workgroup's queries
-    for (int i = threadIdx.x; i < kFlMaxKeys; i += WAVES * kWave) tok_of_pos[i] = -1;
+    for (int i = threadIdx.x; i < kFlMaxKeys; i += kFlWaves * kWave) tok_of_pos[i] = -1;
     __syncthreads();
-    for (int tt = threadIdx.x; tt < len; tt += WAVES * kWave) {
+    for (int tt = threadIdx.x; tt < len; tt += kFlWaves * kWave) {
       const int pos = word_idx[t0 + tt];
       if (pos >= 0 && pos < seq_len) tok_of_pos[pos] = tt;             // relative to the sequence's first packed row
     }
@@ -835,8 +833,6 @@ __global__ __launch_bounds__(WAVES * kWave, OCC) void attention_flash_kernel(
   } else if (first_q >= n) {
     return;                                                            // (nothing has been requested)
   }
-#pragma unroll
-  for (int i = 1; i < kFlRing - 1; ++i) issue(i, min(i, stages - 1), dense, layout == 1 ? len : n);
 
   // the queries are waited for here: left pending, they would have the compiler put a wait for every outstanding request,
   // the DMA included, into the stage loop
@@ -1007,15 +1003,12 @@ __global__ __launch_bounds__(WAVES * kWave, OCC) void attention_flash_kernel(
   };
 
   auto run = [&](auto PLAINc) {
-    int slot = 0;
     for (int st = 0; st < stages; ++st) {
-      constexpr int kFly = 2 * kPer * (kFlRing - 2);                   // this wavefront's share of the stage has landed; those
-      __builtin_amdgcn_s_waitcnt((kFly & 15) | (7 << 4) | (15 << 8) | ((kFly >> 4) << 14));      // behind it may fly
-      wide_barrier();                                                  // everybody's has, and the slot before this one is free
-      // (stages past the end re-load the last one, which keeps the count of requests in flight uniform)
-      issue(slot == 0 ? kFlRing - 1 : slot - 1, min(st + kFlRing - 1, stages - 1), dense, layout == 1 ? len : n);
-      if (active) stage(PLAINc, st, slot);
-      slot = slot + 1 == kFlRing ? 0 : slot + 1;
+      wide_wait_dma();                                                 // this wavefront's share of the stage has landed,
+      wide_barrier();                                                  // everybody's has, and the other slot is free
+      // (the last stage is loaded once more behind it: a condition here costs the loop registers, 256 x 128 28.5 -> 30.4 us)
+      issue((st + 1) & 1, min(st + 1, stages - 1), dense, layout == 1 ? len : n);
+      if (active) stage(PLAINc, st, st & 1);
     }
   };
   if (plain) run(std::true_type{});
@@ -1088,17 +1081,17 @@ void attention_flash_launch(const void* q, const void* k, const void* v, int lay
                             const uint8_t* mask_class, void* dst, const int32_t* seq_start, const int32_t* word_idx,
                             int batch, int seq_len, int heads, float scaler, hipStream_t stream) {
   const int pairs8 = (batch * heads + 7) / 8 * 8;
-  auto go = [&](auto kern, int waves, int queries) {
+  auto go = [&](auto kern, int queries) {
     const int q_blocks = (seq_len + queries - 1) / queries;
     allow_dynamic_lds(reinterpret_cast<const void*>(kern), kFlSmem);
-    kern<<<pairs8 * q_blocks, waves * kWave, kFlSmem, stream>>>(
+    kern<<<pairs8 * q_blocks, kFlWaves * kWave, kFlSmem, stream>>>(
         (const _Float16*)q, (const _Float16*)k, (const _Float16*)v, layout, packed_ld, (const _Float16*)attr_mask, mask_class,
         (_Float16*)dst, seq_start, word_idx, batch, seq_len, heads, q_blocks, scaler);
   };
   // Two query tiles per wavefront halve the LDS reads per score; with few workgroups the CUs are better filled by twice as
   // many of one tile.
-  if ((long)batch * heads * ((seq_len + 127) / 128) >= 2L * attention_cu_count()) go(attention_flash_kernel<2, 4, 4>, 4, 128);
-  else go(attention_flash_kernel<1, 4, 4>, 4, 64);
+  if ((long)batch * heads * ((seq_len + 127) / 128) >= 2L * attention_cu_count()) go(attention_flash_kernel<2>, 128);
+  else go(attention_flash_kernel<1>, 64);
 }
 
 // ------------------------------------------------------------------------------------------
