@@ -768,10 +768,6 @@ et_status wait_for_count(et_handle h, const uint64_t* word, uint32_t tag, const 
   }
 }
 
-// Batches of at most this many padded positions are launched for all of them without waiting for the count: the launches
-// of fewer rows would hardly be smaller (a handful of 32-row tiles), and the host may run ahead.
-constexpr int kWaitForCountRows = 256;
-
 }  // namespace
 
 size_t et_encoder_workspace_bytes(et_dtype dtype, int batch_size, int seq_len, int head_num, int size_per_head) {
@@ -815,7 +811,10 @@ et_status et_encoder(et_handle h, et_dtype dtype, int num_layers, const et_layer
   // The count comes back through the caller's pinned word, stored by the scan itself: no copy on the stream, no event.
   // Every call has a tag of its own, so a word left by an earlier batch is never taken for this one's.
   static std::atomic<uint32_t> next_tag{1};
-  const bool wait_for_layers = b->rows_bound == 0 && num_layers > 1 && B * S > kWaitForCountRows;
+  // The layers of a stack wait for it at every size.  12 layers, waiting and launched for all positions, us per pass in a stream
+  // of passes: fp16 1 x 32 405 and 405, 4 x 32 with 41 tokens 414 and 424, 8 x 32 with 120 434 and 457, 12 x 32 with 172 449 and
+  // 492, 32 x 32 with 546 545 and 635; fp32 854 and 872, 899 and 968, 964 and 1054, 1019 and 1283, 1379 and 1743.
+  const bool wait_for_layers = b->rows_bound == 0 && num_layers > 1;
   et::ScanExtras scan;
   scan.seq_start = seq;
   if (b->count_word && (wait_for_layers || b->valid_word_num)) {

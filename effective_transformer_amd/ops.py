@@ -388,6 +388,7 @@ class EffectiveTransformerEncoder:
         self._count_words: Dict[tuple, torch.Tensor] = {}
         self._lock = threading.Lock()
         self._table: Optional[tuple] = None
+        self._layer_table()
 
     def _layer_table(self):
         """The layers' weight and prepared structs as the arrays et_encoder takes.  Every struct is made a view of its array
@@ -463,9 +464,9 @@ class EffectiveTransformerEncoder:
         return self._run(batch, B, S, (B, S, embeddings.hidden), input_mask, attention_mask, sync_count, None)
 
     def _run(self, batch, B, S, shape, input_mask, attention_mask, sync_count, rows_bound):
-        """One et_encoder call.  sync_count: the valid-token count is read back once per batch, so that the launches of
-        layers 2 .. L are sized exactly (the reference reads it back in every layer); the host waits for it behind the
-        launches of the first layer, which is sized for B*S rows and bounded on the device, so the GPU never idles for it."""
+        """One et_encoder call.  sync_count: the host waits for the valid-token count once per batch (the reference reads it
+        back in every layer), in front of the layers and while the input rows are still being moved, so that every layer is
+        launched for exactly that many rows; a single layer is launched for B*S rows and bounded on the device instead."""
         lib = _lib.load()
         _require_cuda(input_mask, attention_mask)
         if input_mask.dtype != torch.int32:

@@ -117,9 +117,9 @@ class Encoder {
   Encoder& operator=(const Encoder&) = delete;
 
   // from_tensor [B,S,H], mask int32 [B,S], attr_mask [B,S,S] in dtype -> out [B,S,H] (zeros at padding).
-  // sync_count: the valid-token count is read back once per batch, so that the launches of layers 2 .. L are sized
-  // exactly (the reference reads it back in every layer), or left on the device (launches sized for B*S rows); the host
-  // waits for it behind the launches of the first layer, so the GPU never idles for the read-back.
+  // sync_count: the valid-token count is read back once per batch (the reference reads it back in every layer), or left on
+  // the device (launches sized for B*S rows).  The host waits for it in front of the layers, while the input rows are still
+  // being moved, so that every layer is launched for exactly that many rows.
   // Returns the valid-token count, or -1 when it was not read back.
   int forward(const void* from_tensor, const int32_t* mask, const void* attr_mask, void* out, int batch, int seq_len,
               hipStream_t stream, bool sync_count = true) {
