@@ -93,6 +93,7 @@ def fold_traffic(workload, fetch_csv, write_csv, commit, command):
 PUBLISHED_MS = {"cfg2": (8.75, "Readme.md:65"), "cfg3": (133.61, "Readme.md:80"), "cfg4": (325.37, "Readme.md:89")}
 HBM_PEAK_GBS = 8000.0
 MFMA_PEAK_TFLOPS = {"fp16": 2500.0, "fp32": 157.3}
+SPLIT_PEAK_TFLOPS = 2500.0 / 6      # fp32 products of split rows: six 16-bit products for one of floats
 
 
 def _time_kernel(fn, iters, warm=3):
@@ -152,11 +153,11 @@ def per_kernel(wl, T, mask_np, iters=20, vendor_gemm=False):
     to, vwn, bidx, widx = ops.effective_transformer_input(x, mask, B, S, S, heads, d)
     res = {}
 
-    def add(name, ms, bound, work):
+    def add(name, ms, bound, work, mfma_peak=MFMA_PEAK_TFLOPS[wl.dtype]):
         if bound == "hbm":
             ach, peak, unit = work / ms / 1e6, HBM_PEAK_GBS, "GB/s"
         else:
-            ach, peak, unit = work / ms / 1e9, MFMA_PEAK_TFLOPS[wl.dtype], "TFLOP/s"
+            ach, peak, unit = work / ms / 1e9, mfma_peak, "TFLOP/s"
         res[name] = {"ms": round(ms, 5), "bound": bound, "achieved": round(ach, 2), "peak": peak, "unit": unit,
                      "frac": round(ach / peak, 4)}
 
@@ -206,7 +207,8 @@ def per_kernel(wl, T, mask_np, iters=20, vendor_gemm=False):
     ms = _time_kernel(lambda: k.add_bias_act(inter, bF), iters)
     add("bias_gelu", ms, "hbm", 2 * T * F * e + F * e)
     res["bias_gelu"]["on_path"] = False       # et_add_bias_act on its own; the layer fuses it into the FFN-up GEMM
-    # fused attention on packed rows
+    # fused attention on packed rows (beyond 64 positions in fp16 and 32 in fp32 the layer also knows what the mask's rows look
+    # like, which this call does not, and its launch is the faster one)
     qkv = rnd(B * S, 3 * H)
     ctx = torch.empty(B * S, H, device="cuda", dtype=dt)
     starts = ops.sequence_starts(vwn, bidx, B, S)          # one table per batch, as the encoder builds it
@@ -222,6 +224,13 @@ def per_kernel(wl, T, mask_np, iters=20, vendor_gemm=False):
         kw = {"bias": bF, "gelu": True} if name == "gemm_ffn_up" else {}
         fn = lambda: k.gemm(A, Bm, out=Cm, **kw)
         plain = lambda: k.gemm(A, Bm, out=Cm)
+        split = dt == torch.float32 and kk % 32 == 0
+        if split:
+            # the layer's products read split rows; the kernels in front of them write that form
+            sa, sb = k.split_rows(A), k.transpose_weight(Bm)
+            Cs = torch.empty(T, 3 * n, device="cuda", dtype=torch.bfloat16) if kw else Cm
+            fn = lambda: k.gemm_split(sa, sb, out=Cs, **kw)
+            plain = lambda: k.gemm_split(sa, sb, out=Cm)
         if dt == torch.float16:
             # the encoder object hands k-contiguous copies of its (constant) weights to the layer op, which runs them
             # on the large-M kernel once the batch fills the chip
@@ -233,7 +242,7 @@ def per_kernel(wl, T, mask_np, iters=20, vendor_gemm=False):
             except Exception:
                 pass
         ms = _time_kernel(fn, iters)
-        add(name, ms, "mfma", 2.0 * T * n * kk)
+        add(name, ms, "mfma", 2.0 * T * n * kk, SPLIT_PEAK_TFLOPS if split else MFMA_PEAK_TFLOPS[wl.dtype])
         if kw:
             res[name]["epilogue"] = "bias+gelu"
         if vendor_gemm:
@@ -279,8 +288,9 @@ def in_layer_kernels(wl, T, mask_np, reps=4):
     bias = {n: rnd(w.shape[1]) * 0.02 for n, w in weights.items()}
     gam, bet = torch.ones(H, device="cuda", dtype=dt), torch.zeros(H, device="cuda", dtype=dt)
     mm = {}
+    split = dt == torch.float32 and H % 32 == 0      # products on split rows: made here between the timed launches
     for n, w in weights.items():          # the kernel the encoder object runs this projection on
-        mm[n] = (k.gemm, w)
+        mm[n] = (k.gemm_split, k.transpose_weight(w)) if split else (k.gemm, w)
         if dt == torch.float16:
             wt = k.transpose_weight(w)
             try:
@@ -290,47 +300,54 @@ def in_layer_kernels(wl, T, mask_np, reps=4):
                 pass
     qkv = torch.empty(T, 3 * H, device="cuda", dtype=dt)
     ctx, ao, spare = (torch.empty(T, H, device="cuda", dtype=dt) for _ in range(3))
-    inter = torch.empty(T, F, device="cuda", dtype=dt)
+    inter = torch.empty(T, 3 * F, device="cuda", dtype=torch.bfloat16) if split else torch.empty(T, F, device="cuda", dtype=dt)
+    rows = torch.empty(T, 3 * H, device="cuda", dtype=torch.bfloat16) if split else None
     names = ("gemm_qkv", "attention", "gemm_attn_out", "bias_residual_layernorm", "gemm_ffn_up", "gemm_ffn_down",
              "bias_residual_layernorm")
     starts = ops.sequence_starts(vwn, bidx, B, S)          # one table per batch, as the encoder builds it
 
-    def layer(ev):
+    def layer(marks):
         cur, down = x, spare
-        for l in range(wl.layers):
-            e = ev[l] if ev else None
-            f, w = mm["gemm_qkv"]
-            if e: e[0].record()
-            f(cur, w, bias=bias["gemm_qkv"], out=qkv)
-            if e: e[1].record()
+
+        def mark(name):                    # the end of launch `name`; None: only the start of the next one
+            if marks is not None:
+                marks.append((name, events[len(marks)]))
+                marks[-1][1].record()
+
+        def product(n, a, **kw):
+            if split and a is not inter:
+                a = k.split_rows(a, out=rows)
+                mark(None)
+            f, w = mm[n]
+            f(a, w, **kw)
+            mark(n)
+
+        for _ in range(wl.layers):
+            mark(None)
+            product("gemm_qkv", cur, bias=bias["gemm_qkv"], out=qkv)
             k.attention(qkv, qkv[:, H:], qkv[:, 2 * H:], 1, 3 * H, attr, vwn, B, S, heads, d, bidx, widx, dst=ctx,
                         seq_start=starts)
-            if e: e[2].record()
-            f, w = mm["gemm_attn_out"]
-            f(ctx, w, out=ao)
-            if e: e[3].record()
+            mark("attention")
+            product("gemm_attn_out", ctx[:T], out=ao)
             k.add_bias_input_layernorm(ao, cur, bias["gemm_attn_out"], gam, bet)
-            if e: e[4].record()
-            f, w = mm["gemm_ffn_up"]
-            f(ao, w, bias=bias["gemm_ffn_up"], gelu=True, out=inter)
-            if e: e[5].record()
-            f, w = mm["gemm_ffn_down"]
-            f(inter, w, out=down)
-            if e: e[6].record()
+            mark("bias_residual_layernorm")
+            product("gemm_ffn_up", ao, bias=bias["gemm_ffn_up"], gelu=True, out=inter)
+            product("gemm_ffn_down", inter, out=down)
             k.add_bias_input_layernorm(down, ao, bias["gemm_ffn_down"], gam, bet)
-            if e: e[7].record()
+            mark("bias_residual_layernorm")
             cur, down = down, cur      # the layer's output feeds the next layer
 
     layer(None)
     tot = {n: 0.0 for n in names}
     for _ in range(reps):
-        ev = [[torch.cuda.Event(enable_timing=True) for _ in range(8)] for _ in range(wl.layers)]
+        events = [torch.cuda.Event(enable_timing=True) for _ in range(11 * wl.layers)]
         torch.cuda.synchronize()
-        layer(ev)
+        marks = []
+        layer(marks)
         torch.cuda.synchronize()
-        for e in ev:
-            for i, n in enumerate(names):
-                tot[n] += e[i].elapsed_time(e[i + 1])
+        for (_, start), (n, end) in zip(marks, marks[1:]):
+            if n is not None:
+                tot[n] += start.elapsed_time(end)
     calls = {n: reps * wl.layers * names.count(n) for n in tot}
     per = {n: tot[n] / calls[n] for n in tot}
     return per, sum(per[n] * names.count(n) for n in per)

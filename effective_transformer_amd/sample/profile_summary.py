@@ -22,7 +22,7 @@ import sys
 from .workloads import WORKLOADS
 
 ROLES = ["QKV", "attention", "attention out", "LayerNorm 1", "FFN up + GELU", "FFN down", "LayerNorm 2"]
-SIDE = ("scan_index", "compress_rows", "embed_layernorm", "seq_start", "seq_order", "mask_class", "restore_rows")
+SIDE = ("scan_index", "compress_rows", "embed_layernorm", "seq_start", "seq_order", "mask_class", "split_weight", "restore_rows")
 LAYER_KINDS = ("attention", "bias_residual_layernorm", "gemm_f16_pair", "gemm_f16_bt", "gemm_f16_persistent", "gemm_f16_kernel",
                "gemm_f32", "gemm_split")
 
@@ -162,8 +162,8 @@ def cmd_kernels(d, name, workload, bench_json=None):
             float(r["MinNs"]) / 1e3, float(r["MaxNs"]) / 1e3, r["Percentage"]))
     out.append("\nThe counts include `bench.py`'s per-kernel loops and its replica of the layer's launch sequence; `bias_gelu_kernel`,")
     out.append("`layer_prologue_kernel` and `embed_layernorm_kernel` only run there (the layer applies bias + GELU in the FFN-up GEMM's")
-    out.append("epilogue and, with prepared weights, launches no prologue).  `seq_start_kernel` + `seq_order_kernel` build the sequence")
-    out.append("table once per batch.\n")
+    out.append("epilogue and, with prepared weights, launches no prologue), and so do `seq_start_kernel` and `seq_order_kernel` (the encoder's")
+    out.append("scan writes the sequence table, its first row kernel sorts it).\n")
     trace = load_trace("%s/%s_kernel_trace.csv" % (d, name))
     agg, names, nsteps = role_durations(trace, wl.layers)
     if agg:
@@ -183,7 +183,8 @@ def cmd_kernels(d, name, workload, bench_json=None):
             if "flops" in w:
                 work = "%.1f GFLOP" % (w["flops"] / 1e9)
                 ach = "%.0f TFLOP/s" % (w["flops"] / a / 1e6)
-                frac = w["flops"] / a / 1e6 / peak
+                # split products: six 16-bit products for one of floats
+                frac = w["flops"] / a / 1e6 / (2500.0 / 6 if "gemm_split" in names[role] else peak)
             else:
                 work = "%.1f MB" % ((w["read"] + w["write"]) / 1e6)
                 ach = "%.2f TB/s" % ((w["read"] + w["write"]) / a / 1e6)
@@ -192,11 +193,13 @@ def cmd_kernels(d, name, workload, bench_json=None):
         side = {}
         for k in SIDE:
             v = [t["us"] for t in trace if t["kind"] == k]
-            if v:
+            if v and k not in ("embed_layernorm", "seq_start", "seq_order"):       # (these three: not in the encoder's steps)
                 side[k] = mean(v)
-        out.append("\nPeaks: %s MFMA %.1f TFLOP/s, HBM 8 TB/s.  Sum per layer: %.1f us; x %d layers + input / output ops and the sequence table (%s) = %.3f ms per batch."
-                   % (wl.dtype, peak, tot, wl.layers, ", ".join("%s %.1f" % kv for kv in side.items() if kv[0] != "embed_layernorm"),
-                      (tot * wl.layers + sum(v for k, v in side.items() if k != "embed_layernorm")) / 1e3))
+        tot += side.get("split_weight", 0.0)                                       # fp32: once per layer
+        out.append("\nPeaks: fp16 MFMA 2500 TFLOP/s, fp32 MFMA 157.3, products of split rows 2500 / 6, HBM 8 TB/s.  Sum per layer%s: %.1f us; x %d layers + what a batch takes once (%s) = %.3f ms per batch."
+                   % (" with split_weight %.1f" % side["split_weight"] if "split_weight" in side else "", tot, wl.layers,
+                      ", ".join("%s %.1f" % kv for kv in side.items() if kv[0] != "split_weight"),
+                      (tot * wl.layers + sum(v for k, v in side.items() if k != "split_weight")) / 1e3))
     print("\n".join(out))
 
 
@@ -287,7 +290,8 @@ def cmd_vendor(paths):
     out.append("the weights in TF's `[k][n]` order and in the k-contiguous `[n][k]` order; the own kernel includes the bias (QKV) or")
     out.append("bias + GELU (FFN up; `plain` = the same kernel without the epilogue). `in layer` = the own kernel inside the layer's")
     out.append("launch sequence (its input still in the last-level cache). TFLOP/s of the fastest vendor variant and of the own kernel")
-    out.append("alone are given for the roofline (fp16 peak 2500, fp32 157.3).\n")
+    out.append("alone are given for the roofline (fp16 peak 2500; fp32: the own kernel is the product of split rows, peak 2500 / 6, the")
+    out.append("vendor's the fp32 MFMA one, 157.3).\n")
     for path in paths:
         d = last_json_line(path)
         T = d["config"]["valid_tokens"]
