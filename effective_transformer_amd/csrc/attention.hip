@@ -7,9 +7,11 @@
 //                       (tf_op/bert_transformer_op.cu.cc:159-192); reads Q/K/V either from the padded
 //                       buffers or straight from packed token rows, writes packed [T,H].
 //
-// Softmax semantics (both kernels): t = qk*scale + (1-mask)*(-10000); m = max(max_k t, 0);
-// e = exp(t-m); p = e / (sum e + 1e-6).  In fp16 the score is rounded to half before the softmax
-// and the probability after it, as the reference stores both in half.
+// Softmax semantics (all kernels): t = qk*scale + (1-mask)*(-10000); m = max(max_k t, 0), at 1024 keys
+// max_k t; e = exp(t-m); p = e / (sum e + 1e-6).  In fp16 the score is rounded to half before the
+// softmax, as the reference stores it, and the probability before P.V: up to 64 positions p itself, as
+// the reference, beyond (streaming kernel) e, whose rounded values the sum adds up, in float, before the
+// division.
 #include <type_traits>
 
 #include "et_device.hpp"
@@ -591,20 +593,23 @@ inline int attention_cu_count() {
 // workgroups share a CU and fill each other's waits, and a stage's K and V operands serve all queries of a wavefront.
 // Bound: VALU issue while it runs (a wavefront and stage of 64 keys x 32 queries: about 1060 cycles of VALU, exp2 at a quarter
 // of the rate, against 576 of MFMA), and the start of a workgroup (order -> start table -> rows, then the first stage) over
-// the one and a half rounds its grid takes: the kernel without its arithmetic takes 23 of the 53 us.  Measured per launch,
-// 12 heads: 8 x 128 positions / 580 tokens 5.1 us (11.3 us with one workgroup's four wavefronts serving a whole head, two
-// query tiles each, and scores, mask and next rows in registers), 16 heads and 256 x 128 skewed 30 us (40 us), 16 x 1024 positions / 10700 tokens 53 us (172 us with K or V of a whole sequence in 128 KB of LDS, one workgroup
-// per CU and the scores of a query in registers), 32 x 512 positions 39 us (60 us).  Deeper rings of stages, 8 wavefronts
-// per workgroup or a bound of 3 wavefronts per SIMD: 1 to 5 % slower.
-// Rounding points are those of the other kernels (score rounded to half, softmax in float, probabilities rounded to half
-// for P.V, here before the division by the sum instead of after it).
+// the one and a half rounds its grid takes (16 x 1024: 24 of 48 us without the stages' arithmetic).  Measured per launch,
+// 12 heads: 8 x 128 positions / 570 tokens 5.4 us (11.3 us with one workgroup's four wavefronts serving a whole head, two
+// query tiles each, and scores, mask and next rows in registers), 16 heads and 256 x 128 skewed 30 us (40 us), 16 x 1024 positions
+// / 11200 tokens 46 us (172 us with K or V of a whole sequence in 128 KB of LDS, one workgroup per CU and the scores of a query
+// in registers), 32 x 512 positions / 12300 tokens 32 us (60 us).  Deeper rings of stages, 8 wavefronts per workgroup or a bound
+// of 3 wavefronts per SIMD: 1 to 5 % slower.
+// Rounding points: the score to half, the exponentials to half for P.V and, as that product's row of ones, for their sum; sums
+// in float, division last.  (The short kernel sums the exponentials before they are rounded, and rounds after the division.
+// Relative error of the output against float64, this way and that way, normal operands: 80 positions 4.50e-4 and 4.69e-4, 512
+// 5.25e-4 and 5.30e-4, 1024 5.34e-4 and 5.35e-4, 512 with scores nine times as wide 1.527e-3 and 1.534e-3.)
 //
 // Behind the stage of the last token K and V are zero, so nothing streams there: a score is the mask's bias alone, and a key
 // without a value only enters the maximum and the sum (`Unseen`).  `mask_class` says of every block of 16 queries whether its
 // mask rows are plain (1 up to the sequence's last token and 0 from there on: then no mask is read), and whether they are all 0
 // or all 1 behind the last token; other rows, and those of a caller without classes, are read 64 keys at a time.  Per launch, 12
-// heads, fp16, sequences of 16 .. 128 tokens in 32 x 512 positions: plain 13.8 us, causal 17.4, all ones 17.7, random behind
-// the tokens 38 (47 each but the first with the stages run over all positions); 64 .. 384 tokens in 64 x 384, causal: 46 (56).
+// heads, fp16, sequences of 16 .. 128 tokens in 32 x 512 positions: plain 13.6 us, causal 16.2, all ones 16.3, random behind
+// the tokens 38 (47 each but the first with the stages run over all positions); 64 .. 384 tokens in 64 x 384, causal: 42 (54).
 // ------------------------------------------------------------------------------------------
 constexpr int kFlKeys = 64;                                  // keys per stage
 constexpr int kFlStage = kFlKeys * 128;                      // bytes of K (and of V) per stage
@@ -1011,7 +1016,8 @@ __global__ __launch_bounds__(kFlWaves * kWave, 4) void attention_flash_kernel(
       if (active) stage(PLAINc, st, st & 1);
     }
   };
-  if (plain) run(std::true_type{});
+  // (expected, so that the plain loop's code runs straight into the end: 8 x 128 5.6 -> 5.4 us, and nothing is spilled)
+  if (__builtin_expect(plain, 1)) run(std::true_type{});
   else run(std::false_type{});
   wide_wait_dma();                                                     // no DMA may still target this workgroup's LDS when it ends
 
@@ -1026,7 +1032,7 @@ __global__ __launch_bounds__(kFlWaves * kWave, 4) void attention_flash_kernel(
     // the keys behind the last token's stage: no rows, the mask alone
     Unseen unseen(seq_len);
     const int keys = seq_len - stages * kFlKeys;
-    if (plain) {
+    if (__builtin_expect(plain, 1)) {
       unseen.add_zeros(seq_len, seq_len - n, ref[u]);
     } else if (zeros_behind >> (wave * QSUB + u) & 1) {
       unseen.add_zeros(seq_len, keys, ref[u]);
@@ -1102,7 +1108,7 @@ void attention_flash_launch(const void* q, const void* k, const void* v, int lay
 // with 16 consecutive features of its query; K's chunks are XOR-swizzled with the key, which spreads an operand read (16
 // rows x one chunk) over all banks.
 // Bound: the fp32 matrix instructions (a wavefront and stage: 2048 cycles of MFMA, about 400 of VALU, 16 LDS reads) over the
-// rounds of workgroups, long sequences first.  15 x 379 positions / 3850 tokens, 12 heads: 48 us per launch, 104 us with K
+// rounds of workgroups, long sequences first.  15 x 379 positions / 3820 tokens, 12 heads: 47 us per launch, 104 us with K
 // and V in chunks of 128 keys behind barriers and the scores of a query against all keys in registers.
 // ------------------------------------------------------------------------------------------
 constexpr int kF32Keys = 32;                                 // keys per stage
@@ -1321,14 +1327,14 @@ __global__ __launch_bounds__(kAttnThreads, 4) void attention_flash_f32_kernel(
       if (active) stage(PLAINc, st, st & 1);
     }
   };
-  if (plain) run(std::true_type{});
+  if (__builtin_expect(plain, 1)) run(std::true_type{});
   else run(std::false_type{});
 
   // the keys behind the last token's stage, as above
   Unseen unseen(seq_len);
   {
     const int keys = seq_len - stages * kF32Keys;
-    if (plain) {
+    if (__builtin_expect(plain, 1)) {
       unseen.add_zeros(seq_len, seq_len - n, ref);
     } else if (zeros_behind >> wave & 1) {
       unseen.add_zeros(seq_len, keys, ref);
@@ -1390,8 +1396,8 @@ void attention_flash_f32_launch(const void* q, const void* k, const void* v, int
 }
 
 // ------------------------------------------------------------------------------------------
-// fused attention for every shape the MFMA kernels above are not built for: size_per_head other than 64 (any
-// multiple of 16 bytes up to 256 elements) and 512 < seq_len <= 1024.  One wavefront per (query, head): the lanes
+// fused attention for every shape the MFMA kernels above are not built for: size_per_head other than 64 (1 to 256
+// elements), head rows off the 16-byte boundaries, and rows further apart than 31 bits reach.  One wavefront per (query, head): the lanes
 // split the keys for the scores (full dot products in float, rounded to the element type as the reference stores
 // them), the softmax runs on wave reductions, then the lanes split the features for P.V, skipping keys whose
 // probability is 0.  Same arithmetic and rounding points as the other kernels; at seq_len = 1024 the reference's block
