@@ -588,8 +588,8 @@ inline int attention_cu_count() {
 // ------------------------------------------------------------------------------------------
 // fp16 fused attention for 64 < seq_len <= 1024: one workgroup of 4 wavefronts per (64 QSUB queries, head, sequence),
 // a wavefront serves QSUB tiles of 16 queries.  K and V stream through LDS in stages of 64 keys (two stages of 16 KB, the
-// next one arriving by DMA under the work on this one), and the softmax runs along with them: per query the maximum so
-// far, the sum and the output so far, rescaled where the maximum moves.  Nothing grows with the sequence, so several
+// next one arriving by DMA under the work on this one), and the softmax runs along with them (a published method: Milakov and
+// Gimelshein, 2018): per query the maximum so far, the sum and the output so far, rescaled where the maximum moves.  Nothing grows with the sequence, so several
 // workgroups share a CU and fill each other's waits, and a stage's K and V operands serve all queries of a wavefront.
 // Bound: VALU issue while it runs (a wavefront and stage of 64 keys x 32 queries: about 1060 cycles of VALU, exp2 at a quarter
 // of the rate, against 576 of MFMA), and the start of a workgroup (order -> start table -> rows, then the first stage) over

@@ -4,14 +4,17 @@
 // A float is the exact sum of three bfloat16 numbers h + m + l, each the rest of the ones before it rounded to nearest
 // (8 significand bits and a sign apiece cover the 24 bits, in the float's own exponent range).  A product of two such
 // floats is nine products of pieces; the three of weight 2^-26 and less (m.l, l.m, l.l) lie below a quarter unit of the
-// float product and are left out, the other six go through v_mfma_f32_16x16x32_bf16, each exact and summed in float.  The leading
+// float product and are left out, the other six go through v_mfma_f32_16x16x32_bf16, each exact and summed in float (splitting
+// floats into bfloat16 pieces for such a product is a published method: Henry, Tang and Heinecke, 2019).  Infinities, NaNs and
+// magnitudes above 3.38e38 have NaN pieces.  The leading
 // products (h.h) and the five corrections have an accumulator of their own: the matrix core cuts an addend that is
 // small beside its accumulator, which would otherwise bias every correction towards zero.  Against float64 the result is
 // closer than the fp32 matrix instructions' (k = 3072, normal operands: 3.4e-7 relative against 9.9e-7; all operands
 // positive: 3.0e-7 against 8.6e-7), at six times the work of a 16-bit product on units sixteen times as fast.
 //
 // Both operands come as "split rows": [row][k / 32][h, m, l][32] bfloat16, 192 contiguous bytes per row and k-step of 32.
-// The kernels that produce A (input, attention, LayerNorm, GELU) write that form themselves; weights are split once.
+// The kernels that produce A (input, attention, LayerNorm, GELU) write that form themselves; weights are split by every layer
+// call unless the caller hands the copies over (15 us per layer of BERT-base in the trace, 9 us of its time).
 // Bound: at large m the power limit of the matrix cores (20000 rows, k = 768 / n = 2304, 768, 3072 + GELU and k = 3072 /
 // n = 768: 385, 113, 490, 427 us, i.e. 1090 .. 1330 TFLOP/s of 16-bit products; all-zero operands 288, 100, 441, 383 us;
 // the fp32 matrix instructions took 617, 211, 780, 767 us); below a round of the chip the k loop of one tile (160 rows:

@@ -130,7 +130,10 @@ et_status et_input_static(et_handle h, et_dtype dtype, const void* from_tensor, 
  * alias from_tensor/to_tensor.  Shapes: seq_len <= 1024, batch_size <= 65535, any size_per_head from 1 to 256 (see
  * et_attention), head_num * size_per_head <= 1048576 (every entry point), activations below 4 GB per matrix.  The tuned kernels take head size 64 and hidden sizes in multiples of 32 (fp16) or 16 (fp32); every
  * other shape runs element-wise kernels with the same arithmetic (the reference's kernels index by element too,
- * cuda/attention.cu:190-219). */
+ * cuda/attention.cu:190-219).
+ * The weights are read anew by every call and stay as they are: the copies the products read (k-contiguous in fp16, split
+ * rows in fp32, see et_gemm_split) are made in the workspace.  fp32 products of hidden sizes in multiples of 32 run on split
+ * rows: what et_gemm_split says of infinities and of the terms it leaves out goes for them. */
 et_status et_layer(et_handle h, et_dtype dtype, const et_layer_weights* weights,
                    const void* from_tensor, const void* to_tensor, const void* attr_mask,
                    const int32_t* valid_word_num_dev, const int32_t* batch_idx, const int32_t* word_idx,
@@ -140,9 +143,9 @@ et_status et_layer(et_handle h, et_dtype dtype, const et_layer_weights* weights,
 /* What a caller that keeps a layer's weights constant can prepare once instead of having et_layer redo it on every
  * call.  No counterpart in the reference, whose op receives the weights as inputs of every call (tf_op/
  * bert_transformer_op.cc:44-77) and rebuilds nothing across calls either.  Every member may be NULL.
- *   *_t: the dense kernel as et_transpose_weight leaves it: [out,in] (k-contiguous) in fp16, split rows in fp32.  The
- *        call then skips making that copy itself; Q, K and V go together.  Ignored for hidden sizes whose GEMMs read the
- *        [in,out] tensors (no multiple of 64 in fp16, of 32 in fp32).
+ *   *_t: the dense kernel as et_transpose_weight leaves it: [out,in] (k-contiguous) in fp16, split rows in fp32 (6 bytes a
+ *        value).  The call then skips making that copy itself and does not look at the tensor it was made of; Q, K and V go
+ *        together.  Ignored for hidden sizes whose GEMMs read the [in,out] tensors (no multiple of 64 in fp16, of 32 in fp32).
  *   seq_start, seq_start_bytes: the sequence table et_sequence_starts wrote for THIS batch and the size of its buffer
  *        (at least et_seq_workspace_bytes(batch_size), ET_WORKSPACE_TOO_SMALL below); the same table serves every
  *        layer of the batch.
@@ -316,7 +319,12 @@ et_status et_transpose_rm_padding(et_handle h, et_dtype dtype, const void* src, 
  *                 stride `packed_ld` elements (bias already added).
  *   dst packed [T,heads*d].  workspace: et_seq_workspace_bytes(B).
  * seq_len <= 1024; size_per_head from 1 to 256.  size_per_head = 64 (head rows on 16-byte boundaries) runs the MFMA
- * kernels, every other head size a slower general kernel with the same arithmetic. */
+ * kernels, every other head size a slower general kernel.  Rounding in fp16: the score to half in all of them; up to 64
+ * positions and in the general kernel the exponentials are summed in float and the probability is rounded to half; beyond, the
+ * exponentials are rounded to half, their sum adds up the rounded values in float, and the output is divided by it.
+ * Masks that end with the sequence (rows of 1 up to the last token, 0 behind it) are the fastest form; with a workspace of
+ * et_seq_workspace_bytes(B) the call finds out which blocks of 16 queries have it, and which have all 0 or all 1 behind the
+ * last token. */
 et_status et_attention(et_handle h, et_dtype dtype, const void* q, const void* k, const void* v, int qkv_layout,
                        int packed_ld, const void* attr_mask, void* dst,
                        const int32_t* valid_word_num_dev, int batch_size, int seq_len,
@@ -374,7 +382,10 @@ et_status et_gemm_bt_bias_gelu(et_handle h, et_dtype dtype, const void* A, const
  * split rows, [row][k / 32][3][32] bfloat16: every float is the exact sum of three bfloat16 pieces (h, m, l, each the rest
  * of the ones before it rounded to nearest), kept side by side for every 32 values.  The six products of pieces that
  * reach into the float result are summed in float, leading ones and corrections apart; against float64 the result is
- * closer than that of the fp32 matrix instructions et_gemm runs on.  k % 32 == 0, n % 4 == 0.  C is float [m,n]; with
+ * closer than that of the fp32 matrix instructions et_gemm runs on; the other three (middle by low, low by middle and low by
+ * low: below a quarter of a unit of each float product) are left out.  The pieces are exact for finite values up to 3.38e38;
+ * larger ones, infinities and NaN give NaN pieces, and with them NaN results where et_gemm may give an infinity.
+ * k % 32 == 0, n % 4 == 0.  C is float [m,n]; with
  * gelu it holds the split rows of gelu(A.Bt^T + bias) instead (6 n bytes per row, n % 32 == 0, bias required).  Bt comes
  * from et_transpose_weight(ET_FP32), A from et_split_rows: dst = the split rows of the first m (or *m_dev) rows of
  * src[m][k]. */
