@@ -123,3 +123,33 @@ def test_padding_costs_little_under_any_mask(dtype, form):
     narrow, wide = microseconds(128), microseconds(512)
     print("padding", dtype, form, "us", narrow, wide, flush=True)
     assert wide < 2 * narrow
+
+
+def test_workspaces_with_and_without_room_for_the_classes():
+    """et_attention takes a workspace that holds the sequence table alone and makes no classes then; the first size that holds
+    both is et_seq_workspace_bytes' at 1024 positions.  A plain mask: the same bits either way."""
+    from effective_transformer_amd import _lib
+    lib, B, S = _lib.load(), 40, 1024
+    rng = np.random.RandomState(5)
+    lens = rng.randint(1, 200, size=B)
+    mask = dev((np.arange(S)[None] < lens[:, None]).astype(np.int32))
+    attr = mask[:, None].expand(B, S, S).half().contiguous()
+    _, count, bi, wi = ops.effective_transformer_input(torch.zeros(B, S, 64, dtype=torch.float16, device="cuda"), mask, B, S, S, 1, 64)
+    T = int(lens.sum())
+    qkv = dev(rng.randn(T, 192).astype(np.float16))
+    full = lib.et_seq_workspace_bytes(B)
+    table = full - B * 64
+    assert table == ((2 * B + 1) * 4 + 255) // 256 * 256
+    want, h = None, ops.handle(qkv.device)
+    for nbytes in (table, full - 1, full):
+        ws = torch.zeros(full + 256, dtype=torch.uint8, device="cuda")
+        dst = torch.zeros(T, 64, dtype=torch.float16, device="cuda")
+        _lib.check(lib.et_attention(h, _lib.ET_FP16, qkv.data_ptr(), qkv[:, 64:].data_ptr(), qkv[:, 128:].data_ptr(), 1, 192,
+                                    attr.data_ptr(), dst.data_ptr(), count.data_ptr(), B, S, 1, 64, bi.data_ptr(), wi.data_ptr(),
+                                    ws.data_ptr(), nbytes, torch.cuda.current_stream().cuda_stream), h)
+        want = dst if want is None else want
+        assert torch.equal(dst, want)
+        assert (ws[nbytes:] == 0).all() and bool((ws[table:] != 0).any()) == (nbytes == full)
+    assert lib.et_attention(h, _lib.ET_FP16, qkv.data_ptr(), qkv.data_ptr(), qkv.data_ptr(), 1, 192, attr.data_ptr(),
+                            want.data_ptr(), count.data_ptr(), B, S, 1, 64, bi.data_ptr(), wi.data_ptr(), ws.data_ptr(), table - 1,
+                            None) == 2
