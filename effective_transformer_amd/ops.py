@@ -481,7 +481,7 @@ class EffectiveTransformerEncoder:
             if not 0 < rows_bound <= B * S:
                 raise ValueError("rows_bound must be in 1 .. batch * seq_len")
             batch.rows_bound = int(rows_bound)
-        if sync_count:
+        if sync_count and len(self.layers) > 1:      # (a single layer does not wait: it may be captured as it is)
             key = (stream, threading.get_ident())
             word = self._count_words.get(key)
             if word is None:

@@ -102,6 +102,24 @@ def test_one_encoder_on_two_streams():
         assert all(torch.equal(o, w) for o in g)
 
 
+@pytest.mark.parametrize("dtype", ["fp32", "fp16"])
+def test_single_layer_under_capture(dtype):
+    """An encoder of one layer waits for nothing, so a caller may capture the call as it is (a deeper one with sync_count=False)."""
+    wl, enc, x, mask, attr, _ = _batch(12, 40, 1, dtype)
+    fewer, m = mask.clone(), mask.clone()
+    fewer[5:, 10:] = 0
+    want = [enc(x, k, attr).clone() for k in (mask, fewer)]
+    torch.cuda.synchronize()
+    graph = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(graph):
+        out = enc(x, m, attr)
+    for i in (0, 1, 0, 1):
+        m.copy_((mask, fewer)[i])
+        graph.replay()
+        assert torch.equal(out, want[i])
+        assert torch.equal(enc(x, m, attr), want[i])         # eager work between the replays
+
+
 def test_refused_arguments():
     wl, enc, x, mask, attr, _ = _batch(2, 8, 2, "fp16")
     lib = _lib.load()
