@@ -352,7 +352,7 @@ def _require_masks(B: int, S: int, input_mask: torch.Tensor, attention_mask: tor
     """The masks of B sequences of S positions, in full: the kernels read that much of them."""
     if input_mask.dim() != 2 or input_mask.shape[0] < B or input_mask.shape[1] != S:
         raise ValueError("mask %s must be [%d, %d]" % (tuple(input_mask.shape), B, S))
-    if attention_mask.shape[-1] != S or attention_mask.numel() < B * S * S:
+    if (attention_mask.dim() > 1 and attention_mask.shape[-1] != S) or attention_mask.numel() < B * S * S:
         raise ValueError("attention mask %s must be [%d, %d, %d]" % (tuple(attention_mask.shape), B, S, S))
 
 
@@ -444,7 +444,7 @@ class EffectiveTransformerEncoder:
         input_mask [B,S]; the other tensors may hold more sequences."""
         B, S = input_mask.shape
         for ids in (input_ids,) if token_type_ids is None else (input_ids, token_type_ids):
-            if ids.shape[-1] != S or ids.numel() < B * S:
+            if (ids.dim() > 1 and ids.shape[-1] != S) or ids.numel() < B * S:
                 raise ValueError("ids %s must be [%d, %d] (mask)" % (tuple(ids.shape), B, S))
         if embeddings.hidden != self.head_num * self.size_per_head:
             raise ValueError("embeddings of %d columns for a hidden size of %d" %

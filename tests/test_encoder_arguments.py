@@ -51,7 +51,8 @@ def test_fewer_sequences_than_the_masks_hold(dtype):
     got = enc(x[:3], mask, attr)
     assert got.shape == x[:3].shape and torch.equal(got, want)
     assert torch.equal(enc(x[:3], mask, attr, sync_count=False), want)
-    assert torch.equal(enc(x[:3], mask, attr[:, None]), want)        # [B,1,S,S]
+    for same in (attr[:, None], attr.reshape(-1)):                    # [B,1,S,S], flat
+        assert torch.equal(enc(x[:3], mask, same), want)
 
 
 def _layer(n):
