@@ -243,8 +243,8 @@ def test_softmax(k, dtype, S):
 @pytest.mark.parametrize("dtype", ["fp32", "fp16"])
 @pytest.mark.parametrize("S,holes,weird", [(5, False, False), (32, False, False), (64, False, False),
                                            (64, True, True), (100, True, False), (128, False, True), (21, True, True),
-                                           # beyond 128 positions: fp32 the chunked kernel (K and V in 128-key chunks),
-                                           # fp16 the kernel that keeps K and V of a sequence in LDS
+                                           # beyond 64 (fp32: 32) positions: the streaming kernels, K and V in stages of
+                                           # 64 (32) keys
                                            (129, False, False), (200, True, True), (256, False, False),
                                            (300, True, False), (384, False, True), (512, False, False), (509, True, True)])
 def test_fused_attention_both_layouts(k, dtype, S, holes, weird):
@@ -279,9 +279,8 @@ def test_fused_attention_both_layouts(k, dtype, S, holes, weird):
         np.testing.assert_allclose(got0[:T].astype(np.float32), want.astype(np.float32), rtol=4e-3, atol=4e-3)
 
 
-# fp16, 128 < seq_len <= 512: K and V of a sequence stay in LDS for all of its query tiles, which are dealt to one, two
-# or four workgroups per (head, sequence) depending on how many such pairs the batch has (on a 256-CU part: 288, 144
-# and 12 pairs here).
+# fp16 beyond 64 positions: one or two query tiles per wavefront, depending on how many (head, sequence, 128 queries) the batch
+# has (two from 512 on a 256-CU part: 576, 432, 48 and 528 here).
 @pytest.mark.parametrize("B,heads,S,holes,weird", [(24, 12, 200, True, False), (12, 12, 300, False, True),
                                                    (3, 4, 500, True, True), (22, 12, 130, False, False)])
 def test_fused_attention_with_resident_keys(k, B, heads, S, holes, weird):
@@ -342,7 +341,7 @@ def test_fused_attention_other_head_sizes_and_long_sequences(k, dtype, S, d, hol
 def test_fused_attention_long_sequences_same_bits_in_any_batch(k, dtype, S):
     """A sequence's attention output does not depend on what else is in the batch or where it stands in it: the same
     five sequences in two orders, and one of them alone, give the same bits (kernels that split a sequence's queries
-    or keys over workgroups and wavefronts: keys resident in LDS up to 512 positions, key halves beyond)."""
+    over workgroups and wavefronts and stream the keys)."""
     print("attention batch independence", dtype, S, flush=True)
     heads, d = 3, 64
     H = heads * d
@@ -379,7 +378,7 @@ def test_fused_attention_long_sequences_same_bits_in_any_batch(k, dtype, S):
 @pytest.mark.parametrize("S", [40, 64, 100, 128])
 @pytest.mark.parametrize("layout", [1, 0])
 def test_fused_attention_mixed_lengths_same_bits_in_any_batch(k, dtype, S, layout):
-    """The kernel for up to 128 positions on a batch of very different sequences: every sequence must give the bits it
+    """Up to 128 positions (the short kernel and the streaming ones) on a batch of very different sequences: every sequence must give the bits it
     gives alone in a batch of one, whatever stands beside it, and match the oracle: short and long sequences,
     token-less ones, a short one whose tokens sit at late positions, holes, and masks that attend to padded keys
     (their zero scores count in the softmax of the sequence they belong to)."""
