@@ -768,6 +768,15 @@ et_status wait_for_count(et_handle h, const uint64_t* word, uint32_t tag, const 
   }
 }
 
+bool is_capturing(hipStream_t st) {
+  hipStreamCaptureStatus status = hipStreamCaptureStatusNone;
+  if (hipStreamIsCapturing(st, &status) != hipSuccess) {
+    (void)hipGetLastError();
+    return false;
+  }
+  return status != hipStreamCaptureStatusNone;
+}
+
 }  // namespace
 
 size_t et_encoder_workspace_bytes(et_dtype dtype, int batch_size, int seq_len, int head_num, int size_per_head) {
@@ -814,10 +823,11 @@ et_status et_encoder(et_handle h, et_dtype dtype, int num_layers, const et_layer
   // The layers of a stack wait for it at every size.  12 layers, waiting and launched for all positions, us per pass in a stream
   // of passes: fp16 1 x 32 405 and 405, 4 x 32 with 41 tokens 414 and 424, 8 x 32 with 120 434 and 457, 12 x 32 with 172 449 and
   // 492, 32 x 32 with 546 545 and 635; fp32 854 and 872, 899 and 968, 964 and 1054, 1019 and 1283, 1379 and 1743.
-  const bool wait_for_layers = b->rows_bound == 0 && num_layers > 1;
+  // (Nothing runs while a stream is being captured, so there the launches are sized for all positions.)
+  const bool wait_for_layers = b->rows_bound == 0 && num_layers > 1 && b->count_word && !is_capturing(st);
   et::ScanExtras scan;
   scan.seq_start = seq;
-  if (b->count_word && (wait_for_layers || b->valid_word_num)) {
+  if (wait_for_layers || (b->count_word && b->valid_word_num)) {
     scan.host_word = b->count_word;
     scan.host_tag = next_tag.fetch_add(1, std::memory_order_relaxed);
     if (scan.host_tag == 0) scan.host_tag = next_tag.fetch_add(1, std::memory_order_relaxed);
@@ -857,7 +867,7 @@ et_status et_encoder(et_handle h, et_dtype dtype, int num_layers, const et_layer
   c.workspace = layer_base;
   c.stream = st;
   int T = -1;
-  if (wait_for_layers && scan.host_word) {
+  if (wait_for_layers) {
     // The count is there when the scan ends and the host has it while the input rows are still being moved: the layers
     // are launched for exactly that many rows (other threads may use the handle meanwhile).
     entry.lock.unlock();

@@ -240,9 +240,9 @@ typedef struct et_encoder_batch {
  * (et_encoder_workspace_bytes).  weights, prepared (may be NULL; its seq_start members are not used): one per layer.  Same
  * results as the ops called one by one, bit for bit.
  * With count_word, rows_bound 0 and more than one layer the host waits for the valid-token count, which the scan stores there
- * while the input rows are still being moved, and every layer is launched for exactly that many rows; otherwise nothing is
- * waited for and every launch is sized for B*S rows (or rows_bound) and bounded on the device (what a call under graph
- * capture needs). */
+ * while the input rows are still being moved, and every layer is launched for exactly that many rows; otherwise, and while
+ * `stream` is being captured, nothing is waited for and every launch is sized for B*S rows (or rows_bound) and bounded on the
+ * device. */
 size_t et_encoder_workspace_bytes(et_dtype dtype, int batch_size, int seq_len, int head_num, int size_per_head);
 et_status et_encoder(et_handle h, et_dtype dtype, int num_layers, const et_layer_weights* weights,
                      const et_layer_prepared* prepared, const et_encoder_batch* batch, int head_num, int size_per_head,

@@ -120,6 +120,29 @@ def test_single_layer_under_capture(dtype):
         assert torch.equal(enc(x, m, attr), want[i])         # eager work between the replays
 
 
+@pytest.mark.parametrize("B,S", [(2, 40), (12, 40)])
+def test_call_that_would_wait_under_capture(B, S):
+    """A deeper encoder whose pinned word exists already (an earlier call on the stream that captures): the call does not wait
+    while the stream is being captured, and the replays follow the mask."""
+    wl, enc, x, mask, attr, _ = _batch(B, S, 2, "fp16")
+    fewer, m = mask.clone(), mask.clone()
+    fewer[B // 2:, 10:] = 0
+    want = [enc(x, k, attr).clone() for k in (mask, fewer)]
+    side = torch.cuda.Stream()
+    side.wait_stream(torch.cuda.current_stream())
+    with torch.cuda.stream(side):
+        enc(x, m, attr)
+    torch.cuda.synchronize()
+    graph = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(graph, stream=side):
+        out = enc(x, m, attr)
+    for i in (0, 1, 0, 1):
+        m.copy_((mask, fewer)[i])
+        graph.replay()
+        assert torch.equal(out, want[i])
+        assert torch.equal(enc(x, m, attr), want[i])         # eager work between the replays
+
+
 def test_refused_arguments():
     wl, enc, x, mask, attr, _ = _batch(2, 8, 2, "fp16")
     lib = _lib.load()
