@@ -93,7 +93,7 @@ def fold_traffic(workload, fetch_csv, write_csv, commit, command):
 PUBLISHED_MS = {"cfg2": (8.75, "Readme.md:65"), "cfg3": (133.61, "Readme.md:80"), "cfg4": (325.37, "Readme.md:89")}
 HBM_PEAK_GBS = 8000.0
 MFMA_PEAK_TFLOPS = {"fp16": 2500.0, "fp32": 157.3}
-SPLIT_PEAK_TFLOPS = 2500.0 / 6      # fp32 products of split rows: six 16-bit products for one of floats
+PAIR_PEAK_TFLOPS = 2500.0 / 3       # fp32 products of pair rows: three 16-bit products for one of floats
 
 
 def _time_kernel(fn, iters, warm=3):
@@ -224,13 +224,19 @@ def per_kernel(wl, T, mask_np, iters=20, vendor_gemm=False):
         kw = {"bias": bF, "gelu": True} if name == "gemm_ffn_up" else {}
         fn = lambda: k.gemm(A, Bm, out=Cm, **kw)
         plain = lambda: k.gemm(A, Bm, out=Cm)
-        split = dt == torch.float32 and kk % 32 == 0
-        if split:
-            # the layer's products read split rows; the kernels in front of them write that form
-            sa, sb = k.split_rows(A), k.transpose_weight(Bm)
-            Cs = torch.empty(T, 3 * n, device="cuda", dtype=torch.bfloat16) if kw else Cm
-            fn = lambda: k.gemm_split(sa, sb, out=Cs, **kw)
-            plain = lambda: k.gemm_split(sa, sb, out=Cm)
+        pairs = dt == torch.float32          # (every fp32 workload's hidden size is one that runs on pair rows)
+        if pairs:
+            # the layer's products read pair rows; the kernels in front of them write that form
+            sb, stats = k.pair_weight(Bm, kw.get("bias"))
+            if kk <= 2048:
+                sa = k.pair_rows(A)
+            else:                            # as wide as the intermediate: made by the product that makes it there
+                narrow = rnd(T, H)
+                up, up_stats = k.pair_weight(rnd(H, kk) * 0.02, bF)
+                sa = k.gemm_pair(k.pair_rows(narrow), up, bias=bF, stats=up_stats, gelu=True)
+            Cs = k.PairRows(T, n, "cuda") if kw else Cm
+            fn = lambda: k.gemm_pair(sa, sb, out=Cs, stats=stats, **kw)
+            plain = lambda: k.gemm_pair(sa, sb, out=Cm)
         if dt == torch.float16:
             # the encoder object hands k-contiguous copies of its (constant) weights to the layer op, which runs them
             # on the large-M kernel once the batch fills the chip
@@ -242,7 +248,7 @@ def per_kernel(wl, T, mask_np, iters=20, vendor_gemm=False):
             except Exception:
                 pass
         ms = _time_kernel(fn, iters)
-        add(name, ms, "mfma", 2.0 * T * n * kk, SPLIT_PEAK_TFLOPS if split else MFMA_PEAK_TFLOPS[wl.dtype])
+        add(name, ms, "mfma", 2.0 * T * n * kk, PAIR_PEAK_TFLOPS if pairs else MFMA_PEAK_TFLOPS[wl.dtype])
         if kw:
             res[name]["epilogue"] = "bias+gelu"
         if vendor_gemm:
@@ -288,9 +294,14 @@ def in_layer_kernels(wl, T, mask_np, reps=4):
     bias = {n: rnd(w.shape[1]) * 0.02 for n, w in weights.items()}
     gam, bet = torch.ones(H, device="cuda", dtype=dt), torch.zeros(H, device="cuda", dtype=dt)
     mm = {}
-    split = dt == torch.float32 and H % 32 == 0      # products on split rows: made here between the timed launches
+    pairs = dt == torch.float32                      # products on pair rows: made here between the timed launches
+    stats = None
     for n, w in weights.items():          # the kernel the encoder object runs this projection on
-        mm[n] = (k.gemm_split, k.transpose_weight(w)) if split else (k.gemm, w)
+        if pairs:
+            wp, st = k.pair_weight(w, bias[n] if n == "gemm_ffn_up" else None)
+            mm[n], stats = (k.gemm_pair, wp), st if st is not None else stats
+            continue
+        mm[n] = (k.gemm, w)
         if dt == torch.float16:
             wt = k.transpose_weight(w)
             try:
@@ -300,8 +311,8 @@ def in_layer_kernels(wl, T, mask_np, reps=4):
                 pass
     qkv = torch.empty(T, 3 * H, device="cuda", dtype=dt)
     ctx, ao, spare = (torch.empty(T, H, device="cuda", dtype=dt) for _ in range(3))
-    inter = torch.empty(T, 3 * F, device="cuda", dtype=torch.bfloat16) if split else torch.empty(T, F, device="cuda", dtype=dt)
-    rows = torch.empty(T, 3 * H, device="cuda", dtype=torch.bfloat16) if split else None
+    inter = k.PairRows(T, F, "cuda") if pairs else torch.empty(T, F, device="cuda", dtype=dt)
+    rows = k.PairRows(T, H, "cuda") if pairs else None
     names = ("gemm_qkv", "attention", "gemm_attn_out", "bias_residual_layernorm", "gemm_ffn_up", "gemm_ffn_down",
              "bias_residual_layernorm")
     starts = ops.sequence_starts(vwn, bidx, B, S)          # one table per batch, as the encoder builds it
@@ -315,9 +326,11 @@ def in_layer_kernels(wl, T, mask_np, reps=4):
                 marks[-1][1].record()
 
         def product(n, a, **kw):
-            if split and a is not inter:
-                a = k.split_rows(a, out=rows)
+            if pairs and a is not inter:
+                a = k.pair_rows(a, out=rows)
                 mark(None)
+            if pairs and kw.get("gelu"):
+                kw["stats"] = stats
             f, w = mm[n]
             f(a, w, **kw)
             mark(n)

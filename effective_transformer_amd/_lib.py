@@ -35,6 +35,10 @@ class LayerPrepared(C.Structure):
                 ("seq_start_bytes", C.c_size_t)]
 
 
+class PairMatrix(C.Structure):
+    _fields_ = [("rows", C.c_void_p), ("exp", C.c_void_p), ("norm", C.c_void_p)]
+
+
 class EmbeddingWeights(C.Structure):
     _fields_ = [("word_embeddings", C.c_void_p), ("token_type_embeddings", C.c_void_p),
                 ("position_embeddings", C.c_void_p), ("layernorm_gamma", C.c_void_p), ("layernorm_beta", C.c_void_p),
@@ -99,6 +103,11 @@ SIGNATURES = {
     "et_gemm_bt_bias_gelu": (_i, [_vp, _i, _vp, _vp, _vp, _vp, _i, _i, _i, _vp, _vp]),
     "et_split_rows": (_i, [_vp, _vp, _vp, _i, _i, _vp, _vp]),
     "et_gemm_split": (_i, [_vp, _vp, _vp, _vp, _vp, _i, _i, _i, _i, _vp, _vp]),
+    "et_pair_weight_stats": (_sz, [_i, _i]),
+    "et_pair_weight_workspace_bytes": (_sz, [_i, _i]),
+    "et_pair_rows": (_i, [_vp, _vp, C.POINTER(PairMatrix), _i, _i, _vp, _vp]),
+    "et_pair_weight": (_i, [_vp, _vp, _vp, _vp, _vp, _vp, _i, _i, _vp, _sz, _vp]),
+    "et_gemm_pair": (_i, [_vp, C.POINTER(PairMatrix), _vp, _vp, _vp, _vp, _vp, _vp, _i, _i, _i, _vp, _vp]),
     "et_calibrate_mfma_sink_bytes": (_sz, [_vp]),
     "et_calibrate_mfma": (_i, [_vp, _i, _i, _vp, _sz, C.POINTER(C.c_double), _vp]),
 }

@@ -22,7 +22,7 @@ OBJDIR = os.path.join(LIBDIR, "obj")
 LIB = os.path.join(LIBDIR, "libet_hip.so")
 EXAMPLE = os.path.join(LIBDIR, "et_encoder_example")      # C++ host sample (csrc/encoder_example.cpp)
 
-SOURCES = ["input_output.hip", "row_kernels.hip", "attention.hip", "gemm.hip", "gemm_split.hip", "generic.hip", "calibrate.hip", "et_api.cpp"]
+SOURCES = ["input_output.hip", "row_kernels.hip", "attention.hip", "gemm.hip", "gemm_split.hip", "gemm_pair.hip", "generic.hip", "calibrate.hip", "et_api.cpp"]
 
 FLAGS = [
     "--offload-arch=gfx950", "-O3", "-std=c++17", "-fPIC", "-fno-gpu-rdc",
@@ -35,7 +35,8 @@ FLAGS = [
 # per source: the attention kernels keep their MFMA accumulators in VGPRs (with the accumulator registers as
 # destination every score and output value costs a v_accvgpr_read before the VALU can touch it: 24 of the 193 VALU
 # instructions per head and query tile of the short fp16 kernel)
-EXTRA_FLAGS = {"attention.hip": ["-mllvm", "-amdgpu-mfma-vgpr-form=1"], "gemm_split.hip": ["-mllvm", "-amdgpu-mfma-vgpr-form=1"]}
+EXTRA_FLAGS = {"attention.hip": ["-mllvm", "-amdgpu-mfma-vgpr-form=1"], "gemm_split.hip": ["-mllvm", "-amdgpu-mfma-vgpr-form=1"],
+               "gemm_pair.hip": ["-mllvm", "-amdgpu-mfma-vgpr-form=1"]}
 
 
 def hipcc() -> str:

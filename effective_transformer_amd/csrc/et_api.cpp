@@ -174,32 +174,65 @@ et_status check_launch(et_handle h, const char* what) {
 bool dtype_ok(et_dtype d) { return d == ET_FP32 || d == ET_FP16; }
 et::DType to_dt(et_dtype d) { return d == ET_FP32 ? et::DType::F32 : et::DType::F16; }
 
-// fp32 layers of these hidden sizes run their products on split rows (gemm_split.hip); the rest on the fp32 kernels
-bool layer_splits(et_dtype dtype, int H) { return dtype == ET_FP32 && H % 32 == 0 && et::gemm_split_supported(H, 4 * H); }
+// How fp32 layers run their products: on pair rows (gemm_pair.hip) from 512 hidden values on, where they are closer to float64
+// than split rows (k = 512: 1.22e-7 against 1.27e-7, wider: gemm_pair.hip) at half the work, up to the rows the row kernels hold
+// in registers; on split rows (gemm_split.hip) at the other multiples of 32; the rest on the fp32 kernels.
+bool layer_pairs(et_dtype dtype, int H) {
+  return dtype == ET_FP32 && H >= 512 && et::pair_rows_supported(H) && et::gemm_pair_supported(H, 4 * H);
+}
+bool layer_splits(et_dtype dtype, int H) {
+  return dtype == ET_FP32 && !layer_pairs(dtype, H) && H % 32 == 0 && et::gemm_split_supported(H, 4 * H);
+}
 
 struct LayerWs {
-  size_t qkv, ctx, attn, attn_split, inter, seq, cls, wt, total;
+  size_t qkv, ctx, attn, attn_split, inter, seq, cls, wt, pair, total;
 };
+
+// Row arrays and weight arrays of a layer on pair rows, behind its matrices.
+struct PairWs {
+  int32_t *from_exp, *to_exp, *ctx_exp, *attn_exp, *inter_exp, *w_exp;      // w_exp: Q, K, V, output, up, down
+  float *from_norm, *to_norm, *attn_norm, *v_stats, *up_stats, *tops;
+};
+size_t pair_array_rows(size_t rows) { return align_up(rows, 256) + 256; }      // whole tiles of any height up to 256
+size_t pair_ws_words(size_t rows, size_t H) {
+  const int h = (int)H;
+  return 8 * pair_array_rows(rows) + 9 * H + 2 * (et::pair_weight_stats(h, h) + et::pair_weight_stats(4 * h, h)) +
+         8 * et::pair_weight_tops(h, h) + et::pair_weight_tops(h, 4 * h);
+}
+PairWs pair_ws(char* p, size_t rows, size_t H) {
+  const size_t r = pair_array_rows(rows);
+  int32_t* i = (int32_t*)p;
+  PairWs w;
+  w.from_exp = i; w.to_exp = i + r; w.ctx_exp = i + 2 * r; w.attn_exp = i + 3 * r; w.inter_exp = i + 4 * r;
+  float* f = (float*)(i + 5 * r);
+  w.from_norm = f; w.to_norm = f + r; w.attn_norm = f + 2 * r;
+  w.w_exp = (int32_t*)(f + 3 * r);
+  w.v_stats = (float*)(w.w_exp + 9 * H);
+  w.up_stats = w.v_stats + 2 * et::pair_weight_stats((int)H, (int)H);
+  w.tops = w.up_stats + 2 * et::pair_weight_stats(4 * (int)H, (int)H);
+  return w;
+}
 
 LayerWs layer_ws(et_dtype dtype, int B, int S, int heads, int d) {
   const size_t e = dtype == ET_FP32 ? 4 : 2;
   const size_t rows = (size_t)B * S, H = (size_t)heads * d;
-  const bool split = layer_splits(dtype, heads * d);
-  const size_t ea = split ? 6 : e;               // bytes of a value that only a product reads
+  const bool pairs = layer_pairs(dtype, heads * d), split = pairs || layer_splits(dtype, heads * d);
+  const size_t ea = split && !pairs ? 6 : e;     // bytes of a value that only a product reads
   LayerWs w;
   size_t off = 0;
   w.qkv = off;   off += align_up(rows * 3 * H * e, 256);
   w.ctx = off;   off += align_up(rows * H * ea, 256);
   w.attn = off;  off += align_up(rows * H * e, 256);
   w.attn_split = off; off += split ? align_up(rows * H * ea, 256) : 0;
-  // whole tiles of 256 rows: the FFN's intermediate may be handed over in blocks of [256 rows][64 columns].  The split
+  // whole tiles of 256 rows: the FFN's intermediate may be handed over in blocks of [256 rows][64 columns].  The split (pair)
   // rows of from_tensor and to_tensor lie here while the Q/K/V projections read them, those of the layer's output once
   // the intermediate has been consumed.
   w.inter = off; off += align_up(align_up(rows, 256) * 4 * H * ea, 256);
   w.seq = off;   off += align_up(et::seq_table_words(B) * sizeof(int32_t), 256);
   w.cls = off;   off += align_up(et::mask_class_bytes(dtype == ET_FP32 ? et::DType::F32 : et::DType::F16, B, S, d), 256);
-  // k-contiguous copies (fp32: split rows) of the six dense kernels (3 H^2 + H^2 + 4 H^2 + 4 H^2 elements)
+  // k-contiguous copies (fp32: split or pair rows) of the six dense kernels (3 H^2 + H^2 + 4 H^2 + 4 H^2 elements)
   w.wt = off;    off += dtype == ET_FP16 || split ? align_up(12 * H * H * ea, 256) : 0;
+  w.pair = off;  off += pairs ? align_up(4 * pair_ws_words(rows, H), 256) : 0;
   w.total = off;
   return w;
 }
@@ -300,13 +333,120 @@ struct LayerCall {
   int rows;                           // launches are sized for this many rows
   bool rows_exact = false;            //   ... which is the count itself: no kernel asks the device for it
   char* workspace;
-  bool from_split_ready = false;      // split layers: the split rows of `from` are in the workspace's intermediate already
+  bool from_split_ready = false;      // fp32: the split (pair) rows of `from` are in the workspace's intermediate already
   bool write_out_split = false;       //   ... and those of `out` are to be left there
   hipStream_t stream;
 };
 et_status run_layer(et_handle h, const LayerCall& c);
 
+// The pair rows of a layer's first input, where et_encoder leaves them and the Q/K/V projections find them.
+et::PairRows first_pair_rows(char* layer_base, const LayerWs& ws, int B, int S, int H) {
+  const PairWs p = pair_ws(layer_base + ws.pair, (size_t)B * S, (size_t)H);
+  return {(_Float16*)(layer_base + ws.inter), p.from_exp, p.from_norm};
+}
+
+// fp32 layer on pair rows: launch order of run_layer.
+et_status run_layer_pairs(et_handle h, const LayerCall& c) {
+  const et_layer_weights* w = c.w;
+  static const et_layer_prepared kNoPrep = {nullptr, nullptr, nullptr, nullptr, nullptr, nullptr, nullptr, nullptr, 0, 0};
+  const et_layer_prepared& pp = c.prep ? *c.prep : kNoPrep;
+  const int B = c.B, S = c.S, H = c.heads * c.d, F = 4 * H, rows = c.rows;
+  const LayerWs ws = layer_ws(c.dtype, B, S, c.heads, c.d);
+  const et::DType dt = et::DType::F32;
+  const int32_t* T = c.rows_exact ? nullptr : c.count;
+  hipStream_t st = c.stream;
+  et_status s;
+  char* base = c.workspace;
+  const PairWs pw = pair_ws(base + ws.pair, (size_t)B * S, (size_t)H);
+  float *qkv = (float*)(base + ws.qkv), *attn = (float*)(base + ws.attn);
+  const int32_t* seq_start = c.seq_start ? c.seq_start : (int32_t*)(base + ws.seq);
+
+  // Weights, made anew by every call.  A caller's split copies (et_layer_prepared) hold the same floats: they are what is
+  // read where they are handed over.
+  _Float16* wt = (_Float16*)(base + ws.wt);
+  const size_t HH = (size_t)2 * H * H;
+  et::PairWeightJobs jobs;
+  float* tops = pw.tops;
+  auto weight = [&](const void* plain, const void* split, int k, int n, size_t at, const void* bias, float* stats) {
+    jobs.job[jobs.count++] = {split ? split : plain, split != nullptr, k, n, wt + at * HH, pw.w_exp + at * H, tops, (const float*)bias, stats};
+    tops += et::pair_weight_tops(n, k);
+  };
+  weight(w->attr_kernel_Q, pp.attr_kernel_Q_t, H, H, 0, nullptr, nullptr);
+  weight(w->attr_kernel_K, pp.attr_kernel_K_t, H, H, 1, nullptr, nullptr);
+  weight(w->attr_kernel_V, pp.attr_kernel_V_t, H, H, 2, w->attr_bias_V, pw.v_stats);
+  weight(w->attr_output_kernel, pp.attr_output_kernel_t, H, H, 3, nullptr, nullptr);
+  weight(w->inter_kernel, pp.inter_kernel_t, H, F, 4, w->inter_bias, pw.up_stats);
+  weight(w->output_kernel, pp.output_kernel_t, F, H, 8, nullptr, nullptr);
+  et::launch_pair_weights(jobs, st);
+  if (!c.seq_start) {
+    const et::SeqStartJob seq{c.batch_idx, T, rows, B, (int32_t*)(base + ws.seq)};
+    et::launch_transpose_weights(et::TransposeJobs(), st, &seq);
+  }
+
+  // the inputs, in the room of the intermediate, which nothing needs before they have been read
+  et::PairRows from = first_pair_rows(base, ws, B, S, H), to = from;
+  if (!c.from_split_ready) et::launch_pair_rows((const float*)c.from, nullptr, from, nullptr, nullptr, rows, H, S, T, st);
+  if (c.to != c.from) {
+    to = {from.rows + (size_t)rows * 2 * H, pw.to_exp, pw.to_norm};
+    et::launch_pair_rows((const float*)c.to, nullptr, to, nullptr, nullptr, rows, H, S, T, st);
+  }
+  et::PairProduct p3;
+  p3.groups = 3;
+  p3.A[0] = from; p3.A[1] = to; p3.A[2] = to;
+  const void* qkv_bias[3] = {w->attr_bias_Q, w->attr_bias_K, w->attr_bias_V};
+  for (int i = 0; i < 3; ++i) {
+    p3.B[i] = wt + i * HH;
+    p3.b_exp[i] = pw.w_exp + i * H;
+    p3.bias[i] = (const float*)qkv_bias[i];
+  }
+  et::launch_gemm_pair(p3, qkv, 3 * H, rows, H, H, T, st);
+  if ((s = check_launch(h, "QKV projection")) != ET_OK) return s;
+
+  const float *q = qkv, *k = q + H, *v = k + H;
+  const bool ctx_pairs = et::attention_writes_split(q, k, v, 1, 3 * H, c.d);
+  const uint8_t* cls = c.mask_class;
+  if (!cls && et::mask_class_bytes(dt, B, S, c.d)) {
+    et::launch_mask_class(dt, c.attr_mask, seq_start, c.word_idx, B, S, (uint8_t*)(base + ws.cls), st);
+    cls = (const uint8_t*)(base + ws.cls);
+  }
+  et::PairContext ctx;
+  const et::PairRows ctx_rows{(_Float16*)(base + ws.ctx), pw.ctx_exp, pw.attn_norm};      // (the norms are rewritten by LayerNorm)
+  if (ctx_pairs) ctx = {ctx_rows, to.norm, pw.v_stats, (int)et::pair_weight_stats(H, H)};
+  // (where the attention kernel writes floats only, they take the attention output's place until they are paired)
+  et::launch_attention(dt, q, k, v, 1, 3 * H, c.attr_mask, attn, seq_start, c.word_idx, B, S, c.heads, c.d,
+                       softmax_scaler(c.dtype, c.d), st, false, cls, ctx);
+  if (!ctx_pairs) et::launch_pair_rows(attn, nullptr, ctx_rows, nullptr, nullptr, rows, H, S, T, st);
+  if ((s = check_launch(h, "attention")) != ET_OK) return s;
+
+  auto product = [&](const et::PairRows& a, int w_at, void* C, int n, int k_) {
+    et::PairProduct p;
+    p.A[0] = a;
+    p.B[0] = wt + w_at * HH;
+    p.b_exp[0] = pw.w_exp + w_at * H;
+    et::launch_gemm_pair(p, C, n, rows, n, k_, T, st);
+  };
+  product(ctx_rows, 3, attn, H, H);
+  const et::PairRows attn_rows{(_Float16*)(base + ws.attn_split), pw.attn_exp, pw.attn_norm};
+  et::launch_bias_residual_layernorm(dt, attn, c.from, w->attr_output_bias, w->attr_output_layernorm_gamma,
+                                     w->attr_output_layernorm_beta, rows, H, T, st, et::WarmList(), nullptr, attn_rows);
+  if ((s = check_launch(h, "attention output")) != ET_OK) return s;
+  et::PairProduct up;
+  up.A[0] = attn_rows;
+  up.B[0] = wt + 4 * HH;
+  up.b_exp[0] = pw.w_exp + 4 * H;
+  up.bias[0] = (const float*)w->inter_bias;
+  up.stats = pw.up_stats;
+  up.c_exp = pw.inter_exp;
+  et::launch_gemm_pair(up, base + ws.inter, F, rows, F, H, T, st);
+  if ((s = check_launch(h, "FFN up")) != ET_OK) return s;
+  product({(_Float16*)(base + ws.inter), pw.inter_exp, nullptr}, 8, c.out, H, F);
+  et::launch_bias_residual_layernorm(dt, c.out, attn, w->output_bias, w->output_layernorm_gamma, w->output_layernorm_beta, rows, H,
+                                     T, st, et::WarmList(), nullptr, c.write_out_split ? from : et::PairRows());
+  return check_launch(h, "FFN down");
+}
+
 et_status run_layer(et_handle h, const LayerCall& c) {
+  if (layer_pairs(c.dtype, c.heads * c.d)) return run_layer_pairs(h, c);
   const et_layer_weights* w = c.w;
   const int B = c.B, S = c.S, H = c.heads * c.d, F = 4 * H, rows = c.rows;
   const LayerWs ws = layer_ws(c.dtype, B, S, c.heads, c.d);
@@ -837,15 +977,19 @@ et_status et_encoder(et_handle h, et_dtype dtype, int num_layers, const et_layer
   const bool split = layer_splits(dtype, H);
   et::CompressExtras extras;
   extras.seq_table = seq;
-  // (split layers read their first input from the room of the layer workspace's intermediate)
+  // (such layers read their first input from the room of the layer workspace's intermediate)
   const size_t split_off = layer_ws(dtype, B, S, head_num, size_per_head).inter;
   if (split) extras.split = (uint16_t*)(layer_base + split_off);
+  const bool pairs = layer_pairs(dtype, H);
+  if (pairs) extras.pair = first_pair_rows(layer_base, layer_ws(dtype, B, S, head_num, size_per_head), B, S, H);
   if (b->embeddings) {
     const et_embedding_weights& emb = *b->embeddings;
     et::launch_embed_layernorm(dt, x[0], b->input_ids, b->token_type_ids, batch_idx, word_idx, emb.word_embeddings,
                                emb.vocab_size, emb.token_type_embeddings, emb.type_vocab_size, emb.position_embeddings,
                                emb.max_position_embeddings, emb.layernorm_gamma, emb.layernorm_beta, B * S, H, S, count, st,
                                extras, B);
+  } else if (pairs) {
+    et::launch_pair_rows((const float*)b->from_tensor, (float*)x[0], extras.pair, batch_idx, word_idx, B * S, H, S, count, st, seq, B);
   } else {
     et::launch_compress_rows(b->from_tensor, x[0], batch_idx, word_idx, count, nullptr, nullptr, B, S, (int)row_bytes, st,
                              extras);
@@ -883,7 +1027,7 @@ et_status et_encoder(et_handle h, et_dtype dtype, int num_layers, const et_layer
     c.prep = prepared ? prepared + l : nullptr;
     c.from = c.to = x[cur];
     c.out = x[cur ^ 1];
-    c.from_split_ready = split;
+    c.from_split_ready = split || pairs;
     c.write_out_split = l + 1 < num_layers;
     if ((s = run_layer(h, c)) != ET_OK) return s;
     cur ^= 1;
@@ -1192,6 +1336,60 @@ et_status et_gemm_split(et_handle h, const void* A, const void* Bt, void* C, con
   g.gelu = gelu != 0;
   et::launch_gemm_split(g, C, n, m, n, k, m_dev, (hipStream_t)stream);
   return check_launch(h, "et_gemm_split");
+}
+
+size_t et_pair_weight_stats(int n, int k) { return n < 1 || k < 64 ? 0 : 2 * et::pair_weight_stats(n, k); }
+
+size_t et_pair_weight_workspace_bytes(int n, int k) { return n < 1 || k < 1 ? 0 : et::pair_weight_tops(n, k) * sizeof(float); }
+
+et_status et_pair_rows(et_handle h, const void* src, const et_pair_matrix* dst, int m, int k, const int32_t* m_dev, void* stream) {
+  Entry entry(h);
+  et_status s = entry.status;
+  if (s != ET_OK) return s;
+  ET_REQUIRE(h, src && dst && dst->rows && dst->exp && dst->norm && src != dst->rows, "null or aliased tensor pointer");
+  ET_REQUIRE(h, m >= 0, "bad dimensions");
+  if (!et::pair_rows_supported(k)) return fail(h, ET_UNSUPPORTED, "k must be a multiple of 64 up to 2048");
+  const et::PairRows out{(_Float16*)dst->rows, dst->exp, dst->norm};
+  et::launch_pair_rows((const float*)src, nullptr, out, nullptr, nullptr, m, k, 0, m_dev, (hipStream_t)stream);
+  return check_launch(h, "pair rows");
+}
+
+et_status et_pair_weight(et_handle h, const void* src, void* dst, int32_t* exp, const void* bias, float* stats, int k, int n,
+                         void* workspace, size_t workspace_bytes, void* stream) {
+  Entry entry(h);
+  et_status s = entry.status;
+  if (s != ET_OK) return s;
+  ET_REQUIRE(h, src && dst && exp && src != dst, "null or aliased tensor pointer");
+  ET_REQUIRE(h, stats == nullptr || bias != nullptr, "stats need the bias");
+  ET_REQUIRE(h, workspace != nullptr, "null workspace");
+  if (!et::gemm_pair_supported(n, k)) return fail(h, ET_UNSUPPORTED, "k must be a multiple of 64 and n of 16");
+  if (workspace_bytes < et_pair_weight_workspace_bytes(n, k))
+    return fail(h, ET_WORKSPACE_TOO_SMALL, "et_pair_weight needs et_pair_weight_workspace_bytes(n, k)");
+  et::PairWeightJobs jobs;
+  jobs.job[jobs.count++] = {src, false, k, n, (_Float16*)dst, exp, (float*)workspace, (const float*)bias, stats};
+  et::launch_pair_weights(jobs, (hipStream_t)stream);
+  return check_launch(h, "weight pairs");
+}
+
+et_status et_gemm_pair(et_handle h, const et_pair_matrix* A, const void* Bt, const int32_t* b_exp, const float* b_stats,
+                       const void* bias, void* C, int32_t* c_exp, int m, int n, int k, const int32_t* m_dev, void* stream) {
+  Entry entry(h);
+  et_status s = entry.status;
+  if (s != ET_OK) return s;
+  ET_REQUIRE(h, A && A->rows && A->exp && Bt && b_exp && C, "null tensor pointer");
+  ET_REQUIRE(h, !c_exp || (A->norm && b_stats && bias), "pair rows as the result need the norms, the bias and the weight's stats");
+  ET_REQUIRE(h, m >= 0 && n >= 1 && k >= 1, "bad dimensions");
+  if (!et::gemm_pair_supported(n, k) || (c_exp && n % 32 != 0))
+    return fail(h, ET_UNSUPPORTED, "et_gemm_pair needs k % 64 == 0 and n % 16 == 0 (with c_exp n % 32 == 0)");
+  et::PairProduct p;
+  p.A[0] = {(_Float16*)A->rows, A->exp, A->norm};
+  p.B[0] = (const _Float16*)Bt;
+  p.b_exp[0] = b_exp;
+  p.bias[0] = (const float*)bias;
+  p.stats = b_stats;
+  p.c_exp = c_exp;
+  et::launch_gemm_pair(p, C, n, m, n, k, m_dev, (hipStream_t)stream);
+  return check_launch(h, "et_gemm_pair");
 }
 
 namespace {

@@ -6,6 +6,8 @@
 #include <hip/hip_fp16.h>
 #include <stdint.h>
 
+#include "kernels.hpp"
+
 namespace et {
 
 constexpr int kWave = 64;
@@ -166,6 +168,90 @@ __device__ __forceinline__ void store_split(uint16_t* row, int col, const V& v) 
     else if constexpr (N == 4) *reinterpret_cast<u32x2*>(d) = u32x2{w[0], w[1]};
     else *reinterpret_cast<u32x4*>(d) = u32x4{w[0], w[1], w[2], w[3]};
   }
+}
+
+// ---- floats as pairs of halves -----------------------------------------------------------
+// x = 2^e (h + l) for the values of a row that stay below a bound (gemm_pair.hip).  The exponent that puts values up to `bound`
+// below 2^15, kept where 2^e and 2^-e are ordinary floats; NaN counts as the largest.
+__device__ __forceinline__ int pair_exponent(float bound) {
+  return min(max(__builtin_amdgcn_frexp_expf(fminf(bound, 3.4e38f)) - 15, -112), 113);
+}
+__device__ __forceinline__ float pair_scale(int e) { return __builtin_ldexpf(1.0f, -e); }
+// N consecutive values (N = 1, 2 or 4; col a multiple of N) of a pair row: [k / 32][h, l][32] halves; scale = pair_scale(e)
+template <int N, typename V>
+__device__ __forceinline__ void store_pair(_Float16* row, int col, const V& v, float scale) {
+  typedef _Float16 hvec __attribute__((ext_vector_type(N)));
+  hvec h, l;
+#pragma unroll
+  for (int j = 0; j < N; ++j) {
+    const float y = v[j] * scale;
+    h[j] = f2h(y);
+    l[j] = f2h(y - h2f(h[j]));
+  }
+  _Float16* d = row + (col >> 5) * 64 + (col & 31);
+  *reinterpret_cast<hvec*>(d) = h;
+  *reinterpret_cast<hvec*>(d + 32) = l;
+}
+// Row r of `out` from a wavefront that holds it, lane + 64 i the i-th four values (zero beyond vpr): the exponent from the
+// largest value, and the row's Euclidean norm.  Whoever writes a row writes the same bits.
+template <int ITERS, typename V>
+__device__ __forceinline__ void store_pair_row(const V (&x)[ITERS], int vpr, const PairRows& out, int r, int n) {
+  const int lane = threadIdx.x & (kWave - 1);
+  float top = 0.f;
+#pragma unroll
+  for (int i = 0; i < ITERS; ++i)
+#pragma unroll
+    for (int j = 0; j < 4; ++j) top = fmaxf(top, fabsf(x[i][j]));
+  const int e = pair_exponent(wave_max(top));
+  const float scale = pair_scale(e);
+  float sq = 0.f;
+#pragma unroll
+  for (int i = 0; i < ITERS; ++i)
+#pragma unroll
+    for (int j = 0; j < 4; ++j) {
+      const float y = x[i][j] * scale;
+      sq = __builtin_fmaf(y, y, sq);
+    }
+  sq = wave_sum(sq);
+#pragma unroll
+  for (int i = 0; i < ITERS; ++i) {
+    const int c = lane + i * kWave;
+    if (c < vpr) store_pair<4>(out.rows + (size_t)r * 2 * n, c * 4, x[i], scale);
+  }
+  if (lane == 0) {
+    out.exp[r] = e;
+    out.norm[r] = __builtin_ldexpf(__builtin_sqrtf(sq), e);
+  }
+}
+// The largest first and the largest second word of `n` pairs of non-negative floats, by one wavefront; eight loads in flight.
+__device__ __forceinline__ float2v pair_stats_max(const float* __restrict__ stats, int n) {
+  const int lane = threadIdx.x & (kWave - 1);
+  const float2v* p = reinterpret_cast<const float2v*>(stats);
+  float2v top = {0.f, 0.f};
+  for (int i0 = 0; i0 < n; i0 += 8 * kWave) {
+    float2v v[8];
+#pragma unroll
+    for (int u = 0; u < 8; ++u) v[u] = p[min(i0 + u * kWave + lane, n - 1)];
+#pragma unroll
+    for (int u = 0; u < 8; ++u) top = float2v{fmaxf(top[0], v[u][0]), fmaxf(top[1], v[u][1])};
+  }
+  return float2v{wave_max(top[0]), wave_max(top[1])};
+}
+// The exponent of a sequence's context rows: every value of them is a weighted mean (weights of sum <= 1) of the values
+// x.w + b of its tokens, with |x.w + b| <= |x| |w| + |b|.  One wavefront; `stats`: bounds of |w| and |b| (PairWeightJob).
+__device__ __forceinline__ int context_exponent(const float* __restrict__ norm, int t0, int t1, const float* __restrict__ stats,
+                                                int n_stats) {
+  const int lane = threadIdx.x & (kWave - 1);
+  float top = 0.f;
+  for (int i0 = t0; i0 < t1; i0 += 4 * kWave) {
+    float v[4];
+#pragma unroll
+    for (int u = 0; u < 4; ++u) v[u] = norm[min(i0 + u * kWave + lane, t1 - 1)];
+#pragma unroll
+    for (int u = 0; u < 4; ++u) top = fmaxf(top, v[u]);
+  }
+  const float2v w = pair_stats_max(stats, n_stats);
+  return pair_exponent(wave_max(top) * (w[0] * 1.01f) + w[1]);
 }
 
 // seq_start[b] = first packed row of sequence b (b in [0, batch]; seq_start[batch] = T), written by the thread that

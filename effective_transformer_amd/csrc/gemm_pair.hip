@@ -1,0 +1,693 @@
+// fp32 GEMMs of the encoder layer on the fp16 matrix cores of gfx950 (replace the fp32 cublasGemmEx call sites,
+// reference: tf_op/bert_transformer_op.cu.cc:110-141, 200-240), for hidden sizes of 512 and more in multiples of 64.
+//
+// A float x of a row whose values stay below 2^(e+15) is held as the pair h + l of halves, h = x 2^-e rounded to nearest and
+// l the rest rounded to nearest: 22 to 24 significant bits, down to 2^-40 of the row's bound.  A product of two such floats is
+// h.h + h.l + l.h (l.l is at most 2^-24 of it, the size of a float's own rounding), three products for v_mfma_f32_16x16x32_f16
+// where three bfloat16 pieces take six (gemm_split.hip).  They are summed in chunks of 64 k, smallest first within each 32, and
+// the chunks in float adds: fewer roundings at the size of the whole sum than one chain of matrix instructions has.  Error
+// against float64, normal operands, relative (this / three bfloat16 pieces / fp32 matrix instructions): k = 512 1.22e-7 /
+// 1.27e-7 / 3.8e-7, 768 1.28e-7 / 1.59e-7, 1024 1.34e-7 / 1.87e-7, 3072 1.73e-7 / 3.41e-7 / 9.9e-7, 4096 1.87e-7 / 3.96e-7; all
+// operands positive: 5.0e-8 / 1.21e-7 at k = 512, 1.1e-7 / 3.05e-7 at 3072.  Below k = 512 the three pieces are closer, and
+// layers of smaller hidden sizes keep them.  Infinities and NaNs give NaN.
+//
+// Both operands come as "pair rows": [row][k / 32][h, l][32] halves, one 128-byte line per row and k-step of 32.  Both have
+// an exponent per row, which are applied to the result.  The kernels that produce A write that form themselves: input and LayerNorm know the largest value
+// of the row; attention and the FFN's first product, whose workgroups see parts of a row, take a bound instead, which costs
+// range and no bits: |x.w + b| <= |x| max|w| + max|b| (Euclidean norms), and a row of the context is at most the largest such
+// value of its sequence.  Weights are taken anew by every layer call: pair_weight_top_kernel looks for the largest value of each
+// column, pair_weight_kernel writes the rows (8 + 11.5 us per layer of BERT-base, split rows 15).
+// Bound: at large m the power limit of the matrix cores (20000 rows, k = 768 / n = 2304, 768, 3072 + GELU and k = 3072 / n = 768:
+// 172, 62, 258, 223 us, 1100 .. 1270 TFLOP/s of 16-bit products; split rows 301, 113, 450, 417); below a round of the chip the
+// k loop of one tile (160 rows: 8.6, 7.8, 10, 14.3 us against 15, 10, 16.5, 21).
+#include <algorithm>
+#include <atomic>
+#include <iterator>
+#include <type_traits>
+
+#include "et_device.hpp"
+#include "kernels.hpp"
+
+namespace et {
+
+namespace {
+
+constexpr int kXcds = 8;
+constexpr int kLine = 128;                      // bytes of a row and k-step of 32
+
+struct PairGemmArgs {
+  const _Float16* A[3];
+  const _Float16* B[3];
+  const int32_t* a_exp[3];
+  const int32_t* b_exp[3];
+  const float* bias[3];
+  void* C;
+  const int32_t* rows_dev;
+  // GELU: the bound of a row of C is a_norm[row] * (largest first word of b_stats) + (largest second word)
+  const float* a_norm;
+  const float* b_stats;
+  int32_t* c_exp;
+  int n_stats;
+  int ldc, m_bound, n, k;
+  int tiles_n, tiles_n_all;                     // column tiles per group of B, and of all groups
+  int col_groups;                               // the tile order takes the column tiles in this many groups
+};
+
+#define ET_LDS_PTR(p) ((__attribute__((address_space(3))) void*)(p))
+
+template <int VM>
+__device__ __forceinline__ void wait_vmcnt() {
+  __builtin_amdgcn_s_waitcnt((VM & 15) | (7 << 4) | (15 << 8) | ((VM >> 4) << 14));
+}
+__device__ __forceinline__ void wait_lgkmcnt0() { __builtin_amdgcn_s_waitcnt(15 | (7 << 4) | (0 << 8) | (3 << 14)); }
+__device__ __forceinline__ void barrier_only() { asm volatile("s_barrier" ::: "memory"); }
+
+// WM x WN wavefronts of MI x NJ blocks of 16 x 16, a ring of ST stages of KS k-steps in LDS.
+template <int WM, int WN, int MI, int NJ, int ST, int KS>
+struct PairTile {
+  static constexpr int BM = WM * 16 * MI, BN = WN * 16 * NJ, WAVES = WM * WN, THREADS = WAVES * kWave;
+  static constexpr int A_BYTES = BM * kLine, STEP = (BM + BN) * kLine, SLOT = KS * STEP, SMEM = ST * SLOT;
+  static constexpr int DMA_ALL = STEP / 1024, DMA = (DMA_ALL + WAVES - 1) / WAVES;     // instructions per k-step: all, per wavefront
+  static constexpr bool BIG = KS == 1;
+  static_assert(KS * DMA * (ST - 1) < 64, "the DMA instructions in flight must fit the 6-bit vmcnt");
+  static_assert(SMEM <= 160 * 1024, "LDS");
+};
+
+// Persistent: a workgroup per CU walks the tiles of its XCD's band, one DMA stream across tile boundaries.
+// Per k-step the products run as h.l, l.h, h.h (A's piece first); the chunk's accumulator starts from zero every second k-step
+// and is added to the sum there.  The order does not depend on the tile, so a row has the same bits in every batch.
+//   KS = 1 (large tiles, two wavefronts per SIMD): the operands of a group of MI x NJ MFMAs are read from LDS under the group in
+//   front of it.  At the bar every piece of the k-step has been read: one barrier there frees the slot for the DMA ST k-steps
+//   ahead.
+//   KS = 2 (small tiles): a stage is a chunk; one barrier per stage, the next stage's operands are read into a second register
+//   set under this one's MFMAs.
+// GELU: C = gelu(A.B + bias) as pair rows with their exponents in c_exp; otherwise C is float, + bias if given.
+template <int WM, int WN, int MI, int NJ, int ST, int KS, bool GELU>
+__global__ __launch_bounds__(WM * WN * kWave) void gemm_pair_kernel(PairGemmArgs args) {
+#if defined(__HIP_DEVICE_COMPILE__)   // device-only types in the body; the host pass only needs the stub
+  using Tile = PairTile<WM, WN, MI, NJ, ST, KS>;
+  constexpr int BM = Tile::BM, BN = Tile::BN;
+  extern __shared__ __attribute__((aligned(1024))) unsigned char smem[];
+
+  const int rows = args.rows_dev ? min(*args.rows_dev, args.m_bound) : args.m_bound;
+  const int total = ((rows + BM - 1) / BM) * args.tiles_n_all;      // tiles that hold valid rows
+  // workgroups are dealt round-robin to the XCDs: a contiguous band of tiles for each
+  const int per_xcd = (total + kXcds - 1) / kXcds;
+  const int xcd = blockIdx.x % kXcds, wgs = gridDim.x / kXcds;      // the grid is a multiple of 8
+  const int n_loc = max(0, min(per_xcd, total - xcd * per_xcd));
+  int idx = blockIdx.x / kXcds;
+  if (idx >= n_loc) return;
+  const int N = args.n, K = args.k;
+  const int nst = K / (32 * KS);                                    // stages of a tile
+  const uint32_t row_bytes = (uint32_t)K * 4u;
+
+  const int lane = threadIdx.x & (kWave - 1);
+  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x / kWave);
+  const int wm = wave / WN, wn = wave % WN;
+  const int l16 = lane & 15, g = lane >> 4;
+
+  struct Src {
+    __amdgpu_buffer_rsrc_t a, b;
+    int m0, n0, grp;
+  };
+  auto locate = [&](int i) {
+    Src t;
+    const int tile = xcd * per_xcd + i;
+    const int cpg = args.tiles_n_all / args.col_groups;
+    const int per_group = (total / args.tiles_n_all) * cpg;
+    const int cg = tile / per_group;
+    const int in_group = tile - cg * per_group;
+    const int tm = in_group / cpg;
+    const int tn_all = cg * cpg + (in_group - tm * cpg);
+    t.grp = tn_all / args.tiles_n;
+    t.m0 = tm * BM;
+    t.n0 = (tn_all - t.grp * args.tiles_n) * BN;
+    // rows at or beyond the valid count and columns at or beyond n read as zero
+    t.a = __builtin_amdgcn_make_buffer_rsrc(const_cast<char*>((const char*)args.A[t.grp] + (size_t)t.m0 * row_bytes), 0,
+                                            min(rows - t.m0, BM) * (int)row_bytes, 0x00020000);
+    t.b = __builtin_amdgcn_make_buffer_rsrc(const_cast<char*>((const char*)args.B[t.grp] + (size_t)t.n0 * row_bytes), 0,
+                                            min(N - t.n0, BN) * (int)row_bytes, 0x00020000);
+    return t;
+  };
+
+  // DMA: one instruction fills 1 KB of LDS, eight lines of 128 bytes, their 16-byte chunks XOR-swizzled with row bits 1-3, so
+  // that an operand read (16 rows x one chunk) covers all banks evenly.  LDS row j*16+l of a wave's column group holds column
+  // NJ*l+j of the group: a lane then owns NJ consecutive columns of C.  Where the instructions do not divide evenly, the last
+  // wavefront repeats the last one (same bytes to the same place).
+  uint32_t voff[Tile::DMA];
+#pragma unroll
+  for (int q = 0; q < Tile::DMA; ++q) {
+    const int c = min(wave * Tile::DMA + q, Tile::DMA_ALL - 1) * kWave + lane;
+    int row = c / 8;
+    const uint32_t in_row = (uint32_t)(((c & 7) ^ ((row >> 1) & 7)) * 16);
+    if (row >= BM) {
+      row -= BM;
+      const int in_wave = row % (16 * NJ);
+      row = row - in_wave + (in_wave & 15) * NJ + (in_wave >> 4);
+    }
+    voff[q] = (uint32_t)row * row_bytes + in_row;
+  }
+  // instructions [q0, q1) of this wave's share of k-step `u` of stage `t` of tile `c` (past its end: of the first stages of
+  // tile `n`) into slot `slot`
+  auto issue = [&](int slot, int t, int u, const Src& c, const Src& n, int q0, int q1) {
+    const bool over = t >= nst;
+    const __amdgpu_buffer_rsrc_t ra = over ? n.a : c.a;
+    const __amdgpu_buffer_rsrc_t rb = over ? n.b : c.b;
+    const int koff = ((over ? t - nst : t) * KS + u) * kLine;
+#pragma unroll
+    for (int q = q0; q < q1; ++q) {
+      const int i = min(wave * Tile::DMA + q, Tile::DMA_ALL - 1);
+      unsigned char* dst = smem + slot * Tile::SLOT + u * Tile::STEP + i * 1024;
+      if (i < Tile::A_BYTES / 1024) __builtin_amdgcn_raw_ptr_buffer_load_lds(ra, ET_LDS_PTR(dst), 16, voff[q], koff, 0, 0);
+      else __builtin_amdgcn_raw_ptr_buffer_load_lds(rb, ET_LDS_PTR(dst), 16, voff[q], koff, 0, 0);
+    }
+  };
+  auto issue_stage = [&](int slot, int t, const Src& c, const Src& n) {
+#pragma unroll
+    for (int u = 0; u < KS; ++u) issue(slot, t, u, c, n, 0, Tile::DMA);
+  };
+
+  // chunk g of a piece, swizzled: the pieces h and l are chunks 0-3 and 4-7 of a line
+  const int sw = (g ^ ((l16 >> 1) & 7)) * 16;
+  const int a_rd = (wm * 16 * MI + l16) * kLine, b_rd = Tile::A_BYTES + (wn * 16 * NJ + l16) * kLine;
+  auto read_a = [&](half8 (&v)[MI], int slot, int u, int piece) {
+#pragma unroll
+    for (int i = 0; i < MI; ++i)
+      v[i] = *reinterpret_cast<const half8*>(smem + slot * Tile::SLOT + u * Tile::STEP + a_rd + i * 16 * kLine + (sw ^ (piece * 64)));
+  };
+  auto read_b = [&](half8 (&v)[NJ], int slot, int u, int piece) {
+#pragma unroll
+    for (int j = 0; j < NJ; ++j)
+      v[j] = *reinterpret_cast<const half8*>(smem + slot * Tile::SLOT + u * Tile::STEP + b_rd + j * 16 * kLine + (sw ^ (piece * 64)));
+  };
+
+  float4v sum[MI][NJ], acc[MI][NJ];
+  const float4v zero = {0.f, 0.f, 0.f, 0.f};
+  // one row of blocks; FIRST: the chunk's first product, behind the fold of the chunk before it
+  auto mfma_row = [&](auto FIRSTc, const half8 (&a)[MI], const half8 (&b)[NJ], int i) {
+    constexpr bool FIRST = decltype(FIRSTc)::value;
+#pragma unroll
+    for (int jj = 0; jj < NJ; ++jj) {
+      const int j = (i & 1) ? NJ - 1 - jj : jj;          // only one operand changes from one MFMA to the next
+      if constexpr (FIRST) {
+#pragma unroll
+        for (int r = 0; r < 4; ++r) sum[i][j][r] += acc[i][j][r];
+        acc[i][j] = __builtin_amdgcn_mfma_f32_16x16x32_f16(a[i], b[j], zero, 0, 0, 0);
+      } else {
+        acc[i][j] = __builtin_amdgcn_mfma_f32_16x16x32_f16(a[i], b[j], acc[i][j], 0, 0, 0);
+      }
+    }
+  };
+  auto mfma = [&](auto FIRSTc, const half8 (&a)[MI], const half8 (&b)[NJ]) {
+#pragma unroll
+    for (int i = 0; i < MI; ++i) mfma_row(FIRSTc, a, b, i);
+  };
+  constexpr std::true_type kFirst{};
+  constexpr std::false_type kMore{};
+
+  half8 ah[2][MI], al[MI], bh[NJ], bl[NJ];                       // KS = 1
+  half8 pa[2][2][2][MI], pb[2][2][2][NJ];                        // KS = 2: [register set][k-step][piece]
+
+  Src cur = locate(idx), nxt = cur;
+#pragma unroll
+  for (int s = 0; s < ST; ++s) issue_stage(s, min(s, nst - 1), cur, cur);
+  wait_vmcnt<KS * Tile::DMA*(ST - 1)>();
+  barrier_only();
+  auto read_set = [&](half8 (&a)[2][2][MI], half8 (&b)[2][2][NJ], int slot) {
+#pragma unroll
+    for (int u = 0; u < KS; ++u)
+#pragma unroll
+      for (int piece = 0; piece < 2; ++piece) {
+        read_a(a[u][piece], slot, u, piece);
+        read_b(b[u][piece], slot, u, piece);
+      }
+  };
+  if constexpr (Tile::BIG) {
+    read_a(ah[0], 0, 0, 0);
+    read_b(bl, 0, 0, 1);
+  } else {
+    read_set(pa[0], pb[0], 0);
+  }
+
+  // GELU: what bounds the rows of C, the same for every row
+  float2v bounds = {0.f, 0.f};
+  if constexpr (GELU) bounds = pair_stats_max(args.b_stats, args.n_stats);
+
+  int s = 0;                                     // slot of the current stage
+  bool first_tile = true;
+  while (true) {
+    const int nidx = idx + wgs;
+    const bool has_next = nidx < n_loc;
+    if (has_next) nxt = locate(nidx);            // otherwise the stream re-loads this tile; the data is never used
+#pragma unroll
+    for (int i = 0; i < MI; ++i)
+#pragma unroll
+      for (int j = 0; j < NJ; ++j) sum[i][j] = acc[i][j] = zero;
+    const int col = cur.n0 + wn * 16 * NJ + l16 * NJ;
+    if constexpr (Tile::BIG) {
+      auto step = [&](auto Pc, int t) {
+        constexpr int P = decltype(Pc)::value;
+        read_a(al, s, 0, 1);
+        read_b(bh, s, 0, 0);
+        mfma(std::integral_constant<bool, P == 0>{}, ah[P], bl);
+        __builtin_amdgcn_sched_barrier(0);
+        // this wave's share of k-step t+1 has landed, those behind it may fly; right after a tile boundary all of them
+        // were confirmed before the C stores went out
+        if (first_tile || t >= ST - 1) wait_vmcnt<Tile::DMA*(ST - 2)>();
+        wait_lgkmcnt0();                           // its last reads of slot s are complete
+        barrier_only();
+        const int s1 = s + 1 == ST ? 0 : s + 1;
+        // the DMA instructions go out between the rows of MFMAs: in one piece they would keep the wavefront from issuing
+        constexpr int kPer = (Tile::DMA + 2 * MI - 1) / (2 * MI);
+        read_a(ah[1 - P], s1, 0, 0);
+#pragma unroll
+        for (int i = 0; i < MI; ++i) {
+          mfma_row(kMore, al, bh, i);
+          issue(s, t + ST, 0, cur, nxt, min(i * kPer, Tile::DMA), min((i + 1) * kPer, Tile::DMA));
+          __builtin_amdgcn_sched_barrier(0);
+        }
+        read_b(bl, s1, 0, 1);
+#pragma unroll
+        for (int i = 0; i < MI; ++i) {
+          mfma_row(kMore, ah[P], bh, i);
+          issue(s, t + ST, 0, cur, nxt, min((MI + i) * kPer, Tile::DMA), min((MI + i + 1) * kPer, Tile::DMA));
+          __builtin_amdgcn_sched_barrier(0);
+        }
+        s = s1;
+      };
+      for (int t = 0; t < nst; t += 2) {           // (K is a multiple of 64)
+        step(std::integral_constant<int, 0>{}, t);
+        step(std::integral_constant<int, 1>{}, t + 1);
+      }
+    } else {
+      // one stage on register set P
+      auto stage = [&](auto Pc, int t) {
+        constexpr int P = decltype(Pc)::value;
+        if (first_tile || t >= ST - 1) wait_vmcnt<KS * Tile::DMA*(ST - 2)>();       // as above
+        wait_lgkmcnt0();
+        barrier_only();
+        const int s1 = s + 1 == ST ? 0 : s + 1;
+        read_set(pa[1 - P], pb[1 - P], s1);
+        __builtin_amdgcn_sched_barrier(0);
+        mfma(kFirst, pa[P][0][0], pb[P][0][1]);
+        issue_stage(s, t + ST, cur, nxt);
+        mfma(kMore, pa[P][0][1], pb[P][0][0]);
+        mfma(kMore, pa[P][0][0], pb[P][0][0]);
+        mfma(kMore, pa[P][1][0], pb[P][1][1]);
+        mfma(kMore, pa[P][1][1], pb[P][1][0]);
+        mfma(kMore, pa[P][1][0], pb[P][1][0]);
+        __builtin_amdgcn_sched_barrier(0);
+        s = s1;
+      };
+      int t = 0;
+      for (; t + 1 < nst; t += 2) {
+        stage(std::integral_constant<int, 0>{}, t);
+        stage(std::integral_constant<int, 1>{}, t + 1);
+      }
+      if (t < nst) {                              // an odd number of stages
+        stage(std::integral_constant<int, 0>{}, t);
+        wait_lgkmcnt0();
+#pragma unroll
+        for (int u = 0; u < 2; ++u)
+#pragma unroll
+          for (int piece = 0; piece < 2; ++piece) {
+#pragma unroll
+            for (int i = 0; i < MI; ++i) pa[0][u][piece][i] = pa[1][u][piece][i];
+#pragma unroll
+            for (int j = 0; j < NJ; ++j) pb[0][u][piece][j] = pb[1][u][piece][j];
+          }
+      }
+    }
+    wait_vmcnt<0>();
+
+    if (col < N) {
+      typedef float fvec __attribute__((ext_vector_type(NJ)));
+      fvec bias = {};
+      int ce[NJ];
+#pragma unroll
+      for (int j = 0; j < NJ; ++j) ce[j] = args.b_exp[cur.grp][col + j];
+      if (args.bias[cur.grp] != nullptr) bias = *reinterpret_cast<const fvec*>(args.bias[cur.grp] + col);
+      // (the row arrays reach beyond the last tile: PairRows)
+      typedef int int4v __attribute__((ext_vector_type(4)));
+      int4v re[MI];
+      float4v bound[MI];
+      const int row0 = cur.m0 + wm * 16 * MI + g * 4;
+#pragma unroll
+      for (int i = 0; i < MI; ++i) {
+        re[i] = *reinterpret_cast<const int4v*>(args.a_exp[cur.grp] + row0 + i * 16);
+        if constexpr (GELU) bound[i] = *reinterpret_cast<const float4v*>(args.a_norm + row0 + i * 16);
+      }
+      // the loads are waited for here: left pending on the paths that store nothing, they would have the compiler put a wait
+      // for every outstanding load, the DMA included, in front of the k loop's reuse of their registers
+#pragma unroll
+      for (int j = 0; j < NJ; ++j) {
+        float b = bias[j];
+        asm volatile("" : "+v"(b), "+v"(ce[j]));
+        bias[j] = b;
+      }
+#pragma unroll
+      for (int i = 0; i < MI; ++i) {
+        asm volatile("" : "+v"(re[i]));
+        if constexpr (GELU) asm volatile("" : "+v"(bound[i]));
+      }
+#pragma unroll
+      for (int i = 0; i < MI; ++i)
+#pragma unroll
+        for (int r = 0; r < 4; ++r) {
+          const int row = row0 + i * 16 + r;
+          if (row >= rows) continue;
+          fvec o;
+#pragma unroll
+          for (int j = 0; j < NJ; ++j) o[j] = __builtin_ldexpf(sum[i][j][r] + acc[i][j][r], re[i][r] + ce[j]) + bias[j];
+          if constexpr (GELU) {
+            const int e = pair_exponent(bound[i][r] * (bounds[0] * 1.01f) + bounds[1]);
+#pragma unroll
+            for (int j = 0; j < NJ; ++j) o[j] *= gelu_cdf(o[j], o[j] * o[j] * o[j]);
+            store_pair<NJ>((_Float16*)args.C + (size_t)row * 2 * args.ldc, cur.grp * N + col, o, pair_scale(e));
+            if (col == 0) args.c_exp[row] = e;
+          } else {
+            *reinterpret_cast<fvec*>((float*)args.C + (size_t)row * args.ldc + (size_t)cur.grp * N + col) = o;
+          }
+        }
+    }
+    if (!has_next) break;
+    idx = nidx;
+    cur = nxt;
+    first_tile = false;
+  }
+  wait_vmcnt<0>();                               // no DMA may still target this workgroup's LDS when it ends
+#else
+  (void)args;
+#endif
+}
+
+int device_cu_count() {
+  constexpr int kMaxDevices = 64;
+  static std::atomic<int> cus[kMaxDevices] = {};      // handles on several GPUs may launch from different threads
+  int dev = 0;
+  if (hipGetDevice(&dev) != hipSuccess || dev < 0 || dev >= kMaxDevices) return 256;
+  int n = cus[dev].load(std::memory_order_relaxed);
+  if (n == 0) {
+    hipDeviceProp_t prop;
+    n = hipGetDeviceProperties(&prop, dev) == hipSuccess && prop.multiProcessorCount > 0 ? prop.multiProcessorCount : 256;
+    cus[dev].store(n, std::memory_order_relaxed);
+  }
+  return n;
+}
+
+// Tile of a launch.  Below a round of the chip a launch takes the k loop of one tile, so small problems want small tiles;
+// large ones want the tile with the fewest operand bytes per product.  A launch takes rounds of tiles over the CUs, each
+// as long as its k-steps and a part for filling the ring and storing C.
+enum PairPick { p256x128, p192x128, p128x128, p96x128, p64x128, p64x64, p32x64, p32x32, kPairPicks };
+PairPick pick_pair_tile(int m, int n, int k, int groups) {
+  static constexpr struct { int bm, bn; float step; } kTiles[] = {
+      {256, 128, 0.8f}, {192, 128, 0.66f}, {128, 128, 0.48f}, {96, 128, 0.4f}, {64, 128, 0.3f}, {64, 64, 0.19f}, {32, 64, 0.135f}, {32, 32, 0.085f}};
+  const long cus = device_cu_count();
+  int best = 0;
+  float best_cost = 0.f;
+  for (int i = 0; i < (int)std::size(kTiles); ++i) {
+    const long tiles = (long)((m + kTiles[i].bm - 1) / kTiles[i].bm) * ((n + kTiles[i].bn - 1) / kTiles[i].bn) * groups;
+    const float cost = (float)((tiles + cus - 1) / cus) * (kTiles[i].step * (float)(k / 32) + 3.f);
+    if (i == 0 || cost < best_cost) {
+      best = i;
+      best_cost = cost;
+    }
+  }
+  return (PairPick)best;
+}
+
+template <int WM, int WN, int MI, int NJ, int ST, int KS>
+void launch_tile(PairGemmArgs a, bool gelu, int groups, hipStream_t stream) {
+  using Tile = PairTile<WM, WN, MI, NJ, ST, KS>;
+  a.tiles_n = (a.n + Tile::BN - 1) / Tile::BN;
+  a.tiles_n_all = a.tiles_n * groups;
+  // The workgroups of an XCD advance through k side by side, so what its L2 has to deliver per k-step is the distinct
+  // rows of A and columns of B they touch: about square blocks of tiles are the best.  Wide outputs take their column
+  // tiles in groups of about 1024 columns.
+  a.col_groups = 1;
+  for (int c = 2; c <= a.tiles_n_all; ++c)
+    if (a.tiles_n_all % c == 0 && a.tiles_n_all / c * Tile::BN >= 768) a.col_groups = c;
+  const int tiles = ((a.m_bound + Tile::BM - 1) / Tile::BM) * a.tiles_n_all;
+  // (a stream of fewer stages than the ring holds must not cross into a second tile)
+  const int grid = ((a.k / (32 * KS) < ST ? tiles : std::min(tiles, device_cu_count())) + kXcds - 1) / kXcds * kXcds;
+  auto go = [&](auto kern) {
+    allow_dynamic_lds(reinterpret_cast<const void*>(kern), Tile::SMEM);
+    kern<<<grid, Tile::THREADS, Tile::SMEM, stream>>>(a);
+  };
+  if (gelu) go(gemm_pair_kernel<WM, WN, MI, NJ, ST, KS, true>);
+  else go(gemm_pair_kernel<WM, WN, MI, NJ, ST, KS, false>);
+}
+
+void launch_pick(PairPick pick, const PairGemmArgs& a, bool gelu, int groups, hipStream_t stream) {
+  switch (pick) {
+    case p256x128: return launch_tile<4, 2, 4, 4, 3, 1>(a, gelu, groups, stream);
+    case p192x128: return launch_tile<4, 2, 3, 4, 3, 1>(a, gelu, groups, stream);
+    case p128x128: return launch_tile<2, 4, 4, 2, 4, 1>(a, gelu, groups, stream);
+    case p96x128: return launch_tile<2, 4, 3, 2, 4, 1>(a, gelu, groups, stream);
+    case p64x128: return launch_tile<2, 4, 2, 2, 3, 2>(a, gelu, groups, stream);
+    case p64x64: return launch_tile<4, 2, 1, 2, 4, 2>(a, gelu, groups, stream);
+    case p32x64: return launch_tile<2, 4, 1, 1, 5, 2>(a, gelu, groups, stream);
+    case p32x32: return launch_tile<2, 2, 1, 1, 6, 2>(a, gelu, groups, stream);
+    default: return;
+  }
+}
+
+// Rows into pair rows: one wavefront per row, which stays in registers (n <= 256 ITERS, a multiple of 4).  With indices the
+// source is the padded tensor, and the packed rows are written as well; then the first workgroup sorts the batch's table.
+template <int ITERS>
+__global__ __launch_bounds__(256) void pair_rows_kernel(const float* __restrict__ src, float* __restrict__ packed, PairRows out,
+                                                        const int32_t* __restrict__ batch_idx,
+                                                        const int32_t* __restrict__ word_idx, int m, int n, int seq_len,
+                                                        const int32_t* __restrict__ rows_dev, int32_t* __restrict__ seq_table,
+                                                        int batch) {
+  const int first = seq_table ? 1 : 0;
+  if (first && blockIdx.x == 0) {
+    sort_sequences<256>(seq_table, batch, seq_table + batch + 1);
+    return;
+  }
+  const int rows = rows_dev ? min(*rows_dev, m) : m;
+  const int lane = threadIdx.x & (kWave - 1);
+  const int vpr = n / 4;
+  for (int r = ((int)blockIdx.x - first) * 4 + threadIdx.x / kWave; r < rows; r += ((int)gridDim.x - first) * 4) {
+    const size_t from = batch_idx ? (size_t)batch_idx[r] * seq_len + word_idx[r] : (size_t)r;
+    const float4v* s = reinterpret_cast<const float4v*>(src + from * n);
+    float4v x[ITERS];
+#pragma unroll
+    for (int i = 0; i < ITERS; ++i) {
+      const int c = lane + i * kWave;
+      x[i] = float4v{0.f, 0.f, 0.f, 0.f};
+      if (c < vpr) {
+        x[i] = s[c];
+        if (packed) reinterpret_cast<float4v*>(packed + (size_t)r * n)[c] = x[i];
+      }
+    }
+    store_pair_row<ITERS>(x, vpr, out, r, n);
+  }
+}
+
+// Weights into n pair rows in two launches, whose loads are whole lines (one launch of workgroups that hold all k of 16 columns
+// took 35 .. 45 us at H = 768; exponents that go by chunks of 64 k and are applied where a chunk is added need one launch, and
+// cost the products 3 to 20 %).  First the largest value of each column in blocks of 256 k, as [k / 256][n].
+struct PairWeightArgs {
+  PairWeightJobs jobs;
+  int tile_begin[PairWeightJobs::kMax + 1];
+};
+constexpr int kTopRows = 256;
+__global__ __launch_bounds__(256) void pair_weight_top_kernel(PairWeightArgs args) {
+  __shared__ float part[16][64];
+  int job = 0;
+  while (job + 1 < args.jobs.count && (int)blockIdx.x >= args.tile_begin[job + 1]) ++job;
+  const PairWeightJob& jb = args.jobs.job[job];
+  const int K = jb.k, N = jb.n, tiles_n = (N + 63) / 64;
+  const int t = blockIdx.x - args.tile_begin[job];
+  const int block = t / tiles_n, k0 = block * kTopRows, n0 = (t - block * tiles_n) * 64;
+  if (jb.src_split) {                            // rows of three bfloat16 pieces: four lanes per row, 64 k each
+    const int r = threadIdx.x >> 2, kk = k0 + (threadIdx.x & 3) * 64;
+    float top = 0.f;
+    if (n0 + r < N && kk < K) {
+      const __bf16* p = (const __bf16*)jb.src + (size_t)(n0 + r) * K * 3 + (kk >> 5) * 96;
+      for (int i = 0; i < 64; ++i) {
+        const __bf16* q = p + (i >> 5) * 96 + (i & 31);
+        top = fmaxf(top, fabsf(((float)q[0] + (float)q[32]) + (float)q[64]));
+      }
+    }
+    top = fmaxf(top, dpp_f32<kDppQuadXor1>(top, top));
+    top = fmaxf(top, dpp_f32<kDppQuadXor2>(top, top));
+    if (n0 + r < N && (threadIdx.x & 3) == 0) jb.top[(size_t)block * N + n0 + r] = top;
+    return;
+  }
+  const float* __restrict__ src = (const float*)jb.src;
+  const int r = threadIdx.x >> 4, c = (threadIdx.x & 15) * 4;
+  float4v v[kTopRows / 16];
+#pragma unroll
+  for (int u = 0; u < kTopRows / 16; ++u) {
+    v[u] = float4v{0.f, 0.f, 0.f, 0.f};
+    if (k0 + u * 16 + r < K && n0 + c < N) v[u] = *reinterpret_cast<const float4v*>(src + (size_t)(k0 + u * 16 + r) * N + n0 + c);
+  }
+#pragma unroll
+  for (int j = 0; j < 4; ++j) {
+    float top = 0.f;
+#pragma unroll
+    for (int u = 0; u < kTopRows / 16; ++u) top = fmaxf(top, fabsf(v[u][j]));
+    part[r][c + j] = top;
+  }
+  __syncthreads();
+  if (threadIdx.x < 64 && n0 + (int)threadIdx.x < N) {
+    float top = part[0][threadIdx.x];
+#pragma unroll
+    for (int i = 1; i < 16; ++i) top = fmaxf(top, part[i][threadIdx.x]);
+    jb.top[(size_t)block * N + n0 + threadIdx.x] = top;
+  }
+}
+
+// Then 64 x 64 tiles through LDS.
+__global__ __launch_bounds__(256) void pair_weight_kernel(PairWeightArgs args) {
+  __shared__ float tile[64][65];
+  __shared__ float part[2][4];
+  __shared__ int exps[64];
+  int job = 0;
+  while (job + 1 < args.jobs.count && (int)blockIdx.x >= args.tile_begin[job + 1]) ++job;
+  const PairWeightJob& jb = args.jobs.job[job];
+  const int K = jb.k, N = jb.n, tiles_n = (N + 63) / 64;
+  const int t = blockIdx.x - args.tile_begin[job];
+  const int chunk = t / tiles_n, k0 = chunk * 64, n0 = (t - chunk * tiles_n) * 64;
+  if (threadIdx.x < 64 && n0 + (int)threadIdx.x < N) {
+    float top = 0.f;
+    for (int b = 0; b < (K + kTopRows - 1) / kTopRows; ++b) top = fmaxf(top, jb.top[(size_t)b * N + n0 + threadIdx.x]);
+    exps[threadIdx.x] = pair_exponent(top);
+    if (chunk == 0) jb.exp[n0 + threadIdx.x] = exps[threadIdx.x];
+  }
+  if (jb.src_split) {                            // rows of three bfloat16 pieces, whose sum is the float
+    typedef __bf16 bf16x8 __attribute__((ext_vector_type(8)));
+#pragma unroll
+    for (int u = 0; u < 2; ++u) {
+      const int i = threadIdx.x + u * 256, r = i >> 3, c = (i & 7) * 8;      // row n0+r, k0+c ..
+      if (n0 + r >= N) continue;
+      const __bf16* p = (const __bf16*)jb.src + (size_t)(n0 + r) * K * 3 + ((k0 + c) >> 5) * 96 + (c & 31);
+      const bf16x8 h = *reinterpret_cast<const bf16x8*>(p), m = *reinterpret_cast<const bf16x8*>(p + 32),
+                   l = *reinterpret_cast<const bf16x8*>(p + 64);
+#pragma unroll
+      for (int j = 0; j < 8; ++j) tile[r][c + j] = ((float)h[j] + (float)m[j]) + (float)l[j];
+    }
+  } else {
+    const float* __restrict__ src = (const float*)jb.src;
+#pragma unroll
+    for (int u = 0; u < 4; ++u) {
+      const int i = threadIdx.x + u * 256, r = i >> 4, c = (i & 15) * 4;     // source row k0+r, columns n0+c ..
+      float4v v = {};
+      if (n0 + c < N) v = *reinterpret_cast<const float4v*>(src + (size_t)(k0 + r) * N + n0 + c);
+#pragma unroll
+      for (int j = 0; j < 4; ++j) tile[c + j][r] = v[j];
+    }
+  }
+  __syncthreads();
+  float norm = 0.f, bias = 0.f;
+#pragma unroll
+  for (int u = 0; u < 2; ++u) {
+    const int i = threadIdx.x + u * 256, r = i >> 3, c = (i & 7) * 8;        // row n0+r of the result, k0+c ..
+    if (n0 + r >= N) continue;                   // (whole groups of eight lanes)
+    const int e = exps[r];
+    const float by = pair_scale(e);
+    float sq = 0.f;
+    half8 h, l;
+#pragma unroll
+    for (int j = 0; j < 8; ++j) {
+      const float y = tile[r][c + j] * by;
+      h[j] = f2h(y);
+      l[j] = f2h(y - h2f(h[j]));
+      sq = __builtin_fmaf(y, y, sq);
+    }
+    _Float16* d = jb.dst + (size_t)(n0 + r) * 2 * K + ((k0 + c) >> 5) * 64 + (c & 31);
+    *reinterpret_cast<half8*>(d) = h;
+    *reinterpret_cast<half8*>(d + 32) = l;
+    if (jb.stats != nullptr) {
+      sq += dpp_f32<kDppQuadXor1>(0.f, sq);
+      sq += dpp_f32<kDppQuadXor2>(0.f, sq);
+      sq += dpp_f32<kDppRowHalfMirror>(0.f, sq);
+      norm = fmaxf(norm, __builtin_ldexpf(__builtin_sqrtf(sq), e));
+      if (chunk == 0) bias = fmaxf(bias, fabsf(jb.bias[n0 + r]));
+    }
+  }
+  if (jb.stats == nullptr) return;
+  // |column| <= sqrt(chunks) times the largest part of a column in one chunk
+  norm = wave_max(norm) * __builtin_sqrtf((float)(K / 64));
+  bias = wave_max(bias);
+  if ((threadIdx.x & (kWave - 1)) == 0) {
+    part[0][threadIdx.x / kWave] = norm;
+    part[1][threadIdx.x / kWave] = bias;
+  }
+  __syncthreads();
+  if (threadIdx.x < 2)
+    jb.stats[2 * t + threadIdx.x] = fmaxf(fmaxf(part[threadIdx.x][0], part[threadIdx.x][1]), fmaxf(part[threadIdx.x][2], part[threadIdx.x][3]));
+}
+
+}  // namespace
+
+bool gemm_pair_supported(int n, int k) {
+  return k % 64 == 0 && k >= 64 && n % 16 == 0 && (uint64_t)k * 4u * 256u < 0x80000000ull;
+}
+
+void launch_pair_rows(const float* src, float* packed, const PairRows& out, const int32_t* batch_idx, const int32_t* word_idx,
+                      int m, int n, int seq_len, const int32_t* rows_dev, hipStream_t stream, int32_t* seq_table, int batch) {
+  if (m <= 0) return;
+  const int grid = std::min((m + 3) / 4, 2048) + (seq_table ? 1 : 0);
+  auto go = [&](auto kern) {
+    kern<<<grid, 256, 0, stream>>>(src, packed, out, batch_idx, word_idx, m, n, seq_len, rows_dev, seq_table, batch);
+  };
+  switch ((n / 4 + kWave - 1) / kWave) {
+    case 1: return go(pair_rows_kernel<1>);
+    case 2: return go(pair_rows_kernel<2>);
+    case 3: return go(pair_rows_kernel<3>);
+    case 4: return go(pair_rows_kernel<4>);
+    case 5: case 6: return go(pair_rows_kernel<6>);
+    case 7: case 8: return go(pair_rows_kernel<8>);
+    default: return;                             // (pair_rows_supported)
+  }
+}
+
+bool pair_rows_supported(int n) { return n % 64 == 0 && n >= 64 && n <= 2048; }
+
+void launch_pair_weights(const PairWeightJobs& jobs, hipStream_t stream) {
+  if (jobs.count == 0) return;
+  PairWeightArgs a;
+  a.jobs = jobs;
+  auto grid = [&](int rows) {
+    int total = 0;
+    for (int j = 0; j < jobs.count; ++j) {
+      a.tile_begin[j] = total;
+      total += ((jobs.job[j].k + rows - 1) / rows) * ((jobs.job[j].n + 63) / 64);
+    }
+    for (int j = jobs.count; j <= PairWeightJobs::kMax; ++j) a.tile_begin[j] = total;
+    return total;
+  };
+  const int tops = grid(kTopRows);
+  pair_weight_top_kernel<<<tops, 256, 0, stream>>>(a);
+  const int tiles = grid(64);
+  pair_weight_kernel<<<tiles, 256, 0, stream>>>(a);
+}
+
+void launch_gemm_pair(const PairProduct& p, void* C, int ldc, int m_bound, int n, int k, const int32_t* rows_dev,
+                      hipStream_t stream) {
+  if (m_bound <= 0) return;
+  PairGemmArgs a = {};
+  for (int i = 0; i < p.groups; ++i) {
+    a.A[i] = p.A[i].rows;
+    a.a_exp[i] = p.A[i].exp;
+    a.B[i] = p.B[i];
+    a.b_exp[i] = p.b_exp[i];
+    a.bias[i] = p.bias[i];
+  }
+  a.a_norm = p.A[0].norm;
+  a.b_stats = p.stats;
+  a.n_stats = (int)pair_weight_stats(n, k);
+  a.c_exp = p.c_exp;
+  a.C = C;
+  a.rows_dev = rows_dev;
+  a.ldc = ldc;
+  a.m_bound = m_bound;
+  a.n = n;
+  a.k = k;
+  launch_pick(pick_pair_tile(m_bound, n, k, p.groups), a, p.c_exp != nullptr, p.groups, stream);
+}
+
+}  // namespace et

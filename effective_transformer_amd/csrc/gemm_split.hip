@@ -1,5 +1,6 @@
 // fp32 GEMMs of the encoder layer on the 16-bit matrix cores of gfx950 (replace the fp32 cublasGemmEx call sites,
-// reference: tf_op/bert_transformer_op.cu.cc:110-141, 200-240).
+// reference: tf_op/bert_transformer_op.cu.cc:110-141, 200-240), for the hidden sizes gemm_pair.hip does not take: multiples of
+// 32 below 512, odd multiples of 32, and rows of more than 2048 values.
 //
 // A float is the exact sum of three bfloat16 numbers h + m + l, each the rest of the ones before it rounded to nearest
 // (8 significand bits and a sign apiece cover the 24 bits, in the float's own exponent range).  A product of two such

@@ -18,6 +18,23 @@ void allow_dynamic_lds(const void* kernel, int bytes);
 // The error of a failed allow_dynamic_lds on this thread since the last call (hipSuccess if none); clears it.
 hipError_t take_attribute_error();
 
+// A matrix of pair rows (gemm_pair.hip): n values per row as [n / 32][h, l][32] halves, the exponent of each row, and the
+// row's Euclidean norm, from which what is computed of it is bounded.  Row arrays have room for 256 rows
+// more than the matrix (a tile reads them whole).
+struct PairRows {
+  _Float16* rows = nullptr;
+  int32_t* exp = nullptr;
+  float* norm = nullptr;             // (not of matrices that nothing is bounded by)
+};
+// What attention needs to write its rows as pair rows: the matrix, the norms of the rows that K and V were made of, and what
+// bounds the column norms and the bias of V (n_stats pairs, see PairWeightJob).
+struct PairContext {
+  PairRows out;
+  const float* norm = nullptr;
+  const float* stats = nullptr;
+  int n_stats = 0;
+};
+
 // ---- input_output.hip --------------------------------------------------------------------
 // Number of int32 words of scratch the scan needs for `length` elements.
 size_t scan_scratch_words(int length);
@@ -30,6 +47,7 @@ struct ScanExtras {
 struct CompressExtras {
   int32_t* seq_table = nullptr;      // the table whose first half the scan wrote: its second half is filled in
   uint16_t* split = nullptr;         // float rows of a multiple of 32 values: the packed rows once more as split rows
+  PairRows pair;                     // ... or as pair rows (pair_rows_supported)
 };
 // Exclusive prefix sum of `in`; optionally (seq_len > 0) also writes batch_idx / word_idx for
 // every element > 0 and the valid-token count.  prefix_out may be null.
@@ -81,8 +99,9 @@ struct WarmList {
 void launch_bias_residual_layernorm(DType t, void* out, const void* input, const void* bias,
                                     const void* gamma, const void* beta, int m, int n,
                                     const int32_t* rows_dev, hipStream_t stream, const WarmList& warm = WarmList(),
-                                    uint16_t* split = nullptr);
-// split (fp32, rows in registers, n % 32 == 0): the output rows once more as split rows (see gemm_split.hip)
+                                    uint16_t* split = nullptr, const PairRows& pair = PairRows());
+// split (fp32, rows in registers, n % 32 == 0): the output rows once more as split rows (see gemm_split.hip); pair: as pair
+// rows (pair_rows_supported)
 
 // out[t,:] = LayerNorm(word[ids[p]] + type[type_ids[p]] + pos[word_idx[t]]) * gamma + beta for packed row t at padded
 // position p = batch_idx[t]*seq_len + word_idx[t]; eps 1e-12.  type_ids/type_table and pos_table may be null.
@@ -108,14 +127,15 @@ bool attention_supported(DType t, int seq_len, int d);
 void launch_attention(DType t, const void* q, const void* k, const void* v, int layout, int packed_ld,
                       const void* attr_mask, void* dst, const int32_t* seq_start, const int32_t* word_idx,
                       int batch, int seq_len, int heads, int d, float scaler, hipStream_t stream,
-                      bool split_out = false, const uint8_t* mask_class = nullptr);
+                      bool split_out = false, const uint8_t* mask_class = nullptr, const PairContext& pair = PairContext());
 // Classes of the mask rows (one byte per 16 query positions of a sequence) for the kernel that makes use of them; the same
 // array serves every layer of a batch.  0 bytes: the kernel of this shape has no use for them.
 size_t mask_class_bytes(DType t, int batch, int seq_len, int d);
 size_t mask_class_bytes_max(int batch);                // at any length
 void launch_mask_class(DType t, const void* attr_mask, const int32_t* seq_start, const int32_t* word_idx, int batch, int seq_len,
                        uint8_t* cls, hipStream_t stream);
-// split_out (fp32): dst gets split rows (see gemm_split.hip) instead of float rows; only where this says so
+// split_out (fp32): dst gets split rows (see gemm_split.hip) instead of float rows, with pair.out.rows that one gets pair rows;
+// only where this says so
 bool attention_writes_split(const void* q, const void* k, const void* v, int layout, int packed_ld, int d);
 
 // ---- gemm.hip ----------------------------------------------------------------------------
@@ -185,6 +205,46 @@ void launch_split_rows(const float* src, uint16_t* dst, int m, int k, const int3
 void launch_split_weights(const TransposeJobs& jobs, hipStream_t stream);
 void launch_gemm_split(const GemmGroups& g, void* C, int ldc, int m_bound, int n, int k, const int32_t* rows_dev,
                        hipStream_t stream);
+
+// ---- gemm_pair.hip: fp32 products on the fp16 matrix cores, half the work of split rows ---------------------------
+bool gemm_pair_supported(int n, int k);
+bool pair_rows_supported(int n);
+// float rows -> pair rows.  With batch_idx / word_idx: gathered from the padded tensor, the float rows go to `packed` too;
+// seq_table: its second half is filled in on the way.
+void launch_pair_rows(const float* src, float* packed, const PairRows& out, const int32_t* batch_idx, const int32_t* word_idx,
+                      int m, int n, int seq_len, const int32_t* rows_dev, hipStream_t stream, int32_t* seq_table = nullptr,
+                      int batch = 0);
+struct PairWeightJob {
+  const void* src;                   // float [k][n], or (src_split) its n split rows
+  bool src_split;
+  int k, n;
+  _Float16* dst;                     // n pair rows
+  int32_t* exp;                      // n
+  float* top;                        // scratch: pair_weight_tops(n, k) words
+  const float* bias;                 // with stats: n
+  float* stats;                      // may be null; pair_weight_stats pairs: a bound of columns' norms, and of |bias|
+};
+inline size_t pair_weight_tops(int n, int k) { return (size_t)((k + 255) / 256) * n; }
+inline size_t pair_weight_stats(int n, int k) { return (size_t)(k / 64) * ((n + 63) / 64); }
+struct PairWeightJobs {
+  static constexpr int kMax = 6;
+  PairWeightJob job[kMax] = {};
+  int count = 0;
+};
+void launch_pair_weights(const PairWeightJobs& jobs, hipStream_t stream);
+// C[:, g n : (g + 1) n] = A[g].B[g] + bias[g] (bias may be null), float with leading dimension ldc; with c_exp
+// C = gelu(A.B + bias) as pair rows of ldc values, from A[0].norm and the weights' `stats`.
+struct PairProduct {
+  int groups = 1;
+  PairRows A[3];
+  const _Float16* B[3] = {};
+  const int32_t* b_exp[3] = {};
+  const float* bias[3] = {};
+  const float* stats = nullptr;
+  int32_t* c_exp = nullptr;
+};
+void launch_gemm_pair(const PairProduct& p, void* C, int ldc, int m_bound, int n, int k, const int32_t* rows_dev,
+                      hipStream_t stream);
 
 // ---- generic.hip: element-wise kernels for the shapes the tuned kernels do not take ------------------------------
 // (rows or head rows that are no whole number of 16-byte pieces, GEMM k / n the MFMA tiles cannot take); the launchers

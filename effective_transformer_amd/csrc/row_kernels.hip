@@ -89,7 +89,7 @@ template <typename T, int VEC, int ITERS>
 __global__ __launch_bounds__(kLnThreads) void bias_residual_layernorm_kernel(
     T* __restrict__ out, const T* __restrict__ input, const T* __restrict__ bias, const T* __restrict__ gamma,
     const T* __restrict__ beta, int m, int n, const int32_t* __restrict__ rows_dev, WarmList warm,
-    uint16_t* __restrict__ split) {
+    uint16_t* __restrict__ split, PairRows pair) {
   using V = typename RowVec<T, VEC>::type;
   const int rows = rows_dev ? min(*rows_dev, m) : m;
   const int lane = threadIdx.x & (kWave - 1);
@@ -161,6 +161,22 @@ __global__ __launch_bounds__(kLnThreads) void bias_residual_layernorm_kernel(
       }
     }
     const float rstd = __builtin_amdgcn_rsqf(wave_sum(sq) * inv_n + 1e-6f);
+    if constexpr (sizeof(T) == 4 && VEC == 4)
+      if (pair.rows) {
+        V y[ITERS];
+#pragma unroll
+        for (int i = 0; i < ITERS; ++i) {
+          const int c = lane + i * kWave;
+          y[i] = V{0.f, 0.f, 0.f, 0.f};
+          if (c < vpr) {
+#pragma unroll
+            for (int j = 0; j < VEC; ++j) y[i][j] = ((x[i][j] - mean) * rstd) * g[i][j] + be[i][j];
+            orow[c] = y[i];
+          }
+        }
+        store_pair_row<ITERS>(y, vpr, pair, r, n);
+        continue;
+      }
 #pragma unroll
     for (int i = 0; i < ITERS; ++i) {
       const int c = lane + i * kWave;
@@ -260,6 +276,22 @@ __global__ __launch_bounds__(kLnThreads) void embed_layernorm_kernel(
     }
     const float rstd = __builtin_amdgcn_rsqf(wave_sum(sq) * inv_n + 1e-12f);
     V* orow = reinterpret_cast<V*>(out + (size_t)r * n);
+    if constexpr (sizeof(T) == 4 && VEC == 4)
+      if (extras.pair.rows) {
+        V y[ITERS];
+#pragma unroll
+        for (int i = 0; i < ITERS; ++i) {
+          const int c = lane + i * kWave;
+          y[i] = V{0.f, 0.f, 0.f, 0.f};
+          if (c < vpr) {
+#pragma unroll
+            for (int j = 0; j < VEC; ++j) y[i][j] = ((x[i][j] - mean) * rstd) * g[i][j] + be[i][j];
+            orow[c] = y[i];
+          }
+        }
+        store_pair_row<ITERS>(y, vpr, extras.pair, r, n);
+        continue;
+      }
 #pragma unroll
     for (int i = 0; i < ITERS; ++i) {
       const int c = lane + i * kWave;
@@ -292,11 +324,12 @@ bool ln_pick(int n, int& vec, int& iters) {
 
 template <typename T, int VEC>
 void ln_launch_iters(int iters, int grid, hipStream_t stream, T* out, const T* input, const T* bias, const T* gamma,
-                     const T* beta, int m, int n, const int32_t* rows_dev, const WarmList& warm, uint16_t* split) {
+                     const T* beta, int m, int n, const int32_t* rows_dev, const WarmList& warm, uint16_t* split,
+                     const PairRows& pair) {
 #define ET_LN_CASE(I)                                                                                          \
   case I:                                                                                                      \
     bias_residual_layernorm_kernel<T, VEC, I><<<grid, kLnThreads, 0, stream>>>(out, input, bias, gamma, beta, m, n, \
-                                                                               rows_dev, warm, split);         \
+                                                                               rows_dev, warm, split, pair);   \
     break;
   switch (iters) {
     ET_LN_CASE(1)
@@ -313,7 +346,7 @@ void ln_launch_iters(int iters, int grid, hipStream_t stream, T* out, const T* i
 
 template <typename T>
 void ln_launch(void* out, const void* input, const void* bias, const void* gamma, const void* beta, int m, int n,
-               const int32_t* rows_dev, hipStream_t stream, const WarmList& warm, uint16_t* split) {
+               const int32_t* rows_dev, hipStream_t stream, const WarmList& warm, uint16_t* split, const PairRows& pair) {
   int vec = 0, iters = 0;
   if (!ln_pick<T>(n, vec, iters)) return;
   // enough wavefronts to fill 256 CUs several times over; rows beyond that are looped.  A list of lines to request brings
@@ -324,11 +357,11 @@ void ln_launch(void* out, const void* input, const void* bias, const void* gamma
   const T *i = (const T*)input, *b = (const T*)bias, *g = (const T*)gamma, *be = (const T*)beta;
   constexpr int MV = 16 / (int)sizeof(T);
   if (vec == MV)
-    ln_launch_iters<T, MV>(iters, grid, stream, o, i, b, g, be, m, n, rows_dev, warm, split);
+    ln_launch_iters<T, MV>(iters, grid, stream, o, i, b, g, be, m, n, rows_dev, warm, split, pair);
   else if (vec == MV / 2)
-    ln_launch_iters<T, MV / 2>(iters, grid, stream, o, i, b, g, be, m, n, rows_dev, warm, split);
+    ln_launch_iters<T, MV / 2>(iters, grid, stream, o, i, b, g, be, m, n, rows_dev, warm, split, pair);
   else
-    ln_launch_iters<T, MV / 4>(iters, grid, stream, o, i, b, g, be, m, n, rows_dev, warm, split);
+    ln_launch_iters<T, MV / 4>(iters, grid, stream, o, i, b, g, be, m, n, rows_dev, warm, split, pair);
 }
 
 struct EmbedArgs {
@@ -436,15 +469,15 @@ void WarmList::add(const void* region, size_t bytes) {
 
 void launch_bias_residual_layernorm(DType t, void* out, const void* input, const void* bias, const void* gamma,
                                     const void* beta, int m, int n, const int32_t* rows_dev, hipStream_t stream,
-                                    const WarmList& warm, uint16_t* split) {
+                                    const WarmList& warm, uint16_t* split, const PairRows& pair) {
   if (!layernorm_row_in_registers(t, n)) {      // odd or very long rows: three passes over memory
     launch_layernorm_generic(t, out, input, bias, gamma, beta, m, n, rows_dev, 1e-6f, stream);
     return;
   }
   if (t == DType::F32)
-    ln_launch<float>(out, input, bias, gamma, beta, m, n, rows_dev, stream, warm, split);
+    ln_launch<float>(out, input, bias, gamma, beta, m, n, rows_dev, stream, warm, split, pair);
   else
-    ln_launch<_Float16>(out, input, bias, gamma, beta, m, n, rows_dev, stream, warm, nullptr);
+    ln_launch<_Float16>(out, input, bias, gamma, beta, m, n, rows_dev, stream, warm, nullptr, PairRows());
 }
 
 }  // namespace et

@@ -157,3 +157,49 @@ def gemm_split(a, bt, bias=None, m_dev: Optional[torch.Tensor] = None, out: Opti
             torch.zeros(rows, n, dtype=torch.float32, device=a.device)
     _call("et_gemm_split", a.device, _p(a), _p(bt), _p(out), _p(bias), 1 if gelu else 0, rows, n, k, _p(m_dev), _stream())
     return out
+
+
+class PairRows:
+    """A matrix of pair rows (layout: et_gemm_pair in et.h): rows [m, 2 k] halves, exp int32 and norm float32 of every row."""
+
+    def __init__(self, m: int, k: int, device):
+        self.rows = torch.zeros(m, 2 * k, dtype=torch.float16, device=device)
+        self.exp = torch.zeros(m + 511, dtype=torch.int32, device=device)
+        self.norm = torch.zeros(m + 511, dtype=torch.float32, device=device)
+
+    def c_struct(self):
+        return _lib.PairMatrix(self.rows.data_ptr(), self.exp.data_ptr(), self.norm.data_ptr())
+
+    def values(self) -> torch.Tensor:
+        """The float64 matrix it stands for."""
+        m = self.rows.shape[0]
+        return torch.ldexp(self.rows.double().reshape(m, -1, 2, 32).sum(2).reshape(m, -1), self.exp[:m, None])
+
+
+def pair_rows(a, m_dev: Optional[torch.Tensor] = None, out: Optional[PairRows] = None) -> PairRows:
+    """fp32 [m, k] -> pair rows."""
+    m, k = a.shape
+    out = PairRows(m, k, a.device) if out is None else out
+    _call("et_pair_rows", a.device, _p(a), C.byref(out.c_struct()), m, k, _p(m_dev), _stream())
+    return out
+
+
+def pair_weight(w, bias=None):
+    """fp32 [k, n] -> (n pair rows, stats for gemm_pair(gelu=True) if a bias is given)."""
+    k, n = w.shape
+    lib = _lib.load()
+    out = PairRows(n, k, w.device)
+    ws = _workspace(w.device, "pair_weight", lib.et_pair_weight_workspace_bytes(n, k))
+    stats = None if bias is None else torch.zeros(lib.et_pair_weight_stats(n, k), dtype=torch.float32, device=w.device)
+    _call("et_pair_weight", w.device, _p(w), _p(out.rows), _p(out.exp), _p(bias), _p(stats), k, n, _p(ws), ws.numel(), _stream())
+    return out, stats
+
+
+def gemm_pair(a: PairRows, b: PairRows, bias=None, stats=None, m_dev: Optional[torch.Tensor] = None, out=None, gelu: bool = False):
+    """Pair rows a [m, k], b [n, k] -> fp32 [m, n] (+ bias), or with gelu the pair rows of gelu(product + bias)."""
+    m, n, k = a.rows.shape[0], b.rows.shape[0], a.rows.shape[1] // 2
+    if out is None:
+        out = PairRows(m, n, a.rows.device) if gelu else torch.zeros(m, n, dtype=torch.float32, device=a.rows.device)
+    _call("et_gemm_pair", a.rows.device, C.byref(a.c_struct()), _p(b.rows), _p(b.exp), _p(stats), _p(bias),
+          _p(out.rows if gelu else out), _p(out.exp) if gelu else None, m, n, k, _p(m_dev), _stream())
+    return out

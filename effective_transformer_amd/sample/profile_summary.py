@@ -22,9 +22,9 @@ import sys
 from .workloads import WORKLOADS
 
 ROLES = ["QKV", "attention", "attention out", "LayerNorm 1", "FFN up + GELU", "FFN down", "LayerNorm 2"]
-SIDE = ("scan_index", "compress_rows", "embed_layernorm", "seq_start", "seq_order", "mask_class", "split_weight", "restore_rows")
+SIDE = ("scan_index", "compress_rows", "embed_layernorm", "seq_start", "seq_order", "mask_class", "pair_weight", "pair_rows", "restore_rows")
 LAYER_KINDS = ("attention", "bias_residual_layernorm", "gemm_f16_pair", "gemm_f16_bt", "gemm_f16_persistent", "gemm_f16_kernel",
-               "gemm_f32", "gemm_split")
+               "gemm_f32", "gemm_pair_kernel", "gemm_split")
 
 
 def describe(workload: str) -> str:
@@ -45,7 +45,7 @@ def short(name: str) -> str:
 def kind(name: str) -> str:
     """What a dispatch is, by its kernel name."""
     for k in SIDE + ("attention", "bias_residual_layernorm", "bias_gelu", "layer_prologue", "gemm_f16_pair", "gemm_f16_bt",
-                     "gemm_f16_persistent", "gemm_f16_kernel", "gemm_f32", "gemm_split", "mfma_ceiling", "copyBuffer"):
+                     "gemm_f16_persistent", "gemm_f16_kernel", "gemm_f32", "gemm_pair_kernel", "gemm_split", "mfma_ceiling", "copyBuffer"):
         if k in name:
             return k
     return name[:30]
@@ -56,9 +56,9 @@ def encoder_steps(kinds, layers):
     dispatch sequence."""
     steps, i = [], 0
     while i < len(kinds):
-        if kinds[i] in ("compress_rows", "embed_layernorm"):
+        if kinds[i] in ("compress_rows", "pair_rows", "embed_layernorm"):
             j = i + 1
-            while j < len(kinds) and kinds[j] not in ("restore_rows", "compress_rows", "embed_layernorm", "scan_index"):
+            while j < len(kinds) and kinds[j] not in ("restore_rows", "compress_rows", "pair_rows", "embed_layernorm", "scan_index"):
                 j += 1
             if j < len(kinds) and kinds[j] == "restore_rows":
                 # the layer kernels only: no table build, no prologue, no runtime copy kernel (read-back of the count)
@@ -183,8 +183,8 @@ def cmd_kernels(d, name, workload, bench_json=None):
             if "flops" in w:
                 work = "%.1f GFLOP" % (w["flops"] / 1e9)
                 ach = "%.0f TFLOP/s" % (w["flops"] / a / 1e6)
-                # split products: six 16-bit products for one of floats
-                frac = w["flops"] / a / 1e6 / (2500.0 / 6 if "gemm_split" in names[role] else peak)
+                # products of pair rows: three 16-bit products for one of floats
+                frac = w["flops"] / a / 1e6 / (2500.0 / 3 if "gemm_pair_kernel" in names[role] else peak)
             else:
                 work = "%.1f MB" % ((w["read"] + w["write"]) / 1e6)
                 ach = "%.2f TB/s" % ((w["read"] + w["write"]) / a / 1e6)
@@ -195,11 +195,13 @@ def cmd_kernels(d, name, workload, bench_json=None):
             v = [t["us"] for t in trace if t["kind"] == k]
             if v and k not in ("embed_layernorm", "seq_start", "seq_order"):       # (these three: not in the encoder's steps)
                 side[k] = mean(v)
-        tot += side.get("split_weight", 0.0)                                       # fp32: once per layer
-        out.append("\nPeaks: fp16 MFMA 2500 TFLOP/s, fp32 MFMA 157.3, products of split rows 2500 / 6, HBM 8 TB/s.  Sum per layer%s: %.1f us; x %d layers + what a batch takes once (%s) = %.3f ms per batch."
-                   % (" with split_weight %.1f" % side["split_weight"] if "split_weight" in side else "", tot, wl.layers,
-                      ", ".join("%s %.1f" % kv for kv in side.items() if kv[0] != "split_weight"),
-                      (tot * wl.layers + sum(v for k, v in side.items() if k != "split_weight")) / 1e3))
+        if "pair_weight" in side:                                                  # fp32: two launches per layer
+            side["pair_weight"] *= 2
+        tot += side.get("pair_weight", 0.0)
+        out.append("\nPeaks: fp16 MFMA 2500 TFLOP/s, fp32 MFMA 157.3, products of pair rows 2500 / 3, HBM 8 TB/s.  Sum per layer%s: %.1f us; x %d layers + what a batch takes once (%s) = %.3f ms per batch."
+                   % (" with pair_weight %.1f" % side["pair_weight"] if "pair_weight" in side else "", tot, wl.layers,
+                      ", ".join("%s %.1f" % kv for kv in side.items() if kv[0] != "pair_weight"),
+                      (tot * wl.layers + sum(v for k, v in side.items() if k != "pair_weight")) / 1e3))
     print("\n".join(out))
 
 
@@ -290,7 +292,7 @@ def cmd_vendor(paths):
     out.append("the weights in TF's `[k][n]` order and in the k-contiguous `[n][k]` order; the own kernel includes the bias (QKV) or")
     out.append("bias + GELU (FFN up; `plain` = the same kernel without the epilogue). `in layer` = the own kernel inside the layer's")
     out.append("launch sequence (its input still in the last-level cache). TFLOP/s of the fastest vendor variant and of the own kernel")
-    out.append("alone are given for the roofline (fp16 peak 2500; fp32: the own kernel is the product of split rows, peak 2500 / 6, the")
+    out.append("alone are given for the roofline (fp16 peak 2500; fp32: the own kernel is the product of pair rows, peak 2500 / 3, the")
     out.append("vendor's the fp32 MFMA one, 157.3).\n")
     for path in paths:
         d = last_json_line(path)

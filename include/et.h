@@ -132,8 +132,9 @@ et_status et_input_static(et_handle h, et_dtype dtype, const void* from_tensor, 
  * other shape runs element-wise kernels with the same arithmetic (the reference's kernels index by element too,
  * cuda/attention.cu:190-219).
  * The weights are read anew by every call and stay as they are: the copies the products read (k-contiguous in fp16, split
- * rows in fp32, see et_gemm_split) are made in the workspace.  fp32 products of hidden sizes in multiples of 32 run on split
- * rows: what et_gemm_split says of infinities and of the terms it leaves out goes for them. */
+ * rows in fp32, see et_gemm_split) are made in the workspace.  fp32 products of hidden sizes in multiples of 64 from 512 to 2048
+ * run on pair rows, other multiples of 32 on split rows: what et_gemm_pair and et_gemm_split say of infinities and of the terms
+ * they leave out goes for them. */
 et_status et_layer(et_handle h, et_dtype dtype, const et_layer_weights* weights,
                    const void* from_tensor, const void* to_tensor, const void* attr_mask,
                    const int32_t* valid_word_num_dev, const int32_t* batch_idx, const int32_t* word_idx,
@@ -392,6 +393,31 @@ et_status et_gemm_bt_bias_gelu(et_handle h, et_dtype dtype, const void* A, const
 et_status et_split_rows(et_handle h, const void* src, void* dst, int m, int k, const int32_t* m_dev, void* stream);
 et_status et_gemm_split(et_handle h, const void* A, const void* Bt, void* C, const void* bias, int gelu, int m, int n,
                         int k, const int32_t* m_dev, void* stream);
+
+/* The fp32 product of the layer at hidden sizes in multiples of 64 from 512 to 2048, on the fp16 matrix cores:
+ * C[m,n] = A[m,k] . Bt[n,k]^T (+ bias).  Both operands are pair rows, [row][k / 32][2][32] halves, with an exponent e per row:
+ * x 2^-e = h + l, h rounded to nearest (below 2^15) and l the rest rounded to nearest.  That keeps 22 to 24 significant bits of
+ * values down to about 2^-30 of the row's largest, and 2^-40 of it below.  h.h, h.l and l.h are summed in float, l.l (at most 2^-24
+ * of a product) is left out; from k = 512 on the result is closer to float64 than et_gemm_split's and et_gemm's.  Infinities and
+ * NaN give NaN in every result they enter.  k % 64 == 0, n % 16 == 0.
+ * et_pair_rows writes the first m (or *m_dev) rows of src[m][k] (k <= 2048) with their exponents and Euclidean norms.
+ * et_pair_weight writes the n pair rows of the transpose of src[k][n] and their exponents; `stats` (may be NULL, otherwise
+ * et_pair_weight_stats(n, k) floats) receives what bounds |column| and |bias| for et_gemm_pair.  C is float [m,n]; with c_exp
+ * (needs A->norm, bias and stats; n % 32 == 0) it holds the pair rows of gelu(A.Bt^T + bias) instead, whose exponents go to
+ * c_exp and come from the bound |a| |column| + |bias|.  The arrays of exponents and norms of A and C have room for 511 entries
+ * behind the last row (whole tiles are read). */
+typedef struct et_pair_matrix {
+  void* rows;                        /* 4 k bytes per row */
+  int32_t* exp;
+  float* norm;                       /* may be NULL for a matrix that is only multiplied without c_exp */
+} et_pair_matrix;
+size_t et_pair_weight_stats(int n, int k);
+size_t et_pair_weight_workspace_bytes(int n, int k);
+et_status et_pair_rows(et_handle h, const void* src, const et_pair_matrix* dst, int m, int k, const int32_t* m_dev, void* stream);
+et_status et_pair_weight(et_handle h, const void* src, void* dst, int32_t* exp, const void* bias, float* stats, int k, int n,
+                         void* workspace, size_t workspace_bytes, void* stream);
+et_status et_gemm_pair(et_handle h, const et_pair_matrix* A, const void* Bt, const int32_t* b_exp, const float* b_stats,
+                       const void* bias, void* C, int32_t* c_exp, int m, int n, int k, const int32_t* m_dev, void* stream);
 
 /* Measurement aid, no counterpart in the reference and no part of the encoder path: one launch of `iters` k-steps of
  * the large fp16 GEMM's inner loop (per wavefront 32 v_mfma_f32_16x16x32_f16 and 12 16-byte LDS operand reads, 8

@@ -1,0 +1,118 @@
+"""fp32 products on pair rows (csrc/gemm_pair.hip) against float64, at the edges of their tiles, and layers that run on them."""
+import numpy as np
+import pytest
+import torch
+
+from effective_transformer_amd import kernel_ops as k, ops
+from oracle import et_oracle as o
+from gpu_util import dev
+
+pytestmark = pytest.mark.gpu
+
+
+def _operands(m, n, kk, positive=False):
+    g = torch.Generator(device="cuda").manual_seed(m * 7 + n * 3 + kk)
+    a = torch.randn(m, kk, device="cuda", generator=g)
+    b = torch.randn(kk, n, device="cuda", generator=g) * 0.02
+    bias = torch.randn(n, device="cuda", generator=g)
+    return (a.abs(), b.abs(), bias) if positive else (a, b, bias)
+
+
+def _rel(got, want):
+    return ((got - want).norm() / want.norm()).item()
+
+
+# rows and columns around 32, 64, 96, 128, 192 and 256 (tiles' sides), one and an odd number of chunks of 64 k, fewer stages than
+# a ring holds, grids of one to several rounds of the chip (every tile shape is picked by one of them)
+@pytest.mark.parametrize("m,n,kk", [(1, 16, 64), (31, 48, 64), (33, 64, 192), (64, 112, 320), (65, 768, 768), (127, 144, 128),
+                                    (257, 144, 448), (600, 768, 1024), (700, 3072, 768), (1025, 2304, 768), (1500, 768, 2048),
+                                    (4000, 2304, 512), (5761, 784, 768), (8000, 768, 1536), (9000, 1536, 128)])
+@pytest.mark.parametrize("positive", [False, True])
+def test_gemm_pair(m, n, kk, positive):
+    print("gemm_pair", m, n, kk, positive, flush=True)
+    a, b, bias = _operands(m, n, kk, positive)
+    pa = k.pair_rows(a)
+    pb, stats = k.pair_weight(b, bias)
+    # h holds 11 bits, l 11 of the rest: half a unit of 2^-22 of the value at most, 2^-40 of the row's bound below that
+    assert ((pa.values() - a.double()).abs() <= a.double().abs() * 2.0 ** -23 + a.abs().amax(1, keepdim=True).double() * 2.0 ** -39).all()
+    assert torch.allclose(pa.norm[:m], a.norm(dim=1), rtol=1e-6)
+    assert stats[0::2].max() >= b.norm(dim=0).max() * 0.999 and stats[1::2].max() == bias.abs().max()
+    want = (a.cpu().double() @ b.cpu().double()).cuda()
+    got = k.gemm_pair(pa, pb)
+    # two operands rounded to 23 bits (rms 0.44 units of 2^-23 each), h.h + h.l + l.h without l.l (as much again), and a chunk of
+    # six roundings per 64 k: below what split rows have from k = 512 on, below twice that at any k
+    split = _rel(k.gemm_split(k.split_rows(a), k.transpose_weight(b)), want)
+    err = _rel(got, want)
+    assert err <= (split if kk >= 512 else max(2 * split, 2e-7)), (err, split)
+    assert torch.equal(k.gemm_pair(pa, pb, bias=bias), got + bias)
+    # a row has the same bits whatever the number of rows (other tiles), and rows beyond the device's count stay as they are
+    for rows in (1, (m + 1) // 2):
+        assert torch.equal(k.gemm_pair(k.pair_rows(a[:rows].contiguous()), pb), got[:rows])
+    count = torch.tensor([m // 2], dtype=torch.int32, device="cuda")
+    part = k.gemm_pair(pa, pb, m_dev=count)
+    assert torch.equal(part[:m // 2], got[:m // 2]) and (part[m // 2:] == 0).all()
+    rows = k.pair_rows(a, m_dev=count)
+    assert torch.equal(rows.rows[:m // 2], pa.rows[:m // 2]) and (rows.rows[m // 2:] == 0).all()
+    if n % 32 == 0:
+        act = k.gemm_pair(pa, pb, bias=bias, stats=stats, gelu=True)
+        ref = torch.nn.functional.gelu(want + bias.double(), approximate="tanh")
+        assert torch.isfinite(act.rows.float()).all() and _rel(act.values(), ref) < 1e-6
+
+
+# the exponents take what rows and columns differ by: the same relative error at 1e30, 1e-30 and in between, row by row; zero
+# rows and columns are zero; what a row cannot hold (2^-40 of its largest value) is all that is lost
+def test_magnitudes():
+    a, b, _ = _operands(70, 64, 768)
+    rows = torch.tensor([1e30, 1e-25, 1.0, 1e5, 1e-5], device="cuda").repeat(14)[:, None]
+    cols = torch.tensor([1e-12, 1e6, 1.0, 1e-4], device="cuda").repeat(16)[None]
+    a, b = a * rows, b * cols
+    a[3], b[:, 5] = 0, 0
+    got = k.gemm_pair(k.pair_rows(a), k.pair_weight(b)[0]).double().cpu()
+    want = a.cpu().double() @ b.cpu().double()
+    assert (got[3] == 0).all() and (got[:, 5] == 0).all()
+    scale = (a.double().norm(dim=1)[:, None] * b.double().norm(dim=0)[None]).cpu()
+    assert ((got - want).abs() <= 1e-6 * scale).all()
+    wide = torch.randn(8, 768, device="cuda") * torch.logspace(0, -9, 768, device="cuda")
+    err = (k.pair_rows(wide).values() - wide.double()).abs()
+    assert (err <= wide.double().abs() * 2.0 ** -23 + wide.abs().amax(1, keepdim=True).double() * 2.0 ** -39).all()
+
+
+# infinities and NaN reach the results of their row and no others
+def test_special_values():
+    a, b, bias = _operands(40, 64, 128)
+    clean = k.gemm_pair(k.pair_rows(a), k.pair_weight(b)[0])
+    a[7, 3], a[9, 100], a[11] = float("inf"), float("nan"), 3.4e38
+    got = k.gemm_pair(k.pair_rows(a), k.pair_weight(b)[0])
+    assert torch.isnan(got[7]).all() and torch.isnan(got[9]).all()
+    keep = [r for r in range(40) if r not in (7, 9, 11)]
+    assert torch.equal(got[keep], clean[keep])
+    assert torch.allclose(got[11].double(), 3.4e38 * b.double().sum(0), rtol=1e-4, atol=1e33)
+
+
+# layers on pair rows: head sizes with and without an attention kernel that writes them, hidden sizes of one and an odd number of
+# chunks, positions of either fp32 attention kernel; weights and rows of very different sizes.  Split and plain copies of the
+# weights: the same bits.
+@pytest.mark.parametrize("heads,d,B,S", [(8, 64, 3, 32), (16, 32, 3, 20), (9, 64, 2, 40), (12, 64, 5, 130)])
+@pytest.mark.parametrize("scale", [1.0, 1e3])
+def test_layer(heads, d, B, S, scale):
+    print("layer", heads, d, B, S, scale, flush=True)
+    H = heads * d
+    rng = np.random.RandomState(B * S + heads)
+    w = []
+    for i in range(4):
+        w += [rng.randn(H, H).astype(np.float32) * 0.02 / (scale if i < 2 else 1), rng.randn(H).astype(np.float32) * 0.02]
+    w += [rng.randn(H).astype(np.float32) * 0.05, 1 + rng.randn(H).astype(np.float32) * 0.05,
+          rng.randn(H, 4 * H).astype(np.float32) * 0.02, rng.randn(4 * H).astype(np.float32) * 0.02,
+          rng.randn(4 * H, H).astype(np.float32) * 0.02, rng.randn(H).astype(np.float32) * 0.02,
+          rng.randn(H).astype(np.float32) * 0.05, 1 + rng.randn(H).astype(np.float32) * 0.05]
+    lens = rng.randint(1, S + 1, size=B)
+    mask = (np.arange(S)[None] < lens[:, None]).astype(np.int32)
+    attr = np.ascontiguousarray(np.broadcast_to(mask[:, None], (B, S, S))).astype(np.float32)
+    x = rng.randn(B, S, H).astype(np.float32) * scale
+    enc = ops.EffectiveTransformerEncoder(2, heads, d, [dev(t) for t in w + w], torch.float32)
+    got = enc(dev(x), dev(mask), dev(attr)).cpu().numpy().astype(np.float64)
+    want = o.encoder(x, mask, attr, w + w, heads, d, "fp32").astype(np.float64)
+    valid = mask.astype(bool)
+    # (the oracle is float32 itself: about 1e-7 per product on either side, eight of them in a row)
+    assert (got[~valid] == 0).all()
+    assert np.linalg.norm(got[valid] - want[valid]) <= 2e-6 * np.linalg.norm(want[valid])
