@@ -652,60 +652,14 @@ struct Unseen {
     extra += (float)keys * __builtin_amdgcn_exp2f(-ref);
   }
 };
-// what is known of a block's mask rows behind the last token
-constexpr int kMaskPlain = 1, kMaskZeros = 2, kMaskOnes = 4;
 typedef uint32_t uint4x __attribute__((ext_vector_type(4)));
 
-// class of every block of 16 query positions: kMaskPlain = the rows of the mask are 1 for keys up to the last token's and 0
-// beyond, kMaskZeros / kMaskOnes = they are all 0 / all 1 beyond it
 template <typename T>
 __global__ __launch_bounds__(256) void mask_class_kernel(const T* __restrict__ attr_mask, const int32_t* __restrict__ seq_start,
                                                          const int32_t* __restrict__ word_idx, int seq_len, int blocks,
                                                          uint8_t* __restrict__ cls) {
-  constexpr int kElems = Chunk16<T>::kElems;
   const int b = blockIdx.y, qb = blockIdx.x;
-  const int t0 = seq_start[b], t1 = seq_start[b + 1];
-  if (t1 <= t0) return;
-  const int n = min(max(word_idx[t1 - 1], 0), seq_len - 1) + 1;
-  if (qb * 16 >= n) return;                                  // never looked at
-  const int rows = min(16, n - qb * 16);
-  const T* m = attr_mask + ((size_t)b * seq_len + qb * 16) * seq_len;
-  // what differs from 1 up to the last token, from 0 behind it, from 1 behind it (bit patterns)
-  uint32_t no_token = 0, no_zero = 0, no_one = 0;
-  if (seq_len % kElems == 0) {
-    constexpr uint32_t kOne = sizeof(T) == 2 ? 0x3c003c00u : 0x3f800000u;
-    const int cpr = seq_len / kElems;
-#pragma unroll 4
-    for (int i = threadIdx.x; i < rows * cpr; i += 256) {
-      const uint4x w = reinterpret_cast<const uint4x*>(m)[i];
-      const int bits = (n - (i % cpr) * kElems) * (int)sizeof(T) * 8;       // of the 128 here, those up to the last token
-#pragma unroll
-      for (int j = 0; j < 4; ++j) {
-        const int t = min(max(bits - j * 32, 0), 32);
-        const uint32_t token = (uint32_t)((1ull << t) - 1), one = w[j] ^ kOne;
-        no_token |= one & token;
-        no_zero |= w[j] & ~token;
-        no_one |= one & ~token;
-      }
-    }
-  } else {
-    for (int i = threadIdx.x; i < rows * seq_len; i += 256) {
-      const T v = m[i];
-      const uint32_t zero = v == (T)0.0f ? 0u : 1u, one = v == (T)1.0f ? 0u : 1u;
-      if (i % seq_len < n) {
-        no_token |= one;
-      } else {
-        no_zero |= zero;
-        no_one |= one;
-      }
-    }
-  }
-  __shared__ int found[4];
-  const bool plain = !__any(no_token != 0), zeros = !__any(no_zero != 0), ones = !__any(no_one != 0);
-  if ((threadIdx.x & (kWave - 1)) == 0)
-    found[threadIdx.x / kWave] = (plain && zeros ? kMaskPlain : 0) | (zeros ? kMaskZeros : 0) | (ones ? kMaskOnes : 0);
-  __syncthreads();
-  if (threadIdx.x == 0) cls[(size_t)b * blocks + qb] = (uint8_t)(found[0] & found[1] & found[2] & found[3]);
+  mask_class_block(attr_mask, word_idx, b, qb, seq_start[b], seq_start[b + 1], seq_len, blocks, cls);
 }
 
 __device__ __forceinline__ int v_swizzle(int key) { return (((key >> 1) & 1) | ((key >> 2) & 2)) * 2; }

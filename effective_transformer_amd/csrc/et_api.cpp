@@ -339,6 +339,25 @@ struct LayerCall {
 };
 et_status run_layer(et_handle h, const LayerCall& c);
 
+// What the call does not bring along of its batch: the sequence table, and the mask's classes where the attention kernel makes
+// use of them.
+et::BatchJobs layer_batch_jobs(const LayerCall& c, const LayerWs& ws) {
+  et::BatchJobs j;
+  if (c.seq_start) return j;
+  j.batch_idx = c.batch_idx;
+  j.word_idx = c.word_idx;
+  j.rows_dev = c.rows_exact ? nullptr : c.count;
+  j.rows_bound = c.rows;
+  j.batch = c.B;
+  j.seq_len = c.S;
+  j.seq_table = (int32_t*)(c.workspace + ws.seq);
+  j.attr_mask = c.attr_mask;
+  j.fp32 = c.dtype == ET_FP32;
+  if (!c.mask_class && et::mask_class_bytes(to_dt(c.dtype), c.B, c.S, c.d)) j.cls = (uint8_t*)(c.workspace + ws.cls);
+  et::count_batch_jobs(&j);
+  return j;
+}
+
 // The pair rows of a layer's first input, where et_encoder leaves them and the Q/K/V projections find them.
 et::PairRows first_pair_rows(char* layer_base, const LayerWs& ws, int B, int S, int H) {
   const PairWs p = pair_ws(layer_base + ws.pair, (size_t)B * S, (size_t)H);
@@ -377,11 +396,8 @@ et_status run_layer_pairs(et_handle h, const LayerCall& c) {
   weight(w->attr_output_kernel, pp.attr_output_kernel_t, H, H, 3, nullptr, nullptr);
   weight(w->inter_kernel, pp.inter_kernel_t, H, F, 4, w->inter_bias, pw.up_stats);
   weight(w->output_kernel, pp.output_kernel_t, F, H, 8, nullptr, nullptr);
-  et::launch_pair_weights(jobs, st);
-  if (!c.seq_start) {
-    const et::SeqStartJob seq{c.batch_idx, T, rows, B, (int32_t*)(base + ws.seq)};
-    et::launch_transpose_weights(et::TransposeJobs(), st, &seq);
-  }
+  const et::BatchJobs batch = layer_batch_jobs(c, ws);
+  et::launch_pair_weights(jobs, st, &batch);
 
   // the inputs, in the room of the intermediate, which nothing needs before they have been read
   et::PairRows from = first_pair_rows(base, ws, B, S, H), to = from;
@@ -404,7 +420,7 @@ et_status run_layer_pairs(et_handle h, const LayerCall& c) {
 
   const float *q = qkv, *k = q + H, *v = k + H;
   const bool ctx_pairs = et::attention_writes_split(q, k, v, 1, 3 * H, c.d);
-  const uint8_t* cls = c.mask_class;
+  const uint8_t* cls = c.mask_class ? c.mask_class : batch.cls;
   if (!cls && et::mask_class_bytes(dt, B, S, c.d)) {
     et::launch_mask_class(dt, c.attr_mask, seq_start, c.word_idx, B, S, (uint8_t*)(base + ws.cls), st);
     cls = (const uint8_t*)(base + ws.cls);
@@ -481,6 +497,7 @@ et_status run_layer(et_handle h, const LayerCall& c) {
   const size_t HH = (size_t)H * H * (split ? 6 : e);
   const void* wt_q = wt; const void* wt_k = wt + HH; const void* wt_v = wt + 2 * HH; const void* wt_o = wt + 3 * HH;
   const void* wt_up = wt + 4 * HH; const void* wt_down = wt + 8 * HH;
+  const et::BatchJobs batch = layer_batch_jobs(c, ws);
   {
     et::TransposeJobs jobs;
     if (t_qkv && pp.attr_kernel_Q_t) {
@@ -496,13 +513,12 @@ et_status run_layer(et_handle h, const LayerCall& c) {
     else if (t_up) jobs.add(w->inter_kernel, wt + 4 * HH, H, F);
     if (t_down && pp.output_kernel_t) wt_down = pp.output_kernel_t;
     else if (t_down) jobs.add(w->output_kernel, wt + 8 * HH, F, H);
-    // one launch builds the sequence start table and the transposed copies; none when the caller prepared both
-    const et::SeqStartJob seq{c.batch_idx, T, rows, B, (int32_t*)(base + ws.seq)};
+    // one launch makes the sequence table, the mask's classes and the transposed copies; none when the caller prepared all
     if (split) {
       et::launch_split_weights(jobs, st);
       jobs.count = 0;
     }
-    et::launch_transpose_weights(jobs, st, c.seq_start ? nullptr : &seq);
+    et::launch_transpose_weights(jobs, st, &batch);
   }
   // split rows of the two inputs, in the room of the intermediate, which nothing needs before they have been read
   const void *from_a = c.from, *to_a = c.to;
@@ -537,7 +553,7 @@ et_status run_layer(et_handle h, const LayerCall& c) {
   // QK^T, softmax, PV, un-pad (:159-192)
   const char *q = (const char*)qkv, *k = q + (size_t)H * e, *v = k + (size_t)H * e;
   const bool ctx_split = split && et::attention_writes_split(q, k, v, 1, 3 * H, c.d);
-  const uint8_t* cls = c.mask_class;
+  const uint8_t* cls = c.mask_class ? c.mask_class : batch.cls;
   if (!cls && et::mask_class_bytes(dt, B, S, c.d)) {
     et::launch_mask_class(dt, c.attr_mask, seq_start, c.word_idx, B, S, (uint8_t*)(base + ws.cls), st);
     cls = (const uint8_t*)(base + ws.cls);

@@ -268,7 +268,7 @@ __device__ __forceinline__ void seq_start_for_row(const int32_t* __restrict__ ba
 // order[0..batch) = the sequences sorted by length, longest first (buckets of 16 tokens; the order inside a bucket is
 // whatever the atomics give: it only decides which workgroup of the attention kernel starts first).  All THREADS threads
 // of one workgroup.
-constexpr int kOrderBuckets = 65;             // lengths up to 1024
+constexpr int kOrderBuckets = kWave + 1;      // lengths up to 1024
 template <int THREADS>
 __device__ __forceinline__ void sort_sequences(const int32_t* __restrict__ seq_start, int batch, int32_t* __restrict__ order) {
   __shared__ int hist[kOrderBuckets], base[kOrderBuckets];
@@ -280,15 +280,174 @@ __device__ __forceinline__ void sort_sequences(const int32_t* __restrict__ seq_s
   };
   for (int b = threadIdx.x; b < batch; b += THREADS) atomicAdd(&hist[bucket_of(b)], 1);
   __syncthreads();
-  if (threadIdx.x == 0) {
-    int run = 0;
-    for (int i = 0; i < kOrderBuckets; ++i) {
-      base[i] = run;
-      run += hist[i];
-    }
+  if (threadIdx.x < kWave) {                  // 65 buckets: one per lane, and the last one behind them all
+    const int mine = hist[threadIdx.x], upto = wave_inclusive_scan_i32(mine);
+    base[threadIdx.x] = upto - mine;
+    if (threadIdx.x == kWave - 1) base[kWave] = upto;
   }
   __syncthreads();
   for (int b = threadIdx.x; b < batch; b += THREADS) order[atomicAdd(&base[bucket_of(b)], 1)] = b;
+}
+
+// The smallest t in [0, T] from which on batch_idx[t] >= b; batch_idx is ascending.  Whole wavefronts.
+__device__ __forceinline__ int wave_lower_bound(const int32_t* __restrict__ batch_idx, int T, int b) {
+  int lo = 0, hi = T;
+  while (hi > lo) {
+    const int len = hi - lo, step = (len + kWave - 1) / kWave, probe = lo + lane_id() * step;
+    const int c = __popcll(__ballot(probe < hi && batch_idx[min(probe, hi - 1)] < b));
+    hi = c == 0 ? lo : min(lo + c * step, hi);
+    lo = c == 0 ? lo : lo + (c - 1) * step + 1;
+  }
+  return lo;
+}
+
+// ---- classes of the mask rows --------------------------------------------------------------
+// what is known of a block's mask rows behind the last token
+constexpr int kMaskPlain = 1, kMaskZeros = 2, kMaskOnes = 4;
+
+// class of a block of 16 query positions: kMaskPlain = the rows of the mask are 1 for keys up to the last token's and 0
+// beyond, kMaskZeros / kMaskOnes = they are all 0 / all 1 beyond it.  All 256 threads of a workgroup; the rows of sequence b are
+// t0 .. t1.
+template <typename T>
+__device__ __forceinline__ void mask_class_block(const T* __restrict__ attr_mask, const int32_t* __restrict__ word_idx, int b, int qb,
+                                                 int t0, int t1, int seq_len, int blocks, uint8_t* __restrict__ cls) {
+  constexpr int kElems = 16 / (int)sizeof(T);
+  typedef uint32_t words __attribute__((ext_vector_type(4)));
+  if (t1 <= t0) return;
+  const int n = min(max(word_idx[t1 - 1], 0), seq_len - 1) + 1;
+  if (qb * 16 >= n) return;                                  // never looked at
+  const int rows = min(16, n - qb * 16);
+  const T* m = attr_mask + ((size_t)b * seq_len + qb * 16) * seq_len;
+  // what differs from 1 up to the last token, from 0 behind it, from 1 behind it (bit patterns)
+  uint32_t no_token = 0, no_zero = 0, no_one = 0;
+  if (seq_len % kElems == 0) {
+    constexpr uint32_t kOne = sizeof(T) == 2 ? 0x3c003c00u : 0x3f800000u;
+    const int cpr = seq_len / kElems;
+#pragma unroll 4
+    for (int i = threadIdx.x; i < rows * cpr; i += 256) {
+      const words w = reinterpret_cast<const words*>(m)[i];
+      const int bits = (n - (i % cpr) * kElems) * (int)sizeof(T) * 8;       // of the 128 here, those up to the last token
+#pragma unroll
+      for (int j = 0; j < 4; ++j) {
+        const int t = min(max(bits - j * 32, 0), 32);
+        const uint32_t token = (uint32_t)((1ull << t) - 1), one = w[j] ^ kOne;
+        no_token |= one & token;
+        no_zero |= w[j] & ~token;
+        no_one |= one & ~token;
+      }
+    }
+  } else {
+    for (int i = threadIdx.x; i < rows * seq_len; i += 256) {
+      const T v = m[i];
+      const uint32_t zero = v == (T)0.0f ? 0u : 1u, one = v == (T)1.0f ? 0u : 1u;
+      if (i % seq_len < n) {
+        no_token |= one;
+      } else {
+        no_zero |= zero;
+        no_one |= one;
+      }
+    }
+  }
+  __shared__ int found[4];
+  const bool plain = !__any(no_token != 0), zeros = !__any(no_zero != 0), ones = !__any(no_one != 0);
+  if ((threadIdx.x & (kWave - 1)) == 0)
+    found[threadIdx.x / kWave] = (plain && zeros ? kMaskPlain : 0) | (zeros ? kMaskZeros : 0) | (ones ? kMaskOnes : 0);
+  __syncthreads();
+  if (threadIdx.x == 0) cls[(size_t)b * blocks + qb] = (uint8_t)(found[0] & found[1] & found[2] & found[3]);
+}
+
+// ---- what a layer needs to know of its batch, by blocks of the launch that prepares its weights ---------------
+// (a launch of its own for each of them costs the layer 2 .. 5 us and the calling thread 3 us: seq_order_kernel and
+// mask_class_kernel behind the weights' launch, 8.8 + 1.7 + 5.0 us, against 9.6 us with their blocks in it at 39 x 117 positions;
+// six layer calls 675 -> 640 us)
+constexpr int kTableBatch = 2303;             // sequences whose starts a block keeps in LDS
+// Up to this many rows one block looks at all of batch_idx (12 single-layer calls: 1 x 32 positions 719 -> 680 us, 8 x 128 829 ->
+// 810 us, 64 x 32 972 -> 946 us against the starts by many blocks and the sort in a launch of its own); beyond, it searches for
+// the starts of up to kTableSearch sequences, three to six dependent loads.
+constexpr int kTableRows = 2048;
+constexpr int kTableSearch = 1024;
+
+// starts[b] for the sequences threadIdx.x + 256 q: a step leaves one part in PROBES + 1 of the rows that may hold the start.
+template <int SEQS, int PROBES>
+__device__ __forceinline__ void search_starts(const int32_t* __restrict__ batch_idx, int T, int batch, int32_t* starts) {
+  int lo[SEQS];
+#pragma unroll
+  for (int q = 0; q < SEQS; ++q) lo[q] = 0;
+  for (int span = T; span > 0;) {              // the start lies in [lo, lo + span]
+    const int step = span / (PROBES + 1) + 1;
+    int seen[SEQS][PROBES];
+#pragma unroll
+    for (int q = 0; q < SEQS; ++q)
+#pragma unroll
+      for (int i = 0; i < PROBES; ++i) seen[q][i] = batch_idx[min(lo[q] + step * (i + 1) - 1, T - 1)];
+#pragma unroll
+    for (int q = 0; q < SEQS; ++q) {
+      const int b = (int)threadIdx.x + q * 256;
+      int c = 0;
+#pragma unroll
+      for (int i = 0; i < PROBES; ++i) c += lo[q] + step * (i + 1) - 1 < T && seen[q][i] < b ? 1 : 0;
+      lo[q] += c * step;
+    }
+    span = max(step - 1, span - PROBES * step);
+  }
+#pragma unroll
+  for (int q = 0; q < SEQS; ++q) {
+    const int b = (int)threadIdx.x + q * 256;
+    if (b < batch) starts[b] = lo[q];
+  }
+}
+
+// The whole sequence table by one block of 256 threads, the starts in LDS for the sort.
+__device__ __forceinline__ void sequence_table_block(const BatchJobs& jobs, int T, int32_t* starts) {
+  const int32_t* __restrict__ batch_idx = jobs.batch_idx;
+  if (T <= kTableRows) {
+    constexpr int kFly = 8;                                   // rows per thread requested together
+    for (int t0 = 0; t0 <= T; t0 += 256 * kFly) {
+      int prev[kFly], cur[kFly];
+#pragma unroll
+      for (int u = 0; u < kFly; ++u) {
+        const int t = t0 + u * 256 + (int)threadIdx.x;
+        prev[u] = t > 0 && t <= T ? batch_idx[t - 1] : -1;
+        cur[u] = t < T ? batch_idx[t] : jobs.batch;
+      }
+#pragma unroll
+      for (int u = 0; u < kFly; ++u) {
+        const int t = t0 + u * 256 + (int)threadIdx.x;
+        if (t > T) continue;
+        const int last = t == T ? jobs.batch : min(cur[u], jobs.batch - 1);
+        for (int b = max(prev[u], -1) + 1; b <= last; ++b) starts[b] = t;     // entries (prev, last] start at t
+      }
+    }
+  } else {
+    if (jobs.batch <= 256) search_starts<1, 32>(batch_idx, T, jobs.batch, starts);
+    else search_starts<kTableSearch / 256, 8>(batch_idx, T, jobs.batch, starts);
+    if (threadIdx.x == 0) starts[jobs.batch] = T;
+  }
+  __syncthreads();
+  for (int b = threadIdx.x; b <= jobs.batch; b += 256) jobs.seq_table[b] = starts[b];
+  sort_sequences<256>(starts, jobs.batch, jobs.seq_table + jobs.batch + 1);
+}
+
+// Block `block` of the jobs' batch_job_blocks() blocks; `scratch`: room for kTableBatch + 1 words of LDS.
+__device__ __forceinline__ void batch_job_block(const BatchJobs& jobs, int block, int32_t* scratch) {
+  const int T = jobs.rows_dev ? min(*jobs.rows_dev, jobs.rows_bound) : jobs.rows_bound;
+  if (block < jobs.table_blocks) {
+    if (jobs.one_block_table) sequence_table_block(jobs, T, scratch);
+    else seq_start_for_row(jobs.batch_idx, T, block * 256 + (int)threadIdx.x, jobs.batch, jobs.seq_table);
+    return;
+  }
+  // a class block: its sequence's rows, looked for by two of its wavefronts
+  block -= jobs.table_blocks;
+  const int blocks = (jobs.seq_len + 15) / 16, b = block / blocks, qb = block - b * blocks;
+  const int wave = threadIdx.x / kWave;
+  if (wave < 2) {
+    const int t = b + wave == jobs.batch ? T : wave_lower_bound(jobs.batch_idx, T, b + wave);
+    if ((threadIdx.x & (kWave - 1)) == 0) scratch[wave] = t;
+  }
+  __syncthreads();
+  const int t0 = scratch[0], t1 = scratch[1];
+  if (jobs.fp32) mask_class_block((const float*)jobs.attr_mask, jobs.word_idx, b, qb, t0, t1, jobs.seq_len, blocks, jobs.cls);
+  else mask_class_block((const _Float16*)jobs.attr_mask, jobs.word_idx, b, qb, t0, t1, jobs.seq_len, blocks, jobs.cls);
 }
 
 }  // namespace et

@@ -1475,59 +1475,20 @@ bool use_persistent_bt(int m_bound, int ldc, int n, int k, int groups) {
 struct TransposeArgs {
   TransposeJobs jobs;
   int tile_begin[TransposeJobs::kMax + 1];
-  SeqStartJob seq;             // blocks from tile_begin[kMax] on build the sequence start table (seq_start != null)
-  int one_block_table = 0;     // ... one block, the whole table, sorted half included; the first one of the launch
+  BatchJobs batch;             // the first blocks of the launch
 };
 constexpr int kTrTile = 64;
 constexpr int kTrStride = kTrTile + 8;    // halves; 144-byte rows keep the 16-byte row reads aligned
 
-// The whole sequence table by one block of 256 threads: the starts from one look at all of batch_idx, kept in LDS for the
-// sort behind it.  `starts`: room for batch + 1 words.
-constexpr int kTableBatch = kTrTile * kTrStride / 2 - 1;      // what the transposes' LDS tile holds
-// (12 single-layer calls: 1 x 32 positions 719 -> 680 us, 8 x 128 829 -> 810 us, 64 x 32 972 -> 946 us against the starts by many
-// blocks and the sort in a launch of its own; from 5000 rows on this block would take longer than the transposes beside it:
-// 217 x 53 2.15 -> 2.20 ms)
-constexpr int kTableRows = 2048;
-__device__ __forceinline__ void sequence_table_block(const SeqStartJob& seq, int T, int32_t* starts) {
-  constexpr int kFly = 8;                                     // rows per thread requested together
-  for (int t0 = 0; t0 <= T; t0 += 256 * kFly) {
-    int prev[kFly], cur[kFly];
-#pragma unroll
-    for (int u = 0; u < kFly; ++u) {
-      const int t = t0 + u * 256 + (int)threadIdx.x;
-      prev[u] = t > 0 && t <= T ? seq.batch_idx[t - 1] : -1;
-      cur[u] = t < T ? seq.batch_idx[t] : seq.batch;
-    }
-#pragma unroll
-    for (int u = 0; u < kFly; ++u) {
-      const int t = t0 + u * 256 + (int)threadIdx.x;
-      if (t > T) continue;
-      const int last = t == T ? seq.batch : min(cur[u], seq.batch - 1);
-      for (int b = max(prev[u], -1) + 1; b <= last; ++b) starts[b] = t;       // entries (prev, last] start at t
-    }
-  }
-  __syncthreads();
-  for (int b = threadIdx.x; b <= seq.batch; b += 256) seq.seq_start[b] = starts[b];
-  sort_sequences<256>(starts, seq.batch, seq.seq_start + seq.batch + 1);
-}
-
 __global__ __launch_bounds__(256) void layer_prologue_kernel(TransposeArgs args) {
   __shared__ __attribute__((aligned(16))) _Float16 tile[kTrTile * kTrStride];
   int block = blockIdx.x;
-  if (args.one_block_table) {
-    if (block == 0) {
-      const int T = args.seq.rows_dev ? min(*args.seq.rows_dev, args.seq.rows_bound) : args.seq.rows_bound;
-      sequence_table_block(args.seq, T, reinterpret_cast<int32_t*>(tile));
-      return;
-    }
-    --block;
-  }
-  if (block >= args.tile_begin[TransposeJobs::kMax]) {
-    const int T = args.seq.rows_dev ? min(*args.seq.rows_dev, args.seq.rows_bound) : args.seq.rows_bound;
-    seq_start_for_row(args.seq.batch_idx, T, (block - args.tile_begin[TransposeJobs::kMax]) * 256 + threadIdx.x,
-                      args.seq.batch, args.seq.seq_start);
+  if (block < args.batch.blocks) {
+    static_assert(sizeof(tile) >= (kTableBatch + 1) * sizeof(int32_t), "the sequences' starts");
+    batch_job_block(args.batch, block, reinterpret_cast<int32_t*>(tile));
     return;
   }
+  block -= args.batch.blocks;
   int job = 0;
   while (job + 1 < args.jobs.count && block >= args.tile_begin[job + 1]) ++job;
   const int K = args.jobs.k[job], N = args.jobs.n[job];
@@ -1589,8 +1550,8 @@ bool gemm_prefers_transposed_b(DType t, int m_bound, int ldc, int n, int k, int 
   return gemm_takes_transposed_b(t, m_bound, ldc, n, k, groups);
 }
 
-void launch_transpose_weights(const TransposeJobs& jobs, hipStream_t stream, const SeqStartJob* seq) {
-  if (jobs.count == 0 && seq == nullptr) return;
+void launch_transpose_weights(const TransposeJobs& jobs, hipStream_t stream, const BatchJobs* batch) {
+  if (jobs.count == 0 && (batch == nullptr || batch->blocks == 0)) return;
   TransposeArgs a;
   a.jobs = jobs;
   int total = 0;
@@ -1599,12 +1560,9 @@ void launch_transpose_weights(const TransposeJobs& jobs, hipStream_t stream, con
     total += ((jobs.k[j] + kTrTile - 1) / kTrTile) * ((jobs.n[j] + kTrTile - 1) / kTrTile);
   }
   for (int j = jobs.count; j <= TransposeJobs::kMax; ++j) a.tile_begin[j] = total;
-  a.seq = seq ? *seq : SeqStartJob{nullptr, nullptr, 0, 0, nullptr};
-  a.one_block_table = seq && seq->batch <= kTableBatch && seq->rows_bound <= kTableRows;
-  if (a.one_block_table) ++total;
-  else if (seq) total += (seq->rows_bound + 1 + 255) / 256;
-  layer_prologue_kernel<<<total, 256, 0, stream>>>(a);
-  if (seq && !a.one_block_table) launch_seq_order(seq->seq_start, seq->batch, stream);
+  if (batch) a.batch = *batch;
+  layer_prologue_kernel<<<total + a.batch.blocks, 256, 0, stream>>>(a);
+  if (a.batch.seq_table && !a.batch.one_block_table) launch_seq_order(a.batch.seq_table, a.batch.batch, stream);
 }
 
 bool gemm_supported(DType t, int n, int k, int groups) {

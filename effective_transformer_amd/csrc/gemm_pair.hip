@@ -493,13 +493,23 @@ struct PairWeightArgs {
   int tile_begin[PairWeightJobs::kMax + 1];
 };
 constexpr int kTopRows = 256;
-__global__ __launch_bounds__(256) void pair_weight_top_kernel(PairWeightArgs args) {
-  __shared__ float part[16][64];
+__global__ __launch_bounds__(256) void pair_weight_top_kernel(PairWeightArgs args, BatchJobs batch) {
+  __shared__ union {
+    float part[16][64];
+    int32_t starts[kTableBatch + 1];
+  } lds;
+  float (&part)[16][64] = lds.part;
+  int wg = blockIdx.x;
+  if (wg < batch.blocks) {
+    batch_job_block(batch, wg, lds.starts);
+    return;
+  }
+  wg -= batch.blocks;
   int job = 0;
-  while (job + 1 < args.jobs.count && (int)blockIdx.x >= args.tile_begin[job + 1]) ++job;
+  while (job + 1 < args.jobs.count && wg >= args.tile_begin[job + 1]) ++job;
   const PairWeightJob& jb = args.jobs.job[job];
   const int K = jb.k, N = jb.n, tiles_n = (N + 63) / 64;
-  const int t = blockIdx.x - args.tile_begin[job];
+  const int t = wg - args.tile_begin[job];
   const int block = t / tiles_n, k0 = block * kTopRows, n0 = (t - block * tiles_n) * 64;
   if (jb.src_split) {                            // rows of three bfloat16 pieces: four lanes per row, 64 k each
     const int r = threadIdx.x >> 2, kk = k0 + (threadIdx.x & 3) * 64;
@@ -647,7 +657,7 @@ void launch_pair_rows(const float* src, float* packed, const PairRows& out, cons
 
 bool pair_rows_supported(int n) { return n % 64 == 0 && n >= 64 && n <= 2048; }
 
-void launch_pair_weights(const PairWeightJobs& jobs, hipStream_t stream) {
+void launch_pair_weights(const PairWeightJobs& jobs, hipStream_t stream, const BatchJobs* batch) {
   if (jobs.count == 0) return;
   PairWeightArgs a;
   a.jobs = jobs;
@@ -661,7 +671,9 @@ void launch_pair_weights(const PairWeightJobs& jobs, hipStream_t stream) {
     return total;
   };
   const int tops = grid(kTopRows);
-  pair_weight_top_kernel<<<tops, 256, 0, stream>>>(a);
+  const BatchJobs b = batch ? *batch : BatchJobs();
+  pair_weight_top_kernel<<<tops + b.blocks, 256, 0, stream>>>(a, b);
+  if (b.seq_table && !b.one_block_table) launch_seq_order(b.seq_table, b.batch, stream);
   const int tiles = grid(64);
   pair_weight_kernel<<<tiles, 256, 0, stream>>>(a);
 }

@@ -405,6 +405,15 @@ void launch_restore_rows(void* to, const void* from, const int32_t* batch_idx, c
                                                                      word_idx, rows_dev, n_pos, seq_len, cpr);
 }
 
+void count_batch_jobs(BatchJobs* j) {
+  j->table_blocks = j->one_block_table = 0;
+  if (j->seq_table) {
+    j->one_block_table = j->batch <= kTableBatch && (j->rows_bound <= kTableRows || j->batch <= kTableSearch);
+    j->table_blocks = j->one_block_table ? 1 : (j->rows_bound + 1 + 255) / 256;
+  }
+  j->blocks = j->table_blocks + (j->cls ? j->batch * ((j->seq_len + 15) / 16) : 0);
+}
+
 void launch_seq_order(int32_t* seq_table, int batch, hipStream_t stream) {
   seq_order_kernel<<<1, 1024, 0, stream>>>(seq_table, batch, seq_table + batch + 1);
 }

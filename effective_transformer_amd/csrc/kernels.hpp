@@ -80,6 +80,22 @@ void launch_seq_start(const int32_t* batch_idx, const int32_t* rows_dev, int row
 // second half of the table from its first half (for tables whose first half another kernel wrote)
 void launch_seq_order(int32_t* seq_table, int batch, hipStream_t stream);
 
+// What a layer that is called without them needs to know of its batch: the sequence table and the classes of its mask rows
+// (either may be null).  Extra blocks of 256 threads in front of the launch that prepares the layer's weights; count_batch_jobs
+// counts them; a table that one block cannot make needs launch_seq_order behind the launch.
+struct BatchJobs {
+  const int32_t* batch_idx = nullptr;
+  const int32_t* word_idx = nullptr;
+  const int32_t* rows_dev = nullptr;
+  int rows_bound = 0, batch = 0, seq_len = 0;
+  int32_t* seq_table = nullptr;
+  const void* attr_mask = nullptr;
+  uint8_t* cls = nullptr;
+  int fp32 = 0;
+  int table_blocks = 0, one_block_table = 0, blocks = 0;      // filled in
+};
+void count_batch_jobs(BatchJobs* jobs);
+
 // ---- row_kernels.hip ---------------------------------------------------------------------
 bool bias_gelu_supported(DType t, int n);
 void launch_bias_gelu(DType t, void* out, const void* bias, int m, int n, const int32_t* rows_dev,
@@ -184,15 +200,8 @@ struct TransposeJobs {
   int count = 0;
   void add(const void* s, void* d, int k_, int n_) { src[count] = s; dst[count] = d; k[count] = k_; n[count] = n_; ++count; }
 };
-// The layer needs the per-sequence start table as well; `seq` (optional) makes the same launch build it, which saves a
-// launch per layer.
-struct SeqStartJob {
-  const int32_t* batch_idx;
-  const int32_t* rows_dev;
-  int rows_bound, batch;
-  int32_t* seq_start;
-};
-void launch_transpose_weights(const TransposeJobs& jobs, hipStream_t stream, const SeqStartJob* seq = nullptr);
+// `batch` (optional): the same launch makes what the layer needs to know of its batch.
+void launch_transpose_weights(const TransposeJobs& jobs, hipStream_t stream, const BatchJobs* batch = nullptr);
 void launch_gemm(DType t, const GemmGroups& g, void* C, int ldc, int m_bound, int n, int k,
                  const int32_t* rows_dev, hipStream_t stream);
 
@@ -231,7 +240,7 @@ struct PairWeightJobs {
   PairWeightJob job[kMax] = {};
   int count = 0;
 };
-void launch_pair_weights(const PairWeightJobs& jobs, hipStream_t stream);
+void launch_pair_weights(const PairWeightJobs& jobs, hipStream_t stream, const BatchJobs* batch = nullptr);
 // C[:, g n : (g + 1) n] = A[g].B[g] + bias[g] (bias may be null), float with leading dimension ldc; with c_exp
 // C = gelu(A.B + bias) as pair rows of ldc values, from A[0].norm and the weights' `stats`.
 struct PairProduct {
