@@ -223,17 +223,30 @@ __device__ __forceinline__ void store_pair_row(const V (&x)[ITERS], int vpr, con
     out.norm[r] = __builtin_ldexpf(__builtin_sqrtf(sq), e);
   }
 }
-// The largest first and the largest second word of `n` pairs of non-negative floats, by one wavefront; eight loads in flight.
-__device__ __forceinline__ float2v pair_stats_max(const float* __restrict__ stats, int n) {
-  const int lane = threadIdx.x & (kWave - 1);
+// a < b as an integer, without a compare of its own (what the scalar unit makes of a difference's sign)
+__device__ __forceinline__ int uniform_less(int a, int b) { return (int)((unsigned)(a - b) >> 31); }
+// a / b, a >= 0, b > 0, same in all lanes.  The compiler's division takes about twice the instructions.
+__device__ __forceinline__ int uniform_div(int a, int b) {
+  if (__builtin_expect(a >= 1 << 22, 0)) return a / b;     // the quotient of the two floats may be off by more than one
+  int q = __builtin_amdgcn_readfirstlane((int)((float)a * __builtin_amdgcn_rcpf((float)b)));
+  const int r = a - q * b;
+  return q - uniform_less(r, 0) + 1 - uniform_less(r, b);
+}
+// The largest first and the largest second word of `n` pairs of non-negative floats, by one wavefront: eight requests a lane, and
+// what becomes of them (and of the pairs behind the first 512).
+__device__ __forceinline__ void pair_stats_request(const float* __restrict__ stats, int n, int i0, float2v (&v)[8]) {
   const float2v* p = reinterpret_cast<const float2v*>(stats);
-  float2v top = {0.f, 0.f};
-  for (int i0 = 0; i0 < n; i0 += 8 * kWave) {
-    float2v v[8];
 #pragma unroll
-    for (int u = 0; u < 8; ++u) v[u] = p[min(i0 + u * kWave + lane, n - 1)];
+  for (int u = 0; u < 8; ++u) v[u] = p[min(i0 + u * kWave + (int)(threadIdx.x & (kWave - 1)), n - 1)];
+}
+__device__ __forceinline__ float2v pair_stats_max(const float* __restrict__ stats, int n, float2v (&v)[8]) {
+  float2v top = {0.f, 0.f};
+  for (int i0 = 0;;) {
 #pragma unroll
     for (int u = 0; u < 8; ++u) top = float2v{fmaxf(top[0], v[u][0]), fmaxf(top[1], v[u][1])};
+    i0 += 8 * kWave;
+    if (i0 >= n) break;
+    pair_stats_request(stats, n, i0, v);
   }
   return float2v{wave_max(top[0]), wave_max(top[1])};
 }
@@ -243,6 +256,8 @@ __device__ __forceinline__ int context_exponent(const float* __restrict__ norm, 
                                                 int n_stats) {
   const int lane = threadIdx.x & (kWave - 1);
   float top = 0.f;
+  float2v first[8];
+  pair_stats_request(stats, n_stats, 0, first);
   for (int i0 = t0; i0 < t1; i0 += 4 * kWave) {
     float v[4];
 #pragma unroll
@@ -250,7 +265,7 @@ __device__ __forceinline__ int context_exponent(const float* __restrict__ norm, 
 #pragma unroll
     for (int u = 0; u < 4; ++u) top = fmaxf(top, v[u]);
   }
-  const float2v w = pair_stats_max(stats, n_stats);
+  const float2v w = pair_stats_max(stats, n_stats, first);
   return pair_exponent(wave_max(top) * (w[0] * 1.01f) + w[1]);
 }
 

@@ -49,8 +49,8 @@ struct PairGemmArgs {
   int32_t* c_exp;
   int n_stats;
   int ldc, m_bound, n, k;
-  int tiles_n, tiles_n_all;                     // column tiles per group of B, and of all groups
-  int col_groups;                               // the tile order takes the column tiles in this many groups
+  int tiles_n, groups;                          // column tiles per group of B
+  int columns;                                  // the tile order takes the column tiles of all groups this many at a time
 };
 
 #define ET_LDS_PTR(p) ((__attribute__((address_space(3))) void*)(p))
@@ -83,22 +83,30 @@ struct PairTile {
 //   set under this one's MFMAs.
 // GELU: C = gelu(A.B + bias) as pair rows with their exponents in c_exp; otherwise C is float, + bias if given.
 template <int WM, int WN, int MI, int NJ, int ST, int KS, bool GELU>
-__global__ __launch_bounds__(WM * WN * kWave) void gemm_pair_kernel(PairGemmArgs args) {
+__global__ __launch_bounds__(WM * WN * kWave) void gemm_pair_kernel(
+    // what comes before the first request, as arguments of their own (gemm_f16_bt_kernel has the reason)
+    const _Float16* a0, const _Float16* b0, const int32_t* rows_dev, int m_bound, int N, int K, int tiles_n, int groups, int columns, PairGemmArgs args) {
 #if defined(__HIP_DEVICE_COMPILE__)   // device-only types in the body; the host pass only needs the stub
   using Tile = PairTile<WM, WN, MI, NJ, ST, KS>;
   constexpr int BM = Tile::BM, BN = Tile::BN;
   extern __shared__ __attribute__((aligned(1024))) unsigned char smem[];
 
-  const int rows = args.rows_dev ? min(*args.rows_dev, args.m_bound) : args.m_bound;
-  const int total = ((rows + BM - 1) / BM) * args.tiles_n_all;      // tiles that hold valid rows
+  int rows = rows_dev ? *rows_dev : m_bound;
+  uint64_t to_a1 = 0, to_a2 = 0, to_b1 = 0, to_b2 = 0;              // from the operands of the first group, in bytes
+  if (groups > 1) {
+    to_a1 = (uint64_t)args.A[1], to_a2 = (uint64_t)args.A[2], to_b1 = (uint64_t)args.B[1], to_b2 = (uint64_t)args.B[2];
+    asm volatile("" : "+s"(rows), "+s"(to_a1), "+s"(to_a2), "+s"(to_b1), "+s"(to_b2));       // all in one go
+    to_a1 -= (uint64_t)a0, to_a2 -= (uint64_t)a0, to_b1 -= (uint64_t)b0, to_b2 -= (uint64_t)b0;
+  }
+  rows = max(min(rows, m_bound), 0);
+  const int tiles_m = (int)((unsigned)(rows + BM - 1) / BM), total = tiles_m * tiles_n * groups;      // tiles that hold valid rows
   // workgroups are dealt round-robin to the XCDs: a contiguous band of tiles for each
   const int per_xcd = (total + kXcds - 1) / kXcds;
   const int xcd = blockIdx.x % kXcds, wgs = gridDim.x / kXcds;      // the grid is a multiple of 8
   const int n_loc = max(0, min(per_xcd, total - xcd * per_xcd));
   int idx = blockIdx.x / kXcds;
   if (idx >= n_loc) return;
-  const int N = args.n, K = args.k;
-  const int nst = K / (32 * KS);                                    // stages of a tile
+  const int nst = (int)((unsigned)K / (32 * KS));                                    // stages of a tile
   const uint32_t row_bytes = (uint32_t)K * 4u;
 
   const int lane = threadIdx.x & (kWave - 1);
@@ -113,19 +121,18 @@ __global__ __launch_bounds__(WM * WN * kWave) void gemm_pair_kernel(PairGemmArgs
   auto locate = [&](int i) {
     Src t;
     const int tile = xcd * per_xcd + i;
-    const int cpg = args.tiles_n_all / args.col_groups;
-    const int per_group = (total / args.tiles_n_all) * cpg;
-    const int cg = tile / per_group;
-    const int in_group = tile - cg * per_group;
-    const int tm = in_group / cpg;
-    const int tn_all = cg * cpg + (in_group - tm * cpg);
-    t.grp = tn_all / args.tiles_n;
+    const int cg = columns == tiles_n * groups ? 0 : uniform_div(tile, tiles_m * columns), in_group = tile - cg * tiles_m * columns;
+    const int tm = uniform_div(in_group, columns);
+    const int tn_all = cg * columns + (in_group - tm * columns);
+    t.grp = groups == 1 ? 0 : 2 - uniform_less(tn_all, tiles_n) - uniform_less(tn_all, 2 * tiles_n);
     t.m0 = tm * BM;
-    t.n0 = (tn_all - t.grp * args.tiles_n) * BN;
+    t.n0 = (tn_all - t.grp * tiles_n) * BN;
+    const uint64_t second = t.grp == 1 ? ~0ull : 0ull, third = t.grp == 2 ? ~0ull : 0ull;
+    const char *ptr_a = (const char*)a0 + ((to_a1 & second) | (to_a2 & third)), *ptr_b = (const char*)b0 + ((to_b1 & second) | (to_b2 & third));
     // rows at or beyond the valid count and columns at or beyond n read as zero
-    t.a = __builtin_amdgcn_make_buffer_rsrc(const_cast<char*>((const char*)args.A[t.grp] + (size_t)t.m0 * row_bytes), 0,
+    t.a = __builtin_amdgcn_make_buffer_rsrc(const_cast<char*>(ptr_a + (size_t)t.m0 * row_bytes), 0,
                                             min(rows - t.m0, BM) * (int)row_bytes, 0x00020000);
-    t.b = __builtin_amdgcn_make_buffer_rsrc(const_cast<char*>((const char*)args.B[t.grp] + (size_t)t.n0 * row_bytes), 0,
+    t.b = __builtin_amdgcn_make_buffer_rsrc(const_cast<char*>(ptr_b + (size_t)t.n0 * row_bytes), 0,
                                             min(N - t.n0, BN) * (int)row_bytes, 0x00020000);
     return t;
   };
@@ -211,6 +218,10 @@ __global__ __launch_bounds__(WM * WN * kWave) void gemm_pair_kernel(PairGemmArgs
   Src cur = locate(idx), nxt = cur;
 #pragma unroll
   for (int s = 0; s < ST; ++s) issue_stage(s, min(s, nst - 1), cur, cur);
+  // GELU: what bounds the rows of C, the same for every row.  Small tiles look at it, and at all that the epilogue reads, behind
+  // the k loop: their launches take little longer than a round trip or two.
+  float2v bounds = {0.f, 0.f}, stats[8];
+  if constexpr (GELU) pair_stats_request(args.b_stats, args.n_stats, 0, stats);
   wait_vmcnt<KS * Tile::DMA*(ST - 1)>();
   barrier_only();
   auto read_set = [&](half8 (&a)[2][2][MI], half8 (&b)[2][2][NJ], int slot) {
@@ -229,9 +240,7 @@ __global__ __launch_bounds__(WM * WN * kWave) void gemm_pair_kernel(PairGemmArgs
     read_set(pa[0], pb[0], 0);
   }
 
-  // GELU: what bounds the rows of C, the same for every row
-  float2v bounds = {0.f, 0.f};
-  if constexpr (GELU) bounds = pair_stats_max(args.b_stats, args.n_stats);
+  if constexpr (GELU && Tile::BIG) bounds = pair_stats_max(args.b_stats, args.n_stats, stats);
 
   int s = 0;                                     // slot of the current stage
   bool first_tile = true;
@@ -244,6 +253,26 @@ __global__ __launch_bounds__(WM * WN * kWave) void gemm_pair_kernel(PairGemmArgs
 #pragma unroll
       for (int j = 0; j < NJ; ++j) sum[i][j] = acc[i][j] = zero;
     const int col = cur.n0 + wn * 16 * NJ + l16 * NJ;
+    typedef float fvec __attribute__((ext_vector_type(NJ)));
+    typedef int int4v __attribute__((ext_vector_type(4)));
+    fvec bias = {};
+    int ce[NJ] = {};
+    int4v re[MI] = {};
+    float4v bound[MI] = {};
+    const int row0 = cur.m0 + wm * 16 * MI + g * 4;
+    auto request = [&](const int32_t* a_exp, const int32_t* b_exp, const float* add, const float* norm) {
+      if (col >= N) return;
+#pragma unroll
+      for (int j = 0; j < NJ; ++j) ce[j] = b_exp[col + j];
+      if (add != nullptr) bias = *reinterpret_cast<const fvec*>(add + col);
+      // (the row arrays reach beyond the last tile: PairRows)
+#pragma unroll
+      for (int i = 0; i < MI; ++i) {
+        re[i] = *reinterpret_cast<const int4v*>(a_exp + row0 + i * 16);
+        if constexpr (GELU) bound[i] = *reinterpret_cast<const float4v*>(norm + row0 + i * 16);
+      }
+    };
+    if constexpr (!Tile::BIG) request(args.a_exp[cur.grp], args.b_exp[cur.grp], args.bias[cur.grp], args.a_norm);
     if constexpr (Tile::BIG) {
       auto step = [&](auto Pc, int t) {
         constexpr int P = decltype(Pc)::value;
@@ -320,36 +349,23 @@ __global__ __launch_bounds__(WM * WN * kWave) void gemm_pair_kernel(PairGemmArgs
     }
     wait_vmcnt<0>();
 
+    if constexpr (Tile::BIG) request(args.a_exp[cur.grp], args.b_exp[cur.grp], args.bias[cur.grp], args.a_norm);
+    // the loads are waited for here: left pending on the paths that store nothing, they would have the compiler put a wait
+    // for every outstanding load, the DMA included, in front of the k loop's reuse of their registers
+#pragma unroll
+    for (int j = 0; j < NJ; ++j) {
+      float b = bias[j];
+      asm volatile("" : "+v"(b), "+v"(ce[j]));
+      bias[j] = b;
+    }
+#pragma unroll
+    for (int i = 0; i < MI; ++i) {
+      asm volatile("" : "+v"(re[i]));
+      if constexpr (GELU) asm volatile("" : "+v"(bound[i]));
+    }
+    if constexpr (GELU && !Tile::BIG)
+      if (first_tile) bounds = pair_stats_max(args.b_stats, args.n_stats, stats);
     if (col < N) {
-      typedef float fvec __attribute__((ext_vector_type(NJ)));
-      fvec bias = {};
-      int ce[NJ];
-#pragma unroll
-      for (int j = 0; j < NJ; ++j) ce[j] = args.b_exp[cur.grp][col + j];
-      if (args.bias[cur.grp] != nullptr) bias = *reinterpret_cast<const fvec*>(args.bias[cur.grp] + col);
-      // (the row arrays reach beyond the last tile: PairRows)
-      typedef int int4v __attribute__((ext_vector_type(4)));
-      int4v re[MI];
-      float4v bound[MI];
-      const int row0 = cur.m0 + wm * 16 * MI + g * 4;
-#pragma unroll
-      for (int i = 0; i < MI; ++i) {
-        re[i] = *reinterpret_cast<const int4v*>(args.a_exp[cur.grp] + row0 + i * 16);
-        if constexpr (GELU) bound[i] = *reinterpret_cast<const float4v*>(args.a_norm + row0 + i * 16);
-      }
-      // the loads are waited for here: left pending on the paths that store nothing, they would have the compiler put a wait
-      // for every outstanding load, the DMA included, in front of the k loop's reuse of their registers
-#pragma unroll
-      for (int j = 0; j < NJ; ++j) {
-        float b = bias[j];
-        asm volatile("" : "+v"(b), "+v"(ce[j]));
-        bias[j] = b;
-      }
-#pragma unroll
-      for (int i = 0; i < MI; ++i) {
-        asm volatile("" : "+v"(re[i]));
-        if constexpr (GELU) asm volatile("" : "+v"(bound[i]));
-      }
 #pragma unroll
       for (int i = 0; i < MI; ++i)
 #pragma unroll
@@ -420,19 +436,20 @@ template <int WM, int WN, int MI, int NJ, int ST, int KS>
 void launch_tile(PairGemmArgs a, bool gelu, int groups, hipStream_t stream) {
   using Tile = PairTile<WM, WN, MI, NJ, ST, KS>;
   a.tiles_n = (a.n + Tile::BN - 1) / Tile::BN;
-  a.tiles_n_all = a.tiles_n * groups;
+  a.groups = groups;
+  const int tiles_n_all = a.tiles_n * groups;
   // The workgroups of an XCD advance through k side by side, so what its L2 has to deliver per k-step is the distinct
   // rows of A and columns of B they touch: about square blocks of tiles are the best.  Wide outputs take their column
   // tiles in groups of about 1024 columns.
-  a.col_groups = 1;
-  for (int c = 2; c <= a.tiles_n_all; ++c)
-    if (a.tiles_n_all % c == 0 && a.tiles_n_all / c * Tile::BN >= 768) a.col_groups = c;
-  const int tiles = ((a.m_bound + Tile::BM - 1) / Tile::BM) * a.tiles_n_all;
+  a.columns = tiles_n_all;
+  for (int c = 2; c <= tiles_n_all; ++c)
+    if (tiles_n_all % c == 0 && tiles_n_all / c * Tile::BN >= 768) a.columns = tiles_n_all / c;
+  const int tiles = ((a.m_bound + Tile::BM - 1) / Tile::BM) * tiles_n_all;
   // (a stream of fewer stages than the ring holds must not cross into a second tile)
   const int grid = ((a.k / (32 * KS) < ST ? tiles : std::min(tiles, device_cu_count())) + kXcds - 1) / kXcds * kXcds;
   auto go = [&](auto kern) {
     allow_dynamic_lds(reinterpret_cast<const void*>(kern), Tile::SMEM);
-    kern<<<grid, Tile::THREADS, Tile::SMEM, stream>>>(a);
+    kern<<<grid, Tile::THREADS, Tile::SMEM, stream>>>(a.A[0], a.B[0], a.rows_dev, a.m_bound, a.n, a.k, a.tiles_n, groups, a.columns, a);
   };
   if (gelu) go(gemm_pair_kernel<WM, WN, MI, NJ, ST, KS, true>);
   else go(gemm_pair_kernel<WM, WN, MI, NJ, ST, KS, false>);
