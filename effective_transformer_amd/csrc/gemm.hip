@@ -14,6 +14,7 @@
 //
 // The M dimension (valid tokens) may live on the device: tiles beyond *rows_dev exit, the last tile
 // is predicated.  Up to three column groups (Q/K/V) share one launch.
+#include <climits>
 #include <algorithm>
 #include <atomic>
 
@@ -35,12 +36,11 @@ struct GemmArgs {
   int ldc, m_bound, n, k, groups;
   int tiles_m, tiles_n;      // tiles_n per group
   int per_xcd;               // workgroups per XCD slot of the launch
-  int reverse_walk = 0;      // persistent kernel: walk the tiles from the last one
+  int reverse_walk = 0;      // persistent kernels: walk the tiles from the last one
   int gelu = 0;              // C = gelu(A.B + bias) instead of A.B + bias (bias must be set)
   int a_blocked = 0;         // pair kernel: A / C hold every tile of 256 rows as blocks of [256 rows][64 columns]
   int c_blocked = 0;         //   (see GemmGroups)
   int c_cached = 0;          // persistent k-contiguous kernel: plain stores for C instead of non-temporal ones
-  int col_groups = 1;        // persistent k-contiguous kernel: the tile order takes the column tiles in this many groups
 };
 
 typedef uint32_t uint4v __attribute__((ext_vector_type(4)));
@@ -545,6 +545,37 @@ constexpr int kQSmemA3 = 3 * kQAPair + 2 * (kQPair - kQAPair);   // 160 KB: thre
 
 __device__ __forceinline__ int pair_swizzle(int row) { return (row >> 1) & 7; }
 
+// What a workgroup needs before its first request, as kernel arguments of their own in front of the rest: the hardware can hand
+// the first 14 words of a launch's arguments over in registers, and read as members of GemmArgs where they are used they came in
+// a chain of four or more dependent scalar loads, with divisions between them: 0.3 to 0.7 us in front of the first request (the four
+// products of BERT-base on 100 rows 22.9 -> 22.0 us, on 500 rows 33.7 -> 31.1, on 1024 43.7 -> 40.5, on 11501 177.7 -> 172.9).
+// how the persistent kernel walks its tiles: flags, and the workgroups per XCD above them
+constexpr int kWalkReverse = 1, kWalkBlockedA = 2, kWalkWgs = 2;
+#define ET_HEAD_ARGS const void *a0, const void *b0, const int32_t *rows_dev, int m_bound, int n, int k, int groups, int tiles_n, int columns, int walk
+struct TileHead {
+  const char *a, *b;                           // operands of the first group, and from there to the others' in bytes
+  uint64_t to_a1, to_b1, to_a2, to_b2;
+  int rows, n, k, groups;
+
+  __device__ __forceinline__ const char* a_of(int grp) const { return a + ((to_a1 & -(uint64_t)(grp == 1)) | (to_a2 & -(uint64_t)(grp == 2))); }
+  __device__ __forceinline__ const char* b_of(int grp) const { return b + ((to_b1 & -(uint64_t)(grp == 1)) | (to_b2 & -(uint64_t)(grp == 2))); }
+};
+// The row count and, for several groups, their operands, read in one go.
+__device__ __forceinline__ TileHead tile_head(const void* a0, const void* b0, const int32_t* rows_dev, int m_bound, int n, int k, int groups,
+                                              const GemmArgs& args) {
+  TileHead h{(const char*)a0, (const char*)b0, 0, 0, 0, 0, 0, n, k, groups};
+  int rows = rows_dev ? *rows_dev : m_bound;
+  if (groups > 1) {
+    h.to_a1 = (uint64_t)args.A[1], h.to_b1 = (uint64_t)args.B[1], h.to_a2 = (uint64_t)args.A[2], h.to_b2 = (uint64_t)args.B[2];
+#if defined(__HIP_DEVICE_COMPILE__)
+    asm volatile("" : "+s"(rows), "+s"(h.to_a1), "+s"(h.to_b1), "+s"(h.to_a2), "+s"(h.to_b2));   // not later, one by one
+#endif
+    h.to_a1 -= (uint64_t)a0, h.to_b1 -= (uint64_t)b0, h.to_a2 -= (uint64_t)a0, h.to_b2 -= (uint64_t)b0;
+  }
+  h.rows = max(min(rows, m_bound), 0);
+  return h;
+}
+
 // MI: 16-row blocks per wave, i.e. tiles of 32 MI rows (256, 224, 192 or 160).  The tile count of a launch rarely
 // fills whole rounds of the chip; a lower tile can turn "one round and a bit" into one round (launch_f16_persistent
 // chooses).  The A part of an LDS slot keeps its 256 rows; the rows beyond the tile lie outside the tile's buffer
@@ -555,34 +586,31 @@ __device__ __forceinline__ int pair_swizzle(int row) { return (row >> 1) & 7; }
 // of their first use instead of two (B^T as before).  For the projection whose A is the big matrix and comes from
 // HBM (k >= 2048: FFN-down), where a pair's time does not cover that latency.  Same instructions on the same data in
 // the same order: same bits.
-template <bool GELU, int MI, bool NT, bool A3 = false>
-__global__ __launch_bounds__(kPThreads) void gemm_f16_pair_kernel(GemmArgs args) {
+template <bool GELU, int MI, bool NT, bool A3>
+__device__ __forceinline__ void pair_tiles(const TileHead& head, int tiles_n, int columns, int walk, const GemmArgs& args, unsigned char* smem) {
 #if defined(__HIP_DEVICE_COMPILE__)   // device-only types in the body; the host pass only needs the stub
-  extern __shared__ __attribute__((aligned(1024))) unsigned char smem[];
   const int tid = threadIdx.x;
   const int lane = tid & (kWave - 1);
   const int wave = __builtin_amdgcn_readfirstlane(tid / kWave);   // 0..7, scalar
   constexpr int BM = 32 * MI;                                     // rows of a tile
   const int wm = wave & 1, wn = (wave >> 1) & 3;                  // (16 MI)-row half, 64-column quarter of the tile
   const int l16 = lane & 15, g = lane >> 4;
-  const int N = args.n, K = args.k;
-  const int np = K / 64;                                          // pairs of k-steps per tile, >= 2
+  const int rows = head.rows, N = head.n, K = head.k;
+  const int np = (int)((unsigned)K / 64);                         // pairs of k-steps per tile, >= 2
+  const bool a_blocked = walk & kWalkBlockedA;
 
-  const int rows = args.rows_dev ? min(*args.rows_dev, args.m_bound) : args.m_bound;
-  const int tiles_n_all = args.tiles_n * args.groups;
-  const int total = ((rows + BM - 1) / BM) * tiles_n_all;     // tiles that hold valid rows (a prefix in tile order)
+  const int tiles_n_all = tiles_n * head.groups;
+  const int tiles_m = (int)((unsigned)(rows + BM - 1) / BM), total = tiles_m * tiles_n_all;   // tiles that hold valid rows (a prefix in tile order)
   const int per_xcd = (total + kXcds - 1) / kXcds;
   const int xcd = blockIdx.x % kXcds;
-  const int G = gridDim.x;                                        // multiple of 8
-
   // This XCD's band holds n_loc tiles for wgs workgroups: `full` of them fill whole rounds.  When the rest would keep at
   // most half of the workgroups busy for a last round, each of those tiles is shared by two workgroups, one per
   // 128-column half: the waves of the other half only keep the operand stream going, a SIMD then has one MFMA wave
   // instead of two, and the last round takes about half a tile time.  Every element is still accumulated by one wave in
   // the same k order, so the bits do not depend on the split.
-  const int wgs = G / kXcds, local = blockIdx.x / kXcds;
+  const int wgs = walk >> kWalkWgs, local = blockIdx.x / kXcds;
   const int n_loc = max(0, min(per_xcd, total - xcd * per_xcd));
-  const int full = (n_loc / wgs) * wgs, rem = n_loc - full;
+  const int rounds = uniform_div(n_loc, wgs), full = rounds * wgs, rem = n_loc - full;
   const bool split = rem > 0 && 2 * rem <= wgs;
   // slot s (= local + round * wgs) of the band -> tile and half (-1: the whole tile)
   auto valid = [&](int s) { return s < full || (split ? s - full < 2 * rem : s < n_loc); };
@@ -599,24 +627,22 @@ __global__ __launch_bounds__(kPThreads) void gemm_f16_pair_kernel(GemmArgs args)
       t.half = (s - full) & 1;
       tile = xcd * per_xcd + full + ((s - full) >> 1);
     }
-    if (args.reverse_walk) tile = total - 1 - tile;
-    // column groups: the tile order runs through all row tiles of the first tiles_n_all / col_groups column tiles,
-    // then through those of the next group
-    const int cpg = tiles_n_all / args.col_groups;
-    const int per_group = (total / tiles_n_all) * cpg;
-    const int cg = tile / per_group;
+    if (walk & kWalkReverse) tile = total - 1 - tile;
+    // column groups: the tile order runs through all row tiles of the first `columns` column tiles, then through those of the
+    // next group
+    const int per_group = tiles_m * columns, cg = columns == tiles_n_all ? 0 : uniform_div(tile, per_group);
     const int r = tile - cg * per_group;
-    const int tm = r / cpg;
-    const int tn_all = cg * cpg + (r - tm * cpg);
-    t.grp = tn_all / args.tiles_n;
+    const int tm = uniform_div(r, columns);
+    const int tn_all = cg * columns + (r - tm * columns);
+    t.grp = head.groups == 1 ? 0 : 2 - uniform_less(tn_all, tiles_n) - uniform_less(tn_all, 2 * tiles_n);
     t.m0 = tm * BM;
-    t.n0 = (tn_all - t.grp * args.tiles_n) * kPBN;
+    t.n0 = (tn_all - t.grp * tiles_n) * kPBN;
     // a blocked A holds whole tiles: rows beyond the valid count are there (written by the producer from zero rows)
     t.a = __builtin_amdgcn_make_buffer_rsrc(
-        const_cast<_Float16*>((const _Float16*)args.A[t.grp] + (size_t)t.m0 * K), 0,
-        (args.a_blocked ? BM : min(rows - t.m0, BM)) * K * 2, 0x00020000);
+        const_cast<char*>(head.a_of(t.grp) + (size_t)t.m0 * K * 2), 0,
+        (a_blocked ? BM : min(rows - t.m0, BM)) * K * 2, 0x00020000);
     t.b = __builtin_amdgcn_make_buffer_rsrc(
-        const_cast<_Float16*>((const _Float16*)args.B[t.grp] + (size_t)t.n0 * K), 0, min(N - t.n0, kPBN) * K * 2, 0x00020000);
+        const_cast<char*>(head.b_of(t.grp) + (size_t)t.n0 * K * 2), 0, min(N - t.n0, kPBN) * K * 2, 0x00020000);
     return t;
   };
 
@@ -629,12 +655,12 @@ __global__ __launch_bounds__(kPThreads) void gemm_f16_pair_kernel(GemmArgs args)
     const int row = wave * 32 + j * 8 + (lane >> 3);
     const int c = (lane & 7) ^ pair_swizzle(row);
     // blocked A: the 128 bytes of a row and pair lie 128 bytes from the next row's, a pair is one block of 32 KB
-    voff_a[j] = args.a_blocked ? (uint32_t)row * 128u + (uint32_t)c * 16u
+    voff_a[j] = a_blocked ? (uint32_t)row * 128u + (uint32_t)c * 16u
                                : ((uint32_t)row * (uint32_t)K + (uint32_t)c * 8u) * 2u;
     const int col = (row & ~63) + (row & 15) * 4 + ((row >> 4) & 3);
     voff_b[j] = ((uint32_t)col * (uint32_t)K + (uint32_t)c * 8u) * 2u;
   }
-  const int a_pair_bytes = args.a_blocked ? kQAPair : 128;       // from one pair of k-steps of A to the next
+  const int a_pair_bytes = a_blocked ? kQAPair : 128;       // from one pair of k-steps of A to the next
   // LDS: slot s = A rows, then B^T rows of a pair (two slots); with A3 a ring of three A slots, then two B^T slots
   auto a_slot = [&](int sa) -> unsigned char* { return smem + sa * (A3 ? kQAPair : kQPair); };
   auto b_slot = [&](int sb) -> unsigned char* {
@@ -674,7 +700,7 @@ __global__ __launch_bounds__(kPThreads) void gemm_f16_pair_kernel(GemmArgs args)
     // moments.  Those that walk one tile less than the others have a tile time to spare: they start late, spread over
     // about a quarter of a tile time (960 cycles per pair of k-steps), which takes their traffic out of step with the
     // rest at no cost to the last round (measured: -1.3 % on the encoder step, nothing gained beyond that spread).
-    const int max_tiles = (n_loc + wgs - 1) / wgs;
+    const int max_tiles = rounds + (rem > 0 ? 1 : 0);
     // first workgroup of this XCD with max_tiles - 1 tiles
     const int first_short = split ? 2 * rem : n_loc - (max_tiles - 1) * wgs;
     if (local >= first_short && first_short < wgs) {
@@ -853,6 +879,50 @@ __global__ __launch_bounds__(kPThreads) void gemm_f16_pair_kernel(GemmArgs args)
 #endif
 }
 
+template <bool GELU, int MI, bool NT, bool A3 = false>
+__global__ __launch_bounds__(kPThreads) void gemm_f16_pair_kernel(ET_HEAD_ARGS, GemmArgs args) {
+  extern __shared__ __attribute__((aligned(1024))) unsigned char smem[];
+  pair_tiles<GELU, MI, NT, A3>(tile_head(a0, b0, rows_dev, m_bound, n, k, groups, args), tiles_n, columns, walk, args, smem);
+}
+
+// Tile height of a launch of `wgs` workgroups per XCD, as 16-row blocks per wave: see launch_f16_persistent.
+__host__ __device__ inline int pair_row_blocks(int rows, int tiles_n, int wgs) {
+  // (in twentieths of a round; a rest of at most half the workgroups is shared, two workgroups per tile)
+  auto cost = [&](int mi) {
+    const long tiles = (long)((rows + 32 * mi - 1) / (32 * mi)) * tiles_n;
+    const int n_loc = (int)((tiles + kXcds - 1) / kXcds), full = n_loc / wgs, rem = n_loc - full * wgs;
+    return (full * 20 + (rem == 0 ? 0 : (2 * rem <= wgs ? 11 : 20))) * (mi + 21);
+  };
+  const int cost8 = cost(8);
+  int best = cost8, best_mi = 8;
+#pragma unroll
+  for (int mi = 7; mi >= 5; --mi) {
+    const int c = cost(mi);
+    if (100l * c < 97l * cost8 && c < best) {
+      best = c;
+      best_mi = mi;
+    }
+  }
+  return best_mi;
+}
+
+// The tile height for the row count that only the device knows (a height for the launch's bound of 11501 rows takes 34 us for the
+// Q/K/V projection of the 7161 rows that are there, the right one 27; FFN-down of 9526 out of 16384: 54 and 45 us).
+template <bool GELU, bool NT, bool A3>
+__global__ __launch_bounds__(kPThreads) void gemm_f16_pair_rows_kernel(ET_HEAD_ARGS, GemmArgs args) {
+  extern __shared__ __attribute__((aligned(1024))) unsigned char smem[];
+  const TileHead head = tile_head(a0, b0, rows_dev, m_bound, n, k, groups, args);
+  // (below 128 tiles of 256 rows, where this kernel would not run if the host knew, the lowest tile: FFN-down of 7161 rows 47 us,
+  // 51 on shared tiles of 192)
+  const bool few = (int)((unsigned)(head.rows + 255) / 256) * tiles_n * groups < 128;
+  switch (few ? 5 : pair_row_blocks(head.rows, tiles_n * groups, walk >> kWalkWgs)) {
+    case 8: return pair_tiles<GELU, 8, NT, A3>(head, tiles_n, columns, walk, args, smem);
+    case 7: return pair_tiles<GELU, 7, NT, A3>(head, tiles_n, columns, walk, args, smem);
+    case 6: return pair_tiles<GELU, 6, NT, false>(head, tiles_n, columns, walk, args, smem);
+    default: return pair_tiles<GELU, 5, NT, false>(head, tiles_n, columns, walk, args, smem);
+  }
+}
+
 // ------------------------------------------------------------------------------------------
 // fp16, problems below the persistent regime, B k-contiguous ([n][k]): one (32 MI) x (32 NJ) tile per workgroup,
 // 4 wavefronts (2 x 2), LDS slots of two k-steps like the persistent kernel above.  MI = 1 .. 4 blocks of 32 rows,
@@ -874,10 +944,17 @@ struct BtTile {
   static constexpr int DMA = MI + NJ;                         // instructions per wavefront and pair: MI for A, NJ for B^T
 };
 
-// COLUMNS: the tile order runs down the columns of tiles instead of along the rows (see band_rows); a template parameter,
-// because the choice at run time would put 0.3 us in front of the first request of every launch.
-template <int MI, int NJ, int ST, bool COLUMNS>
-__global__ __launch_bounds__(kHThreads) __attribute__((amdgpu_waves_per_eu(2))) void gemm_f16_bt_kernel(GemmArgs args) {
+// The tiles (row blocks, column blocks, two workgroups per CU) and the slots of their rings.
+#define ET_BT_TILES(X)                                                                                              \
+  X(1, 1, 0, 5) X(1, 2, 0, 5) X(1, 2, 1, 3) X(2, 2, 0, 4) X(2, 2, 1, 3) X(2, 4, 0, 4) X(2, 4, 1, 3) X(3, 2, 0, 4) \
+  X(3, 2, 1, 3) X(3, 4, 0, 4) X(3, 4, 1, 2) X(3, 6, 0, 3) X(3, 6, 1, 2) X(4, 2, 0, 4) X(4, 2, 1, 3) X(4, 4, 0, 4)  \
+  X(4, 4, 1, 2) X(4, 6, 0, 3) X(4, 6, 1, 2) X(4, 8, 0, 3)
+// those of them with a CU to themselves that gemm_f16_bt_rows_kernel chooses from (128 x 256 would cost all of them registers)
+#define ET_BT_ROWS_TILES(X) X(1, 1, 0, 5) X(1, 2, 0, 5) X(2, 2, 0, 4) X(2, 4, 0, 4) X(3, 2, 0, 4) X(3, 4, 0, 4) X(3, 6, 0, 3) X(4, 2, 0, 4) X(4, 4, 0, 4) X(4, 6, 0, 3)
+
+// The tile in row `tm` and column `tn_all` of tiles, whose columns run through the groups; `tiles_n` of them to a group.
+template <int MI, int NJ, int ST>
+__device__ __forceinline__ void bt_tile(const TileHead& head, int tiles_n, const GemmArgs& args, int tm, int tn_all, unsigned char* smem) {
 #if defined(__HIP_DEVICE_COMPILE__)   // device-only types in the body; the host pass only needs the stub
   using Tile = BtTile<MI, NJ, ST>;
   static_assert(Tile::DMA * (ST - 1) < 64, "the DMA instructions in flight must fit the 6-bit vmcnt");
@@ -885,26 +962,11 @@ __global__ __launch_bounds__(kHThreads) __attribute__((amdgpu_waves_per_eu(2))) 
   using HalfN = typename std::conditional<NJ == 8, half8, typename std::conditional<NJ == 4, half4,
                                           typename std::conditional<NJ == 1, half1v, half2v>::type>::type>::type;
   constexpr int BM = Tile::BM, BN = Tile::BN, WC = 16 * NJ;       // WC: columns of a wave tile
-  extern __shared__ __attribute__((aligned(1024))) unsigned char smem[];
-
-  const int rows = args.rows_dev ? min(*args.rows_dev, args.m_bound) : args.m_bound;
-  const int tiles_n_all = args.tiles_n * args.groups;
-  const int tile = remap_valid_tile(blockIdx.x, ((rows + BM - 1) / BM) * tiles_n_all);
-  if (tile < 0) return;
-  int tm, tn_all;
-  if constexpr (COLUMNS) {
-    const int tiles_m = (rows + BM - 1) / BM;
-    tn_all = tile / tiles_m;
-    tm = tile - tn_all * tiles_m;
-  } else {
-    tm = tile / tiles_n_all;
-    tn_all = tile - tm * tiles_n_all;
-  }
-  const int grp = tn_all / args.tiles_n;
+  const int rows = head.rows, N = head.n, K = head.k;
+  const int grp = head.groups == 1 ? 0 : 2 - uniform_less(tn_all, tiles_n) - uniform_less(tn_all, 2 * tiles_n);
   const int m0 = tm * BM;
-  const int n0 = (tn_all - grp * args.tiles_n) * BN;
-  const int N = args.n, K = args.k;
-  const int np = K / 64;                                          // pairs of k-steps
+  const int n0 = (tn_all - grp * tiles_n) * BN;
+  const int np = (int)((unsigned)K / 64);                         // pairs of k-steps
 
   const int tid = threadIdx.x;
   const int lane = tid & (kWave - 1);
@@ -915,9 +977,9 @@ __global__ __launch_bounds__(kHThreads) __attribute__((amdgpu_waves_per_eu(2))) 
   // descriptors start at the tile and end with the matrix: rows at or beyond the valid-token count and columns at or
   // beyond n read as zero, and lane offsets do not grow with the matrices
   const __amdgpu_buffer_rsrc_t rsrc_a = __builtin_amdgcn_make_buffer_rsrc(
-      const_cast<_Float16*>((const _Float16*)args.A[grp] + (size_t)m0 * K), 0, min(rows - m0, BM) * K * 2, 0x00020000);
+      const_cast<char*>(head.a_of(grp) + (size_t)m0 * K * 2), 0, min(rows - m0, BM) * K * 2, 0x00020000);
   const __amdgpu_buffer_rsrc_t rsrc_b = __builtin_amdgcn_make_buffer_rsrc(
-      const_cast<_Float16*>((const _Float16*)args.B[grp] + (size_t)n0 * K), 0, min(N - n0, BN) * K * 2, 0x00020000);
+      const_cast<char*>(head.b_of(grp) + (size_t)n0 * K * 2), 0, min(N - n0, BN) * K * 2, 0x00020000);
 
   // DMA: one instruction fills 1 KB of LDS = 8 rows x 128 bytes; the lane picks the 16-byte chunk that belongs at its
   // (XOR-swizzled) position.  LDS row j*16+l of a wave's column group holds column NJ*l+j of the group, so that the
@@ -991,6 +1053,19 @@ __global__ __launch_bounds__(kHThreads) __attribute__((amdgpu_waves_per_eu(2))) 
   for (int s = 0; s < ST; ++s)
 #pragma unroll
     for (int q = 0; q < Tile::DMA; ++q) issue1(s, s, q);
+  // The bias of the lane's columns is read here, behind the first requests: where it is cold, in the epilogue it would add its
+  // way from memory to the launch.  Without a bias the addend is -0, which leaves every value (and the sign of a zero) as it is.
+  const int col = n0 + wn * WC + l16 * (NJ == 6 ? 4 : NJ), col2 = n0 + wn * WC + 64 + l16 * 2;   // col2: NJ = 6 only
+  constexpr int NB = NJ == 6 ? 4 : NJ;
+  using BiasN = typename std::conditional<NJ == 6, half4, HalfN>::type;
+  BiasN biasv;
+  half2v bias2 = {(_Float16)-0.0f, (_Float16)-0.0f};
+#pragma unroll
+  for (int j = 0; j < NB; ++j) biasv[j] = (_Float16)-0.0f;
+  if (const _Float16* bias = (const _Float16*)args.bias[grp]; bias != nullptr && col < N) {
+    biasv = *reinterpret_cast<const BiasN*>(bias + col);
+    if (NJ == 6 && col2 < N) bias2 = *reinterpret_cast<const half2v*>(bias + col2);
+  }
   wait_vmcnt<Tile::DMA * (ST - 1)>();
   barrier_only();
 #pragma unroll
@@ -1014,16 +1089,10 @@ __global__ __launch_bounds__(kHThreads) __attribute__((amdgpu_waves_per_eu(2))) 
   // epilogue: lane owns rows g*4+r of every 16-row block and NJ consecutive columns.  Plain stores, not the
   // non-temporal ones of the persistent kernel: the output of a launch this small is still in the caches when the
   // next kernel reads it (12 layers on 2000 tokens: 0.905 -> 0.843 ms; no difference from about 4000 tokens on).
-  const int col = n0 + wn * WC + l16 * (NJ == 6 ? 4 : NJ);
   if (col < N) {
     _Float16* C = (_Float16*)args.C + (size_t)grp * N + col;
     if constexpr (NJ == 1 || NJ == 2 || NJ == 4 || NJ == 8) {
-      // bias added in half on the rounded product, as the reference's next kernel does; without a bias the addend is
-      // -0, which leaves every value (and the sign of a zero) as it is
-      HalfN biasv;
-#pragma unroll
-      for (int j = 0; j < NJ; ++j) biasv[j] = (_Float16)-0.0f;
-      if (args.bias[grp] != nullptr) biasv = *reinterpret_cast<const HalfN*>((const _Float16*)args.bias[grp] + col);
+      // bias added in half on the rounded product, as the reference's next kernel does
 #pragma unroll
       for (int i = 0; i < MI; ++i)
 #pragma unroll
@@ -1040,14 +1109,8 @@ __global__ __launch_bounds__(kHThreads) __attribute__((amdgpu_waves_per_eu(2))) 
     } else {
       // 6 columns per lane: 4 consecutive ones in the first 64 columns of the wave tile, 2 in the last 32
       static_assert(NJ == 6, "wave tiles are 32, 64, 96 or 128 columns wide");
-      _Float16* C2 = C - col + n0 + wn * WC + 64 + l16 * 2;
-      half4 bias4 = {(_Float16)-0.0f, (_Float16)-0.0f, (_Float16)-0.0f, (_Float16)-0.0f};
-      half2v bias2 = {(_Float16)-0.0f, (_Float16)-0.0f};
-      const bool ok2 = n0 + wn * WC + 64 + l16 * 2 < N;
-      if (args.bias[grp] != nullptr) {
-        bias4 = *reinterpret_cast<const half4*>((const _Float16*)args.bias[grp] + col);
-        if (ok2) bias2 = *reinterpret_cast<const half2v*>((const _Float16*)args.bias[grp] + n0 + wn * WC + 64 + l16 * 2);
-      }
+      _Float16* C2 = C - col + col2;
+      const bool ok2 = col2 < N;
 #pragma unroll
       for (int i = 0; i < MI; ++i)
 #pragma unroll
@@ -1056,7 +1119,7 @@ __global__ __launch_bounds__(kHThreads) __attribute__((amdgpu_waves_per_eu(2))) 
           if (row < rows) {
             half4 o4 = {f2h(acc[i][0][r]), f2h(acc[i][1][r]), f2h(acc[i][2][r]), f2h(acc[i][3][r])};
             half2v o2 = {f2h(acc[i][4][r]), f2h(acc[i][5][r])};
-            o4 = args.gelu ? bias_gelu_half<half4, 4>(o4, bias4) : o4 + bias4;
+            o4 = args.gelu ? bias_gelu_half<half4, 4>(o4, biasv) : o4 + biasv;
             o2 = args.gelu ? bias_gelu_half<half2v, 2>(o2, bias2) : o2 + bias2;
             *reinterpret_cast<half4*>(C + (size_t)row * args.ldc) = o4;
             if (ok2) *reinterpret_cast<half2v*>(C2 + (size_t)row * args.ldc) = o2;
@@ -1067,6 +1130,55 @@ __global__ __launch_bounds__(kHThreads) __attribute__((amdgpu_waves_per_eu(2))) 
 #else
   (void)args;
 #endif
+}
+
+// COLUMNS: the tile order runs down the columns of tiles instead of along the rows (see band_rows).
+template <int MI, int NJ, int ST, bool COLUMNS>
+__global__ __launch_bounds__(kHThreads) __attribute__((amdgpu_waves_per_eu(2))) void gemm_f16_bt_kernel(ET_HEAD_ARGS, GemmArgs args) {
+  extern __shared__ __attribute__((aligned(1024))) unsigned char smem[];
+  const TileHead head = tile_head(a0, b0, rows_dev, m_bound, n, k, groups, args);
+  const int tiles_n_all = tiles_n * groups, tiles_m = (int)((unsigned)(head.rows + 32 * MI - 1) / (32 * MI));
+  const int tile = remap_valid_tile(blockIdx.x, tiles_m * tiles_n_all);
+  if (tile < 0) return;
+  const int by = COLUMNS ? tiles_m : tiles_n_all, outer = uniform_div(tile, by), inner = tile - outer * by;
+  bt_tile<MI, NJ, ST>(head, tiles_n, args, COLUMNS ? inner : outer, COLUMNS ? outer : inner, smem);
+}
+
+// Where only the device knows the row count, it picks the tile: the tiles that are the best for some count up to the launch's
+// bound come along, cheapest first, each with the rows it serves in one round, and every workgroup takes the first that serves the
+// rows that are there.  The four products of a BERT-base layer, tile picked for the bound and for the rows: 614 of 1024 rows 41.9 and
+// 31.6 us, 1024 of 1024 43.7 and 40.5 (the start of the kernel costs no more than that of a kernel for one tile); 2457 of 4096 77.9
+// and 66.2, 4096 of 4096 88.8 and 86.2; 300 of 500 33.0 and 25.1.
+struct BtRowsPlan {
+  static constexpr int kPicks = 7, kColumns = 0x80;
+  uint64_t picks = 0;          // a byte each, the first in the lowest: index into ET_BT_ROWS_TILES, kColumns
+  int up_to[kPicks - 1];       // rows a pick serves (the last one: the rest)
+};
+__global__ __launch_bounds__(kHThreads) __attribute__((amdgpu_waves_per_eu(2))) void gemm_f16_bt_rows_kernel(ET_HEAD_ARGS, BtRowsPlan plan, GemmArgs args) {
+  extern __shared__ __attribute__((aligned(1024))) unsigned char smem[];
+  int rows = *rows_dev;
+  TileHead head{(const char*)a0, (const char*)b0, (uint64_t)args.A[1], (uint64_t)args.B[1], (uint64_t)args.A[2], (uint64_t)args.B[2], 0, n, k, groups};
+#if defined(__HIP_DEVICE_COMPILE__)
+  asm volatile("" : "+s"(rows), "+s"(head.to_a1), "+s"(head.to_b1), "+s"(head.to_a2), "+s"(head.to_b2), "+s"(plan.picks));    // all in one go
+#endif
+  head.to_a1 -= (uint64_t)a0, head.to_b1 -= (uint64_t)b0, head.to_a2 -= (uint64_t)a0, head.to_b2 -= (uint64_t)b0;
+  head.rows = rows = max(min(rows, m_bound), 0);
+  int at = 0;
+#pragma unroll
+  for (int i = 0; i < BtRowsPlan::kPicks - 1; ++i) at += 8 * uniform_less(plan.up_to[i], rows);
+  const int pick = (int)(plan.picks >> at), by_columns = pick & BtRowsPlan::kColumns;
+  int index = 0;
+#define ET_BT_CASE(MI, NJ, DUO, ST)                                                                                     \
+  if ((pick & 15) == index++) {                                                                                          \
+    tiles_n = (int)((unsigned)(n + 32 * NJ - 1) / (32 * NJ));                                                             \
+    const int all_n = tiles_n * groups, tiles_m = (int)((unsigned)(rows + 32 * MI - 1) / (32 * MI));                 \
+    const int tile = remap_valid_tile(blockIdx.x, tiles_m * all_n);                                                      \
+    if (tile < 0) return;                                                                                                \
+    const int by = by_columns ? tiles_m : all_n, outer = uniform_div(tile, by), inner = tile - outer * by;                  \
+    return bt_tile<MI, NJ, ST>(head, tiles_n, args, by_columns ? inner : outer, by_columns ? outer : inner, smem); \
+  }
+  ET_BT_ROWS_TILES(ET_BT_CASE)
+#undef ET_BT_CASE
 }
 
 // ------------------------------------------------------------------------------------------
@@ -1257,7 +1369,7 @@ void launch_f16_bt(GemmArgs a, hipStream_t stream) {
   a.per_xcd = (total + kXcds - 1) / kXcds;
   auto go = [&](auto kern) {
     allow_dynamic_lds(reinterpret_cast<const void*>(kern), (int)Tile::SMEM_BYTES);
-    kern<<<a.per_xcd * kXcds, kHThreads, Tile::SMEM_BYTES, stream>>>(a);
+    kern<<<a.per_xcd * kXcds, kHThreads, Tile::SMEM_BYTES, stream>>>(a.A[0], a.B[0], a.rows_dev, a.m_bound, a.n, a.k, a.groups, a.tiles_n, 0, 0, a);
   };
   // Few rows want the columns: the weights are then spread over the XCDs instead of read by each of them (12 layers on 580
   // rows of BERT-base 594 -> 572 us, on 300 rows of BERT-large 633 -> 575 us).  Where the two orders fetch about the same
@@ -1290,36 +1402,14 @@ int device_cu_count() {
 // lower tile must win 3 % by that estimate (measured: FFN-down of 13097 rows 75 -> 64 us, of 15866 rows 76 -> 70 us,
 // attention-out 26 -> 24 us; the 13097 x 1024 one of BERT-large 35 -> 31.5 us; all with the same bits).
 int pair_kernel_row_blocks(int m_bound, int n, int groups) {
-  const int cus = device_cu_count();
-  const int wgs = std::max(1, cus / kXcds);
-  const int tiles_n = (n + kPBN - 1) / kPBN * groups;
-  auto cost = [&](int mi) {
-    const long tiles = (long)((m_bound + 32 * mi - 1) / (32 * mi)) * tiles_n;
-    const long n_loc = (tiles + kXcds - 1) / kXcds;
-    const long full = n_loc / wgs, rem = n_loc % wgs;
-    // a rest of at most half the workgroups is shared, two workgroups per tile
-    const double rounds = (double)full + (rem == 0 ? 0.0 : (2 * rem <= wgs ? 0.55 : 1.0));
-    return rounds * (mi + 21);
-  };
-  const double cost8 = cost(8);
-  double best = cost8;
-  int best_mi = 8;
-  for (int mi = 7; mi >= 5; --mi) {
-    const double c = cost(mi);
-    if (c < 0.97 * cost8 && c < best) {
-      best = c;
-      best_mi = mi;
-    }
-  }
-  return best_mi;
+  return pair_row_blocks(m_bound, (n + kPBN - 1) / kPBN * groups, std::max(1, device_cu_count() / kXcds));
 }
 
-template <bool GELU, int MI, bool NT, bool A3 = false>
-void launch_pair(const GemmArgs& a, int grid, hipStream_t stream) {
-  auto kern = gemm_f16_pair_kernel<GELU, MI, NT, A3>;
-  constexpr int lds = A3 ? kQSmemA3 : kQSmem;
+template <typename Kernel>
+void launch_pair(Kernel kern, int lds, const GemmArgs& a, int columns, int grid, hipStream_t stream) {
   allow_dynamic_lds(reinterpret_cast<const void*>(kern), lds);
-  kern<<<grid, kPThreads, lds, stream>>>(a);
+  const int walk = (a.reverse_walk ? kWalkReverse : 0) | (a.a_blocked ? kWalkBlockedA : 0) | grid / kXcds << kWalkWgs;
+  kern<<<grid, kPThreads, lds, stream>>>(a.A[0], a.B[0], a.rows_dev, a.m_bound, a.n, a.k, a.groups, a.tiles_n, columns, walk, a);
 }
 
 void launch_f16_persistent(GemmArgs a, hipStream_t stream, bool b_transposed) {
@@ -1341,14 +1431,14 @@ void launch_f16_persistent(GemmArgs a, hipStream_t stream, bool b_transposed) {
   // through the column tiles in groups whose weight slice stays in the L2 (at most 2.5 MB, at least 3 column tiles), at
   // the price of reading A once per group: 241 MiB per launch there, 290 -> 170 MiB for BERT-large's FFN-up; the
   // launches themselves gain about 1 %.
-  a.col_groups = 1;
+  int columns = a.tiles_n * a.groups;
   {
     const int tn = a.tiles_n * a.groups;
     const double w_bytes = (double)a.n * a.groups * a.k * 2.0;
     if (b_transposed && (long)a.n * a.groups >= 2L * a.k && w_bytes > 4.0 * 1048576.0)
       for (int cg = 2; cg <= tn / 3; ++cg)
         if (tn % cg == 0 && w_bytes / cg <= 2.5 * 1048576.0) {
-          a.col_groups = cg;
+          columns = tn / cg;
           break;
         }
   }
@@ -1357,20 +1447,31 @@ void launch_f16_persistent(GemmArgs a, hipStream_t stream, bool b_transposed) {
     gemm_f16_persistent_kernel<<<grid, kPThreads, kPSmem, stream>>>(a);
     return;
   }
+  if (a.rows_dev != nullptr && !a.a_blocked && !a.c_blocked) {
+    grid = device_cu_count() / kXcds * kXcds;
+    auto go = [&](auto kern, int lds) { launch_pair(kern, lds, a, columns, grid, stream); };
+    if (a.gelu && a.c_cached) go(gemm_f16_pair_rows_kernel<true, false, false>, kQSmem);
+    else if (a.gelu) go(gemm_f16_pair_rows_kernel<true, true, false>, kQSmem);
+    else if (a.k >= 2048 && a.c_cached) go(gemm_f16_pair_rows_kernel<false, false, true>, kQSmemA3);
+    else if (a.k >= 2048) go(gemm_f16_pair_rows_kernel<false, true, true>, kQSmemA3);
+    else if (a.c_cached) go(gemm_f16_pair_rows_kernel<false, false, false>, kQSmem);
+    else go(gemm_f16_pair_rows_kernel<false, true, false>, kQSmem);
+    return;
+  }
   // A from HBM, few long tiles per workgroup: the A rows are requested a pair earlier (three LDS slots for A)
   if (!a.gelu && a.k >= 2048 && mi >= 7) {
-    if (mi == 8 && !a.c_cached) launch_pair<false, 8, true, true>(a, grid, stream);
-    else if (mi == 8) launch_pair<false, 8, false, true>(a, grid, stream);
-    else if (!a.c_cached) launch_pair<false, 7, true, true>(a, grid, stream);
-    else launch_pair<false, 7, false, true>(a, grid, stream);
+    if (mi == 8 && !a.c_cached) launch_pair(gemm_f16_pair_kernel<false, 8, true, true>, kQSmemA3, a, columns, grid, stream);
+    else if (mi == 8) launch_pair(gemm_f16_pair_kernel<false, 8, false, true>, kQSmemA3, a, columns, grid, stream);
+    else if (!a.c_cached) launch_pair(gemm_f16_pair_kernel<false, 7, true, true>, kQSmemA3, a, columns, grid, stream);
+    else launch_pair(gemm_f16_pair_kernel<false, 7, false, true>, kQSmemA3, a, columns, grid, stream);
     return;
   }
 #define ET_PAIR_CASE(M)                                                      \
   case M:                                                                    \
-    if (a.gelu && a.c_cached) launch_pair<true, M, false>(a, grid, stream);  \
-    else if (a.gelu) launch_pair<true, M, true>(a, grid, stream);            \
-    else if (a.c_cached) launch_pair<false, M, false>(a, grid, stream);      \
-    else launch_pair<false, M, true>(a, grid, stream);                       \
+    if (a.gelu && a.c_cached) launch_pair(gemm_f16_pair_kernel<true, M, false>, kQSmem, a, columns, grid, stream);  \
+    else if (a.gelu) launch_pair(gemm_f16_pair_kernel<true, M, true>, kQSmem, a, columns, grid, stream);            \
+    else if (a.c_cached) launch_pair(gemm_f16_pair_kernel<false, M, false>, kQSmem, a, columns, grid, stream);      \
+    else launch_pair(gemm_f16_pair_kernel<false, M, true>, kQSmem, a, columns, grid, stream);                       \
     break;
   switch (mi) {
     ET_PAIR_CASE(8)
@@ -1432,27 +1533,62 @@ BtPick pick_bt_tile(int m_bound, int n, int groups, int cus, bool proven_only) {
 
 void launch_bt_tile(BtPick p, const GemmArgs& a, hipStream_t stream) {
   switch (p.mi * 100 + p.nj * 10 + (p.duo ? 1 : 0)) {
-    case 110: return launch_f16_bt<1, 1, 5>(a, stream);
-    case 120: return launch_f16_bt<1, 2, 5>(a, stream);
-    case 121: return launch_f16_bt<1, 2, 3>(a, stream);
-    case 220: return launch_f16_bt<2, 2, 4>(a, stream);
-    case 221: return launch_f16_bt<2, 2, 3>(a, stream);
-    case 240: return launch_f16_bt<2, 4, 4>(a, stream);
-    case 241: return launch_f16_bt<2, 4, 3>(a, stream);
-    case 320: return launch_f16_bt<3, 2, 4>(a, stream);
-    case 321: return launch_f16_bt<3, 2, 3>(a, stream);
-    case 340: return launch_f16_bt<3, 4, 4>(a, stream);
-    case 341: return launch_f16_bt<3, 4, 2>(a, stream);
-    case 360: return launch_f16_bt<3, 6, 3>(a, stream);
-    case 361: return launch_f16_bt<3, 6, 2>(a, stream);
-    case 420: return launch_f16_bt<4, 2, 4>(a, stream);
-    case 421: return launch_f16_bt<4, 2, 3>(a, stream);
-    case 440: return launch_f16_bt<4, 4, 4>(a, stream);
-    case 460: return launch_f16_bt<4, 6, 3>(a, stream);
-    case 461: return launch_f16_bt<4, 6, 2>(a, stream);
-    case 480: return launch_f16_bt<4, 8, 3>(a, stream);
+#define ET_BT_CASE(MI, NJ, DUO, ST) \
+  case MI * 100 + NJ * 10 + DUO: return launch_f16_bt<MI, NJ, ST>(a, stream);
+    ET_BT_TILES(ET_BT_CASE)
+#undef ET_BT_CASE
     default: return launch_f16_bt<4, 4, 2>(a, stream);     // 128 x 128 in rounds of two workgroups per CU
   }
+}
+
+// A launch for a row count on the device, up to a.m_bound.  False where the bound itself needs another kind of tile (two
+// workgroups per CU, 128 x 256) that is more than 5 % cheaper by the estimate of pick_bt_tile.
+bool launch_bt_rows(GemmArgs a, hipStream_t stream) {
+  const int cus = device_cu_count();
+  struct Tile {
+    int index, mi, nj, lds;
+    float cost;
+    int rows, tiles_n;
+  } tiles[] = {
+#define ET_BT_CASE(MI, NJ, DUO, ST) {0, MI, NJ, BtTile<MI, NJ, ST>::SMEM_BYTES, (float)(MI + NJ + (NJ == 6 ? 1 : 0)), 0, 0},
+      ET_BT_ROWS_TILES(ET_BT_CASE)
+#undef ET_BT_CASE
+  };
+  int index = 0;
+  for (Tile& t : tiles) {
+    t.index = index++;
+    t.tiles_n = (a.n + 32 * t.nj - 1) / (32 * t.nj) * a.groups;
+    t.rows = cus / t.tiles_n * 32 * t.mi;
+  }
+  std::sort(std::begin(tiles), std::end(tiles), [](const Tile& x, const Tile& y) { return x.cost != y.cost ? x.cost < y.cost : x.rows > y.rows; });
+  BtRowsPlan plan;
+  for (int& rows : plan.up_to) rows = INT_MAX;
+  int picks = 0, served = 0, lds = 0;
+  long wgs = 0;
+  float cost = 0.f;
+  for (const Tile& t : tiles) {
+    if (served >= a.m_bound || t.rows <= served) continue;
+    // (counts below an eighth of the bound get the tile of the next ones)
+    if (t.rows < a.m_bound / 8 || picks == BtRowsPlan::kPicks) continue;
+    const int rows = std::min(t.rows, a.m_bound), tiles_m = (rows + 32 * t.mi - 1) / (32 * t.mi);
+    const BandRows band = band_rows(tiles_m, t.tiles_n, 32 * t.mi, 32 * t.nj);
+    const bool columns = rows <= kColumnRows && 4 * band.down <= 3 * band.along;
+    if (rows < a.m_bound && picks < BtRowsPlan::kPicks - 1) plan.up_to[picks] = rows;
+    plan.picks |= (uint64_t)(t.index | (columns ? BtRowsPlan::kColumns : 0)) << (8 * picks);
+    wgs = std::max(wgs, (long)tiles_m * t.tiles_n);
+    lds = std::max(lds, t.lds);
+    cost = t.cost;
+    served = rows;
+    ++picks;
+  }
+  if (served < a.m_bound || picks < 2) return false;
+  const BtPick best = pick_bt_tile(a.m_bound, a.n, a.groups, cus, false);
+  const float best_cost = (float)(best.mi + best.nj + (best.nj == 6 ? 1 : 0)) * (best.duo ? 2.f / 1.3f : 1.f);
+  if (best.mi != 0 && cost > 1.05f * best_cost) return false;
+  allow_dynamic_lds(reinterpret_cast<const void*>(gemm_f16_bt_rows_kernel), 160 * 1024);
+  gemm_f16_bt_rows_kernel<<<(int)((wgs + kXcds - 1) / kXcds * kXcds), kHThreads, lds, stream>>>(a.A[0], a.B[0], a.rows_dev, a.m_bound, a.n, a.k,
+                                                                                                 a.groups, 0, 0, 0, plan, a);
+  return true;
 }
 
 // few big tiles would leave most of the 256 CUs idle: the persistent 256x256 kernel only runs when there is work
@@ -1600,8 +1736,8 @@ void launch_gemm(DType t, const GemmGroups& g, void* C, int ldc, int m_bound, in
       launch_f16_persistent(a, stream, g.b_transposed);
     } else if (g.b_transposed) {
       // one tile per workgroup, the tile chosen for the launch's shape (pick_bt_tile)
-      const int cus = device_cu_count();
-      launch_bt_tile(pick_bt_tile(m_bound, n, g.groups, cus, false), a, stream);
+      if (rows_dev != nullptr && launch_bt_rows(a, stream)) return;
+      launch_bt_tile(pick_bt_tile(m_bound, n, g.groups, device_cu_count(), false), a, stream);
     } else {
       // Below a round of the chip the time of a launch is the k loop of one tile.  With fewer 64 x 256 tiles than CUs
       // that loop runs at the rate one CU's DMA fills its LDS: the 64 x 128 tile halves the B bytes per workgroup and
