@@ -89,7 +89,7 @@ template <typename T, int VEC, int ITERS>
 __global__ __launch_bounds__(kLnThreads) void bias_residual_layernorm_kernel(
     T* __restrict__ out, const T* __restrict__ input, const T* __restrict__ bias, const T* __restrict__ gamma,
     const T* __restrict__ beta, int m, int n, const int32_t* __restrict__ rows_dev, WarmList warm,
-    uint16_t* __restrict__ split, PairRows pair) {
+    uint16_t* __restrict__ split, PairRows pair, int warm_begin) {
   using V = typename RowVec<T, VEC>::type;
   const int rows = rows_dev ? min(*rows_dev, m) : m;
   const int lane = threadIdx.x & (kWave - 1);
@@ -99,10 +99,11 @@ __global__ __launch_bounds__(kLnThreads) void bias_residual_layernorm_kernel(
 
   // `warm`: regions (weight matrices) that one of the next kernels would read cold; one word of each of their 128-byte
   // lines is requested here, which pulls the line into the last-level cache.  The values are only looked at behind
-  // the row loop, so no wavefront waits for them.
+  // the row loop; but requests return in order, so a wavefront that also has rows sees the first of them behind its words
+  // from memory: few rows leave the list to workgroups of its own, from warm_begin on.
   uint32_t warm0 = 0, warm1 = 0;
-  if (warm.total > 0) {
-    const int tid = blockIdx.x * kLnThreads + threadIdx.x, nth = gridDim.x * kLnThreads;
+  if (warm.total > 0 && (int)blockIdx.x >= warm_begin) {
+    const int tid = (blockIdx.x - warm_begin) * kLnThreads + threadIdx.x, nth = (gridDim.x - warm_begin) * kLnThreads;
     auto word = [&](int i) {
       int r = 0;
       while (r + 1 < WarmList::kMax && i >= warm.lines[r]) i -= warm.lines[r++];
@@ -322,15 +323,24 @@ bool ln_pick(int n, int& vec, int& iters) {
   return false;
 }
 
+// Enough wavefronts to fill 256 CUs several times over; rows beyond that are looped.  A list of lines to request brings as many
+// threads as it has lines (up to the same bound): few rows must not be held up by a long list.  Up to 256 workgroups of rows, the
+// list has workgroups of its own: 12 layers on 16 rows 400 us with the lines requested by the wavefronts with rows, 387 apart; 2000
+// rows 824 and 827, 7000 rows 1915 and up to 1938.
+template <typename T, int VEC, int ITERS>
+void ln_launch_kernel(hipStream_t stream, T* out, const T* input, const T* bias, const T* gamma, const T* beta, int m, int n,
+                      const int32_t* rows_dev, const WarmList& warm, uint16_t* split, const PairRows& pair) {
+  const long lines = (warm.total + kLnThreads - 1) / kLnThreads, needed = ((long)m + kLnWaves - 1) / kLnWaves;
+  const int begin = needed <= 256 ? (int)needed : 0;
+  const int grid = (int)min(max(needed, begin + lines), 256L * 8);
+  bias_residual_layernorm_kernel<T, VEC, ITERS><<<grid, kLnThreads, 0, stream>>>(out, input, bias, gamma, beta, m, n, rows_dev, warm, split, pair, begin);
+}
+
 template <typename T, int VEC>
-void ln_launch_iters(int iters, int grid, hipStream_t stream, T* out, const T* input, const T* bias, const T* gamma,
-                     const T* beta, int m, int n, const int32_t* rows_dev, const WarmList& warm, uint16_t* split,
-                     const PairRows& pair) {
-#define ET_LN_CASE(I)                                                                                          \
-  case I:                                                                                                      \
-    bias_residual_layernorm_kernel<T, VEC, I><<<grid, kLnThreads, 0, stream>>>(out, input, bias, gamma, beta, m, n, \
-                                                                               rows_dev, warm, split, pair);   \
-    break;
+void ln_launch_iters(int iters, hipStream_t stream, T* out, const T* input, const T* bias, const T* gamma, const T* beta, int m, int n,
+                     const int32_t* rows_dev, const WarmList& warm, uint16_t* split, const PairRows& pair) {
+#define ET_LN_CASE(I) \
+  case I: return ln_launch_kernel<T, VEC, I>(stream, out, input, bias, gamma, beta, m, n, rows_dev, warm, split, pair);
   switch (iters) {
     ET_LN_CASE(1)
     ET_LN_CASE(2)
@@ -349,19 +359,15 @@ void ln_launch(void* out, const void* input, const void* bias, const void* gamma
                const int32_t* rows_dev, hipStream_t stream, const WarmList& warm, uint16_t* split, const PairRows& pair) {
   int vec = 0, iters = 0;
   if (!ln_pick<T>(n, vec, iters)) return;
-  // enough wavefronts to fill 256 CUs several times over; rows beyond that are looped.  A list of lines to request brings
-  // as many threads as it has lines (up to the same bound): few rows must not be held up by a long list.
-  const long lines = (warm.total + kLnThreads - 1) / kLnThreads;
-  const int grid = (int)min(max((long)(m + kLnWaves - 1) / kLnWaves, lines), 256L * 8);
   T* o = (T*)out;
   const T *i = (const T*)input, *b = (const T*)bias, *g = (const T*)gamma, *be = (const T*)beta;
   constexpr int MV = 16 / (int)sizeof(T);
   if (vec == MV)
-    ln_launch_iters<T, MV>(iters, grid, stream, o, i, b, g, be, m, n, rows_dev, warm, split, pair);
+    ln_launch_iters<T, MV>(iters, stream, o, i, b, g, be, m, n, rows_dev, warm, split, pair);
   else if (vec == MV / 2)
-    ln_launch_iters<T, MV / 2>(iters, grid, stream, o, i, b, g, be, m, n, rows_dev, warm, split, pair);
+    ln_launch_iters<T, MV / 2>(iters, stream, o, i, b, g, be, m, n, rows_dev, warm, split, pair);
   else
-    ln_launch_iters<T, MV / 4>(iters, grid, stream, o, i, b, g, be, m, n, rows_dev, warm, split, pair);
+    ln_launch_iters<T, MV / 4>(iters, stream, o, i, b, g, be, m, n, rows_dev, warm, split, pair);
 }
 
 struct EmbedArgs {
