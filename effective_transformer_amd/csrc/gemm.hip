@@ -1182,6 +1182,148 @@ __global__ __launch_bounds__(kHThreads) __attribute__((amdgpu_waves_per_eu(2))) 
 }
 
 // ------------------------------------------------------------------------------------------
+// fp16, a handful of rows: one wavefront, one 16 x 16 tile.
+//
+// With no more tiles than this a launch takes the k loop of one of them, and what the 32 x 32 tile of four wavefronts spends
+// there is LDS traffic (16 KB of operand reads and 8 KB of DMA per pair of k-steps, half of it for rows that are not there)
+// between two barriers a pair.  A wavefront of its own has no barriers, a sixth of the traffic and as many CUs as there are
+// 16-column strips; its ring of 13 slots has the twelve pairs of k = 768 on their way before the first one is used.
+// BERT-base on 16 rows: k = 768 4.2 -> 3.6 us (a launch that does nothing takes 2.3), k = 3072 7.6 -> 6.3, of which each pair takes
+// 76 ns: 50 for its four DMA instructions and 38 for operand reads and MFMAs, which one wavefront does not fully overlap.
+// ------------------------------------------------------------------------------------------
+// at most 4 * pairs requests left on their way (a constant once the loop around it is unrolled)
+__device__ __forceinline__ void wait_pairs(int pairs) {
+  switch (pairs) {
+    case 0: return wait_vmcnt<0>();
+    case 1: return wait_vmcnt<4>();
+    case 2: return wait_vmcnt<8>();
+    case 3: return wait_vmcnt<12>();
+    case 4: return wait_vmcnt<16>();
+    case 5: return wait_vmcnt<20>();
+    case 6: return wait_vmcnt<24>();
+    case 7: return wait_vmcnt<28>();
+    case 8: return wait_vmcnt<32>();
+    case 9: return wait_vmcnt<36>();
+    case 10: return wait_vmcnt<40>();
+    default: return wait_vmcnt<44>();
+  }
+}
+constexpr int kWaveSlots = 13, kWaveSlotBytes = 2 * 16 * 128;
+
+__global__ __launch_bounds__(kWave) __attribute__((amdgpu_waves_per_eu(1))) void gemm_f16_bt_wave_kernel(ET_HEAD_ARGS, GemmArgs args) {
+#if defined(__HIP_DEVICE_COMPILE__)   // device-only types in the body; the host pass only needs the stub
+  constexpr int kAhead = kWaveSlots - 1;                          // pairs in flight behind the one in use
+  static_assert(kAhead % 2 == 0 && 4 * kAhead < 64, "the register sets alternate; vmcnt has six bits");
+  extern __shared__ __attribute__((aligned(1024))) unsigned char smem[];
+  const TileHead head = tile_head(a0, b0, rows_dev, m_bound, n, k, groups, args);
+  const int rows = head.rows, N = n, K = k;
+  // the tiles of a strip of columns follow each other: an XCD reads its strips of B once
+  const int tiles_m = (int)((unsigned)(rows + 15) / 16);
+  const int tile = remap_valid_tile(blockIdx.x, tiles_m * tiles_n * groups);
+  if (tile < 0) return;
+  const int tn_all = uniform_div(tile, tiles_m), tm = tile - tn_all * tiles_m;
+  const int grp = groups == 1 ? 0 : 2 - uniform_less(tn_all, tiles_n) - uniform_less(tn_all, 2 * tiles_n);
+  const int m0 = tm * 16, n0 = (tn_all - grp * tiles_n) * 16;
+  const int np = (int)((unsigned)K / 64);                         // pairs of k-steps
+  const int lane = threadIdx.x, l16 = lane & 15, g = lane >> 4;
+
+  // rows at or beyond the valid-token count and columns at or beyond n read as zero
+  const __amdgpu_buffer_rsrc_t rsrc_a =
+      __builtin_amdgcn_make_buffer_rsrc(const_cast<char*>(head.a_of(grp) + (size_t)m0 * K * 2), 0, min(rows - m0, 16) * K * 2, 0x00020000);
+  const __amdgpu_buffer_rsrc_t rsrc_b =
+      __builtin_amdgcn_make_buffer_rsrc(const_cast<char*>(head.b_of(grp) + (size_t)n0 * K * 2), 0, min(N - n0, 16) * K * 2, 0x00020000);
+  uint32_t voff[2];                                               // of an instruction's 8 rows x 128 bytes
+#pragma unroll
+  for (int j = 0; j < 2; ++j) {
+    const int row = j * 8 + (lane >> 3);
+    voff[j] = ((uint32_t)row * (uint32_t)K + (uint32_t)((lane & 7) ^ pair_swizzle(row)) * 8u) * 2u;
+  }
+  auto issue = [&](int slot, int pr) {
+    unsigned char* st = smem + slot * kWaveSlotBytes;
+#pragma unroll
+    for (int j = 0; j < 2; ++j) __builtin_amdgcn_raw_ptr_buffer_load_lds(rsrc_a, ET_LDS_PTR(st + j * 1024), 16, voff[j], pr * 128, 0, 0);
+#pragma unroll
+    for (int j = 0; j < 2; ++j) __builtin_amdgcn_raw_ptr_buffer_load_lds(rsrc_b, ET_LDS_PTR(st + 2048 + j * 1024), 16, voff[j], pr * 128, 0, 0);
+  };
+  const int sw = pair_swizzle(l16);
+  const int rd[2] = {l16 * 128 + ((g ^ sw) * 16), l16 * 128 + (((4 + g) ^ sw) * 16)};
+
+  // Pairs are counted from the end: `left` behind the one in use, in register set left & 1.  The MFMAs of a pair run while the
+  // operands of the next one are on their way from the LDS.
+  const half8 zeros = {};
+  half8 a[2][2] = {{zeros, zeros}, {zeros, zeros}}, b[2][2] = {{zeros, zeros}, {zeros, zeros}};
+  float4v acc = {0.f, 0.f, 0.f, 0.f};
+  int slot = 0;                                                   // of the pair in use
+  auto read = [&](auto Pc) {
+    constexpr int P = decltype(Pc)::value;
+    const unsigned char* st = smem + slot * kWaveSlotBytes;
+    slot = slot + 1 == kWaveSlots ? 0 : slot + 1;
+#pragma unroll
+    for (int h = 0; h < 2; ++h) {
+      b[P][h] = *reinterpret_cast<const half8*>(st + 2048 + rd[h]);
+      a[P][h] = *reinterpret_cast<const half8*>(st + rd[h]);
+    }
+  };
+  // the operands in this order leave four consecutive columns of a row of C in a lane
+  auto multiply = [&](auto Pc) {
+    constexpr int P = decltype(Pc)::value;
+#pragma unroll
+    for (int h = 0; h < 2; ++h) acc = __builtin_amdgcn_mfma_f32_16x16x32_f16(b[P][h], a[P][h], acc, 0, 0, 0);
+  };
+  using Even = std::integral_constant<int, 0>;
+  using Odd = std::integral_constant<int, 1>;
+
+#pragma unroll
+  for (int s = 0; s < kAhead; ++s)
+    if (s < np) issue(s, s);
+  const int col = n0 + g * 4;
+  half4 biasv = {(_Float16)-0.0f, (_Float16)-0.0f, (_Float16)-0.0f, (_Float16)-0.0f};
+  // (behind the first requests, see bt_tile; the waits below count it as one of the pair in front of it)
+  if (const _Float16* bias = (const _Float16*)args.bias[grp]; bias != nullptr && col < N) biasv = *reinterpret_cast<const half4*>(bias + col);
+  int left = np - 1, free_slot = kAhead;
+  auto advance = [&](auto Pc) {
+    using Other = std::integral_constant<int, 1 - decltype(Pc)::value>;
+    wait_vmcnt<4 * (kAhead - 1)>();              // the pair has landed, those behind it may fly
+    read(Pc);
+    __builtin_amdgcn_sched_barrier(0);
+    multiply(Other{});                           // its operands are there, so nobody reads the slot they came from any more
+    __builtin_amdgcn_sched_barrier(0);
+    issue(free_slot, np - 1 - left + kAhead);
+    free_slot = free_slot + 1 == kWaveSlots ? 0 : free_slot + 1;
+    --left;
+  };
+  if (left >= kAhead && (left & 1) == 0) advance(Even{});
+  while (left >= kAhead) {
+    advance(Odd{});
+    advance(Even{});
+  }
+#pragma unroll
+  for (int l = kAhead - 1; l >= 0; --l)
+    if (l <= left) {
+      wait_pairs(l);
+      if (l & 1) {
+        read(Odd{});
+        __builtin_amdgcn_sched_barrier(0);
+        multiply(Even{});
+      } else {
+        read(Even{});
+        __builtin_amdgcn_sched_barrier(0);
+        multiply(Odd{});
+      }
+      __builtin_amdgcn_sched_barrier(0);
+    }
+  multiply(Even{});
+
+  const int row = m0 + l16;
+  if (row < rows && col < N) {
+    half4 o = {f2h(acc[0]), f2h(acc[1]), f2h(acc[2]), f2h(acc[3])};
+    o = args.gelu ? bias_gelu_half<half4, 4>(o, biasv) : o + biasv;
+    *reinterpret_cast<half4*>((_Float16*)args.C + (size_t)row * args.ldc + (size_t)grp * N + col) = o;
+  }
+#endif
+}
+
+// ------------------------------------------------------------------------------------------
 // fp32: 128x128x16 tile, 4 wavefronts (2x2) of 64x64, v_mfma_f32_32x32x2_f32
 // ------------------------------------------------------------------------------------------
 constexpr int kFThreads = 256;
@@ -1541,6 +1683,22 @@ void launch_bt_tile(BtPick p, const GemmArgs& a, hipStream_t stream) {
   }
 }
 
+// One wavefront per 16 x 16 tile, up to two tiles a CU: 100 to 256 rows of n = 768 or 512 (up to 512 tiles) still gain 4 to 10 %, at 640
+// to 768 tiles it is a tie, and beyond the three workgroups that fit a CU's LDS the second round costs 40 % (QKV of 96 rows: 5.8 us, 4.3).
+// False where C does not take stores of four columns.
+bool launch_bt_wave(GemmArgs a, hipStream_t stream) {
+  a.tiles_n = (a.n + 15) / 16;
+  const long wgs = (long)((a.m_bound + 15) / 16) * a.tiles_n * a.groups;
+  if (wgs > 2l * device_cu_count()) return false;
+  bool aligned = ((uintptr_t)a.C | (uintptr_t)a.ldc * 2) % 8 == 0;
+  for (int g = 0; g < a.groups; ++g) aligned = aligned && (uintptr_t)a.bias[g] % 8 == 0;
+  if (!aligned) return false;
+  constexpr int lds = kWaveSlots * kWaveSlotBytes;
+  gemm_f16_bt_wave_kernel<<<(int)((wgs + kXcds - 1) / kXcds * kXcds), kWave, lds, stream>>>(a.A[0], a.B[0], a.rows_dev, a.m_bound, a.n, a.k, a.groups,
+                                                                                             a.tiles_n, 0, 0, a);
+  return true;
+}
+
 // A launch for a row count on the device, up to a.m_bound.  False where the bound itself needs another kind of tile (two
 // workgroups per CU, 128 x 256) that is more than 5 % cheaper by the estimate of pick_bt_tile.
 bool launch_bt_rows(GemmArgs a, hipStream_t stream) {
@@ -1736,6 +1894,7 @@ void launch_gemm(DType t, const GemmGroups& g, void* C, int ldc, int m_bound, in
       launch_f16_persistent(a, stream, g.b_transposed);
     } else if (g.b_transposed) {
       // one tile per workgroup, the tile chosen for the launch's shape (pick_bt_tile)
+      if (launch_bt_wave(a, stream)) return;
       if (rows_dev != nullptr && launch_bt_rows(a, stream)) return;
       launch_bt_tile(pick_bt_tile(m_bound, n, g.groups, device_cu_count(), false), a, stream);
     } else {
