@@ -89,29 +89,13 @@ template <typename T, int VEC, int ITERS>
 __global__ __launch_bounds__(kLnThreads) void bias_residual_layernorm_kernel(
     T* __restrict__ out, const T* __restrict__ input, const T* __restrict__ bias, const T* __restrict__ gamma,
     const T* __restrict__ beta, int m, int n, const int32_t* __restrict__ rows_dev, WarmList warm,
-    uint16_t* __restrict__ split, PairRows pair, int warm_begin) {
+    uint16_t* __restrict__ split, PairRows pair) {
   using V = typename RowVec<T, VEC>::type;
   const int rows = rows_dev ? min(*rows_dev, m) : m;
   const int lane = threadIdx.x & (kWave - 1);
   const int wave = blockIdx.x * kLnWaves + threadIdx.x / kWave;
   const int nwaves = gridDim.x * kLnWaves;
   const int vpr = n / VEC;                       // vectors per row
-
-  // `warm`: regions (weight matrices) that one of the next kernels would read cold; one word of each of their 128-byte
-  // lines is requested here, which pulls the line into the last-level cache.  The values are only looked at behind
-  // the row loop; but requests return in order, so a wavefront that also has rows sees the first of them behind its words
-  // from memory: few rows leave the list to workgroups of its own, from warm_begin on.
-  uint32_t warm0 = 0, warm1 = 0;
-  if (warm.total > 0 && (int)blockIdx.x >= warm_begin) {
-    const int tid = (blockIdx.x - warm_begin) * kLnThreads + threadIdx.x, nth = (gridDim.x - warm_begin) * kLnThreads;
-    auto word = [&](int i) {
-      int r = 0;
-      while (r + 1 < WarmList::kMax && i >= warm.lines[r]) i -= warm.lines[r++];
-      return warm.p[r][(size_t)i * 32];
-    };
-    if (tid < warm.total) warm0 = word(tid);
-    for (int i = tid + nth; i < warm.total; i += nth) warm1 ^= word(i);
-  }
 
   V b[ITERS], g[ITERS], be[ITERS];
 #pragma unroll
@@ -125,10 +109,10 @@ __global__ __launch_bounds__(kLnThreads) void bias_residual_layernorm_kernel(
   }
   const float inv_n = 1.0f / (float)n;
 
-  for (int r = wave; r < rows; r += nwaves) {
-    V* orow = reinterpret_cast<V*>(out + (size_t)r * n);
+  V xo[ITERS], xi[ITERS];
+  auto request = [&](int r) {
+    const V* orow = reinterpret_cast<const V*>(out + (size_t)r * n);
     const V* irow = reinterpret_cast<const V*>(input + (size_t)r * n);
-    V xo[ITERS], xi[ITERS];
 #pragma unroll
     for (int i = 0; i < ITERS; ++i) {
       const int c = lane + i * kWave;
@@ -137,6 +121,9 @@ __global__ __launch_bounds__(kLnThreads) void bias_residual_layernorm_kernel(
         xi[i] = irow[c];
       }
     }
+  };
+  auto finish = [&](int r) {
+    V* orow = reinterpret_cast<V*>(out + (size_t)r * n);
     float x[ITERS][VEC];
     float sum = 0.f;
 #pragma unroll
@@ -176,7 +163,7 @@ __global__ __launch_bounds__(kLnThreads) void bias_residual_layernorm_kernel(
           }
         }
         store_pair_row<ITERS>(y, vpr, pair, r, n);
-        continue;
+        return;
       }
 #pragma unroll
     for (int i = 0; i < ITERS; ++i) {
@@ -191,7 +178,30 @@ __global__ __launch_bounds__(kLnThreads) void bias_residual_layernorm_kernel(
           if (split) store_split<4>(split + (size_t)r * 3 * n, c * VEC, y);
       }
     }
+  };
+
+  // `warm`: regions (weight matrices) that one of the next kernels would read cold; one word of each of their 128-byte
+  // lines is requested here, which pulls the line into the last-level cache.  Requests return in order, so the words go out behind
+  // the wavefront's first row, every thread's one of them without a condition (a request that might be missing would have the row
+  // wait for it as well), and are only looked at behind the row loop.  In front of the first row, which then came a trip to memory
+  // later: 12 layers of BERT-base in graphs for 16 x 64 positions 574 us, 549 so, for 1 x 32 365 and 355; from 2000 rows on 1 to 2 %.
+  if (wave < rows) request(wave);
+  const int line = (int)blockIdx.x * kLnThreads + (int)threadIdx.x, lines = (int)gridDim.x * kLnThreads;
+  static_assert(WarmList::kMax == 3);
+  const int end0 = warm.lines[0], end1 = end0 + warm.lines[1];
+  auto word = [&](int i) {
+    const uint32_t* p = i < end0 ? warm.p[0] : i < end1 ? warm.p[1] : warm.p[2];
+    return p + (size_t)(i - (i < end0 ? 0 : i < end1 ? end0 : end1)) * 32;
+  };
+  const uint32_t* first_word = reinterpret_cast<const uint32_t*>(gamma);
+  if (line < warm.total) first_word = word(line);
+  uint32_t warm0 = *first_word, warm1 = 0;
+  if (wave < rows) finish(wave);
+  for (int r = wave + nwaves; r < rows; r += nwaves) {
+    request(r);
+    finish(r);
   }
+  for (int i = line + lines; i < warm.total; i += lines) warm1 ^= *word(i);
   // The requested words are consumed here, behind the row loop, by an empty instruction sequence: the loads cannot be
   // dropped, and nothing that depends on a corrupt row count decides whether they stay.
   asm volatile("" ::"v"(warm0), "v"(warm1));
@@ -324,16 +334,13 @@ bool ln_pick(int n, int& vec, int& iters) {
 }
 
 // Enough wavefronts to fill 256 CUs several times over; rows beyond that are looped.  A list of lines to request brings as many
-// threads as it has lines (up to the same bound): few rows must not be held up by a long list.  Up to 256 workgroups of rows, the
-// list has workgroups of its own: 12 layers on 16 rows 400 us with the lines requested by the wavefronts with rows, 387 apart; 2000
-// rows 824 and 827, 7000 rows 1915 and up to 1938.
+// threads as it has lines (up to the same bound): few rows must not be held up by a long list.
 template <typename T, int VEC, int ITERS>
 void ln_launch_kernel(hipStream_t stream, T* out, const T* input, const T* bias, const T* gamma, const T* beta, int m, int n,
                       const int32_t* rows_dev, const WarmList& warm, uint16_t* split, const PairRows& pair) {
-  const long lines = (warm.total + kLnThreads - 1) / kLnThreads, needed = ((long)m + kLnWaves - 1) / kLnWaves;
-  const int begin = needed <= 256 ? (int)needed : 0;
-  const int grid = (int)min(max(needed, begin + lines), 256L * 8);
-  bias_residual_layernorm_kernel<T, VEC, ITERS><<<grid, kLnThreads, 0, stream>>>(out, input, bias, gamma, beta, m, n, rows_dev, warm, split, pair, begin);
+  const long lines = (warm.total + kLnThreads - 1) / kLnThreads;
+  const int grid = (int)min(max(((long)m + kLnWaves - 1) / kLnWaves, lines), 256L * 8);
+  bias_residual_layernorm_kernel<T, VEC, ITERS><<<grid, kLnThreads, 0, stream>>>(out, input, bias, gamma, beta, m, n, rows_dev, warm, split, pair);
 }
 
 template <typename T, int VEC>
