@@ -224,10 +224,10 @@ __device__ __forceinline__ float xor_lanes_16_32_sum(float v) {
 // one matrix a thread moves per head (ceil(seq rows * chunks per row / threads)).
 template <typename T, int NKT, int WAVES, int CPT>
 __global__ __launch_bounds__(WAVES * kWave) void attention_kernel(
-    const T* __restrict__ q_src, const T* __restrict__ k_src, const T* __restrict__ v_src, int layout, int packed_ld,
-    const T* __restrict__ attr_mask, T* __restrict__ dst, const int32_t* __restrict__ seq_start,
-    const int32_t* __restrict__ word_idx, int batch, int seq_len, int heads, int heads_per_wg, float scaler,
-    int split_out, PairContext ctx) {
+    // (the first 14 words come in registers: what the chain order -> start table -> positions and rows needs)
+    const int32_t* __restrict__ seq_start, const int32_t* __restrict__ word_idx, int batch, int seq_len, int heads, int heads_per_wg,
+    int layout, int packed_ld, const T* __restrict__ q_src, const T* __restrict__ k_src, const T* __restrict__ v_src,
+    const T* __restrict__ attr_mask, T* __restrict__ dst, float scaler, int split_out, PairContext ctx) {
   using Cfg = AttnCfg<T>;
   using Sm = AttnSmem<T, NKT>;
   using C = Chunk16<T>;
@@ -560,9 +560,8 @@ void attention_launch(const void* q, const void* k, const void* v, int layout, i
       break;
     }
   dim3 grid((heads + hpw - 1) / hpw, batch);
-  kern<<<grid, kThreads, Sm::kBytes, stream>>>((const T*)q, (const T*)k, (const T*)v, layout, packed_ld,
-                                                   (const T*)attr_mask, (T*)dst, seq_start, word_idx, batch, seq_len,
-                                                   heads, hpw, scaler, split_out ? 1 : 0, ctx);
+  kern<<<grid, kThreads, Sm::kBytes, stream>>>(seq_start, word_idx, batch, seq_len, heads, hpw, layout, packed_ld, (const T*)q,
+                                               (const T*)k, (const T*)v, (const T*)attr_mask, (T*)dst, scaler, split_out ? 1 : 0, ctx);
 }
 
 
@@ -675,10 +674,10 @@ __device__ __forceinline__ half4 read_transposed(const unsigned char* p) {
 
 template <int QSUB>
 __global__ __launch_bounds__(kFlWaves * kWave, 4) void attention_flash_kernel(
-    const _Float16* __restrict__ q_src, const _Float16* __restrict__ k_src, const _Float16* __restrict__ v_src, int layout,
-    int packed_ld, const _Float16* __restrict__ attr_mask, const uint8_t* __restrict__ mask_class,
-    _Float16* __restrict__ dst, const int32_t* __restrict__ seq_start, const int32_t* __restrict__ word_idx, int batch,
-    int seq_len, int heads, int q_blocks, float scaler) {
+    const int32_t* __restrict__ seq_start, int batch, int heads, int q_blocks, int seq_len, int layout, int packed_ld,
+    const _Float16* __restrict__ q_src, const _Float16* __restrict__ k_src, const _Float16* __restrict__ v_src,
+    const int32_t* __restrict__ word_idx, const _Float16* __restrict__ attr_mask, const uint8_t* __restrict__ mask_class,
+    _Float16* __restrict__ dst, float scaler) {
 #if defined(__HIP_DEVICE_COMPILE__)   // device-only types in the body; the host pass only needs the stub
   using T = _Float16;
   typedef _Float16 half2x __attribute__((ext_vector_type(2)));
@@ -689,10 +688,10 @@ __global__ __launch_bounds__(kFlWaves * kWave, 4) void attention_flash_kernel(
   // The query blocks of one (head, sequence) go to one XCD, whose L2 then fetches their K and V once: workgroup ids are
   // dealt round-robin to the XCDs, pair p = 8 * (slot / q_blocks) + xcd.
   const int xcd = blockIdx.x & 7, slot_id = blockIdx.x >> 3;
-  const int pair = (slot_id / q_blocks) * 8 + xcd, qblock = slot_id % q_blocks;
+  const int pair_of_xcd = uniform_div(slot_id, q_blocks), pair = pair_of_xcd * 8 + xcd, qblock = slot_id - pair_of_xcd * q_blocks;
   if (pair >= batch * heads) return;
-  const int head = pair % heads;
-  const int b = min(max(seq_start[batch + 1 + pair / heads], 0), batch - 1);
+  const int place = uniform_div(pair, heads), head = pair - place * heads;
+  const int b = min(max(seq_start[batch + 1 + place], 0), batch - 1);
   const int t0 = seq_start[b], t1 = seq_start[b + 1];
   const int len = t1 - t0;
   if (len <= 0) return;
@@ -1053,8 +1052,8 @@ void attention_flash_launch(const void* q, const void* k, const void* v, int lay
     const int q_blocks = (seq_len + queries - 1) / queries;
     allow_dynamic_lds(reinterpret_cast<const void*>(kern), kFlSmem);
     kern<<<pairs8 * q_blocks, kFlWaves * kWave, kFlSmem, stream>>>(
-        (const _Float16*)q, (const _Float16*)k, (const _Float16*)v, layout, packed_ld, (const _Float16*)attr_mask, mask_class,
-        (_Float16*)dst, seq_start, word_idx, batch, seq_len, heads, q_blocks, scaler);
+        seq_start, batch, heads, q_blocks, seq_len, layout, packed_ld, (const _Float16*)q, (const _Float16*)k, (const _Float16*)v, word_idx,
+        (const _Float16*)attr_mask, mask_class, (_Float16*)dst, scaler);
   };
   // Two query tiles per wavefront halve the LDS reads per score; with few workgroups the CUs are better filled by twice as
   // many of one tile.
@@ -1082,10 +1081,10 @@ constexpr int kF32MinKeys = 32;
 constexpr int kF32Smem = 2 * 2 * kF32Stage + kFlMaxKeys * (int)sizeof(int);
 
 __global__ __launch_bounds__(kAttnThreads, 4) void attention_flash_f32_kernel(
-    const float* __restrict__ q_src, const float* __restrict__ k_src, const float* __restrict__ v_src, int layout, int packed_ld,
-    const float* __restrict__ attr_mask, const uint8_t* __restrict__ mask_class, float* __restrict__ dst,
-    const int32_t* __restrict__ seq_start, const int32_t* __restrict__ word_idx, int batch, int seq_len, int heads, int q_blocks,
-    float scaler, int split_out, PairContext ctx) {
+    const int32_t* __restrict__ seq_start, int batch, int heads, int q_blocks, int seq_len, int layout, int packed_ld,
+    const float* __restrict__ q_src, const float* __restrict__ k_src, const float* __restrict__ v_src,
+    const int32_t* __restrict__ word_idx, const float* __restrict__ attr_mask, const uint8_t* __restrict__ mask_class,
+    float* __restrict__ dst, float scaler, int split_out, PairContext ctx) {
 #if defined(__HIP_DEVICE_COMPILE__)   // device-only types in the body; the host pass only needs the stub
   extern __shared__ __attribute__((aligned(1024))) unsigned char smem_raw[];
   unsigned char* kv = smem_raw;                                        // [stage][K, V]
@@ -1093,10 +1092,10 @@ __global__ __launch_bounds__(kAttnThreads, 4) void attention_flash_f32_kernel(
 
   // the query blocks of one (head, sequence) go to one XCD, as above
   const int xcd = blockIdx.x & 7, slot_id = blockIdx.x >> 3;
-  const int pair = (slot_id / q_blocks) * 8 + xcd, qblock = slot_id % q_blocks;
+  const int pair_of_xcd = uniform_div(slot_id, q_blocks), pair = pair_of_xcd * 8 + xcd, qblock = slot_id - pair_of_xcd * q_blocks;
   if (pair >= batch * heads) return;
-  const int head = pair % heads;
-  const int b = min(max(seq_start[batch + 1 + pair / heads], 0), batch - 1);
+  const int place = uniform_div(pair, heads), head = pair - place * heads;
+  const int b = min(max(seq_start[batch + 1 + place], 0), batch - 1);
   const int t0 = seq_start[b], t1 = seq_start[b + 1];
   const int len = t1 - t0;
   if (len <= 0) return;
@@ -1357,8 +1356,8 @@ void attention_flash_f32_launch(const void* q, const void* k, const void* v, int
   const int q_blocks = (seq_len + 63) / 64;
   const int grid = (batch * heads + 7) / 8 * 8 * q_blocks;
   attention_flash_f32_kernel<<<grid, kAttnThreads, kF32Smem, stream>>>(
-      (const float*)q, (const float*)k, (const float*)v, layout, packed_ld, (const float*)attr_mask, mask_class, (float*)dst,
-      seq_start, word_idx, batch, seq_len, heads, q_blocks, scaler, split_out ? 1 : 0, ctx);
+      seq_start, batch, heads, q_blocks, seq_len, layout, packed_ld, (const float*)q, (const float*)k, (const float*)v, word_idx,
+      (const float*)attr_mask, mask_class, (float*)dst, scaler, split_out ? 1 : 0, ctx);
 }
 
 // ------------------------------------------------------------------------------------------
