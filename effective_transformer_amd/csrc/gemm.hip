@@ -906,23 +906,6 @@ __host__ __device__ inline int pair_row_blocks(int rows, int tiles_n, int wgs) {
   return best_mi;
 }
 
-// The tile height for the row count that only the device knows (a height for the launch's bound of 11501 rows takes 34 us for the
-// Q/K/V projection of the 7161 rows that are there, the right one 27; FFN-down of 9526 out of 16384: 54 and 45 us).
-template <bool GELU, bool NT, bool A3>
-__global__ __launch_bounds__(kPThreads) void gemm_f16_pair_rows_kernel(ET_HEAD_ARGS, GemmArgs args) {
-  extern __shared__ __attribute__((aligned(1024))) unsigned char smem[];
-  const TileHead head = tile_head(a0, b0, rows_dev, m_bound, n, k, groups, args);
-  // (below 128 tiles of 256 rows, where this kernel would not run if the host knew, the lowest tile: FFN-down of 7161 rows 47 us,
-  // 51 on shared tiles of 192)
-  const bool few = (int)((unsigned)(head.rows + 255) / 256) * tiles_n * groups < 128;
-  switch (few ? 5 : pair_row_blocks(head.rows, tiles_n * groups, walk >> kWalkWgs)) {
-    case 8: return pair_tiles<GELU, 8, NT, A3>(head, tiles_n, columns, walk, args, smem);
-    case 7: return pair_tiles<GELU, 7, NT, A3>(head, tiles_n, columns, walk, args, smem);
-    case 6: return pair_tiles<GELU, 6, NT, false>(head, tiles_n, columns, walk, args, smem);
-    default: return pair_tiles<GELU, 5, NT, false>(head, tiles_n, columns, walk, args, smem);
-  }
-}
-
 // ------------------------------------------------------------------------------------------
 // fp16, problems below the persistent regime, B k-contiguous ([n][k]): one (32 MI) x (32 NJ) tile per workgroup,
 // 4 wavefronts (2 x 2), LDS slots of two k-steps like the persistent kernel above.  MI = 1 .. 4 blocks of 32 rows,
@@ -1179,6 +1162,40 @@ __global__ __launch_bounds__(kHThreads) __attribute__((amdgpu_waves_per_eu(2))) 
   }
   ET_BT_ROWS_TILES(ET_BT_CASE)
 #undef ET_BT_CASE
+}
+
+// The persistent kernel where only the device knows the row count: it picks the tile height (a height for the launch's bound of 11501
+// rows takes 34 us for the Q/K/V projection of the 7161 rows that are there, the right one 27; FFN-down of 9526 out of 16384: 54 and
+// 45 us).  Below 128 tiles of 256 rows, where the host would not have launched it, the rows go to tiles with a CU to themselves as
+// far as one round of them lasts, by half of the wavefronts (FFN-down of 6900 rows in a launch for 11501: 36 us, 49 on the lowest
+// tiles of this kernel; attention output 14.6 and 17.6; FFN-down of 2300 rows 18.6 and 46).
+template <bool GELU, bool NT, bool A3>
+__global__ __launch_bounds__(kPThreads) void gemm_f16_pair_rows_kernel(ET_HEAD_ARGS, GemmArgs args) {
+  extern __shared__ __attribute__((aligned(1024))) unsigned char smem[];
+  const TileHead head = tile_head(a0, b0, rows_dev, m_bound, n, k, groups, args);
+  if ((int)((unsigned)(head.rows + 255) / 256) * tiles_n * groups < 128) {
+#define ET_BT_CASE(MI, NJ, ST)                                                                                          \
+  {                                                                                                                      \
+    const int bt_n = (int)((unsigned)(n + 32 * NJ - 1) / (32 * NJ)), all_n = bt_n * groups;                              \
+    const int total = (int)((unsigned)(head.rows + 32 * MI - 1) / (32 * MI)) * all_n;                                    \
+    static_assert(BtTile<MI, NJ, ST>::SMEM_BYTES <= kQSmem);                                                             \
+    if (total <= (walk >> kWalkWgs) * kXcds) {                                                                           \
+      const int tile = remap_valid_tile(blockIdx.x, total);                                                              \
+      if (tile < 0 || threadIdx.x >= kHThreads) return;                                                                  \
+      const int tm = uniform_div(tile, all_n);                                                                           \
+      return bt_tile<MI, NJ, ST>(head, bt_n, args, tm, tile - tm * all_n, smem);                                         \
+    }                                                                                                                    \
+  }
+    ET_BT_CASE(2, 4, 4) ET_BT_CASE(3, 4, 4) ET_BT_CASE(4, 4, 4) ET_BT_CASE(4, 6, 3)
+#undef ET_BT_CASE
+    return pair_tiles<GELU, 5, NT, false>(head, tiles_n, columns, walk, args, smem);
+  }
+  switch (pair_row_blocks(head.rows, tiles_n * groups, walk >> kWalkWgs)) {
+    case 8: return pair_tiles<GELU, 8, NT, A3>(head, tiles_n, columns, walk, args, smem);
+    case 7: return pair_tiles<GELU, 7, NT, A3>(head, tiles_n, columns, walk, args, smem);
+    case 6: return pair_tiles<GELU, 6, NT, false>(head, tiles_n, columns, walk, args, smem);
+    default: return pair_tiles<GELU, 5, NT, false>(head, tiles_n, columns, walk, args, smem);
+  }
 }
 
 // ------------------------------------------------------------------------------------------
