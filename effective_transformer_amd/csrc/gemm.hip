@@ -1644,18 +1644,27 @@ void launch_f16_persistent(GemmArgs a, hipStream_t stream, bool b_transposed) {
 // Tile of the one-tile-per-workgroup k-contiguous kernel.  A workgroup's k loop runs at the rate its CU's load path
 // delivers operand rows, MI + NJ units of 4 KB per pair of k-steps, so the launch takes about as long as the busiest
 // CU's units: the smallest tile that still gives every workgroup a CU to itself ("solo", ring of 3 to 5 slots), or
-// two workgroups per CU ("duo", rings that fit twice into the LDS) where 2 (MI + NJ) / 1.3 is less: two resident
-// workgroups draw 1.3 times the rows of one.  A 96-column wave tile stores in two pieces and counts one unit more.
+// two workgroups per CU ("duo", rings that fit twice into the LDS) where 2 (MI + NJ) / 1.25 is less: two resident
+// workgroups draw 1.25 times the rows of one.  A 96-column wave tile stores in two pieces and counts half a unit more.
+// Filling the ring and storing C pass under the other workgroup's loop in a duo and are added in a solo launch, half a unit of
+// one pair for every 32 x 32 of the tile (3400 x 2304, k = 768: 128 x 256 solo 19.4 us, 128 x 128 duo 17.4; 7500 x 1024, k = 4096:
+// 56.8 and 58.9).
 // 32 x 32 is for launches that stay within a round with it (320 rows at n = 768; up to 32 rows: k = 768 / 3072 5.1 / 9.7 us
 // on 32 x 64, 4.5 / 8.3 us on it; 12 layers on one query 469 -> 439 us, on 180 rows 539 -> 518 us).
-// Ties go to the tile whose XCD bands touch fewer distinct operand rows.  (Timed for n = 768 .. 4096, k = 768 .. 4096,
-// 250 .. 16000 rows with the weights of twelve layers taking turns: within 2 % of the best tile on average.)
+// Ties go to the wider tile where the k loop is short (it stores C in longer pieces: 450 x 4096, k = 1024: 64 x 128 10.0 us, 128 x 64
+// 10.6), and else to the tile whose XCD bands touch fewer distinct operand rows (1800 x 1024, k = 4096: 25.2 and 22.9).
+// (Timed for n = 512 .. 4096, k = 512 .. 4096, 130 .. 9000 rows with the weights of four layers taking turns: within 0.7 % of the best
+// tile on average, at most 11 %; without the share for filling and storing 1.4 %, at most 13 %.)
+inline float bt_cost(int mi, int nj, bool duo, int k) {
+  const float units = ((float)(mi + nj) + (nj == 6 ? 0.5f : 0.f)) * (float)(k / 64);
+  return duo ? 2.f / 1.25f * units : units + 0.5f * (float)(mi * nj);
+}
 struct BtPick {
   int mi = 0, nj = 0;      // mi == 0: no tile keeps the launch within two workgroups per CU
   bool duo = false;
 };
 
-BtPick pick_bt_tile(int m_bound, int n, int groups, int cus, bool proven_only) {
+BtPick pick_bt_tile(int m_bound, int n, int k, int groups, int cus, bool proven_only) {
   BtPick best;
   float best_cost = 0.f;
   long best_band = 0;
@@ -1667,18 +1676,10 @@ BtPick pick_bt_tile(int m_bound, int n, int groups, int cus, bool proven_only) {
     const int mi = tile.mi, nj = tile.nj;
     const long tiles_n = (long)((n + 32 * nj - 1) / (32 * nj)) * groups;
     const long wgs = (long)((m_bound + 32 * mi - 1) / (32 * mi)) * tiles_n;
-    const float units = (float)(mi + nj + (nj == 6 ? 1 : 0));
-    float cost;
-    bool duo = false;
-    if (wgs <= cus) {
-      cost = units;
-    } else if (wgs <= 2L * cus && tile.duo && !(proven_only && nj > 4)) {
-      cost = 2.f * units / 1.3f;
-      duo = true;
-    } else {
-      continue;
-    }
-    const long band = band_rows((m_bound + 32 * mi - 1) / (32 * mi), tiles_n, 32 * mi, 32 * nj).along;
+    const bool duo = wgs > cus;
+    if (duo && !(wgs <= 2L * cus && tile.duo && !(proven_only && nj > 4))) continue;
+    const float cost = bt_cost(mi, nj, duo, k);
+    const long band = k < 2048 ? -nj : band_rows((m_bound + 32 * mi - 1) / (32 * mi), tiles_n, 32 * mi, 32 * nj).along;
     if (best.mi == 0 || cost < best_cost || (cost == best_cost && band < best_band)) {
       best.mi = mi;
       best.nj = nj;
@@ -1725,7 +1726,7 @@ bool launch_bt_rows(GemmArgs a, hipStream_t stream) {
     float cost;
     int rows, tiles_n;
   } tiles[] = {
-#define ET_BT_CASE(MI, NJ, DUO, ST) {0, MI, NJ, BtTile<MI, NJ, ST>::SMEM_BYTES, (float)(MI + NJ + (NJ == 6 ? 1 : 0)), 0, 0},
+#define ET_BT_CASE(MI, NJ, DUO, ST) {0, MI, NJ, BtTile<MI, NJ, ST>::SMEM_BYTES, bt_cost(MI, NJ, false, a.k), 0, 0},
       ET_BT_ROWS_TILES(ET_BT_CASE)
 #undef ET_BT_CASE
   };
@@ -1757,9 +1758,8 @@ bool launch_bt_rows(GemmArgs a, hipStream_t stream) {
     ++picks;
   }
   if (served < a.m_bound || picks < 2) return false;
-  const BtPick best = pick_bt_tile(a.m_bound, a.n, a.groups, cus, false);
-  const float best_cost = (float)(best.mi + best.nj + (best.nj == 6 ? 1 : 0)) * (best.duo ? 2.f / 1.3f : 1.f);
-  if (best.mi != 0 && cost > 1.05f * best_cost) return false;
+  const BtPick best = pick_bt_tile(a.m_bound, a.n, a.k, a.groups, cus, false);
+  if (best.mi != 0 && cost > 1.05f * bt_cost(best.mi, best.nj, best.duo, a.k)) return false;
   allow_dynamic_lds(reinterpret_cast<const void*>(gemm_f16_bt_rows_kernel), 160 * 1024);
   gemm_f16_bt_rows_kernel<<<(int)((wgs + kXcds - 1) / kXcds * kXcds), kHThreads, lds, stream>>>(a.A[0], a.B[0], a.rows_dev, a.m_bound, a.n, a.k,
                                                                                                  a.groups, 0, 0, 0, plan, a);
@@ -1777,7 +1777,7 @@ bool use_persistent(int m_bound, int ldc, int n, int k, int groups) {
 // 128 x 256 tiles or two workgroups of 128 x 128 per CU (2000 rows at n = 4096, k = 1024: 21 us against 27; 8000 rows
 // at n = 1024, k = 4096: 59 against 73); narrower duo tiles only tie with the persistent kernel there.
 bool use_persistent_bt(int m_bound, int ldc, int n, int k, int groups) {
-  return use_persistent(m_bound, ldc, n, k, groups) && pick_bt_tile(m_bound, n, groups, device_cu_count(), true).mi == 0;
+  return use_persistent(m_bound, ldc, n, k, groups) && pick_bt_tile(m_bound, n, k, groups, device_cu_count(), true).mi == 0;
 }
 
 // ------------------------------------------------------------------------------------------
@@ -1913,7 +1913,7 @@ void launch_gemm(DType t, const GemmGroups& g, void* C, int ldc, int m_bound, in
       // one tile per workgroup, the tile chosen for the launch's shape (pick_bt_tile)
       if (launch_bt_wave(a, stream)) return;
       if (rows_dev != nullptr && launch_bt_rows(a, stream)) return;
-      launch_bt_tile(pick_bt_tile(m_bound, n, g.groups, device_cu_count(), false), a, stream);
+      launch_bt_tile(pick_bt_tile(m_bound, n, k, g.groups, device_cu_count(), false), a, stream);
     } else {
       // Below a round of the chip the time of a launch is the k loop of one tile.  With fewer 64 x 256 tiles than CUs
       // that loop runs at the rate one CU's DMA fills its LDS: the 64 x 128 tile halves the B bytes per workgroup and
