@@ -333,6 +333,7 @@ struct LayerCall {
   int rows;                           // launches are sized for this many rows
   bool rows_exact = false;            //   ... which is the count itself: no kernel asks the device for it
   char* workspace;
+  const et::PairRowsJob* input = nullptr;   // fp32 on pair rows: what makes `from` and its pair rows, with this call's first launch
   bool from_split_ready = false;      // fp32: the split (pair) rows of `from` are in the workspace's intermediate already
   bool write_out_split = false;       //   ... and those of `out` are to be left there
   hipStream_t stream;
@@ -397,15 +398,21 @@ et_status run_layer_pairs(et_handle h, const LayerCall& c) {
   weight(w->inter_kernel, pp.inter_kernel_t, H, F, 4, w->inter_bias, pw.up_stats);
   weight(w->output_kernel, pp.output_kernel_t, F, H, 8, nullptr, nullptr);
   const et::BatchJobs batch = layer_batch_jobs(c, ws);
-  et::launch_pair_weights(jobs, st, &batch);
-
   // the inputs, in the room of the intermediate, which nothing needs before they have been read
   et::PairRows from = first_pair_rows(base, ws, B, S, H), to = from;
-  if (!c.from_split_ready) et::launch_pair_rows((const float*)c.from, nullptr, from, nullptr, nullptr, rows, H, S, T, st);
+  et::PairRowsJob inputs[2];
+  int count = 0;
+  auto input = [&](const void* src, const et::PairRows& out) {
+    et::PairRowsJob& job = inputs[count++];
+    job.src = (const float*)src, job.out = out, job.m = rows, job.n = H, job.rows_dev = T;
+  };
+  if (c.input) inputs[count++] = *c.input;
+  else if (!c.from_split_ready) input(c.from, from);
   if (c.to != c.from) {
     to = {from.rows + (size_t)rows * 2 * H, pw.to_exp, pw.to_norm};
-    et::launch_pair_rows((const float*)c.to, nullptr, to, nullptr, nullptr, rows, H, S, T, st);
+    input(c.to, to);
   }
+  et::launch_pair_weights(jobs, st, &batch, inputs, count);
   et::PairProduct p3;
   p3.groups = 3;
   p3.A[0] = from; p3.A[1] = to; p3.A[2] = to;
@@ -431,7 +438,11 @@ et_status run_layer_pairs(et_handle h, const LayerCall& c) {
   // (where the attention kernel writes floats only, they take the attention output's place until they are paired)
   et::launch_attention(dt, q, k, v, 1, 3 * H, c.attr_mask, attn, seq_start, c.word_idx, B, S, c.heads, c.d,
                        softmax_scaler(c.dtype, c.d), st, false, cls, ctx);
-  if (!ctx_pairs) et::launch_pair_rows(attn, nullptr, ctx_rows, nullptr, nullptr, rows, H, S, T, st);
+  if (!ctx_pairs) {
+    et::PairRowsJob job;
+    job.src = attn, job.out = ctx_rows, job.m = rows, job.n = H, job.rows_dev = T;
+    et::launch_pair_rows(job, st);
+  }
   if ((s = check_launch(h, "attention")) != ET_OK) return s;
 
   auto product = [&](const et::PairRows& a, int w_at, void* C, int n, int k_) {
@@ -998,6 +1009,7 @@ et_status et_encoder(et_handle h, et_dtype dtype, int num_layers, const et_layer
   if (split) extras.split = (uint16_t*)(layer_base + split_off);
   const bool pairs = layer_pairs(dtype, H);
   if (pairs) extras.pair = first_pair_rows(layer_base, layer_ws(dtype, B, S, head_num, size_per_head), B, S, H);
+  et::PairRowsJob input;
   if (b->embeddings) {
     const et_embedding_weights& emb = *b->embeddings;
     et::launch_embed_layernorm(dt, x[0], b->input_ids, b->token_type_ids, batch_idx, word_idx, emb.word_embeddings,
@@ -1005,7 +1017,11 @@ et_status et_encoder(et_handle h, et_dtype dtype, int num_layers, const et_layer
                                emb.max_position_embeddings, emb.layernorm_gamma, emb.layernorm_beta, B * S, H, S, count, st,
                                extras, B);
   } else if (pairs) {
-    et::launch_pair_rows((const float*)b->from_tensor, (float*)x[0], extras.pair, batch_idx, word_idx, B * S, H, S, count, st, seq, B);
+    input.src = (const float*)b->from_tensor, input.packed = (float*)x[0], input.out = extras.pair;
+    input.batch_idx = batch_idx, input.word_idx = word_idx, input.m = B * S, input.n = H, input.seq_len = S, input.rows_dev = count;
+    input.seq_table = seq, input.batch = B;
+    // (while the host waits for the count there is nothing else to do; where it does not, the first layer's weights take it along)
+    if (wait_for_layers) et::launch_pair_rows(input, st);
   } else {
     et::launch_compress_rows(b->from_tensor, x[0], batch_idx, word_idx, count, nullptr, nullptr, B, S, (int)row_bytes, st,
                              extras);
@@ -1044,6 +1060,7 @@ et_status et_encoder(et_handle h, et_dtype dtype, int num_layers, const et_layer
     c.from = c.to = x[cur];
     c.out = x[cur ^ 1];
     c.from_split_ready = split || pairs;
+    c.input = l == 0 && input.src && !wait_for_layers ? &input : nullptr;
     c.write_out_split = l + 1 < num_layers;
     if ((s = run_layer(h, c)) != ET_OK) return s;
     cur ^= 1;
@@ -1366,7 +1383,9 @@ et_status et_pair_rows(et_handle h, const void* src, const et_pair_matrix* dst, 
   ET_REQUIRE(h, m >= 0, "bad dimensions");
   if (!et::pair_rows_supported(k)) return fail(h, ET_UNSUPPORTED, "k must be a multiple of 64 up to 2048");
   const et::PairRows out{(_Float16*)dst->rows, dst->exp, dst->norm};
-  et::launch_pair_rows((const float*)src, nullptr, out, nullptr, nullptr, m, k, 0, m_dev, (hipStream_t)stream);
+  et::PairRowsJob job;
+  job.src = (const float*)src, job.out = out, job.m = m, job.n = k, job.rows_dev = m_dev;
+  et::launch_pair_rows(job, (hipStream_t)stream);
   return check_launch(h, "pair rows");
 }
 

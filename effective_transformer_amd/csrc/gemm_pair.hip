@@ -472,22 +472,18 @@ void launch_pick(PairPick pick, const PairGemmArgs& a, bool gelu, int groups, hi
 // Rows into pair rows: one wavefront per row, which stays in registers (n <= 256 ITERS, a multiple of 4).  With indices the
 // source is the padded tensor, and the packed rows are written as well; then the first workgroup sorts the batch's table.
 template <int ITERS>
-__global__ __launch_bounds__(256) void pair_rows_kernel(const float* __restrict__ src, float* __restrict__ packed, PairRows out,
-                                                        const int32_t* __restrict__ batch_idx,
-                                                        const int32_t* __restrict__ word_idx, int m, int n, int seq_len,
-                                                        const int32_t* __restrict__ rows_dev, int32_t* __restrict__ seq_table,
-                                                        int batch) {
-  const int first = seq_table ? 1 : 0;
-  if (first && blockIdx.x == 0) {
-    sort_sequences<256>(seq_table, batch, seq_table + batch + 1);
+__device__ __forceinline__ void pair_rows_blocks(const PairRowsJob& job, int block, int blocks) {
+  const int first = job.seq_table ? 1 : 0;
+  if (first && block == 0) {
+    sort_sequences<256>(job.seq_table, job.batch, job.seq_table + job.batch + 1);
     return;
   }
-  const int rows = rows_dev ? min(*rows_dev, m) : m;
+  const int rows = job.rows_dev ? min(*job.rows_dev, job.m) : job.m, n = job.n;
   const int lane = threadIdx.x & (kWave - 1);
   const int vpr = n / 4;
-  for (int r = ((int)blockIdx.x - first) * 4 + threadIdx.x / kWave; r < rows; r += ((int)gridDim.x - first) * 4) {
-    const size_t from = batch_idx ? (size_t)batch_idx[r] * seq_len + word_idx[r] : (size_t)r;
-    const float4v* s = reinterpret_cast<const float4v*>(src + from * n);
+  for (int r = (block - first) * 4 + threadIdx.x / kWave; r < rows; r += (blocks - first) * 4) {
+    const size_t from = job.batch_idx ? (size_t)job.batch_idx[r] * job.seq_len + job.word_idx[r] : (size_t)r;
+    const float4v* s = reinterpret_cast<const float4v*>(job.src + from * n);
     float4v x[ITERS];
 #pragma unroll
     for (int i = 0; i < ITERS; ++i) {
@@ -495,12 +491,17 @@ __global__ __launch_bounds__(256) void pair_rows_kernel(const float* __restrict_
       x[i] = float4v{0.f, 0.f, 0.f, 0.f};
       if (c < vpr) {
         x[i] = s[c];
-        if (packed) reinterpret_cast<float4v*>(packed + (size_t)r * n)[c] = x[i];
+        if (job.packed) reinterpret_cast<float4v*>(job.packed + (size_t)r * n)[c] = x[i];
       }
     }
-    store_pair_row<ITERS>(x, vpr, out, r, n);
+    store_pair_row<ITERS>(x, vpr, job.out, r, n);
   }
 }
+template <int ITERS>
+__global__ __launch_bounds__(256) void pair_rows_kernel(PairRowsJob job) {
+  pair_rows_blocks<ITERS>(job, blockIdx.x, gridDim.x);
+}
+inline int pair_rows_grid(const PairRowsJob& job) { return std::min((job.m + 3) / 4, 2048) + (job.seq_table ? 1 : 0); }
 
 // Weights into n pair rows in two launches, whose loads are whole lines (one launch of workgroups that hold all k of 16 columns
 // took 35 .. 45 us at H = 768; exponents that go by chunks of 64 k and are applied where a chunk is added need one launch, and
@@ -510,7 +511,12 @@ struct PairWeightArgs {
   int tile_begin[PairWeightJobs::kMax + 1];
 };
 constexpr int kTopRows = 256;
-__global__ __launch_bounds__(256) void pair_weight_top_kernel(PairWeightArgs args, BatchJobs batch) {
+// Rows go along in the first blocks: a launch of their own (8 x 32 tokens: 4 us) would only stand in front of this one.
+struct PairRowsArgs {
+  PairRowsJob job[2];
+  int blocks[2];
+};
+__global__ __launch_bounds__(256) void pair_weight_top_kernel(PairWeightArgs args, BatchJobs batch, PairRowsArgs rows) {
   __shared__ union {
     float part[16][64];
     int32_t starts[kTableBatch + 1];
@@ -522,6 +528,20 @@ __global__ __launch_bounds__(256) void pair_weight_top_kernel(PairWeightArgs arg
     return;
   }
   wg -= batch.blocks;
+  if (wg < rows.blocks[0] + rows.blocks[1]) {
+    const int which = wg < rows.blocks[0] ? 0 : 1;
+    const PairRowsJob& job = rows.job[which];
+    const int block = wg - (which ? rows.blocks[0] : 0), blocks = rows.blocks[which];
+    switch ((job.n / 4 + kWave - 1) / kWave) {
+      case 1: return pair_rows_blocks<1>(job, block, blocks);
+      case 2: return pair_rows_blocks<2>(job, block, blocks);
+      case 3: return pair_rows_blocks<3>(job, block, blocks);
+      case 4: return pair_rows_blocks<4>(job, block, blocks);
+      case 5: case 6: return pair_rows_blocks<6>(job, block, blocks);
+      default: return pair_rows_blocks<8>(job, block, blocks);
+    }
+  }
+  wg -= rows.blocks[0] + rows.blocks[1];
   int job = 0;
   while (job + 1 < args.jobs.count && wg >= args.tile_begin[job + 1]) ++job;
   const PairWeightJob& jb = args.jobs.job[job];
@@ -654,14 +674,11 @@ bool gemm_pair_supported(int n, int k) {
   return k % 64 == 0 && k >= 64 && n % 16 == 0 && (uint64_t)k * 4u * 256u < 0x80000000ull;
 }
 
-void launch_pair_rows(const float* src, float* packed, const PairRows& out, const int32_t* batch_idx, const int32_t* word_idx,
-                      int m, int n, int seq_len, const int32_t* rows_dev, hipStream_t stream, int32_t* seq_table, int batch) {
-  if (m <= 0) return;
-  const int grid = std::min((m + 3) / 4, 2048) + (seq_table ? 1 : 0);
-  auto go = [&](auto kern) {
-    kern<<<grid, 256, 0, stream>>>(src, packed, out, batch_idx, word_idx, m, n, seq_len, rows_dev, seq_table, batch);
-  };
-  switch ((n / 4 + kWave - 1) / kWave) {
+void launch_pair_rows(const PairRowsJob& job, hipStream_t stream) {
+  if (job.m <= 0) return;
+  const int grid = pair_rows_grid(job);
+  auto go = [&](auto kern) { kern<<<grid, 256, 0, stream>>>(job); };
+  switch ((job.n / 4 + kWave - 1) / kWave) {
     case 1: return go(pair_rows_kernel<1>);
     case 2: return go(pair_rows_kernel<2>);
     case 3: return go(pair_rows_kernel<3>);
@@ -674,7 +691,7 @@ void launch_pair_rows(const float* src, float* packed, const PairRows& out, cons
 
 bool pair_rows_supported(int n) { return n % 64 == 0 && n >= 64 && n <= 2048; }
 
-void launch_pair_weights(const PairWeightJobs& jobs, hipStream_t stream, const BatchJobs* batch) {
+void launch_pair_weights(const PairWeightJobs& jobs, hipStream_t stream, const BatchJobs* batch, const PairRowsJob* rows, int row_jobs) {
   if (jobs.count == 0) return;
   PairWeightArgs a;
   a.jobs = jobs;
@@ -689,7 +706,12 @@ void launch_pair_weights(const PairWeightJobs& jobs, hipStream_t stream, const B
   };
   const int tops = grid(kTopRows);
   const BatchJobs b = batch ? *batch : BatchJobs();
-  pair_weight_top_kernel<<<tops + b.blocks, 256, 0, stream>>>(a, b);
+  PairRowsArgs r = {};
+  for (int j = 0; j < row_jobs; ++j) {
+    r.job[j] = rows[j];
+    r.blocks[j] = rows[j].m > 0 ? pair_rows_grid(rows[j]) : 0;
+  }
+  pair_weight_top_kernel<<<tops + b.blocks + r.blocks[0] + r.blocks[1], 256, 0, stream>>>(a, b, r);
   if (b.seq_table && !b.one_block_table) launch_seq_order(b.seq_table, b.batch, stream);
   const int tiles = grid(64);
   pair_weight_kernel<<<tiles, 256, 0, stream>>>(a);

@@ -220,9 +220,17 @@ bool gemm_pair_supported(int n, int k);
 bool pair_rows_supported(int n);
 // float rows -> pair rows.  With batch_idx / word_idx: gathered from the padded tensor, the float rows go to `packed` too;
 // seq_table: its second half is filled in on the way.
-void launch_pair_rows(const float* src, float* packed, const PairRows& out, const int32_t* batch_idx, const int32_t* word_idx,
-                      int m, int n, int seq_len, const int32_t* rows_dev, hipStream_t stream, int32_t* seq_table = nullptr,
-                      int batch = 0);
+struct PairRowsJob {
+  const float* src = nullptr;
+  float* packed = nullptr;            // the packed rows as they are, with indices only (may be null)
+  PairRows out;
+  const int32_t *batch_idx = nullptr, *word_idx = nullptr;      // of the packed rows in the padded src; null: src is packed
+  int m = 0, n = 0, seq_len = 0;
+  const int32_t* rows_dev = nullptr;
+  int32_t* seq_table = nullptr;       // starts of `batch` sequences; their order is added (see sort_sequences)
+  int batch = 0;
+};
+void launch_pair_rows(const PairRowsJob& job, hipStream_t stream);
 struct PairWeightJob {
   const void* src;                   // float [k][n], or (src_split) its n split rows
   bool src_split;
@@ -240,7 +248,9 @@ struct PairWeightJobs {
   PairWeightJob job[kMax] = {};
   int count = 0;
 };
-void launch_pair_weights(const PairWeightJobs& jobs, hipStream_t stream, const BatchJobs* batch = nullptr);
+// (`rows`: up to two jobs of launch_pair_rows that go along)
+void launch_pair_weights(const PairWeightJobs& jobs, hipStream_t stream, const BatchJobs* batch = nullptr, const PairRowsJob* rows = nullptr,
+                         int row_jobs = 0);
 // C[:, g n : (g + 1) n] = A[g].B[g] + bias[g] (bias may be null), float with leading dimension ldc; with c_exp
 // C = gelu(A.B + bias) as pair rows of ldc values, from A[0].norm and the weights' `stats`.
 struct PairProduct {
