@@ -366,7 +366,7 @@ et_status et_transpose_weight(et_handle h, et_dtype dtype, const void* src, void
 
 /* et_gemm with the second operand k-contiguous: C[m,n] = A[m,k] . Bt[n,k]^T (+ bias), fp16 only.  This is the kernel
  * et_layer runs where it has such a copy of a weight (same cublasGemmEx call sites as et_gemm): a persistent kernel
- * from 128 tiles of 256x256 on, one tile of 32x64 .. 128x128 per workgroup below that.  Same bits as et_gemm on the
+ * from 128 tiles of 256x256 on, one tile of 16x16 .. 128x256 per workgroup below that.  Same bits as et_gemm on the
  * same operands.  ET_UNSUPPORTED for k % 64 != 0 or n % 8 != 0. */
 et_status et_gemm_bt(et_handle h, et_dtype dtype, const void* A, const void* Bt, void* C, const void* bias,
                      int m, int n, int k, const int32_t* m_dev, void* stream);
