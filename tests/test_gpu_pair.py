@@ -116,3 +116,40 @@ def test_layer(heads, d, B, S, scale):
     # (the oracle is float32 itself: about 1e-7 per product on either side, eight of them in a row)
     assert (got[~valid] == 0).all()
     assert np.linalg.norm(got[valid] - want[valid]) <= 2e-6 * np.linalg.norm(want[valid])
+
+
+# attention that takes Q, K and V as pair rows (more than 32 positions): lengths around its stages of 32 keys and blocks of 64
+# queries, holes, masks that are read and masks that are not, rows of a mask on 16-byte boundaries and odd ones; wide: scores tens
+# apart, so that the exponents' reference moves
+@pytest.mark.parametrize("S", [33, 64, 101, 200, 1024])
+@pytest.mark.parametrize("wide", [False, True])
+def test_attention_on_pair_rows(S, wide):
+    print("attention on pair rows", S, wide, flush=True)
+    heads, d, H = 8, 64, 512
+    rng = np.random.RandomState(S)
+    w = []
+    for i in range(4):
+        w += [rng.randn(H, H).astype(np.float32) * (0.2 if wide and i < 2 else 0.02), rng.randn(H).astype(np.float32) * 0.02]
+    w += [rng.randn(H).astype(np.float32) * 0.05, 1 + rng.randn(H).astype(np.float32) * 0.05,
+          rng.randn(H, 4 * H).astype(np.float32) * 0.02, rng.randn(4 * H).astype(np.float32) * 0.02,
+          rng.randn(4 * H, H).astype(np.float32) * 0.02, rng.randn(H).astype(np.float32) * 0.02,
+          rng.randn(H).astype(np.float32) * 0.05, 1 + rng.randn(H).astype(np.float32) * 0.05]
+    lens = np.minimum([1, 31, 32, 33, S // 2, S - 1, S] if S < 1024 else [S, 65, S // 2], S)
+    B = len(lens)
+    mask = (np.arange(S)[None] < lens[:, None]).astype(np.int32)
+    mask[-1, S // 8:S // 4] = 0                              # a hole
+    attr = np.ascontiguousarray(np.broadcast_to(mask[:, None], (B, S, S))).astype(np.float32)
+    attr[1] = np.tril(attr[1])                               # causal
+    attr[2] = 1                                              # every key
+    attr[-2, : S // 2] = rng.random_sample((S // 2, S)) < 0.6
+    x = rng.randn(B, S, H).astype(np.float32)
+    got = ops.EffectiveTransformerEncoder(1, heads, d, [dev(t) for t in w], torch.float32)(dev(x), dev(mask), dev(attr)).cpu().numpy()
+    want = o.encoder(x, mask, attr, w, heads, d, "fp32").astype(np.float64)
+    valid = mask.astype(bool)
+    # as above, and what the roundings of a score (a few units of the sum of its products, on either side) make of a weight
+    q, k_ = (np.abs(x[valid] @ w[2 * i]).reshape(-1, heads, d) for i in range(2))
+    score = np.sqrt((q ** 2).sum(-1)).max() * np.sqrt((k_ ** 2).sum(-1)).max() / 8
+    tol = 2e-6 + 4 * 2.0 ** -24 * score
+    assert (got[~valid] == 0).all()
+    assert np.linalg.norm(got[valid] - want[valid]) <= tol * np.linalg.norm(want[valid])
+    assert np.abs(got[valid] - want[valid]).max() <= 12 * tol * np.abs(want[valid]).max()
