@@ -1317,11 +1317,13 @@ __global__ __launch_bounds__(kAttnThreads, 4) void attention_flash_f32_kernel(
         const int4x e = *reinterpret_cast<const int4x*>(stage_exps + slot * kF32Exps + (kF32Keys + kt * 16 + g * 4) * 4);
 #pragma unroll
         for (int r = 0; r < 4; ++r) {
-          const float w = __builtin_ldexpf(s[kt][r], min(e[r] - pair_exp, 1) + kWeightBits);
-          ph[kt * 4 + r] = f2h(w);
-          pl[kt * 4 + r] = f2h(w - h2f(ph[kt * 4 + r]));
+          s[kt][r] = __builtin_ldexpf(s[kt][r], min(e[r] - pair_exp, 1) + kWeightBits);
+          ph[kt * 4 + r] = f2h(s[kt][r]);
         }
       }
+      asm("" : "+v"(ph));                                              // pl comes from these halves, as in store_pair
+#pragma unroll
+      for (int i = 0; i < 8; ++i) pl[i] = f2h(s[i >> 2][i & 3] - h2f(ph[i]));
 #pragma unroll
       for (int dt = 0; dt < 4; ++dt) {
         half8 v[2];
