@@ -45,6 +45,7 @@ constexpr int kDppQuadXor1 = 0xB1;      // quad_perm:[1,0,3,2]
 constexpr int kDppQuadXor2 = 0x4E;      // quad_perm:[2,3,0,1]
 constexpr int kDppRowHalfMirror = 0x141;
 constexpr int kDppRowMirror = 0x140;
+constexpr int kDppRowNewBcast = 0x150;  // + n: lane n of every 16 lanes, to all of them
 constexpr int kDppRowBcast15 = 0x142;
 constexpr int kDppRowBcast31 = 0x143;
 

@@ -64,6 +64,14 @@ __device__ __forceinline__ void wait_vmcnt() {
 __device__ __forceinline__ void wait_lgkmcnt0() { __builtin_amdgcn_s_waitcnt(15 | (7 << 4) | (0 << 8) | (3 << 14)); }
 __device__ __forceinline__ void barrier_only() { asm volatile("s_barrier" ::: "memory"); }
 
+// v[i][r]: what lane 4 i + r of the 16 lanes around this one holds
+template <int I, int MI>
+__device__ __forceinline__ void from_lanes(float4v (&v)[MI], float x) {
+  v[I] = float4v{dpp_f32<kDppRowNewBcast + 4 * I>(0.f, x), dpp_f32<kDppRowNewBcast + 4 * I + 1>(0.f, x),
+                 dpp_f32<kDppRowNewBcast + 4 * I + 2>(0.f, x), dpp_f32<kDppRowNewBcast + 4 * I + 3>(0.f, x)};
+  if constexpr (I + 1 < MI) from_lanes<I + 1>(v, x);
+}
+
 // WM x WN wavefronts of MI x NJ blocks of 16 x 16, a ring of ST stages of KS k-steps in LDS.
 template <int WM, int WN, int MI, int NJ, int ST, int KS>
 struct PairTile {
@@ -271,19 +279,20 @@ __global__ __launch_bounds__(WM * WN * kWave) void gemm_pair_kernel(
     fvec bias = {};
     int ce[NJ] = {};
     int4v re[MI] = {};
-    float4v bound[MI] = {};
     const int row0 = cur.m0 + wm * 16 * MI + g * 4;
+    // Pair rows out: the 16 lanes that store the same 4 MI rows see to one row's exponent each, and hand it round (every lane for
+    // all of them was a fifth of an epilogue's instructions: encoders of 500 x 64 2860 -> 2844 us, 4 x 1000 915 -> 906).
+    const int own_row = row0 + min(l16 >> 2, MI - 1) * 16 + (l16 & 3);
+    float own_norm = 0.f;
     auto request = [&](const int32_t* a_exp, const int32_t* b_exp, const float* add, const float* norm) {
+      if constexpr (OUT != kFloat) own_norm = norm[own_row];
       if (col >= N) return;
 #pragma unroll
       for (int j = 0; j < NJ; ++j) ce[j] = b_exp[col + j];
       if (add != nullptr) bias = *reinterpret_cast<const fvec*>(add + col);
       // (the row arrays reach beyond the last tile: PairRows)
 #pragma unroll
-      for (int i = 0; i < MI; ++i) {
-        re[i] = *reinterpret_cast<const int4v*>(a_exp + row0 + i * 16);
-        if constexpr (OUT != kFloat) bound[i] = *reinterpret_cast<const float4v*>(norm + row0 + i * 16);
-      }
+      for (int i = 0; i < MI; ++i) re[i] = *reinterpret_cast<const int4v*>(a_exp + row0 + i * 16);
     };
     if constexpr (!Tile::BIG) request(args.a_exp[cur.grp], args.b_exp[cur.grp], args.bias[cur.grp], args.a_norm[cur.grp]);
     if constexpr (Tile::BIG) {
@@ -372,13 +381,17 @@ __global__ __launch_bounds__(WM * WN * kWave) void gemm_pair_kernel(
       bias[j] = b;
     }
 #pragma unroll
-    for (int i = 0; i < MI; ++i) {
-      asm volatile("" : "+v"(re[i]));
-      if constexpr (OUT != kFloat) asm volatile("" : "+v"(bound[i]));
-    }
+    for (int i = 0; i < MI; ++i) asm volatile("" : "+v"(re[i]));
+    if constexpr (OUT != kFloat) asm volatile("" : "+v"(own_norm));
     if constexpr (OUT == kGelu && !Tile::BIG)
       if (first_tile) bounds = pair_stats_max(args.b_stats[0], args.n_stats, stats);
     if constexpr (OUT == kPairs) bounds = cur.grp == 0 ? linear_bounds[0] : cur.grp == 1 ? linear_bounds[1] : linear_bounds[2];
+    float4v scale[MI];
+    if constexpr (OUT != kFloat) {                 // (every lane is active here)
+      const int e = pair_exponent(own_norm * (bounds[0] * 1.01f) + bounds[1]);
+      from_lanes<0>(scale, pair_scale(e));
+      if (cur.n0 == 0 && wn == 0 && l16 < 4 * MI && own_row < rows) args.c_exp[cur.grp * args.c_stride + own_row] = e;
+    }
     if (col < N) {
 #pragma unroll
       for (int i = 0; i < MI; ++i)
@@ -390,13 +403,11 @@ __global__ __launch_bounds__(WM * WN * kWave) void gemm_pair_kernel(
 #pragma unroll
           for (int j = 0; j < NJ; ++j) o[j] = __builtin_ldexpf(sum[i][j][r] + acc[i][j][r], re[i][r] + ce[j]) + bias[j];
           if constexpr (OUT != kFloat) {
-            const int e = pair_exponent(bound[i][r] * (bounds[0] * 1.01f) + bounds[1]);
             if constexpr (OUT == kGelu) {
 #pragma unroll
               for (int j = 0; j < NJ; ++j) o[j] *= gelu_cdf(o[j], o[j] * o[j] * o[j]);
             }
-            store_pair<NJ>((_Float16*)args.C + (size_t)row * 2 * args.ldc, cur.grp * N + col, o, pair_scale(e));
-            if (col == 0) args.c_exp[cur.grp * args.c_stride + row] = e;
+            store_pair<NJ>((_Float16*)args.C + (size_t)row * 2 * args.ldc, cur.grp * N + col, o, scale[i][r]);
           } else {
             *reinterpret_cast<fvec*>((float*)args.C + (size_t)row * args.ldc + (size_t)cur.grp * N + col) = o;
           }
