@@ -59,6 +59,23 @@ def test_gemm_pair(m, n, kk, positive):
         assert torch.isfinite(act.rows.float()).all() and _rel(act.values(), ref) < 1e-6
 
 
+# pair rows as the result: widths that fill a wavefront's columns in part, rows that end inside the 16 whose exponents 16 lanes
+# share, every tile shape; row by row (another lane's exponent would be off by powers of two), the rows' sizes far apart
+@pytest.mark.parametrize("m,n,kk", [(1, 32, 64), (7, 96, 128), (50, 160, 192), (67, 1056, 768), (331, 800, 512), (1500, 800, 768),
+                                    (3001, 1184, 768), (9003, 1056, 512)])
+def test_pair_rows_out(m, n, kk):
+    print("pair rows out", m, n, kk, flush=True)
+    a, b, bias = _operands(m, n, kk, False)
+    a *= torch.logspace(-3, 1, 5, device="cuda").repeat((m + 4) // 5)[:m, None]
+    pb, stats = k.pair_weight(b, bias)
+    act = k.gemm_pair(k.pair_rows(a), pb, bias=bias, stats=stats, gelu=True).values()
+    want = torch.nn.functional.gelu((a.cpu().double() @ b.cpu().double()).cuda() + bias.double(), approximate="tanh")
+    # the product's own error as above; h + l: half a unit of 2^-22 of a value and 2^-39 of the row's bound; GELU's exp2 and
+    # reciprocal one unit each
+    bound = a.double().norm(dim=1) * b.double().norm(dim=0).max() * 1.02 + bias.abs().max().double()
+    assert ((act - want).norm(dim=1) <= 1e-6 * want.norm(dim=1) + bound * n ** 0.5 * 2.0 ** -38).all()
+
+
 # the exponents take what rows and columns differ by: the same relative error at 1e30, 1e-30 and in between, row by row; zero
 # rows and columns are zero; what a row cannot hold (2^-40 of its largest value) is all that is lost
 def test_magnitudes():
