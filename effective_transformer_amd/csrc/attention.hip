@@ -652,7 +652,6 @@ struct Unseen {
   }
 };
 typedef uint32_t uint4x __attribute__((ext_vector_type(4)));
-typedef int int4x __attribute__((ext_vector_type(4)));
 
 template <typename T>
 __global__ __launch_bounds__(256) void mask_class_kernel(const T* __restrict__ attr_mask, const int32_t* __restrict__ seq_start,
@@ -1072,12 +1071,6 @@ void attention_flash_launch(const void* q, const void* k, const void* v, int lay
 // Bound: the fp32 matrix instructions (a wavefront and stage: 2048 cycles of MFMA, about 400 of VALU, 16 LDS reads) over the
 // rounds of workgroups, long sequences first.  15 x 379 positions / 3820 tokens, 12 heads: 47 us per launch, 104 us with K
 // and V in chunks of 128 keys behind barriers and the scores of a query against all keys in registers.
-// PAIRS: Q, K and V come as pair rows (gemm_pair.hip), three products of halves on v_mfma_f32_16x16x32_f16 for one of floats, 384
-// cycles of MFMA a stage in place of 2048.  A score takes its rows' exponents; a weight takes its key's, against the exponent of the
-// sequence's context rows, and becomes h + l itself; V is read transposed, its chunks XOR-swizzled in pairs with the key.  Bound:
-// VALU (about 600 cycles a stage) and the start of a workgroup.  Encoders of 15 x 379 positions 266 -> 249 us a layer, 4 x 1000 267 ->
-// 227, 64 x 256 556 -> 521, 40 x 128 217 -> 212, 500 x 64 951 -> 947; error against float64 as before (12 layers, 2 x 379: 3.87e-7 and
-// 3.82e-7; 4 x 64: 3.85e-7 and 3.84e-7).
 // ------------------------------------------------------------------------------------------
 constexpr int kF32Keys = 32;                                 // keys per stage
 constexpr int kF32Stage = kF32Keys * kD * 4;                 // bytes of K (and of V) per stage
@@ -1085,10 +1078,8 @@ constexpr int kF32Stage = kF32Keys * kD * 4;                 // bytes of K (and 
 // 91.7 us); beyond, this kernel (12 layers: 7 x 50 1.056 -> 1.025 ms, 500 x 64 17.76 -> 17.61 ms, 9 x 101 1.59 -> 1.39 ms,
 // 40 x 128 4.16 -> 3.91 ms; single layer calls with their masks looked at each time, 200 x 64: 8.30 -> 8.18 ms).
 constexpr int kF32MinKeys = 32;
-constexpr int kF32Exps = 2 * kF32Keys * (int)sizeof(int);    // PAIRS: exponents of a stage's K rows, then of its V rows
-constexpr int kF32Smem = 2 * 2 * kF32Stage + kFlMaxKeys * (int)sizeof(int) + 2 * kF32Exps;
+constexpr int kF32Smem = 2 * 2 * kF32Stage + kFlMaxKeys * (int)sizeof(int);
 
-template <bool PAIRS>
 __global__ __launch_bounds__(kAttnThreads, 4) void attention_flash_f32_kernel(
     const int32_t* __restrict__ seq_start, int batch, int heads, int q_blocks, int seq_len, int layout, int packed_ld,
     const float* __restrict__ q_src, const float* __restrict__ k_src, const float* __restrict__ v_src,
@@ -1097,12 +1088,7 @@ __global__ __launch_bounds__(kAttnThreads, 4) void attention_flash_f32_kernel(
 #if defined(__HIP_DEVICE_COMPILE__)   // device-only types in the body; the host pass only needs the stub
   extern __shared__ __attribute__((aligned(1024))) unsigned char smem_raw[];
   unsigned char* kv = smem_raw;                                        // [stage][K, V]
-  // PAIRS: weights are halves h + l, of which l must not fall below the normal halves for weights that count: up to 2^3 of them, at
-  // most doubled by an exponent, fill the range of a half, and those above 2^-13 have all of l
-  constexpr float kSlack = PAIRS ? 3.f : kFlSlack;
-  constexpr int kWeightBits = 11;
   int* tok_of_pos = reinterpret_cast<int*>(smem_raw + 2 * 2 * kF32Stage);
-  unsigned char* stage_exps = smem_raw + 2 * 2 * kF32Stage + kFlMaxKeys * sizeof(int);
 
   // the query blocks of one (head, sequence) go to one XCD, as above
   const int xcd = blockIdx.x & 7, slot_id = blockIdx.x >> 3;
@@ -1131,18 +1117,10 @@ __global__ __launch_bounds__(kAttnThreads, 4) void attention_flash_f32_kernel(
   for (int i = 0; i < 2; ++i) {
     dma_key[i] = (wave * 2 + i) * 4 + g;
     voff_k[i] = ((uint32_t)dma_key[i] * ld + (uint32_t)(l16 ^ (dma_key[i] & 15)) * 4u) * 4u;
-    voff_v[i] = ((uint32_t)dma_key[i] * ld + (uint32_t)(PAIRS ? l16 ^ ((dma_key[i] & 7) * 2) : l16) * 4u) * 4u;
+    voff_v[i] = ((uint32_t)dma_key[i] * ld + (uint32_t)l16 * 4u) * 4u;
   }
   auto issue = [&](int slot, int st, bool dense, int rows) {
     unsigned char* base = kv + slot * 2 * kF32Stage;
-    if (PAIRS && wave == 0) {                                          // a word per key: K's exponents in the lower lanes, V's in the upper
-      const int key = st * kF32Keys + (lane & (kF32Keys - 1));
-      const int tk = dense ? (key < rows ? key : -1) : (key < kFlMaxKeys ? tok_of_pos[key] : -1);
-      const uint32_t array = lane < kF32Keys ? 1u : 2u;
-      const __amdgpu_buffer_rsrc_t re = __builtin_amdgcn_make_buffer_rsrc(const_cast<int32_t*>(ctx.qkv_exp), 0, 3 * ctx.qkv_stride * 4, 0x00020000);
-      __builtin_amdgcn_raw_ptr_buffer_load_lds(re, ET_ATTN_LDS_PTR(stage_exps + slot * kF32Exps), 4,
-                                               tk >= 0 ? (array * (uint32_t)ctx.qkv_stride + (uint32_t)(t0 + tk)) * 4u : 0x80000000u, 0, 0, 0);
-    }
     const int bytes = (int)(((uint32_t)(rows - 1) * ld + kD) * 4u);
     const __amdgpu_buffer_rsrc_t rk = __builtin_amdgcn_make_buffer_rsrc(const_cast<float*>(kb), 0, bytes, 0x00020000);
     const __amdgpu_buffer_rsrc_t rv = __builtin_amdgcn_make_buffer_rsrc(const_cast<float*>(vb), 0, bytes, 0x00020000);
@@ -1164,16 +1142,14 @@ __global__ __launch_bounds__(kAttnThreads, 4) void attention_flash_f32_kernel(
     }
   };
   int tq;
-  float4v bq[4];                           // features 16 g .. 16 g + 15 of the lane's query; PAIRS: h and l of features 8 g .. of each half
-  int eq = 0;                                                          // PAIRS: exponent of the query's row
+  float4v bq[4];                                                       // features 16 g .. 16 g + 15 of the lane's query
   auto load_q = [&](bool dense, int n) {
     tq = q < n ? (dense ? q : tok_of_pos[q]) : -1;
 #pragma unroll
     for (int i = 0; i < 4; ++i) {
       bq[i] = float4v{0.f, 0.f, 0.f, 0.f};
-      if (tq >= 0) bq[i] = *reinterpret_cast<const float4v*>(qb + (size_t)(layout == 1 ? tq : q) * ld + (PAIRS ? i * 16 + g * 4 : g * 16 + i * 4));
+      if (tq >= 0) bq[i] = *reinterpret_cast<const float4v*>(qb + (size_t)(layout == 1 ? tq : q) * ld + g * 16 + i * 4);
     }
-    if (PAIRS && tq >= 0) eq = ctx.qkv_exp[t0 + tq];
   };
 
   // without a hole in the sequence position p holds token p: requested on that assumption beside what decides it
@@ -1215,7 +1191,6 @@ __global__ __launch_bounds__(kAttnThreads, 4) void attention_flash_f32_kernel(
   // (the queries are waited for here and not in the stage loop, where the wait would cover the DMA)
 #pragma unroll
   for (int i = 0; i < 4; ++i) asm volatile("" : "+v"(bq[i]));
-  if (PAIRS) asm volatile("" : "+v"(eq));
   const int pair_exp = ctx.out.rows != nullptr ? context_exponent(ctx.norm, t0, t1, ctx.stats, ctx.n_stats) : 0;
 
   float ref = kFlLowest, top = -INFINITY, l = 0.f;                     // as above; l: of this lane's keys
@@ -1238,7 +1213,7 @@ __global__ __launch_bounds__(kAttnThreads, 4) void attention_flash_f32_kernel(
   };
   auto move_ref = [&](float mx) {                                      // as above
     const float up = xor_lanes_16_32_max(mx);
-    const float next = up > ref + kSlack ? up : ref;                 // the same in all lanes of a query
+    const float next = up > ref + kFlSlack ? up : ref;                 // the same in all lanes of a query
     const float alpha = __builtin_amdgcn_exp2f(ref - next);
     ref = next;
     l *= alpha;
@@ -1253,25 +1228,14 @@ __global__ __launch_bounds__(kAttnThreads, 4) void attention_flash_f32_kernel(
 #pragma unroll
     for (int kt = 0; kt < 2; ++kt) {
       float4v acc = {0.f, 0.f, 0.f, 0.f};
-      if constexpr (PAIRS) {
-        half8 a[4];                                                    // h and l of features 0 .. 31, then of 32 .. 63
 #pragma unroll
-        for (int i = 0; i < 4; ++i) a[i] = *reinterpret_cast<const half8*>(base + (kt * 16 + l16) * 256 + (((i * 4 + g) ^ l16) * 16));
-        auto mul = [&](int i, int j) { acc = __builtin_amdgcn_mfma_f32_16x16x32_f16(a[i], __builtin_bit_cast(half8, bq[j]), acc, 0, 0, 0); };
-        mul(1, 0), mul(3, 2), mul(0, 1), mul(2, 3), mul(0, 0), mul(2, 2);
-        const int4x e = *reinterpret_cast<const int4x*>(stage_exps + slot * kF32Exps + (kt * 16 + g * 4) * 4);
+      for (int i = 0; i < 4; ++i) {
+        const float4v a = *reinterpret_cast<const float4v*>(base + (kt * 16 + l16) * 256 + (((g * 4 + i) ^ l16) * 16));
 #pragma unroll
-        for (int r = 0; r < 4; ++r) s[kt][r] = __builtin_ldexpf(acc[r], e[r] + eq);
-      } else {
-#pragma unroll
-        for (int i = 0; i < 4; ++i) {
-          const float4v a = *reinterpret_cast<const float4v*>(base + (kt * 16 + l16) * 256 + (((g * 4 + i) ^ l16) * 16));
-#pragma unroll
-          for (int j = 0; j < 4; ++j) acc = __builtin_amdgcn_mfma_f32_16x16x4f32(a[j], bq[i][j], acc, 0, 0, 0);
-        }
-#pragma unroll
-        for (int r = 0; r < 4; ++r) s[kt][r] = acc[r];
+        for (int j = 0; j < 4; ++j) acc = __builtin_amdgcn_mfma_f32_16x16x4f32(a[j], bq[i][j], acc, 0, 0, 0);
       }
+#pragma unroll
+      for (int r = 0; r < 4; ++r) s[kt][r] = acc[r];
     }
     // the exponents' factor: log2 units of the plain scores, of the masked ones otherwise
     const float unit = PLAIN ? c_exp : kLog2e;
@@ -1300,7 +1264,7 @@ __global__ __launch_bounds__(kAttnThreads, 4) void attention_flash_f32_kernel(
       for (int r = 0; r < 4; ++r) mx = fmaxf(mx, s[kt][r]);
     mx *= unit;
     top = fmaxf(top, mx);
-    if (__any(mx > ref + kSlack)) move_ref(mx);                      // the first stage, and seldom after it
+    if (__any(mx > ref + kFlSlack)) move_ref(mx);                      // the first stage, and seldom after it
 #pragma unroll
     for (int kt = 0; kt < 2; ++kt)
 #pragma unroll
@@ -1308,49 +1272,14 @@ __global__ __launch_bounds__(kAttnThreads, 4) void attention_flash_f32_kernel(
         s[kt][r] = __builtin_amdgcn_exp2f(__builtin_fmaf(s[kt][r], unit, -ref));
         l += s[kt][r];
       }
-    if constexpr (PAIRS) {
-      // The weights take their keys' exponents, against that of the sequence's context rows, which is the largest of them (a key
-      // without a row in the stage has a zero row and any exponent).  Element 4 kt + r of a lane is key 16 kt + 4 g + r on both sides.
-      half8 ph, pl;
 #pragma unroll
-      for (int kt = 0; kt < 2; ++kt) {
-        const int4x e = *reinterpret_cast<const int4x*>(stage_exps + slot * kF32Exps + (kF32Keys + kt * 16 + g * 4) * 4);
+    for (int kt = 0; kt < 2; ++kt)
 #pragma unroll
-        for (int r = 0; r < 4; ++r) {
-          s[kt][r] = __builtin_ldexpf(s[kt][r], min(e[r] - pair_exp, 1) + kWeightBits);
-          ph[kt * 4 + r] = f2h(s[kt][r]);
-        }
+      for (int r = 0; r < 4; ++r) {
+        const float4v v = *reinterpret_cast<const float4v*>(base + kF32Stage + (kt * 16 + g * 4 + r) * 256 + l16 * 16);
+#pragma unroll
+        for (int dt = 0; dt < 4; ++dt) o[dt] = __builtin_amdgcn_mfma_f32_16x16x4f32(v[dt], s[kt][r], o[dt], 0, 0, 0);
       }
-      asm("" : "+v"(ph));                                              // pl comes from these halves, as in store_pair
-#pragma unroll
-      for (int i = 0; i < 8; ++i) pl[i] = f2h(s[i >> 2][i & 3] - h2f(ph[i]));
-#pragma unroll
-      for (int dt = 0; dt < 4; ++dt) {
-        half8 v[2];
-#pragma unroll
-        for (int piece = 0; piece < 2; ++piece) {
-          half4 part[2];
-#pragma unroll
-          for (int kt = 0; kt < 2; ++kt) {
-            const int key = kt * 16 + g * 4 + (l16 >> 2), chunk = (dt >> 1) * 8 + piece * 4 + (dt & 1) * 2 + ((l16 >> 1) & 1);
-            part[kt] = read_transposed(base + kF32Stage + key * 256 + ((chunk ^ ((key & 7) * 2)) * 16) + (l16 & 1) * 8);
-          }
-          v[piece] = __builtin_shufflevector(part[0], part[1], 0, 1, 2, 3, 4, 5, 6, 7);
-        }
-        o[dt] = __builtin_amdgcn_mfma_f32_16x16x32_f16(v[1], ph, o[dt], 0, 0, 0);
-        o[dt] = __builtin_amdgcn_mfma_f32_16x16x32_f16(v[0], pl, o[dt], 0, 0, 0);
-        o[dt] = __builtin_amdgcn_mfma_f32_16x16x32_f16(v[0], ph, o[dt], 0, 0, 0);
-      }
-    } else {
-#pragma unroll
-      for (int kt = 0; kt < 2; ++kt)
-#pragma unroll
-        for (int r = 0; r < 4; ++r) {
-          const float4v v = *reinterpret_cast<const float4v*>(base + kF32Stage + (kt * 16 + g * 4 + r) * 256 + l16 * 16);
-#pragma unroll
-          for (int dt = 0; dt < 4; ++dt) o[dt] = __builtin_amdgcn_mfma_f32_16x16x4f32(v[dt], s[kt][r], o[dt], 0, 0, 0);
-        }
-    }
   };
   auto run = [&](auto PLAINc) {
     for (int st = 0; st < stages; ++st) {
@@ -1395,7 +1324,7 @@ __global__ __launch_bounds__(kAttnThreads, 4) void attention_flash_f32_kernel(
         for (int j = 0; j < 16; ++j) high = fmaxf(high, bias(j >> 2, j & 3));
         high *= kLog2e;
         top = fmaxf(top, high);
-        if (__any(high > ref + kSlack)) move_ref(high);
+        if (__any(high > ref + kFlSlack)) move_ref(high);
 #pragma unroll
         for (int j = 0; j < 16; ++j) l += __builtin_amdgcn_exp2f(__builtin_fmaf(bias(j >> 2, j & 3), kLog2e, -ref));
       }
@@ -1407,17 +1336,6 @@ __global__ __launch_bounds__(kAttnThreads, 4) void attention_flash_f32_kernel(
   const float sum = xor_lanes_16_32_sum(l) + unseen.extra;
   if (tq < 0) return;
   const float inv = 1.0f / (sum + 1e-6f * __builtin_amdgcn_exp2f(mx - ref));
-  if constexpr (PAIRS) {                                               // o[dt][r] is feature 16 dt + 4 g + r, in units of the exponent
-#pragma unroll
-    for (int dt = 0; dt < 4; ++dt) {
-      float4v v = o[dt] * (inv * (1.0f / (1 << kWeightBits)));
-      // (h and l must come from one rounded product: fused into the conversion of h, it would be another one than l's)
-      asm volatile("" : "+v"(v));
-      store_pair<4>(ctx.out.rows + (size_t)(t0 + tq) * 2 * H, head * kD + dt * 16 + g * 4, v, 1.0f);
-    }
-    if (head == 0 && g == 0) ctx.out.exp[t0 + tq] = pair_exp;
-    return;
-  }
   // o[dt][r] is feature 16 g + 4 r + dt
 #pragma unroll
   for (int r = 0; r < 4; ++r) {
@@ -1437,13 +1355,9 @@ void attention_flash_f32_launch(const void* q, const void* k, const void* v, int
                                 hipStream_t stream) {
   const int q_blocks = (seq_len + 63) / 64;
   const int grid = (batch * heads + 7) / 8 * 8 * q_blocks;
-  auto go = [&](auto kern) {
-    kern<<<grid, kAttnThreads, kF32Smem, stream>>>(seq_start, batch, heads, q_blocks, seq_len, layout, packed_ld, (const float*)q, (const float*)k,
-                                                   (const float*)v, word_idx, (const float*)attr_mask, mask_class, (float*)dst, scaler,
-                                                   split_out ? 1 : 0, ctx);
-  };
-  if (ctx.qkv_exp) go(attention_flash_f32_kernel<true>);
-  else go(attention_flash_f32_kernel<false>);
+  attention_flash_f32_kernel<<<grid, kAttnThreads, kF32Smem, stream>>>(
+      seq_start, batch, heads, q_blocks, seq_len, layout, packed_ld, (const float*)q, (const float*)k, (const float*)v, word_idx,
+      (const float*)attr_mask, mask_class, (float*)dst, scaler, split_out ? 1 : 0, ctx);
 }
 
 // ------------------------------------------------------------------------------------------
@@ -1683,10 +1597,6 @@ void launch_mask_class(DType t, const void* attr_mask, const int32_t* seq_start,
     mask_class_kernel<<<grid, 256, 0, stream>>>((const float*)attr_mask, seq_start, word_idx, seq_len, blocks, cls);
   else
     mask_class_kernel<<<grid, 256, 0, stream>>>((const _Float16*)attr_mask, seq_start, word_idx, seq_len, blocks, cls);
-}
-
-bool attention_takes_pairs(int seq_len, int heads, int d) {
-  return d == kD && seq_len > kF32MinKeys && seq_len <= kFlMaxKeys && (uint64_t)seq_len * (uint64_t)(3 * heads * d) * 4u < 0x80000000ull;
 }
 
 bool attention_writes_split(const void* q, const void* k, const void* v, int layout, int packed_ld, int d) {

@@ -190,14 +190,13 @@ struct LayerWs {
 
 // Row arrays and weight arrays of a layer on pair rows, behind its matrices.
 struct PairWs {
-  int32_t *from_exp, *to_exp, *ctx_exp, *attn_exp, *inter_exp, *qkv_exp, *w_exp;      // w_exp: Q, K, V, output, up, down
-  int qkv_stride;
-  float *from_norm, *to_norm, *attn_norm, *qkv_stats[3], *up_stats, *tops;
+  int32_t *from_exp, *to_exp, *ctx_exp, *attn_exp, *inter_exp, *w_exp;      // w_exp: Q, K, V, output, up, down
+  float *from_norm, *to_norm, *attn_norm, *v_stats, *up_stats, *tops;
 };
 size_t pair_array_rows(size_t rows) { return align_up(rows, 256) + 256; }      // whole tiles of any height up to 256
 size_t pair_ws_words(size_t rows, size_t H) {
   const int h = (int)H;
-  return 11 * pair_array_rows(rows) + 9 * H + 2 * (3 * et::pair_weight_stats(h, h) + et::pair_weight_stats(4 * h, h)) +
+  return 8 * pair_array_rows(rows) + 9 * H + 2 * (et::pair_weight_stats(h, h) + et::pair_weight_stats(4 * h, h)) +
          8 * et::pair_weight_tops(h, h) + et::pair_weight_tops(h, 4 * h);
 }
 PairWs pair_ws(char* p, size_t rows, size_t H) {
@@ -207,12 +206,9 @@ PairWs pair_ws(char* p, size_t rows, size_t H) {
   w.from_exp = i; w.to_exp = i + r; w.ctx_exp = i + 2 * r; w.attn_exp = i + 3 * r; w.inter_exp = i + 4 * r;
   float* f = (float*)(i + 5 * r);
   w.from_norm = f; w.to_norm = f + r; w.attn_norm = f + 2 * r;
-  w.qkv_exp = (int32_t*)(f + 3 * r);
-  w.qkv_stride = (int)r;
-  w.w_exp = w.qkv_exp + 3 * r;
-  const size_t stats = 2 * et::pair_weight_stats((int)H, (int)H);
-  for (int g = 0; g < 3; ++g) w.qkv_stats[g] = (float*)(w.w_exp + 9 * H) + g * stats;
-  w.up_stats = w.qkv_stats[2] + stats;
+  w.w_exp = (int32_t*)(f + 3 * r);
+  w.v_stats = (float*)(w.w_exp + 9 * H);
+  w.up_stats = w.v_stats + 2 * et::pair_weight_stats((int)H, (int)H);
   w.tops = w.up_stats + 2 * et::pair_weight_stats(4 * (int)H, (int)H);
   return w;
 }
@@ -389,19 +385,15 @@ et_status run_layer_pairs(et_handle h, const LayerCall& c) {
   // read where they are handed over.
   _Float16* wt = (_Float16*)(base + ws.wt);
   const size_t HH = (size_t)2 * H * H;
-  const float *q = qkv, *k = q + H, *v = k + H;
-  const bool ctx_pairs = et::attention_writes_split(q, k, v, 1, 3 * H, c.d);
-  // (Q, K and V are pair rows on their way to the attention kernel where it takes them)
-  const bool qkv_pairs = ctx_pairs && et::attention_takes_pairs(S, c.heads, c.d);
   et::PairWeightJobs jobs;
   float* tops = pw.tops;
   auto weight = [&](const void* plain, const void* split, int k, int n, size_t at, const void* bias, float* stats) {
     jobs.job[jobs.count++] = {split ? split : plain, split != nullptr, k, n, wt + at * HH, pw.w_exp + at * H, tops, (const float*)bias, stats};
     tops += et::pair_weight_tops(n, k);
   };
-  weight(w->attr_kernel_Q, pp.attr_kernel_Q_t, H, H, 0, qkv_pairs ? w->attr_bias_Q : nullptr, qkv_pairs ? pw.qkv_stats[0] : nullptr);
-  weight(w->attr_kernel_K, pp.attr_kernel_K_t, H, H, 1, qkv_pairs ? w->attr_bias_K : nullptr, qkv_pairs ? pw.qkv_stats[1] : nullptr);
-  weight(w->attr_kernel_V, pp.attr_kernel_V_t, H, H, 2, w->attr_bias_V, pw.qkv_stats[2]);
+  weight(w->attr_kernel_Q, pp.attr_kernel_Q_t, H, H, 0, nullptr, nullptr);
+  weight(w->attr_kernel_K, pp.attr_kernel_K_t, H, H, 1, nullptr, nullptr);
+  weight(w->attr_kernel_V, pp.attr_kernel_V_t, H, H, 2, w->attr_bias_V, pw.v_stats);
   weight(w->attr_output_kernel, pp.attr_output_kernel_t, H, H, 3, nullptr, nullptr);
   weight(w->inter_kernel, pp.inter_kernel_t, H, F, 4, w->inter_bias, pw.up_stats);
   weight(w->output_kernel, pp.output_kernel_t, F, H, 8, nullptr, nullptr);
@@ -429,12 +421,12 @@ et_status run_layer_pairs(et_handle h, const LayerCall& c) {
     p3.B[i] = wt + i * HH;
     p3.b_exp[i] = pw.w_exp + i * H;
     p3.bias[i] = (const float*)qkv_bias[i];
-    p3.stats[i] = pw.qkv_stats[i];
   }
-  if (qkv_pairs) p3.c_exp = pw.qkv_exp, p3.c_stride = pw.qkv_stride, p3.linear = true;
   et::launch_gemm_pair(p3, qkv, 3 * H, rows, H, H, T, st);
   if ((s = check_launch(h, "QKV projection")) != ET_OK) return s;
 
+  const float *q = qkv, *k = q + H, *v = k + H;
+  const bool ctx_pairs = et::attention_writes_split(q, k, v, 1, 3 * H, c.d);
   const uint8_t* cls = c.mask_class ? c.mask_class : batch.cls;
   if (!cls && et::mask_class_bytes(dt, B, S, c.d)) {
     et::launch_mask_class(dt, c.attr_mask, seq_start, c.word_idx, B, S, (uint8_t*)(base + ws.cls), st);
@@ -442,7 +434,7 @@ et_status run_layer_pairs(et_handle h, const LayerCall& c) {
   }
   et::PairContext ctx;
   const et::PairRows ctx_rows{(_Float16*)(base + ws.ctx), pw.ctx_exp, pw.attn_norm};      // (the norms are rewritten by LayerNorm)
-  if (ctx_pairs) ctx = {ctx_rows, to.norm, pw.qkv_stats[2], (int)et::pair_weight_stats(H, H), qkv_pairs ? pw.qkv_exp : nullptr, pw.qkv_stride};
+  if (ctx_pairs) ctx = {ctx_rows, to.norm, pw.v_stats, (int)et::pair_weight_stats(H, H)};
   // (where the attention kernel writes floats only, they take the attention output's place until they are paired)
   et::launch_attention(dt, q, k, v, 1, 3 * H, c.attr_mask, attn, seq_start, c.word_idx, B, S, c.heads, c.d,
                        softmax_scaler(c.dtype, c.d), st, false, cls, ctx);
@@ -470,7 +462,7 @@ et_status run_layer_pairs(et_handle h, const LayerCall& c) {
   up.B[0] = wt + 4 * HH;
   up.b_exp[0] = pw.w_exp + 4 * H;
   up.bias[0] = (const float*)w->inter_bias;
-  up.stats[0] = pw.up_stats;
+  up.stats = pw.up_stats;
   up.c_exp = pw.inter_exp;
   et::launch_gemm_pair(up, base + ws.inter, F, rows, F, H, T, st);
   if ((s = check_launch(h, "FFN up")) != ET_OK) return s;
@@ -1429,7 +1421,7 @@ et_status et_gemm_pair(et_handle h, const et_pair_matrix* A, const void* Bt, con
   p.B[0] = (const _Float16*)Bt;
   p.b_exp[0] = b_exp;
   p.bias[0] = (const float*)bias;
-  p.stats[0] = b_stats;
+  p.stats = b_stats;
   p.c_exp = c_exp;
   et::launch_gemm_pair(p, C, n, m, n, k, m_dev, (hipStream_t)stream);
   return check_launch(h, "et_gemm_pair");

@@ -35,8 +35,6 @@ namespace {
 constexpr int kXcds = 8;
 constexpr int kLine = 128;                      // bytes of a row and k-step of 32
 
-// what a product leaves behind: floats, pair rows of gelu(A.B + bias), pair rows of A.B + bias
-enum PairOut { kFloat, kGelu, kPairs };
 struct PairGemmArgs {
   const _Float16* A[3];
   const _Float16* B[3];
@@ -45,11 +43,11 @@ struct PairGemmArgs {
   const float* bias[3];
   void* C;
   const int32_t* rows_dev;
-  // pair rows out: the bound of a row of C is a_norm[row] * (largest first word of b_stats) + (largest second word)
-  const float* a_norm[3];
-  const float* b_stats[3];
+  // GELU: the bound of a row of C is a_norm[row] * (largest first word of b_stats) + (largest second word)
+  const float* a_norm;
+  const float* b_stats;
   int32_t* c_exp;
-  int c_stride, n_stats;
+  int n_stats;
   int ldc, m_bound, n, k;
   int tiles_n, groups;                          // column tiles per group of B
   int columns;                                  // the tile order takes the column tiles of all groups this many at a time
@@ -91,8 +89,8 @@ struct PairTile {
 //   ahead.
 //   KS = 2 (small tiles): a stage is a chunk; one barrier per stage, the next stage's operands are read into a second register
 //   set under this one's MFMAs.
-// kGelu, kPairs: C = gelu(A.B + bias), A.B + bias as pair rows with their exponents in c_exp; kFloat: C is float, + bias if given.
-template <int WM, int WN, int MI, int NJ, int ST, int KS, int OUT>
+// GELU: C = gelu(A.B + bias) as pair rows with their exponents in c_exp; otherwise C is float, + bias if given.
+template <int WM, int WN, int MI, int NJ, int ST, int KS, bool GELU>
 __global__ __launch_bounds__(WM * WN * kWave) void gemm_pair_kernel(
     // what comes before the first request, as arguments of their own (gemm_f16_bt_kernel has the reason)
     const _Float16* a0, const _Float16* b0, const int32_t* rows_dev, int m_bound, int N, int K, int tiles_n, int groups, int columns, PairGemmArgs args) {
@@ -228,21 +226,10 @@ __global__ __launch_bounds__(WM * WN * kWave) void gemm_pair_kernel(
   Src cur = locate(idx), nxt = cur;
 #pragma unroll
   for (int s = 0; s < ST; ++s) issue_stage(s, min(s, nst - 1), cur, cur);
-  // Pair rows out: what bounds the rows of C, the same for every row of a group.  With GELU small tiles look at it, and at all that the epilogue reads, behind
+  // GELU: what bounds the rows of C, the same for every row.  Small tiles look at it, and at all that the epilogue reads, behind
   // the k loop: their launches take little longer than a round trip or two.
   float2v bounds = {0.f, 0.f}, stats[8];
-  float2v linear_bounds[3] = {};
-  if constexpr (OUT == kGelu) {
-    pair_stats_request(args.b_stats[0], args.n_stats, 0, stats);
-  } else if constexpr (OUT == kPairs) {
-    for (int grp = 0; grp < groups; ++grp) {
-      pair_stats_request(args.b_stats[grp], args.n_stats, 0, stats);
-      const float2v top = pair_stats_max(args.b_stats[grp], args.n_stats, stats);
-      if (grp == 0) linear_bounds[0] = top;
-      else if (grp == 1) linear_bounds[1] = top;
-      else linear_bounds[2] = top;
-    }
-  }
+  if constexpr (GELU) pair_stats_request(args.b_stats, args.n_stats, 0, stats);
   wait_vmcnt<KS * Tile::DMA*(ST - 1)>();
   barrier_only();
   auto read_set = [&](half8 (&a)[2][2][MI], half8 (&b)[2][2][NJ], int slot) {
@@ -261,7 +248,7 @@ __global__ __launch_bounds__(WM * WN * kWave) void gemm_pair_kernel(
     read_set(pa[0], pb[0], 0);
   }
 
-  if constexpr (OUT == kGelu && Tile::BIG) bounds = pair_stats_max(args.b_stats[0], args.n_stats, stats);
+  if constexpr (GELU && Tile::BIG) bounds = pair_stats_max(args.b_stats, args.n_stats, stats);
 
   int s = 0;                                     // slot of the current stage
   bool first_tile = true;
@@ -285,7 +272,7 @@ __global__ __launch_bounds__(WM * WN * kWave) void gemm_pair_kernel(
     const int own_row = row0 + min(l16 >> 2, MI - 1) * 16 + (l16 & 3);
     float own_norm = 0.f;
     auto request = [&](const int32_t* a_exp, const int32_t* b_exp, const float* add, const float* norm) {
-      if constexpr (OUT != kFloat) own_norm = norm[own_row];
+      if constexpr (GELU) own_norm = norm[own_row];
       if (col >= N) return;
 #pragma unroll
       for (int j = 0; j < NJ; ++j) ce[j] = b_exp[col + j];
@@ -294,7 +281,7 @@ __global__ __launch_bounds__(WM * WN * kWave) void gemm_pair_kernel(
 #pragma unroll
       for (int i = 0; i < MI; ++i) re[i] = *reinterpret_cast<const int4v*>(a_exp + row0 + i * 16);
     };
-    if constexpr (!Tile::BIG) request(args.a_exp[cur.grp], args.b_exp[cur.grp], args.bias[cur.grp], args.a_norm[cur.grp]);
+    if constexpr (!Tile::BIG) request(args.a_exp[cur.grp], args.b_exp[cur.grp], args.bias[cur.grp], args.a_norm);
     if constexpr (Tile::BIG) {
       auto step = [&](auto Pc, int t) {
         constexpr int P = decltype(Pc)::value;
@@ -371,7 +358,7 @@ __global__ __launch_bounds__(WM * WN * kWave) void gemm_pair_kernel(
     }
     wait_vmcnt<0>();
 
-    if constexpr (Tile::BIG) request(args.a_exp[cur.grp], args.b_exp[cur.grp], args.bias[cur.grp], args.a_norm[cur.grp]);
+    if constexpr (Tile::BIG) request(args.a_exp[cur.grp], args.b_exp[cur.grp], args.bias[cur.grp], args.a_norm);
     // the loads are waited for here: left pending on the paths that store nothing, they would have the compiler put a wait
     // for every outstanding load, the DMA included, in front of the k loop's reuse of their registers
 #pragma unroll
@@ -382,15 +369,14 @@ __global__ __launch_bounds__(WM * WN * kWave) void gemm_pair_kernel(
     }
 #pragma unroll
     for (int i = 0; i < MI; ++i) asm volatile("" : "+v"(re[i]));
-    if constexpr (OUT != kFloat) asm volatile("" : "+v"(own_norm));
-    if constexpr (OUT == kGelu && !Tile::BIG)
-      if (first_tile) bounds = pair_stats_max(args.b_stats[0], args.n_stats, stats);
-    if constexpr (OUT == kPairs) bounds = cur.grp == 0 ? linear_bounds[0] : cur.grp == 1 ? linear_bounds[1] : linear_bounds[2];
+    if constexpr (GELU) asm volatile("" : "+v"(own_norm));
+    if constexpr (GELU && !Tile::BIG)
+      if (first_tile) bounds = pair_stats_max(args.b_stats, args.n_stats, stats);
     float4v scale[MI];
-    if constexpr (OUT != kFloat) {                 // (every lane is active here)
+    if constexpr (GELU) {                          // (every lane is active here)
       const int e = pair_exponent(own_norm * (bounds[0] * 1.01f) + bounds[1]);
       from_lanes<0>(scale, pair_scale(e));
-      if (cur.n0 == 0 && wn == 0 && l16 < 4 * MI && own_row < rows) args.c_exp[cur.grp * args.c_stride + own_row] = e;
+      if (cur.n0 == 0 && wn == 0 && l16 < 4 * MI && own_row < rows) args.c_exp[own_row] = e;
     }
     if (col < N) {
 #pragma unroll
@@ -402,11 +388,9 @@ __global__ __launch_bounds__(WM * WN * kWave) void gemm_pair_kernel(
           fvec o;
 #pragma unroll
           for (int j = 0; j < NJ; ++j) o[j] = __builtin_ldexpf(sum[i][j][r] + acc[i][j][r], re[i][r] + ce[j]) + bias[j];
-          if constexpr (OUT != kFloat) {
-            if constexpr (OUT == kGelu) {
+          if constexpr (GELU) {
 #pragma unroll
-              for (int j = 0; j < NJ; ++j) o[j] *= gelu_cdf(o[j], o[j] * o[j] * o[j]);
-            }
+            for (int j = 0; j < NJ; ++j) o[j] *= gelu_cdf(o[j], o[j] * o[j] * o[j]);
             store_pair<NJ>((_Float16*)args.C + (size_t)row * 2 * args.ldc, cur.grp * N + col, o, scale[i][r]);
           } else {
             *reinterpret_cast<fvec*>((float*)args.C + (size_t)row * args.ldc + (size_t)cur.grp * N + col) = o;
@@ -460,7 +444,7 @@ PairPick pick_pair_tile(int m, int n, int k, int groups) {
 }
 
 template <int WM, int WN, int MI, int NJ, int ST, int KS>
-void launch_tile(PairGemmArgs a, PairOut out, int groups, hipStream_t stream) {
+void launch_tile(PairGemmArgs a, bool gelu, int groups, hipStream_t stream) {
   using Tile = PairTile<WM, WN, MI, NJ, ST, KS>;
   a.tiles_n = (a.n + Tile::BN - 1) / Tile::BN;
   a.groups = groups;
@@ -478,21 +462,20 @@ void launch_tile(PairGemmArgs a, PairOut out, int groups, hipStream_t stream) {
     allow_dynamic_lds(reinterpret_cast<const void*>(kern), Tile::SMEM);
     kern<<<grid, Tile::THREADS, Tile::SMEM, stream>>>(a.A[0], a.B[0], a.rows_dev, a.m_bound, a.n, a.k, a.tiles_n, groups, a.columns, a);
   };
-  if (out == kGelu) go(gemm_pair_kernel<WM, WN, MI, NJ, ST, KS, kGelu>);
-  else if (out == kPairs) go(gemm_pair_kernel<WM, WN, MI, NJ, ST, KS, kPairs>);
-  else go(gemm_pair_kernel<WM, WN, MI, NJ, ST, KS, kFloat>);
+  if (gelu) go(gemm_pair_kernel<WM, WN, MI, NJ, ST, KS, true>);
+  else go(gemm_pair_kernel<WM, WN, MI, NJ, ST, KS, false>);
 }
 
-void launch_pick(PairPick pick, const PairGemmArgs& a, PairOut out, int groups, hipStream_t stream) {
+void launch_pick(PairPick pick, const PairGemmArgs& a, bool gelu, int groups, hipStream_t stream) {
   switch (pick) {
-    case p256x128: return launch_tile<4, 2, 4, 4, 3, 1>(a, out, groups, stream);
-    case p192x128: return launch_tile<4, 2, 3, 4, 3, 1>(a, out, groups, stream);
-    case p128x128: return launch_tile<2, 4, 4, 2, 4, 1>(a, out, groups, stream);
-    case p96x128: return launch_tile<2, 4, 3, 2, 4, 1>(a, out, groups, stream);
-    case p64x128: return launch_tile<2, 4, 2, 2, 3, 2>(a, out, groups, stream);
-    case p64x64: return launch_tile<4, 2, 1, 2, 4, 2>(a, out, groups, stream);
-    case p32x64: return launch_tile<2, 4, 1, 1, 5, 2>(a, out, groups, stream);
-    case p32x32: return launch_tile<2, 2, 1, 1, 6, 2>(a, out, groups, stream);
+    case p256x128: return launch_tile<4, 2, 4, 4, 3, 1>(a, gelu, groups, stream);
+    case p192x128: return launch_tile<4, 2, 3, 4, 3, 1>(a, gelu, groups, stream);
+    case p128x128: return launch_tile<2, 4, 4, 2, 4, 1>(a, gelu, groups, stream);
+    case p96x128: return launch_tile<2, 4, 3, 2, 4, 1>(a, gelu, groups, stream);
+    case p64x128: return launch_tile<2, 4, 2, 2, 3, 2>(a, gelu, groups, stream);
+    case p64x64: return launch_tile<4, 2, 1, 2, 4, 2>(a, gelu, groups, stream);
+    case p32x64: return launch_tile<2, 4, 1, 1, 5, 2>(a, gelu, groups, stream);
+    case p32x32: return launch_tile<2, 2, 1, 1, 6, 2>(a, gelu, groups, stream);
     default: return;
   }
 }
@@ -756,11 +739,8 @@ void launch_gemm_pair(const PairProduct& p, void* C, int ldc, int m_bound, int n
     a.b_exp[i] = p.b_exp[i];
     a.bias[i] = p.bias[i];
   }
-  for (int i = 0; i < p.groups; ++i) {
-    a.a_norm[i] = p.A[i].norm;
-    a.b_stats[i] = p.stats[i];
-  }
-  a.c_stride = p.c_stride;
+  a.a_norm = p.A[0].norm;
+  a.b_stats = p.stats;
   a.n_stats = (int)pair_weight_stats(n, k);
   a.c_exp = p.c_exp;
   a.C = C;
@@ -769,7 +749,7 @@ void launch_gemm_pair(const PairProduct& p, void* C, int ldc, int m_bound, int n
   a.m_bound = m_bound;
   a.n = n;
   a.k = k;
-  launch_pick(pick_pair_tile(m_bound, n, k, p.groups), a, p.c_exp == nullptr ? kFloat : p.linear ? kPairs : kGelu, p.groups, stream);
+  launch_pick(pick_pair_tile(m_bound, n, k, p.groups), a, p.c_exp != nullptr, p.groups, stream);
 }
 
 }  // namespace et

@@ -27,15 +27,12 @@ struct PairRows {
   float* norm = nullptr;             // (not of matrices that nothing is bounded by)
 };
 // What attention needs to write its rows as pair rows: the matrix, the norms of the rows that K and V were made of, and what
-// bounds the column norms and the bias of V (n_stats pairs, see PairWeightJob).  qkv_exp: Q, K and V are pair rows themselves (packed
-// rows of 3 heads d values; attention_takes_pairs), with the exponents of the Q rows, and of the K and V rows qkv_stride words on each.
+// bounds the column norms and the bias of V (n_stats pairs, see PairWeightJob).
 struct PairContext {
   PairRows out;
   const float* norm = nullptr;
   const float* stats = nullptr;
   int n_stats = 0;
-  const int32_t* qkv_exp = nullptr;
-  int qkv_stride = 0;
 };
 
 // ---- input_output.hip --------------------------------------------------------------------
@@ -156,8 +153,6 @@ void launch_mask_class(DType t, const void* attr_mask, const int32_t* seq_start,
 // split_out (fp32): dst gets split rows (see gemm_split.hip) instead of float rows, with pair.out.rows that one gets pair rows;
 // only where this says so
 bool attention_writes_split(const void* q, const void* k, const void* v, int layout, int packed_ld, int d);
-// fp32: the kernel for these shapes takes Q, K and V as pair rows (PairContext::qkv_exp)
-bool attention_takes_pairs(int seq_len, int heads, int d);
 
 // ---- gemm.hip ----------------------------------------------------------------------------
 // Up to three independent column groups share one launch (the Q/K/V projections): group g
@@ -257,18 +252,15 @@ struct PairWeightJobs {
 void launch_pair_weights(const PairWeightJobs& jobs, hipStream_t stream, const BatchJobs* batch = nullptr, const PairRowsJob* rows = nullptr,
                          int row_jobs = 0);
 // C[:, g n : (g + 1) n] = A[g].B[g] + bias[g] (bias may be null), float with leading dimension ldc; with c_exp
-// C = gelu(A.B + bias) (no gelu with `linear`) as pair rows of ldc values, from A[g].norm and the weights' `stats`; the groups'
-// exponents lie c_stride words apart.
+// C = gelu(A.B + bias) as pair rows of ldc values, from A[0].norm and the weights' `stats`.
 struct PairProduct {
   int groups = 1;
   PairRows A[3];
   const _Float16* B[3] = {};
   const int32_t* b_exp[3] = {};
   const float* bias[3] = {};
-  const float* stats[3] = {};
+  const float* stats = nullptr;
   int32_t* c_exp = nullptr;
-  int c_stride = 0;
-  bool linear = false;
 };
 void launch_gemm_pair(const PairProduct& p, void* C, int ldc, int m_bound, int n, int k, const int32_t* rows_dev,
                       hipStream_t stream);

@@ -135,7 +135,7 @@ def test_layer(heads, d, B, S, scale):
     assert np.linalg.norm(got[valid] - want[valid]) <= 2e-6 * np.linalg.norm(want[valid])
 
 
-# attention that takes Q, K and V as pair rows (more than 32 positions): lengths around its stages of 32 keys and blocks of 64
+# the streaming attention of layers on pair rows (more than 32 positions): lengths around its stages of 32 keys and blocks of 64
 # queries, holes, masks that are read and masks that are not, rows of a mask on 16-byte boundaries and odd ones; wide: scores tens
 # apart, so that the exponents' reference moves
 @pytest.mark.parametrize("S", [33, 64, 101, 200, 1024])
