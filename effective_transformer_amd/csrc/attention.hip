@@ -227,7 +227,7 @@ __global__ __launch_bounds__(WAVES * kWave) void attention_kernel(
     // (the first 14 words come in registers: what the chain order -> start table -> positions and rows needs)
     const int32_t* __restrict__ seq_start, const int32_t* __restrict__ word_idx, int batch, int seq_len, int heads, int heads_per_wg,
     int layout, int packed_ld, const T* __restrict__ q_src, const T* __restrict__ k_src, const T* __restrict__ v_src,
-    const T* __restrict__ attr_mask, T* __restrict__ dst, float scaler, int split_out, PairContext ctx) {
+    const T* __restrict__ attr_mask, T* __restrict__ dst, float scaler, int split_out) {
   using Cfg = AttnCfg<T>;
   using Sm = AttnSmem<T, NKT>;
   using C = Chunk16<T>;
@@ -353,13 +353,6 @@ __global__ __launch_bounds__(WAVES * kWave) void attention_kernel(
   T* out_row = tq >= 0 ? dst + (size_t)tq * H + g * (sizeof(T) == 2 ? 16 : 4) : nullptr;
   if (sizeof(T) == 4 && split_out && tq >= 0)
     out_row = reinterpret_cast<T*>(reinterpret_cast<uint16_t*>(dst) + (size_t)tq * 3 * H);
-  float pair_by = 0.f;
-  if constexpr (sizeof(T) == 4)
-    if (ctx.out.rows != nullptr) {
-      const int e = context_exponent(ctx.norm, t0, t1, ctx.stats, ctx.n_stats);
-      pair_by = pair_scale(e);
-      if (blockIdx.x == 0 && g == 0 && tq >= 0) ctx.out.exp[tq] = e;
-    }
 
   for (int head = h_begin; head < h_end; ++head) {
     if (head != h_begin) __syncthreads();      // every wavefront is done with the previous head's tiles
@@ -525,8 +518,7 @@ __global__ __launch_bounds__(WAVES * kWave) void attention_kernel(
             out4 v;
 #pragma unroll
             for (int r = 0; r < 4; ++r) v[r] = (T)o[dt][r];
-            if (ctx.out.rows != nullptr) store_pair<4>(ctx.out.rows + (size_t)tq * 2 * H, head * kD + dt * 16 + g * 4, v, pair_by);
-            else if (split_out) store_split<4>(reinterpret_cast<uint16_t*>(out_row), head * kD + dt * 16 + g * 4, v);
+            if (split_out) store_split<4>(reinterpret_cast<uint16_t*>(out_row), head * kD + dt * 16 + g * 4, v);
             else *reinterpret_cast<out4*>(orow + dt * 16) = v;
           }
         }
@@ -540,7 +532,7 @@ __global__ __launch_bounds__(WAVES * kWave) void attention_kernel(
 template <typename T, int NKT>
 void attention_launch(const void* q, const void* k, const void* v, int layout, int packed_ld, const void* attr_mask,
                       void* dst, const int32_t* seq_start, const int32_t* word_idx, int batch, int seq_len, int heads,
-                      float scaler, bool split_out, const PairContext& ctx, hipStream_t stream) {
+                      float scaler, bool split_out, hipStream_t stream) {
   using Sm = AttnSmem<T, NKT>;
   constexpr int kCpr = kD * (int)sizeof(T) / 16;
   constexpr int WAVES = 4;
@@ -561,7 +553,7 @@ void attention_launch(const void* q, const void* k, const void* v, int layout, i
     }
   dim3 grid((heads + hpw - 1) / hpw, batch);
   kern<<<grid, kThreads, Sm::kBytes, stream>>>(seq_start, word_idx, batch, seq_len, heads, hpw, layout, packed_ld, (const T*)q,
-                                               (const T*)k, (const T*)v, (const T*)attr_mask, (T*)dst, scaler, split_out ? 1 : 0, ctx);
+                                               (const T*)k, (const T*)v, (const T*)attr_mask, (T*)dst, scaler, split_out ? 1 : 0);
 }
 
 
@@ -1084,7 +1076,7 @@ __global__ __launch_bounds__(kAttnThreads, 4) void attention_flash_f32_kernel(
     const int32_t* __restrict__ seq_start, int batch, int heads, int q_blocks, int seq_len, int layout, int packed_ld,
     const float* __restrict__ q_src, const float* __restrict__ k_src, const float* __restrict__ v_src,
     const int32_t* __restrict__ word_idx, const float* __restrict__ attr_mask, const uint8_t* __restrict__ mask_class,
-    float* __restrict__ dst, float scaler, int split_out, PairContext ctx) {
+    float* __restrict__ dst, float scaler, int split_out) {
 #if defined(__HIP_DEVICE_COMPILE__)   // device-only types in the body; the host pass only needs the stub
   extern __shared__ __attribute__((aligned(1024))) unsigned char smem_raw[];
   unsigned char* kv = smem_raw;                                        // [stage][K, V]
@@ -1191,7 +1183,6 @@ __global__ __launch_bounds__(kAttnThreads, 4) void attention_flash_f32_kernel(
   // (the queries are waited for here and not in the stage loop, where the wait would cover the DMA)
 #pragma unroll
   for (int i = 0; i < 4; ++i) asm volatile("" : "+v"(bq[i]));
-  const int pair_exp = ctx.out.rows != nullptr ? context_exponent(ctx.norm, t0, t1, ctx.stats, ctx.n_stats) : 0;
 
   float ref = kFlLowest, top = -INFINITY, l = 0.f;                     // as above; l: of this lane's keys
   float4v o[4];
@@ -1341,23 +1332,20 @@ __global__ __launch_bounds__(kAttnThreads, 4) void attention_flash_f32_kernel(
   for (int r = 0; r < 4; ++r) {
     const float4v v = {o[0][r] * inv, o[1][r] * inv, o[2][r] * inv, o[3][r] * inv};
     const int col = head * kD + g * 16 + r * 4;
-    if (ctx.out.rows != nullptr) store_pair<4>(ctx.out.rows + (size_t)(t0 + tq) * 2 * H, col, v, pair_scale(pair_exp));
-    else if (split_out) store_split<4>(reinterpret_cast<uint16_t*>(dst) + (size_t)(t0 + tq) * 3 * H, col, v);
+    if (split_out) store_split<4>(reinterpret_cast<uint16_t*>(dst) + (size_t)(t0 + tq) * 3 * H, col, v);
     else *reinterpret_cast<float4v*>(dst + (size_t)(t0 + tq) * H + col) = v;
   }
-  if (ctx.out.rows != nullptr && head == 0 && g == 0) ctx.out.exp[t0 + tq] = pair_exp;
 #endif
 }
 
 void attention_flash_f32_launch(const void* q, const void* k, const void* v, int layout, int packed_ld, const void* attr_mask,
                                 const uint8_t* mask_class, void* dst, const int32_t* seq_start, const int32_t* word_idx,
-                                int batch, int seq_len, int heads, float scaler, bool split_out, const PairContext& ctx,
-                                hipStream_t stream) {
+                                int batch, int seq_len, int heads, float scaler, bool split_out, hipStream_t stream) {
   const int q_blocks = (seq_len + 63) / 64;
   const int grid = (batch * heads + 7) / 8 * 8 * q_blocks;
   attention_flash_f32_kernel<<<grid, kAttnThreads, kF32Smem, stream>>>(
       seq_start, batch, heads, q_blocks, seq_len, layout, packed_ld, (const float*)q, (const float*)k, (const float*)v, word_idx,
-      (const float*)attr_mask, mask_class, (float*)dst, scaler, split_out ? 1 : 0, ctx);
+      (const float*)attr_mask, mask_class, (float*)dst, scaler, split_out ? 1 : 0);
 }
 
 // ------------------------------------------------------------------------------------------
@@ -1502,8 +1490,7 @@ void attention_generic_launch(const void* q, const void* k, const void* v, int l
 template <typename T>
 void attention_dispatch(const void* q, const void* k, const void* v, int layout, int packed_ld, const void* attr_mask,
                         void* dst, const int32_t* seq_start, const int32_t* word_idx, int batch, int seq_len, int heads,
-                        int d, float scaler, bool split_out, const uint8_t* mask_class, const PairContext& ctx,
-                        hipStream_t stream) {
+                        int d, float scaler, bool split_out, const uint8_t* mask_class, hipStream_t stream) {
   // (the streaming kernels address the rows of a sequence with 31 bits)
   const bool far = (uint64_t)seq_len * (uint64_t)(layout == 1 ? packed_ld : kD) * sizeof(T) >= 0x80000000ull;
   if (d != kD || !head_rows_16b<T>(q, k, v, layout, packed_ld, d) || (far && seq_len > kF32MinKeys))
@@ -1514,13 +1501,13 @@ void attention_dispatch(const void* q, const void* k, const void* v, int layout,
                            scaler, stream);
   else if (sizeof(T) == 4 && seq_len > kF32MinKeys)
     attention_flash_f32_launch(q, k, v, layout, packed_ld, attr_mask, mask_class, dst, seq_start, word_idx, batch, seq_len,
-                               heads, scaler, split_out, ctx, stream);
+                               heads, scaler, split_out, stream);
   else if (seq_len <= 32)
     attention_launch<T, 2>(q, k, v, layout, packed_ld, attr_mask, dst, seq_start, word_idx, batch, seq_len, heads,
-                           scaler, split_out, ctx, stream);
+                           scaler, split_out, stream);
   else if constexpr (sizeof(T) == 2)
     attention_launch<T, 4>(q, k, v, layout, packed_ld, attr_mask, dst, seq_start, word_idx, batch, seq_len, heads,
-                           scaler, split_out, ctx, stream);
+                           scaler, split_out, stream);
 }
 
 }  // namespace
@@ -1606,13 +1593,13 @@ bool attention_writes_split(const void* q, const void* k, const void* v, int lay
 void launch_attention(DType t, const void* q, const void* k, const void* v, int layout, int packed_ld,
                       const void* attr_mask, void* dst, const int32_t* seq_start, const int32_t* word_idx, int batch,
                       int seq_len, int heads, int d, float scaler, hipStream_t stream,
-                      bool split_out, const uint8_t* mask_class, const PairContext& ctx) {
+                      bool split_out, const uint8_t* mask_class) {
   if (t == DType::F32)
     attention_dispatch<float>(q, k, v, layout, packed_ld, attr_mask, dst, seq_start, word_idx, batch, seq_len, heads, d,
-                              scaler, split_out, mask_class, ctx, stream);
+                              scaler, split_out, mask_class, stream);
   else
     attention_dispatch<_Float16>(q, k, v, layout, packed_ld, attr_mask, dst, seq_start, word_idx, batch, seq_len,
-                                 heads, d, scaler, false, mask_class, PairContext(), stream);
+                                 heads, d, scaler, false, mask_class, stream);
 }
 
 }  // namespace et

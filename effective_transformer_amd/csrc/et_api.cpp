@@ -191,12 +191,12 @@ struct LayerWs {
 // Row arrays and weight arrays of a layer on pair rows, behind its matrices.
 struct PairWs {
   int32_t *from_exp, *to_exp, *ctx_exp, *attn_exp, *inter_exp, *w_exp;      // w_exp: Q, K, V, output, up, down
-  float *from_norm, *to_norm, *attn_norm, *v_stats, *up_stats, *tops;
+  float *from_norm, *to_norm, *attn_norm, *up_stats, *tops;
 };
 size_t pair_array_rows(size_t rows) { return align_up(rows, 256) + 256; }      // whole tiles of any height up to 256
 size_t pair_ws_words(size_t rows, size_t H) {
   const int h = (int)H;
-  return 8 * pair_array_rows(rows) + 9 * H + 2 * (et::pair_weight_stats(h, h) + et::pair_weight_stats(4 * h, h)) +
+  return 8 * pair_array_rows(rows) + 9 * H + 2 * et::pair_weight_stats(4 * h, h) +
          8 * et::pair_weight_tops(h, h) + et::pair_weight_tops(h, 4 * h);
 }
 PairWs pair_ws(char* p, size_t rows, size_t H) {
@@ -207,8 +207,7 @@ PairWs pair_ws(char* p, size_t rows, size_t H) {
   float* f = (float*)(i + 5 * r);
   w.from_norm = f; w.to_norm = f + r; w.attn_norm = f + 2 * r;
   w.w_exp = (int32_t*)(f + 3 * r);
-  w.v_stats = (float*)(w.w_exp + 9 * H);
-  w.up_stats = w.v_stats + 2 * et::pair_weight_stats((int)H, (int)H);
+  w.up_stats = (float*)(w.w_exp + 9 * H);
   w.tops = w.up_stats + 2 * et::pair_weight_stats(4 * (int)H, (int)H);
   return w;
 }
@@ -393,7 +392,7 @@ et_status run_layer_pairs(et_handle h, const LayerCall& c) {
   };
   weight(w->attr_kernel_Q, pp.attr_kernel_Q_t, H, H, 0, nullptr, nullptr);
   weight(w->attr_kernel_K, pp.attr_kernel_K_t, H, H, 1, nullptr, nullptr);
-  weight(w->attr_kernel_V, pp.attr_kernel_V_t, H, H, 2, w->attr_bias_V, pw.v_stats);
+  weight(w->attr_kernel_V, pp.attr_kernel_V_t, H, H, 2, nullptr, nullptr);
   weight(w->attr_output_kernel, pp.attr_output_kernel_t, H, H, 3, nullptr, nullptr);
   weight(w->inter_kernel, pp.inter_kernel_t, H, F, 4, w->inter_bias, pw.up_stats);
   weight(w->output_kernel, pp.output_kernel_t, F, H, 8, nullptr, nullptr);
@@ -425,24 +424,20 @@ et_status run_layer_pairs(et_handle h, const LayerCall& c) {
   et::launch_gemm_pair(p3, qkv, 3 * H, rows, H, H, T, st);
   if ((s = check_launch(h, "QKV projection")) != ET_OK) return s;
 
-  const float *q = qkv, *k = q + H, *v = k + H;
-  const bool ctx_pairs = et::attention_writes_split(q, k, v, 1, 3 * H, c.d);
   const uint8_t* cls = c.mask_class ? c.mask_class : batch.cls;
   if (!cls && et::mask_class_bytes(dt, B, S, c.d)) {
     et::launch_mask_class(dt, c.attr_mask, seq_start, c.word_idx, B, S, (uint8_t*)(base + ws.cls), st);
     cls = (const uint8_t*)(base + ws.cls);
   }
-  et::PairContext ctx;
   const et::PairRows ctx_rows{(_Float16*)(base + ws.ctx), pw.ctx_exp, pw.attn_norm};      // (the norms are rewritten by LayerNorm)
-  if (ctx_pairs) ctx = {ctx_rows, to.norm, pw.v_stats, (int)et::pair_weight_stats(H, H)};
-  // (where the attention kernel writes floats only, they take the attention output's place until they are paired)
-  et::launch_attention(dt, q, k, v, 1, 3 * H, c.attr_mask, attn, seq_start, c.word_idx, B, S, c.heads, c.d,
-                       softmax_scaler(c.dtype, c.d), st, false, cls, ctx);
-  if (!ctx_pairs) {
-    et::PairRowsJob job;
-    job.src = attn, job.out = ctx_rows, job.m = rows, job.n = H, job.rows_dev = T;
-    et::launch_pair_rows(job, st);
-  }
+  // The context takes the attention output's place until its rows are paired.  A launch of its own, because no workgroup of the
+  // attention kernel sees a whole row: with an exponent from a bound instead, the same for all rows of a sequence, a token of large
+  // values took the bits of queries that do not see it (V of that token 2^30 of the others': rows off by 1.9e-3, now 1.1e-6).
+  et::launch_attention(dt, qkv, qkv + H, qkv + 2 * H, 1, 3 * H, c.attr_mask, attn, seq_start, c.word_idx, B, S, c.heads, c.d,
+                       softmax_scaler(c.dtype, c.d), st, false, cls);
+  et::PairRowsJob context;
+  context.src = attn, context.out = ctx_rows, context.m = rows, context.n = H, context.rows_dev = T;
+  et::launch_pair_rows(context, st);
   if ((s = check_launch(h, "attention")) != ET_OK) return s;
 
   auto product = [&](const et::PairRows& a, int w_at, void* C, int n, int k_) {

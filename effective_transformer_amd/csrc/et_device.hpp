@@ -252,25 +252,6 @@ __device__ __forceinline__ float2v pair_stats_max(const float* __restrict__ stat
   }
   return float2v{wave_max(top[0]), wave_max(top[1])};
 }
-// The exponent of a sequence's context rows: every value of them is a weighted mean (weights of sum <= 1) of the values
-// x.w + b of its tokens, with |x.w + b| <= |x| |w| + |b|.  One wavefront; `stats`: bounds of |w| and |b| (PairWeightJob).
-__device__ __forceinline__ int context_exponent(const float* __restrict__ norm, int t0, int t1, const float* __restrict__ stats,
-                                                int n_stats) {
-  const int lane = threadIdx.x & (kWave - 1);
-  float top = 0.f;
-  float2v first[8];
-  pair_stats_request(stats, n_stats, 0, first);
-  for (int i0 = t0; i0 < t1; i0 += 4 * kWave) {
-    float v[4];
-#pragma unroll
-    for (int u = 0; u < 4; ++u) v[u] = norm[min(i0 + u * kWave + lane, t1 - 1)];
-#pragma unroll
-    for (int u = 0; u < 4; ++u) top = fmaxf(top, v[u]);
-  }
-  const float2v w = pair_stats_max(stats, n_stats, first);
-  return pair_exponent(wave_max(top) * (w[0] * 1.01f) + w[1]);
-}
-
 // seq_start[b] = first packed row of sequence b (b in [0, batch]; seq_start[batch] = T), written by the thread that
 // owns packed row t in [0, T]: it covers the sequences that begin at t (token-less sequences included).
 __device__ __forceinline__ void seq_start_for_row(const int32_t* __restrict__ batch_idx, int T, int t, int batch,

@@ -12,10 +12,9 @@
 // layers of smaller hidden sizes keep them.  Infinities and NaNs give NaN.
 //
 // Both operands come as "pair rows": [row][k / 32][h, l][32] halves, one 128-byte line per row and k-step of 32.  Both have
-// an exponent per row, which are applied to the result.  The kernels that produce A write that form themselves: input and LayerNorm know the largest value
-// of the row; attention and the FFN's first product, whose workgroups see parts of a row, take a bound instead, which costs
-// range and no bits: |x.w + b| <= |x| max|w| + max|b| (Euclidean norms), and a row of the context is at most the largest such
-// value of its sequence.  Weights are taken anew by every layer call: pair_weight_top_kernel looks for the largest value of each
+// an exponent per row, which are applied to the result.  Input, LayerNorm and the pass over the context take it from the row's
+// largest value; the FFN's first product, whose workgroups see parts of a row, takes a bound instead, which costs
+// range and no bits: |x.w + b| <= |x| max|w| + max|b| (Euclidean norms).  Weights are taken anew by every layer call: pair_weight_top_kernel looks for the largest value of each
 // column, pair_weight_kernel writes the rows (8 + 11.5 us per layer of BERT-base, split rows 15).
 // Bound: at large m the power limit of the matrix cores (20000 rows, k = 768 / n = 2304, 768, 3072 + GELU and k = 3072 / n = 768:
 // 172, 62, 258, 223 us, 1100 .. 1270 TFLOP/s of 16-bit products; split rows 301, 113, 450, 417); below a round of the chip the

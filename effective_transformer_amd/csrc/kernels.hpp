@@ -26,15 +26,6 @@ struct PairRows {
   int32_t* exp = nullptr;
   float* norm = nullptr;             // (not of matrices that nothing is bounded by)
 };
-// What attention needs to write its rows as pair rows: the matrix, the norms of the rows that K and V were made of, and what
-// bounds the column norms and the bias of V (n_stats pairs, see PairWeightJob).
-struct PairContext {
-  PairRows out;
-  const float* norm = nullptr;
-  const float* stats = nullptr;
-  int n_stats = 0;
-};
-
 // ---- input_output.hip --------------------------------------------------------------------
 // Number of int32 words of scratch the scan needs for `length` elements.
 size_t scan_scratch_words(int length);
@@ -143,15 +134,14 @@ bool attention_supported(DType t, int seq_len, int d);
 void launch_attention(DType t, const void* q, const void* k, const void* v, int layout, int packed_ld,
                       const void* attr_mask, void* dst, const int32_t* seq_start, const int32_t* word_idx,
                       int batch, int seq_len, int heads, int d, float scaler, hipStream_t stream,
-                      bool split_out = false, const uint8_t* mask_class = nullptr, const PairContext& pair = PairContext());
+                      bool split_out = false, const uint8_t* mask_class = nullptr);
 // Classes of the mask rows (one byte per 16 query positions of a sequence) for the kernel that makes use of them; the same
 // array serves every layer of a batch.  0 bytes: the kernel of this shape has no use for them.
 size_t mask_class_bytes(DType t, int batch, int seq_len, int d);
 size_t mask_class_bytes_max(int batch);                // at any length
 void launch_mask_class(DType t, const void* attr_mask, const int32_t* seq_start, const int32_t* word_idx, int batch, int seq_len,
                        uint8_t* cls, hipStream_t stream);
-// split_out (fp32): dst gets split rows (see gemm_split.hip) instead of float rows, with pair.out.rows that one gets pair rows;
-// only where this says so
+// split_out (fp32): dst gets split rows (see gemm_split.hip) instead of float rows; only where this says so
 bool attention_writes_split(const void* q, const void* k, const void* v, int layout, int packed_ld, int d);
 
 // ---- gemm.hip ----------------------------------------------------------------------------

@@ -37,7 +37,22 @@ def _qk_head(w, x, by):
         w[at][..., 64:128] /= by
 
 
-CHANGES = [_plain, _qk_head]
+def _unseen_token(w, x, by):
+    """The last token of every sequence has large values in V (each factor within what a row and a column hold), and nobody sees it
+    but its own query (UNSEEN)."""
+    s = np.sqrt(by)
+    x[..., 7] = 0
+    x[np.arange(len(x)), _lengths(x.shape[1]) - 1, 7] = s
+    w[Q][7], w[K][7] = 0, 0
+    w[V][7] *= s
+
+
+CHANGES = [_plain, _qk_head, _unseen_token]
+UNSEEN = [_unseen_token]
+
+
+def _lengths(S):
+    return np.array([S, S - 3, S - 7])
 
 
 # both fp32 attention kernels
@@ -53,9 +68,12 @@ def test_layer(change, by, S, split_copies):
     x, to = (rng.randn(B, S, H).astype(np.float32) for _ in range(2))
     x *= 0.05
     change(w, to, np.float32(by))
-    lens = np.array([S, S - 3, S - 7])
+    lens = _lengths(S)
     mask = (np.arange(S)[None] < lens[:, None]).astype(np.int32)
     attr = np.ascontiguousarray(np.broadcast_to(mask[:, None], (B, S, S))).astype(np.float32)
+    if change in UNSEEN:
+        for b in range(B):
+            attr[b, :lens[b] - 1, lens[b] - 1] = 0
     packed, T, bi, wi = o.input_op_fast(x, mask)[:4]
     packed_to = o.input_op_fast(to, mask)[0]
     want = o.layer(packed, packed_to, attr, T, bi, wi, w, B, S, HEADS, D, "fp32").astype(np.float64)
@@ -72,6 +90,10 @@ def test_layer(change, by, S, split_copies):
     got = ops.effective_transformer(dx, dto, dev(attr), count, dbi, dwi, lw, B, S, S, HEADS, D)
     got = got.reshape(-1, H)[:T].cpu().numpy().astype(np.float64)
     assert np.isfinite(want).all() and np.isfinite(got).all()
+    if change in UNSEEN:
+        keep = np.ones(T, bool)
+        keep[np.cumsum(lens) - 1] = False
+        want, got = want[keep], got[keep]
     # row by row; the oracle is float32 itself: about 1e-7 per product on either side, and what these wider layers make of the
     # first ones' (scores of up to a few units: 4 x the error of plain layers, 2e-6 in test_gpu_pair.py)
     err = np.linalg.norm(got - want, axis=1) / np.linalg.norm(want, axis=1)
