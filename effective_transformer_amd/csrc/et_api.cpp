@@ -196,7 +196,7 @@ struct PairWs {
 size_t pair_array_rows(size_t rows) { return align_up(rows, 256) + 256; }      // whole tiles of any height up to 256
 size_t pair_ws_words(size_t rows, size_t H) {
   const int h = (int)H;
-  return 8 * pair_array_rows(rows) + 9 * H + 2 * et::pair_weight_stats(4 * h, h) +
+  return 8 * pair_array_rows(rows) + 9 * H + et::pair_weight_stats(4 * h, h) +
          8 * et::pair_weight_tops(h, h) + et::pair_weight_tops(h, 4 * h);
 }
 PairWs pair_ws(char* p, size_t rows, size_t H) {
@@ -208,7 +208,7 @@ PairWs pair_ws(char* p, size_t rows, size_t H) {
   w.from_norm = f; w.to_norm = f + r; w.attn_norm = f + 2 * r;
   w.w_exp = (int32_t*)(f + 3 * r);
   w.up_stats = (float*)(w.w_exp + 9 * H);
-  w.tops = w.up_stats + 2 * et::pair_weight_stats(4 * (int)H, (int)H);
+  w.tops = w.up_stats + et::pair_weight_stats(4 * (int)H, (int)H);
   return w;
 }
 
@@ -1366,7 +1366,7 @@ et_status et_gemm_split(et_handle h, const void* A, const void* Bt, void* C, con
   return check_launch(h, "et_gemm_split");
 }
 
-size_t et_pair_weight_stats(int n, int k) { return n < 1 || k < 64 ? 0 : 2 * et::pair_weight_stats(n, k); }
+size_t et_pair_weight_stats(int n, int k) { return n < 1 || k < 64 ? 0 : et::pair_weight_stats(n, k); }
 
 size_t et_pair_weight_workspace_bytes(int n, int k) { return n < 1 || k < 1 ? 0 : et::pair_weight_tops(n, k) * sizeof(float); }
 

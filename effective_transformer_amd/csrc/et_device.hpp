@@ -234,24 +234,45 @@ __device__ __forceinline__ int uniform_div(int a, int b) {
   const int r = a - q * b;
   return q - uniform_less(r, 0) + 1 - uniform_less(r, b);
 }
-// The largest first and the largest second word of `n` pairs of non-negative floats, by one wavefront: eight requests a lane, and
-// what becomes of them (and of the pairs behind the first 512).
-__device__ __forceinline__ void pair_stats_request(const float* __restrict__ stats, int n, int i0, float2v (&v)[8]) {
+// What bounds a product's columns, from the `stats` of its weight (PairWeightJob): the largest column norm, |bias| and bias (or 0).
+struct PairBounds {
+  float norm = 0.f, bias = 0.f, above = 0.f;
+};
+// By one wavefront: nine requests a lane, and what becomes of them and of the words behind them.
+struct PairStats {
+  float2v pair[8];
+  float above;
+};
+__device__ __forceinline__ void pair_stats_request(const float* __restrict__ stats, int pairs, int i0, float2v (&v)[8]) {
   const float2v* p = reinterpret_cast<const float2v*>(stats);
 #pragma unroll
-  for (int u = 0; u < 8; ++u) v[u] = p[min(i0 + u * kWave + (int)(threadIdx.x & (kWave - 1)), n - 1)];
+  for (int u = 0; u < 8; ++u) v[u] = p[min(i0 + u * kWave + (int)(threadIdx.x & (kWave - 1)), pairs - 1)];
 }
-__device__ __forceinline__ float2v pair_stats_max(const float* __restrict__ stats, int n, float2v (&v)[8]) {
+__device__ __forceinline__ void pair_stats_request(const float* __restrict__ stats, int pairs, int tiles, PairStats& s) {
+  pair_stats_request(stats, pairs, 0, s.pair);
+  s.above = stats[2 * pairs + min((int)(threadIdx.x & (kWave - 1)), tiles - 1)];
+}
+__device__ __forceinline__ PairBounds pair_stats_max(const float* __restrict__ stats, int pairs, int tiles, PairStats& s) {
   float2v top = {0.f, 0.f};
   for (int i0 = 0;;) {
 #pragma unroll
-    for (int u = 0; u < 8; ++u) top = float2v{fmaxf(top[0], v[u][0]), fmaxf(top[1], v[u][1])};
+    for (int u = 0; u < 8; ++u) top = float2v{fmaxf(top[0], s.pair[u][0]), fmaxf(top[1], s.pair[u][1])};
     i0 += 8 * kWave;
-    if (i0 >= n) break;
-    pair_stats_request(stats, n, i0, v);
+    if (i0 >= pairs) break;
+    pair_stats_request(stats, pairs, i0, s.pair);
   }
-  return float2v{wave_max(top[0]), wave_max(top[1])};
+  for (int i = (int)(threadIdx.x & (kWave - 1)) + kWave; i < tiles; i += kWave) s.above = fmaxf(s.above, stats[2 * pairs + i]);
+  return {wave_max(top[0]), wave_max(top[1]), wave_max(s.above)};
 }
+// A bound of |gelu(v)| for all v = x.w + b of a row x of this Euclidean norm: |v| <= |x| |w| + |b|, and gelu(v) lies between -0.171
+// and max(v, 0).  Without the second one bias that switches its neuron off took the bits of all others of the row (one of -2^30:
+// rows of the layer's result off by 2.9e-3).  What is above the largest value costs no bits: the product's own rounding of a value
+// is 2^-24 |x| |w| of its column, a pair's 2^-40 of this, so columns may differ by 2^14 in norm.
+__device__ __forceinline__ float pair_gelu_bound(float norm, const PairBounds& b) {
+  const float v = norm * (b.norm * 1.01f);
+  return fminf(v + b.bias, fmaxf(v + b.above, 0.171f));
+}
+
 // seq_start[b] = first packed row of sequence b (b in [0, batch]; seq_start[batch] = T), written by the thread that
 // owns packed row t in [0, T]: it covers the sequences that begin at t (token-less sequences included).
 __device__ __forceinline__ void seq_start_for_row(const int32_t* __restrict__ batch_idx, int T, int t, int batch,

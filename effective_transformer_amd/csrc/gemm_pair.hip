@@ -13,8 +13,7 @@
 //
 // Both operands come as "pair rows": [row][k / 32][h, l][32] halves, one 128-byte line per row and k-step of 32.  Both have
 // an exponent per row, which are applied to the result.  Input, LayerNorm and the pass over the context take it from the row's
-// largest value; the FFN's first product, whose workgroups see parts of a row, takes a bound instead, which costs
-// range and no bits: |x.w + b| <= |x| max|w| + max|b| (Euclidean norms).  Weights are taken anew by every layer call: pair_weight_top_kernel looks for the largest value of each
+// largest value; the FFN's first product, whose workgroups see parts of a row, takes a bound instead (pair_gelu_bound).  Weights are taken anew by every layer call: pair_weight_top_kernel looks for the largest value of each
 // column, pair_weight_kernel writes the rows (8 + 11.5 us per layer of BERT-base, split rows 15).
 // Bound: at large m the power limit of the matrix cores (20000 rows, k = 768 / n = 2304, 768, 3072 + GELU and k = 3072 / n = 768:
 // 172, 62, 258, 223 us, 1100 .. 1270 TFLOP/s of 16-bit products; split rows 301, 113, 450, 417); below a round of the chip the
@@ -42,11 +41,11 @@ struct PairGemmArgs {
   const float* bias[3];
   void* C;
   const int32_t* rows_dev;
-  // GELU: the bound of a row of C is a_norm[row] * (largest first word of b_stats) + (largest second word)
+  // GELU: what bounds the rows of C (pair_gelu_bound)
   const float* a_norm;
   const float* b_stats;
   int32_t* c_exp;
-  int n_stats;
+  int stat_pairs;
   int ldc, m_bound, n, k;
   int tiles_n, groups;                          // column tiles per group of B
   int columns;                                  // the tile order takes the column tiles of all groups this many at a time
@@ -227,8 +226,9 @@ __global__ __launch_bounds__(WM * WN * kWave) void gemm_pair_kernel(
   for (int s = 0; s < ST; ++s) issue_stage(s, min(s, nst - 1), cur, cur);
   // GELU: what bounds the rows of C, the same for every row.  Small tiles look at it, and at all that the epilogue reads, behind
   // the k loop: their launches take little longer than a round trip or two.
-  float2v bounds = {0.f, 0.f}, stats[8];
-  if constexpr (GELU) pair_stats_request(args.b_stats, args.n_stats, 0, stats);
+  PairBounds bounds;
+  PairStats stats;
+  if constexpr (GELU) pair_stats_request(args.b_stats, args.stat_pairs, (int)((unsigned)(N + 63) / 64), stats);
   wait_vmcnt<KS * Tile::DMA*(ST - 1)>();
   barrier_only();
   auto read_set = [&](half8 (&a)[2][2][MI], half8 (&b)[2][2][NJ], int slot) {
@@ -247,7 +247,7 @@ __global__ __launch_bounds__(WM * WN * kWave) void gemm_pair_kernel(
     read_set(pa[0], pb[0], 0);
   }
 
-  if constexpr (GELU && Tile::BIG) bounds = pair_stats_max(args.b_stats, args.n_stats, stats);
+  if constexpr (GELU && Tile::BIG) bounds = pair_stats_max(args.b_stats, args.stat_pairs, (int)((unsigned)(N + 63) / 64), stats);
 
   int s = 0;                                     // slot of the current stage
   bool first_tile = true;
@@ -370,10 +370,10 @@ __global__ __launch_bounds__(WM * WN * kWave) void gemm_pair_kernel(
     for (int i = 0; i < MI; ++i) asm volatile("" : "+v"(re[i]));
     if constexpr (GELU) asm volatile("" : "+v"(own_norm));
     if constexpr (GELU && !Tile::BIG)
-      if (first_tile) bounds = pair_stats_max(args.b_stats, args.n_stats, stats);
+      if (first_tile) bounds = pair_stats_max(args.b_stats, args.stat_pairs, (int)((unsigned)(N + 63) / 64), stats);
     float4v scale[MI];
     if constexpr (GELU) {                          // (every lane is active here)
-      const int e = pair_exponent(own_norm * (bounds[0] * 1.01f) + bounds[1]);
+      const int e = pair_exponent(pair_gelu_bound(own_norm, bounds));
       from_lanes<0>(scale, pair_scale(e));
       if (cur.n0 == 0 && wn == 0 && l16 < 4 * MI && own_row < rows) args.c_exp[own_row] = e;
     }
@@ -600,7 +600,7 @@ __global__ __launch_bounds__(256) void pair_weight_top_kernel(PairWeightArgs arg
 // Then 64 x 64 tiles through LDS.
 __global__ __launch_bounds__(256) void pair_weight_kernel(PairWeightArgs args) {
   __shared__ float tile[64][65];
-  __shared__ float part[2][4];
+  __shared__ float part[3][4];
   __shared__ int exps[64];
   int job = 0;
   while (job + 1 < args.jobs.count && (int)blockIdx.x >= args.tile_begin[job + 1]) ++job;
@@ -638,7 +638,7 @@ __global__ __launch_bounds__(256) void pair_weight_kernel(PairWeightArgs args) {
     }
   }
   __syncthreads();
-  float norm = 0.f, bias = 0.f;
+  float norm = 0.f, bias = 0.f, above = 0.f;
 #pragma unroll
   for (int u = 0; u < 2; ++u) {
     const int i = threadIdx.x + u * 256, r = i >> 3, c = (i & 7) * 8;        // row n0+r of the result, k0+c ..
@@ -662,20 +662,27 @@ __global__ __launch_bounds__(256) void pair_weight_kernel(PairWeightArgs args) {
       sq += dpp_f32<kDppQuadXor2>(0.f, sq);
       sq += dpp_f32<kDppRowHalfMirror>(0.f, sq);
       norm = fmaxf(norm, __builtin_ldexpf(__builtin_sqrtf(sq), e));
-      if (chunk == 0) bias = fmaxf(bias, fabsf(jb.bias[n0 + r]));
+      if (chunk == 0) {
+        const float b = jb.bias[n0 + r];
+        bias = fmaxf(bias, fabsf(b));
+        above = fmaxf(above, b);
+      }
     }
   }
   if (jb.stats == nullptr) return;
   // |column| <= sqrt(chunks) times the largest part of a column in one chunk
   norm = wave_max(norm) * __builtin_sqrtf((float)(K / 64));
   bias = wave_max(bias);
+  above = wave_max(above);
   if ((threadIdx.x & (kWave - 1)) == 0) {
     part[0][threadIdx.x / kWave] = norm;
     part[1][threadIdx.x / kWave] = bias;
+    part[2][threadIdx.x / kWave] = above;
   }
   __syncthreads();
-  if (threadIdx.x < 2)
-    jb.stats[2 * t + threadIdx.x] = fmaxf(fmaxf(part[threadIdx.x][0], part[threadIdx.x][1]), fmaxf(part[threadIdx.x][2], part[threadIdx.x][3]));
+  if (threadIdx.x < (chunk == 0 ? 3 : 2))
+    jb.stats[threadIdx.x < 2 ? 2 * t + (int)threadIdx.x : 2 * (K / 64) * tiles_n + t] =
+        fmaxf(fmaxf(part[threadIdx.x][0], part[threadIdx.x][1]), fmaxf(part[threadIdx.x][2], part[threadIdx.x][3]));
 }
 
 }  // namespace
@@ -740,7 +747,7 @@ void launch_gemm_pair(const PairProduct& p, void* C, int ldc, int m_bound, int n
   }
   a.a_norm = p.A[0].norm;
   a.b_stats = p.stats;
-  a.n_stats = (int)pair_weight_stats(n, k);
+  a.stat_pairs = (int)pair_weight_stat_pairs(n, k);
   a.c_exp = p.c_exp;
   a.C = C;
   a.rows_dev = rows_dev;

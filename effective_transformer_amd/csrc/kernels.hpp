@@ -229,10 +229,12 @@ struct PairWeightJob {
   int32_t* exp;                      // n
   float* top;                        // scratch: pair_weight_tops(n, k) words
   const float* bias;                 // with stats: n
-  float* stats;                      // may be null; pair_weight_stats pairs: a bound of columns' norms, and of |bias|
+  // may be null; per 64 k and 64 n a bound of the columns' norms and the largest |bias|, then per 64 n the largest bias (or 0)
+  float* stats;
 };
 inline size_t pair_weight_tops(int n, int k) { return (size_t)((k + 255) / 256) * n; }
-inline size_t pair_weight_stats(int n, int k) { return (size_t)(k / 64) * ((n + 63) / 64); }
+inline size_t pair_weight_stat_pairs(int n, int k) { return (size_t)(k / 64) * ((n + 63) / 64); }
+inline size_t pair_weight_stats(int n, int k) { return 2 * pair_weight_stat_pairs(n, k) + (n + 63) / 64; }
 struct PairWeightJobs {
   static constexpr int kMax = 6;
   PairWeightJob job[kMax] = {};

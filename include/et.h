@@ -402,9 +402,9 @@ et_status et_gemm_split(et_handle h, const void* A, const void* Bt, void* C, con
  * NaN give NaN in every result they enter.  k % 64 == 0, n % 16 == 0.
  * et_pair_rows writes the first m (or *m_dev) rows of src[m][k] (k <= 2048) with their exponents and Euclidean norms.
  * et_pair_weight writes the n pair rows of the transpose of src[k][n] and their exponents; `stats` (may be NULL, otherwise
- * et_pair_weight_stats(n, k) floats) receives what bounds |column| and |bias| for et_gemm_pair.  C is float [m,n]; with c_exp
+ * et_pair_weight_stats(n, k) floats) receives what bounds |column| and the bias for et_gemm_pair.  C is float [m,n]; with c_exp
  * (needs A->norm, bias and stats; n % 32 == 0) it holds the pair rows of gelu(A.Bt^T + bias) instead, whose exponents go to
- * c_exp and come from the bound |a| |column| + |bias|.  The arrays of exponents and norms of A and C have room for 511 entries
+ * c_exp and come from the bound min(|a| |column| + |bias|, max(|a| |column| + max(bias, 0), 0.171)).  The arrays of exponents and norms of A and C have room for 511 entries
  * behind the last row (whole tiles are read). */
 typedef struct et_pair_matrix {
   void* rows;                        /* 4 k bytes per row */

@@ -37,6 +37,11 @@ def _qk_head(w, x, by):
         w[at][..., 64:128] /= by
 
 
+def _neuron_off(w, x, by):
+    """One entry of the first FFN bias large and negative: its GELU is 0."""
+    w[BUP][5] = -by
+
+
 def _unseen_token(w, x, by):
     """The last token of every sequence has large values in V (each factor within what a row and a column hold), and nobody sees it
     but its own query (UNSEEN)."""
@@ -47,7 +52,7 @@ def _unseen_token(w, x, by):
     w[V][7] *= s
 
 
-CHANGES = [_plain, _qk_head, _unseen_token]
+CHANGES = [_plain, _qk_head, _neuron_off, _unseen_token]
 UNSEEN = [_unseen_token]
 
 
