@@ -521,6 +521,7 @@ struct PairWeightArgs {
   int tile_begin[PairWeightJobs::kMax + 1];
 };
 constexpr int kTopRows = 256;
+typedef __bf16 bf16x8 __attribute__((ext_vector_type(8)));
 // Rows go along in the first blocks: a launch of their own (8 x 32 tokens: 4 us) would only stand in front of this one.
 struct PairRowsArgs {
   PairRowsJob job[2];
@@ -558,14 +559,19 @@ __global__ __launch_bounds__(256) void pair_weight_top_kernel(PairWeightArgs arg
   const int K = jb.k, N = jb.n, tiles_n = (N + 63) / 64;
   const int t = wg - args.tile_begin[job];
   const int block = t / tiles_n, k0 = block * kTopRows, n0 = (t - block * tiles_n) * 64;
-  if (jb.src_split) {                            // rows of three bfloat16 pieces: four lanes per row, 64 k each
-    const int r = threadIdx.x >> 2, kk = k0 + (threadIdx.x & 3) * 64;
+  if (jb.src_split) {                            // rows of three bfloat16 pieces: four lanes per row, every fourth 8 k each
+    // (64 consecutive k a lane, value by value: a layer of 32 positions from split copies 74 us, so 69; from floats 67)
+    const int r = threadIdx.x >> 2, c = (threadIdx.x & 3) * 8;
     float top = 0.f;
-    if (n0 + r < N && kk < K) {
-      const __bf16* p = (const __bf16*)jb.src + (size_t)(n0 + r) * K * 3 + (kk >> 5) * 96;
-      for (int i = 0; i < 64; ++i) {
-        const __bf16* q = p + (i >> 5) * 96 + (i & 31);
-        top = fmaxf(top, fabsf(((float)q[0] + (float)q[32]) + (float)q[64]));
+    if (n0 + r < N) {
+      const __bf16* p = (const __bf16*)jb.src + (size_t)(n0 + r) * K * 3 + (size_t)(k0 >> 5) * 96 + c;
+      const int lines = min(K - k0, kTopRows) / 32;
+#pragma unroll 4
+      for (int i = 0; i < lines; ++i) {
+        const bf16x8 h = *reinterpret_cast<const bf16x8*>(p + i * 96), m = *reinterpret_cast<const bf16x8*>(p + i * 96 + 32),
+                     l = *reinterpret_cast<const bf16x8*>(p + i * 96 + 64);
+#pragma unroll
+        for (int j = 0; j < 8; ++j) top = fmaxf(top, fabsf(((float)h[j] + (float)m[j]) + (float)l[j]));
       }
     }
     top = fmaxf(top, dpp_f32<kDppQuadXor1>(top, top));
@@ -615,7 +621,6 @@ __global__ __launch_bounds__(256) void pair_weight_kernel(PairWeightArgs args) {
     if (chunk == 0) jb.exp[n0 + threadIdx.x] = exps[threadIdx.x];
   }
   if (jb.src_split) {                            // rows of three bfloat16 pieces, whose sum is the float
-    typedef __bf16 bf16x8 __attribute__((ext_vector_type(8)));
 #pragma unroll
     for (int u = 0; u < 2; ++u) {
       const int i = threadIdx.x + u * 256, r = i >> 3, c = (i & 7) * 8;      // row n0+r, k0+c ..

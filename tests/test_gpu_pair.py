@@ -3,7 +3,7 @@ import numpy as np
 import pytest
 import torch
 
-from effective_transformer_amd import kernel_ops as k, ops
+from effective_transformer_amd import _lib, kernel_ops as k, ops
 from oracle import et_oracle as o
 from gpu_util import dev
 
@@ -133,6 +133,26 @@ def test_layer(heads, d, B, S, scale):
     # (the oracle is float32 itself: about 1e-7 per product on either side, eight of them in a row)
     assert (got[~valid] == 0).all()
     assert np.linalg.norm(got[valid] - want[valid]) <= 2e-6 * np.linalg.norm(want[valid])
+
+
+# split copies of the weights (et_layer_prepared) hold the same floats: the same bits.  Widths that end inside the 256 k a block looks
+# at for the columns' largest values.
+@pytest.mark.parametrize("heads", [8, 9, 17])
+def test_split_copies(heads):
+    print("split copies", heads, flush=True)
+    d, B, S, H = 64, 2, 24, heads * 64
+    g = torch.Generator(device="cuda").manual_seed(heads)
+    sizes = [(H, H), (H,)] * 4 + [(H,), (H,), (H, 4 * H), (4 * H,), (4 * H, H), (H,), (H,), (H,)]
+    w = [torch.randn(*s, device="cuda", generator=g) * 0.05 for s in sizes]
+    x = torch.randn(B, S, H, device="cuda", generator=g)
+    mask = torch.ones(B, S, dtype=torch.int32, device="cuda")
+    attr = torch.ones(B, S, S, device="cuda")
+    dx, count, bi, wi = ops.effective_transformer_input(x, mask, B, S, S, heads, d)
+    lw = ops.LayerWeights.from_slots(torch.device("cuda"), torch.float32, w)
+    plain = ops.effective_transformer(dx, dx, attr, count, bi, wi, lw, B, S, S, heads, d)
+    copies = [k.transpose_weight(w[i]) for i in (0, 2, 4, 6, 10, 12)]
+    lw.prepared = _lib.LayerPrepared(*[t.data_ptr() for t in copies])
+    assert torch.equal(ops.effective_transformer(dx, dx, attr, count, bi, wi, lw, B, S, S, heads, d), plain)
 
 
 # the streaming attention of layers on pair rows (more than 32 positions): lengths around its stages of 32 keys and blocks of 64
