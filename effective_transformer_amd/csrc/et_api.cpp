@@ -193,7 +193,7 @@ struct PairWs {
   int32_t *from_exp, *to_exp, *ctx_exp, *attn_exp, *inter_exp, *w_exp;      // w_exp: Q, K, V, output, up, down
   float *from_norm, *to_norm, *attn_norm, *up_stats, *tops;
 };
-size_t pair_array_rows(size_t rows) { return align_up(rows, 256) + 256; }      // whole tiles of any height up to 256
+size_t pair_array_rows(size_t rows) { return align_up(rows + 255, 256); }      // whole tiles of any height up to 256
 size_t pair_ws_words(size_t rows, size_t H) {
   const int h = (int)H;
   return 8 * pair_array_rows(rows) + 9 * H + et::pair_weight_stats(4 * h, h) +

@@ -2,8 +2,10 @@
 // reference: tf_op/bert_transformer_op.cu.cc:110-141, 200-240), for hidden sizes of 512 and more in multiples of 64.
 //
 // A float x of a row whose values stay below 2^(e+15) is held as the pair h + l of halves, h = x 2^-e rounded to nearest and
-// l the rest rounded to nearest: 22 to 24 significant bits, down to 2^-40 of the row's bound.  A product of two such floats is
-// h.h + h.l + l.h (l.l is at most 2^-24 of it, the size of a float's own rounding), three products for v_mfma_f32_16x16x32_f16
+// l the rest rounded to nearest (the two-piece split of Ootomo and Yokota, "Recovering single precision accuracy from Tensor Cores
+// while surpassing the FP32 theoretical peak performance", 2022, with an exponent per row): off by at most 2^-23 of x, or, below
+// 2^-16 of the row's bound, where l is a subnormal half, 2^-39 of the bound.  A product of two such floats is h.h + h.l + l.h (l.l
+// is at most 2^-22 of it, 2^-25 in the mean), three products for v_mfma_f32_16x16x32_f16
 // where three bfloat16 pieces take six (gemm_split.hip).  They are summed in chunks of 64 k, smallest first within each 32, and
 // the chunks in float adds: fewer roundings at the size of the whole sum than one chain of matrix instructions has.  Error
 // against float64, normal operands, relative (this / three bfloat16 pieces / fp32 matrix instructions): k = 512 1.22e-7 /
@@ -544,8 +546,7 @@ __global__ __launch_bounds__(256) void pair_weight_top_kernel(PairWeightArgs arg
     const PairRowsJob& job = rows.job[which];
     const int block = wg - (which ? rows.blocks[0] : 0), blocks = rows.blocks[which];
     switch ((job.n / 4 + kWave - 1) / kWave) {
-      case 1: return pair_rows_blocks<1>(job, block, blocks);
-      case 2: return pair_rows_blocks<2>(job, block, blocks);
+      case 2: return pair_rows_blocks<2>(job, block, blocks);      // (layers on pair rows have 512 values a row and more)
       case 3: return pair_rows_blocks<3>(job, block, blocks);
       case 4: return pair_rows_blocks<4>(job, block, blocks);
       case 5: case 6: return pair_rows_blocks<6>(job, block, blocks);

@@ -19,8 +19,8 @@ void allow_dynamic_lds(const void* kernel, int bytes);
 hipError_t take_attribute_error();
 
 // A matrix of pair rows (gemm_pair.hip): n values per row as [n / 32][h, l][32] halves, the exponent of each row, and the
-// row's Euclidean norm, from which what is computed of it is bounded.  Row arrays have room for 256 rows
-// more than the matrix (a tile reads them whole).
+// row's Euclidean norm, from which what is computed of it is bounded.  Row arrays have room for 255 entries
+// behind the last row (a tile reads them whole).
 struct PairRows {
   _Float16* rows = nullptr;
   int32_t* exp = nullptr;

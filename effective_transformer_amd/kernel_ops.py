@@ -164,8 +164,8 @@ class PairRows:
 
     def __init__(self, m: int, k: int, device):
         self.rows = torch.zeros(m, 2 * k, dtype=torch.float16, device=device)
-        self.exp = torch.zeros(m + 511, dtype=torch.int32, device=device)
-        self.norm = torch.zeros(m + 511, dtype=torch.float32, device=device)
+        self.exp = torch.zeros(m + 255, dtype=torch.int32, device=device)
+        self.norm = torch.zeros(m + 255, dtype=torch.float32, device=device)
 
     def c_struct(self):
         return _lib.PairMatrix(self.rows.data_ptr(), self.exp.data_ptr(), self.norm.data_ptr())

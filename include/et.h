@@ -133,8 +133,8 @@ et_status et_input_static(et_handle h, et_dtype dtype, const void* from_tensor, 
  * cuda/attention.cu:190-219).
  * The weights are read anew by every call and stay as they are: the copies the products read (k-contiguous in fp16, split
  * rows in fp32, see et_gemm_split) are made in the workspace.  fp32 products of hidden sizes in multiples of 64 from 512 to 2048
- * run on pair rows, other multiples of 32 on split rows: what et_gemm_pair and et_gemm_split say of infinities and of the terms
- * they leave out goes for them. */
+ * run on pair rows, other multiples of 32 on split rows: what et_gemm_pair and et_gemm_split say of infinities, of the terms they
+ * leave out and of how values far below the largest of their row or column are held goes for them. */
 et_status et_layer(et_handle h, et_dtype dtype, const et_layer_weights* weights,
                    const void* from_tensor, const void* to_tensor, const void* attr_mask,
                    const int32_t* valid_word_num_dev, const int32_t* batch_idx, const int32_t* word_idx,
@@ -397,16 +397,22 @@ et_status et_gemm_split(et_handle h, const void* A, const void* Bt, void* C, con
 
 /* The fp32 product of the layer at hidden sizes in multiples of 64 from 512 to 2048, on the fp16 matrix cores:
  * C[m,n] = A[m,k] . Bt[n,k]^T (+ bias).  Both operands are pair rows, [row][k / 32][2][32] halves, with an exponent e per row:
- * x 2^-e = h + l, h rounded to nearest (below 2^15) and l the rest rounded to nearest.  That keeps 22 to 24 significant bits of
- * values down to about 2^-30 of the row's largest, and 2^-40 of it below.  h.h, h.l and l.h are summed in float, l.l (at most 2^-24
- * of a product) is left out; from k = 512 on the result is closer to float64 than et_gemm_split's and et_gemm's.  Infinities and
- * NaN give NaN in every result they enter.  k % 64 == 0, n % 16 == 0.
+ * x 2^-e = h + l, h rounded to nearest (below 2^15) and l the rest rounded to nearest.  A value is held to 2^-23 of itself down to
+ * 2^-16 of the largest value of its row (of A; of its column for a weight), and to 2^-39 of that largest value below: one 2^-20 of
+ * it keeps 19 bits, one 2^-30 of it 9.  (With c_exp the bound below stands for the row's largest value.)  So a sum to which the
+ * large values of a row contribute nothing, because they meet weights of zero or far below their column's largest, is as good as
+ * the small values are held; where that matters, et_gemm_split and et_gemm keep every value's own exponent.  h.h, h.l and l.h are
+ * summed in float, l.l (at most 2^-22 of a product, 2^-25 in the mean) is left out; for values of ordinary spread the result is closer to
+ * float64 than et_gemm_split's and et_gemm's from k = 512 on.  Infinities and NaN give NaN in every result they enter.
+ * k % 64 == 0, n % 16 == 0.
  * et_pair_rows writes the first m (or *m_dev) rows of src[m][k] (k <= 2048) with their exponents and Euclidean norms.
  * et_pair_weight writes the n pair rows of the transpose of src[k][n] and their exponents; `stats` (may be NULL, otherwise
  * et_pair_weight_stats(n, k) floats) receives what bounds |column| and the bias for et_gemm_pair.  C is float [m,n]; with c_exp
  * (needs A->norm, bias and stats; n % 32 == 0) it holds the pair rows of gelu(A.Bt^T + bias) instead, whose exponents go to
- * c_exp and come from the bound min(|a| |column| + |bias|, max(|a| |column| + max(bias, 0), 0.171)).  The arrays of exponents and norms of A and C have room for 511 entries
- * behind the last row (whole tiles are read). */
+ * c_exp and come from the bound min(|a| |column| + |bias|, max(|a| |column| + max(bias, 0), 0.171)), with the
+ * largest column norm, |bias| and bias of the whole weight: no bits are lost to it while the columns' norms lie within 2^14 of each
+ * other.  The arrays of exponents and norms of A and C are 16-byte aligned and have room for 255 entries behind the last row (whole
+ * tiles are read). */
 typedef struct et_pair_matrix {
   void* rows;                        /* 4 k bytes per row */
   int32_t* exp;
