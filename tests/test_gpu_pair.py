@@ -60,24 +60,31 @@ def test_gemm_pair(m, n, kk, positive):
 
 
 # pair rows as the result: widths that fill a wavefront's columns in part, rows that end inside the 16 whose exponents 16 lanes
-# share, every tile shape; row by row (another lane's exponent would be off by powers of two), the rows' sizes far apart
+# share, every tile shape, more weight statistics than one wavefront requests at once; row by row (another lane's exponent would be off
+# by powers of two), the rows' sizes far apart; off: a bias that switches its column off
 @pytest.mark.parametrize("m,n,kk", [(1, 32, 64), (7, 96, 128), (50, 160, 192), (67, 1056, 768), (331, 800, 512), (1500, 800, 768),
-                                    (3001, 1184, 768), (9003, 1056, 512)])
-def test_pair_rows_out(m, n, kk):
-    print("pair rows out", m, n, kk, flush=True)
+                                    (3001, 1184, 768), (9003, 1056, 512), (40, 8192, 64), (300, 4608, 1024)])
+@pytest.mark.parametrize("off", [0.0, -1e6, -1e12])
+def test_pair_rows_out(m, n, kk, off):
+    print("pair rows out", m, n, kk, off, flush=True)
     a, b, bias = _operands(m, n, kk, False)
+    bias[n // 2] += off
     a *= torch.logspace(-3, 1, 5, device="cuda").repeat((m + 4) // 5)[:m, None]
     pb, stats = k.pair_weight(b, bias)
     act = k.gemm_pair(k.pair_rows(a), pb, bias=bias, stats=stats, gelu=True).values()
     want = torch.nn.functional.gelu((a.cpu().double() @ b.cpu().double()).cuda() + bias.double(), approximate="tanh")
-    # the product's own error as above; h + l: half a unit of 2^-22 of a value and 2^-39 of the row's bound; GELU's exp2 and
-    # reciprocal one unit each
-    bound = a.double().norm(dim=1) * b.double().norm(dim=0).max() * 1.02 + bias.abs().max().double()
-    assert ((act - want).norm(dim=1) <= 1e-6 * want.norm(dim=1) + bound * n ** 0.5 * 2.0 ** -38).all()
+    # The product's own error, a few units of 2^-24 of |a| |column| (and as much of the bias's rounding), which GELU's slope of at most
+    # 1.13 passes on; h + l: 2^-23 of a value and 2^-39 of the row's bound, which is no more than |a| |column| + the largest bias
+    # above 0 or 0.171, so far below the first; GELU's exp2 and reciprocal a unit each, of v where the result is 0.  What does not
+    # enter: a bias far below 0.
+    sizes = a.double().norm(dim=1)[:, None] * b.double().norm(dim=0)[None] + bias.clamp(-8, 8).abs().double()[None]
+    bound = a.double().norm(dim=1) * b.double().norm(dim=0).max() * 1.03 + bias.clamp(min=0).max().double()
+    assert ((act - want).abs() <= 2.0 ** -20 * want.abs() + 2.0 ** -22 * sizes + 2.0 ** -39 * bound.clamp(min=0.171)[:, None]).all()
 
 
 # the exponents take what rows and columns differ by: the same relative error at 1e30, 1e-30 and in between, row by row; zero
-# rows and columns are zero; what a row cannot hold (2^-40 of its largest value) is all that is lost
+# rows and columns are zero; what a row or a column cannot hold (2^-39 of its largest value) is all that is lost, also where its
+# largest value meets zeros
 def test_magnitudes():
     a, b, _ = _operands(70, 64, 768)
     rows = torch.tensor([1e30, 1e-25, 1.0, 1e5, 1e-5], device="cuda").repeat(14)[:, None]
@@ -87,8 +94,19 @@ def test_magnitudes():
     got = k.gemm_pair(k.pair_rows(a), k.pair_weight(b)[0]).double().cpu()
     want = a.cpu().double() @ b.cpu().double()
     assert (got[3] == 0).all() and (got[:, 5] == 0).all()
-    scale = (a.double().norm(dim=1)[:, None] * b.double().norm(dim=0)[None]).cpu()
-    assert ((got - want).abs() <= 1e-6 * scale).all()
+    # operands off by 2^-23 each, l.l of 2^-22 at most, a chunk's sums and theirs by a few units
+    scale = a.cpu().double().abs() @ b.cpu().double().abs()
+    assert ((got - want).abs() <= 2.0 ** -20 * scale).all()
+    for spread in (2.0 ** 12, 2.0 ** 20, 2.0 ** 30):
+        a, b, _ = _operands(40, 64, 768)
+        a[:, 5] *= spread                                    # large values of A meet zeros, but in column 3
+        b[5], b[5, 3] = 0, 0.01
+        b[9, :32] *= spread                                  # and large values of half the columns of B
+        a[:, 9] = 0
+        got = k.gemm_pair(k.pair_rows(a), k.pair_weight(b)[0]).double().cpu()
+        a, b = a.cpu().double(), b.cpu().double()
+        lost = a.abs().amax(1, keepdim=True) * b.abs().sum(0) + a.abs().sum(1, keepdim=True) * b.abs().amax(0)
+        assert ((got - a @ b).abs() <= 2.0 ** -20 * (a.abs() @ b.abs()) + 2.0 ** -39 * lost).all()
     wide = torch.randn(8, 768, device="cuda") * torch.logspace(0, -9, 768, device="cuda")
     err = (k.pair_rows(wide).values() - wide.double()).abs()
     assert (err <= wide.double().abs() * 2.0 ** -23 + wide.abs().amax(1, keepdim=True).double() * 2.0 ** -39).all()

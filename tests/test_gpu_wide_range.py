@@ -1,5 +1,5 @@
-"""fp32 layers on pair rows whose weights or rows hold values of very different size: what lies far below the largest value of a
-row, a column, a head or a sequence keeps the precision of float."""
+"""fp32 layers on pair rows whose weights or rows hold values of very different size: heads of Q and K, biases and tokens may differ
+by any power of two, values of one row or column by 2^20, and the layer's rows keep the precision of float."""
 import numpy as np
 import pytest
 import torch
@@ -52,7 +52,15 @@ def _unseen_token(w, x, by):
     w[V][7] *= s
 
 
-CHANGES = [_plain, _qk_head, _neuron_off, _unseen_token]
+def _v_head(w, x, by):
+    """A head of V and its rows of the output kernel: what a row and a column hold reaches 2^20 down."""
+    s = np.sqrt(by)
+    for at in (V, BV):
+        w[at][..., 64:128] *= s
+    w[OUT][64:128] /= s
+
+
+CHANGES = [_plain, _qk_head, _neuron_off, _unseen_token, _v_head]
 UNSEEN = [_unseen_token]
 
 
