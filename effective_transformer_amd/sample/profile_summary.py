@@ -23,7 +23,9 @@ from .workloads import WORKLOADS
 
 ROLES = ["QKV", "attention", "attention out", "LayerNorm 1", "FFN up + GELU", "FFN down", "LayerNorm 2"]
 SIDE = ("scan_index", "compress_rows", "embed_layernorm", "seq_start", "seq_order", "mask_class", "pair_weight", "pair_rows", "restore_rows")
-LAYER_KINDS = ("attention", "bias_residual_layernorm", "gemm_f16_pair", "gemm_f16_bt", "gemm_f16_persistent", "gemm_f16_kernel",
+# fp32 products on pair rows: the context's rows are paired by a launch of their own
+PAIR_ROLES = ROLES[:2] + ["context to pair rows"] + ROLES[2:]
+LAYER_KINDS = ("context_rows", "attention", "bias_residual_layernorm", "gemm_f16_pair", "gemm_f16_bt", "gemm_f16_persistent", "gemm_f16_kernel",
                "gemm_f32", "gemm_pair_kernel", "gemm_split")
 
 
@@ -51,19 +53,33 @@ def kind(name: str) -> str:
     return name[:30]
 
 
+def mark_context(dispatches):
+    """Pair rows made right behind an attention kernel are the context's."""
+    for a, b in zip(dispatches, dispatches[1:]):
+        if a["kind"] == "attention" and b["kind"] == "pair_rows":
+            b["kind"] = "context_rows"
+    return dispatches
+
+
+def roles_of(body, layers):
+    return PAIR_ROLES if len(body) == len(PAIR_ROLES) * layers else ROLES
+
+
 def encoder_steps(kinds, layers):
-    """Index lists of the 7 x layers layer kernels of every complete encoder step (input op ... output op) in a
-    dispatch sequence."""
+    """Index lists of the 7 (fp32 on pair rows: 8) x layers layer kernels of every complete encoder step (input op ... output
+    op) in a dispatch sequence."""
     steps, i = [], 0
     while i < len(kinds):
-        if kinds[i] in ("compress_rows", "pair_rows", "embed_layernorm"):
+        # (one layer: the first rows are made in the launch that looks at its weights)
+        if kinds[i] in ("compress_rows", "pair_rows", "embed_layernorm", "scan_index"):
             j = i + 1
             while j < len(kinds) and kinds[j] not in ("restore_rows", "compress_rows", "pair_rows", "embed_layernorm", "scan_index"):
                 j += 1
             if j < len(kinds) and kinds[j] == "restore_rows":
                 # the layer kernels only: no table build, no prologue, no runtime copy kernel (read-back of the count)
                 body = [q for q in range(i + 1, j) if kinds[q] in LAYER_KINDS]
-                if len(body) == 7 * layers:
+                contexts = sum(kinds[q] == "context_rows" for q in body)
+                if len(body) == (7 + (contexts > 0)) * layers and contexts in (0, layers):
                     steps.append(body)
             i = j
         else:
@@ -74,8 +90,8 @@ def encoder_steps(kinds, layers):
 def load_trace(path):
     rows = list(csv.DictReader(open(path)))
     rows.sort(key=lambda r: int(r["Start_Timestamp"]))
-    return [dict(name=r["Kernel_Name"], kind=kind(r["Kernel_Name"]),
-                 us=(int(r["End_Timestamp"]) - int(r["Start_Timestamp"])) / 1e3) for r in rows]
+    return mark_context([dict(name=r["Kernel_Name"], kind=kind(r["Kernel_Name"]),
+                              us=(int(r["End_Timestamp"]) - int(r["Start_Timestamp"])) / 1e3) for r in rows])
 
 
 def role_durations(trace, layers, skip=3):
@@ -83,9 +99,11 @@ def role_durations(trace, layers, skip=3):
     steps = encoder_steps([t["kind"] for t in trace], layers)
     agg, names = collections.defaultdict(list), {}
     for body in steps[min(skip, max(0, len(steps) - 1)):]:
+        roles = roles_of(body, layers)
         for q, idx in enumerate(body):
-            agg[ROLES[q % 7]].append(trace[idx]["us"])
-            names[ROLES[q % 7]] = short(trace[idx]["name"])
+            role = roles[q % len(roles)]
+            agg[role].append(trace[idx]["us"])
+            names[role] = short(trace[idx]["name"])
     return agg, names, len(steps)
 
 
@@ -95,7 +113,7 @@ def load_counters(path):
     for r in csv.DictReader(open(path)):
         d = by_id.setdefault(int(r["Dispatch_Id"]), dict(name=r["Kernel_Name"], kind=kind(r["Kernel_Name"]), counters={}))
         d["counters"][r["Counter_Name"]] = d["counters"].get(r["Counter_Name"], 0.0) + float(r["Counter_Value"])
-    return [by_id[k] for k in sorted(by_id)]
+    return mark_context([by_id[k] for k in sorted(by_id)])
 
 
 def role_counters(disp, layers):
@@ -103,9 +121,10 @@ def role_counters(disp, layers):
     steps = encoder_steps([d["kind"] for d in disp], layers)
     agg = collections.defaultdict(lambda: collections.defaultdict(list))
     for body in steps:
+        roles = roles_of(body, layers)
         for q, idx in enumerate(body):
             for c, v in disp[idx]["counters"].items():
-                agg[ROLES[q % 7]][c].append(v)
+                agg[roles[q % len(roles)]][c].append(v)
     side = collections.defaultdict(lambda: collections.defaultdict(list))
     for d in disp:
         if d["kind"] in SIDE + ("bias_gelu", "copyBuffer", "layer_prologue"):
@@ -128,6 +147,7 @@ def algorithmic(workload, tokens):
             "FFN up + GELU": dict(flops=2.0 * T * F * H, read=(T * H + H * F) * e, write=T * F * e),
             "FFN down": dict(flops=2.0 * T * F * H, read=(T * F + H * F) * e, write=T * H * e),
             "attention": dict(read=3 * T * H * e + B * S * S * e + 8 * T, write=T * H * e),
+            "context to pair rows": dict(read=T * H * e, write=T * H * e + 8 * T),
             "LayerNorm 1": dict(read=2 * T * H * e + 3 * H * e, write=T * H * e),
             "LayerNorm 2": dict(read=2 * T * H * e + 3 * H * e, write=T * H * e)}
 
@@ -160,10 +180,15 @@ def cmd_kernels(d, name, workload, bench_json=None):
         out.append("| %s | %s | %.3f | %.2f | %.2f | %.2f | %s |" % (
             short(r["Name"]), r["Calls"], float(r["TotalDurationNs"]) / 1e6, float(r["AverageNs"]) / 1e3,
             float(r["MinNs"]) / 1e3, float(r["MaxNs"]) / 1e3, r["Percentage"]))
-    out.append("\nThe counts include `bench.py`'s per-kernel loops and its replica of the layer's launch sequence; `bias_gelu_kernel`,")
-    out.append("`layer_prologue_kernel` and `embed_layernorm_kernel` only run there (the layer applies bias + GELU in the FFN-up GEMM's")
-    out.append("epilogue and, with prepared weights, launches no prologue), and so do `seq_start_kernel` and `seq_order_kernel` (the encoder's")
-    out.append("scan writes the sequence table, its first row kernel sorts it).\n")
+    rows = [r["Name"] for r in csv.DictReader(open("%s/%s_kernel_stats.csv" % (d, name)))]
+    why = {"bias_gelu_kernel": "the layer applies bias + GELU in the FFN-up GEMM's epilogue",
+           "layer_prologue_kernel": "with prepared weights the layer launches no prologue",
+           "embed_layernorm_kernel": "the encoder is given rows, not ids",
+           "seq_start_kernel": "the encoder's scan writes the sequence table",
+           "seq_order_kernel": "its first row kernel sorts it"}
+    there = [k for k in why if any(k in r for r in rows)]
+    out.append("\nThe counts include `bench.py`'s per-kernel loops and its replica of the layer's launch sequence; only there run "
+               + ", ".join("`%s` (%s)" % (k, why[k]) for k in there) + ".\n")
     trace = load_trace("%s/%s_kernel_trace.csv" % (d, name))
     agg, names, nsteps = role_durations(trace, wl.layers)
     if agg:
@@ -175,7 +200,7 @@ def cmd_kernels(d, name, workload, bench_json=None):
         out.append("| launch | kernel | calls | avg us | min us | max us | algorithmic work | achieved | of peak |")
         out.append("|---|---|---|---|---|---|---|---|---|")
         tot = 0.0
-        for role in ROLES:
+        for role in (r for r in PAIR_ROLES if r in agg):
             v = agg[role]
             a = mean(v)
             tot += a
@@ -197,6 +222,7 @@ def cmd_kernels(d, name, workload, bench_json=None):
                 side[k] = mean(v)
         if "pair_weight" in side:                                                  # fp32: two launches per layer
             side["pair_weight"] *= 2
+            side.pop("compress_rows", None)                                        # (bench.py's own call of the input op)
         tot += side.get("pair_weight", 0.0)
         out.append("\nPeaks: fp16 MFMA 2500 TFLOP/s, fp32 MFMA 157.3, products of pair rows 2500 / 3, HBM 8 TB/s.  Sum per layer%s: %.1f us; x %d layers + what a batch takes once (%s) = %.3f ms per batch."
                    % (" with pair_weight %.1f" % side["pair_weight"] if "pair_weight" in side else "", tot, wl.layers,
@@ -230,7 +256,7 @@ def cmd_traffic(fetch_csv, write_csv, workload):
     out.append("takes `roofline.traffic` from.\n")
     out.append("| launch | dispatches | read MiB | write MiB | algorithmic read / write MiB | read / algorithmic | total / algorithmic |")
     out.append("|---|---|---|---|---|---|---|")
-    for role in ROLES:
+    for role in (r for r in PAIR_ROLES if r in fagg):
         f = mean(fagg[role].get("FETCH_SIZE", [])) * sf / 1024.0
         w = mean(wagg[role].get("WRITE_SIZE", [])) * sw / 1024.0
         a = alg[role]
@@ -263,10 +289,8 @@ def cmd_counters(counter_csv, trace_csv, workload):
     out.append("per XCD x 1024 SIMDs)`; MFMA GFLOP = `%s x 512`.\n" % mops)
     out.append("| launch | dispatches | GUI active cycles per XCD | avg duration us (kernel trace) | cycles / duration (GHz) | MFMA busy % | MFMA GFLOP per launch | algorithmic GFLOP | LDS bank-conflict cycles / LDS active cycles |")
     out.append("|---|---|---|---|---|---|---|---|---|")
-    for role in ROLES:
+    for role in (r for r in PAIR_ROLES if r in agg):
         c = agg[role]
-        if not c:
-            continue
         gui = mean(c.get("GRBM_GUI_ACTIVE", [])) / 8.0
         busy = mean(c.get("SQ_VALU_MFMA_BUSY_CYCLES", []))
         us = mean(dur.get(role, []))

@@ -134,6 +134,22 @@ def test_profile_summary_cuts_encoder_steps_out_of_a_dispatch_sequence(tmp_path)
     assert ps.encoder_steps([t["kind"] for t in trace], layers=3) == []  # a different layer count matches nothing
 
 
+def test_profile_summary_tells_the_contexts_rows_from_the_inputs(tmp_path):
+    """fp32 layers on pair rows: eight launches, the third of them the kernel that also makes the first layer's rows; one layer
+    alone has no launch for those."""
+    from effective_transformer_amd.sample import profile_summary as ps
+    layer = ["gemm_pair_kernel<a>", "attention_flash_f32_kernel", "pair_rows_kernel<3>", "gemm_pair_kernel<a>",
+             "bias_residual_layernorm_kernel<c>", "gemm_pair_kernel<b>", "gemm_pair_kernel<a>", "bias_residual_layernorm_kernel<c>"]
+    weights = ["pair_weight_top_kernel", "pair_weight_kernel"]
+    for first, layers in ((["scan_index_kernel", "pair_rows_kernel<3>", "mask_class_kernel<f>"], 2), (["scan_index_kernel"], 1)):
+        names = 2 * (first + layers * (weights + layer) + ["restore_rows_kernel<x>"])
+        trace = ps.mark_context([dict(name=n, kind=ps.kind(n), us=1.0) for n in names])
+        steps = ps.encoder_steps([t["kind"] for t in trace], layers)
+        assert len(steps) == 2 and [names[i] for i in steps[1]] == layers * layer
+        agg, _, _ = ps.role_durations(trace, layers, skip=0)
+        assert list(agg) == ps.PAIR_ROLES and all(len(v) == 2 * layers for v in agg.values())
+
+
 def test_profile_summary_prices_launches_with_the_documented_formulas():
     from effective_transformer_amd.sample import profile_summary as ps
     from effective_transformer_amd.sample.workloads import WORKLOADS
