@@ -5,9 +5,9 @@
 // l the rest rounded to nearest (the two-piece split of Ootomo and Yokota, "Recovering single precision accuracy from Tensor Cores
 // while surpassing the FP32 theoretical peak performance", 2022, with an exponent per row): off by at most 2^-23 of x, or, below
 // 2^-16 of the row's bound, where l is a subnormal half, 2^-39 of the bound.  A product of two such floats is h.h + h.l + l.h (l.l
-// is at most 2^-22 of it, 2^-25 in the mean), three products for v_mfma_f32_16x16x32_f16
-// where three bfloat16 pieces take six (gemm_split.hip).  They are summed in chunks of 64 k, smallest first within each 32, and
-// the chunks in float adds: fewer roundings at the size of the whole sum than one chain of matrix instructions has.  Error
+// is at most 2^-22 of it, 2^-25 in the mean), three products for v_mfma_f32_16x16x32_f16 where three bfloat16 pieces take six
+// (gemm_split.hip).  They are summed in chunks of 64 k, smallest first within each 32, and the chunks in float adds: fewer
+// roundings at the size of the whole sum than one chain of matrix instructions has.  Error
 // against float64, normal operands, relative (this / three bfloat16 pieces / fp32 matrix instructions): k = 512 1.22e-7 /
 // 1.27e-7 / 3.8e-7, 768 1.28e-7 / 1.59e-7, 1024 1.34e-7 / 1.87e-7, 3072 1.73e-7 / 3.41e-7 / 9.9e-7, 4096 1.87e-7 / 3.96e-7; all
 // operands positive: 5.0e-8 / 1.21e-7 at k = 512, 1.1e-7 / 3.05e-7 at 3072.  Below k = 512 the three pieces are closer, and
@@ -15,11 +15,12 @@
 //
 // Both operands come as "pair rows": [row][k / 32][h, l][32] halves, one 128-byte line per row and k-step of 32.  Both have
 // an exponent per row, which are applied to the result.  Input, LayerNorm and the pass over the context take it from the row's
-// largest value; the FFN's first product, whose workgroups see parts of a row, takes a bound instead (pair_gelu_bound).  Weights are taken anew by every layer call: pair_weight_top_kernel looks for the largest value of each
-// column, pair_weight_kernel writes the rows (8 + 11.5 us per layer of BERT-base, split rows 15).
-// Bound: at large m the power limit of the matrix cores (20000 rows, k = 768 / n = 2304, 768, 3072 + GELU and k = 3072 / n = 768:
-// 172, 62, 258, 223 us, 1100 .. 1270 TFLOP/s of 16-bit products; split rows 301, 113, 450, 417); below a round of the chip the
-// k loop of one tile (160 rows: 8.6, 7.8, 10, 14.3 us against 15, 10, 16.5, 21).
+// largest value; the FFN's first product, whose workgroups see parts of a row, takes a bound instead (pair_gelu_bound).  Weights
+// are taken anew by every layer call: pair_weight_top_kernel looks for the largest value of each column, pair_weight_kernel
+// writes the rows (9 + 11.5 us per layer of BERT-base, split rows 15).
+// Bound: at large m the power limit of the matrix cores (20375 rows, k = 768 / n = 2304, 768, 3072 + GELU and k = 3072 / n = 768:
+// 180, 64, 270, 233 us in the layer, 1070 .. 1240 TFLOP/s of 16-bit products; split rows 307, 112, 451, 413); below a round of the
+// chip the k loop of one tile (134 rows: 10.2, 6.5, 12.8, 14.3 us against 15.2, 8.7, 16.1, 21.3).
 #include <algorithm>
 #include <atomic>
 #include <iterator>
@@ -269,7 +270,7 @@ __global__ __launch_bounds__(WM * WN * kWave) void gemm_pair_kernel(
     int4v re[MI] = {};
     const int row0 = cur.m0 + wm * 16 * MI + g * 4;
     // Pair rows out: the 16 lanes that store the same 4 MI rows see to one row's exponent each, and hand it round (every lane for
-    // all of them was a fifth of an epilogue's instructions: encoders of 500 x 64 2860 -> 2844 us, 4 x 1000 915 -> 906).
+    // all of them was a fifth of an epilogue's instructions: store_pair has the figure).
     const int own_row = row0 + min(l16 >> 2, MI - 1) * 16 + (l16 & 3);
     float own_norm = 0.f;
     auto request = [&](const int32_t* a_exp, const int32_t* b_exp, const float* add, const float* norm) {

@@ -147,7 +147,8 @@ et_status et_layer(et_handle h, et_dtype dtype, const et_layer_weights* weights,
  *   *_t: the dense kernel as et_transpose_weight leaves it: [out,in] (k-contiguous) in fp16, split rows in fp32 (6 bytes a
  *        value).  The call then skips making that copy itself and does not look at the tensor it was made of; Q, K and V go
  *        together.  fp32 at hidden sizes that run on pair rows (et_gemm_pair): these are made by every call, of the copies where
- *        they are handed over, which takes 2 to 7 us longer than of the [in,out] tensors.  Ignored for hidden sizes whose GEMMs read the [in,out] tensors (no multiple of 64 in fp16, of 32 in fp32).
+ *        they are handed over, which takes 2 to 7 us longer than of the [in,out] tensors.  Ignored for hidden sizes whose
+ *        GEMMs read the [in,out] tensors (no multiple of 64 in fp16, of 32 in fp32).
  *   seq_start, seq_start_bytes: the sequence table et_sequence_starts wrote for THIS batch and the size of its buffer
  *        (at least et_seq_workspace_bytes(batch_size), ET_WORKSPACE_TOO_SMALL below); the same table serves every
  *        layer of the batch.
