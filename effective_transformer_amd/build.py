@@ -3,7 +3,7 @@
     python -m effective_transformer_amd.build            # rebuild everything
     python -m effective_transformer_amd.build --if-missing
 
-The objects and the library stay in-tree (git-ignored) so that a GPU box that receives a
+The objects and the library stay in-tree (git-ignored) so that a machine that receives a
 copy of the tree can load the library without a compiler run.
 """
 from __future__ import annotations
