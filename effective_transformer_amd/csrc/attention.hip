@@ -1054,23 +1054,42 @@ void attention_flash_launch(const void* q, const void* k, const void* v, int lay
 }
 
 // ------------------------------------------------------------------------------------------
-// fp32 fused attention for 32 < seq_len <= 1024, built like the kernel above: one workgroup of 4 wavefronts per (64 queries,
-// head, sequence), 16 queries per wavefront, K and V by DMA in stages of 32 keys (two stages of 16 KB), the softmax along
-// with them, everything in float on v_mfma_f32_16x16x4_f32.  A lane's 16-byte V read is four features of one key, one for
-// each of the four feature tiles (row l16 of tile dt is feature 4 l16 + dt), so V needs no transpose and a lane ends up
-// with 16 consecutive features of its query; K's chunks are XOR-swizzled with the key, which spreads an operand read (16
-// rows x one chunk) over all banks.
-// Bound: the fp32 matrix instructions (a wavefront and stage: 2048 cycles of MFMA, about 400 of VALU, 16 LDS reads) over the
-// rounds of workgroups, long sequences first.  15 x 379 positions / 3820 tokens, 12 heads: 47 us per launch, 104 us with K
-// and V in chunks of 128 keys behind barriers and the scores of a query against all keys in registers.
+// fp32 fused attention for 32 < seq_len <= 1024, built like the kernel above: one workgroup of 4 wavefronts per (64 queries, head,
+// sequence), 16 queries per wavefront, K and V in stages of 32 keys, the softmax along with them in floats.  The products run on
+// the 16-bit matrix instructions with every float as the exact sum of three bfloat16 pieces (round_pair_bf16): six of the nine
+// products of pieces, the others at most 2^-24 of the largest.  A float MFMA takes 16 times as long per product.
+// The pieces of K and V are made once per workgroup: a thread brings eight floats of a key's K and of its V into registers under
+// the stage in front, splits them and writes them to LDS in rows of 64 values per piece, laid out as in the fp16 kernel (which
+// explains the order of the keys).
+// Bound: a wavefront and stage issue 768 cycles of MFMA and about 900 of VALU (352 of them the split of K and V, 180 that of the
+// probabilities, exp2 at a quarter of the rate), 24 KB of LDS reads; short sequences the start of a workgroup.  One stage in LDS
+// and the next in registers take two barriers a stage, but leave room for four workgroups per CU.  15 x 379 positions / 3820
+// tokens, 12 heads: 47.0 -> 32.0 us per launch against floats on v_mfma_f32_16x16x4_f32 (2048 cycles of MFMA a stage), 500 x 64 /
+// 20375 tokens 64.8 -> 53.1.  32 queries per wavefront: 35 and 73 us; three wavefronts per SIMD instead of four: 34 and 60.
+// Relative error against float64 (this / the float instructions), normal operands: 64 positions 1.59e-7 / 2.44e-7, 379 3.01e-7 /
+// 4.00e-7, 1000 5.27e-7 / 6.47e-7; with scores nine times as wide 3.9e-7 / 6.4e-7, 6.2e-7 / 9.9e-7, 7.6e-7 / 1.14e-6.  An infinity
+// gives NaN, as does a magnitude above 3.38e38.
 // ------------------------------------------------------------------------------------------
 constexpr int kF32Keys = 32;                                 // keys per stage
-constexpr int kF32Stage = kF32Keys * kD * 4;                 // bytes of K (and of V) per stage
-// Up to 32 positions attention_kernel is level or ahead (12 layers, 200 x 32: 4.41 ms either way; one layer, 8 x 32: 90.4 and
-// 91.7 us); beyond, this kernel (12 layers: 7 x 50 1.056 -> 1.025 ms, 500 x 64 17.76 -> 17.61 ms, 9 x 101 1.59 -> 1.39 ms,
-// 40 x 128 4.16 -> 3.91 ms; single layer calls with their masks looked at each time, 200 x 64: 8.30 -> 8.18 ms).
+constexpr int kF32Piece = kF32Keys * kD * 2;                 // bytes of a piece of K (and of V) per stage
+// Up to 32 positions attention_kernel is ahead where there are many sequences, because its workgroups serve several heads for one
+// start (per launch, 12 heads, this kernel second: 1000 x 16 32.2 and 51.3 us, 1000 x 31 52.9 and 66.3, 100 x 20 9.3 and 9.4, 200 x 32
+// 19.1 and 17.0, 8 x 32 5.8 and 5.1).
 constexpr int kF32MinKeys = 32;
-constexpr int kF32Smem = 2 * 2 * kF32Stage + kFlMaxKeys * (int)sizeof(int);
+constexpr int kF32Smem = 2 * 3 * kF32Piece + kFlMaxKeys * (int)sizeof(int);
+typedef __bf16 bf16x8 __attribute__((ext_vector_type(8)));
+// eight floats as three pieces; x keeps the rests
+__device__ __forceinline__ void split_eight(float (&x)[8], uint4x (&piece)[3]) {
+#pragma unroll
+  for (int i = 0; i < 3; ++i)
+#pragma unroll
+    for (int j = 0; j < 4; ++j) piece[i][j] = round_pair_bf16(x[2 * j], x[2 * j + 1]);
+}
+// a . b of three pieces each, smallest products first
+template <typename F>
+__device__ __forceinline__ void piece_products(F&& mfma) {
+  mfma(1, 1); mfma(0, 2); mfma(2, 0); mfma(0, 1); mfma(1, 0); mfma(0, 0);
+}
 
 __global__ __launch_bounds__(kAttnThreads, 4) void attention_flash_f32_kernel(
     const int32_t* __restrict__ seq_start, int batch, int heads, int q_blocks, int seq_len, int layout, int packed_ld,
@@ -1079,8 +1098,8 @@ __global__ __launch_bounds__(kAttnThreads, 4) void attention_flash_f32_kernel(
     float* __restrict__ dst, float scaler, int split_out) {
 #if defined(__HIP_DEVICE_COMPILE__)   // device-only types in the body; the host pass only needs the stub
   extern __shared__ __attribute__((aligned(1024))) unsigned char smem_raw[];
-  unsigned char* kv = smem_raw;                                        // [stage][K, V]
-  int* tok_of_pos = reinterpret_cast<int*>(smem_raw + 2 * 2 * kF32Stage);
+  unsigned char* kv = smem_raw;                                        // [K, V][piece][key][64]
+  int* tok_of_pos = reinterpret_cast<int*>(smem_raw + 2 * 3 * kF32Piece);
 
   // the query blocks of one (head, sequence) go to one XCD, as above
   const int xcd = blockIdx.x & 7, slot_id = blockIdx.x >> 3;
@@ -1101,53 +1120,58 @@ __global__ __launch_bounds__(kAttnThreads, 4) void attention_flash_f32_kernel(
   const float *kb = k_src + first, *vb = v_src + first, *qb = q_src + first;
   const uint32_t ld = layout == 1 ? (uint32_t)packed_ld : (uint32_t)kD;
 
-  // DMA: one instruction fills four rows of 256 bytes (lane -> row lane / 16, 16-byte chunk l16, K's swizzled); a
-  // wavefront's share of a stage is eight keys of K and of V
-  uint32_t voff_k[2], voff_v[2];
-  int dma_key[2];
-#pragma unroll
-  for (int i = 0; i < 2; ++i) {
-    dma_key[i] = (wave * 2 + i) * 4 + g;
-    voff_k[i] = ((uint32_t)dma_key[i] * ld + (uint32_t)(l16 ^ (dma_key[i] & 15)) * 4u) * 4u;
-    voff_v[i] = ((uint32_t)dma_key[i] * ld + (uint32_t)l16 * 4u) * 4u;
-  }
-  auto issue = [&](int slot, int st, bool dense, int rows) {
-    unsigned char* base = kv + slot * 2 * kF32Stage;
+  // this thread's eight features of K and of V: key `my_key` of the stage; a row without a token is requested beyond the
+  // descriptor's range and arrives as zeros
+  const int my_key = threadIdx.x >> 3, my_chunk = threadIdx.x & 7;
+  const uint32_t voff = ((uint32_t)my_key * ld + (uint32_t)my_chunk * 8u) * 4u;
+  float4v in[4];                                                       // K, V
+  auto request = [&](int st, bool dense, int rows) {
     const int bytes = (int)(((uint32_t)(rows - 1) * ld + kD) * 4u);
     const __amdgpu_buffer_rsrc_t rk = __builtin_amdgcn_make_buffer_rsrc(const_cast<float*>(kb), 0, bytes, 0x00020000);
     const __amdgpu_buffer_rsrc_t rv = __builtin_amdgcn_make_buffer_rsrc(const_cast<float*>(vb), 0, bytes, 0x00020000);
+    uint32_t off = voff, stage_off = (uint32_t)st * kF32Keys * ld * 4u;
+    if (!dense) {                                                      // the row of the key, or nowhere
+      const int key = st * kF32Keys + my_key;
+      const int tk = key < kFlMaxKeys ? tok_of_pos[key] : -1;
+      const uint32_t row = layout == 1 ? (uint32_t)tk : (uint32_t)key;
+      off = tk >= 0 ? off + (row - (uint32_t)my_key) * ld * 4u : 0x80000000u;
+      stage_off = 0;
+    }
 #pragma unroll
     for (int i = 0; i < 2; ++i) {
-      uint32_t off_k = voff_k[i], off_v = voff_v[i];
-      uint32_t stage_off = (uint32_t)st * kF32Keys * ld * 4u;
-      if (!dense) {                                                    // the row of the key, or nowhere
-        const int key = st * kF32Keys + dma_key[i];
-        const int tk = key < kFlMaxKeys ? tok_of_pos[key] : -1;
-        const uint32_t row = layout == 1 ? (uint32_t)tk : (uint32_t)key;
-        const uint32_t by = (row - (uint32_t)dma_key[i]) * ld * 4u;
-        off_k = tk >= 0 ? off_k + by : 0x80000000u;
-        off_v = tk >= 0 ? off_v + by : 0x80000000u;
-        stage_off = 0;
-      }
-      __builtin_amdgcn_raw_ptr_buffer_load_lds(rk, ET_ATTN_LDS_PTR(base + (wave * 2 + i) * 1024), 16, off_k, stage_off, 0, 0);
-      __builtin_amdgcn_raw_ptr_buffer_load_lds(rv, ET_ATTN_LDS_PTR(base + kF32Stage + (wave * 2 + i) * 1024), 16, off_v, stage_off, 0, 0);
+      in[i] = __builtin_bit_cast(float4v, __builtin_amdgcn_raw_buffer_load_b128(rk, off + 16u * i, stage_off, 0));
+      in[2 + i] = __builtin_bit_cast(float4v, __builtin_amdgcn_raw_buffer_load_b128(rv, off + 16u * i, stage_off, 0));
+    }
+  };
+  unsigned char* const k_wr = kv + wide_slot(my_key) * 128 + ((my_chunk ^ wide_swizzle(wide_slot(my_key))) * 16);
+  unsigned char* const v_wr = kv + 3 * kF32Piece + my_key * 128 + ((my_chunk ^ v_swizzle(my_key)) * 16);
+  auto write = [&] {
+#pragma unroll
+    for (int m = 0; m < 2; ++m) {
+      float x[8];
+#pragma unroll
+      for (int j = 0; j < 8; ++j) x[j] = in[2 * m + (j >> 2)][j & 3];
+      uint4x piece[3];
+      split_eight(x, piece);
+#pragma unroll
+      for (int i = 0; i < 3; ++i) *reinterpret_cast<uint4x*>((m ? v_wr : k_wr) + i * kF32Piece) = piece[i];
     }
   };
   int tq;
-  float4v bq[4];                                                       // features 16 g .. 16 g + 15 of the lane's query
-  auto load_q = [&](bool dense, int n) {
+  float4v q_in[4];                                                     // features 8 g .. and 32 + 8 g .. of the lane's query
+  auto request_q = [&](bool dense, int n) {
     tq = q < n ? (dense ? q : tok_of_pos[q]) : -1;
 #pragma unroll
     for (int i = 0; i < 4; ++i) {
-      bq[i] = float4v{0.f, 0.f, 0.f, 0.f};
-      if (tq >= 0) bq[i] = *reinterpret_cast<const float4v*>(qb + (size_t)(layout == 1 ? tq : q) * ld + g * 16 + i * 4);
+      q_in[i] = float4v{0.f, 0.f, 0.f, 0.f};
+      if (tq >= 0) q_in[i] = *reinterpret_cast<const float4v*>(qb + (size_t)(layout == 1 ? tq : q) * ld + (i >> 1) * 32 + g * 8 + (i & 1) * 4);
     }
   };
 
   // without a hole in the sequence position p holds token p: requested on that assumption beside what decides it
   if (first_q < len) {
-    issue(0, 0, true, len);
-    load_q(true, len);
+    request(0, true, len);
+    request_q(true, len);
   }
   const int n = min(max(word_idx[t1 - 1], 0), seq_len - 1) + 1;        // positions up to the last token
   const int cblocks = (seq_len + 15) / 16;
@@ -1162,12 +1186,11 @@ __global__ __launch_bounds__(kAttnThreads, 4) void attention_flash_f32_kernel(
     ones_behind = (uint32_t)__ballot(cl & kMaskOnes);
   }
   const bool dense = n == len;
-  const bool active = first_q + wave * 16 < n;                         // wave-uniform
+  const bool active = first_q + wave * 16 < n;                                          // wave-uniform
   const int stages = (n + kF32Keys - 1) / kF32Keys;
+  const int stage_rows = dense || layout == 1 ? len : n;               // of the matrices behind kb, vb that exist
+  if (first_q >= n) return;                                            // no token among this workgroup's queries
   if (!dense) {
-    wide_wait_dma();
-    __syncthreads();
-    if (first_q >= n) return;                                          // no token among this workgroup's queries
     for (int i = threadIdx.x; i < kFlMaxKeys; i += kAttnThreads) tok_of_pos[i] = -1;
     __syncthreads();
     for (int tt = threadIdx.x; tt < len; tt += kAttnThreads) {
@@ -1175,20 +1198,40 @@ __global__ __launch_bounds__(kAttnThreads, 4) void attention_flash_f32_kernel(
       if (pos >= 0 && pos < seq_len) tok_of_pos[pos] = tt;             // relative to the sequence's first packed row
     }
     __syncthreads();
-    issue(0, 0, false, layout == 1 ? len : n);
-    load_q(false, n);
-  } else if (first_q >= n) {
-    return;                                                            // (nothing has been requested)
+    request(0, false, stage_rows);
+    request_q(false, n);
   }
-  // (the queries are waited for here and not in the stage loop, where the wait would cover the DMA)
+  bf16x8 bq[2][3];
 #pragma unroll
-  for (int i = 0; i < 4; ++i) asm volatile("" : "+v"(bq[i]));
+  for (int ks = 0; ks < 2; ++ks) {
+    float x[8];
+#pragma unroll
+    for (int j = 0; j < 8; ++j) x[j] = q_in[2 * ks + (j >> 2)][j & 3];
+    uint4x piece[3];
+    split_eight(x, piece);
+#pragma unroll
+    for (int i = 0; i < 3; ++i) bq[ks][i] = __builtin_bit_cast(bf16x8, piece[i]);
+  }
+
+  // operand addresses, as in the fp16 kernel
+  int k_rd[2], v_rd[4];
+  {
+    const int L = wide_slot((l16 >> 2) * 8 + (l16 & 3));
+    const int sw = wide_swizzle(L);
+#pragma unroll
+    for (int ks = 0; ks < 2; ++ks) k_rd[ks] = L * 128 + (((ks * 4 + g) ^ sw) * 16);
+    const int key = g * 8 + (l16 >> 2);
+#pragma unroll
+    for (int dt = 0; dt < 4; ++dt)
+      v_rd[dt] = 3 * kF32Piece + key * 128 + (((dt * 2 + ((l16 >> 1) & 1)) ^ v_swizzle(key)) * 16) + (l16 & 1) * 8;
+  }
 
   float ref = kFlLowest, top = -INFINITY, l = 0.f;                     // as above; l: of this lane's keys
   float4v o[4];
 #pragma unroll
   for (int dt = 0; dt < 4; ++dt) o[dt] = float4v{0.f, 0.f, 0.f, 0.f};
   const float c_exp = scaler * kLog2e;
+
   const float* mrow = attr_mask + ((size_t)b * seq_len + min(q, seq_len - 1)) * seq_len;
 
   auto load_mask = [&](int k0) -> float4v {                            // of keys k0 .. k0 + 3, 0 beyond the row
@@ -1212,72 +1255,83 @@ __global__ __launch_bounds__(kAttnThreads, 4) void attention_flash_f32_kernel(
     for (int dt = 0; dt < 4; ++dt) o[dt] *= alpha;
   };
 
-  auto stage = [&](auto PLAINc, int st, int slot) {
+  auto stage = [&](auto PLAINc, int st) {
     constexpr bool PLAIN = decltype(PLAINc)::value;
-    const unsigned char* base = kv + slot * 2 * kF32Stage;
-    float s[2][4];                                                     // keys 32 st + 16 kt + 4 g + r
+    float4v acc[2];                                                    // keys 32 st + 8 g + 4 t + r
 #pragma unroll
-    for (int kt = 0; kt < 2; ++kt) {
-      float4v acc = {0.f, 0.f, 0.f, 0.f};
+    for (int t = 0; t < 2; ++t) acc[t] = float4v{0.f, 0.f, 0.f, 0.f};
 #pragma unroll
-      for (int i = 0; i < 4; ++i) {
-        const float4v a = *reinterpret_cast<const float4v*>(base + (kt * 16 + l16) * 256 + (((g * 4 + i) ^ l16) * 16));
+    for (int ks = 0; ks < 2; ++ks) {
+      bf16x8 a[2][3];
 #pragma unroll
-        for (int j = 0; j < 4; ++j) acc = __builtin_amdgcn_mfma_f32_16x16x4f32(a[j], bq[i][j], acc, 0, 0, 0);
-      }
+      for (int t = 0; t < 2; ++t)
 #pragma unroll
-      for (int r = 0; r < 4; ++r) s[kt][r] = acc[r];
+        for (int i = 0; i < 3; ++i) a[t][i] = *reinterpret_cast<const bf16x8*>(kv + k_rd[ks] + i * kF32Piece + t * 4 * 128);
+      piece_products([&](int i, int j) {
+#pragma unroll
+        for (int t = 0; t < 2; ++t) acc[t] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a[t][i], bq[ks][j], acc[t], 0, 0, 0);
+      });
+      __builtin_amdgcn_sched_barrier(0);         // (six operands at a time, for their registers)
     }
+    float s[8];                                                        // keys key0 .. key0 + 7
+#pragma unroll
+    for (int j = 0; j < 8; ++j) s[j] = acc[j >> 2][j & 3];
     // the exponents' factor: log2 units of the plain scores, of the masked ones otherwise
     const float unit = PLAIN ? c_exp : kLog2e;
-    const int key0 = st * kF32Keys + g * 4;
+    const int key0 = st * kF32Keys + g * 8;
     float mx = -INFINITY;
     if constexpr (PLAIN) {
       if ((st + 1) * kF32Keys > n) {                                   // workgroup-uniform: the last, partial stage
 #pragma unroll
-        for (int kt = 0; kt < 2; ++kt)
-#pragma unroll
-          for (int r = 0; r < 4; ++r)
-            if (key0 + kt * 16 + r >= n) s[kt][r] = -INFINITY;
+        for (int j = 0; j < 8; ++j)
+          if (key0 + j >= n) s[j] = -INFINITY;
       }
     } else {
 #pragma unroll
-      for (int kt = 0; kt < 2; ++kt) {
-        const int k0 = key0 + kt * 16;
+      for (int t = 0; t < 2; ++t) {
+        const int k0 = key0 + t * 4;
         const float4v m4 = load_mask(k0);
 #pragma unroll
-        for (int r = 0; r < 4; ++r) s[kt][r] = k0 + r < seq_len ? s[kt][r] * scaler + (1.0f - m4[r]) * -10000.0f : -INFINITY;
+        for (int r = 0; r < 4; ++r) s[t * 4 + r] = k0 + r < seq_len ? s[t * 4 + r] * scaler + (1.0f - m4[r]) * -10000.0f : -INFINITY;
       }
     }
 #pragma unroll
-    for (int kt = 0; kt < 2; ++kt)
-#pragma unroll
-      for (int r = 0; r < 4; ++r) mx = fmaxf(mx, s[kt][r]);
+    for (int j = 0; j < 8; ++j) mx = fmaxf(mx, s[j]);
     mx *= unit;
     top = fmaxf(top, mx);
     if (__any(mx > ref + kFlSlack)) move_ref(mx);                      // the first stage, and seldom after it
 #pragma unroll
-    for (int kt = 0; kt < 2; ++kt)
+    for (int j = 0; j < 8; ++j) {
+      s[j] = __builtin_amdgcn_exp2f(__builtin_fmaf(s[j], unit, -ref));
+      l += s[j];
+    }
+    uint4x p[3];
+    split_eight(s, p);
 #pragma unroll
-      for (int r = 0; r < 4; ++r) {
-        s[kt][r] = __builtin_amdgcn_exp2f(__builtin_fmaf(s[kt][r], unit, -ref));
-        l += s[kt][r];
+    for (int dt = 0; dt < 4; ++dt) {
+      bf16x8 v[3];
+#pragma unroll
+      for (int i = 0; i < 3; ++i) {
+        const half4 lo = read_transposed(kv + v_rd[dt] + i * kF32Piece), hi = read_transposed(kv + v_rd[dt] + i * kF32Piece + 4 * 128);
+        v[i] = __builtin_bit_cast(bf16x8, __builtin_shufflevector(lo, hi, 0, 1, 2, 3, 4, 5, 6, 7));
       }
-#pragma unroll
-    for (int kt = 0; kt < 2; ++kt)
-#pragma unroll
-      for (int r = 0; r < 4; ++r) {
-        const float4v v = *reinterpret_cast<const float4v*>(base + kF32Stage + (kt * 16 + g * 4 + r) * 256 + l16 * 16);
-#pragma unroll
-        for (int dt = 0; dt < 4; ++dt) o[dt] = __builtin_amdgcn_mfma_f32_16x16x4f32(v[dt], s[kt][r], o[dt], 0, 0, 0);
-      }
+      piece_products([&](int i, int j) {
+        o[dt] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(v[i], __builtin_bit_cast(bf16x8, p[j]), o[dt], 0, 0, 0);
+      });
+    }
+  };
+  // this wavefront's LDS reads and writes are complete, and everybody's; requests may be on their way
+  auto lds_barrier = [] {
+    __builtin_amdgcn_s_waitcnt(15 | (7 << 4) | (0 << 8) | (3 << 14));
+    wide_barrier();
   };
   auto run = [&](auto PLAINc) {
     for (int st = 0; st < stages; ++st) {
-      wide_wait_dma();                                                 // this wavefront's share of the stage has landed,
-      wide_barrier();                                                  // everybody's has, and the other slot is free
-      if (st + 1 < stages) issue((st + 1) & 1, st + 1, dense, layout == 1 ? len : n);
-      if (active) stage(PLAINc, st, st & 1);
+      if (st > 0) lds_barrier();                                       // everybody has read the stage in front of this one
+      write();
+      lds_barrier();
+      if (st + 1 < stages) request(st + 1, dense, stage_rows);
+      if (active) stage(PLAINc, st);
     }
   };
   if (__builtin_expect(plain, 1)) run(std::true_type{});
@@ -1327,11 +1381,11 @@ __global__ __launch_bounds__(kAttnThreads, 4) void attention_flash_f32_kernel(
   const float sum = xor_lanes_16_32_sum(l) + unseen.extra;
   if (tq < 0) return;
   const float inv = 1.0f / (sum + 1e-6f * __builtin_amdgcn_exp2f(mx - ref));
-  // o[dt][r] is feature 16 g + 4 r + dt
+  // o[dt][r] is feature 16 dt + 4 g + r
 #pragma unroll
-  for (int r = 0; r < 4; ++r) {
-    const float4v v = {o[0][r] * inv, o[1][r] * inv, o[2][r] * inv, o[3][r] * inv};
-    const int col = head * kD + g * 16 + r * 4;
+  for (int dt = 0; dt < 4; ++dt) {
+    const float4v v = o[dt] * inv;
+    const int col = head * kD + dt * 16 + g * 4;
     if (split_out) store_split<4>(reinterpret_cast<uint16_t*>(dst) + (size_t)(t0 + tq) * 3 * H, col, v);
     else *reinterpret_cast<float4v*>(dst + (size_t)(t0 + tq) * H + col) = v;
   }
