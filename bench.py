@@ -203,10 +203,6 @@ def per_kernel(wl, T, mask_np, iters=20, vendor_gemm=False):
     a = rnd(T, H); r = rnd(T, H); bias = rnd(H); gam = rnd(H); bet = rnd(H)
     ms = _time_kernel(lambda: k.add_bias_input_layernorm(a, r, bias, gam, bet), iters)
     add("bias_residual_layernorm", ms, "hbm", 3 * T * H * e + 3 * H * e)
-    if dt == torch.float32:                   # between attention and its output product (see in_layer_kernels)
-        paired = k.PairRows(T, H, "cuda")
-        ms = _time_kernel(lambda: k.pair_rows(a, out=paired), iters)
-        add("pair_rows", ms, "hbm", 2 * T * H * e + 8 * T)
     inter = rnd(T, F) * 0.1; bF = rnd(F)
     ms = _time_kernel(lambda: k.add_bias_act(inter, bF), iters)
     add("bias_gelu", ms, "hbm", 2 * T * F * e + F * e)
@@ -298,9 +294,8 @@ def in_layer_kernels(wl, T, mask_np, reps=4):
     bias = {n: rnd(w.shape[1]) * 0.02 for n, w in weights.items()}
     gam, bet = torch.ones(H, device="cuda", dtype=dt), torch.zeros(H, device="cuda", dtype=dt)
     mm = {}
-    # fp32 products read pair rows.  Those of the context are made by a launch of the layer's, those of the input and of
-    # LayerNorm's rows by the launches that write these: here by calls of their own between the timed launches (so LayerNorm
-    # is timed without them)
+    # fp32 products read pair rows, which the launches in front of them write in the layer: here calls of their own make them
+    # between the timed launches (so attention and LayerNorm are timed without them)
     pairs = dt == torch.float32
     stats = None
     for n, w in weights.items():          # the kernel the encoder object runs this projection on
@@ -321,7 +316,7 @@ def in_layer_kernels(wl, T, mask_np, reps=4):
     inter = k.PairRows(T, F, "cuda") if pairs else torch.empty(T, F, device="cuda", dtype=dt)
     rows = k.PairRows(T, H, "cuda") if pairs else None
     names = ("gemm_qkv", "attention", "gemm_attn_out", "bias_residual_layernorm", "gemm_ffn_up", "gemm_ffn_down",
-             "bias_residual_layernorm") + (("pair_rows",) if pairs else ())
+             "bias_residual_layernorm")
     starts = ops.sequence_starts(vwn, bidx, B, S)          # one table per batch, as the encoder builds it
 
     def layer(marks):
@@ -335,7 +330,7 @@ def in_layer_kernels(wl, T, mask_np, reps=4):
         def product(n, a, **kw):
             if pairs and a is not inter:
                 a = k.pair_rows(a, out=rows)
-                mark("pair_rows" if n == "gemm_attn_out" else None)
+                mark(None)
             if pairs and kw.get("gelu"):
                 kw["stats"] = stats
             f, w = mm[n]

@@ -220,6 +220,33 @@ __device__ __forceinline__ float xor_lanes_16_32_sum(float v) {
   return a + b;
 }
 
+// The lane's 16 values of row `row` (-1: none) and head `head`, o[dt][r] = feature 16 dt + 4 g + r (RUN: 16 g + 4 dt + r), as pairs under
+// the exponent of the head's largest value.  Whole wavefronts; the four lanes of a query have the same row.
+template <bool RUN>
+__device__ __forceinline__ void store_head_pairs(float* dst, int row, int H, int head, const float4v (&o)[4], HeadExps head_exp) {
+#if defined(__HIP_DEVICE_COMPILE__)
+  const int g = (threadIdx.x & (kWave - 1)) >> 4;
+  float top = 0.f;
+#pragma unroll
+  for (int dt = 0; dt < 4; ++dt)
+#pragma unroll
+    for (int r = 0; r < 4; ++r) top = fmaxf(top, fabsf(o[dt][r]));
+  const int e = pair_exponent(xor_lanes_16_32_max(top));
+  if (row < 0) return;
+  const float scale = pair_scale(e);
+  _Float16* out = reinterpret_cast<_Float16*>(dst) + (size_t)row * 2 * H;
+  if constexpr (RUN) {
+#pragma unroll
+    for (int half = 0; half < 2; ++half)
+      store_pair<8>(out, head * kD + g * 16 + half * 8, __builtin_shufflevector(o[2 * half], o[2 * half + 1], 0, 1, 2, 3, 4, 5, 6, 7), scale);
+  } else {
+#pragma unroll
+    for (int dt = 0; dt < 4; ++dt) store_pair<4>(out, head * kD + dt * 16 + g * 4, o[dt], scale);
+  }
+  if (g == 0) head_exp.exp[(size_t)head * head_exp.stride + row] = (int8_t)e;
+#endif
+}
+
 // WAVES: wavefronts per workgroup, one 16-query tile each.  CPT = 16-byte chunks of
 // one matrix a thread moves per head (ceil(seq rows * chunks per row / threads)).
 template <typename T, int NKT, int WAVES, int CPT>
@@ -227,7 +254,7 @@ __global__ __launch_bounds__(WAVES * kWave) void attention_kernel(
     // (the first 14 words come in registers: what the chain order -> start table -> positions and rows needs)
     const int32_t* __restrict__ seq_start, const int32_t* __restrict__ word_idx, int batch, int seq_len, int heads, int heads_per_wg,
     int layout, int packed_ld, const T* __restrict__ q_src, const T* __restrict__ k_src, const T* __restrict__ v_src,
-    const T* __restrict__ attr_mask, T* __restrict__ dst, float scaler, int split_out) {
+    const T* __restrict__ attr_mask, T* __restrict__ dst, float scaler, AttentionOut out, HeadExps head_exp) {
   using Cfg = AttnCfg<T>;
   using Sm = AttnSmem<T, NKT>;
   using C = Chunk16<T>;
@@ -351,7 +378,7 @@ __global__ __launch_bounds__(WAVES * kWave) void attention_kernel(
   // where this lane's query writes its output row (head 0; null without a token): the same for every head
   const int tq = wave < n_tiles && wave < NKT ? tok_of_pos[wave * 16 + l16] : -1;
   T* out_row = tq >= 0 ? dst + (size_t)tq * H + g * (sizeof(T) == 2 ? 16 : 4) : nullptr;
-  if (sizeof(T) == 4 && split_out && tq >= 0)
+  if (sizeof(T) == 4 && out == AttentionOut::kSplit && tq >= 0)
     out_row = reinterpret_cast<T*>(reinterpret_cast<uint16_t*>(dst) + (size_t)tq * 3 * H);
 
   for (int head = h_begin; head < h_end; ++head) {
@@ -495,6 +522,12 @@ __global__ __launch_bounds__(WAVES * kWave) void attention_kernel(
           }
         }
       }
+      if constexpr (sizeof(T) == 4) {
+        if (out == AttentionOut::kPairs) {       // (uniform)
+          store_head_pairs<false>(dst, tq, H, head, o, head_exp);
+          continue;
+        }
+      }
       // ---- write the lane's 16 features of its query's packed row --------------------------
       if (out_row != nullptr) {
         if constexpr (sizeof(T) == 2) {
@@ -518,7 +551,7 @@ __global__ __launch_bounds__(WAVES * kWave) void attention_kernel(
             out4 v;
 #pragma unroll
             for (int r = 0; r < 4; ++r) v[r] = (T)o[dt][r];
-            if (split_out) store_split<4>(reinterpret_cast<uint16_t*>(out_row), head * kD + dt * 16 + g * 4, v);
+            if (out == AttentionOut::kSplit) store_split<4>(reinterpret_cast<uint16_t*>(out_row), head * kD + dt * 16 + g * 4, v);
             else *reinterpret_cast<out4*>(orow + dt * 16) = v;
           }
         }
@@ -532,7 +565,7 @@ __global__ __launch_bounds__(WAVES * kWave) void attention_kernel(
 template <typename T, int NKT>
 void attention_launch(const void* q, const void* k, const void* v, int layout, int packed_ld, const void* attr_mask,
                       void* dst, const int32_t* seq_start, const int32_t* word_idx, int batch, int seq_len, int heads,
-                      float scaler, bool split_out, hipStream_t stream) {
+                      float scaler, AttentionOut out, HeadExps head_exp, hipStream_t stream) {
   using Sm = AttnSmem<T, NKT>;
   constexpr int kCpr = kD * (int)sizeof(T) / 16;
   constexpr int WAVES = 4;
@@ -553,7 +586,7 @@ void attention_launch(const void* q, const void* k, const void* v, int layout, i
     }
   dim3 grid((heads + hpw - 1) / hpw, batch);
   kern<<<grid, kThreads, Sm::kBytes, stream>>>(seq_start, word_idx, batch, seq_len, heads, hpw, layout, packed_ld, (const T*)q,
-                                               (const T*)k, (const T*)v, (const T*)attr_mask, (T*)dst, scaler, split_out ? 1 : 0);
+                                               (const T*)k, (const T*)v, (const T*)attr_mask, (T*)dst, scaler, out, head_exp);
 }
 
 
@@ -1065,7 +1098,7 @@ void attention_flash_launch(const void* q, const void* k, const void* v, int lay
 // probabilities, exp2 at a quarter of the rate), 24 KB of LDS reads; short sequences the start of a workgroup.  One stage in LDS
 // and the next in registers take two barriers a stage, but leave room for four workgroups per CU.  15 x 379 positions / 3820
 // tokens, 12 heads: 47.0 -> 32.0 us per launch against floats on v_mfma_f32_16x16x4_f32 (2048 cycles of MFMA a stage), 500 x 64 /
-// 20375 tokens 64.8 -> 53.1.  32 queries per wavefront: 35 and 73 us; three wavefronts per SIMD instead of four: 34 and 60.
+// 20375 tokens 64.8 -> 53.1 (33.1 and 59.8 where the result is left as pair rows).  32 queries per wavefront: 35 and 73 us; three wavefronts per SIMD instead of four: 34 and 60.
 // Relative error against float64 (this / the float instructions), normal operands: 64 positions 1.59e-7 / 2.44e-7, 379 3.01e-7 /
 // 4.00e-7, 1000 5.27e-7 / 6.47e-7; with scores nine times as wide 3.9e-7 / 6.4e-7, 6.2e-7 / 9.9e-7, 7.6e-7 / 1.14e-6.  An infinity
 // gives NaN, as does a magnitude above 3.38e38.
@@ -1095,7 +1128,7 @@ __global__ __launch_bounds__(kAttnThreads, 4) void attention_flash_f32_kernel(
     const int32_t* __restrict__ seq_start, int batch, int heads, int q_blocks, int seq_len, int layout, int packed_ld,
     const float* __restrict__ q_src, const float* __restrict__ k_src, const float* __restrict__ v_src,
     const int32_t* __restrict__ word_idx, const float* __restrict__ attr_mask, const uint8_t* __restrict__ mask_class,
-    float* __restrict__ dst, float scaler, int split_out) {
+    float* __restrict__ dst, float scaler, AttentionOut out, HeadExps head_exp) {
 #if defined(__HIP_DEVICE_COMPILE__)   // device-only types in the body; the host pass only needs the stub
   extern __shared__ __attribute__((aligned(1024))) unsigned char smem_raw[];
   unsigned char* kv = smem_raw;                                        // [K, V][piece][key][64]
@@ -1124,6 +1157,7 @@ __global__ __launch_bounds__(kAttnThreads, 4) void attention_flash_f32_kernel(
   // descriptor's range and arrives as zeros
   const int my_key = threadIdx.x >> 3, my_chunk = threadIdx.x & 7;
   const uint32_t voff = ((uint32_t)my_key * ld + (uint32_t)my_chunk * 8u) * 4u;
+  const uint32_t v_swap = (uint32_t)(my_key >> 1 & 1) * 16u;           // (see v_wr)
   float4v in[4];                                                       // K, V
   auto request = [&](int st, bool dense, int rows) {
     const int bytes = (int)(((uint32_t)(rows - 1) * ld + kD) * 4u);
@@ -1140,11 +1174,13 @@ __global__ __launch_bounds__(kAttnThreads, 4) void attention_flash_f32_kernel(
 #pragma unroll
     for (int i = 0; i < 2; ++i) {
       in[i] = __builtin_bit_cast(float4v, __builtin_amdgcn_raw_buffer_load_b128(rk, off + 16u * i, stage_off, 0));
-      in[2 + i] = __builtin_bit_cast(float4v, __builtin_amdgcn_raw_buffer_load_b128(rv, off + 16u * i, stage_off, 0));
+      in[2 + i] = __builtin_bit_cast(float4v, __builtin_amdgcn_raw_buffer_load_b128(rv, off + (16u * i ^ v_swap), stage_off, 0));
     }
   };
   unsigned char* const k_wr = kv + wide_slot(my_key) * 128 + ((my_chunk ^ wide_swizzle(wide_slot(my_key))) * 16);
-  unsigned char* const v_wr = kv + 3 * kF32Piece + my_key * 128 + ((my_chunk ^ v_swizzle(my_key)) * 16);
+  // V is read transposed, four keys x four times four features 16 apart, so that a lane ends up with 16 consecutive features: chunks
+  // are XORed with key bit 3, and key bit 1 swaps a chunk's halves (requested the other way round), which spreads a read over all banks
+  unsigned char* const v_wr = kv + 3 * kF32Piece + my_key * 128 + ((my_chunk ^ (my_key >> 3 & 1)) * 16);
   auto write = [&] {
 #pragma unroll
     for (int m = 0; m < 2; ++m) {
@@ -1223,7 +1259,7 @@ __global__ __launch_bounds__(kAttnThreads, 4) void attention_flash_f32_kernel(
     const int key = g * 8 + (l16 >> 2);
 #pragma unroll
     for (int dt = 0; dt < 4; ++dt)
-      v_rd[dt] = 3 * kF32Piece + key * 128 + (((dt * 2 + ((l16 >> 1) & 1)) ^ v_swizzle(key)) * 16) + (l16 & 1) * 8;
+      v_rd[dt] = 3 * kF32Piece + key * 128 + ((((l16 & 3) * 2 + (dt >> 1)) ^ (key >> 3 & 1)) * 16) + (((dt & 1) ^ (key >> 1 & 1)) * 8);
   }
 
   float ref = kFlLowest, top = -INFINITY, l = 0.f;                     // as above; l: of this lane's keys
@@ -1379,27 +1415,33 @@ __global__ __launch_bounds__(kAttnThreads, 4) void attention_flash_f32_kernel(
 
   const float mx = fmaxf(xor_lanes_16_32_max(top), unseen.lowest);
   const float sum = xor_lanes_16_32_sum(l) + unseen.extra;
-  if (tq < 0) return;
   const float inv = 1.0f / (sum + 1e-6f * __builtin_amdgcn_exp2f(mx - ref));
-  // o[dt][r] is feature 16 dt + 4 g + r
+  // o[dt][r] is feature 16 g + 4 dt + r
+#pragma unroll
+  for (int dt = 0; dt < 4; ++dt) o[dt] *= inv;
+  if (out == AttentionOut::kPairs) {
+    store_head_pairs<true>(dst, tq < 0 ? -1 : t0 + tq, H, head, o, head_exp);
+    return;
+  }
+  if (tq < 0) return;
 #pragma unroll
   for (int dt = 0; dt < 4; ++dt) {
-    const float4v v = o[dt] * inv;
-    const int col = head * kD + dt * 16 + g * 4;
-    if (split_out) store_split<4>(reinterpret_cast<uint16_t*>(dst) + (size_t)(t0 + tq) * 3 * H, col, v);
-    else *reinterpret_cast<float4v*>(dst + (size_t)(t0 + tq) * H + col) = v;
+    const int col = head * kD + g * 16 + dt * 4;
+    if (out == AttentionOut::kSplit) store_split<4>(reinterpret_cast<uint16_t*>(dst) + (size_t)(t0 + tq) * 3 * H, col, o[dt]);
+    else *reinterpret_cast<float4v*>(dst + (size_t)(t0 + tq) * H + col) = o[dt];
   }
 #endif
 }
 
 void attention_flash_f32_launch(const void* q, const void* k, const void* v, int layout, int packed_ld, const void* attr_mask,
                                 const uint8_t* mask_class, void* dst, const int32_t* seq_start, const int32_t* word_idx,
-                                int batch, int seq_len, int heads, float scaler, bool split_out, hipStream_t stream) {
+                                int batch, int seq_len, int heads, float scaler, AttentionOut out, HeadExps head_exp,
+                                hipStream_t stream) {
   const int q_blocks = (seq_len + 63) / 64;
   const int grid = (batch * heads + 7) / 8 * 8 * q_blocks;
   attention_flash_f32_kernel<<<grid, kAttnThreads, kF32Smem, stream>>>(
       seq_start, batch, heads, q_blocks, seq_len, layout, packed_ld, (const float*)q, (const float*)k, (const float*)v, word_idx,
-      (const float*)attr_mask, mask_class, (float*)dst, scaler, split_out ? 1 : 0);
+      (const float*)attr_mask, mask_class, (float*)dst, scaler, out, head_exp);
 }
 
 // ------------------------------------------------------------------------------------------
@@ -1544,7 +1586,7 @@ void attention_generic_launch(const void* q, const void* k, const void* v, int l
 template <typename T>
 void attention_dispatch(const void* q, const void* k, const void* v, int layout, int packed_ld, const void* attr_mask,
                         void* dst, const int32_t* seq_start, const int32_t* word_idx, int batch, int seq_len, int heads,
-                        int d, float scaler, bool split_out, const uint8_t* mask_class, hipStream_t stream) {
+                        int d, float scaler, AttentionOut out, const uint8_t* mask_class, HeadExps head_exp, hipStream_t stream) {
   // (the streaming kernels address the rows of a sequence with 31 bits)
   const bool far = (uint64_t)seq_len * (uint64_t)(layout == 1 ? packed_ld : kD) * sizeof(T) >= 0x80000000ull;
   if (d != kD || !head_rows_16b<T>(q, k, v, layout, packed_ld, d) || (far && seq_len > kF32MinKeys))
@@ -1555,13 +1597,13 @@ void attention_dispatch(const void* q, const void* k, const void* v, int layout,
                            scaler, stream);
   else if (sizeof(T) == 4 && seq_len > kF32MinKeys)
     attention_flash_f32_launch(q, k, v, layout, packed_ld, attr_mask, mask_class, dst, seq_start, word_idx, batch, seq_len,
-                               heads, scaler, split_out, stream);
+                               heads, scaler, out, head_exp, stream);
   else if (seq_len <= 32)
     attention_launch<T, 2>(q, k, v, layout, packed_ld, attr_mask, dst, seq_start, word_idx, batch, seq_len, heads,
-                           scaler, split_out, stream);
+                           scaler, out, head_exp, stream);
   else if constexpr (sizeof(T) == 2)
     attention_launch<T, 4>(q, k, v, layout, packed_ld, attr_mask, dst, seq_start, word_idx, batch, seq_len, heads,
-                           scaler, split_out, stream);
+                           scaler, out, head_exp, stream);
 }
 
 }  // namespace
@@ -1640,20 +1682,20 @@ void launch_mask_class(DType t, const void* attr_mask, const int32_t* seq_start,
     mask_class_kernel<<<grid, 256, 0, stream>>>((const _Float16*)attr_mask, seq_start, word_idx, seq_len, blocks, cls);
 }
 
-bool attention_writes_split(const void* q, const void* k, const void* v, int layout, int packed_ld, int d) {
+bool attention_writes_pieces(const void* q, const void* k, const void* v, int layout, int packed_ld, int d) {
   return d == kD && head_rows_16b<float>(q, k, v, layout, packed_ld, d);
 }
 
 void launch_attention(DType t, const void* q, const void* k, const void* v, int layout, int packed_ld,
                       const void* attr_mask, void* dst, const int32_t* seq_start, const int32_t* word_idx, int batch,
                       int seq_len, int heads, int d, float scaler, hipStream_t stream,
-                      bool split_out, const uint8_t* mask_class) {
+                      AttentionOut out, const uint8_t* mask_class, HeadExps head_exp) {
   if (t == DType::F32)
     attention_dispatch<float>(q, k, v, layout, packed_ld, attr_mask, dst, seq_start, word_idx, batch, seq_len, heads, d,
-                              scaler, split_out, mask_class, stream);
+                              scaler, out, mask_class, head_exp, stream);
   else
     attention_dispatch<_Float16>(q, k, v, layout, packed_ld, attr_mask, dst, seq_start, word_idx, batch, seq_len,
-                                 heads, d, scaler, false, mask_class, stream);
+                                 heads, d, scaler, AttentionOut::kPlain, mask_class, HeadExps(), stream);
 }
 
 }  // namespace et

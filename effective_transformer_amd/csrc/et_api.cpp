@@ -430,24 +430,32 @@ et_status run_layer_pairs(et_handle h, const LayerCall& c) {
     cls = (const uint8_t*)(base + ws.cls);
   }
   const et::PairRows ctx_rows{(_Float16*)(base + ws.ctx), pw.ctx_exp, pw.attn_norm};      // (the norms are rewritten by LayerNorm)
-  // The context takes the attention output's place until its rows are paired.  A launch of its own, because no workgroup of the
-  // attention kernel sees a whole row: with an exponent from a bound instead, the same for all rows of a sequence, a token of large
-  // values took the bits of queries that do not see it (V of that token 2^30 of the others': rows off by 1.9e-3, now 1.1e-6).
-  et::launch_attention(dt, qkv, qkv + H, qkv + 2 * H, 1, 3 * H, c.attr_mask, attn, seq_start, c.word_idx, B, S, c.heads, c.d,
-                       softmax_scaler(c.dtype, c.d), st, false, cls);
-  et::PairRowsJob context;
-  context.src = attn, context.out = ctx_rows, context.m = rows, context.n = H, context.rows_dev = T;
-  et::launch_pair_rows(context, st);
+  // The attention kernels leave the context as pair rows with an exponent for each head, from its own largest value: no workgroup
+  // sees a whole row, and a bound over all rows of a sequence took the bits of queries that do not see a token of large values
+  // (V of that token 2^30 of the others': rows off by 1.9e-3, now 1.1e-6).  Where they cannot (heads of another size than 64) the
+  // context takes the attention output's place until a launch of its own has paired its rows.
+  const bool by_heads = et::attention_writes_pieces(qkv, qkv + H, qkv + 2 * H, 1, 3 * H, c.d);
+  et::HeadExps head_exp;
+  if (by_heads) head_exp = {(int8_t*)(base + ws.attn_split), et::head_exp_stride(rows)};      // (LayerNorm's rows come there behind the product)
+  et::launch_attention(dt, qkv, qkv + H, qkv + 2 * H, 1, 3 * H, c.attr_mask, by_heads ? (void*)ctx_rows.rows : attn, seq_start, c.word_idx, B,
+                       S, c.heads, c.d, softmax_scaler(c.dtype, c.d), st, by_heads ? et::AttentionOut::kPairs : et::AttentionOut::kPlain, cls,
+                       head_exp);
+  if (!by_heads) {
+    et::PairRowsJob context;
+    context.src = attn, context.out = ctx_rows, context.m = rows, context.n = H, context.rows_dev = T;
+    et::launch_pair_rows(context, st);
+  }
   if ((s = check_launch(h, "attention")) != ET_OK) return s;
 
-  auto product = [&](const et::PairRows& a, int w_at, void* C, int n, int k_) {
+  auto product = [&](const et::PairRows& a, const int8_t* a_head_exp, int w_at, void* C, int n, int k_) {
     et::PairProduct p;
     p.A[0] = a;
+    p.head_exp = a_head_exp;
     p.B[0] = wt + w_at * HH;
     p.b_exp[0] = pw.w_exp + w_at * H;
     et::launch_gemm_pair(p, C, n, rows, n, k_, T, st);
   };
-  product(ctx_rows, 3, attn, H, H);
+  product(ctx_rows, head_exp.exp, 3, attn, H, H);
   const et::PairRows attn_rows{(_Float16*)(base + ws.attn_split), pw.attn_exp, pw.attn_norm};
   et::launch_bias_residual_layernorm(dt, attn, c.from, w->attr_output_bias, w->attr_output_layernorm_gamma,
                                      w->attr_output_layernorm_beta, rows, H, T, st, et::WarmList(), nullptr, attn_rows);
@@ -461,7 +469,7 @@ et_status run_layer_pairs(et_handle h, const LayerCall& c) {
   up.c_exp = pw.inter_exp;
   et::launch_gemm_pair(up, base + ws.inter, F, rows, F, H, T, st);
   if ((s = check_launch(h, "FFN up")) != ET_OK) return s;
-  product({(_Float16*)(base + ws.inter), pw.inter_exp, nullptr}, 8, c.out, H, F);
+  product({(_Float16*)(base + ws.inter), pw.inter_exp, nullptr}, nullptr, 8, c.out, H, F);
   et::launch_bias_residual_layernorm(dt, c.out, attn, w->output_bias, w->output_layernorm_gamma, w->output_layernorm_beta, rows, H,
                                      T, st, et::WarmList(), nullptr, c.write_out_split ? from : et::PairRows());
   return check_launch(h, "FFN down");
@@ -558,7 +566,7 @@ et_status run_layer(et_handle h, const LayerCall& c) {
   if ((s = check_launch(h, "QKV projection")) != ET_OK) return s;
   // QK^T, softmax, PV, un-pad (:159-192)
   const char *q = (const char*)qkv, *k = q + (size_t)H * e, *v = k + (size_t)H * e;
-  const bool ctx_split = split && et::attention_writes_split(q, k, v, 1, 3 * H, c.d);
+  const bool ctx_split = split && et::attention_writes_pieces(q, k, v, 1, 3 * H, c.d);
   const uint8_t* cls = c.mask_class ? c.mask_class : batch.cls;
   if (!cls && et::mask_class_bytes(dt, B, S, c.d)) {
     et::launch_mask_class(dt, c.attr_mask, seq_start, c.word_idx, B, S, (uint8_t*)(base + ws.cls), st);
@@ -566,7 +574,7 @@ et_status run_layer(et_handle h, const LayerCall& c) {
   }
   // (where the attention kernel writes floats only, they take the attention output's place until they are split)
   et::launch_attention(dt, q, k, v, 1, 3 * H, c.attr_mask, split && !ctx_split ? attn : ctx, seq_start, c.word_idx, B, S,
-                       c.heads, c.d, softmax_scaler(c.dtype, c.d), st, ctx_split, cls);
+                       c.heads, c.d, softmax_scaler(c.dtype, c.d), st, ctx_split ? et::AttentionOut::kSplit : et::AttentionOut::kPlain, cls);
   if (split && !ctx_split) et::launch_split_rows((const float*)attn, (uint16_t*)ctx, rows, H, T, st);
   if ((s = check_launch(h, "attention")) != ET_OK) return s;
   // attention output projection + bias + residual(from_tensor) + LayerNorm (:195-213)
@@ -1278,7 +1286,7 @@ et_status et_attention_with_starts(et_handle h, et_dtype dtype, const void* q, c
     }
   }
   et::launch_attention(to_dt(dtype), q, k, v, qkv_layout, packed_ld, attr_mask, dst, seq_start, word_idx, batch_size,
-                       seq_len, head_num, size_per_head, softmax_scaler(dtype, size_per_head), st, false, cls);
+                       seq_len, head_num, size_per_head, softmax_scaler(dtype, size_per_head), st, et::AttentionOut::kPlain, cls);
   return check_launch(h, "attention");
 }
 

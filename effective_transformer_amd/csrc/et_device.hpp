@@ -178,7 +178,7 @@ __device__ __forceinline__ int pair_exponent(float bound) {
   return min(max(__builtin_amdgcn_frexp_expf(fminf(bound, 3.4e38f)) - 15, -112), 113);
 }
 __device__ __forceinline__ float pair_scale(int e) { return __builtin_ldexpf(1.0f, -e); }
-// N consecutive values (N = 1, 2 or 4; col a multiple of N) of a pair row: [k / 32][h, l][32] halves; scale = pair_scale(e)
+// N consecutive values (N = 1, 2, 4 or 8; col a multiple of N) of a pair row: [k / 32][h, l][32] halves; scale = pair_scale(e)
 // The epilogues that store pair rows are bound by their arithmetic: with l made from the stored halves a pair of values takes one
 // conversion, where the compiler converted every value a second time for l (FFN-up on 20375 rows 277 -> 263 us together with
 // gemm_pair_kernel's one lane per exponent, same bits).

@@ -14,12 +14,15 @@
 // layers of smaller hidden sizes keep them.  Infinities and NaNs give NaN.
 //
 // Both operands come as "pair rows": [row][k / 32][h, l][32] halves, one 128-byte line per row and k-step of 32.  Both have
-// an exponent per row, which are applied to the result.  Input, LayerNorm and the pass over the context take it from the row's
-// largest value; the FFN's first product, whose workgroups see parts of a row, takes a bound instead (pair_gelu_bound).  Weights
+// an exponent per row, which are applied to the result.  Input and LayerNorm take it from the row's
+// largest value; the FFN's first product, whose workgroups see parts of a row, takes a bound instead (pair_gelu_bound).  The
+// attention kernels see a head of a row, 64 values: context rows have an exponent per 64 k, and the output product (HEADS) weighs
+// its chunks where it adds them up (20375 rows, attention and product: 141 us with a launch in between that found the rows' own
+// exponents, 130 us; 3820 rows 57 and 53; one tile's worth, 160 rows, level; encoders of 12 layers 1 to 2 %).  Weights
 // are taken anew by every layer call: pair_weight_top_kernel looks for the largest value of each column, pair_weight_kernel
 // writes the rows (9 + 11.5 us per layer of BERT-base, split rows 15).
 // Bound: at large m the power limit of the matrix cores (20375 rows, k = 768 / n = 2304, 768, 3072 + GELU and k = 3072 / n = 768:
-// 180, 64, 270, 233 us in the layer, 1070 .. 1240 TFLOP/s of 16-bit products; split rows 307, 112, 451, 413); below a round of the
+// 180, 71, 270, 233 us in the layer, 1070 .. 1240 TFLOP/s of 16-bit products; split rows 307, 112, 451, 413); below a round of the
 // chip the k loop of one tile (134 rows: 10.2, 6.5, 12.8, 14.3 us against 15.2, 8.7, 16.1, 21.3).
 #include <algorithm>
 #include <atomic>
@@ -90,11 +93,13 @@ struct PairTile {
 //   ahead.
 //   KS = 2 (small tiles): a stage is a chunk; one barrier per stage, the next stage's operands are read into a second register
 //   set under this one's MFMAs.
-// GELU: C = gelu(A.B + bias) as pair rows with their exponents in c_exp; otherwise C is float, + bias if given.
-template <int WM, int WN, int MI, int NJ, int ST, int KS, bool GELU>
+// GELU: C = gelu(A.B + bias) as pair rows with their exponents in c_exp; otherwise C is float, + bias if given.  HEADS: A's rows
+// have an exponent per chunk.
+template <int WM, int WN, int MI, int NJ, int ST, int KS, bool GELU, bool HEADS>
 __global__ __launch_bounds__(WM * WN * kWave) void gemm_pair_kernel(
     // what comes before the first request, as arguments of their own (gemm_f16_bt_kernel has the reason)
-    const _Float16* a0, const _Float16* b0, const int32_t* rows_dev, int m_bound, int N, int K, int tiles_n, int groups, int columns, PairGemmArgs args) {
+    const _Float16* a0, const _Float16* b0, const int32_t* rows_dev, int m_bound, int N, int K, int tiles_n, int groups, int columns,
+    const uint32_t* head_exp, PairGemmArgs args) {
 #if defined(__HIP_DEVICE_COMPILE__)   // device-only types in the body; the host pass only needs the stub
   using Tile = PairTile<WM, WN, MI, NJ, ST, KS>;
   constexpr int BM = Tile::BM, BN = Tile::BN;
@@ -199,6 +204,57 @@ __global__ __launch_bounds__(WM * WN * kWave) void gemm_pair_kernel(
 
   float4v sum[MI][NJ], acc[MI][NJ];
   const float4v zero = {0.f, 0.f, 0.f, 0.f};
+  // HEADS: behind the ring the exponent of each row of the tile, the largest of its chunks', and per chunk 2^(the chunk's exponent -
+  // the row's) as the upper half of the float.  Eight lanes see to four rows (a word of every chunk), every eighth chunk each;
+  // `exps` is requested early.
+  constexpr int kExpChunks = kMaxHeadExps / 8;
+  static_assert(BM * 2 <= Tile::THREADS, "eight lanes for four rows");
+  int* const row_exp = reinterpret_cast<int*>(smem + Tile::SMEM);
+  uint16_t* const chunk_scale = reinterpret_cast<uint16_t*>(smem + Tile::SMEM + BM * 4);
+  uint32_t exps[kExpChunks] = {};
+  const int exp_first = threadIdx.x & 7, exp_rows = (int)(threadIdx.x >> 3) * 4;
+  auto request_exps = [&](int m0) {
+    const int chunks = (int)((unsigned)K / 64), word = min(m0 + min(exp_rows, BM - 4), rows - 1) >> 2;
+#pragma unroll
+    for (int u = 0; u < kExpChunks; ++u)
+      if (u * 8 < chunks) exps[u] = head_exp[(size_t)min(exp_first + u * 8, chunks - 1) * ((unsigned)(m_bound + 3) / 4) + word];
+  };
+  auto write_exps = [&] {
+    const int chunks = (int)((unsigned)K / 64);
+    int top[4];
+#pragma unroll
+    for (int r = 0; r < 4; ++r) {
+      top[r] = -128;
+#pragma unroll
+      for (int u = 0; u < kExpChunks; ++u)       // (the last chunk stands for those behind it)
+        if (u * 8 < chunks) top[r] = max(top[r], (int)(exps[u] << (24 - 8 * r)) >> 24);
+      top[r] = max(top[r], dpp_i32<kDppQuadXor1>(top[r], top[r]));
+      top[r] = max(top[r], dpp_i32<kDppQuadXor2>(top[r], top[r]));
+      top[r] = max(top[r], dpp_i32<kDppRowHalfMirror>(top[r], top[r]));
+    }
+    if (exp_rows >= BM) return;
+    typedef int int4v __attribute__((ext_vector_type(4)));
+    if (exp_first == 0) *reinterpret_cast<int4v*>(row_exp + exp_rows) = int4v{top[0], top[1], top[2], top[3]};
+#pragma unroll
+    for (int u = 0; u < kExpChunks; ++u) {
+      if (exp_first + u * 8 >= chunks) break;
+      uint32_t s[4];
+#pragma unroll
+      for (int r = 0; r < 4; ++r) s[r] = (uint32_t)max(127 + ((int)(exps[u] << (24 - 8 * r)) >> 24) - top[r], 0) << 7;
+      *reinterpret_cast<u32x2*>(chunk_scale + (exp_first + u * 8) * BM + exp_rows) = u32x2{s[0] | s[1] << 16, s[2] | s[3] << 16};
+    }
+  };
+  u32x2 scales[MI] = {};                         // of the chunk that is added next (in front of a tile's first one, of anything: acc is 0)
+  auto read_scales = [&](int chunk) {
+#pragma unroll
+    for (int i = 0; i < MI; ++i) scales[i] = *reinterpret_cast<const u32x2*>(chunk_scale + chunk * BM + wm * 16 * MI + i * 16 + g * 4);
+  };
+  // the sum with the chunk whose products are in acc
+  auto folded = [&](int i, int j, int r) {
+    if constexpr (!HEADS) return sum[i][j][r] + acc[i][j][r];
+    const uint32_t w = r < 2 ? scales[i].x : scales[i].y;
+    return __builtin_fmaf(acc[i][j][r], __builtin_bit_cast(float, r & 1 ? w & 0xffff0000u : w << 16), sum[i][j][r]);
+  };
   // one row of blocks; FIRST: the chunk's first product, behind the fold of the chunk before it
   auto mfma_row = [&](auto FIRSTc, const half8 (&a)[MI], const half8 (&b)[NJ], int i) {
     constexpr bool FIRST = decltype(FIRSTc)::value;
@@ -207,7 +263,7 @@ __global__ __launch_bounds__(WM * WN * kWave) void gemm_pair_kernel(
       const int j = (i & 1) ? NJ - 1 - jj : jj;          // only one operand changes from one MFMA to the next
       if constexpr (FIRST) {
 #pragma unroll
-        for (int r = 0; r < 4; ++r) sum[i][j][r] += acc[i][j][r];
+        for (int r = 0; r < 4; ++r) sum[i][j][r] = folded(i, j, r);
         acc[i][j] = __builtin_amdgcn_mfma_f32_16x16x32_f16(a[i], b[j], zero, 0, 0, 0);
       } else {
         acc[i][j] = __builtin_amdgcn_mfma_f32_16x16x32_f16(a[i], b[j], acc[i][j], 0, 0, 0);
@@ -225,6 +281,7 @@ __global__ __launch_bounds__(WM * WN * kWave) void gemm_pair_kernel(
   half8 pa[2][2][2][MI], pb[2][2][2][NJ];                        // KS = 2: [register set][k-step][piece]
 
   Src cur = locate(idx), nxt = cur;
+  if constexpr (HEADS) request_exps(cur.m0);
 #pragma unroll
   for (int s = 0; s < ST; ++s) issue_stage(s, min(s, nst - 1), cur, cur);
   // GELU: what bounds the rows of C, the same for every row.  Small tiles look at it, and at all that the epilogue reads, behind
@@ -233,6 +290,10 @@ __global__ __launch_bounds__(WM * WN * kWave) void gemm_pair_kernel(
   PairStats stats;
   if constexpr (GELU) pair_stats_request(args.b_stats, args.stat_pairs, (int)((unsigned)(N + 63) / 64), stats);
   wait_vmcnt<KS * Tile::DMA*(ST - 1)>();
+  if constexpr (HEADS) {
+    write_exps();
+    wait_lgkmcnt0();
+  }
   barrier_only();
   auto read_set = [&](half8 (&a)[2][2][MI], half8 (&b)[2][2][NJ], int slot) {
 #pragma unroll
@@ -281,7 +342,8 @@ __global__ __launch_bounds__(WM * WN * kWave) void gemm_pair_kernel(
       if (add != nullptr) bias = *reinterpret_cast<const fvec*>(add + col);
       // (the row arrays reach beyond the last tile: PairRows)
 #pragma unroll
-      for (int i = 0; i < MI; ++i) re[i] = *reinterpret_cast<const int4v*>(a_exp + row0 + i * 16);
+      for (int i = 0; i < MI; ++i)
+        if constexpr (!HEADS) re[i] = *reinterpret_cast<const int4v*>(a_exp + row0 + i * 16);
     };
     if constexpr (!Tile::BIG) request(args.a_exp[cur.grp], args.b_exp[cur.grp], args.bias[cur.grp], args.a_norm);
     if constexpr (Tile::BIG) {
@@ -296,6 +358,7 @@ __global__ __launch_bounds__(WM * WN * kWave) void gemm_pair_kernel(
         if (first_tile || t >= ST - 1) wait_vmcnt<Tile::DMA*(ST - 2)>();
         wait_lgkmcnt0();                           // its last reads of slot s are complete
         barrier_only();
+        if constexpr (HEADS && P == 1) read_scales(t >> 1);
         const int s1 = s + 1 == ST ? 0 : s + 1;
         // the DMA instructions go out between the rows of MFMAs: in one piece they would keep the wavefront from issuing
         constexpr int kPer = (Tile::DMA + 2 * MI - 1) / (2 * MI);
@@ -330,6 +393,7 @@ __global__ __launch_bounds__(WM * WN * kWave) void gemm_pair_kernel(
         read_set(pa[1 - P], pb[1 - P], s1);
         __builtin_amdgcn_sched_barrier(0);
         mfma(kFirst, pa[P][0][0], pb[P][0][1]);
+        if constexpr (HEADS) read_scales(t);
         issue_stage(s, t + ST, cur, nxt);
         mfma(kMore, pa[P][0][1], pb[P][0][0]);
         mfma(kMore, pa[P][0][0], pb[P][0][0]);
@@ -359,7 +423,11 @@ __global__ __launch_bounds__(WM * WN * kWave) void gemm_pair_kernel(
       }
     }
     wait_vmcnt<0>();
-
+    if constexpr (HEADS) {
+      request_exps(nxt.m0);
+#pragma unroll
+      for (int i = 0; i < MI; ++i) re[i] = *reinterpret_cast<const int4v*>(row_exp + wm * 16 * MI + i * 16 + g * 4);
+    }
     if constexpr (Tile::BIG) request(args.a_exp[cur.grp], args.b_exp[cur.grp], args.bias[cur.grp], args.a_norm);
     // the loads are waited for here: left pending on the paths that store nothing, they would have the compiler put a wait
     // for every outstanding load, the DMA included, in front of the k loop's reuse of their registers
@@ -372,6 +440,13 @@ __global__ __launch_bounds__(WM * WN * kWave) void gemm_pair_kernel(
 #pragma unroll
     for (int i = 0; i < MI; ++i) asm volatile("" : "+v"(re[i]));
     if constexpr (GELU) asm volatile("" : "+v"(own_norm));
+    if constexpr (HEADS) {
+#pragma unroll
+      for (int u = 0; u < kExpChunks; ++u) asm volatile("" : "+v"(exps[u]));
+      wait_lgkmcnt0();                             // everybody has read what this tile needs of the exponents:
+      barrier_only();
+      write_exps();                                // the next one's, which the bar of its first step shows to all
+    }
     if constexpr (GELU && !Tile::BIG)
       if (first_tile) bounds = pair_stats_max(args.b_stats, args.stat_pairs, (int)((unsigned)(N + 63) / 64), stats);
     float4v scale[MI];
@@ -389,7 +464,7 @@ __global__ __launch_bounds__(WM * WN * kWave) void gemm_pair_kernel(
           if (row >= rows) continue;
           fvec o;
 #pragma unroll
-          for (int j = 0; j < NJ; ++j) o[j] = __builtin_ldexpf(sum[i][j][r] + acc[i][j][r], re[i][r] + ce[j]) + bias[j];
+          for (int j = 0; j < NJ; ++j) o[j] = __builtin_ldexpf(folded(i, j, r), re[i][r] + ce[j]) + bias[j];
           if constexpr (GELU) {
 #pragma unroll
             for (int j = 0; j < NJ; ++j) o[j] *= gelu_cdf(o[j], o[j] * o[j] * o[j]);
@@ -428,16 +503,18 @@ int device_cu_count() {
 // large ones want the tile with the fewest operand bytes per product.  A launch takes rounds of tiles over the CUs, each
 // as long as its k-steps and a part for filling the ring and storing C.
 enum PairPick { p256x128, p192x128, p128x128, p96x128, p64x128, p64x64, p32x64, p32x32, kPairPicks };
-PairPick pick_pair_tile(int m, int n, int k, int groups) {
+PairPick pick_pair_tile(int m, int n, int k, int groups, bool heads) {
   static constexpr struct { int bm, bn; float step; } kTiles[] = {
       {256, 128, 0.8f}, {192, 128, 0.66f}, {128, 128, 0.48f}, {96, 128, 0.4f}, {64, 128, 0.3f}, {64, 64, 0.19f}, {32, 64, 0.135f}, {32, 32, 0.085f}};
   const long cus = device_cu_count();
   int best = 0;
   float best_cost = 0.f;
-  for (int i = 0; i < (int)std::size(kTiles); ++i) {
+  // (256 rows' exponents of more than 30 chunks do not fit the LDS beside the ring)
+  const int first = heads && k > 30 * 64 ? 1 : 0;
+  for (int i = first; i < (int)std::size(kTiles); ++i) {
     const long tiles = (long)((m + kTiles[i].bm - 1) / kTiles[i].bm) * ((n + kTiles[i].bn - 1) / kTiles[i].bn) * groups;
     const float cost = (float)((tiles + cus - 1) / cus) * (kTiles[i].step * (float)(k / 32) + 3.f);
-    if (i == 0 || cost < best_cost) {
+    if (i == first || cost < best_cost) {
       best = i;
       best_cost = cost;
     }
@@ -446,7 +523,7 @@ PairPick pick_pair_tile(int m, int n, int k, int groups) {
 }
 
 template <int WM, int WN, int MI, int NJ, int ST, int KS>
-void launch_tile(PairGemmArgs a, bool gelu, int groups, hipStream_t stream) {
+void launch_tile(PairGemmArgs a, bool gelu, int groups, const uint32_t* head_exp, hipStream_t stream) {
   using Tile = PairTile<WM, WN, MI, NJ, ST, KS>;
   a.tiles_n = (a.n + Tile::BN - 1) / Tile::BN;
   a.groups = groups;
@@ -461,23 +538,25 @@ void launch_tile(PairGemmArgs a, bool gelu, int groups, hipStream_t stream) {
   // (a stream of fewer stages than the ring holds must not cross into a second tile)
   const int grid = ((a.k / (32 * KS) < ST ? tiles : std::min(tiles, device_cu_count())) + kXcds - 1) / kXcds * kXcds;
   auto go = [&](auto kern) {
-    allow_dynamic_lds(reinterpret_cast<const void*>(kern), Tile::SMEM);
-    kern<<<grid, Tile::THREADS, Tile::SMEM, stream>>>(a.A[0], a.B[0], a.rows_dev, a.m_bound, a.n, a.k, a.tiles_n, groups, a.columns, a);
+    const int lds = Tile::SMEM + (head_exp ? Tile::BM * (4 + 2 * (a.k / 64)) : 0);
+    allow_dynamic_lds(reinterpret_cast<const void*>(kern), lds);
+    kern<<<grid, Tile::THREADS, lds, stream>>>(a.A[0], a.B[0], a.rows_dev, a.m_bound, a.n, a.k, a.tiles_n, groups, a.columns, head_exp, a);
   };
-  if (gelu) go(gemm_pair_kernel<WM, WN, MI, NJ, ST, KS, true>);
-  else go(gemm_pair_kernel<WM, WN, MI, NJ, ST, KS, false>);
+  if (gelu) go(gemm_pair_kernel<WM, WN, MI, NJ, ST, KS, true, false>);
+  else if (head_exp) go(gemm_pair_kernel<WM, WN, MI, NJ, ST, KS, false, true>);
+  else go(gemm_pair_kernel<WM, WN, MI, NJ, ST, KS, false, false>);
 }
 
-void launch_pick(PairPick pick, const PairGemmArgs& a, bool gelu, int groups, hipStream_t stream) {
+void launch_pick(PairPick pick, const PairGemmArgs& a, bool gelu, int groups, const uint32_t* head_exp, hipStream_t stream) {
   switch (pick) {
-    case p256x128: return launch_tile<4, 2, 4, 4, 3, 1>(a, gelu, groups, stream);
-    case p192x128: return launch_tile<4, 2, 3, 4, 3, 1>(a, gelu, groups, stream);
-    case p128x128: return launch_tile<2, 4, 4, 2, 4, 1>(a, gelu, groups, stream);
-    case p96x128: return launch_tile<2, 4, 3, 2, 4, 1>(a, gelu, groups, stream);
-    case p64x128: return launch_tile<2, 4, 2, 2, 3, 2>(a, gelu, groups, stream);
-    case p64x64: return launch_tile<4, 2, 1, 2, 4, 2>(a, gelu, groups, stream);
-    case p32x64: return launch_tile<2, 4, 1, 1, 5, 2>(a, gelu, groups, stream);
-    case p32x32: return launch_tile<2, 2, 1, 1, 6, 2>(a, gelu, groups, stream);
+    case p256x128: return launch_tile<4, 2, 4, 4, 3, 1>(a, gelu, groups, head_exp, stream);
+    case p192x128: return launch_tile<4, 2, 3, 4, 3, 1>(a, gelu, groups, head_exp, stream);
+    case p128x128: return launch_tile<2, 4, 4, 2, 4, 1>(a, gelu, groups, head_exp, stream);
+    case p96x128: return launch_tile<2, 4, 3, 2, 4, 1>(a, gelu, groups, head_exp, stream);
+    case p64x128: return launch_tile<2, 4, 2, 2, 3, 2>(a, gelu, groups, head_exp, stream);
+    case p64x64: return launch_tile<4, 2, 1, 2, 4, 2>(a, gelu, groups, head_exp, stream);
+    case p32x64: return launch_tile<2, 4, 1, 1, 5, 2>(a, gelu, groups, head_exp, stream);
+    case p32x32: return launch_tile<2, 2, 1, 1, 6, 2>(a, gelu, groups, head_exp, stream);
     default: return;
   }
 }
@@ -762,7 +841,8 @@ void launch_gemm_pair(const PairProduct& p, void* C, int ldc, int m_bound, int n
   a.m_bound = m_bound;
   a.n = n;
   a.k = k;
-  launch_pick(pick_pair_tile(m_bound, n, k, p.groups), a, p.c_exp != nullptr, p.groups, stream);
+  launch_pick(pick_pair_tile(m_bound, n, k, p.groups, p.head_exp != nullptr), a, p.c_exp != nullptr, p.groups,
+              (const uint32_t*)p.head_exp, stream);
 }
 
 }  // namespace et

@@ -130,19 +130,28 @@ void launch_transpose_rm_padding(DType t, const void* src, void* dst, const int3
                                  int rows_bound, int batch, int seq_len, int heads, int d,
                                  const int32_t* batch_idx, const int32_t* word_idx, hipStream_t stream);
 bool attention_supported(DType t, int seq_len, int d);
+// What an fp32 launch leaves in dst; the others than float rows only where attention_writes_pieces says so.  kPairs: pair rows whose
+// heads have an exponent each (gemm_pair.hip).
+enum class AttentionOut { kPlain, kSplit, kPairs };
+// [head][row], a byte each, with the bound of the rows rounded up to 4 as the stride; memory aligned to 4 bytes.
+constexpr int kMaxHeadExps = 32;       // heads
+inline int head_exp_stride(int rows) { return (rows + 3) / 4 * 4; }
+struct HeadExps {
+  int8_t* exp = nullptr;
+  int stride = 0;
+};
 // layout 0: padded [B,heads,S,d]; layout 1: packed rows with leading dimension packed_ld.
 void launch_attention(DType t, const void* q, const void* k, const void* v, int layout, int packed_ld,
                       const void* attr_mask, void* dst, const int32_t* seq_start, const int32_t* word_idx,
                       int batch, int seq_len, int heads, int d, float scaler, hipStream_t stream,
-                      bool split_out = false, const uint8_t* mask_class = nullptr);
+                      AttentionOut out = AttentionOut::kPlain, const uint8_t* mask_class = nullptr, HeadExps head_exp = HeadExps());
 // Classes of the mask rows (one byte per 16 query positions of a sequence) for the kernel that makes use of them; the same
 // array serves every layer of a batch.  0 bytes: the kernel of this shape has no use for them.
 size_t mask_class_bytes(DType t, int batch, int seq_len, int d);
 size_t mask_class_bytes_max(int batch);                // at any length
 void launch_mask_class(DType t, const void* attr_mask, const int32_t* seq_start, const int32_t* word_idx, int batch, int seq_len,
                        uint8_t* cls, hipStream_t stream);
-// split_out (fp32): dst gets split rows (see gemm_split.hip) instead of float rows; only where this says so
-bool attention_writes_split(const void* q, const void* k, const void* v, int layout, int packed_ld, int d);
+bool attention_writes_pieces(const void* q, const void* k, const void* v, int layout, int packed_ld, int d);
 
 // ---- gemm.hip ----------------------------------------------------------------------------
 // Up to three independent column groups share one launch (the Q/K/V projections): group g
@@ -253,6 +262,8 @@ struct PairProduct {
   const float* bias[3] = {};
   const float* stats = nullptr;
   int32_t* c_exp = nullptr;
+  // one group, C float, k up to 64 kMaxHeadExps: A's rows have an exponent per 64 k, and A[0].exp is not read
+  const int8_t* head_exp = nullptr;
 };
 void launch_gemm_pair(const PairProduct& p, void* C, int ldc, int m_bound, int n, int k, const int32_t* rows_dev,
                       hipStream_t stream);

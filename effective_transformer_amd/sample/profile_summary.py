@@ -23,7 +23,7 @@ from .workloads import WORKLOADS
 
 ROLES = ["QKV", "attention", "attention out", "LayerNorm 1", "FFN up + GELU", "FFN down", "LayerNorm 2"]
 SIDE = ("scan_index", "compress_rows", "embed_layernorm", "seq_start", "seq_order", "mask_class", "pair_weight", "pair_rows", "restore_rows")
-# fp32 products on pair rows: the context's rows are paired by a launch of their own
+# fp32 products on pair rows with heads of another size than 64: the context's rows are paired by a launch of their own
 PAIR_ROLES = ROLES[:2] + ["context to pair rows"] + ROLES[2:]
 LAYER_KINDS = ("context_rows", "attention", "bias_residual_layernorm", "gemm_f16_pair", "gemm_f16_bt", "gemm_f16_persistent", "gemm_f16_kernel",
                "gemm_f32", "gemm_pair_kernel", "gemm_split")
@@ -66,7 +66,7 @@ def roles_of(body, layers):
 
 
 def encoder_steps(kinds, layers):
-    """Index lists of the 7 (fp32 on pair rows: 8) x layers layer kernels of every complete encoder step (input op ... output
+    """Index lists of the 7 (where a launch pairs the context's rows: 8) x layers layer kernels of every complete encoder step (input op ... output
     op) in a dispatch sequence."""
     steps, i = [], 0
     while i < len(kinds):
