@@ -542,6 +542,8 @@ constexpr int kQAPair = kPBM * 128;                            // 32 KB: 256 row
 constexpr int kQPair = kQAPair + kPBN * 128;                   // 64 KB: A rows, then B^T rows
 constexpr int kQSmem = 2 * kQPair;
 constexpr int kQSmemA3 = 3 * kQAPair + 2 * (kQPair - kQAPair);   // 160 KB: three A slots, two B^T slots
+// LDS slots for A (two or three) and where the DMA instructions go: all eight under the odd k-step, or A's under the even one
+enum class PairRing { kTwo, kThreeA, kThreeASpread };
 
 __device__ __forceinline__ int pair_swizzle(int row) { return (row >> 1) & 7; }
 
@@ -582,17 +584,24 @@ __device__ __forceinline__ TileHead tile_head(const void* a0, const void* b0, co
 // descriptor and cost no traffic.
 // NT: C leaves through non-temporal stores (a matrix too big to be found in the last-level cache by its reader);
 // plain stores otherwise.
-// A3: three LDS slots for A instead of two, all of the 160 KB: the A rows of a pair are requested three pairs ahead
+// kThreeA: three LDS slots for A instead of two, all of the 160 KB: the A rows of a pair are requested three pairs ahead
 // of their first use instead of two (B^T as before).  For the projection whose A is the big matrix and comes from
 // HBM (k >= 2048: FFN-down), where a pair's time does not cover that latency.  Same instructions on the same data in
 // the same order: same bits.
-template <bool GELU, int MI, bool NT, bool A3>
+// kThreeASpread: the same slots, but the four A instructions of a pair go out under the even k-step and only the four of B^T under
+// the odd one.  Eight of every wavefront under one k-step take the address unit 1024 cycles, as long as the step's MFMAs at 256
+// rows and longer at fewer, where the wavefronts then wait to issue; A's third slot is what an even step can fill.  Per launch in
+// the layer: 13097 x 1024, k = 4096 (192 rows) 88.7 -> 84.7 us, k = 1024 27.4 -> 26.5; 12290 x 768, k = 3072 (160 rows) 56.6 -> 55.1,
+// k = 768 19.9 -> 19.6.  At 256 rows it takes A's longer way back (20375 x 768, k = 3072: 81.9 -> 82.9) and for wide outputs the
+// power of the requests kept in flight (FFN-up and QKV +1 to +2 %).
+template <bool GELU, int MI, bool NT, PairRing RING>
 __device__ __forceinline__ void pair_tiles(const TileHead& head, int tiles_n, int columns, int walk, const GemmArgs& args, unsigned char* smem) {
 #if defined(__HIP_DEVICE_COMPILE__)   // device-only types in the body; the host pass only needs the stub
   const int tid = threadIdx.x;
   const int lane = tid & (kWave - 1);
   const int wave = __builtin_amdgcn_readfirstlane(tid / kWave);   // 0..7, scalar
   constexpr int BM = 32 * MI;                                     // rows of a tile
+  constexpr bool SPREAD = RING == PairRing::kThreeASpread, A3 = RING != PairRing::kTwo;
   const int wm = wave & 1, wn = (wave >> 1) & 3;                  // (16 MI)-row half, 64-column quarter of the tile
   const int l16 = lane & 15, g = lane >> 4;
   const int rows = head.rows, N = head.n, K = head.k;
@@ -675,7 +684,7 @@ __device__ __forceinline__ void pair_tiles(const TileHead& head, int tiles_n, in
     __builtin_amdgcn_raw_ptr_buffer_load_lds(rb, ET_LDS_PTR(b_slot(sb) + (wave * 4 + q) * 1024), 16, voff_b[q], pr * 128,
                                              0, 0);
   };
-  // instruction q (0..7) of a whole pair: A first, then B^T; with A3 the other way round, and the A rows are those
+  // instruction q (0..7) of a whole pair: A first, then B^T; with kThreeA the other way round, and the A rows are those
   // of the pair one further ahead, so that they are the newest requests and may stay in flight at the next wait
   auto issue1 = [&](int sa, int sb, int pr_a, int pr_b, const __amdgpu_buffer_rsrc_t& ra,
                     const __amdgpu_buffer_rsrc_t& rb, int q) {
@@ -714,14 +723,15 @@ __device__ __forceinline__ void pair_tiles(const TileHead& head, int tiles_n, in
   half8 a[2][MI], b[2][4];
   int pairs_done = 0;                            // by this workgroup: slot of a pair = pairs_done & 1
 
-  // One k-step: MFMAs on operand set P; half `rh` of the slots rsa / rsb is read into the other set; with DMA set, this
-  // wave's eight DMA instructions (A rows of pair dpa into slot dsa, B^T rows of pair dpb into slot dsb; descriptors
-  // da, db) go out, one after each group of four MFMAs.
+  // One k-step: MFMAs on operand set P; half `rh` of the slots rsa / rsb is read into the other set; this wave's DMA
+  // instructions (A rows of pair dpa into slot dsa, B^T rows of pair dpb into slot dsb; descriptors da, db), all eight or those of
+  // A or of B^T, go out between the groups of four MFMAs.
+  enum class Dma { kNone, kA, kB, kBoth };
   auto step = [&](auto Pc, auto FIRSTc, auto DMAc, int rsa, int rsb, int dsa, int dsb, int dpa, int dpb,
                   const __amdgpu_buffer_rsrc_t& da, const __amdgpu_buffer_rsrc_t& db) {
     constexpr int P = decltype(Pc)::value;
     constexpr bool FIRST = decltype(FIRSTc)::value;
-    constexpr bool DMA = decltype(DMAc)::value;
+    constexpr Dma DMA = decltype(DMAc)::value;
     constexpr int rh = 1 - P;                    // the even step reads half 1 of its own pair, the odd step half 0 of the next
     const unsigned char* nsa = a_slot(rsa);
     const unsigned char* nsb = b_slot(rsb);
@@ -741,18 +751,26 @@ __device__ __forceinline__ void pair_tiles(const TileHead& head, int tiles_n, in
         acc[i][j] = __builtin_amdgcn_mfma_f32_16x16x32_f16(a[P][i], b[P][j],
                                                            FIRST ? float4v{0.f, 0.f, 0.f, 0.f} : acc[i][j], 0, 0, 0);
       }
-      if (DMA) {
+      if (DMA == Dma::kBoth) {
 #pragma unroll
         for (int q = 0; q < 8; ++q)
           if (q * MI / 8 == i) issue1(dsa, dsb, dpa, dpb, da, db, q);      // the eight DMA instructions spread over the MI groups
+      } else {
+#pragma unroll
+        for (int q = 0; q < 4; ++q) {
+          if (DMA == Dma::kA && q * MI / 4 == i) issue_a(dsa, dpa, da, q);
+          if (DMA == Dma::kB && q * MI / 4 == i) issue_b(dsb, dpb, db, q);
+        }
       }
       __builtin_amdgcn_sched_barrier(0);         // keeps the reads and the DMA where they are between the MFMA groups
     }
   };
   using Even = std::integral_constant<int, 0>;
   using Odd = std::integral_constant<int, 1>;
+  using EvenDma = std::integral_constant<Dma, SPREAD ? Dma::kA : Dma::kNone>;
+  using OddDma = std::integral_constant<Dma, SPREAD ? Dma::kB : Dma::kBoth>;
 
-  // pairs 0 and 1 of the first tile (with A3 also the A rows of pair 2), operands of k-step 0
+  // pairs 0 and 1 of the first tile (with kThreeA also the A rows of pair 2), operands of k-step 0
 #pragma unroll
   for (int q = 0; q < 4; ++q) issue_a(0, 0, cur.a, q);
 #pragma unroll
@@ -761,7 +779,7 @@ __device__ __forceinline__ void pair_tiles(const TileHead& head, int tiles_n, in
   for (int q = 0; q < 4; ++q) issue_a(1, 1, cur.a, q);
 #pragma unroll
   for (int q = 0; q < 4; ++q) issue_b(1, 1, cur.b, q);
-  if (A3) {
+  if (A3 && !SPREAD) {
 #pragma unroll
     for (int q = 0; q < 4; ++q) issue_a(2, 2, cur.a, q);
     wait_vmcnt<12>();
@@ -787,10 +805,13 @@ __device__ __forceinline__ void pair_tiles(const TileHead& head, int tiles_n, in
       for (int p = 0; p < np; ++p) {
         const int s = pairs_done & 1;
         const int ra = A3 ? sa : s;                // this pair's A slot
-        if (p == 0) step(Even{}, std::true_type{}, std::false_type{}, ra, s, 0, 0, 0, 0, cur.a, cur.b);
-        else step(Even{}, std::false_type{}, std::false_type{}, ra, s, 0, 0, 0, 0, cur.a, cur.b);
+        // SPREAD: the A rows of pair p+2 replace those of pair p-1
+        const int pe = p + 2 < np ? p + 2 : p + 2 - np, ea_slot = sa == 0 ? 2 : sa - 1;
+        const __amdgpu_buffer_rsrc_t ea = p + 2 < np ? cur.a : nxt.a;
+        if (p == 0) step(Even{}, std::true_type{}, EvenDma{}, ra, s, ea_slot, 0, pe, 0, ea, cur.b);
+        else step(Even{}, std::false_type{}, EvenDma{}, ra, s, ea_slot, 0, pe, 0, ea, cur.b);
         // this wave's share of the next pair has landed (right after a tile boundary that was confirmed before the C
-        // stores went out) and its last reads of slot s, which feed the odd step, are complete; with A3 the four
+        // stores went out) and its last reads of slot s, which feed the odd step, are complete; with three A slots the four
         // newest requests, the A rows of the pair after the next, may still be on their way
         if (first_tile || p >= 1) {
           if (A3) wait_vmcnt<4>();
@@ -798,12 +819,12 @@ __device__ __forceinline__ void pair_tiles(const TileHead& head, int tiles_n, in
         }
         wait_lgkmcnt0();
         barrier_only();
-        // B^T of pair p+2 (A of pair p+2, with A3 of pair p+3) of this tile, or the matching pair of the next one,
+        // B^T of pair p+2 (A of pair p+2, with kThreeA of pair p+3) of this tile, or the matching pair of the next one,
         // replaces what this pair held
         const int pa = A3 ? p + 3 : p + 2, pb = p + 2;
         const __amdgpu_buffer_rsrc_t da = pa < np ? cur.a : nxt.a;
         const __amdgpu_buffer_rsrc_t db = pb < np ? cur.b : nxt.b;
-        step(Odd{}, std::false_type{}, std::true_type{}, A3 ? next3(sa) : s ^ 1, s ^ 1, ra, s, pa < np ? pa : pa - np,
+        step(Odd{}, std::false_type{}, OddDma{}, A3 ? next3(sa) : s ^ 1, s ^ 1, ra, s, pa < np ? pa : pa - np,
              pb < np ? pb : pb - np, da, db);
         ++pairs_done;
         sa = next3(sa);
@@ -812,6 +833,11 @@ __device__ __forceinline__ void pair_tiles(const TileHead& head, int tiles_n, in
       // the other half's waves: same barriers, same share of the DMA, no operand reads and no MFMAs
       for (int p = 0; p < np; ++p) {
         const int s = pairs_done & 1;
+        if (SPREAD) {
+          const __amdgpu_buffer_rsrc_t ea = p + 2 < np ? cur.a : nxt.a;
+#pragma unroll
+          for (int q = 0; q < 4; ++q) issue_a(sa == 0 ? 2 : sa - 1, p + 2 < np ? p + 2 : p + 2 - np, ea, q);
+        }
         if (first_tile || p >= 1) {
           if (A3) wait_vmcnt<4>();
           else wait_vmcnt<0>();
@@ -820,9 +846,13 @@ __device__ __forceinline__ void pair_tiles(const TileHead& head, int tiles_n, in
         const int pa = A3 ? p + 3 : p + 2, pb = p + 2;
         const __amdgpu_buffer_rsrc_t da = pa < np ? cur.a : nxt.a;
         const __amdgpu_buffer_rsrc_t db = pb < np ? cur.b : nxt.b;
+        if (SPREAD) {
 #pragma unroll
-        for (int q = 0; q < 8; ++q)
-          issue1(A3 ? sa : s, s, pa < np ? pa : pa - np, pb < np ? pb : pb - np, da, db, q);
+          for (int q = 0; q < 4; ++q) issue_b(s, pb < np ? pb : pb - np, db, q);
+        } else {
+#pragma unroll
+          for (int q = 0; q < 8; ++q) issue1(A3 ? sa : s, s, pa < np ? pa : pa - np, pb < np ? pb : pb - np, da, db, q);
+        }
         ++pairs_done;
         sa = next3(sa);
       }
@@ -879,10 +909,10 @@ __device__ __forceinline__ void pair_tiles(const TileHead& head, int tiles_n, in
 #endif
 }
 
-template <bool GELU, int MI, bool NT, bool A3 = false>
+template <bool GELU, int MI, bool NT, PairRing RING = PairRing::kTwo>
 __global__ __launch_bounds__(kPThreads) void gemm_f16_pair_kernel(ET_HEAD_ARGS, GemmArgs args) {
   extern __shared__ __attribute__((aligned(1024))) unsigned char smem[];
-  pair_tiles<GELU, MI, NT, A3>(tile_head(a0, b0, rows_dev, m_bound, n, k, groups, args), tiles_n, columns, walk, args, smem);
+  pair_tiles<GELU, MI, NT, RING>(tile_head(a0, b0, rows_dev, m_bound, n, k, groups, args), tiles_n, columns, walk, args, smem);
 }
 
 // Tile height of a launch of `wgs` workgroups per XCD, as 16-row blocks per wave: see launch_f16_persistent.
@@ -1169,8 +1199,9 @@ __global__ __launch_bounds__(kHThreads) __attribute__((amdgpu_waves_per_eu(2))) 
 // 45 us).  Below 128 tiles of 256 rows, where the host would not have launched it, the rows go to tiles with a CU to themselves as
 // far as one round of them lasts, by half of the wavefronts (FFN-down of 6900 rows in a launch for 11501: 36 us, 49 on the lowest
 // tiles of this kernel; attention output 14.6 and 17.6; FFN-down of 2300 rows 18.6 and 46).
-template <bool GELU, bool NT, bool A3>
+template <bool GELU, bool NT, PairRing RING>
 __global__ __launch_bounds__(kPThreads) void gemm_f16_pair_rows_kernel(ET_HEAD_ARGS, GemmArgs args) {
+  constexpr PairRing kLow = RING == PairRing::kThreeA ? PairRing::kThreeASpread : PairRing::kTwo;      // of the low tiles
   extern __shared__ __attribute__((aligned(1024))) unsigned char smem[];
   const TileHead head = tile_head(a0, b0, rows_dev, m_bound, n, k, groups, args);
   if ((int)((unsigned)(head.rows + 255) / 256) * tiles_n * groups < 128) {
@@ -1188,13 +1219,13 @@ __global__ __launch_bounds__(kPThreads) void gemm_f16_pair_rows_kernel(ET_HEAD_A
   }
     ET_BT_CASE(2, 4, 4) ET_BT_CASE(3, 4, 4) ET_BT_CASE(4, 4, 4) ET_BT_CASE(4, 6, 3)
 #undef ET_BT_CASE
-    return pair_tiles<GELU, 5, NT, false>(head, tiles_n, columns, walk, args, smem);
+    return pair_tiles<GELU, 5, NT, kLow>(head, tiles_n, columns, walk, args, smem);
   }
   switch (pair_row_blocks(head.rows, tiles_n * groups, walk >> kWalkWgs)) {
-    case 8: return pair_tiles<GELU, 8, NT, A3>(head, tiles_n, columns, walk, args, smem);
-    case 7: return pair_tiles<GELU, 7, NT, A3>(head, tiles_n, columns, walk, args, smem);
-    case 6: return pair_tiles<GELU, 6, NT, false>(head, tiles_n, columns, walk, args, smem);
-    default: return pair_tiles<GELU, 5, NT, false>(head, tiles_n, columns, walk, args, smem);
+    case 8: return pair_tiles<GELU, 8, NT, RING>(head, tiles_n, columns, walk, args, smem);
+    case 7: return pair_tiles<GELU, 7, NT, RING>(head, tiles_n, columns, walk, args, smem);
+    case 6: return pair_tiles<GELU, 6, NT, kLow>(head, tiles_n, columns, walk, args, smem);
+    default: return pair_tiles<GELU, 5, NT, kLow>(head, tiles_n, columns, walk, args, smem);
   }
 }
 
@@ -1559,7 +1590,8 @@ int device_cu_count() {
 // of a tile falls much more slowly than its height (the B^T half of the operand stream, the DMA and the LDS traffic
 // stay): measured about 1.45 us per pair of k-steps at 256 rows and 1.3 us at 160, i.e. proportional to MI + 21.  A
 // lower tile must win 3 % by that estimate (measured: FFN-down of 13097 rows 75 -> 64 us, of 15866 rows 76 -> 70 us,
-// attention-out 26 -> 24 us; the 13097 x 1024 one of BERT-large 35 -> 31.5 us; all with the same bits).
+// attention-out 26 -> 24 us; the 13097 x 1024 one of BERT-large 35 -> 31.5 us; all with the same bits.  Narrow outputs run lower
+// tiles 3 to 5 % faster since: kThreeASpread).
 int pair_kernel_row_blocks(int m_bound, int n, int groups) {
   return pair_row_blocks(m_bound, (n + kPBN - 1) / kPBN * groups, std::max(1, device_cu_count() / kXcds));
 }
@@ -1609,20 +1641,28 @@ void launch_f16_persistent(GemmArgs a, hipStream_t stream, bool b_transposed) {
   if (a.rows_dev != nullptr && !a.a_blocked && !a.c_blocked) {
     grid = device_cu_count() / kXcds * kXcds;
     auto go = [&](auto kern, int lds) { launch_pair(kern, lds, a, columns, grid, stream); };
-    if (a.gelu && a.c_cached) go(gemm_f16_pair_rows_kernel<true, false, false>, kQSmem);
-    else if (a.gelu) go(gemm_f16_pair_rows_kernel<true, true, false>, kQSmem);
-    else if (a.k >= 2048 && a.c_cached) go(gemm_f16_pair_rows_kernel<false, false, true>, kQSmemA3);
-    else if (a.k >= 2048) go(gemm_f16_pair_rows_kernel<false, true, true>, kQSmemA3);
-    else if (a.c_cached) go(gemm_f16_pair_rows_kernel<false, false, false>, kQSmem);
-    else go(gemm_f16_pair_rows_kernel<false, true, false>, kQSmem);
+    if (a.gelu && a.c_cached) go(gemm_f16_pair_rows_kernel<true, false, PairRing::kTwo>, kQSmem);
+    else if (a.gelu) go(gemm_f16_pair_rows_kernel<true, true, PairRing::kTwo>, kQSmem);
+    else if (a.k >= 2048 && a.c_cached) go(gemm_f16_pair_rows_kernel<false, false, PairRing::kThreeA>, kQSmemA3);
+    else if (a.k >= 2048) go(gemm_f16_pair_rows_kernel<false, true, PairRing::kThreeA>, kQSmemA3);
+    else if (a.c_cached) go(gemm_f16_pair_rows_kernel<false, false, PairRing::kTwo>, kQSmem);
+    else go(gemm_f16_pair_rows_kernel<false, true, PairRing::kTwo>, kQSmem);
     return;
   }
   // A from HBM, few long tiles per workgroup: the A rows are requested a pair earlier (three LDS slots for A)
   if (!a.gelu && a.k >= 2048 && mi >= 7) {
-    if (mi == 8 && !a.c_cached) launch_pair(gemm_f16_pair_kernel<false, 8, true, true>, kQSmemA3, a, columns, grid, stream);
-    else if (mi == 8) launch_pair(gemm_f16_pair_kernel<false, 8, false, true>, kQSmemA3, a, columns, grid, stream);
-    else if (!a.c_cached) launch_pair(gemm_f16_pair_kernel<false, 7, true, true>, kQSmemA3, a, columns, grid, stream);
-    else launch_pair(gemm_f16_pair_kernel<false, 7, false, true>, kQSmemA3, a, columns, grid, stream);
+    if (mi == 8 && !a.c_cached) launch_pair(gemm_f16_pair_kernel<false, 8, true, PairRing::kThreeA>, kQSmemA3, a, columns, grid, stream);
+    else if (mi == 8) launch_pair(gemm_f16_pair_kernel<false, 8, false, PairRing::kThreeA>, kQSmemA3, a, columns, grid, stream);
+    else if (!a.c_cached) launch_pair(gemm_f16_pair_kernel<false, 7, true, PairRing::kThreeA>, kQSmemA3, a, columns, grid, stream);
+    else launch_pair(gemm_f16_pair_kernel<false, 7, false, PairRing::kThreeA>, kQSmemA3, a, columns, grid, stream);
+    return;
+  }
+  // low tiles of a narrow output (see kThreeASpread)
+  if (!a.gelu && a.groups == 1 && a.n <= a.k && mi <= 6) {
+    if (mi == 6 && !a.c_cached) launch_pair(gemm_f16_pair_kernel<false, 6, true, PairRing::kThreeASpread>, kQSmemA3, a, columns, grid, stream);
+    else if (mi == 6) launch_pair(gemm_f16_pair_kernel<false, 6, false, PairRing::kThreeASpread>, kQSmemA3, a, columns, grid, stream);
+    else if (!a.c_cached) launch_pair(gemm_f16_pair_kernel<false, 5, true, PairRing::kThreeASpread>, kQSmemA3, a, columns, grid, stream);
+    else launch_pair(gemm_f16_pair_kernel<false, 5, false, PairRing::kThreeASpread>, kQSmemA3, a, columns, grid, stream);
     return;
   }
 #define ET_PAIR_CASE(M)                                                      \
