@@ -678,6 +678,61 @@ struct Unseen {
 };
 typedef uint32_t uint4x __attribute__((ext_vector_type(4)));
 
+// The work of workgroup `slot` of XCD `xcd`: a (sequence, head, block of `queries` queries).  Pairs of sequence (in the table's order, the
+// longest first) and head are dealt round-robin to the XCDs, whose L2 then fetches a pair's K and V once for all its blocks.
+// An XCD hands its workgroups to its shader engines strictly in turn, and one that ends at once leaves its place empty until
+// the turn comes round again: so the blocks behind a sequence's tokens come last (they hold queries only where the mask has
+// holes).  16 x 1024 positions, 11200 tokens, 12 heads: 3.3 -> 4 workgroups on a CU while there are any, 16 .. 71 -> 49 .. 62 stages
+// of keys a CU (12 layers 2776 -> 2753 us, fp32 15 x 379 2902 -> 2889; 6 layers of 16 heads, 64 x 512 with 32 .. 128 tokens 1144 -> 1061).
+// All of a wavefront's lanes; b < 0: nothing.
+struct QueryBlock {
+  int b, head, block, t0, t1;
+};
+constexpr int kPlacedBatch = kWave;        // sequences, one to a lane
+// More workgroups than four on every CU (fewer all start at once: 8 x 128 positions +0.7 % with it), and, as the kernel finds, about
+// 15 % of them without queries: a workgroup starts up to a microsecond later for it, with vector loads where the other way has
+// scalar ones (32 x 512 positions, 12 % without queries, +0.5 %).
+constexpr int kPlacedGrid = 1024;
+inline bool query_blocks_placed(int batch, int heads, int q_blocks) {
+  return q_blocks > 1 && batch <= kPlacedBatch && (long)batch * heads * q_blocks > kPlacedGrid;
+}
+template <bool PLACED>
+__device__ __forceinline__ QueryBlock query_block(const int32_t* __restrict__ seq_start, int batch, int heads, int q_blocks, int queries,
+                                                  int xcd, int slot) {
+  QueryBlock w{-1, 0, 0, 0, 0};
+  if (PLACED && 20 * (seq_start[batch] / queries) + 10 * batch < 17 * batch * q_blocks) {
+    const int lane = threadIdx.x & (kWave - 1);
+    const int b = min(max(seq_start[batch + 1 + min(lane, batch - 1)], 0), batch - 1);
+    const int t0 = seq_start[b], t1 = seq_start[b + 1];
+    // this XCD's pairs of the lane's sequence: 8 i + xcd from lane * heads on
+    const int first = (lane * heads - xcd + 7) >> 3, pairs = lane < batch ? (((lane + 1) * heads - xcd + 7) >> 3) - first : 0;
+    const int full = t1 > t0 ? min((t1 - t0 + queries - 1) / queries, q_blocks) : 0;
+    const int upto = wave_inclusive_scan_i32(pairs * full), total = __builtin_amdgcn_readlane(upto, kWave - 1);
+    const bool behind = slot >= total;
+    const int blocks = behind ? q_blocks - full : full;
+    const int end = behind ? total + wave_inclusive_scan_i32(pairs * blocks) : upto;
+    const uint64_t at = __ballot(slot < end);
+    if (at == 0) return w;
+    const int rank = __builtin_ctzll(at);
+    const int in_rank = slot - (__builtin_amdgcn_readlane(end, rank) - __builtin_amdgcn_readlane(pairs * blocks, rank));
+    const int per_pair = __builtin_amdgcn_readlane(blocks, rank), k = uniform_div(in_rank, per_pair);
+    w.b = __builtin_amdgcn_readlane(b, rank);
+    w.t0 = __builtin_amdgcn_readlane(t0, rank);
+    w.t1 = __builtin_amdgcn_readlane(t1, rank);
+    w.head = (__builtin_amdgcn_readlane(first, rank) + k) * 8 + xcd - rank * heads;
+    w.block = in_rank - k * per_pair + (behind ? __builtin_amdgcn_readlane(full, rank) : 0);
+    return w;
+  }
+  const int pair_of_xcd = uniform_div(slot, q_blocks), pair = pair_of_xcd * 8 + xcd;
+  if (pair >= batch * heads) return w;
+  const int place = uniform_div(pair, heads);
+  w.head = pair - place * heads;
+  w.block = slot - pair_of_xcd * q_blocks;
+  w.b = min(max(seq_start[batch + 1 + place], 0), batch - 1);
+  w.t0 = seq_start[w.b], w.t1 = seq_start[w.b + 1];
+  return w;
+}
+
 template <typename T>
 __global__ __launch_bounds__(256) void mask_class_kernel(const T* __restrict__ attr_mask, const int32_t* __restrict__ seq_start,
                                                          const int32_t* __restrict__ word_idx, int seq_len, int blocks,
@@ -697,7 +752,7 @@ __device__ __forceinline__ half4 read_transposed(const unsigned char* p) {
 #endif
 }
 
-template <int QSUB>
+template <int QSUB, bool PLACED>
 __global__ __launch_bounds__(kFlWaves * kWave, 4) void attention_flash_kernel(
     const int32_t* __restrict__ seq_start, int batch, int heads, int q_blocks, int seq_len, int layout, int packed_ld,
     const _Float16* __restrict__ q_src, const _Float16* __restrict__ k_src, const _Float16* __restrict__ v_src,
@@ -710,14 +765,9 @@ __global__ __launch_bounds__(kFlWaves * kWave, 4) void attention_flash_kernel(
   unsigned char* kv = smem_raw;                                        // [stage][K, V]
   int* tok_of_pos = reinterpret_cast<int*>(smem_raw + 2 * 2 * kFlStage);
 
-  // The query blocks of one (head, sequence) go to one XCD, whose L2 then fetches their K and V once: workgroup ids are
-  // dealt round-robin to the XCDs, pair p = 8 * (slot / q_blocks) + xcd.
-  const int xcd = blockIdx.x & 7, slot_id = blockIdx.x >> 3;
-  const int pair_of_xcd = uniform_div(slot_id, q_blocks), pair = pair_of_xcd * 8 + xcd, qblock = slot_id - pair_of_xcd * q_blocks;
-  if (pair >= batch * heads) return;
-  const int place = uniform_div(pair, heads), head = pair - place * heads;
-  const int b = min(max(seq_start[batch + 1 + place], 0), batch - 1);
-  const int t0 = seq_start[b], t1 = seq_start[b + 1];
+  const QueryBlock work = query_block<PLACED>(seq_start, batch, heads, q_blocks, 16 * kFlWaves * QSUB, blockIdx.x & 7, blockIdx.x >> 3);
+  if (work.b < 0) return;
+  const int b = work.b, head = work.head, qblock = work.block, t0 = work.t0, t1 = work.t1;
   const int len = t1 - t0;
   if (len <= 0) return;
   const int H = heads * kD;
@@ -1073,8 +1123,10 @@ void attention_flash_launch(const void* q, const void* k, const void* v, int lay
                             const uint8_t* mask_class, void* dst, const int32_t* seq_start, const int32_t* word_idx,
                             int batch, int seq_len, int heads, float scaler, hipStream_t stream) {
   const int pairs8 = (batch * heads + 7) / 8 * 8;
-  auto go = [&](auto kern, int queries) {
-    const int q_blocks = (seq_len + queries - 1) / queries;
+  auto go = [&](auto qsub) {
+    constexpr int QSUB = decltype(qsub)::value;
+    const int queries = 16 * kFlWaves * QSUB, q_blocks = (seq_len + queries - 1) / queries;
+    auto kern = query_blocks_placed(batch, heads, q_blocks) ? attention_flash_kernel<QSUB, true> : attention_flash_kernel<QSUB, false>;
     allow_dynamic_lds(reinterpret_cast<const void*>(kern), kFlSmem);
     kern<<<pairs8 * q_blocks, kFlWaves * kWave, kFlSmem, stream>>>(
         seq_start, batch, heads, q_blocks, seq_len, layout, packed_ld, (const _Float16*)q, (const _Float16*)k, (const _Float16*)v, word_idx,
@@ -1082,8 +1134,8 @@ void attention_flash_launch(const void* q, const void* k, const void* v, int lay
   };
   // Two query tiles per wavefront halve the LDS reads per score; with few workgroups the CUs are better filled by twice as
   // many of one tile.
-  if ((long)batch * heads * ((seq_len + 127) / 128) >= 2L * attention_cu_count()) go(attention_flash_kernel<2>, 128);
-  else go(attention_flash_kernel<1>, 64);
+  if ((long)batch * heads * ((seq_len + 127) / 128) >= 2L * attention_cu_count()) go(std::integral_constant<int, 2>{});
+  else go(std::integral_constant<int, 1>{});
 }
 
 // ------------------------------------------------------------------------------------------
@@ -1124,6 +1176,7 @@ __device__ __forceinline__ void piece_products(F&& mfma) {
   mfma(1, 1); mfma(0, 2); mfma(2, 0); mfma(0, 1); mfma(1, 0); mfma(0, 0);
 }
 
+template <bool PLACED>
 __global__ __launch_bounds__(kAttnThreads, 4) void attention_flash_f32_kernel(
     const int32_t* __restrict__ seq_start, int batch, int heads, int q_blocks, int seq_len, int layout, int packed_ld,
     const float* __restrict__ q_src, const float* __restrict__ k_src, const float* __restrict__ v_src,
@@ -1134,13 +1187,9 @@ __global__ __launch_bounds__(kAttnThreads, 4) void attention_flash_f32_kernel(
   unsigned char* kv = smem_raw;                                        // [K, V][piece][key][64]
   int* tok_of_pos = reinterpret_cast<int*>(smem_raw + 2 * 3 * kF32Piece);
 
-  // the query blocks of one (head, sequence) go to one XCD, as above
-  const int xcd = blockIdx.x & 7, slot_id = blockIdx.x >> 3;
-  const int pair_of_xcd = uniform_div(slot_id, q_blocks), pair = pair_of_xcd * 8 + xcd, qblock = slot_id - pair_of_xcd * q_blocks;
-  if (pair >= batch * heads) return;
-  const int place = uniform_div(pair, heads), head = pair - place * heads;
-  const int b = min(max(seq_start[batch + 1 + place], 0), batch - 1);
-  const int t0 = seq_start[b], t1 = seq_start[b + 1];
+  const QueryBlock work = query_block<PLACED>(seq_start, batch, heads, q_blocks, 64, blockIdx.x & 7, blockIdx.x >> 3);
+  if (work.b < 0) return;
+  const int b = work.b, head = work.head, qblock = work.block, t0 = work.t0, t1 = work.t1;
   const int len = t1 - t0;
   if (len <= 0) return;
   const int H = heads * kD;
@@ -1439,7 +1488,8 @@ void attention_flash_f32_launch(const void* q, const void* k, const void* v, int
                                 hipStream_t stream) {
   const int q_blocks = (seq_len + 63) / 64;
   const int grid = (batch * heads + 7) / 8 * 8 * q_blocks;
-  attention_flash_f32_kernel<<<grid, kAttnThreads, kF32Smem, stream>>>(
+  auto kern = query_blocks_placed(batch, heads, q_blocks) ? attention_flash_f32_kernel<true> : attention_flash_f32_kernel<false>;
+  kern<<<grid, kAttnThreads, kF32Smem, stream>>>(
       seq_start, batch, heads, q_blocks, seq_len, layout, packed_ld, (const float*)q, (const float*)k, (const float*)v, word_idx,
       (const float*)attr_mask, mask_class, (float*)dst, scaler, out, head_exp);
 }
