@@ -20,7 +20,7 @@
 // its chunks where it adds them up (20375 rows, attention and product: 141 us with a launch in between that found the rows' own
 // exponents, 130 us; 3820 rows 57 and 53; one tile's worth, 160 rows, level; encoders of 12 layers 1 to 2 %).  Weights
 // are taken anew by every layer call: pair_weight_top_kernel looks for the largest value of each column, pair_weight_kernel
-// writes the rows (9 + 11.5 us per layer of BERT-base, split rows 15).
+// writes the rows (8.4 + 10.2 us per layer of BERT-base, split rows 15).
 // Bound: at large m the power limit of the matrix cores (20375 rows, k = 768 / n = 2304, 768, 3072 + GELU and k = 3072 / n = 768:
 // 180, 71, 270, 233 us in the layer, 1070 .. 1240 TFLOP/s of 16-bit products; split rows 307, 112, 451, 413); below a round of the
 // chip the k loop of one tile (134 rows: 10.2, 6.5, 12.8, 14.3 us against 15.2, 8.7, 16.1, 21.3).
@@ -596,7 +596,7 @@ __global__ __launch_bounds__(256) void pair_rows_kernel(PairRowsJob job) {
 inline int pair_rows_grid(const PairRowsJob& job) { return std::min((job.m + 3) / 4, 2048) + (job.seq_table ? 1 : 0); }
 
 // Weights into n pair rows in two launches, whose loads are whole lines (one launch of workgroups that hold all k of 16 columns
-// took 35 .. 45 us at H = 768; exponents that go by chunks of 64 k and are applied where a chunk is added need one launch, and
+// took 35 .. 45 us at H = 768, of 32 columns with 4 x 8 values a lane 24: one workgroup a CU, whose reads and writes take turns; exponents that go by chunks of 64 k and are applied where a chunk is added need one launch, and
 // cost the products 3 to 20 %).  First the largest value of each column in blocks of 256 k, as [k / 256][n].
 struct PairWeightArgs {
   PairWeightJobs jobs;
@@ -684,52 +684,79 @@ __global__ __launch_bounds__(256) void pair_weight_top_kernel(PairWeightArgs arg
   }
 }
 
-// Then 64 x 64 tiles through LDS.
+// Then 64 x 64 tiles through LDS.  All workgroups are on the chip at once, so the launch takes as long as what stands in front of
+// a workgroup's stores: the tile's loads go out first, the columns' largest values behind them, a quarter of a column's to each
+// wavefront (28 MB at H = 768: 11.3 -> 10.2 us, 5.6 TB/s of reads and writes; one wavefront that went through a column's values
+// one by one before it asked for the tile; tiles on the XCD that read them in the launch before: 10.3).
 __global__ __launch_bounds__(256) void pair_weight_kernel(PairWeightArgs args) {
   __shared__ float tile[64][65];
   __shared__ float part[3][4];
-  __shared__ int exps[64];
+  __shared__ float tops[4][64];
   int job = 0;
   while (job + 1 < args.jobs.count && (int)blockIdx.x >= args.tile_begin[job + 1]) ++job;
   const PairWeightJob& jb = args.jobs.job[job];
   const int K = jb.k, N = jb.n, tiles_n = (N + 63) / 64;
   const int t = blockIdx.x - args.tile_begin[job];
   const int chunk = t / tiles_n, k0 = chunk * 64, n0 = (t - chunk * tiles_n) * 64;
-  if (threadIdx.x < 64 && n0 + (int)threadIdx.x < N) {
+  auto find_tops = [&]() {
+    const int wave = threadIdx.x / kWave, c = threadIdx.x & (kWave - 1), blocks = (K + kTopRows - 1) / kTopRows;
     float top = 0.f;
-    for (int b = 0; b < (K + kTopRows - 1) / kTopRows; ++b) top = fmaxf(top, jb.top[(size_t)b * N + n0 + threadIdx.x]);
-    exps[threadIdx.x] = pair_exponent(top);
-    if (chunk == 0) jb.exp[n0 + threadIdx.x] = exps[threadIdx.x];
-  }
+    if (n0 + c < N) {
+      for (int b0 = 0; b0 < blocks; b0 += 16) {  // (blocks past the last one: the last one again)
+        float v[4];
+#pragma unroll
+        for (int u = 0; u < 4; ++u) v[u] = jb.top[(size_t)min(b0 + 4 * u + wave, blocks - 1) * N + n0 + c];
+#pragma unroll
+        for (int u = 0; u < 4; ++u) top = fmaxf(top, v[u]);
+      }
+    }
+    tops[wave][c] = top;
+  };
   if (jb.src_split) {                            // rows of three bfloat16 pieces, whose sum is the float
+    bf16x8 h[2], m[2], l[2];
 #pragma unroll
     for (int u = 0; u < 2; ++u) {
       const int i = threadIdx.x + u * 256, r = i >> 3, c = (i & 7) * 8;      // row n0+r, k0+c ..
       if (n0 + r >= N) continue;
       const __bf16* p = (const __bf16*)jb.src + (size_t)(n0 + r) * K * 3 + ((k0 + c) >> 5) * 96 + (c & 31);
-      const bf16x8 h = *reinterpret_cast<const bf16x8*>(p), m = *reinterpret_cast<const bf16x8*>(p + 32),
-                   l = *reinterpret_cast<const bf16x8*>(p + 64);
+      h[u] = *reinterpret_cast<const bf16x8*>(p);
+      m[u] = *reinterpret_cast<const bf16x8*>(p + 32);
+      l[u] = *reinterpret_cast<const bf16x8*>(p + 64);
+    }
+    find_tops();
 #pragma unroll
-      for (int j = 0; j < 8; ++j) tile[r][c + j] = ((float)h[j] + (float)m[j]) + (float)l[j];
+    for (int u = 0; u < 2; ++u) {
+      const int i = threadIdx.x + u * 256, r = i >> 3, c = (i & 7) * 8;
+      if (n0 + r >= N) continue;
+#pragma unroll
+      for (int j = 0; j < 8; ++j) tile[r][c + j] = ((float)h[u][j] + (float)m[u][j]) + (float)l[u][j];
     }
   } else {
     const float* __restrict__ src = (const float*)jb.src;
+    float4v v[4];
 #pragma unroll
     for (int u = 0; u < 4; ++u) {
       const int i = threadIdx.x + u * 256, r = i >> 4, c = (i & 15) * 4;     // source row k0+r, columns n0+c ..
-      float4v v = {};
-      if (n0 + c < N) v = *reinterpret_cast<const float4v*>(src + (size_t)(k0 + r) * N + n0 + c);
+      v[u] = float4v{0.f, 0.f, 0.f, 0.f};
+      if (n0 + c < N) v[u] = *reinterpret_cast<const float4v*>(src + (size_t)(k0 + r) * N + n0 + c);
+    }
+    find_tops();
 #pragma unroll
-      for (int j = 0; j < 4; ++j) tile[c + j][r] = v[j];
+    for (int u = 0; u < 4; ++u) {
+      const int i = threadIdx.x + u * 256, r = i >> 4, c = (i & 15) * 4;
+#pragma unroll
+      for (int j = 0; j < 4; ++j) tile[c + j][r] = v[u][j];
     }
   }
   __syncthreads();
+  auto exponent = [&](int r) { return pair_exponent(fmaxf(fmaxf(tops[0][r], tops[1][r]), fmaxf(tops[2][r], tops[3][r]))); };
+  if (chunk == 0 && threadIdx.x < 64 && n0 + (int)threadIdx.x < N) jb.exp[n0 + threadIdx.x] = exponent(threadIdx.x);
   float norm = 0.f, bias = 0.f, above = 0.f;
 #pragma unroll
   for (int u = 0; u < 2; ++u) {
     const int i = threadIdx.x + u * 256, r = i >> 3, c = (i & 7) * 8;        // row n0+r of the result, k0+c ..
     if (n0 + r >= N) continue;                   // (whole groups of eight lanes)
-    const int e = exps[r];
+    const int e = exponent(r);
     const float by = pair_scale(e);
     float sq = 0.f;
     half8 h, l;
