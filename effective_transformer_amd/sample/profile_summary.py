@@ -37,6 +37,7 @@ def describe(workload: str) -> str:
 
 def short(name: str) -> str:
     n = re.sub(r"\(anonymous namespace\)::", "", name)
+    n = re.sub(r"\(et::(\w+)\)(\d)", r"\1 \2", n)               # a template argument that is an enumerator
     n = re.sub(r"^void ", "", n)
     m = re.match(r"_ZN2et12_GLOBAL__N_1\d+([a-z_0-9]+)I(.*?)EEv", n)
     if m:
