@@ -247,6 +247,20 @@ __device__ __forceinline__ void store_head_pairs(float* dst, int row, int H, int
 #endif
 }
 
+// What a launch leaves in dst, as its last argument.  fp16 has one form only, and its instances take no more than that: the host
+// issues an encoder of few rows more slowly than the device runs it, and its time goes by the bytes of the arguments too (1 x 32
+// positions, 12 layers: 375 us with the 16 of the exponents, 364 without).
+template <typename T>
+struct AttnOut {
+  AttentionOut form = AttentionOut::kPlain;
+  int exp_stride = 0;
+  int8_t* exp = nullptr;
+};
+template <>
+struct AttnOut<_Float16> {
+  AttentionOut form = AttentionOut::kPlain;
+};
+
 // WAVES: wavefronts per workgroup, one 16-query tile each.  CPT = 16-byte chunks of
 // one matrix a thread moves per head (ceil(seq rows * chunks per row / threads)).
 template <typename T, int NKT, int WAVES, int CPT>
@@ -254,7 +268,7 @@ __global__ __launch_bounds__(WAVES * kWave) void attention_kernel(
     // (the first 14 words come in registers: what the chain order -> start table -> positions and rows needs)
     const int32_t* __restrict__ seq_start, const int32_t* __restrict__ word_idx, int batch, int seq_len, int heads, int heads_per_wg,
     int layout, int packed_ld, const T* __restrict__ q_src, const T* __restrict__ k_src, const T* __restrict__ v_src,
-    const T* __restrict__ attr_mask, T* __restrict__ dst, float scaler, AttentionOut out, HeadExps head_exp) {
+    const T* __restrict__ attr_mask, T* __restrict__ dst, float scaler, AttnOut<T> out) {
   using Cfg = AttnCfg<T>;
   using Sm = AttnSmem<T, NKT>;
   using C = Chunk16<T>;
@@ -378,7 +392,7 @@ __global__ __launch_bounds__(WAVES * kWave) void attention_kernel(
   // where this lane's query writes its output row (head 0; null without a token): the same for every head
   const int tq = wave < n_tiles && wave < NKT ? tok_of_pos[wave * 16 + l16] : -1;
   T* out_row = tq >= 0 ? dst + (size_t)tq * H + g * (sizeof(T) == 2 ? 16 : 4) : nullptr;
-  if (sizeof(T) == 4 && out == AttentionOut::kSplit && tq >= 0)
+  if (sizeof(T) == 4 && out.form == AttentionOut::kSplit && tq >= 0)
     out_row = reinterpret_cast<T*>(reinterpret_cast<uint16_t*>(dst) + (size_t)tq * 3 * H);
 
   for (int head = h_begin; head < h_end; ++head) {
@@ -523,8 +537,8 @@ __global__ __launch_bounds__(WAVES * kWave) void attention_kernel(
         }
       }
       if constexpr (sizeof(T) == 4) {
-        if (out == AttentionOut::kPairs) {       // (uniform)
-          store_head_pairs<false>(dst, tq, H, head, o, head_exp);
+        if (out.form == AttentionOut::kPairs) {  // (uniform)
+          store_head_pairs<false>(dst, tq, H, head, o, HeadExps{out.exp, out.exp_stride});
           continue;
         }
       }
@@ -551,7 +565,7 @@ __global__ __launch_bounds__(WAVES * kWave) void attention_kernel(
             out4 v;
 #pragma unroll
             for (int r = 0; r < 4; ++r) v[r] = (T)o[dt][r];
-            if (out == AttentionOut::kSplit) store_split<4>(reinterpret_cast<uint16_t*>(out_row), head * kD + dt * 16 + g * 4, v);
+            if (out.form == AttentionOut::kSplit) store_split<4>(reinterpret_cast<uint16_t*>(out_row), head * kD + dt * 16 + g * 4, v);
             else *reinterpret_cast<out4*>(orow + dt * 16) = v;
           }
         }
@@ -585,8 +599,11 @@ void attention_launch(const void* q, const void* k, const void* v, int layout, i
       break;
     }
   dim3 grid((heads + hpw - 1) / hpw, batch);
+  AttnOut<T> form;
+  form.form = out;
+  if constexpr (sizeof(T) == 4) form.exp = head_exp.exp, form.exp_stride = head_exp.stride;
   kern<<<grid, kThreads, Sm::kBytes, stream>>>(seq_start, word_idx, batch, seq_len, heads, hpw, layout, packed_ld, (const T*)q,
-                                               (const T*)k, (const T*)v, (const T*)attr_mask, (T*)dst, scaler, out, head_exp);
+                                               (const T*)k, (const T*)v, (const T*)attr_mask, (T*)dst, scaler, form);
 }
 
 
