@@ -547,8 +547,9 @@ void launch_tile(PairGemmArgs a, bool gelu, int groups, const uint32_t* head_exp
   // (a stream of fewer stages than the ring holds must not cross into a second tile)
   const int grid = ((a.k / (32 * KS) < ST ? tiles : std::min(tiles, device_cu_count())) + kXcds - 1) / kXcds * kXcds;
   auto go = [&](auto kern) {
-    const int lds = Tile::SMEM + (head_exp ? Tile::BM * (4 + 2 * (a.k / 64)) : 0);
-    allow_dynamic_lds(reinterpret_cast<const void*>(kern), lds);
+    auto exps = [&](int chunks) { return head_exp ? Tile::BM * (4 + 2 * chunks) : 0; };
+    const int lds = Tile::SMEM + exps(a.k / 64);
+    allow_dynamic_lds(reinterpret_cast<const void*>(kern), std::min(Tile::SMEM + exps(kMaxHeadExps), 160 * 1024));
     kern<<<grid, Tile::THREADS, lds, stream>>>(a.A[0], a.B[0], a.rows_dev, a.m_bound, a.n, a.k, a.tiles_n, groups, a.columns, head_exp, a);
   };
   if (gelu) go(gemm_pair_kernel<WM, WN, MI, NJ, ST, KS, true, false>);

@@ -1,0 +1,58 @@
+"""What the library asks the runtime to launch, without a device: launch_recorder.cpp stands in for the HIP runtime."""
+import os
+import subprocess
+import sys
+
+import pytest
+
+from effective_transformer_amd import build
+
+HERE = os.path.dirname(os.path.abspath(__file__))
+
+# fp32 layers in the order given, a line of output per launch (no device memory is touched, so any address does)
+LAYERS = """
+import ctypes as C, sys
+recorder = C.CDLL(sys.argv[1], mode=C.RTLD_GLOBAL)
+recorder.recorded_launches.restype = C.c_char_p
+sys.path.insert(0, sys.argv[2])
+from effective_transformer_amd import _lib
+lib = _lib.load()
+handle = C.c_void_p()
+assert lib.et_create(C.byref(handle), 0) == 0, lib.et_last_error(None)
+some = C.c_void_p(1 << 40)
+weights = _lib.LayerWeights(*[1 << 40] * len(_lib.WEIGHT_FIELDS))
+for heads, batch, seq, rows in eval(sys.argv[3]):
+    nbytes = lib.et_layer_workspace_bytes(_lib.ET_FP32, batch, seq, heads, 64)
+    s = lib.et_layer(handle, _lib.ET_FP32, C.byref(weights), some, some, some, some, some, some, C.c_void_p(1 << 41), batch, seq, seq,
+                     heads, 64, rows, C.c_void_p(1 << 42), nbytes, None)
+    assert s == 0, lib.et_last_error(handle)
+print(recorder.recorded_launches().decode(), end="")
+"""
+
+
+@pytest.fixture(scope="module")
+def recorder(tmp_path_factory):
+    out = str(tmp_path_factory.mktemp("recorder") / "librecorder.so")
+    # (host code alone, and no runtime of its own beside it)
+    subprocess.run([build.hipcc(), "-std=c++17", "-O1", "-shared", "-fPIC", "--offload-host-only", "-no-hip-rt", "-x", "hip",
+                    os.path.join(HERE, "launch_recorder.cpp"), "-o", out], check=True, capture_output=True)
+    return out
+
+
+def _launches(recorder, layers, cus=256):
+    """[(kernel, workgroups, dynamic LDS, size raised)] of fp32 layers (heads, batch, seq, rows) in a process of their own."""
+    r = subprocess.run([sys.executable, "-c", LAYERS, recorder, os.path.dirname(HERE), repr(layers)], capture_output=True, text=True,
+                       env=dict(os.environ, RECORDER_CUS=str(cus)), timeout=120)
+    assert r.returncode == 0, r.stderr
+    found = [line.split() for line in r.stdout.splitlines()]
+    assert len(found) >= 8 * len(layers)
+    return [(name, int(wgs), int(lds), int(raised)) for name, wgs, lds, raised in found]
+
+
+# rows for every height of tile
+@pytest.mark.parametrize("rows", [30, 200, 900, 3000, 8000, 30000])
+@pytest.mark.parametrize("heads", [(8, 12, 29, 30, 31, 32), (32, 31, 30, 8)])
+def test_no_launch_takes_more_lds_than_its_kernel_was_given(recorder, heads, rows):
+    """The output product's LDS grows with the hidden size: whatever size came first, the next one's must have been asked for."""
+    for name, _, lds, raised in _launches(recorder, [(h, 1000, 32, rows) for h in heads]):
+        assert lds <= max(raised, 64 * 1024), "%s: %d bytes of LDS, %d asked for" % (name, lds, raised)
