@@ -1158,34 +1158,48 @@ void attention_flash_launch(const void* q, const void* k, const void* v, int lay
 // ------------------------------------------------------------------------------------------
 // fp32 fused attention for 32 < seq_len <= 1024, built like the kernel above: one workgroup of 4 wavefronts per (64 queries, head,
 // sequence), 16 queries per wavefront, K and V in stages of 32 keys, the softmax along with them in floats.  The products run on
-// the 16-bit matrix instructions with every float as the exact sum of three bfloat16 pieces (round_pair_bf16): six of the nine
+// the 16-bit matrix instructions with every float as the sum of three bfloat16 pieces (round_pair_bf16): six of the nine
 // products of pieces, the others at most 2^-24 of the largest.  A float MFMA takes 16 times as long per product.
 // The pieces of K and V are made once per workgroup: a thread brings eight floats of a key's K and of its V into registers under
 // the stage in front, splits them and writes them to LDS in rows of 64 values per piece, laid out as in the fp16 kernel (which
 // explains the order of the keys).
-// Bound: a wavefront and stage issue 768 cycles of MFMA and about 900 of VALU (352 of them the split of K and V, 180 that of the
+// Bound: a wavefront and stage issue 768 cycles of MFMA and about 950 of VALU (370 of them the split of K and V, 210 that of the
 // probabilities, exp2 at a quarter of the rate), 24 KB of LDS reads; short sequences the start of a workgroup.  One stage in LDS
 // and the next in registers take two barriers a stage, but leave room for four workgroups per CU.  15 x 379 positions / 3820
 // tokens, 12 heads: 47.0 -> 32.0 us per launch against floats on v_mfma_f32_16x16x4_f32 (2048 cycles of MFMA a stage), 500 x 64 /
-// 20375 tokens 64.8 -> 53.1 (33.1 and 59.8 where the result is left as pair rows).  32 queries per wavefront: 35 and 73 us; three wavefronts per SIMD instead of four: 34 and 60.
+// 20375 tokens 64.8 -> 53.1 (33.1 and 59.8 where the result is left as pair rows).  32 queries per wavefront: 35 and 73 us; three
+// wavefronts per SIMD instead of four: 34 and 60.
 // Relative error against float64 (this / the float instructions), normal operands: 64 positions 1.59e-7 / 2.44e-7, 379 3.01e-7 /
-// 4.00e-7, 1000 5.27e-7 / 6.47e-7; with scores nine times as wide 3.9e-7 / 6.4e-7, 6.2e-7 / 9.9e-7, 7.6e-7 / 1.14e-6.  An infinity
-// gives NaN, as does a magnitude above 3.38e38.
+// 4.00e-7, 1000 5.27e-7 / 6.47e-7; with scores nine times as wide 3.9e-7 / 6.4e-7, 6.2e-7 / 9.9e-7, 7.6e-7 / 1.14e-6.
+//
+// Three pieces are not every float: below 2^-110 the last one ends at 2^-133, the first one is infinite above 3.39e38, and an
+// infinity leaves NaN.  A workgroup that meets such operands does its block once more with the float instructions (FLOATS):
+//   V with bits below 2^-133;  Q with such bits, or of 2^60 and more (below that, K's bits below 2^-133 move a score by 2^-67);
+//   a result that is not finite, which is what an operand without three pieces leaves, as do sums that overflow.
+// Probabilities are split 2^24 times as large, where those down to v_exp_f32's smallest have all their bits.  Looking costs nothing
+// that shows (in the layer 30.9 and 60.7 us a launch before, 30.8 and 60.1 with it), the 2^24 1 % (30.8 -> 31.3).  Where every block
+// is done twice the launches take 74 and 106 us, 48 and 63 with the float instructions alone.
 // ------------------------------------------------------------------------------------------
 constexpr int kF32Keys = 32;                                 // keys per stage
 constexpr int kF32Piece = kF32Keys * kD * 2;                 // bytes of a piece of K (and of V) per stage
-// Up to 32 positions attention_kernel is ahead where there are many sequences, because its workgroups serve several heads for one
-// start (per launch, 12 heads, this kernel second: 1000 x 16 32.2 and 51.3 us, 1000 x 31 52.9 and 66.3, 100 x 20 9.3 and 9.4, 200 x 32
-// 19.1 and 17.0, 8 x 32 5.8 and 5.1).
+// Up to 32 positions attention_kernel, whose workgroups serve several heads for one start.  What decides between the two is the
+// number of sequences more than their length (per launch, 12 heads, this kernel second: 1000 x 16 32.2 and 51.3 us, 1000 x 31 52.9
+// and 66.3, 100 x 20 9.3 and 9.4, but 200 x 32 19.1 and 17.0, 8 x 32 5.8 and 5.1); the rule goes by the length alone.
 constexpr int kF32MinKeys = 32;
-constexpr int kF32Smem = 2 * 3 * kF32Piece + kFlMaxKeys * (int)sizeof(int);
+[[maybe_unused]] constexpr float kF32TopQ = 0x1p60f, kF32Raise = 0x1p24f;
+constexpr int kF32Smem = 2 * 3 * kF32Piece + (kFlMaxKeys + 4) * (int)sizeof(int);
 typedef __bf16 bf16x8 __attribute__((ext_vector_type(8)));
-// eight floats as three pieces; x keeps the rests
-__device__ __forceinline__ void split_eight(float (&x)[8], uint4x (&piece)[3]) {
+// eight floats as three pieces; `rest` collects what the third ones are made of, whose low 16 bits they do not hold
+__device__ __forceinline__ void split_eight(float (&x)[8], uint4x (&piece)[3], uint32_t& rest) {
 #pragma unroll
-  for (int i = 0; i < 3; ++i)
+  for (int i = 0; i < 3; ++i) {
+    if (i == 2) {
+#pragma unroll
+      for (int j = 0; j < 8; ++j) rest |= __builtin_bit_cast(uint32_t, x[j]);
+    }
 #pragma unroll
     for (int j = 0; j < 4; ++j) piece[i][j] = round_pair_bf16(x[2 * j], x[2 * j + 1]);
+  }
 }
 // a . b of three pieces each, smallest products first
 template <typename F>
@@ -1193,16 +1207,17 @@ __device__ __forceinline__ void piece_products(F&& mfma) {
   mfma(1, 1); mfma(0, 2); mfma(2, 0); mfma(0, 1); mfma(1, 0); mfma(0, 0);
 }
 
-template <bool PLACED>
-__global__ __launch_bounds__(kAttnThreads, 4) void attention_flash_f32_kernel(
-    const int32_t* __restrict__ seq_start, int batch, int heads, int q_blocks, int seq_len, int layout, int packed_ld,
+// FLOATS: on the float instructions; tid: threadIdx.x
+template <bool PLACED, bool FLOATS>
+__device__ __forceinline__ void flash_f32_block(
+    int tid, const int32_t* __restrict__ seq_start, int batch, int heads, int q_blocks, int seq_len, int layout, int packed_ld,
     const float* __restrict__ q_src, const float* __restrict__ k_src, const float* __restrict__ v_src,
     const int32_t* __restrict__ word_idx, const float* __restrict__ attr_mask, const uint8_t* __restrict__ mask_class,
-    float* __restrict__ dst, float scaler, AttentionOut out, HeadExps head_exp) {
+    float* __restrict__ dst, float scaler, AttentionOut out, HeadExps head_exp, unsigned char* smem_raw) {
 #if defined(__HIP_DEVICE_COMPILE__)   // device-only types in the body; the host pass only needs the stub
-  extern __shared__ __attribute__((aligned(1024))) unsigned char smem_raw[];
   unsigned char* kv = smem_raw;                                        // [K, V][piece][key][64]
   int* tok_of_pos = reinterpret_cast<int*>(smem_raw + 2 * 3 * kF32Piece);
+  int* votes = tok_of_pos + kFlMaxKeys;                                // a wavefront: its share is to be done again in floats
 
   const QueryBlock work = query_block<PLACED>(seq_start, batch, heads, q_blocks, 64, blockIdx.x & 7, blockIdx.x >> 3);
   if (work.b < 0) return;
@@ -1210,8 +1225,8 @@ __global__ __launch_bounds__(kAttnThreads, 4) void attention_flash_f32_kernel(
   const int len = t1 - t0;
   if (len <= 0) return;
   const int H = heads * kD;
-  const int lane = threadIdx.x & (kWave - 1);
-  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x / kWave);
+  const int lane = tid & (kWave - 1);
+  const int wave = __builtin_amdgcn_readfirstlane(tid / kWave);
   const int l16 = lane & 15, g = lane >> 4;
   const int first_q = qblock * 64, q = first_q + wave * 16 + l16;
 
@@ -1221,7 +1236,7 @@ __global__ __launch_bounds__(kAttnThreads, 4) void attention_flash_f32_kernel(
 
   // this thread's eight features of K and of V: key `my_key` of the stage; a row without a token is requested beyond the
   // descriptor's range and arrives as zeros
-  const int my_key = threadIdx.x >> 3, my_chunk = threadIdx.x & 7;
+  const int my_key = tid >> 3, my_chunk = tid & 7;
   const uint32_t voff = ((uint32_t)my_key * ld + (uint32_t)my_chunk * 8u) * 4u;
   const uint32_t v_swap = (uint32_t)(my_key >> 1 & 1) * 16u;           // (see v_wr)
   float4v in[4];                                                       // K, V
@@ -1247,26 +1262,41 @@ __global__ __launch_bounds__(kAttnThreads, 4) void attention_flash_f32_kernel(
   // V is read transposed, four keys x four times four features 16 apart, so that a lane ends up with 16 consecutive features: chunks
   // are XORed with key bit 3, and key bit 1 swaps a chunk's halves (requested the other way round), which spreads a read over all banks
   unsigned char* const v_wr = kv + 3 * kF32Piece + my_key * 128 + ((my_chunk ^ (my_key >> 3 & 1)) * 16);
+  // FLOATS: K's and V's rows of 64 floats, their 16-byte chunks XORed so that an operand read covers all banks
+  auto write_floats = [&] {
+#pragma unroll
+    for (int i = 0; i < 2; ++i) {
+      const int ck = my_chunk * 2 + i, cv = my_chunk * 2 + (i ^ (my_key >> 1 & 1));
+      *reinterpret_cast<float4v*>(kv + my_key * 256 + ((ck ^ ((my_key >> 3) * 4 + (my_key & 3))) * 16)) = in[i];
+      *reinterpret_cast<float4v*>(kv + kF32Keys * 256 + my_key * 256 + ((cv ^ (my_key >> 3)) * 16)) = in[2 + i];
+    }
+  };
+  uint32_t rest_v = 0, rest_k = 0;                                     // (of K they do not matter)
   auto write = [&] {
+    if constexpr (FLOATS) {
+      write_floats();
+      return;
+    }
 #pragma unroll
     for (int m = 0; m < 2; ++m) {
       float x[8];
 #pragma unroll
       for (int j = 0; j < 8; ++j) x[j] = in[2 * m + (j >> 2)][j & 3];
       uint4x piece[3];
-      split_eight(x, piece);
+      split_eight(x, piece, m ? rest_v : rest_k);
 #pragma unroll
       for (int i = 0; i < 3; ++i) *reinterpret_cast<uint4x*>((m ? v_wr : k_wr) + i * kF32Piece) = piece[i];
     }
   };
   int tq;
-  float4v q_in[4];                                                     // features 8 g .. and 32 + 8 g .. of the lane's query
+  float4v q_in[4];                                                     // features 8 g .. and 32 + 8 g .. of the lane's query, FLOATS: 16 g ..
   auto request_q = [&](bool dense, int n) {
     tq = q < n ? (dense ? q : tok_of_pos[q]) : -1;
 #pragma unroll
     for (int i = 0; i < 4; ++i) {
       q_in[i] = float4v{0.f, 0.f, 0.f, 0.f};
-      if (tq >= 0) q_in[i] = *reinterpret_cast<const float4v*>(qb + (size_t)(layout == 1 ? tq : q) * ld + (i >> 1) * 32 + g * 8 + (i & 1) * 4);
+      const int at = FLOATS ? g * 16 + i * 4 : (i >> 1) * 32 + g * 8 + (i & 1) * 4;
+      if (tq >= 0) q_in[i] = *reinterpret_cast<const float4v*>(qb + (size_t)(layout == 1 ? tq : q) * ld + at);
     }
   };
 
@@ -1293,9 +1323,9 @@ __global__ __launch_bounds__(kAttnThreads, 4) void attention_flash_f32_kernel(
   const int stage_rows = dense || layout == 1 ? len : n;               // of the matrices behind kb, vb that exist
   if (first_q >= n) return;                                            // no token among this workgroup's queries
   if (!dense) {
-    for (int i = threadIdx.x; i < kFlMaxKeys; i += kAttnThreads) tok_of_pos[i] = -1;
+    for (int i = tid; i < kFlMaxKeys; i += kAttnThreads) tok_of_pos[i] = -1;
     __syncthreads();
-    for (int tt = threadIdx.x; tt < len; tt += kAttnThreads) {
+    for (int tt = tid; tt < len; tt += kAttnThreads) {
       const int pos = word_idx[t0 + tt];
       if (pos >= 0 && pos < seq_len) tok_of_pos[pos] = tt;             // relative to the sequence's first packed row
     }
@@ -1303,16 +1333,28 @@ __global__ __launch_bounds__(kAttnThreads, 4) void attention_flash_f32_kernel(
     request(0, false, stage_rows);
     request_q(false, n);
   }
-  bf16x8 bq[2][3];
+  uint4x bq[6];                                                        // [k-step][piece], or floats
+  bool again_q = false;
+  if constexpr (FLOATS) {
 #pragma unroll
-  for (int ks = 0; ks < 2; ++ks) {
-    float x[8];
+    for (int i = 0; i < 4; ++i) bq[i] = __builtin_bit_cast(uint4x, q_in[i]);
+  } else {
+    uint32_t rest_q = 0;
+    float top_q = 0.f;
 #pragma unroll
-    for (int j = 0; j < 8; ++j) x[j] = q_in[2 * ks + (j >> 2)][j & 3];
-    uint4x piece[3];
-    split_eight(x, piece);
+    for (int ks = 0; ks < 2; ++ks) {
+      float x[8];
 #pragma unroll
-    for (int i = 0; i < 3; ++i) bq[ks][i] = __builtin_bit_cast(bf16x8, piece[i]);
+      for (int j = 0; j < 8; ++j) {
+        x[j] = q_in[2 * ks + (j >> 2)][j & 3];
+        top_q = fmaxf(top_q, fabsf(x[j]));
+      }
+      uint4x piece[3];
+      split_eight(x, piece, rest_q);
+#pragma unroll
+      for (int i = 0; i < 3; ++i) bq[ks * 3 + i] = piece[i];
+    }
+    again_q = __any((rest_q & 0xffffu) != 0 || top_q >= kF32TopQ);
   }
 
   // operand addresses, as in the fp16 kernel
@@ -1362,8 +1404,20 @@ __global__ __launch_bounds__(kAttnThreads, 4) void attention_flash_f32_kernel(
     float4v acc[2];                                                    // keys 32 st + 8 g + 4 t + r
 #pragma unroll
     for (int t = 0; t < 2; ++t) acc[t] = float4v{0.f, 0.f, 0.f, 0.f};
+    if constexpr (FLOATS) {
 #pragma unroll
-    for (int ks = 0; ks < 2; ++ks) {
+      for (int t = 0; t < 2; ++t) {
+        const unsigned char* row = kv + ((l16 >> 2) * 8 + t * 4 + (l16 & 3)) * 256;
+#pragma unroll
+        for (int i = 0; i < 4; ++i) {
+          const float4v a = *reinterpret_cast<const float4v*>(row + (((g * 4 + i) ^ l16) * 16)), b = __builtin_bit_cast(float4v, bq[i]);
+#pragma unroll
+          for (int j = 0; j < 4; ++j) acc[t] = __builtin_amdgcn_mfma_f32_16x16x4f32(a[j], b[j], acc[t], 0, 0, 0);
+        }
+      }
+    }
+#pragma unroll
+    for (int ks = 0; ks < (FLOATS ? 0 : 2); ++ks) {
       bf16x8 a[2][3];
 #pragma unroll
       for (int t = 0; t < 2; ++t)
@@ -1371,7 +1425,7 @@ __global__ __launch_bounds__(kAttnThreads, 4) void attention_flash_f32_kernel(
         for (int i = 0; i < 3; ++i) a[t][i] = *reinterpret_cast<const bf16x8*>(kv + k_rd[ks] + i * kF32Piece + t * 4 * 128);
       piece_products([&](int i, int j) {
 #pragma unroll
-        for (int t = 0; t < 2; ++t) acc[t] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a[t][i], bq[ks][j], acc[t], 0, 0, 0);
+        for (int t = 0; t < 2; ++t) acc[t] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a[t][i], __builtin_bit_cast(bf16x8, bq[ks * 3 + j]), acc[t], 0, 0, 0);
       });
       __builtin_amdgcn_sched_barrier(0);         // (six operands at a time, for their registers)
     }
@@ -1379,10 +1433,11 @@ __global__ __launch_bounds__(kAttnThreads, 4) void attention_flash_f32_kernel(
 #pragma unroll
     for (int j = 0; j < 8; ++j) s[j] = acc[j >> 2][j & 3];
     // the exponents' factor: log2 units of the plain scores, of the masked ones otherwise
-    const float unit = PLAIN ? c_exp : kLog2e;
+    const bool no_mask = FLOATS ? plain : PLAIN;
+    const float unit = no_mask ? c_exp : kLog2e;
     const int key0 = st * kF32Keys + g * 8;
     float mx = -INFINITY;
-    if constexpr (PLAIN) {
+    if (no_mask) {
       if ((st + 1) * kF32Keys > n) {                                   // workgroup-uniform: the last, partial stage
 #pragma unroll
         for (int j = 0; j < 8; ++j)
@@ -1407,8 +1462,21 @@ __global__ __launch_bounds__(kAttnThreads, 4) void attention_flash_f32_kernel(
       s[j] = __builtin_amdgcn_exp2f(__builtin_fmaf(s[j], unit, -ref));
       l += s[j];
     }
+    if constexpr (FLOATS) {
+      // tile dt's row m is feature 16 (m >> 2) + 4 dt + (m & 3), the chunk (l16 & ~3) + dt of a row
+#pragma unroll
+      for (int j = 0; j < 8; ++j)
+#pragma unroll
+        for (int dt = 0; dt < 4; ++dt)
+          o[dt] = __builtin_amdgcn_mfma_f32_16x16x4f32(
+              *reinterpret_cast<const float*>(kv + (kF32Keys + g * 8 + j) * 256 + ((((l16 & 12) + dt) ^ g) * 16) + (l16 & 3) * 4), s[j], o[dt], 0, 0, 0);
+      return;
+    }
     uint4x p[3];
-    split_eight(s, p);
+    uint32_t rest_p = 0;
+#pragma unroll
+    for (int j = 0; j < 8; ++j) s[j] *= kF32Raise;
+    split_eight(s, p, rest_p);
 #pragma unroll
     for (int dt = 0; dt < 4; ++dt) {
       bf16x8 v[3];
@@ -1481,10 +1549,32 @@ __global__ __launch_bounds__(kAttnThreads, 4) void attention_flash_f32_kernel(
 
   const float mx = fmaxf(xor_lanes_16_32_max(top), unseen.lowest);
   const float sum = xor_lanes_16_32_sum(l) + unseen.extra;
-  const float inv = 1.0f / (sum + 1e-6f * __builtin_amdgcn_exp2f(mx - ref));
+  const float inv = 1.0f / (sum + 1e-6f * __builtin_amdgcn_exp2f(mx - ref)) * (FLOATS ? 1.0f : 1.0f / kF32Raise);
   // o[dt][r] is feature 16 g + 4 dt + r
 #pragma unroll
   for (int dt = 0; dt < 4; ++dt) o[dt] *= inv;
+  if constexpr (!FLOATS) {
+    bool again = (rest_v & 0xffffu) != 0;
+    if (tq >= 0) {
+      float nan_unless_finite = 0.f;
+#pragma unroll
+      for (int dt = 0; dt < 4; ++dt)
+#pragma unroll
+        for (int r = 0; r < 4; ++r) nan_unless_finite = __builtin_fmaf(o[dt][r], 0.f, nan_unless_finite);
+      again = again || !(nan_unless_finite == 0.f);
+    }
+    const int vote = again_q || __any(again);
+    if (lane == 0) votes[wave] = vote;
+    lds_barrier();                               // (behind it nobody reads K or V any more)
+    const uint4x all = *reinterpret_cast<const uint4x*>(votes);
+    if (__builtin_expect(__builtin_amdgcn_readfirstlane(all[0] | all[1] | all[2] | all[3]) != 0, 0)) {
+      int own = wave * kWave + lane_id();        // (nothing of this way through is kept in registers for the other one)
+      asm volatile("" : "+v"(own));
+      flash_f32_block<PLACED, true>(own, seq_start, batch, heads, q_blocks, seq_len, layout, packed_ld, q_src, k_src, v_src, word_idx,
+                                    attr_mask, mask_class, dst, scaler, out, head_exp, smem_raw);
+      return;
+    }
+  }
   if (out == AttentionOut::kPairs) {
     store_head_pairs<true>(dst, tq < 0 ? -1 : t0 + tq, H, head, o, head_exp);
     return;
@@ -1497,6 +1587,17 @@ __global__ __launch_bounds__(kAttnThreads, 4) void attention_flash_f32_kernel(
     else *reinterpret_cast<float4v*>(dst + (size_t)(t0 + tq) * H + col) = o[dt];
   }
 #endif
+}
+
+template <bool PLACED>
+__global__ __launch_bounds__(kAttnThreads, 4) void attention_flash_f32_kernel(
+    const int32_t* __restrict__ seq_start, int batch, int heads, int q_blocks, int seq_len, int layout, int packed_ld,
+    const float* __restrict__ q_src, const float* __restrict__ k_src, const float* __restrict__ v_src,
+    const int32_t* __restrict__ word_idx, const float* __restrict__ attr_mask, const uint8_t* __restrict__ mask_class,
+    float* __restrict__ dst, float scaler, AttentionOut out, HeadExps head_exp) {
+  extern __shared__ __attribute__((aligned(1024))) unsigned char smem_raw[];
+  flash_f32_block<PLACED, false>(threadIdx.x, seq_start, batch, heads, q_blocks, seq_len, layout, packed_ld, q_src, k_src, v_src, word_idx,
+                                 attr_mask, mask_class, dst, scaler, out, head_exp, smem_raw);
 }
 
 void attention_flash_f32_launch(const void* q, const void* k, const void* v, int layout, int packed_ld, const void* attr_mask,

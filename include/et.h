@@ -324,7 +324,10 @@ et_status et_transpose_rm_padding(et_handle h, et_dtype dtype, const void* src, 
  * seq_len <= 1024; size_per_head from 1 to 256.  size_per_head = 64 (head rows on 16-byte boundaries) runs the MFMA
  * kernels, every other head size a slower general kernel.  Rounding in fp16: the score to half in all of them; up to 64
  * positions and in the general kernel the exponentials are summed in float and the probability is rounded to half; beyond, the
- * exponentials are rounded to half, their sum adds up the rounded values in float, and the output is divided by it.
+ * exponentials are rounded to half, their sum adds up the rounded values in float, and the output is divided by it.  fp32 holds
+ * scores, probabilities and sums as floats; beyond 32 positions its two products run on three bfloat16 pieces of every float and
+ * leave out terms of at most 2^-24 of a product, and blocks of 64 queries whose operands three pieces do not hold (below 2^-110, above
+ * 3.38e38, infinities) run on the float instructions.
  * Masks that end with the sequence (rows of 1 up to the last token, 0 behind it) are the fastest form; with a workspace of
  * et_seq_workspace_bytes(B) the call finds out which blocks of 16 queries have it, and which have all 0 or all 1 behind the
  * last token. */
