@@ -709,9 +709,8 @@ constexpr int kPlacedBatch = kWave;        // sequences, one to a lane
 // More workgroups than four on every CU (fewer all start at once: 8 x 128 positions +0.7 % with it), and, as the kernel finds, about
 // 15 % of them without queries: a workgroup starts up to a microsecond later for it, with vector loads where the other way has
 // scalar ones (32 x 512 positions, 12 % without queries, +0.5 %).
-constexpr int kPlacedGrid = 1024;
 inline bool query_blocks_placed(int batch, int heads, int q_blocks) {
-  return q_blocks > 1 && batch <= kPlacedBatch && (long)batch * heads * q_blocks > kPlacedGrid;
+  return q_blocks > 1 && batch <= kPlacedBatch && (long)batch * heads * q_blocks > 4L * attention_cu_count();
 }
 template <bool PLACED>
 __device__ __forceinline__ QueryBlock query_block(const int32_t* __restrict__ seq_start, int batch, int heads, int q_blocks, int queries,

@@ -56,3 +56,12 @@ def test_no_launch_takes_more_lds_than_its_kernel_was_given(recorder, heads, row
     """The output product's LDS grows with the hidden size: whatever size came first, the next one's must have been asked for."""
     for name, _, lds, raised in _launches(recorder, [(h, 1000, 32, rows) for h in heads]):
         assert lds <= max(raised, 64 * 1024), "%s: %d bytes of LDS, %d asked for" % (name, lds, raised)
+
+
+@pytest.mark.parametrize("cus", [64, 256])
+def test_blocks_without_queries_come_last_beyond_four_workgroups_a_cu(recorder, cus):
+    """8 heads and 192 positions, three blocks of queries: on both sides of four workgroups a CU."""
+    most = 4 * cus // 24
+    for batch in (most, most + 1):
+        attention = [name for name, *_ in _launches(recorder, [(8, batch, 192, batch * 100)], cus) if "attention_flash_f32" in name]
+        assert len(attention) == 1 and ("ILb1E" in attention[0]) == (batch > most)
