@@ -1175,9 +1175,9 @@ void attention_flash_launch(const void* q, const void* k, const void* v, int lay
 // infinity leaves NaN.  A workgroup that meets such operands does its block once more with the float instructions (FLOATS):
 //   V with bits below 2^-133;  Q with such bits, or of 2^60 and more (below that, K's bits below 2^-133 move a score by 2^-67);
 //   a result that is not finite, which is what an operand without three pieces leaves, as do sums that overflow.
-// Probabilities are split 2^24 times as large, where those down to v_exp_f32's smallest have all their bits.  Looking costs nothing
-// that shows (in the layer 30.9 and 60.7 us a launch before, 30.8 and 60.1 with it), the 2^24 1 % (30.8 -> 31.3).  Where every block
-// is done twice the launches take 74 and 106 us, 48 and 63 with the float instructions alone.
+// Probabilities are split 2^24 times as large, where those down to v_exp_f32's smallest have all their bits.  All of it
+// costs nothing that shows (in the layer 31.0 -> 31.2 and 59.1 -> 58.3 us a launch).  Where every block is done twice the launches
+// take 76 and 111 us, 48 and 64 with the float instructions alone.
 // ------------------------------------------------------------------------------------------
 constexpr int kF32Keys = 32;                                 // keys per stage
 constexpr int kF32Piece = kF32Keys * kD * 2;                 // bytes of a piece of K (and of V) per stage
@@ -1270,7 +1270,7 @@ __device__ __forceinline__ void flash_f32_block(
       *reinterpret_cast<float4v*>(kv + kF32Keys * 256 + my_key * 256 + ((cv ^ (my_key >> 3)) * 16)) = in[2 + i];
     }
   };
-  uint32_t rest_v = 0, rest_k = 0;                                     // (of K they do not matter)
+  uint64_t lossy = 0;                                                  // (of K they do not matter)
   auto write = [&] {
     if constexpr (FLOATS) {
       write_floats();
@@ -1282,7 +1282,9 @@ __device__ __forceinline__ void flash_f32_block(
 #pragma unroll
       for (int j = 0; j < 8; ++j) x[j] = in[2 * m + (j >> 2)][j & 3];
       uint4x piece[3];
-      split_eight(x, piece, m ? rest_v : rest_k);
+      uint32_t rest = 0;
+      split_eight(x, piece, rest);
+      if (m) lossy |= __ballot((rest & 0xffffu) != 0);
 #pragma unroll
       for (int i = 0; i < 3; ++i) *reinterpret_cast<uint4x*>((m ? v_wr : k_wr) + i * kF32Piece) = piece[i];
     }
@@ -1552,17 +1554,27 @@ __device__ __forceinline__ void flash_f32_block(
   // o[dt][r] is feature 16 g + 4 dt + r
 #pragma unroll
   for (int dt = 0; dt < 4; ++dt) o[dt] *= inv;
-  if constexpr (!FLOATS) {
-    bool again = (rest_v & 0xffffu) != 0;
-    if (tq >= 0) {
-      float nan_unless_finite = 0.f;
+  if (out == AttentionOut::kPairs) {
+    store_head_pairs<true>(dst, tq < 0 ? -1 : t0 + tq, H, head, o, head_exp);
+  } else if (tq >= 0) {
 #pragma unroll
-      for (int dt = 0; dt < 4; ++dt)
-#pragma unroll
-        for (int r = 0; r < 4; ++r) nan_unless_finite = __builtin_fmaf(o[dt][r], 0.f, nan_unless_finite);
-      again = again || !(nan_unless_finite == 0.f);
+    for (int dt = 0; dt < 4; ++dt) {
+      const int col = head * kD + g * 16 + dt * 4;
+      if (out == AttentionOut::kSplit) store_split<4>(reinterpret_cast<uint16_t*>(dst) + (size_t)(t0 + tq) * 3 * H, col, o[dt]);
+      else *reinterpret_cast<float4v*>(dst + (size_t)(t0 + tq) * H + col) = o[dt];
     }
-    const int vote = again_q || __any(again);
+  }
+  if constexpr (!FLOATS) {
+    // Behind the stores (the second way's come from the same lanes, to the same places), and with what was seen of V in a scalar
+    // register: 12 layers of 4 x 100 positions 1035 us without this look, 1042 with it in front of the stores and in a vector
+    // register, 1035 as it is.
+    float4v not_finite = {0.f, 0.f, 0.f, 0.f};                         // NaN where a result is not
+#pragma unroll
+    for (int dt = 0; dt < 4; ++dt)
+#pragma unroll
+      for (int r = 0; r < 4; ++r) not_finite[r] = __builtin_fmaf(o[dt][r], 0.f, not_finite[r]);
+    const bool bad = tq >= 0 && !((not_finite[0] + not_finite[1]) + (not_finite[2] + not_finite[3]) == 0.f);
+    const int vote = again_q || lossy != 0 || __any(bad);
     if (lane == 0) votes[wave] = vote;
     lds_barrier();                               // (behind it nobody reads K or V any more)
     const uint4x all = *reinterpret_cast<const uint4x*>(votes);
@@ -1571,19 +1583,7 @@ __device__ __forceinline__ void flash_f32_block(
       asm volatile("" : "+v"(own));
       flash_f32_block<PLACED, true>(own, seq_start, batch, heads, q_blocks, seq_len, layout, packed_ld, q_src, k_src, v_src, word_idx,
                                     attr_mask, mask_class, dst, scaler, out, head_exp, smem_raw);
-      return;
     }
-  }
-  if (out == AttentionOut::kPairs) {
-    store_head_pairs<true>(dst, tq < 0 ? -1 : t0 + tq, H, head, o, head_exp);
-    return;
-  }
-  if (tq < 0) return;
-#pragma unroll
-  for (int dt = 0; dt < 4; ++dt) {
-    const int col = head * kD + g * 16 + dt * 4;
-    if (out == AttentionOut::kSplit) store_split<4>(reinterpret_cast<uint16_t*>(dst) + (size_t)(t0 + tq) * 3 * H, col, o[dt]);
-    else *reinterpret_cast<float4v*>(dst + (size_t)(t0 + tq) * H + col) = o[dt];
   }
 #endif
 }
