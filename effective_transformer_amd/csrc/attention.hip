@@ -696,27 +696,34 @@ struct Unseen {
 typedef uint32_t uint4x __attribute__((ext_vector_type(4)));
 
 // The work of workgroup `slot` of XCD `xcd`: a (sequence, head, block of `queries` queries).  Pairs of sequence (in the table's order, the
-// longest first) and head are dealt round-robin to the XCDs, whose L2 then fetches a pair's K and V once for all its blocks.
-// An XCD hands its workgroups to its shader engines strictly in turn, and one that ends at once leaves its place empty until
+// longest first) and head are dealt round-robin to the XCDs, whose L2 then fetches a pair's K and V once for all its blocks:
+// pair = 8 * (slot / q_blocks) + xcd.
+//
+// PLACED launches: an XCD hands its workgroups to its shader engines strictly in turn, and one that ends at once leaves its place empty until
 // the turn comes round again: so the blocks behind a sequence's tokens come last (they hold queries only where the mask has
 // holes).  16 x 1024 positions, 11200 tokens, 12 heads: 3.3 -> 4 workgroups on a CU while there are any, 16 .. 71 -> 49 .. 62 stages
 // of keys a CU (12 layers 2776 -> 2753 us, fp32 15 x 379 2902 -> 2889; 6 layers of 16 heads, 64 x 512 with 32 .. 128 tokens 1144 -> 1061).
-// All of a wavefront's lanes; b < 0: nothing.
+// Launches that are not placed find their pair and leave in the kernel itself: through this function they started later
+// (12 layers of 1 x 1000 positions, fp16, 624 -> 628 us).
 struct QueryBlock {
   int b, head, block, t0, t1;
 };
-constexpr int kPlacedBatch = kWave;        // sequences, one to a lane
+constexpr int kPlacedBatch = kWave;        // sequences, one to a lane (more have not been tried)
 // More workgroups than four on every CU (fewer all start at once: 8 x 128 positions +0.7 % with it), and, as the kernel finds, about
 // 15 % of them without queries: a workgroup starts up to a microsecond later for it, with vector loads where the other way has
 // scalar ones (32 x 512 positions, 12 % without queries, +0.5 %).
 inline bool query_blocks_placed(int batch, int heads, int q_blocks) {
   return q_blocks > 1 && batch <= kPlacedBatch && (long)batch * heads * q_blocks > 4L * attention_cu_count();
 }
-template <bool PLACED>
-__device__ __forceinline__ QueryBlock query_block(const int32_t* __restrict__ seq_start, int batch, int heads, int q_blocks, int queries,
-                                                  int xcd, int slot) {
+__device__ __forceinline__ QueryBlock query_block(const int32_t* __restrict__ seq_start, int batch, int heads, int pair, int block) {
+  const int place = uniform_div(pair, heads), b = min(max(seq_start[batch + 1 + place], 0), batch - 1);
+  return {b, pair - place * heads, block, seq_start[b], seq_start[b + 1]};
+}
+// All of a wavefront's lanes; b < 0: nothing.
+__device__ __forceinline__ QueryBlock placed_query_block(const int32_t* __restrict__ seq_start, int batch, int heads, int q_blocks, int queries,
+                                                         int xcd, int slot) {
   QueryBlock w{-1, 0, 0, 0, 0};
-  if (PLACED && 20 * (seq_start[batch] / queries) + 10 * batch < 17 * batch * q_blocks) {
+  if (20 * (seq_start[batch] / queries) + 10 * batch < 17 * batch * q_blocks) {
     const int lane = threadIdx.x & (kWave - 1);
     const int b = min(max(seq_start[batch + 1 + min(lane, batch - 1)], 0), batch - 1);
     const int t0 = seq_start[b], t1 = seq_start[b + 1];
@@ -739,14 +746,8 @@ __device__ __forceinline__ QueryBlock query_block(const int32_t* __restrict__ se
     w.block = in_rank - k * per_pair + (behind ? __builtin_amdgcn_readlane(full, rank) : 0);
     return w;
   }
-  const int pair_of_xcd = uniform_div(slot, q_blocks), pair = pair_of_xcd * 8 + xcd;
-  if (pair >= batch * heads) return w;
-  const int place = uniform_div(pair, heads);
-  w.head = pair - place * heads;
-  w.block = slot - pair_of_xcd * q_blocks;
-  w.b = min(max(seq_start[batch + 1 + place], 0), batch - 1);
-  w.t0 = seq_start[w.b], w.t1 = seq_start[w.b + 1];
-  return w;
+  const int of_xcd = uniform_div(slot, q_blocks), pair = of_xcd * 8 + xcd;
+  return pair < batch * heads ? query_block(seq_start, batch, heads, pair, slot - of_xcd * q_blocks) : w;
 }
 
 template <typename T>
@@ -781,8 +782,12 @@ __global__ __launch_bounds__(kFlWaves * kWave, 4) void attention_flash_kernel(
   unsigned char* kv = smem_raw;                                        // [stage][K, V]
   int* tok_of_pos = reinterpret_cast<int*>(smem_raw + 2 * 2 * kFlStage);
 
-  const QueryBlock work = query_block<PLACED>(seq_start, batch, heads, q_blocks, 16 * kFlWaves * QSUB, blockIdx.x & 7, blockIdx.x >> 3);
-  if (work.b < 0) return;
+  const int xcd = blockIdx.x & 7, slot_id = blockIdx.x >> 3;
+  const int of_xcd = PLACED ? 0 : uniform_div(slot_id, q_blocks), pair = of_xcd * 8 + xcd;
+  if (!PLACED && pair >= batch * heads) return;
+  const QueryBlock work = PLACED ? placed_query_block(seq_start, batch, heads, q_blocks, 16 * kFlWaves * QSUB, xcd, slot_id)
+                                 : query_block(seq_start, batch, heads, pair, slot_id - of_xcd * q_blocks);
+  if (PLACED && work.b < 0) return;
   const int b = work.b, head = work.head, qblock = work.block, t0 = work.t0, t1 = work.t1;
   const int len = t1 - t0;
   if (len <= 0) return;
@@ -1218,8 +1223,12 @@ __device__ __forceinline__ void flash_f32_block(
   int* tok_of_pos = reinterpret_cast<int*>(smem_raw + 2 * 3 * kF32Piece);
   int* votes = tok_of_pos + kFlMaxKeys;                                // a wavefront: its share is to be done again in floats
 
-  const QueryBlock work = query_block<PLACED>(seq_start, batch, heads, q_blocks, 64, blockIdx.x & 7, blockIdx.x >> 3);
-  if (work.b < 0) return;
+  const int xcd = blockIdx.x & 7, slot_id = blockIdx.x >> 3;
+  const int of_xcd = PLACED ? 0 : uniform_div(slot_id, q_blocks), pair = of_xcd * 8 + xcd;
+  if (!PLACED && pair >= batch * heads) return;
+  const QueryBlock work = PLACED ? placed_query_block(seq_start, batch, heads, q_blocks, 64, xcd, slot_id)
+                                 : query_block(seq_start, batch, heads, pair, slot_id - of_xcd * q_blocks);
+  if (PLACED && work.b < 0) return;
   const int b = work.b, head = work.head, qblock = work.block, t0 = work.t0, t1 = work.t1;
   const int len = t1 - t0;
   if (len <= 0) return;
