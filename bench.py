@@ -11,6 +11,7 @@ standard padded BERT encoder graph on the host cores, on a bounded sample of the
 import argparse
 import json
 import os
+import statistics
 import sys
 import time
 
@@ -273,10 +274,16 @@ def per_kernel(wl, T, mask_np, iters=20, vendor_gemm=False):
     return res
 
 
+OTHER_INSTANCE_FP32 = {
+    "attention": "stores floats; in the layer pair rows with an exponent per head (60 us against 53 at 20375 tokens, 500 x 64)",
+    "gemm_attn_out": "A's rows have one exponent; in the layer one per head (68 us against 64 at 20375 tokens)",
+    "bias_residual_layernorm": "stores floats; in the layer pair rows beside them"}
+
+
 def in_layer_kernels(wl, T, mask_np, reps=4):
     """The kernels of one layer launched in the layer's own order on the layer's own data flow (each kernel reads what
     the one before it wrote, as inside et_layer), with a HIP event between every two launches: the duration a kernel
-    has on the path, where its input is still in the last-level cache.  Returns ms per launch by kernel name and the
+    has on the path, where its input is still in the last-level cache.  Returns the median ms per launch by kernel name and the
     sum over one layer."""
     import torch
     from effective_transformer_amd import kernel_ops as k, ops
@@ -295,10 +302,11 @@ def in_layer_kernels(wl, T, mask_np, reps=4):
     gam, bet = torch.ones(H, device="cuda", dtype=dt), torch.zeros(H, device="cuda", dtype=dt)
     mm = {}
     # fp32 products read pair rows, which the launches in front of them write in the layer: here calls of their own make them
-    # between the timed launches (so attention and LayerNorm are timed without them)
+    # between the timed launches.  So three launches are other instances than the layer's (OTHER_INSTANCE_FP32): attention and
+    # LayerNorm store floats alone, and the attention output reads rows of one exponent, not of one per head
     pairs = dt == torch.float32
     stats = None
-    for n, w in weights.items():          # the kernel the encoder object runs this projection on
+    for n, w in weights.items():          # the kernel the encoder object runs this projection on (but see above)
         if pairs:
             wp, st = k.pair_weight(w, bias[n] if n == "gemm_ffn_up" else None)
             mm[n], stats = (k.gemm_pair, wp), st if st is not None else stats
@@ -353,7 +361,7 @@ def in_layer_kernels(wl, T, mask_np, reps=4):
             cur, down = down, cur      # the layer's output feeds the next layer
 
     layer(None)
-    tot = {n: 0.0 for n in names}
+    took = {n: [] for n in names}
     for _ in range(reps):
         events = [torch.cuda.Event(enable_timing=True) for _ in range(11 * wl.layers)]
         torch.cuda.synchronize()
@@ -362,9 +370,9 @@ def in_layer_kernels(wl, T, mask_np, reps=4):
         torch.cuda.synchronize()
         for (_, start), (n, end) in zip(marks, marks[1:]):
             if n is not None:
-                tot[n] += start.elapsed_time(end)
-    calls = {n: reps * wl.layers * names.count(n) for n in tot}
-    per = {n: tot[n] / calls[n] for n in tot}
+                took[n].append(start.elapsed_time(end))
+    # (the median: a stall of the host between an event and its launch counts as the launch's time, up to 40 ms of one at 24 layers)
+    per = {n: statistics.median(t) for n, t in took.items()}
     return per, sum(per[n] * names.count(n) for n in per)
 
 
@@ -492,6 +500,8 @@ def main():
             kd["ms_in_layer"] = round(ms_l, 5)
             kd["achieved_in_layer"] = round(kd["achieved"] * kd["ms"] / ms_l, 2)
             kd["frac_in_layer"] = round(kd["achieved_in_layer"] / kd["peak"], 4)
+            if wl.dtype == "fp32" and n in OTHER_INSTANCE_FP32:
+                kd["other_instance_than_the_layers"] = OTHER_INSTANCE_FP32[n]
         # dominant kernel = the largest share of a layer's time; its roofline is priced at its duration on the path
         # (the `ms` a launch loop of the kernel alone gives, with cold inputs, stays beside it)
         share = {n: (kernels[n]["ms"] if host_bound else per[n]) * (2 if n == "bias_residual_layernorm" else 1)
@@ -507,7 +517,7 @@ def main():
         else:
             roof = {"kernel": dom, "bound": kd["bound"], "achieved": kd["achieved_in_layer"], "peak": kd["peak"],
                     "unit": kd["unit"], "frac": kd["frac_in_layer"], "ms": kd["ms_in_layer"],
-                    "measured": "HIP events around the kernel inside the layer's launch sequence, %d launches" % (4 * wl.layers),
+                    "measured": "HIP events around the kernel inside the layer's launch sequence, median of %d launches" % (4 * wl.layers),
                     "alone": alone, "traffic": measured_traffic(wl.name, dom)}
     ceiling = None
     if not a.no_calibrate and wl.dtype == "fp16":

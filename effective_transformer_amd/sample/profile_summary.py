@@ -316,7 +316,8 @@ def cmd_vendor(paths):
     out.append("(`kernels[*].ms`, `kernels[*].vendor` in the JSON line). The vendor product is the plain product (no bias, no GELU) with")
     out.append("the weights in TF's `[k][n]` order and in the k-contiguous `[n][k]` order; the own kernel includes the bias (QKV) or")
     out.append("bias + GELU (FFN up; `plain` = the same kernel without the epilogue). `in layer` = the own kernel inside the layer's")
-    out.append("launch sequence (its input still in the last-level cache). TFLOP/s of the fastest vendor variant and of the own kernel")
+    out.append("launch sequence (its input still in the last-level cache; fp32 `attn_out`: with one exponent for a row of A, where the layer's")
+    out.append("instance has one per head: `encoder_cfg4_kernel_stats.md`). TFLOP/s of the fastest vendor variant and of the own kernel")
     out.append("alone are given for the roofline (fp16 peak 2500; fp32: the own kernel is the product of pair rows, peak 2500 / 3, the")
     out.append("vendor's the fp32 MFMA one, 157.3).\n")
     for path in paths:
