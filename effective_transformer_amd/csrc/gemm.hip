@@ -1201,7 +1201,10 @@ __global__ __launch_bounds__(kHThreads) __attribute__((amdgpu_waves_per_eu(2))) 
 // tiles of this kernel; attention output 14.6 and 17.6; FFN-down of 2300 rows 18.6 and 46).
 template <bool GELU, bool NT, PairRing RING>
 __global__ __launch_bounds__(kPThreads) void gemm_f16_pair_rows_kernel(ET_HEAD_ARGS, GemmArgs args) {
-  constexpr PairRing kLow = RING == PairRing::kThreeA ? PairRing::kThreeASpread : PairRing::kTwo;      // of the low tiles
+  // Of the low tiles.  Here, unlike where the host knows the rows, n > k and several groups take spread requests too (Q/K/V of hidden
+  // size 2048: 2940 rows 83.9 -> 83.3 us, 4410 103.3 -> 104.4, 7350 164.1 -> 162.4, 12740 269.4 -> 266.7), and k below 2048 two
+  // slots (with three not tried).
+  constexpr PairRing kLow = RING == PairRing::kThreeA ? PairRing::kThreeASpread : PairRing::kTwo;
   extern __shared__ __attribute__((aligned(1024))) unsigned char smem[];
   const TileHead head = tile_head(a0, b0, rows_dev, m_bound, n, k, groups, args);
   if ((int)((unsigned)(head.rows + 255) / 256) * tiles_n * groups < 128) {

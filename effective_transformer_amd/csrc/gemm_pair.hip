@@ -22,8 +22,8 @@
 // are taken anew by every layer call: pair_weight_top_kernel looks for the largest value of each column, pair_weight_kernel
 // writes the rows (8.4 + 10.2 us per layer of BERT-base, split rows 15).
 // Bound: at large m the power limit of the matrix cores (20375 rows, k = 768 / n = 2304, 768, 3072 + GELU and k = 3072 / n = 768:
-// 171, 68, 259, 226 us in the layer, 1070 .. 1240 TFLOP/s of 16-bit products; split rows 307, 112, 451, 413); below a round of the
-// chip the k loop of one tile (134 rows: 10.2, 7.1, 12.8, 14.3 us against 15.2, 8.7, 16.1, 21.3).
+// 171, 68, 259, 226 us in the layer, 1265, 1060, 1113, 1276 TFLOP/s of 16-bit products, 4 to 6 % less on slower cards; split rows
+// 307, 112, 451, 413); below a round of the chip the k loop of one tile (134 rows: 10.2, 7.1, 12.8, 14.3 us against 15.2, 8.7, 16.1, 21.3).
 #include <algorithm>
 #include <atomic>
 #include <iterator>
