@@ -1188,7 +1188,8 @@ constexpr int kF32Keys = 32;                                 // keys per stage
 constexpr int kF32Piece = kF32Keys * kD * 2;                 // bytes of a piece of K (and of V) per stage
 // Up to 32 positions attention_kernel, whose workgroups serve several heads for one start.  What decides between the two is the
 // number of sequences more than their length (per launch, 12 heads, this kernel second: 1000 x 16 32.2 and 51.3 us, 1000 x 31 52.9
-// and 66.3, 100 x 20 9.3 and 9.4, but 200 x 32 19.1 and 17.0, 8 x 32 5.8 and 5.1); the rule goes by the length alone.
+// and 66.3, 100 x 20 9.3 and 9.4, but 200 x 32 19.1 and 17.0, 8 x 32 5.8 and 5.1); the rule goes by the
+// length alone, as does what depends on it, the making of the mask's classes (mask_class_bytes).
 constexpr int kF32MinKeys = 32;
 [[maybe_unused]] constexpr float kF32TopQ = 0x1p60f, kF32Raise = 0x1p24f;
 constexpr int kF32Smem = 2 * 3 * kF32Piece + (kFlMaxKeys + 4) * (int)sizeof(int);
