@@ -553,11 +553,16 @@ __device__ __forceinline__ int pair_swizzle(int row) { return (row >> 1) & 7; }
 // products of BERT-base on 100 rows 22.9 -> 22.0 us, on 500 rows 33.7 -> 31.1, on 1024 43.7 -> 40.5, on 11501 177.7 -> 172.9).
 // how the persistent kernel walks its tiles: flags, and the workgroups per XCD above them
 constexpr int kWalkReverse = 1, kWalkBlockedA = 2, kWalkWgs = 2;
+// `walk` and `columns` of the tiles below the persistent kernel's: a flag, and C's leading dimension
+// (from kBtLongRows on 128 rows of C lie further apart than 32-bit byte offsets reach)
+constexpr int kBtLongRows = 1 << 24;
+constexpr int kBtGelu = 1;
 #define ET_HEAD_ARGS const void *a0, const void *b0, const int32_t *rows_dev, int m_bound, int n, int k, int groups, int tiles_n, int columns, int walk
 struct TileHead {
   const char *a, *b;                           // operands of the first group, and from there to the others' in bytes
   uint64_t to_a1, to_b1, to_a2, to_b2;
   int rows, n, k, groups;
+  int ldc, gelu;                               // (of the tiles of gemm_f16_bt_kernel)
 
   __device__ __forceinline__ const char* a_of(int grp) const { return a + ((to_a1 & -(uint64_t)(grp == 1)) | (to_a2 & -(uint64_t)(grp == 2))); }
   __device__ __forceinline__ const char* b_of(int grp) const { return b + ((to_b1 & -(uint64_t)(grp == 1)) | (to_b2 & -(uint64_t)(grp == 2))); }
@@ -565,7 +570,7 @@ struct TileHead {
 // The row count and, for several groups, their operands, read in one go.
 __device__ __forceinline__ TileHead tile_head(const void* a0, const void* b0, const int32_t* rows_dev, int m_bound, int n, int k, int groups,
                                               const GemmArgs& args) {
-  TileHead h{(const char*)a0, (const char*)b0, 0, 0, 0, 0, 0, n, k, groups};
+  TileHead h{(const char*)a0, (const char*)b0, 0, 0, 0, 0, 0, n, k, groups, 0, 0};
   int rows = rows_dev ? *rows_dev : m_bound;
   if (groups > 1) {
     h.to_a1 = (uint64_t)args.A[1], h.to_b1 = (uint64_t)args.B[1], h.to_a2 = (uint64_t)args.A[2], h.to_b2 = (uint64_t)args.B[2];
@@ -1075,7 +1080,11 @@ __device__ __forceinline__ void bt_tile(const TileHead& head, int tiles_n, const
   half2v bias2 = {(_Float16)-0.0f, (_Float16)-0.0f};
 #pragma unroll
   for (int j = 0; j < NB; ++j) biasv[j] = (_Float16)-0.0f;
-  if (const _Float16* bias = (const _Float16*)args.bias[grp]; bias != nullptr && col < N) {
+  const _Float16* bias = (const _Float16*)args.bias[grp];
+  _Float16* c_tile = (_Float16*)args.C;
+  asm volatile("" : "+s"(bias), "+s"(c_tile));   // here, and not where they are used
+  c_tile += (size_t)m0 * head.ldc + (size_t)grp * N + n0;
+  if (bias != nullptr && col < N) {
     biasv = *reinterpret_cast<const BiasN*>(bias + col);
     if (NJ == 6 && col2 < N) bias2 = *reinterpret_cast<const half2v*>(bias + col2);
   }
@@ -1097,49 +1106,53 @@ __device__ __forceinline__ void bt_tile(const TileHead& head, int tiles_n, const
     step(Odd{}, std::false_type{}, std::true_type{}, s1, s, p + ST);      // pair p+ST replaces slot s
     s = s1;
   }
-  wait_vmcnt<0>();                               // no DMA may still target this workgroup's LDS when it ends
-
-  // epilogue: lane owns rows g*4+r of every 16-row block and NJ consecutive columns.  Plain stores, not the
+  // Epilogue: the lane owns rows g*4+r of every 16-row block and NJ consecutive columns.  Plain stores, not the
   // non-temporal ones of the persistent kernel: the output of a launch this small is still in the caches when the
   // next kernel reads it (12 layers on 2000 tokens: 0.905 -> 0.843 ms; no difference from about 4000 tokens on).
+  // C leaves through a descriptor that ends with the tile's last valid row, which drops the rows beyond it, and a row's offset is a
+  // scalar.  With a branch, a 64-bit address and scalar loads of ldc and the GELU flag at every row, each waited for, a launch of
+  // 2000 x 2304 took 3.1 us from its last MFMA to its end, of which its bytes need 1.6 (k = 768, us a launch, one that does nothing
+  // 2.2: 2000 rows to 2304 / 768 / 3072 columns 11.5 / 6.8 / 15.9 -> 11.0 / 6.1 / 14.9, 640 rows 6.8 / 4.9 / 8.2 -> 6.2 / 4.5 / 7.7).
   if (col < N) {
-    _Float16* C = (_Float16*)args.C + (size_t)grp * N + col;
-    if constexpr (NJ == 1 || NJ == 2 || NJ == 4 || NJ == 8) {
-      // bias added in half on the rounded product, as the reference's next kernel does
+    const __amdgpu_buffer_rsrc_t rsrc_c = __builtin_amdgcn_make_buffer_rsrc(
+        c_tile, 0, ((uint32_t)(min(rows - m0, BM) - 1) * (uint32_t)head.ldc + (uint32_t)min(N - n0, BN)) * 2u, 0x00020000);
+    const uint32_t voff = ((uint32_t)(wm * 16 * MI + g * 4) * (uint32_t)head.ldc + (uint32_t)(col - n0)) * 2u;
+    const uint32_t voff2 = NJ == 6 ? ((uint32_t)(wm * 16 * MI + g * 4) * (uint32_t)head.ldc + (uint32_t)(col2 - n0)) * 2u : 0u;
+    const bool ok2 = col2 < N;
+    // bias added in half on the rounded product, as the reference's next kernel does
+    auto store = [&](auto GELUc) {
+      constexpr bool GELU = decltype(GELUc)::value;
 #pragma unroll
       for (int i = 0; i < MI; ++i)
 #pragma unroll
         for (int r = 0; r < 4; ++r) {
-          const int row = m0 + wm * 16 * MI + i * 16 + g * 4 + r;
-          if (row < rows) {
-            HalfN o;
+          const int soff = (i * 16 + r) * head.ldc * 2;
+          BiasN o;
 #pragma unroll
-            for (int j = 0; j < NJ; ++j) o[j] = f2h(acc[i][j][r]);
-            o = args.gelu ? bias_gelu_half<HalfN, NJ>(o, biasv) : o + biasv;
-            *reinterpret_cast<HalfN*>(C + (size_t)row * args.ldc) = o;
-          }
+          for (int j = 0; j < NB; ++j) o[j] = f2h(acc[i][j][r]);
+          if constexpr (GELU) o = bias_gelu_half<BiasN, NB>(o, biasv);
+          else o = o + biasv;
+          if constexpr (NB == 1) __builtin_amdgcn_raw_buffer_store_b16(__builtin_bit_cast(uint16_t, o), rsrc_c, voff, soff, 0);
+          else if constexpr (NB == 2) __builtin_amdgcn_raw_buffer_store_b32(__builtin_bit_cast(uint32_t, o), rsrc_c, voff, soff, 0);
+          else if constexpr (NB == 4) __builtin_amdgcn_raw_buffer_store_b64(__builtin_bit_cast(uint2v, o), rsrc_c, voff, soff, 0);
+          else __builtin_amdgcn_raw_buffer_store_b128(__builtin_bit_cast(uint4v, o), rsrc_c, voff, soff, 0);
         }
-    } else {
-      // 6 columns per lane: 4 consecutive ones in the first 64 columns of the wave tile, 2 in the last 32
-      static_assert(NJ == 6, "wave tiles are 32, 64, 96 or 128 columns wide");
-      _Float16* C2 = C - col + col2;
-      const bool ok2 = col2 < N;
+      if (NJ == 6 && ok2) {                      // the other two of a lane's six columns
 #pragma unroll
-      for (int i = 0; i < MI; ++i)
+        for (int i = 0; i < MI; ++i)
 #pragma unroll
-        for (int r = 0; r < 4; ++r) {
-          const int row = m0 + wm * 16 * MI + i * 16 + g * 4 + r;
-          if (row < rows) {
-            half4 o4 = {f2h(acc[i][0][r]), f2h(acc[i][1][r]), f2h(acc[i][2][r]), f2h(acc[i][3][r])};
-            half2v o2 = {f2h(acc[i][4][r]), f2h(acc[i][5][r])};
-            o4 = args.gelu ? bias_gelu_half<half4, 4>(o4, biasv) : o4 + biasv;
-            o2 = args.gelu ? bias_gelu_half<half2v, 2>(o2, bias2) : o2 + bias2;
-            *reinterpret_cast<half4*>(C + (size_t)row * args.ldc) = o4;
-            if (ok2) *reinterpret_cast<half2v*>(C2 + (size_t)row * args.ldc) = o2;
+          for (int r = 0; r < 4; ++r) {
+            half2v o = {f2h(acc[i][NJ - 2][r]), f2h(acc[i][NJ - 1][r])};
+            if constexpr (GELU) o = bias_gelu_half<half2v, 2>(o, bias2);
+            else o = o + bias2;
+            __builtin_amdgcn_raw_buffer_store_b32(__builtin_bit_cast(uint32_t, o), rsrc_c, voff2, (i * 16 + r) * head.ldc * 2, 0);
           }
-        }
-    }
+      }
+    };
+    if (head.gelu) store(std::true_type{});
+    else store(std::false_type{});
   }
+  wait_vmcnt<0>();                               // no DMA may still target this workgroup's LDS when it ends
 #else
   (void)args;
 #endif
@@ -1149,7 +1162,9 @@ __device__ __forceinline__ void bt_tile(const TileHead& head, int tiles_n, const
 template <int MI, int NJ, int ST, bool COLUMNS>
 __global__ __launch_bounds__(kHThreads) __attribute__((amdgpu_waves_per_eu(2))) void gemm_f16_bt_kernel(ET_HEAD_ARGS, GemmArgs args) {
   extern __shared__ __attribute__((aligned(1024))) unsigned char smem[];
-  const TileHead head = tile_head(a0, b0, rows_dev, m_bound, n, k, groups, args);
+  TileHead head = tile_head(a0, b0, rows_dev, m_bound, n, k, groups, args);
+  head.ldc = columns;
+  head.gelu = walk & kBtGelu;
   const int tiles_n_all = tiles_n * groups, tiles_m = (int)((unsigned)(head.rows + 32 * MI - 1) / (32 * MI));
   const int tile = remap_valid_tile(blockIdx.x, tiles_m * tiles_n_all);
   if (tile < 0) return;
@@ -1170,7 +1185,7 @@ struct BtRowsPlan {
 __global__ __launch_bounds__(kHThreads) __attribute__((amdgpu_waves_per_eu(2))) void gemm_f16_bt_rows_kernel(ET_HEAD_ARGS, BtRowsPlan plan, GemmArgs args) {
   extern __shared__ __attribute__((aligned(1024))) unsigned char smem[];
   int rows = *rows_dev;
-  TileHead head{(const char*)a0, (const char*)b0, (uint64_t)args.A[1], (uint64_t)args.B[1], (uint64_t)args.A[2], (uint64_t)args.B[2], 0, n, k, groups};
+  TileHead head{(const char*)a0, (const char*)b0, (uint64_t)args.A[1], (uint64_t)args.B[1], (uint64_t)args.A[2], (uint64_t)args.B[2], 0, n, k, groups, columns, walk & kBtGelu};
 #if defined(__HIP_DEVICE_COMPILE__)
   asm volatile("" : "+s"(rows), "+s"(head.to_a1), "+s"(head.to_b1), "+s"(head.to_a2), "+s"(head.to_b2), "+s"(plan.picks));    // all in one go
 #endif
@@ -1206,8 +1221,10 @@ __global__ __launch_bounds__(kPThreads) void gemm_f16_pair_rows_kernel(ET_HEAD_A
   // slots (with three not tried).
   constexpr PairRing kLow = RING == PairRing::kThreeA ? PairRing::kThreeASpread : PairRing::kTwo;
   extern __shared__ __attribute__((aligned(1024))) unsigned char smem[];
-  const TileHead head = tile_head(a0, b0, rows_dev, m_bound, n, k, groups, args);
+  TileHead head = tile_head(a0, b0, rows_dev, m_bound, n, k, groups, args);
   if ((int)((unsigned)(head.rows + 255) / 256) * tiles_n * groups < 128) {
+    head.ldc = args.ldc;
+    head.gelu = GELU;
 #define ET_BT_CASE(MI, NJ, ST)                                                                                          \
   {                                                                                                                      \
     const int bt_n = (int)((unsigned)(n + 32 * NJ - 1) / (32 * NJ)), all_n = bt_n * groups;                              \
@@ -1562,7 +1579,7 @@ void launch_f16_bt(GemmArgs a, hipStream_t stream) {
   a.per_xcd = (total + kXcds - 1) / kXcds;
   auto go = [&](auto kern) {
     allow_dynamic_lds(reinterpret_cast<const void*>(kern), (int)Tile::SMEM_BYTES);
-    kern<<<a.per_xcd * kXcds, kHThreads, Tile::SMEM_BYTES, stream>>>(a.A[0], a.B[0], a.rows_dev, a.m_bound, a.n, a.k, a.groups, a.tiles_n, 0, 0, a);
+    kern<<<a.per_xcd * kXcds, kHThreads, Tile::SMEM_BYTES, stream>>>(a.A[0], a.B[0], a.rows_dev, a.m_bound, a.n, a.k, a.groups, a.tiles_n, a.ldc, a.gelu ? kBtGelu : 0, a);
   };
   // Few rows want the columns: the weights are then spread over the XCDs instead of read by each of them (12 layers on 580
   // rows of BERT-base 594 -> 572 us, on 300 rows of BERT-large 633 -> 575 us).  Where the two orders fetch about the same
@@ -1750,7 +1767,7 @@ void launch_bt_tile(BtPick p, const GemmArgs& a, hipStream_t stream) {
 bool launch_bt_wave(GemmArgs a, hipStream_t stream) {
   a.tiles_n = (a.n + 15) / 16;
   const long wgs = (long)((a.m_bound + 15) / 16) * a.tiles_n * a.groups;
-  if (wgs > 2l * device_cu_count()) return false;
+  if (wgs > 2l * device_cu_count() && a.ldc < kBtLongRows) return false;
   bool aligned = ((uintptr_t)a.C | (uintptr_t)a.ldc * 2) % 8 == 0;
   for (int g = 0; g < a.groups; ++g) aligned = aligned && (uintptr_t)a.bias[g] % 8 == 0;
   if (!aligned) return false;
@@ -1805,7 +1822,7 @@ bool launch_bt_rows(GemmArgs a, hipStream_t stream) {
   if (best.mi != 0 && cost > 1.05f * bt_cost(best.mi, best.nj, best.duo, a.k)) return false;
   allow_dynamic_lds(reinterpret_cast<const void*>(gemm_f16_bt_rows_kernel), 160 * 1024);
   gemm_f16_bt_rows_kernel<<<(int)((wgs + kXcds - 1) / kXcds * kXcds), kHThreads, lds, stream>>>(a.A[0], a.B[0], a.rows_dev, a.m_bound, a.n, a.k,
-                                                                                                 a.groups, 0, 0, 0, plan, a);
+                                                                                                 a.groups, 0, a.ldc, a.gelu ? kBtGelu : 0, plan, a);
   return true;
 }
 
@@ -1955,6 +1972,7 @@ void launch_gemm(DType t, const GemmGroups& g, void* C, int ldc, int m_bound, in
     } else if (g.b_transposed) {
       // one tile per workgroup, the tile chosen for the launch's shape (pick_bt_tile)
       if (launch_bt_wave(a, stream)) return;
+      if (ldc >= kBtLongRows) return launch_bt_tile({1, 1, false}, a, stream);
       if (rows_dev != nullptr && launch_bt_rows(a, stream)) return;
       launch_bt_tile(pick_bt_tile(m_bound, n, k, g.groups, device_cu_count(), false), a, stream);
     } else {

@@ -1,0 +1,47 @@
+"""How the tiles of small fp16 products on k-contiguous weights leave: every tile shape with rows and columns that end inside it, against
+the [k][n] kernel's bits, and what lies behind C's rows."""
+import pytest
+import torch
+
+from effective_transformer_amd import kernel_ops as ko
+
+pytestmark = pytest.mark.gpu
+
+
+# one of every tile (row blocks x column blocks, d: two workgroups a CU) that a device of 256 CUs chooses, the last one rounds of them
+@pytest.mark.parametrize("m,n,k", [(49, 2152, 192), (40, 4112, 192), (258, 3304, 192), (4167, 72, 192), (289, 4120, 192), (291, 4120, 768),
+                                   (676, 4112, 192), (5461, 136, 192), (5590, 328, 192), (5581, 328, 768), (5948, 648, 192), (5902, 648, 768),
+                                   (5893, 1288, 192), (5471, 264, 768), (5464, 656, 192), (674, 4112, 768), (5379, 1032, 192), (4429, 1288, 768),
+                                   (5394, 1544, 192), (5387, 1040, 2112), (5898, 1928, 192)])
+@pytest.mark.parametrize("gelu", [False, True])
+@pytest.mark.parametrize("on_device", [False, True])
+def test_every_tile(m, n, k, gelu, on_device):
+    print("tile results", m, n, k, gelu, on_device, flush=True)
+    g = torch.Generator(device="cuda").manual_seed(m + n + k)
+    a = torch.randn(m, k, device="cuda", dtype=torch.float16, generator=g)
+    w = torch.randn(k, n, device="cuda", dtype=torch.float16, generator=g).mul_(k ** -0.5)
+    bias = torch.randn(n, device="cuda", dtype=torch.float16, generator=g)
+    want = ko.gemm(a, w, bias=bias, gelu=gelu)
+    bt = ko.transpose_weight(w)
+    rows = m - 37 if on_device else m
+    out = torch.full((m + 300, n), 7.0, device="cuda", dtype=torch.float16)
+    ko.gemm_bt(a, bt, bias, m=m, out=out, gelu=gelu, m_dev=torch.tensor([rows], dtype=torch.int32, device="cuda") if on_device else None)
+    assert torch.equal(out[:rows], want[:rows])
+    assert (out[rows:] == 7.0).all()
+    if not gelu:
+        assert torch.equal(ko.gemm_bt(a, bt), ko.gemm(a, w))
+
+
+# rows of C so long that a tile's last one lies more than 4 GB behind its first
+def test_longest_rows():
+    m, n, k = 33, (1 << 26) + 8, 64
+    print("longest rows", m, n, k, flush=True)
+    g = torch.Generator(device="cuda").manual_seed(3)
+    a = torch.randn(m, k, device="cuda", dtype=torch.float16, generator=g)
+    bt = torch.empty(n, k, device="cuda", dtype=torch.float16)
+    picks = [0, 1000, (1 << 24) - 8, (1 << 25) + 16, n - 264]
+    for p in picks:
+        bt[p:p + 264] = torch.randn(264, k, device="cuda", dtype=torch.float16, generator=g)
+    out = ko.gemm_bt(a, bt, out=torch.empty(m, n, device="cuda", dtype=torch.float16))
+    for p in picks:
+        assert torch.equal(out[:, p:p + 264], ko.gemm_bt(a, bt[p:p + 264].contiguous())), p
