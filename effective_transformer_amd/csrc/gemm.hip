@@ -553,10 +553,10 @@ __device__ __forceinline__ int pair_swizzle(int row) { return (row >> 1) & 7; }
 // products of BERT-base on 100 rows 22.9 -> 22.0 us, on 500 rows 33.7 -> 31.1, on 1024 43.7 -> 40.5, on 11501 177.7 -> 172.9).
 // how the persistent kernel walks its tiles: flags, and the workgroups per XCD above them
 constexpr int kWalkReverse = 1, kWalkBlockedA = 2, kWalkWgs = 2;
-// `walk` and `columns` of the tiles below the persistent kernel's: a flag, and C's leading dimension
+// `walk` and `columns` of the tiles below the persistent kernel's: a flag, strips_log2 above it, and C's leading dimension
 // (from kBtLongRows on 128 rows of C lie further apart than 32-bit byte offsets reach)
 constexpr int kBtLongRows = 1 << 24;
-constexpr int kBtGelu = 1;
+constexpr int kBtGelu = 1, kBtStrips = 1;
 #define ET_HEAD_ARGS const void *a0, const void *b0, const int32_t *rows_dev, int m_bound, int n, int k, int groups, int tiles_n, int columns, int walk
 struct TileHead {
   const char *a, *b;                           // operands of the first group, and from there to the others' in bytes
@@ -970,6 +970,18 @@ struct BtTile {
 // those of them with a CU to themselves that gemm_f16_bt_rows_kernel chooses from (128 x 256 would cost all of them registers)
 #define ET_BT_ROWS_TILES(X) X(1, 1, 0, 5) X(1, 2, 0, 5) X(2, 2, 0, 4) X(2, 4, 0, 4) X(3, 2, 0, 4) X(3, 4, 0, 4) X(3, 6, 0, 3) X(4, 2, 0, 4) X(4, 4, 0, 4) X(4, 6, 0, 3)
 
+// Tiles in the order of 1 << strips_log2 strips of columns, along the rows inside a strip (see band_rows).
+struct TileAt {
+  int row, column;
+};
+__device__ __forceinline__ TileAt strip_order(int tile, int tiles_m, int tiles_n, int strips_log2) {
+  const int wide = (int)((unsigned)(tiles_n + (1 << strips_log2) - 1) >> strips_log2), per_strip = tiles_m * wide;
+  const int strip = strips_log2 == 0 ? 0 : uniform_div(tile, per_strip), first = strip * wide;
+  const int in_strip = tile - strip * per_strip, width = min(wide, tiles_n - first);
+  const int row = wide == 1 ? in_strip : uniform_div(in_strip, width);
+  return {row, first + in_strip - row * width};
+}
+
 // The tile in row `tm` and column `tn_all` of tiles, whose columns run through the groups; `tiles_n` of them to a group.
 template <int MI, int NJ, int ST>
 __device__ __forceinline__ void bt_tile(const TileHead& head, int tiles_n, const GemmArgs& args, int tm, int tn_all, unsigned char* smem) {
@@ -1158,8 +1170,7 @@ __device__ __forceinline__ void bt_tile(const TileHead& head, int tiles_n, const
 #endif
 }
 
-// COLUMNS: the tile order runs down the columns of tiles instead of along the rows (see band_rows).
-template <int MI, int NJ, int ST, bool COLUMNS>
+template <int MI, int NJ, int ST>
 __global__ __launch_bounds__(kHThreads) __attribute__((amdgpu_waves_per_eu(2))) void gemm_f16_bt_kernel(ET_HEAD_ARGS, GemmArgs args) {
   extern __shared__ __attribute__((aligned(1024))) unsigned char smem[];
   TileHead head = tile_head(a0, b0, rows_dev, m_bound, n, k, groups, args);
@@ -1168,8 +1179,8 @@ __global__ __launch_bounds__(kHThreads) __attribute__((amdgpu_waves_per_eu(2))) 
   const int tiles_n_all = tiles_n * groups, tiles_m = (int)((unsigned)(head.rows + 32 * MI - 1) / (32 * MI));
   const int tile = remap_valid_tile(blockIdx.x, tiles_m * tiles_n_all);
   if (tile < 0) return;
-  const int by = COLUMNS ? tiles_m : tiles_n_all, outer = uniform_div(tile, by), inner = tile - outer * by;
-  bt_tile<MI, NJ, ST>(head, tiles_n, args, COLUMNS ? inner : outer, COLUMNS ? outer : inner, smem);
+  const TileAt at = strip_order(tile, tiles_m, tiles_n_all, walk >> kBtStrips);
+  bt_tile<MI, NJ, ST>(head, tiles_n, args, at.row, at.column, smem);
 }
 
 // Where only the device knows the row count, it picks the tile: the tiles that are the best for some count up to the launch's
@@ -1178,8 +1189,8 @@ __global__ __launch_bounds__(kHThreads) __attribute__((amdgpu_waves_per_eu(2))) 
 // 31.6 us, 1024 of 1024 43.7 and 40.5 (the start of the kernel costs no more than that of a kernel for one tile); 2457 of 4096 77.9
 // and 66.2, 4096 of 4096 88.8 and 86.2; 300 of 500 33.0 and 25.1.
 struct BtRowsPlan {
-  static constexpr int kPicks = 7, kColumns = 0x80;
-  uint64_t picks = 0;          // a byte each, the first in the lowest: index into ET_BT_ROWS_TILES, kColumns
+  static constexpr int kPicks = 7, kStrips = 4;
+  uint64_t picks = 0;          // a byte each, the first in the lowest: index into ET_BT_ROWS_TILES, from bit kStrips on strips_log2
   int up_to[kPicks - 1];       // rows a pick serves (the last one: the rest)
 };
 __global__ __launch_bounds__(kHThreads) __attribute__((amdgpu_waves_per_eu(2))) void gemm_f16_bt_rows_kernel(ET_HEAD_ARGS, BtRowsPlan plan, GemmArgs args) {
@@ -1194,7 +1205,7 @@ __global__ __launch_bounds__(kHThreads) __attribute__((amdgpu_waves_per_eu(2))) 
   int at = 0;
 #pragma unroll
   for (int i = 0; i < BtRowsPlan::kPicks - 1; ++i) at += 8 * uniform_less(plan.up_to[i], rows);
-  const int pick = (int)(plan.picks >> at), by_columns = pick & BtRowsPlan::kColumns;
+  const int pick = (int)(plan.picks >> at) & 0xff;
   int index = 0;
 #define ET_BT_CASE(MI, NJ, DUO, ST)                                                                                     \
   if ((pick & 15) == index++) {                                                                                          \
@@ -1202,8 +1213,8 @@ __global__ __launch_bounds__(kHThreads) __attribute__((amdgpu_waves_per_eu(2))) 
     const int all_n = tiles_n * groups, tiles_m = (int)((unsigned)(rows + 32 * MI - 1) / (32 * MI));                 \
     const int tile = remap_valid_tile(blockIdx.x, tiles_m * all_n);                                                      \
     if (tile < 0) return;                                                                                                \
-    const int by = by_columns ? tiles_m : all_n, outer = uniform_div(tile, by), inner = tile - outer * by;                  \
-    return bt_tile<MI, NJ, ST>(head, tiles_n, args, by_columns ? inner : outer, by_columns ? outer : inner, smem); \
+    const TileAt where = strip_order(tile, tiles_m, all_n, pick >> BtRowsPlan::kStrips);                                 \
+    return bt_tile<MI, NJ, ST>(head, tiles_n, args, where.row, where.column, smem);                                        \
   }
   ET_BT_ROWS_TILES(ET_BT_CASE)
 #undef ET_BT_CASE
@@ -1556,18 +1567,33 @@ void launch_f16(GemmArgs a, hipStream_t stream) {
   kern<<<a.per_xcd * kXcds, kHThreads, Tile::SMEM_BYTES, stream>>>(a);
 }
 
-// Distinct operand rows (of A and of B^T) that the tiles of one XCD's band touch, which is what its L2 has to fetch, with
-// the tile order running along the rows of tiles or down the columns.
-constexpr int kColumnRows = 1024;
-struct BandRows {
-  long along, down;
-};
-BandRows band_rows(long tiles_m, long tiles_n, int bm, int bn) {
-  const long band = (tiles_m * tiles_n + kXcds - 1) / kXcds;
-  auto rows = [&](long inner, int b_inner, int b_outer) {
-    return std::min(band, inner) * b_inner + (band + inner - 1) / inner * b_outer;
-  };
-  return {rows(tiles_n, bn, bm), rows(tiles_m, bm, bn)};
+// Operand rows (of A and of B^T) that the tiles of one XCD's band touch, which is what its L2 has to fetch, with the tiles in
+// 1 << strips_log2 strips of columns.
+inline int band_rows(int tiles_m, int tiles_n, int bm, int bn, int strips_log2) {
+  const int band = (int)((unsigned)(tiles_m * tiles_n + kXcds - 1) / kXcds);
+  const int wide = (tiles_n + (1 << strips_log2) - 1) >> strips_log2, per_strip = tiles_m * wide;
+  if (band <= per_strip) return std::min(tiles_m, (int)((unsigned)(band + wide - 1) / wide)) * bm + wide * bn;
+  return tiles_m * bm + (int)((unsigned)(band + per_strip - 1) / per_strip) * wide * bn;
+}
+// Along the rows (0), down the columns (strips of one column), or in two, four or eight strips.  Each XCD fetches the operand rows
+// of its band for itself, so that a band as high as it is wide fetches the fewest.  Up to 1024 rows the columns spread the weights
+// over the XCDs (12 layers on 580 rows of BERT-base 594 -> 572 us, on 300 rows of BERT-large 633 -> 575); strips do it without all
+// of A: k = 768, 1200 rows to 2304 / 3072 columns 9.3 / 12.2 -> 8.6 / 10.8 us, 2000 rows to 3072 15.9 -> 14.8, 640 rows of k = 3072
+// 9.7 -> 9.2; 1200 rows to 3072 columns, k = 1024, 13.7 -> 11.6.
+// What saves less than a quarter of the rows costs more in the second division of a tile's number (0.1 us) than it gives.
+constexpr int kColumnRows = 1024, kMaxStripsLog2 = 3;
+inline int best_strips_log2(int tiles_m, int tiles_n, int bm, int bn) {
+  int best = 0, rows = band_rows(tiles_m, tiles_n, bm, bn, 0);
+  if (tiles_m * bm <= kColumnRows + bm && tiles_n > 1) {
+    const int down = 32 - __builtin_clz((unsigned)(tiles_n - 1)), r = band_rows(tiles_m, tiles_n, bm, bn, down);
+    if (4 * r <= 3 * rows) best = down, rows = r;
+  }
+  int limit = 3 * rows / 4;
+  for (int l = 1; l <= kMaxStripsLog2 && (1 << l) < tiles_n; ++l) {
+    const int r = band_rows(tiles_m, tiles_n, bm, bn, l);
+    if (r <= limit) best = l, limit = r - 1;
+  }
+  return best;
 }
 
 template <int MI, int NJ, int ST>
@@ -1577,16 +1603,11 @@ void launch_f16_bt(GemmArgs a, hipStream_t stream) {
   a.tiles_n = (a.n + Tile::BN - 1) / Tile::BN;
   const int total = a.tiles_m * a.tiles_n * a.groups;
   a.per_xcd = (total + kXcds - 1) / kXcds;
-  auto go = [&](auto kern) {
-    allow_dynamic_lds(reinterpret_cast<const void*>(kern), (int)Tile::SMEM_BYTES);
-    kern<<<a.per_xcd * kXcds, kHThreads, Tile::SMEM_BYTES, stream>>>(a.A[0], a.B[0], a.rows_dev, a.m_bound, a.n, a.k, a.groups, a.tiles_n, a.ldc, a.gelu ? kBtGelu : 0, a);
-  };
-  // Few rows want the columns: the weights are then spread over the XCDs instead of read by each of them (12 layers on 580
-  // rows of BERT-base 594 -> 572 us, on 300 rows of BERT-large 633 -> 575 us).  Where the two orders fetch about the same
-  // they take the same time, and from about 1000 rows on the columns lose up to 1 %.
-  const BandRows band = band_rows(a.tiles_m, (long)a.tiles_n * a.groups, Tile::BM, Tile::BN);
-  if (a.m_bound <= kColumnRows && 4 * band.down <= 3 * band.along) go(gemm_f16_bt_kernel<MI, NJ, ST, true>);
-  else go(gemm_f16_bt_kernel<MI, NJ, ST, false>);
+  auto kern = gemm_f16_bt_kernel<MI, NJ, ST>;
+  allow_dynamic_lds(reinterpret_cast<const void*>(kern), (int)Tile::SMEM_BYTES);
+  const int strips = best_strips_log2(a.tiles_m, a.tiles_n * a.groups, Tile::BM, Tile::BN);
+  kern<<<a.per_xcd * kXcds, kHThreads, Tile::SMEM_BYTES, stream>>>(a.A[0], a.B[0], a.rows_dev, a.m_bound, a.n, a.k, a.groups, a.tiles_n, a.ldc,
+                                                                    strips << kBtStrips | (a.gelu ? kBtGelu : 0), a);
 }
 
 int device_cu_count() {
@@ -1739,7 +1760,7 @@ BtPick pick_bt_tile(int m_bound, int n, int k, int groups, int cus, bool proven_
     const bool duo = wgs > cus;
     if (duo && !(wgs <= 2L * cus && tile.duo && !(proven_only && nj > 4))) continue;
     const float cost = bt_cost(mi, nj, duo, k);
-    const long band = k < 2048 ? -nj : band_rows((m_bound + 32 * mi - 1) / (32 * mi), tiles_n, 32 * mi, 32 * nj).along;
+    const long band = k < 2048 ? -nj : band_rows((m_bound + 32 * mi - 1) / (32 * mi), (int)tiles_n, 32 * mi, 32 * nj, 0);
     if (best.mi == 0 || cost < best_cost || (cost == best_cost && band < best_band)) {
       best.mi = mi;
       best.nj = nj;
@@ -1807,10 +1828,9 @@ bool launch_bt_rows(GemmArgs a, hipStream_t stream) {
     // (counts below an eighth of the bound get the tile of the next ones)
     if (t.rows < a.m_bound / 8 || picks == BtRowsPlan::kPicks) continue;
     const int rows = std::min(t.rows, a.m_bound), tiles_m = (rows + 32 * t.mi - 1) / (32 * t.mi);
-    const BandRows band = band_rows(tiles_m, t.tiles_n, 32 * t.mi, 32 * t.nj);
-    const bool columns = rows <= kColumnRows && 4 * band.down <= 3 * band.along;
+    const int strips = best_strips_log2(tiles_m, t.tiles_n, 32 * t.mi, 32 * t.nj);
     if (rows < a.m_bound && picks < BtRowsPlan::kPicks - 1) plan.up_to[picks] = rows;
-    plan.picks |= (uint64_t)(t.index | (columns ? BtRowsPlan::kColumns : 0)) << (8 * picks);
+    plan.picks |= (uint64_t)(t.index | strips << BtRowsPlan::kStrips) << (8 * picks);
     wgs = std::max(wgs, (long)tiles_m * t.tiles_n);
     lds = std::max(lds, t.lds);
     cost = t.cost;
