@@ -883,7 +883,7 @@ et_status et_layer_with_prepared(et_handle h, et_dtype dtype, const et_layer_wei
 namespace {
 
 struct EncoderWs {
-  size_t x[2], batch_idx, word_idx, count, seq, scan, layer, total;
+  size_t x[2], batch_idx, word_idx, packed_row, count, seq, scan, layer, total;
 };
 
 EncoderWs encoder_ws(et_dtype dtype, int B, int S, int heads, int d) {
@@ -900,6 +900,7 @@ EncoderWs encoder_ws(et_dtype dtype, int B, int S, int heads, int d) {
   w.x[1] = take(rows * H * e);
   w.batch_idx = take(rows * sizeof(int32_t));
   w.word_idx = take(rows * sizeof(int32_t));
+  w.packed_row = take(rows * sizeof(int32_t));
   w.count = take(sizeof(int32_t));
   w.seq = take(seq_table_bytes_min(B));
   w.scan = take(et_input_workspace_bytes(B, S));
@@ -997,6 +998,7 @@ et_status et_encoder(et_handle h, et_dtype dtype, int num_layers, const et_layer
   const bool wait_for_layers = b->rows_bound == 0 && num_layers > 1 && b->count_word && !is_capturing(st);
   et::ScanExtras scan;
   scan.seq_start = seq;
+  scan.packed_row = (int32_t*)(base + ws.packed_row);
   if (wait_for_layers || (b->count_word && b->valid_word_num)) {
     scan.host_word = b->count_word;
     scan.host_tag = next_tag.fetch_add(1, std::memory_order_relaxed);
@@ -1068,7 +1070,7 @@ et_status et_encoder(et_handle h, et_dtype dtype, int num_layers, const et_layer
     if ((s = run_layer(h, c)) != ET_OK) return s;
     cur ^= 1;
   }
-  et::launch_restore_rows(b->out, x[cur], batch_idx, word_idx, count, B, S, (int)row_bytes, st);
+  et::launch_mapped_restore_rows(b->out, x[cur], scan.packed_row, B * S, (int)row_bytes, st);
   if ((s = check_launch(h, "restore")) != ET_OK) return s;
   if (b->valid_word_num) {
     if (T < 0 && scan.host_word) {

@@ -110,6 +110,8 @@ __global__ __launch_bounds__(kScanThreads) void scan_index_kernel(const int32_t*
           batch_idx[excl] = b;
           word_idx[excl] = idx - b * seq_len;
         }
+        // (a last entry above 1 is not counted below)
+        if (extras.packed_row) extras.packed_row[idx] = v > 0 && excl >= 0 && excl < n && (v == 1 || idx != n - 1) ? excl : -1;
         // the first half of the sequence table: the prefix where a sequence begins is its first packed row
         if (extras.seq_start) {
           const int b = idx / seq_len;
@@ -207,22 +209,26 @@ __global__ __launch_bounds__(kMoveThreads) void compress_rows_kernel(
     }
 }
 
-constexpr int kRestorePos = 32;   // padded positions per workgroup
+
+// Positions from which on a workgroup takes 32 of them, and not 8: with fewer positions the launch is short of workgroups, and each
+// goes through its chunks in several trips to memory (us a launch, 32 and 8 positions a workgroup: 256 rows of 3 KB 8.8 and 4.2, 1024
+// of 1.5 KB 6.1 and 3.5, 3200 6.4 and 4.0, 11501 8.3 and 6.8; with 32 at 16384 9.1, 64000 23.2).
+constexpr int kRestoreMany = 16384;
 
 // One pass over the padded output: every 16-byte chunk of [B*S, row] is written exactly once,
 // either from its packed row or with zeros.  The packed row of a padded position is found
 // without scratch memory: keys b*S+s are ascending in t, so a 64-way search by one wavefront
 // locates the first packed row at or after the workgroup's first position and the next
-// kRestorePos keys cover everything that can land in the workgroup's window.
-template <typename CH>
+// POS keys cover everything that can land in the window of the workgroup's POS positions.
+template <typename CH, int POS>
 __global__ __launch_bounds__(kMoveThreads) void restore_rows_kernel(
     CH* __restrict__ to, const CH* __restrict__ from, const int32_t* __restrict__ batch_idx,
     const int32_t* __restrict__ word_idx, const int32_t* __restrict__ rows_dev, int n_pos, int seq_len, int cpr) {
-  __shared__ int inv[kRestorePos];
+  __shared__ int inv[POS];
   __shared__ int t0_sh;
-  const int p0 = blockIdx.x * kRestorePos;
+  const int p0 = blockIdx.x * POS;
   const int T = min(*rows_dev, n_pos);
-  if (threadIdx.x < kRestorePos) inv[threadIdx.x] = -1;
+  if (threadIdx.x < POS) inv[threadIdx.x] = -1;
   if (threadIdx.x < kWave) {
     const int lane = threadIdx.x;
     int lo = 0, hi = T;                 // first t with key(t) >= p0 lies in [lo, hi]
@@ -246,15 +252,15 @@ __global__ __launch_bounds__(kMoveThreads) void restore_rows_kernel(
   }
   __syncthreads();
   const int t0 = t0_sh;
-  if (threadIdx.x < kRestorePos) {
+  if (threadIdx.x < POS) {
     const int t = t0 + threadIdx.x;
     if (t < T) {
       const int key = batch_idx[t] * seq_len + word_idx[t];
-      if (key >= p0 && key < p0 + kRestorePos) inv[key - p0] = t;
+      if (key >= p0 && key < p0 + POS) inv[key - p0] = t;
     }
   }
   __syncthreads();
-  const int npos = min(kRestorePos, n_pos - p0);
+  const int npos = min(POS, n_pos - p0);
   const int total = npos * cpr;
   for (int i0 = 0; i0 < total; i0 += kMoveThreads * kMoveUnroll) {
     CH val[kMoveUnroll];
@@ -275,6 +281,33 @@ __global__ __launch_bounds__(kMoveThreads) void restore_rows_kernel(
       if (i < total) to[(size_t)p0 * cpr + i] = val[u];
     }
   }
+}
+
+// The same pass where the scan left the packed row of every position (et_encoder): flattened over (position, chunk), UNROLL chunks
+// a lane, two dependent loads and the stores where the search takes four or five.  Bound by the loads' latency for a few thousand
+// positions (in an encoder, us a launch, the search with 32 positions a workgroup before: 256 rows of 3 KB 9.3 -> 3.9), by memory for
+// many (64000 of 1.5 KB 23.5 -> 22.5, 16384 10.1 -> 8.3).  Eight chunks a lane once that still gives four workgroups to a CU, else two.
+template <typename CH, int UNROLL>
+__global__ __launch_bounds__(kMoveThreads) void mapped_restore_rows_kernel(CH* __restrict__ to, const CH* __restrict__ from,
+                                                                           const int32_t* __restrict__ packed_row, uint32_t total,
+                                                                           fastdiv cpr) {
+  const uint32_t base = blockIdx.x * (kMoveThreads * UNROLL) + threadIdx.x;
+  uint32_t chunk[UNROLL];
+  int row[UNROLL];
+#pragma unroll
+  for (int u = 0; u < UNROLL; ++u) {
+    const uint32_t i = min(base + u * kMoveThreads, total - 1), pos = div_by(i, cpr);      // (past the end: the last chunk again)
+    chunk[u] = i - pos * cpr.d;
+    row[u] = packed_row[pos];
+  }
+  CH val[UNROLL];
+#pragma unroll
+  for (int u = 0; u < UNROLL; ++u) {
+    val[u] = CH{};
+    if (row[u] >= 0) val[u] = from[(size_t)row[u] * cpr.d + chunk[u]];
+  }
+#pragma unroll
+  for (int u = 0; u < UNROLL; ++u) to[min(base + u * kMoveThreads, total - 1)] = val[u];
 }
 
 __global__ __launch_bounds__(256) void seq_start_kernel(const int32_t* __restrict__ batch_idx,
@@ -391,18 +424,40 @@ void launch_compress_rows(const void* from, void* to, const int32_t* batch_idx, 
 void launch_restore_rows(void* to, const void* from, const int32_t* batch_idx, const int32_t* word_idx,
                          const int32_t* rows_dev, int batch, int seq_len, int row_bytes, hipStream_t stream) {
   const int n_pos = batch * seq_len;
-  const int grid = (n_pos + kRestorePos - 1) / kRestorePos;
   const int cb = move_chunk_bytes(row_bytes);
   const int cpr = row_bytes / cb;
-  if (cb == 16)
-    restore_rows_kernel<u32x4><<<grid, kMoveThreads, 0, stream>>>((u32x4*)to, (const u32x4*)from, batch_idx, word_idx,
-                                                                  rows_dev, n_pos, seq_len, cpr);
-  else if (cb == 4)
-    restore_rows_kernel<uint32_t><<<grid, kMoveThreads, 0, stream>>>((uint32_t*)to, (const uint32_t*)from, batch_idx,
-                                                                     word_idx, rows_dev, n_pos, seq_len, cpr);
-  else
-    restore_rows_kernel<uint16_t><<<grid, kMoveThreads, 0, stream>>>((uint16_t*)to, (const uint16_t*)from, batch_idx,
-                                                                     word_idx, rows_dev, n_pos, seq_len, cpr);
+  auto go = [&](auto chunk, auto positions) {
+    using CH = decltype(chunk);
+    constexpr int kPos = decltype(positions)::value;
+    restore_rows_kernel<CH, kPos><<<(n_pos + kPos - 1) / kPos, kMoveThreads, 0, stream>>>((CH*)to, (const CH*)from, batch_idx, word_idx,
+                                                                                       rows_dev, n_pos, seq_len, cpr);
+  };
+  auto by_size = [&](auto chunk) {
+    if (n_pos >= kRestoreMany) go(chunk, std::integral_constant<int, 32>{});
+    else go(chunk, std::integral_constant<int, 8>{});
+  };
+  if (cb == 16) by_size(u32x4{});
+  else if (cb == 4) by_size(uint32_t{});
+  else by_size(uint16_t{});
+}
+
+void launch_mapped_restore_rows(void* to, const void* from, const int32_t* packed_row, int n_pos, int row_bytes, hipStream_t stream) {
+  const int cb = move_chunk_bytes(row_bytes);
+  const uint32_t cpr = (uint32_t)row_bytes / (uint32_t)cb, total = (uint32_t)n_pos * cpr;
+  auto go = [&](auto chunk, auto unroll) {
+    using CH = decltype(chunk);
+    constexpr int kUnroll = decltype(unroll)::value;
+    constexpr uint32_t kPerWg = kMoveThreads * kUnroll;
+    mapped_restore_rows_kernel<CH, kUnroll><<<(total + kPerWg - 1) / kPerWg, kMoveThreads, 0, stream>>>(
+        (CH*)to, (const CH*)from, packed_row, total, make_fastdiv(cpr));
+  };
+  auto by_size = [&](auto chunk) {
+    if (total >= kMoveThreads * kMoveUnroll * 1024u) go(chunk, std::integral_constant<int, kMoveUnroll>{});
+    else go(chunk, std::integral_constant<int, 2>{});
+  };
+  if (cb == 16) by_size(u32x4{});
+  else if (cb == 4) by_size(uint32_t{});
+  else by_size(uint16_t{});
 }
 
 void count_batch_jobs(BatchJobs* j) {

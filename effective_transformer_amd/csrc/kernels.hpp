@@ -33,6 +33,7 @@ size_t scan_scratch_words(int length);
 // What the scan of a mask can leave behind on its way, and what the compress launch behind it can (each nullable).
 struct ScanExtras {
   int32_t* seq_start = nullptr;      // first half of the batch's sequence table (see launch_seq_start)
+  int32_t* packed_row = nullptr;     // of every position: the row it is packed into, -1 if none
   uint64_t* host_word = nullptr;     // pinned host memory: host_tag << 32 | valid-token count, one 8-byte store
   uint32_t host_tag = 0;
 };
@@ -61,6 +62,8 @@ size_t move_chunks(int n_pos, int row_bytes);
 // to[B*S rows] = 0 at padding, from[t] at batch_idx[t]*S + word_idx[t]; indices ascending.
 void launch_restore_rows(void* to, const void* from, const int32_t* batch_idx, const int32_t* word_idx,
                          const int32_t* rows_dev, int batch, int seq_len, int row_bytes, hipStream_t stream);
+// The same where the packed row of every position is at hand (ScanExtras).
+void launch_mapped_restore_rows(void* to, const void* from, const int32_t* packed_row, int n_pos, int row_bytes, hipStream_t stream);
 // to[b,:] = packed row at position 0 of sequence b (zeros if there is none); indices ascending.
 void launch_first_token(void* to, const void* from, const int32_t* batch_idx, const int32_t* word_idx,
                         const int32_t* rows_dev, int rows_bound, int batch, int row_bytes, hipStream_t stream);
