@@ -558,7 +558,7 @@ et_status run_layer(et_handle h, const LayerCall& c) {
   et::GemmGroups g3;
   g3.groups = 3;
   g3.c_cached = cached;
-  g3.A[0] = from_a; g3.A[1] = to_a; g3.A[2] = to_a;
+  g3.A[0] = from_a; g3.A[1] = to_a;
   g3.B[0] = t_qkv ? wt_q : w->attr_kernel_Q; g3.B[1] = t_qkv ? wt_k : w->attr_kernel_K; g3.B[2] = t_qkv ? wt_v : w->attr_kernel_V;
   g3.bias[0] = w->attr_bias_Q; g3.bias[1] = w->attr_bias_K; g3.bias[2] = w->attr_bias_V;
   g3.b_transposed = t_qkv;

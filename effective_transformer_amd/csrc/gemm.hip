@@ -558,6 +558,15 @@ constexpr int kWalkReverse = 1, kWalkBlockedA = 2, kWalkWgs = 2;
 constexpr int kBtLongRows = 1 << 24;
 constexpr int kBtGelu = 1, kBtStrips = 1;
 #define ET_HEAD_ARGS const void *a0, const void *b0, const int32_t *rows_dev, int m_bound, int n, int k, int groups, int tiles_n, int columns, int walk
+// What else the tiles below the persistent kernel's need: with the head 112 bytes of arguments.  The host issues an encoder of few rows more
+// slowly than the device runs it, and takes 2.8 us for a launch with up to 112 bytes and 3.6 us from 116 on (12 layers of 1 x 32 positions,
+// one pass behind the other 355 -> 342 us, the first pass of a new model 664 -> 526).  The kernel for rows that only the device knows, which is
+// replayed from graphs, is 0.1 us faster with GemmArgs.
+struct TileArgs {
+  const void *a1, *b1, *b2;                    // operands of the second group and of the third, which share A
+  const void* bias[3];
+  void* C;
+};
 struct TileHead {
   const char *a, *b;                           // operands of the first group, and from there to the others' in bytes
   uint64_t to_a1, to_b1, to_a2, to_b2;
@@ -567,13 +576,20 @@ struct TileHead {
   __device__ __forceinline__ const char* a_of(int grp) const { return a + ((to_a1 & -(uint64_t)(grp == 1)) | (to_a2 & -(uint64_t)(grp == 2))); }
   __device__ __forceinline__ const char* b_of(int grp) const { return b + ((to_b1 & -(uint64_t)(grp == 1)) | (to_b2 & -(uint64_t)(grp == 2))); }
 };
+__device__ __forceinline__ void group_operands(const GemmArgs& args, TileHead& h) {
+  h.to_a1 = (uint64_t)args.A[1], h.to_b1 = (uint64_t)args.B[1], h.to_a2 = (uint64_t)args.A[2], h.to_b2 = (uint64_t)args.B[2];
+}
+__device__ __forceinline__ void group_operands(const TileArgs& args, TileHead& h) {
+  h.to_a1 = h.to_a2 = (uint64_t)args.a1, h.to_b1 = (uint64_t)args.b1, h.to_b2 = (uint64_t)args.b2;
+}
 // The row count and, for several groups, their operands, read in one go.
+template <typename Args>
 __device__ __forceinline__ TileHead tile_head(const void* a0, const void* b0, const int32_t* rows_dev, int m_bound, int n, int k, int groups,
-                                              const GemmArgs& args) {
+                                              const Args& args) {
   TileHead h{(const char*)a0, (const char*)b0, 0, 0, 0, 0, 0, n, k, groups, 0, 0};
   int rows = rows_dev ? *rows_dev : m_bound;
   if (groups > 1) {
-    h.to_a1 = (uint64_t)args.A[1], h.to_b1 = (uint64_t)args.B[1], h.to_a2 = (uint64_t)args.A[2], h.to_b2 = (uint64_t)args.B[2];
+    group_operands(args, h);
 #if defined(__HIP_DEVICE_COMPILE__)
     asm volatile("" : "+s"(rows), "+s"(h.to_a1), "+s"(h.to_b1), "+s"(h.to_a2), "+s"(h.to_b2));   // not later, one by one
 #endif
@@ -983,8 +999,8 @@ __device__ __forceinline__ TileAt strip_order(int tile, int tiles_m, int tiles_n
 }
 
 // The tile in row `tm` and column `tn_all` of tiles, whose columns run through the groups; `tiles_n` of them to a group.
-template <int MI, int NJ, int ST>
-__device__ __forceinline__ void bt_tile(const TileHead& head, int tiles_n, const GemmArgs& args, int tm, int tn_all, unsigned char* smem) {
+template <int MI, int NJ, int ST, typename Args>
+__device__ __forceinline__ void bt_tile(const TileHead& head, int tiles_n, const Args& args, int tm, int tn_all, unsigned char* smem) {
 #if defined(__HIP_DEVICE_COMPILE__)   // device-only types in the body; the host pass only needs the stub
   using Tile = BtTile<MI, NJ, ST>;
   static_assert(Tile::DMA * (ST - 1) < 64, "the DMA instructions in flight must fit the 6-bit vmcnt");
@@ -1171,7 +1187,7 @@ __device__ __forceinline__ void bt_tile(const TileHead& head, int tiles_n, const
 }
 
 template <int MI, int NJ, int ST>
-__global__ __launch_bounds__(kHThreads) __attribute__((amdgpu_waves_per_eu(2))) void gemm_f16_bt_kernel(ET_HEAD_ARGS, GemmArgs args) {
+__global__ __launch_bounds__(kHThreads) __attribute__((amdgpu_waves_per_eu(2))) void gemm_f16_bt_kernel(ET_HEAD_ARGS, TileArgs args) {
   extern __shared__ __attribute__((aligned(1024))) unsigned char smem[];
   TileHead head = tile_head(a0, b0, rows_dev, m_bound, n, k, groups, args);
   head.ldc = columns;
@@ -1289,7 +1305,7 @@ __device__ __forceinline__ void wait_pairs(int pairs) {
 }
 constexpr int kWaveSlots = 13, kWaveSlotBytes = 2 * 16 * 128;
 
-__global__ __launch_bounds__(kWave) __attribute__((amdgpu_waves_per_eu(1))) void gemm_f16_bt_wave_kernel(ET_HEAD_ARGS, GemmArgs args) {
+__global__ __launch_bounds__(kWave) __attribute__((amdgpu_waves_per_eu(1))) void gemm_f16_bt_wave_kernel(ET_HEAD_ARGS, TileArgs args) {
 #if defined(__HIP_DEVICE_COMPILE__)   // device-only types in the body; the host pass only needs the stub
   constexpr int kAhead = kWaveSlots - 1;                          // pairs in flight behind the one in use
   static_assert(kAhead % 2 == 0 && 4 * kAhead < 64, "the register sets alternate; vmcnt has six bits");
@@ -1396,8 +1412,8 @@ __global__ __launch_bounds__(kWave) __attribute__((amdgpu_waves_per_eu(1))) void
   const int row = m0 + l16;
   if (row < rows && col < N) {
     half4 o = {f2h(acc[0]), f2h(acc[1]), f2h(acc[2]), f2h(acc[3])};
-    o = args.gelu ? bias_gelu_half<half4, 4>(o, biasv) : o + biasv;
-    *reinterpret_cast<half4*>((_Float16*)args.C + (size_t)row * args.ldc + (size_t)grp * N + col) = o;
+    o = walk & kBtGelu ? bias_gelu_half<half4, 4>(o, biasv) : o + biasv;
+    *reinterpret_cast<half4*>((_Float16*)args.C + (size_t)row * columns + (size_t)grp * N + col) = o;
   }
 #endif
 }
@@ -1596,6 +1612,8 @@ inline int best_strips_log2(int tiles_m, int tiles_n, int bm, int bn) {
   return best;
 }
 
+TileArgs tile_args(const GemmArgs& a) { return {a.A[1], a.B[1], a.B[2], {a.bias[0], a.bias[1], a.bias[2]}, a.C}; }
+
 template <int MI, int NJ, int ST>
 void launch_f16_bt(GemmArgs a, hipStream_t stream) {
   using Tile = BtTile<MI, NJ, ST>;
@@ -1607,7 +1625,7 @@ void launch_f16_bt(GemmArgs a, hipStream_t stream) {
   allow_dynamic_lds(reinterpret_cast<const void*>(kern), (int)Tile::SMEM_BYTES);
   const int strips = best_strips_log2(a.tiles_m, a.tiles_n * a.groups, Tile::BM, Tile::BN);
   kern<<<a.per_xcd * kXcds, kHThreads, Tile::SMEM_BYTES, stream>>>(a.A[0], a.B[0], a.rows_dev, a.m_bound, a.n, a.k, a.groups, a.tiles_n, a.ldc,
-                                                                    strips << kBtStrips | (a.gelu ? kBtGelu : 0), a);
+                                                                    strips << kBtStrips | (a.gelu ? kBtGelu : 0), tile_args(a));
 }
 
 int device_cu_count() {
@@ -1794,7 +1812,7 @@ bool launch_bt_wave(GemmArgs a, hipStream_t stream) {
   if (!aligned) return false;
   constexpr int lds = kWaveSlots * kWaveSlotBytes;
   gemm_f16_bt_wave_kernel<<<(int)((wgs + kXcds - 1) / kXcds * kXcds), kWave, lds, stream>>>(a.A[0], a.B[0], a.rows_dev, a.m_bound, a.n, a.k, a.groups,
-                                                                                             a.tiles_n, 0, 0, a);
+                                                                                             a.tiles_n, a.ldc, a.gelu ? kBtGelu : 0, tile_args(a));
   return true;
 }
 
@@ -1970,7 +1988,7 @@ void launch_gemm(DType t, const GemmGroups& g, void* C, int ldc, int m_bound, in
   }
   GemmArgs a;
   for (int i = 0; i < 3; ++i) {
-    a.A[i] = i < g.groups ? g.A[i] : nullptr;
+    a.A[i] = i < g.groups ? g.A[i > 0] : nullptr;
     a.B[i] = i < g.groups ? g.B[i] : nullptr;
     a.bias[i] = i < g.groups ? g.bias[i] : nullptr;
   }

@@ -478,7 +478,7 @@ void launch_gemm_split(const GemmGroups& g, void* C, int ldc, int m_bound, int n
   if (m_bound <= 0) return;
   SplitGemmArgs a;
   for (int i = 0; i < 3; ++i) {
-    a.A[i] = i < g.groups ? (const uint16_t*)g.A[i] : nullptr;
+    a.A[i] = i < g.groups ? (const uint16_t*)g.A[i > 0] : nullptr;
     a.B[i] = i < g.groups ? (const uint16_t*)g.B[i] : nullptr;
     a.bias[i] = i < g.groups ? (const float*)g.bias[i] : nullptr;
   }

@@ -157,7 +157,7 @@ void launch_gemm_generic(DType t, const GemmGroups& g, void* C, int ldc, int m_b
                          const int32_t* rows_dev, hipStream_t stream) {
   GenericGemmArgs a;
   for (int i = 0; i < 3; ++i) {
-    a.A[i] = i < g.groups ? g.A[i] : nullptr;
+    a.A[i] = i < g.groups ? g.A[i > 0] : nullptr;
     a.B[i] = i < g.groups ? g.B[i] : nullptr;
     a.bias[i] = i < g.groups ? g.bias[i] : nullptr;
   }

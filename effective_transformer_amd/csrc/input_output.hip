@@ -157,13 +157,13 @@ template <typename CH>
 __global__ __launch_bounds__(kMoveThreads) void compress_rows_kernel(
     const CH* __restrict__ from, CH* __restrict__ to, const int32_t* __restrict__ batch_idx,
     const int32_t* __restrict__ word_idx, const int32_t* __restrict__ rows_dev, const int32_t* __restrict__ prefix,
-    const int32_t* __restrict__ mask, int n_pos, int seq_len, fastdiv cpr, CompressExtras extras) {
+    const int32_t* __restrict__ mask, int n_pos, int seq_len, fastdiv cpr, int32_t* seq_table, uint16_t* split) {
   // the first workgroup sorts the sequence table whose first half the scan wrote, where that is asked for
   uint32_t block = blockIdx.x;
-  if (extras.seq_table) {
+  if (seq_table) {
     if (block == 0) {
       const int batch = n_pos / seq_len;
-      sort_sequences<kMoveThreads>(extras.seq_table, batch, extras.seq_table + batch + 1);
+      sort_sequences<kMoveThreads>(seq_table, batch, seq_table + batch + 1);
       return;
     }
     --block;
@@ -202,10 +202,10 @@ __global__ __launch_bounds__(kMoveThreads) void compress_rows_kernel(
   for (int u = 0; u < kMoveUnroll; ++u) to[idx[u]] = val[u];
   // float rows once more as split rows, the form the first layer's products read
   if constexpr (sizeof(CH) == 16)
-    if (extras.split) {
+    if (split) {
 #pragma unroll
       for (int u = 0; u < kMoveUnroll; ++u)
-        store_split<4>(extras.split + (size_t)row[u] * cpr.d * 12, (int)chunk[u] * 4, __builtin_bit_cast(float4v, val[u]));
+        store_split<4>(split + (size_t)row[u] * cpr.d * 12, (int)chunk[u] * 4, __builtin_bit_cast(float4v, val[u]));
     }
 }
 
@@ -410,15 +410,15 @@ void launch_compress_rows(const void* from, void* to, const int32_t* batch_idx, 
   if (cb == 16)
     compress_rows_kernel<u32x4><<<grid, kMoveThreads, 0, stream>>>((const u32x4*)from, (u32x4*)to, batch_idx, word_idx,
                                                                    rows_dev, prefix, mask, n_pos, seq_len, make_fastdiv(cpr),
-                                                                   extras);
+                                                                   extras.seq_table, extras.split);
   else if (cb == 4)
     compress_rows_kernel<uint32_t><<<grid, kMoveThreads, 0, stream>>>((const uint32_t*)from, (uint32_t*)to, batch_idx,
                                                                       word_idx, rows_dev, prefix, mask, n_pos, seq_len,
-                                                                      make_fastdiv(cpr), extras);
+                                                                      make_fastdiv(cpr), extras.seq_table, extras.split);
   else
     compress_rows_kernel<uint16_t><<<grid, kMoveThreads, 0, stream>>>((const uint16_t*)from, (uint16_t*)to, batch_idx,
                                                                       word_idx, rows_dev, prefix, mask, n_pos, seq_len,
-                                                                      make_fastdiv(cpr), extras);
+                                                                      make_fastdiv(cpr), extras.seq_table, extras.split);
 }
 
 void launch_restore_rows(void* to, const void* from, const int32_t* batch_idx, const int32_t* word_idx,

@@ -162,7 +162,7 @@ bool attention_writes_pieces(const void* q, const void* k, const void* v, int la
 // computes C[:, g*n : (g+1)*n] = A[g] . B[g] (+ bias[g]) into a row-major C with leading
 // dimension ldc.  groups == 1 is the plain GEMM.
 struct GemmGroups {
-  const void* A[3];
+  const void* A[2];                  // of the first group, of the others
   const void* B[3];
   const void* bias[3];
   int groups;

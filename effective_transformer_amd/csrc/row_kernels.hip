@@ -83,18 +83,26 @@ template <int VEC> struct RowVec<_Float16, VEC> {
   typedef _Float16 type __attribute__((ext_vector_type(VEC)));
 };
 
+// What fp32 rows are left as beside themselves; nothing in fp16, whose launches keep to 112 bytes of arguments (TileArgs in gemm.hip has the
+// reason; the number of wavefronts is one of them, since the size of the grid would come as 256 bytes more).
+template <typename T> struct RowForms {
+  uint16_t* split;
+  PairRows pair;
+};
+template <> struct RowForms<_Float16> {
+  RowForms(uint16_t*, const PairRows&) {}
+};
+
 // VEC elements per lane per access, ITERS accesses per row: the row has n <= 64*VEC*ITERS
 // elements, n % VEC == 0.
 template <typename T, int VEC, int ITERS>
 __global__ __launch_bounds__(kLnThreads) void bias_residual_layernorm_kernel(
     T* __restrict__ out, const T* __restrict__ input, const T* __restrict__ bias, const T* __restrict__ gamma,
-    const T* __restrict__ beta, int m, int n, const int32_t* __restrict__ rows_dev, WarmList warm,
-    uint16_t* __restrict__ split, PairRows pair) {
+    const T* __restrict__ beta, int m, int n, const int32_t* __restrict__ rows_dev, int nwaves, WarmList warm, RowForms<T> forms) {
   using V = typename RowVec<T, VEC>::type;
   const int rows = rows_dev ? min(*rows_dev, m) : m;
   const int lane = threadIdx.x & (kWave - 1);
   const int wave = blockIdx.x * kLnWaves + threadIdx.x / kWave;
-  const int nwaves = gridDim.x * kLnWaves;
   const int vpr = n / VEC;                       // vectors per row
 
   V b[ITERS], g[ITERS], be[ITERS];
@@ -150,7 +158,7 @@ __global__ __launch_bounds__(kLnThreads) void bias_residual_layernorm_kernel(
     }
     const float rstd = __builtin_amdgcn_rsqf(wave_sum(sq) * inv_n + 1e-6f);
     if constexpr (sizeof(T) == 4 && VEC == 4)
-      if (pair.rows) {
+      if (forms.pair.rows) {
         V y[ITERS];
 #pragma unroll
         for (int i = 0; i < ITERS; ++i) {
@@ -162,7 +170,7 @@ __global__ __launch_bounds__(kLnThreads) void bias_residual_layernorm_kernel(
             orow[c] = y[i];
           }
         }
-        store_pair_row<ITERS>(y, vpr, pair, r, n);
+        store_pair_row<ITERS>(y, vpr, forms.pair, r, n);
         return;
       }
 #pragma unroll
@@ -175,7 +183,7 @@ __global__ __launch_bounds__(kLnThreads) void bias_residual_layernorm_kernel(
         orow[c] = y;
         // fp32: the form the next product reads (6 bytes a value more here, a pass of 10 bytes a value less)
         if constexpr (sizeof(T) == 4 && VEC == 4)
-          if (split) store_split<4>(split + (size_t)r * 3 * n, c * VEC, y);
+          if (forms.split) store_split<4>(forms.split + (size_t)r * 3 * n, c * VEC, y);
       }
     }
   };
@@ -186,7 +194,7 @@ __global__ __launch_bounds__(kLnThreads) void bias_residual_layernorm_kernel(
   // wait for it as well), and are only looked at behind the row loop.  In front of the first row, which then came a trip to memory
   // later: 12 layers of BERT-base in graphs for 16 x 64 positions 574 us, 549 so, for 1 x 32 365 and 355; from 2000 rows on 1 to 2 %.
   if (wave < rows) request(wave);
-  const int line = (int)blockIdx.x * kLnThreads + (int)threadIdx.x, lines = (int)gridDim.x * kLnThreads;
+  const int line = (int)blockIdx.x * kLnThreads + (int)threadIdx.x, lines = nwaves * kWave;
   static_assert(WarmList::kMax == 3);
   const int end0 = warm.lines[0], end1 = end0 + warm.lines[1];
   auto word = [&](int i) {
@@ -340,7 +348,8 @@ void ln_launch_kernel(hipStream_t stream, T* out, const T* input, const T* bias,
                       const int32_t* rows_dev, const WarmList& warm, uint16_t* split, const PairRows& pair) {
   const long lines = (warm.total + kLnThreads - 1) / kLnThreads;
   const int grid = (int)min(max(((long)m + kLnWaves - 1) / kLnWaves, lines), 256L * 8);
-  bias_residual_layernorm_kernel<T, VEC, ITERS><<<grid, kLnThreads, 0, stream>>>(out, input, bias, gamma, beta, m, n, rows_dev, warm, split, pair);
+  bias_residual_layernorm_kernel<T, VEC, ITERS><<<grid, kLnThreads, 0, stream>>>(out, input, bias, gamma, beta, m, n, rows_dev, grid * kLnWaves, warm,
+                                                                                 RowForms<T>{split, pair});
 }
 
 template <typename T, int VEC>
