@@ -51,9 +51,9 @@ hipError_t take_attribute_error() {
 
 namespace {
 
-// The persistent GEMM stores C with plain stores while the matrices of a layer (resp. A and C of a stand-alone call)
+// The persistent GEMM writes C through the L2s while the matrices of a layer (resp. A and C of a stand-alone call)
 // are small enough to be found in the 256 MB last-level cache by the kernels that read them next, and with non-temporal
-// stores beyond.  12-layer BERT-base, fp16: plain stores -6 % at 4000 tokens, -2.4 % at 15900, +-0.5 % at 20000,
+// stores beyond.  12-layer BERT-base, fp16: without non-temporal stores -6 % at 4000 tokens, -2.4 % at 15900, +-0.5 % at 20000,
 // +2 % at 30000 and 40000; 24-layer BERT-large at 13100 tokens: -0.4 %.
 constexpr double kCachedLayerBytes = 320.0 * 1048576.0;
 constexpr double kCachedCallBytes = 96.0 * 1048576.0;
@@ -552,7 +552,7 @@ et_status run_layer(et_handle h, const LayerCall& c) {
   };
   // Every matrix of the layer is read again by the kernel after the one that wrote it.  While the layer's matrices
   // (from, Q/K/V, context, attention output, [T,4H], out) about fit the last-level cache, the GEMMs leave their
-  // outputs there (plain stores); beyond that the outputs would only displace the weights and the A rows.
+  // outputs there (written through the L2s); beyond that the outputs would only displace the weights and the A rows.
   const bool cached = (double)rows * (7.0 * H + F) * (double)e <= kCachedLayerBytes;
   // Q = from.Wq + bq, K = to.Wk + bk, V = to.Wv + bv into one [T,3H] buffer (bert_transformer_op.cu.cc:105-156)
   et::GemmGroups g3;

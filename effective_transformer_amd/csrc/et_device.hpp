@@ -118,6 +118,23 @@ __device__ __forceinline__ uint32_t div_by(uint32_t n, const fastdiv& f) {
 __device__ __forceinline__ float h2f(_Float16 h) { return (float)h; }
 __device__ __forceinline__ _Float16 f2h(float f) { return (_Float16)f; }   // v_cvt_f16_f32, round-to-nearest-even
 
+// ---- stores ------------------------------------------------------------------------------
+// Cache policy of buffer stores: sc1 writes through the L2 to the memory side, where the other XCDs find the value; nt keeps less of
+// the line in the caches on its way.  What lies dirty in the L2s when a kernel ends is written back before the next one starts, which
+// the products' C and the streaming attention's rows are spared so.  Encoders of 12 layers, plain stores and written through, one card
+// in turn: 16 x 64 in a graph 508 -> 502 us, 8 x 128 from ids 475 -> 466, 100 x 32 753 -> 730, the ops on 217 x 53 1877 -> 1809, 32 x 512
+// 2858 -> 2790, 16 x 1024 2841 -> 2693 (another card: 32 x 512 2707 -> 2676, ops level).  It takes stores that fill their lines in
+// whole pieces of 8 or 16 bytes a lane: 16 bytes in two stores of 8 are written twice (ops 1809 -> 1895).  Level or worse, and so plain:
+// LayerNorm's rows, the short attention (1000 x 64 7435 -> 7655), fp32
+// products (500 x 64 +0.7 %).  Matrices beyond the last-level cache keep nt (1000 x 64: sc1 instead or both +0.2 to +0.5 %).
+constexpr int kPolicyNt = 2, kPolicyThrough = 16;
+// 8 bytes, written through.
+template <typename V>
+__device__ __forceinline__ void store_through(void* p, const V& v) {
+  static_assert(sizeof(V) == 8);
+  __hip_atomic_store(reinterpret_cast<uint64_t*>(p), __builtin_bit_cast(uint64_t, v), __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+}
+
 // ---- bias + GELU arithmetic (reference: cuda/cuda_kernels.cu:29-51) -------------------------
 // 0.5*(1+tanh(u)) is evaluated as 1/(1+exp(-2u)), which is the same function without the cancellation of 1+tanh for
 // negative u.
@@ -192,8 +209,13 @@ __device__ __forceinline__ void store_pair(_Float16* row, int col, const V& v, f
 #pragma unroll
   for (int j = 0; j < N; ++j) l[j] = f2h(__builtin_fmaf(v[j], scale, -h2f(h[j])));
   _Float16* d = row + (col >> 5) * 64 + (col & 31);
+  if constexpr (N == 4) {
+    store_through(d, h);
+    store_through(d + 32, l);
+  } else {
   *reinterpret_cast<hvec*>(d) = h;
   *reinterpret_cast<hvec*>(d + 32) = l;
+  }
 }
 // Row r of `out` from a wavefront that holds it, lane + 64 i the i-th four values (zero beyond vpr): the exponent from the
 // largest value, and the row's Euclidean norm.  Whoever writes a row writes the same bits.

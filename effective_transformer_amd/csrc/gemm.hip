@@ -40,7 +40,7 @@ struct GemmArgs {
   int gelu = 0;              // C = gelu(A.B + bias) instead of A.B + bias (bias must be set)
   int a_blocked = 0;         // pair kernel: A / C hold every tile of 256 rows as blocks of [256 rows][64 columns]
   int c_blocked = 0;         //   (see GemmGroups)
-  int c_cached = 0;          // persistent k-contiguous kernel: plain stores for C instead of non-temporal ones
+  int c_cached = 0;          // persistent k-contiguous kernel: C written through the L2s (kPolicyThrough) instead of by non-temporal stores
 };
 
 typedef uint32_t uint4v __attribute__((ext_vector_type(4)));
@@ -604,7 +604,7 @@ __device__ __forceinline__ TileHead tile_head(const void* a0, const void* b0, co
 // chooses).  The A part of an LDS slot keeps its 256 rows; the rows beyond the tile lie outside the tile's buffer
 // descriptor and cost no traffic.
 // NT: C leaves through non-temporal stores (a matrix too big to be found in the last-level cache by its reader);
-// plain stores otherwise.
+// stores that write through otherwise.
 // kThreeA: three LDS slots for A instead of two, all of the 160 KB: the A rows of a pair are requested three pairs ahead
 // of their first use instead of two (B^T as before).  For the projection whose A is the big matrix and comes from
 // HBM (k >= 2048: FFN-down), where a pair's time does not cover that latency.  Same instructions on the same data in
@@ -912,7 +912,7 @@ __device__ __forceinline__ void pair_tiles(const TileHead& head, int tiles_n, in
             for (int j = 0; j < 4; ++j) o[j] = f2h(acc[i][j][r]);
             // GELU here costs no pass over C: its arithmetic runs while the stores of the tile drain
             o = GELU ? bias_gelu_half<half4, 4>(o, bias4) : o + bias4;
-            __builtin_amdgcn_raw_buffer_store_b64(__builtin_bit_cast(uint2v, o), rc, voff, 0, NT ? 2 /* nt */ : 0);
+            __builtin_amdgcn_raw_buffer_store_b64(__builtin_bit_cast(uint2v, o), rc, voff, 0, NT ? kPolicyNt : kPolicyThrough);
             voff += row_bytes;
           }
           voff += 12u * row_bytes;
@@ -1134,8 +1134,8 @@ __device__ __forceinline__ void bt_tile(const TileHead& head, int tiles_n, const
     step(Odd{}, std::false_type{}, std::true_type{}, s1, s, p + ST);      // pair p+ST replaces slot s
     s = s1;
   }
-  // Epilogue: the lane owns rows g*4+r of every 16-row block and NJ consecutive columns.  Plain stores, not the
-  // non-temporal ones of the persistent kernel: the output of a launch this small is still in the caches when the
+  // Epilogue: the lane owns rows g*4+r of every 16-row block and NJ consecutive columns.  Not the
+  // non-temporal stores of the persistent kernel: the output of a launch this small is still in the caches when the
   // next kernel reads it (12 layers on 2000 tokens: 0.905 -> 0.843 ms; no difference from about 4000 tokens on).
   // C leaves through a descriptor that ends with the tile's last valid row, which drops the rows beyond it, and a row's offset is a
   // scalar.  With a branch, a 64-bit address and scalar loads of ldc and the GELU flag at every row, each waited for, a launch of
@@ -1160,10 +1160,10 @@ __device__ __forceinline__ void bt_tile(const TileHead& head, int tiles_n, const
           for (int j = 0; j < NB; ++j) o[j] = f2h(acc[i][j][r]);
           if constexpr (GELU) o = bias_gelu_half<BiasN, NB>(o, biasv);
           else o = o + biasv;
-          if constexpr (NB == 1) __builtin_amdgcn_raw_buffer_store_b16(__builtin_bit_cast(uint16_t, o), rsrc_c, voff, soff, 0);
-          else if constexpr (NB == 2) __builtin_amdgcn_raw_buffer_store_b32(__builtin_bit_cast(uint32_t, o), rsrc_c, voff, soff, 0);
-          else if constexpr (NB == 4) __builtin_amdgcn_raw_buffer_store_b64(__builtin_bit_cast(uint2v, o), rsrc_c, voff, soff, 0);
-          else __builtin_amdgcn_raw_buffer_store_b128(__builtin_bit_cast(uint4v, o), rsrc_c, voff, soff, 0);
+          if constexpr (NB == 1) __builtin_amdgcn_raw_buffer_store_b16(__builtin_bit_cast(uint16_t, o), rsrc_c, voff, soff, kPolicyThrough);
+          else if constexpr (NB == 2) __builtin_amdgcn_raw_buffer_store_b32(__builtin_bit_cast(uint32_t, o), rsrc_c, voff, soff, kPolicyThrough);
+          else if constexpr (NB == 4) __builtin_amdgcn_raw_buffer_store_b64(__builtin_bit_cast(uint2v, o), rsrc_c, voff, soff, kPolicyThrough);
+          else __builtin_amdgcn_raw_buffer_store_b128(__builtin_bit_cast(uint4v, o), rsrc_c, voff, soff, kPolicyThrough);
         }
       if (NJ == 6 && ok2) {                      // the other two of a lane's six columns
 #pragma unroll
@@ -1173,7 +1173,7 @@ __device__ __forceinline__ void bt_tile(const TileHead& head, int tiles_n, const
             half2v o = {f2h(acc[i][NJ - 2][r]), f2h(acc[i][NJ - 1][r])};
             if constexpr (GELU) o = bias_gelu_half<half2v, 2>(o, bias2);
             else o = o + bias2;
-            __builtin_amdgcn_raw_buffer_store_b32(__builtin_bit_cast(uint32_t, o), rsrc_c, voff2, (i * 16 + r) * head.ldc * 2, 0);
+            __builtin_amdgcn_raw_buffer_store_b32(__builtin_bit_cast(uint32_t, o), rsrc_c, voff2, (i * 16 + r) * head.ldc * 2, kPolicyThrough);
           }
       }
     };
@@ -1413,7 +1413,7 @@ __global__ __launch_bounds__(kWave) __attribute__((amdgpu_waves_per_eu(1))) void
   if (row < rows && col < N) {
     half4 o = {f2h(acc[0]), f2h(acc[1]), f2h(acc[2]), f2h(acc[3])};
     o = walk & kBtGelu ? bias_gelu_half<half4, 4>(o, biasv) : o + biasv;
-    *reinterpret_cast<half4*>((_Float16*)args.C + (size_t)row * columns + (size_t)grp * N + col) = o;
+    store_through((_Float16*)args.C + (size_t)row * columns + (size_t)grp * N + col, o);
   }
 #endif
 }

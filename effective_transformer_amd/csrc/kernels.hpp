@@ -179,7 +179,7 @@ struct GemmGroups {
   // gemm_blocked_handover() says so; the matrix must be allocated for a whole number of 256-row tiles.
   bool c_blocked = false, a_blocked = false;
   // C is read again by the next kernels while it can still be in the last-level cache (the working set of the layer
-  // or of the call fits it a few times over): the persistent kernel then stores C with plain stores.  Its non-temporal
+  // or of the call fits it a few times over): the persistent kernel then writes C through the L2s.  Its non-temporal
   // stores are the better choice when C would only push the weights and the A rows out of that cache.
   bool c_cached = false;
 };
