@@ -135,6 +135,17 @@ __device__ __forceinline__ void store_through(void* p, const V& v) {
   __hip_atomic_store(reinterpret_cast<uint64_t*>(p), __builtin_bit_cast(uint64_t, v), __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
 }
 
+#if defined(__HIP_DEVICE_COMPILE__)
+// 16 bytes a lane at byte `off` from `base`, which is the same for the whole wavefront, written through.
+template <typename V>
+__device__ __forceinline__ void store_through(void* base, uint32_t off, const V& v) {
+  static_assert(sizeof(V) == 16);
+  typedef uint32_t uint4v __attribute__((ext_vector_type(4)));
+  const __amdgpu_buffer_rsrc_t r = __builtin_amdgcn_make_buffer_rsrc(base, 0, ~0u, 0x00020000);
+  __builtin_amdgcn_raw_buffer_store_b128(__builtin_bit_cast(uint4v, v), r, off, 0, kPolicyThrough);
+}
+#endif
+
 // ---- bias + GELU arithmetic (reference: cuda/cuda_kernels.cu:29-51) -------------------------
 // 0.5*(1+tanh(u)) is evaluated as 1/(1+exp(-2u)), which is the same function without the cancellation of 1+tanh for
 // negative u.
