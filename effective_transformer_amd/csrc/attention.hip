@@ -1135,7 +1135,7 @@ __global__ __launch_bounds__(kFlWaves * kWave, 4) void attention_flash_kernel(
     if (tq < 0) continue;
     T* orow = dst + (size_t)(t0 + tq) * H + head * kD + g * 4;
 #pragma unroll
-    for (int dt = 0; dt < 4; ++dt) store_through(orow + dt * 16, __builtin_convertvector(o[u][dt] * inv, half4));
+    for (int dt = 0; dt < 4; ++dt) *reinterpret_cast<half4*>(orow + dt * 16) = __builtin_convertvector(o[u][dt] * inv, half4);
   }
 #endif
 }

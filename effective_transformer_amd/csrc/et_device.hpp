@@ -121,12 +121,13 @@ __device__ __forceinline__ _Float16 f2h(float f) { return (_Float16)f; }   // v_
 // ---- stores ------------------------------------------------------------------------------
 // Cache policy of buffer stores: sc1 writes through the L2 to the memory side, where the other XCDs find the value; nt keeps less of
 // the line in the caches on its way.  What lies dirty in the L2s when a kernel ends is written back before the next one starts, which
-// the products' C and the streaming attention's rows are spared so.  Encoders of 12 layers, plain stores and written through, one card
-// in turn: 16 x 64 in a graph 508 -> 502 us, 8 x 128 from ids 475 -> 466, 100 x 32 753 -> 730, the ops on 217 x 53 1877 -> 1809, 32 x 512
-// 2858 -> 2790, 16 x 1024 2841 -> 2693 (another card: 32 x 512 2707 -> 2676, ops level).  It takes stores that fill their lines in
+// the fp16 products' C and the weights' turned copies are spared so.  Encoders of 12 layers, C in plain stores and written through, one
+// card in turn: 16 x 64 in a graph 508 -> 502 us, 8 x 128 from ids 475 -> 467, 100 x 32 753 -> 730, the ops on 217 x 53 1877 -> 1810, 32 x 512
+// 2858 -> 2788, 16 x 1024 2841 -> 2692 (another card: 32 x 512 2707 -> 2676, ops level).  It takes stores that fill their lines in
 // whole pieces of 8 or 16 bytes a lane: 16 bytes in two stores of 8 are written twice (ops 1809 -> 1895).  Level or worse, and so plain:
-// LayerNorm's rows, the short attention (1000 x 64 7435 -> 7655), fp32
-// products (500 x 64 +0.7 %).  Matrices beyond the last-level cache keep nt (1000 x 64: sc1 instead or both +0.2 to +0.5 %).
+// LayerNorm's rows, the short attention (1000 x 64 7435 -> 7655), the streaming one (8-byte pieces of a head's rows: 64 x 512 5412 -> 5538,
+// 193 x 100 2995 -> 3055), fp32 products (500 x 64 +0.7 %).  Matrices beyond the last-level cache keep nt (1000 x 64: sc1 instead or both
+// +0.2 to +0.5 %).
 constexpr int kPolicyNt = 2, kPolicyThrough = 16;
 // 8 bytes, written through.
 template <typename V>

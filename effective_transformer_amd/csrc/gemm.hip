@@ -1928,6 +1928,8 @@ __global__ __launch_bounds__(256) void layer_prologue_kernel(TransposeArgs args)
     if (K < 1 << 28) store_through(dst + (size_t)(n0 + first) * K + k0, ((uint32_t)in * (uint32_t)K + c * 8u) * 2u, v);
     else *reinterpret_cast<half8*>(dst + (size_t)(n0 + r) * K + k0 + c * 8) = v;       // (beyond what 32 bits of an offset reach)
   }
+#else
+  (void)dst;
 #endif
 }
 
