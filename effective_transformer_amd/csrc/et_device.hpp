@@ -126,7 +126,7 @@ __device__ __forceinline__ _Float16 f2h(float f) { return (_Float16)f; }   // v_
 // 2858 -> 2788, 16 x 1024 2841 -> 2692 (another card: 32 x 512 2707 -> 2676, ops level).  It takes stores that fill their lines in
 // whole pieces of 8 or 16 bytes a lane: 16 bytes in two stores of 8 are written twice (ops 1809 -> 1895).  Level or worse, and so plain:
 // LayerNorm's rows, the short attention (1000 x 64 7435 -> 7655), the streaming one (8-byte pieces of a head's rows: 64 x 512 5412 -> 5538,
-// 193 x 100 2995 -> 3055), fp32 products (500 x 64 +0.7 %).  Matrices beyond the last-level cache keep nt (1000 x 64: sc1 instead or both
+// 193 x 100 2995 -> 3055), the fp32 products' C in floats (500 x 64 11330 -> 11440, 210 x 64 5538 -> 5601).  Matrices beyond the last-level cache keep nt (1000 x 64: sc1 instead or both
 // +0.2 to +0.5 %).
 constexpr int kPolicyNt = 2, kPolicyThrough = 16;
 // 8 bytes, written through.
@@ -211,6 +211,8 @@ __device__ __forceinline__ float pair_scale(int e) { return __builtin_ldexpf(1.0
 // The epilogues that store pair rows are bound by their arithmetic: with l made from the stored halves a pair of values takes one
 // conversion, where the compiler converted every value a second time for l (FFN-up on 20375 rows 277 -> 263 us together with
 // gemm_pair_kernel's one lane per exponent, same bits).
+// Pieces of 8 bytes, those of FFN-up's large tiles, of LayerNorm and of the short attention, are written through (kPolicyThrough): fp32
+// encoders of 12 layers, plain and so, 40 x 64 positions 1740 -> 1705 us, 100 x 64 2936 -> 2908, 210 x 64 5573 -> 5538, 500 x 64 11425 -> 11330.
 template <int N, typename V>
 __device__ __forceinline__ void store_pair(_Float16* row, int col, const V& v, float scale) {
   typedef _Float16 hvec __attribute__((ext_vector_type(N)));
@@ -225,8 +227,8 @@ __device__ __forceinline__ void store_pair(_Float16* row, int col, const V& v, f
     store_through(d, h);
     store_through(d + 32, l);
   } else {
-  *reinterpret_cast<hvec*>(d) = h;
-  *reinterpret_cast<hvec*>(d + 32) = l;
+    *reinterpret_cast<hvec*>(d) = h;
+    *reinterpret_cast<hvec*>(d + 32) = l;
   }
 }
 // Row r of `out` from a wavefront that holds it, lane + 64 i the i-th four values (zero beyond vpr): the exponent from the
