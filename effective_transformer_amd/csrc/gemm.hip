@@ -1418,6 +1418,108 @@ __global__ __launch_bounds__(kWave) __attribute__((amdgpu_waves_per_eu(1))) void
 #endif
 }
 
+// The same tile by four wavefronts: each brings one of the four requests of a pair, and the first one multiplies.  A request takes a
+// wavefront 46 cycles, 88 ns a pair for the one above, which overlaps them with its operand reads and MFMAs in part only; here the
+// chain is the reads and the MFMAs.  Chunks of four pairs, up to nine in the ring: at the barrier in front of a chunk everybody's share
+// of it is there, and the operands of the one before it have been read, which frees that one's slots.  The MFMAs of a chunk run
+// between the reads of the next one (behind them: k = 3072 5.3 us for 5.0).
+// us a launch on 20 rows, one wavefront and four: k = 4096, n = 1024 7.0 and 5.8; 3072, 768 5.7 and 5.0; 2048, 512 4.4 and 4.1;
+// k = n = 1024 3.19 and 3.12, 768 2.90 and 2.87, 512 2.63 and 2.54, 256 2.34 and 2.28.
+constexpr int kQuadPairs = 4, kQuadRing = 9, kQuadChunkBytes = kQuadPairs * kWaveSlotBytes;
+
+__global__ __launch_bounds__(kHThreads) void gemm_f16_bt_quad_kernel(ET_HEAD_ARGS, TileArgs args) {
+#if defined(__HIP_DEVICE_COMPILE__)   // device-only types in the body; the host pass only needs the stub
+  extern __shared__ __attribute__((aligned(1024))) unsigned char smem[];
+  const TileHead head = tile_head(a0, b0, rows_dev, m_bound, n, k, groups, args);
+  const int rows = head.rows, N = n, K = k;
+  const int tiles_m = (int)((unsigned)(rows + 15) / 16);
+  const int tile = remap_valid_tile(blockIdx.x, tiles_m * tiles_n * groups);
+  if (tile < 0) return;
+  const int tn_all = uniform_div(tile, tiles_m), tm = tile - tn_all * tiles_m;
+  const int grp = groups == 1 ? 0 : 2 - uniform_less(tn_all, tiles_n) - uniform_less(tn_all, 2 * tiles_n);
+  const int m0 = tm * 16, n0 = (tn_all - grp * tiles_n) * 16;
+  const int chunks = (int)((unsigned)K / (64 * kQuadPairs));
+  const int lane = threadIdx.x & (kWave - 1), l16 = lane & 15, g = lane >> 4;
+  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x / kWave);
+
+  // wavefronts 0 and 1: the upper and the lower eight rows of A, 2 and 3: of B^T
+  const bool of_b = wave >= 2;
+  const __amdgpu_buffer_rsrc_t rsrc = __builtin_amdgcn_make_buffer_rsrc(
+      const_cast<char*>(of_b ? head.b_of(grp) + (size_t)n0 * K * 2 : head.a_of(grp) + (size_t)m0 * K * 2), 0, min(of_b ? N - n0 : rows - m0, 16) * K * 2,
+      0x00020000);
+  const int row = (wave & 1) * 8 + (lane >> 3);
+  const uint32_t voff = ((uint32_t)row * (uint32_t)K + (uint32_t)((lane & 7) ^ pair_swizzle(row)) * 8u) * 2u;
+  auto issue = [&](int slot, int chunk) {
+#pragma unroll
+    for (int i = 0; i < kQuadPairs; ++i)
+      __builtin_amdgcn_raw_ptr_buffer_load_lds(rsrc, ET_LDS_PTR(smem + (slot * kQuadPairs + i) * kWaveSlotBytes + wave * 1024), 16, voff,
+                                               (chunk * kQuadPairs + i) * 128, 0, 0);
+  };
+#pragma unroll
+  for (int c = 0; c < kQuadRing; ++c)
+    if (c < chunks) issue(c, c);
+  const int col = n0 + g * 4;
+  half4 biasv = {(_Float16)-0.0f, (_Float16)-0.0f, (_Float16)-0.0f, (_Float16)-0.0f};
+  // (behind the first requests, see bt_tile; the waits below count it as one of a chunk's)
+  if (wave == 0)
+    if (const _Float16* bias = (const _Float16*)args.bias[grp]; bias != nullptr && col < N) biasv = *reinterpret_cast<const half4*>(bias + col);
+
+  const int sw = pair_swizzle(l16);
+  const int rd[2] = {l16 * 128 + ((g ^ sw) * 16), l16 * 128 + (((4 + g) ^ sw) * 16)};
+  half8 a[2][kQuadPairs][2], b[2][kQuadPairs][2];
+  float4v acc = {0.f, 0.f, 0.f, 0.f};
+  int slot = 0, before = kQuadRing - 1;                           // of the chunk in use and of the one in front of it
+  auto chunk = [&](auto Pc, auto first, int c) {
+    constexpr int P = decltype(Pc)::value;
+    // this wavefront's share of the chunk has landed, the ring's seven behind it may fly
+    if (chunks - 1 - c >= kQuadRing - 2) wait_vmcnt<kQuadPairs * (kQuadRing - 2)>();
+    else wait_pairs(chunks - 1 - c);
+    wait_lgkmcnt0();                                              // the operands of the chunk in front of it have been read
+    barrier_only();
+    if (!decltype(first)::value && c - 1 + kQuadRing < chunks) issue(before, c - 1 + kQuadRing);
+    if (wave == 0) {
+      // (an MFMA waits for the one before it, two reads fit in between)
+      const unsigned char* st = smem + slot * kQuadPairs * kWaveSlotBytes;
+#pragma unroll
+      for (int i = 0; i < kQuadPairs; ++i)
+#pragma unroll
+        for (int h = 0; h < 2; ++h) {
+          if constexpr (!decltype(first)::value) acc = __builtin_amdgcn_mfma_f32_16x16x32_f16(b[1 - P][i][h], a[1 - P][i][h], acc, 0, 0, 0);
+          b[P][i][h] = *reinterpret_cast<const half8*>(st + i * kWaveSlotBytes + 2048 + rd[h]);
+          a[P][i][h] = *reinterpret_cast<const half8*>(st + i * kWaveSlotBytes + rd[h]);
+          __builtin_amdgcn_sched_barrier(0);
+        }
+    }
+    before = slot;
+    slot = slot + 1 == kQuadRing ? 0 : slot + 1;
+  };
+  auto last = [&](auto Pc) {
+    constexpr int P = decltype(Pc)::value;
+#pragma unroll
+    for (int i = 0; i < kQuadPairs; ++i)
+#pragma unroll
+      for (int h = 0; h < 2; ++h) acc = __builtin_amdgcn_mfma_f32_16x16x32_f16(b[P][i][h], a[P][i][h], acc, 0, 0, 0);
+  };
+  using Even = std::integral_constant<int, 0>;
+  using Odd = std::integral_constant<int, 1>;
+  chunk(Even{}, std::true_type{}, 0);
+  int c = 1;
+  for (; c + 1 < chunks; c += 2) {
+    chunk(Odd{}, std::false_type{}, c);
+    chunk(Even{}, std::false_type{}, c + 1);
+  }
+  if (c < chunks) chunk(Odd{}, std::false_type{}, c);
+  if (wave != 0) return;                                          // (their requests have all landed)
+  if (c < chunks) last(Odd{});
+  else last(Even{});
+  if (m0 + l16 < rows && col < N) {
+    half4 o = {f2h(acc[0]), f2h(acc[1]), f2h(acc[2]), f2h(acc[3])};
+    o = walk & kBtGelu ? bias_gelu_half<half4, 4>(o, biasv) : o + biasv;
+    store_through((_Float16*)args.C + (size_t)(m0 + l16) * columns + (size_t)grp * N + col, o);
+  }
+#endif
+}
+
 // ------------------------------------------------------------------------------------------
 // fp32: 128x128x16 tile, 4 wavefronts (2x2) of 64x64, v_mfma_f32_32x32x2_f32
 // ------------------------------------------------------------------------------------------
@@ -1810,6 +1912,15 @@ bool launch_bt_wave(GemmArgs a, hipStream_t stream) {
   bool aligned = ((uintptr_t)a.C | (uintptr_t)a.ldc * 2) % 8 == 0;
   for (int g = 0; g < a.groups; ++g) aligned = aligned && (uintptr_t)a.bias[g] % 8 == 0;
   if (!aligned) return false;
+  // k of whole chunks and a CU for every tile.  Two tiles on a CU take turns at its LDS and its DMA, where four wavefronts are no help:
+  // k = 768, n = 768, 96 rows 3.0 us with one wavefront and 3.2 with four; k = 3072, which leaves no room for a second one, 5.8 and 8.9.
+  if (a.k % (64 * kQuadPairs) == 0 && wgs <= device_cu_count()) {
+    const int lds_quad = std::min(a.k / (64 * kQuadPairs), kQuadRing) * kQuadChunkBytes;
+    allow_dynamic_lds(reinterpret_cast<const void*>(gemm_f16_bt_quad_kernel), kQuadRing * kQuadChunkBytes);
+    gemm_f16_bt_quad_kernel<<<(int)((wgs + kXcds - 1) / kXcds * kXcds), kHThreads, lds_quad, stream>>>(
+        a.A[0], a.B[0], a.rows_dev, a.m_bound, a.n, a.k, a.groups, a.tiles_n, a.ldc, a.gelu ? kBtGelu : 0, tile_args(a));
+    return true;
+  }
   constexpr int lds = kWaveSlots * kWaveSlotBytes;
   gemm_f16_bt_wave_kernel<<<(int)((wgs + kXcds - 1) / kXcds * kXcds), kWave, lds, stream>>>(a.A[0], a.B[0], a.rows_dev, a.m_bound, a.n, a.k, a.groups,
                                                                                              a.tiles_n, a.ldc, a.gelu ? kBtGelu : 0, tile_args(a));
