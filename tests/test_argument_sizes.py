@@ -3,7 +3,7 @@ import pytest
 
 from test_kernel_arguments import _argument_bytes, _kernels
 
-FEW_ROWS = ("gemm_f16_bt_kernel", "gemm_f16_bt_wave_kernel", "bias_residual_layernorm_kernelIDF16_", "16attention_kernelIDF16_",
+FEW_ROWS = ("gemm_f16_bt_kernel", "gemm_f16_bt_wave_kernel", "gemm_f16_bt_quad_kernel", "bias_residual_layernorm_kernelIDF16_", "16attention_kernelIDF16_",
             "attention_flash_kernel", "compress_rows_kernel", "mapped_restore_rows_kernel", "scan_index_kernel", "mask_class_kernel")
 
 
