@@ -511,10 +511,13 @@ int device_cu_count() {
 // Tile of a launch.  Below a round of the chip a launch takes the k loop of one tile, so small problems want small tiles;
 // large ones want the tile with the fewest operand bytes per product.  A launch takes rounds of tiles over the CUs, each
 // as long as its k-steps and a part for filling the ring and storing C.
-enum PairPick { p256x128, p192x128, p128x128, p96x128, p64x128, p64x64, p32x64, p32x32, kPairPicks };
+// 16 x 32 is for launches of one round: a k loop of small tiles is bound by what the LDS takes in and gives out, 12 KB and 16 KB a
+// stage of 64 k where 32 x 32 has 16 and 32 (us a launch, 32 x 32 and it: k = 2048, 16 to 64 rows to 768 columns 9.8 and 8.6, 160 rows 10.3 and
+// 9.3; k = 768 5.6 and 5.3; k = 512, 240 rows to 512 columns 4.7 and 4.6; in two rounds 300 rows to 768 5.7 and 9.0).
+enum PairPick { p256x128, p192x128, p128x128, p96x128, p64x128, p64x64, p32x64, p32x32, p16x32, kPairPicks };
 PairPick pick_pair_tile(int m, int n, int k, int groups, bool heads) {
   static constexpr struct { int bm, bn; float step; } kTiles[] = {
-      {256, 128, 0.8f}, {192, 128, 0.66f}, {128, 128, 0.48f}, {96, 128, 0.4f}, {64, 128, 0.3f}, {64, 64, 0.19f}, {32, 64, 0.135f}, {32, 32, 0.085f}};
+      {256, 128, 0.8f}, {192, 128, 0.66f}, {128, 128, 0.48f}, {96, 128, 0.4f}, {64, 128, 0.3f}, {64, 64, 0.19f}, {32, 64, 0.135f}, {32, 32, 0.085f}, {16, 32, 0.07f}};
   const long cus = device_cu_count();
   int best = 0;
   float best_cost = 0.f;
@@ -531,6 +534,28 @@ PairPick pick_pair_tile(int m, int n, int k, int groups, bool heads) {
   return (PairPick)best;
 }
 
+// `columns` of a launch of one round: the strips of columns with which an XCD's band of tiles touches the fewest operand rows, which is
+// what its L2 has to fetch (a band along all columns fetches all of the weights).  us a launch, one strip and so, k = 768: 160 rows to 768
+// columns 6.1 -> 5.6, 240 rows 6.5 -> 5.6, 64 rows to 2304 6.2 -> 5.9, 160 rows to 2304 7.9 -> 7.6.  Only where they save more than a
+// quarter and the weights are twice as long as A, whose rows the strips fetch more often (480 rows to 768 columns in strips: 12 layers
+// 1048 -> 1055 us).
+int one_round_columns(int columns, int tiles_m, int tiles_n, int bm, int bn) {
+  const int band = (tiles_m * tiles_n + kXcds - 1) / kXcds;
+  auto rows = [&](int wide) {
+    const int strip = tiles_m * wide;
+    if (band <= strip) return std::min(tiles_m, (band + wide - 1) / wide) * bm + std::min(band, wide) * bn;
+    return tiles_m * bm + (band + strip - 1) / strip * wide * bn;
+  };
+  if (tiles_n * bn < 2 * tiles_m * bm) return columns;
+  int best = columns, limit = (3 * rows(columns) - 1) / 4;
+  for (int strips = 2; strips <= tiles_n; ++strips) {
+    if (tiles_n % strips != 0) continue;
+    const int r = rows(tiles_n / strips);
+    if (r <= limit) best = tiles_n / strips, limit = r - 1;
+  }
+  return best;
+}
+
 template <int WM, int WN, int MI, int NJ, int ST, int KS>
 void launch_tile(PairGemmArgs a, bool gelu, int groups, const uint32_t* head_exp, hipStream_t stream) {
   using Tile = PairTile<WM, WN, MI, NJ, ST, KS>;
@@ -543,7 +568,8 @@ void launch_tile(PairGemmArgs a, bool gelu, int groups, const uint32_t* head_exp
   a.columns = tiles_n_all;
   for (int c = 2; c <= tiles_n_all; ++c)
     if (tiles_n_all % c == 0 && tiles_n_all / c * Tile::BN >= 768) a.columns = tiles_n_all / c;
-  const int tiles = ((a.m_bound + Tile::BM - 1) / Tile::BM) * tiles_n_all;
+  const int tiles_m = (a.m_bound + Tile::BM - 1) / Tile::BM, tiles = tiles_m * tiles_n_all;
+  if (tiles <= device_cu_count()) a.columns = one_round_columns(a.columns, tiles_m, tiles_n_all, Tile::BM, Tile::BN);
   // (a stream of fewer stages than the ring holds must not cross into a second tile)
   const int grid = ((a.k / (32 * KS) < ST ? tiles : std::min(tiles, device_cu_count())) + kXcds - 1) / kXcds * kXcds;
   auto go = [&](auto kern) {
@@ -567,6 +593,7 @@ void launch_pick(PairPick pick, const PairGemmArgs& a, bool gelu, int groups, co
     case p64x64: return launch_tile<4, 2, 1, 2, 4, 2>(a, gelu, groups, head_exp, stream);
     case p32x64: return launch_tile<2, 4, 1, 1, 5, 2>(a, gelu, groups, head_exp, stream);
     case p32x32: return launch_tile<2, 2, 1, 1, 6, 2>(a, gelu, groups, head_exp, stream);
+    case p16x32: return launch_tile<1, 2, 1, 1, 8, 2>(a, gelu, groups, head_exp, stream);
     default: return;
   }
 }
