@@ -23,7 +23,8 @@
 // writes the rows (8.4 + 10.2 us per layer of BERT-base, split rows 15).
 // Bound: at large m the power limit of the matrix cores (20375 rows, k = 768 / n = 2304, 768, 3072 + GELU and k = 3072 / n = 768:
 // 171, 68, 259, 226 us in the layer, 1265, 1060, 1113, 1276 TFLOP/s of 16-bit products, 4 to 6 % less on slower cards; split rows
-// 307, 112, 451, 413); below a round of the chip the k loop of one tile (134 rows: 10.2, 7.1, 12.8, 14.3 us against 15.2, 8.7, 16.1, 21.3).
+// 307, 112, 451, 413); below a round of the chip the k loop of one tile, which the LDS bounds (134 rows of at
+// most 256: 9.4, 6.8, 13.1, 13.9 us; split rows 15.2, 8.7, 16.1, 21.3).
 #include <algorithm>
 #include <atomic>
 #include <iterator>
