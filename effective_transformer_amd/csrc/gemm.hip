@@ -554,7 +554,7 @@ __device__ __forceinline__ int pair_swizzle(int row) { return (row >> 1) & 7; }
 // how the persistent kernel walks its tiles: flags, and the workgroups per XCD above them
 constexpr int kWalkReverse = 1, kWalkBlockedA = 2, kWalkWgs = 2;
 // `walk` and `columns` of the tiles below the persistent kernel's: a flag, strips_log2 above it, and C's leading dimension
-// (from kBtLongRows on 128 rows of C lie further apart than 32-bit byte offsets reach)
+// (from kBtLongRows on 128 rows of C lie further apart than 32-bit byte offsets reach: gemm_f16_bt_long_kernel)
 constexpr int kBtLongRows = 1 << 24;
 constexpr int kBtGelu = 1, kBtStrips = 1;
 #define ET_HEAD_ARGS const void *a0, const void *b0, const int32_t *rows_dev, int m_bound, int n, int k, int groups, int tiles_n, int columns, int walk
@@ -999,7 +999,8 @@ __device__ __forceinline__ TileAt strip_order(int tile, int tiles_m, int tiles_n
 }
 
 // The tile in row `tm` and column `tn_all` of tiles, whose columns run through the groups; `tiles_n` of them to a group.
-template <int MI, int NJ, int ST, typename Args>
+// LONG: rows of C from kBtLongRows values on, every row at a 64-bit address of its own.
+template <int MI, int NJ, int ST, bool LONG = false, typename Args>
 __device__ __forceinline__ void bt_tile(const TileHead& head, int tiles_n, const Args& args, int tm, int tn_all, unsigned char* smem) {
 #if defined(__HIP_DEVICE_COMPILE__)   // device-only types in the body; the host pass only needs the stub
   using Tile = BtTile<MI, NJ, ST>;
@@ -1141,7 +1142,21 @@ __device__ __forceinline__ void bt_tile(const TileHead& head, int tiles_n, const
   // scalar.  With a branch, a 64-bit address and scalar loads of ldc and the GELU flag at every row, each waited for, a launch of
   // 2000 x 2304 took 3.1 us from its last MFMA to its end, of which its bytes need 1.6 (k = 768, us a launch, one that does nothing
   // 2.2: 2000 rows to 2304 / 768 / 3072 columns 11.5 / 6.8 / 15.9 -> 11.0 / 6.1 / 14.9, 640 rows 6.8 / 4.9 / 8.2 -> 6.2 / 4.5 / 7.7).
-  if (col < N) {
+  if constexpr (LONG) {
+    static_assert(NJ == NB, "a lane's columns in one piece");
+    const int row = wm * 16 * MI + g * 4;
+    _Float16* c = c_tile + (size_t)row * head.ldc + (col - n0);
+#pragma unroll
+    for (int i = 0; i < MI; ++i)
+#pragma unroll
+      for (int r = 0; r < 4; ++r) {
+        BiasN o;
+#pragma unroll
+        for (int j = 0; j < NB; ++j) o[j] = f2h(acc[i][j][r]);
+        o = head.gelu ? bias_gelu_half<BiasN, NB>(o, biasv) : o + biasv;
+        if (col < N && m0 + row + i * 16 + r < rows) *reinterpret_cast<BiasN*>(c + (size_t)(i * 16 + r) * head.ldc) = o;
+      }
+  } else if (col < N) {
     const __amdgpu_buffer_rsrc_t rsrc_c = __builtin_amdgcn_make_buffer_rsrc(
         c_tile, 0, ((uint32_t)(min(rows - m0, BM) - 1) * (uint32_t)head.ldc + (uint32_t)min(N - n0, BN)) * 2u, 0x00020000);
     const uint32_t voff = ((uint32_t)(wm * 16 * MI + g * 4) * (uint32_t)head.ldc + (uint32_t)(col - n0)) * 2u;
@@ -1197,6 +1212,20 @@ __global__ __launch_bounds__(kHThreads) __attribute__((amdgpu_waves_per_eu(2))) 
   if (tile < 0) return;
   const TileAt at = strip_order(tile, tiles_m, tiles_n_all, walk >> kBtStrips);
   bt_tile<MI, NJ, ST>(head, tiles_n, args, at.row, at.column, smem);
+}
+
+// Rows of C from kBtLongRows values on, which no 32-bit offset from a tile's first row covers (31 rows of 69.3 million values pass
+// 2^32 bytes): 128 x 128 tiles, the ones that so many columns always come out at.
+__global__ __launch_bounds__(kHThreads) __attribute__((amdgpu_waves_per_eu(2))) void gemm_f16_bt_long_kernel(ET_HEAD_ARGS, TileArgs args) {
+  extern __shared__ __attribute__((aligned(1024))) unsigned char smem[];
+  TileHead head = tile_head(a0, b0, rows_dev, m_bound, n, k, groups, args);
+  head.ldc = columns;
+  head.gelu = walk & kBtGelu;
+  const int tiles_n_all = tiles_n * groups, tiles_m = (int)((unsigned)(head.rows + 127) / 128);
+  const int tile = remap_valid_tile(blockIdx.x, tiles_m * tiles_n_all);
+  if (tile < 0) return;
+  const TileAt at = strip_order(tile, tiles_m, tiles_n_all, walk >> kBtStrips);
+  bt_tile<4, 4, 2, true>(head, tiles_n, args, at.row, at.column, smem);
 }
 
 // Where only the device knows the row count, it picks the tile: the tiles that are the best for some count up to the launch's
@@ -1687,11 +1716,11 @@ void launch_f16(GemmArgs a, hipStream_t stream) {
 
 // Operand rows (of A and of B^T) that the tiles of one XCD's band touch, which is what its L2 has to fetch, with the tiles in
 // 1 << strips_log2 strips of columns.
-inline int band_rows(int tiles_m, int tiles_n, int bm, int bn, int strips_log2) {
+inline long band_rows(int tiles_m, int tiles_n, int bm, int bn, int strips_log2) {
   const int band = (int)((unsigned)(tiles_m * tiles_n + kXcds - 1) / kXcds);
   const int wide = (tiles_n + (1 << strips_log2) - 1) >> strips_log2, per_strip = tiles_m * wide;
-  if (band <= per_strip) return std::min(tiles_m, (int)((unsigned)(band + wide - 1) / wide)) * bm + wide * bn;
-  return tiles_m * bm + (int)((unsigned)(band + per_strip - 1) / per_strip) * wide * bn;
+  if (band <= per_strip) return (long)std::min(tiles_m, (int)((unsigned)(band + wide - 1) / wide)) * bm + (long)wide * bn;
+  return (long)tiles_m * bm + (long)((unsigned)(band + per_strip - 1) / per_strip) * wide * bn;
 }
 // Along the rows (0), down the columns (strips of one column), or in two, four or eight strips.  Each XCD fetches the operand rows
 // of its band for itself, so that a band as high as it is wide fetches the fewest.  Up to 1024 rows the columns spread the weights
@@ -1701,14 +1730,16 @@ inline int band_rows(int tiles_m, int tiles_n, int bm, int bn, int strips_log2) 
 // What saves less than a quarter of the rows costs more in the second division of a tile's number (0.1 us) than it gives.
 constexpr int kColumnRows = 1024, kMaxStripsLog2 = 3;
 inline int best_strips_log2(int tiles_m, int tiles_n, int bm, int bn) {
-  int best = 0, rows = band_rows(tiles_m, tiles_n, bm, bn, 0);
+  int best = 0;
+  long rows = band_rows(tiles_m, tiles_n, bm, bn, 0);
   if (tiles_m * bm <= kColumnRows + bm && tiles_n > 1) {
-    const int down = 32 - __builtin_clz((unsigned)(tiles_n - 1)), r = band_rows(tiles_m, tiles_n, bm, bn, down);
+    const int down = 32 - __builtin_clz((unsigned)(tiles_n - 1));
+    const long r = band_rows(tiles_m, tiles_n, bm, bn, down);
     if (4 * r <= 3 * rows) best = down, rows = r;
   }
-  int limit = 3 * rows / 4;
+  long limit = 3 * rows / 4;
   for (int l = 1; l <= kMaxStripsLog2 && (1 << l) < tiles_n; ++l) {
-    const int r = band_rows(tiles_m, tiles_n, bm, bn, l);
+    const long r = band_rows(tiles_m, tiles_n, bm, bn, l);
     if (r <= limit) best = l, limit = r - 1;
   }
   return best;
@@ -1728,6 +1759,18 @@ void launch_f16_bt(GemmArgs a, hipStream_t stream) {
   const int strips = best_strips_log2(a.tiles_m, a.tiles_n * a.groups, Tile::BM, Tile::BN);
   kern<<<a.per_xcd * kXcds, kHThreads, Tile::SMEM_BYTES, stream>>>(a.A[0], a.B[0], a.rows_dev, a.m_bound, a.n, a.k, a.groups, a.tiles_n, a.ldc,
                                                                     strips << kBtStrips | (a.gelu ? kBtGelu : 0), tile_args(a));
+}
+
+void launch_bt_long(GemmArgs a, hipStream_t stream) {
+  using Tile = BtTile<4, 4, 2>;
+  a.tiles_m = (a.m_bound + Tile::BM - 1) / Tile::BM;
+  a.tiles_n = (int)(((unsigned)a.n + Tile::BN - 1) / Tile::BN);
+  const int total = a.tiles_m * a.tiles_n * a.groups;
+  a.per_xcd = (total + kXcds - 1) / kXcds;
+  allow_dynamic_lds(reinterpret_cast<const void*>(gemm_f16_bt_long_kernel), (int)Tile::SMEM_BYTES);
+  const int strips = best_strips_log2(a.tiles_m, a.tiles_n * a.groups, Tile::BM, Tile::BN);
+  gemm_f16_bt_long_kernel<<<a.per_xcd * kXcds, kHThreads, Tile::SMEM_BYTES, stream>>>(a.A[0], a.B[0], a.rows_dev, a.m_bound, a.n, a.k, a.groups, a.tiles_n,
+                                                                                     a.ldc, strips << kBtStrips | (a.gelu ? kBtGelu : 0), tile_args(a));
 }
 
 int device_cu_count() {
@@ -2127,7 +2170,7 @@ void launch_gemm(DType t, const GemmGroups& g, void* C, int ldc, int m_bound, in
     } else if (g.b_transposed) {
       // one tile per workgroup, the tile chosen for the launch's shape (pick_bt_tile)
       if (launch_bt_wave(a, stream)) return;
-      if (ldc >= kBtLongRows) return launch_bt_tile({1, 1, false}, a, stream);
+      if (ldc >= kBtLongRows) return launch_bt_long(a, stream);
       if (rows_dev != nullptr && launch_bt_rows(a, stream)) return;
       launch_bt_tile(pick_bt_tile(m_bound, n, k, g.groups, device_cu_count(), false), a, stream);
     } else {

@@ -45,3 +45,26 @@ def test_longest_rows():
     out = ko.gemm_bt(a, bt, out=torch.empty(m, n, device="cuda", dtype=torch.float16))
     for p in picks:
         assert torch.equal(out[:, p:p + 264], ko.gemm_bt(a, bt[p:p + 264].contiguous())), p
+
+
+# ... and a C and a bias off the 8-byte boundaries: the last row of the first 32 begins behind 4 GB (from 69 273 672 columns on), a lane's first
+# row does (80 000 008), two tiles of rows; once with a row count on the device
+@pytest.mark.parametrize("m,n,shift,on_device", [(33, 69273672, 1, False), (33, 80000008, 2, True), (200, (1 << 24) + 8, 3, False)])
+def test_longest_rows_off_their_boundaries(m, n, shift, on_device):
+    k = 64
+    print("longest rows off their boundaries", m, n, shift, on_device, flush=True)
+    g = torch.Generator(device="cuda").manual_seed(m + n)
+    a = torch.randn(m, k, device="cuda", dtype=torch.float16, generator=g)
+    bt = torch.empty(n, k, device="cuda", dtype=torch.float16)
+    bias = torch.randn(n + 8, device="cuda", dtype=torch.float16, generator=g)[shift:shift + n]
+    picks = [0, 1000, (1 << 23) - 8, n // 2 + 16, n - 264]
+    for p in picks:
+        bt[p:p + 264] = torch.randn(264, k, device="cuda", dtype=torch.float16, generator=g)
+    rows = m - 2 if on_device else m
+    room = torch.full((m * n + 8,), 7.0, device="cuda", dtype=torch.float16)
+    out = room[shift:shift + m * n].view(m, n)
+    ko.gemm_bt(a, bt, bias, out=out, m_dev=torch.tensor([rows], dtype=torch.int32, device="cuda") if on_device else None)
+    for p in picks:
+        want = ko.gemm_bt(a, bt[p:p + 264].contiguous(), bias[p:p + 264].contiguous())
+        assert torch.equal(out[:rows, p:p + 264], want[:rows]), p
+    assert (out[rows:] == 7.0).all() and (room[:shift] == 7.0).all() and (room[shift + m * n:] == 7.0).all()
