@@ -1951,7 +1951,7 @@ void launch_bt_tile(BtPick p, const GemmArgs& a, hipStream_t stream) {
 bool launch_bt_wave(GemmArgs a, hipStream_t stream) {
   a.tiles_n = (a.n + 15) / 16;
   const long wgs = (long)((a.m_bound + 15) / 16) * a.tiles_n * a.groups;
-  if (wgs > 2l * device_cu_count() && a.ldc < kBtLongRows) return false;
+  if (wgs > 2l * device_cu_count()) return false;
   bool aligned = ((uintptr_t)a.C | (uintptr_t)a.ldc * 2) % 8 == 0;
   for (int g = 0; g < a.groups; ++g) aligned = aligned && (uintptr_t)a.bias[g] % 8 == 0;
   if (!aligned) return false;
