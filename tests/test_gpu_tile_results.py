@@ -9,10 +9,12 @@ pytestmark = pytest.mark.gpu
 
 
 # one of every tile (row blocks x column blocks, d: two workgroups a CU) that a device of 256 CUs chooses, the last one rounds of them
-@pytest.mark.parametrize("m,n,k", [(49, 2152, 192), (40, 4112, 192), (258, 3304, 192), (4167, 72, 192), (289, 4120, 192), (291, 4120, 768),
-                                   (676, 4112, 192), (5461, 136, 192), (5590, 328, 192), (5581, 328, 768), (5948, 648, 192), (5902, 648, 768),
-                                   (5893, 1288, 192), (5471, 264, 768), (5464, 656, 192), (674, 4112, 768), (5379, 1032, 192), (4429, 1288, 768),
-                                   (5394, 1544, 192), (5387, 1040, 2112), (5898, 1928, 192)])
+TILES = [(49, 2152, 192), (40, 4112, 192), (258, 3304, 192), (4167, 72, 192), (289, 4120, 192), (291, 4120, 768), (676, 4112, 192), (5461, 136, 192),
+         (5590, 328, 192), (5581, 328, 768), (5948, 648, 192), (5902, 648, 768), (5893, 1288, 192), (5471, 264, 768), (5464, 656, 192),
+         (674, 4112, 768), (5379, 1032, 192), (4429, 1288, 768), (5394, 1544, 192), (5387, 1040, 2112), (5898, 1928, 192)]
+
+
+@pytest.mark.parametrize("m,n,k", TILES)
 @pytest.mark.parametrize("gelu", [False, True])
 @pytest.mark.parametrize("on_device", [False, True])
 def test_every_tile(m, n, k, gelu, on_device):
@@ -30,6 +32,40 @@ def test_every_tile(m, n, k, gelu, on_device):
     assert (out[rows:] == 7.0).all()
     if not gelu:
         assert torch.equal(ko.gemm_bt(a, bt), ko.gemm(a, w))
+
+
+# a C and a bias one, two and three values off the 8-byte boundaries, which C's stores of 2 to 16 bytes a lane then lie across; the last
+# ones are few enough for tiles of 16 x 16, which such a C does not go to
+@pytest.mark.parametrize("m,n,k", TILES + [(20, 768, 192), (5, 8, 256), (33, 40, 768)])
+@pytest.mark.parametrize("on_device", [False, True])
+def test_results_off_their_boundaries(m, n, k, on_device):
+    print("off the boundaries", m, n, k, on_device, flush=True)
+    g = torch.Generator(device="cuda").manual_seed(m + n + k)
+    a = torch.randn(m, k, device="cuda", dtype=torch.float16, generator=g)
+    w = torch.randn(k, n, device="cuda", dtype=torch.float16, generator=g).mul_(k ** -0.5)
+    values = torch.randn(n + 8, device="cuda", dtype=torch.float16, generator=g)
+    bt = ko.transpose_weight(w)
+    rows = max(m - 7, 0) if on_device else m
+    count = torch.tensor([rows], dtype=torch.int32, device="cuda") if on_device else None
+    for shift in (1, 2, 3):
+        bias = values[shift:shift + n]
+        for gelu in (False, True):
+            want = ko.gemm(a, w, bias=bias.clone(), gelu=gelu)
+            room = torch.full((m * n + 16,), 7.0, device="cuda", dtype=torch.float16)
+            ko.gemm_bt(a, bt, bias, out=room[shift:shift + m * n].view(m, n), gelu=gelu, m_dev=count)
+            assert torch.equal(room[shift:shift + rows * n].view(rows, n), want[:rows]), (shift, gelu)
+            assert (room[:shift] == 7.0).all() and (room[shift + rows * n:] == 7.0).all(), (shift, gelu)
+
+
+# turned weights, which leave through a descriptor as well
+@pytest.mark.parametrize("k,n", [(64, 64), (72, 200), (768, 40)])
+def test_turned_weights_off_their_boundaries(k, n):
+    w = torch.randn(k, n, device="cuda", dtype=torch.float16)
+    for shift in (1, 2, 3):
+        room = torch.full((n * k + 16,), 7.0, device="cuda", dtype=torch.float16)
+        ko.transpose_weight(w, out=room[shift:shift + n * k].view(n, k))
+        assert torch.equal(room[shift:shift + n * k].view(n, k), w.t())
+        assert (room[:shift] == 7.0).all() and (room[shift + n * k:] == 7.0).all()
 
 
 # rows of C so long that a tile's last one lies more than 4 GB behind its first
