@@ -123,11 +123,13 @@ __device__ __forceinline__ _Float16 f2h(float f) { return (_Float16)f; }   // v_
 // the line in the caches on its way.  What lies dirty in the L2s when a kernel ends is written back before the next one starts, which
 // the fp16 products' C and the weights' turned copies are spared so.  Encoders of 12 layers, C in plain stores and written through, one
 // card in turn: 16 x 64 in a graph 508 -> 502 us, 8 x 128 from ids 475 -> 467, 100 x 32 753 -> 730, the ops on 217 x 53 1877 -> 1810, 32 x 512
-// 2858 -> 2788, 16 x 1024 2841 -> 2692 (another card: 32 x 512 2707 -> 2676, ops level).  It takes stores that fill their lines in
-// whole pieces of 8 or 16 bytes a lane: 16 bytes in two stores of 8 are written twice (ops 1809 -> 1895).  Level or worse, and so plain:
-// LayerNorm's rows, the short attention (1000 x 64 7435 -> 7655), the streaming one (8-byte pieces of a head's rows: 64 x 512 5412 -> 5538,
-// 193 x 100 2995 -> 3055), the fp32 products' C in floats (500 x 64 11330 -> 11440, 210 x 64 5538 -> 5601).  Matrices beyond the last-level cache keep nt (1000 x 64: sc1 instead or both
-// +0.2 to +0.5 %).
+// 2858 -> 2788, 16 x 1024 2841 -> 2692 (another card: 32 x 512 2707 -> 2676, ops level).  So do the small tiles' pieces of 2 and 4 bytes a lane
+// (12 layers, two runs of one library within 0.4 %): 5 x 64 of 8 heads in a graph, 2 bytes plain 362, 4 bytes plain 362, all through 359; 5 x 64
+// of 12 heads, 4 bytes plain 415, through 411, 2 bytes level; 12 x 64 531 and 529; 31 x 64, the 4 bytes of six columns plain 734, through 727.
+// 16 bytes in two stores of 8 are written twice (ops 1809 -> 1895).  Level or worse, and so plain: LayerNorm's fp16 rows, the short fp16
+// attention (1000 x 64 7435 -> 7655), the streaming one (8-byte pieces of a head's rows: 64 x 512 5412 -> 5538, 193 x 100 2995 -> 3055), the fp32
+// one's 16-byte pieces of pair rows (100 x 64 2770 -> 2805, 500 x 64 10960 -> 11130, 15 x 379 level), the fp32 products' C in floats (500 x 64
+// 11330 -> 11440, 210 x 64 5538 -> 5601).  Matrices beyond the last-level cache keep nt (1000 x 64: sc1 instead or both +0.2 to +0.5 %).
 constexpr int kPolicyNt = 2, kPolicyThrough = 16;
 // 8 bytes, written through.
 template <typename V>
@@ -212,7 +214,8 @@ __device__ __forceinline__ float pair_scale(int e) { return __builtin_ldexpf(1.0
 // conversion, where the compiler converted every value a second time for l (FFN-up on 20375 rows 277 -> 263 us together with
 // gemm_pair_kernel's one lane per exponent, same bits).
 // Pieces of 8 bytes, those of FFN-up's large tiles, of LayerNorm and of the short attention, are written through (kPolicyThrough): fp32
-// encoders of 12 layers, plain and so, 40 x 64 positions 1740 -> 1705 us, 100 x 64 2936 -> 2908, 210 x 64 5573 -> 5538, 500 x 64 11425 -> 11330.
+// encoders of 12 layers, plain and so, 40 x 64 positions 1680 -> 1650 us, 100 x 64 2803 -> 2778, 160 x 64 4081 -> 4072, 15 x 379 2904 -> 2887; from
+// 210 x 64 on level (500 x 64 10995 and 11028, with 0.3 % between two runs of one library).
 template <int N, typename V>
 __device__ __forceinline__ void store_pair(_Float16* row, int col, const V& v, float scale) {
   typedef _Float16 hvec __attribute__((ext_vector_type(N)));

@@ -213,6 +213,9 @@ __global__ __launch_bounds__(kMoveThreads) void compress_rows_kernel(
 // Positions from which on a workgroup takes 32 of them, and not 8: with fewer positions the launch is short of workgroups, and each
 // goes through its chunks in several trips to memory (us a launch, 32 and 8 positions a workgroup: 256 rows of 3 KB 8.8 and 4.2, 1024
 // of 1.5 KB 6.1 and 3.5, 3200 6.4 and 4.0, 11501 8.3 and 6.8; with 32 at 16384 9.1, 64000 23.2).
+// From there on the searches of four times the workgroups cost what the shorter trips give, at any row length (one layer through the ops,
+// 32 and 8: rows of 1 KB, 3840 positions 102.0 and 100.2, 7680 101.0 both, 16384 150.3 both, 19200 170.2 and 172.7, 38400 307.3 and 309.5; of
+// 2 KB 132.4 and 130.5, 213.6 and 212.8, 380.3 and 379.6, 438.8 and 436.7, 816.0 and 819.4; of 4 KB 327.9 and 322.4, and level from 7680 on).
 constexpr int kRestoreMany = 16384;
 
 // One pass over the padded output: every 16-byte chunk of [B*S, row] is written exactly once,
@@ -286,7 +289,9 @@ __global__ __launch_bounds__(kMoveThreads) void restore_rows_kernel(
 // The same pass where the scan left the packed row of every position (et_encoder): flattened over (position, chunk), UNROLL chunks
 // a lane, two dependent loads and the stores where the search takes four or five.  Bound by the loads' latency for a few thousand
 // positions (in an encoder, us a launch, the search with 32 positions a workgroup before: 256 rows of 3 KB 9.3 -> 3.9), by memory for
-// many (64000 of 1.5 KB 23.5 -> 22.5, 16384 10.1 -> 8.3).  Eight chunks a lane once that still gives four workgroups to a CU, else two.
+// many (64000 of 1.5 KB 23.5 -> 22.5, 16384 10.1 -> 8.3).  Eight chunks a lane once that still gives 1024 workgroups, four to a CU of the
+// whole chip, else two (one layer, two and eight: rows of 1 KB, 1920 positions 47.7 and 48.4, 7680 88.2 and 88.5, 21760 171.5 and 173.2, 32000
+// 248.1 and 246.4, 51200 394.3 and 392.4; of 2 and 4 KB two are ahead by up to 1.2 % below 2^21 chunks and level beyond).
 template <typename CH, int UNROLL>
 __global__ __launch_bounds__(kMoveThreads) void mapped_restore_rows_kernel(CH* __restrict__ to, const CH* __restrict__ from,
                                                                            const int32_t* __restrict__ packed_row, uint32_t total,

@@ -158,11 +158,11 @@ void launch_mask_class(DType t, const void* attr_mask, const int32_t* seq_start,
 bool attention_writes_pieces(const void* q, const void* k, const void* v, int layout, int packed_ld, int d);
 
 // ---- gemm.hip ----------------------------------------------------------------------------
-// Up to three independent column groups share one launch (the Q/K/V projections): group g
-// computes C[:, g*n : (g+1)*n] = A[g] . B[g] (+ bias[g]) into a row-major C with leading
-// dimension ldc.  groups == 1 is the plain GEMM.
+// Up to three column groups share one launch (the Q/K/V projections): group g computes
+// C[:, g*n : (g+1)*n] = A[g > 0] . B[g] (+ bias[g]) into a row-major C with leading dimension ldc;
+// groups 1 and 2 share their A (K and V are made of the same rows).  groups == 1 is the plain GEMM.
 struct GemmGroups {
-  const void* A[2];                  // of the first group, of the others
+  const void* A[2];                  // of group 0, of groups 1 and 2
   const void* B[3];
   const void* bias[3];
   int groups;
