@@ -554,7 +554,7 @@ __device__ __forceinline__ int pair_swizzle(int row) { return (row >> 1) & 7; }
 // how the persistent kernel walks its tiles: flags, and the workgroups per XCD above them
 constexpr int kWalkReverse = 1, kWalkBlockedA = 2, kWalkWgs = 2;
 // `walk` and `columns` of the tiles below the persistent kernel's: a flag, strips_log2 above it, and C's leading dimension
-// (from kBtLongRows on 128 rows of C lie further apart than 32-bit byte offsets reach: gemm_f16_bt_long_kernel)
+// (from kBtLongRows on 128 rows of C lie further apart than 32-bit byte offsets reach: kBtLongTile)
 constexpr int kBtLongRows = 1 << 24;
 constexpr int kBtGelu = 1, kBtStrips = 1;
 #define ET_HEAD_ARGS const void *a0, const void *b0, const int32_t *rows_dev, int m_bound, int n, int k, int groups, int tiles_n, int columns, int walk
@@ -986,6 +986,12 @@ struct BtTile {
 // those of them with a CU to themselves that gemm_f16_bt_rows_kernel chooses from (128 x 256 would cost all of them registers)
 #define ET_BT_ROWS_TILES(X) X(1, 1, 0, 5) X(1, 2, 0, 5) X(2, 2, 0, 4) X(2, 4, 0, 4) X(3, 2, 0, 4) X(3, 4, 0, 4) X(3, 6, 0, 3) X(4, 2, 0, 4) X(4, 4, 0, 4) X(4, 6, 0, 3)
 
+// The tile that takes rows of C from kBtLongRows values on, which no 32-bit offset from a tile's first row covers (31 rows of 69.3
+// million values pass 2^32 bytes): the one that so many columns come out at anyway.  In a kernel of their own they cost the others their
+// place in the library (16 x 1024 positions +0.6 %).
+template <int MI, int NJ, int ST>
+constexpr bool kBtLongTile = MI == 4 && NJ == 4 && ST == 2;
+
 // Tiles in the order of 1 << strips_log2 strips of columns, along the rows inside a strip (see band_rows).
 struct TileAt {
   int row, column;
@@ -999,8 +1005,7 @@ __device__ __forceinline__ TileAt strip_order(int tile, int tiles_m, int tiles_n
 }
 
 // The tile in row `tm` and column `tn_all` of tiles, whose columns run through the groups; `tiles_n` of them to a group.
-// LONG: rows of C from kBtLongRows values on, every row at a 64-bit address of its own.
-template <int MI, int NJ, int ST, bool LONG = false, typename Args>
+template <int MI, int NJ, int ST, typename Args>
 __device__ __forceinline__ void bt_tile(const TileHead& head, int tiles_n, const Args& args, int tm, int tn_all, unsigned char* smem) {
 #if defined(__HIP_DEVICE_COMPILE__)   // device-only types in the body; the host pass only needs the stub
   using Tile = BtTile<MI, NJ, ST>;
@@ -1142,21 +1147,23 @@ __device__ __forceinline__ void bt_tile(const TileHead& head, int tiles_n, const
   // scalar.  With a branch, a 64-bit address and scalar loads of ldc and the GELU flag at every row, each waited for, a launch of
   // 2000 x 2304 took 3.1 us from its last MFMA to its end, of which its bytes need 1.6 (k = 768, us a launch, one that does nothing
   // 2.2: 2000 rows to 2304 / 768 / 3072 columns 11.5 / 6.8 / 15.9 -> 11.0 / 6.1 / 14.9, 640 rows 6.8 / 4.9 / 8.2 -> 6.2 / 4.5 / 7.7).
-  if constexpr (LONG) {
-    static_assert(NJ == NB, "a lane's columns in one piece");
-    const int row = wm * 16 * MI + g * 4;
-    _Float16* c = c_tile + (size_t)row * head.ldc + (col - n0);
+  const bool long_rows = kBtLongTile<MI, NJ, ST> && head.ldc >= kBtLongRows;
+  if constexpr (kBtLongTile<MI, NJ, ST>)
+    if (long_rows) {                             // every row at a 64-bit address of its own
+      const int row = wm * 16 * MI + g * 4;
+      _Float16* c = c_tile + (size_t)row * head.ldc + (col - n0);
 #pragma unroll
-    for (int i = 0; i < MI; ++i)
+      for (int i = 0; i < MI; ++i)
 #pragma unroll
-      for (int r = 0; r < 4; ++r) {
-        BiasN o;
+        for (int r = 0; r < 4; ++r) {
+          BiasN o;
 #pragma unroll
-        for (int j = 0; j < NB; ++j) o[j] = f2h(acc[i][j][r]);
-        o = head.gelu ? bias_gelu_half<BiasN, NB>(o, biasv) : o + biasv;
-        if (col < N && m0 + row + i * 16 + r < rows) *reinterpret_cast<BiasN*>(c + (size_t)(i * 16 + r) * head.ldc) = o;
-      }
-  } else if (col < N) {
+          for (int j = 0; j < NB; ++j) o[j] = f2h(acc[i][j][r]);
+          o = head.gelu ? bias_gelu_half<BiasN, NB>(o, biasv) : o + biasv;
+          if (col < N && m0 + row + i * 16 + r < rows) *reinterpret_cast<BiasN*>(c + (size_t)(i * 16 + r) * head.ldc) = o;
+        }
+    }
+  if (!long_rows && col < N) {
     const __amdgpu_buffer_rsrc_t rsrc_c = __builtin_amdgcn_make_buffer_rsrc(
         c_tile, 0, ((uint32_t)(min(rows - m0, BM) - 1) * (uint32_t)head.ldc + (uint32_t)min(N - n0, BN)) * 2u, 0x00020000);
     const uint32_t voff = ((uint32_t)(wm * 16 * MI + g * 4) * (uint32_t)head.ldc + (uint32_t)(col - n0)) * 2u;
@@ -1212,20 +1219,6 @@ __global__ __launch_bounds__(kHThreads) __attribute__((amdgpu_waves_per_eu(2))) 
   if (tile < 0) return;
   const TileAt at = strip_order(tile, tiles_m, tiles_n_all, walk >> kBtStrips);
   bt_tile<MI, NJ, ST>(head, tiles_n, args, at.row, at.column, smem);
-}
-
-// Rows of C from kBtLongRows values on, which no 32-bit offset from a tile's first row covers (31 rows of 69.3 million values pass
-// 2^32 bytes): 128 x 128 tiles, the ones that so many columns always come out at.
-__global__ __launch_bounds__(kHThreads) __attribute__((amdgpu_waves_per_eu(2))) void gemm_f16_bt_long_kernel(ET_HEAD_ARGS, TileArgs args) {
-  extern __shared__ __attribute__((aligned(1024))) unsigned char smem[];
-  TileHead head = tile_head(a0, b0, rows_dev, m_bound, n, k, groups, args);
-  head.ldc = columns;
-  head.gelu = walk & kBtGelu;
-  const int tiles_n_all = tiles_n * groups, tiles_m = (int)((unsigned)(head.rows + 127) / 128);
-  const int tile = remap_valid_tile(blockIdx.x, tiles_m * tiles_n_all);
-  if (tile < 0) return;
-  const TileAt at = strip_order(tile, tiles_m, tiles_n_all, walk >> kBtStrips);
-  bt_tile<4, 4, 2, true>(head, tiles_n, args, at.row, at.column, smem);
 }
 
 // Where only the device knows the row count, it picks the tile: the tiles that are the best for some count up to the launch's
@@ -1761,18 +1754,6 @@ void launch_f16_bt(GemmArgs a, hipStream_t stream) {
                                                                     strips << kBtStrips | (a.gelu ? kBtGelu : 0), tile_args(a));
 }
 
-void launch_bt_long(GemmArgs a, hipStream_t stream) {
-  using Tile = BtTile<4, 4, 2>;
-  a.tiles_m = (a.m_bound + Tile::BM - 1) / Tile::BM;
-  a.tiles_n = (int)(((unsigned)a.n + Tile::BN - 1) / Tile::BN);
-  const int total = a.tiles_m * a.tiles_n * a.groups;
-  a.per_xcd = (total + kXcds - 1) / kXcds;
-  allow_dynamic_lds(reinterpret_cast<const void*>(gemm_f16_bt_long_kernel), (int)Tile::SMEM_BYTES);
-  const int strips = best_strips_log2(a.tiles_m, a.tiles_n * a.groups, Tile::BM, Tile::BN);
-  gemm_f16_bt_long_kernel<<<a.per_xcd * kXcds, kHThreads, Tile::SMEM_BYTES, stream>>>(a.A[0], a.B[0], a.rows_dev, a.m_bound, a.n, a.k, a.groups, a.tiles_n,
-                                                                                     a.ldc, strips << kBtStrips | (a.gelu ? kBtGelu : 0), tile_args(a));
-}
-
 int device_cu_count() {
   constexpr int kMaxDevices = 64;
   static std::atomic<int> cus[kMaxDevices] = {};      // handles on several GPUs may launch from different threads
@@ -2170,7 +2151,7 @@ void launch_gemm(DType t, const GemmGroups& g, void* C, int ldc, int m_bound, in
     } else if (g.b_transposed) {
       // one tile per workgroup, the tile chosen for the launch's shape (pick_bt_tile)
       if (launch_bt_wave(a, stream)) return;
-      if (ldc >= kBtLongRows) return launch_bt_long(a, stream);
+      if (ldc >= kBtLongRows) return launch_f16_bt<4, 4, 2>(a, stream);
       if (rows_dev != nullptr && launch_bt_rows(a, stream)) return;
       launch_bt_tile(pick_bt_tile(m_bound, n, k, g.groups, device_cu_count(), false), a, stream);
     } else {
